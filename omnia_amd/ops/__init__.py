@@ -757,7 +757,10 @@ MOE_LIBRARY_ROWS = 1024  # mean rows/expert above which eager calls use hipBLASL
 # mean rows per local expert from which the grouped GEMMs run on the 256x256
 # prefill tile (pgemm.hip EPI 5 / 6, 256-row expert segments); below it the
 # 64-row grouped kernels (moe.hip) waste less padding.  Both are graph-safe.
-MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "512"))
+# Both products, 64-row / 256-row: at 96 rows 164 / 204 us, at 128 213 / 208, at 512
+# 652 / 268 (8 experts of 2048 x 4096); at 96 174 / 190, at 128 202 / 193 (32 of 2048 x
+# 1024); wide experts cross earlier, at 64 803 / 791 (8 of 4096 x 14336)
+MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
 
 
 def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=None,

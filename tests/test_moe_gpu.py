@@ -86,6 +86,7 @@ def test_moe_library_path_matches_grouped(monkeypatch):
     (2048, 512, 512, 8, 2, 0, 8),    # prefill-sized: 256x256-tile grouped GEMMs
     (2500, 256, 384, 8, 2, 0, 8),    # ragged expert segments, I not a multiple of 256
     (4096, 512, 256, 8, 2, 4, 4),    # expert-parallel shard: experts 4..7 only
+    (513, 256, 256, 8, 2, 0, 8),     # from 128 rows an expert, segments half full
 ])
 def test_moe_tile256_prefill_matches_reference(T, d, I, E, k, e_lo, e_n):
     """Large batches run the 256-row-segment grouped GEMMs (pgemm.hip EPI 5 / 6)
