@@ -205,6 +205,17 @@ class HybridModel(Projections):
             w["layers"].append(seen[own])
         return w
 
+    def prepack_decode(self, max_batch: int) -> int:
+        """Lay projections out for small decode batches; returns the bytes.  Feed-forwards find
+        the copies of theirs beside the weights."""
+        n = self.pack_streams()
+        for w in self.w["layers"]:
+            for m in (w["mlp"], (w["mlp"] or {}).get("shared")):
+                for k in ("gate_up", "up", "down") if m else ():
+                    if k in m and m[k].data_ptr() in self._streams:
+                        m[k + "_stream"] = self._streams[m[k].data_ptr()]
+        return n
+
     # ------------------------------------------------------------ cache
     def allocate_cache(self, num_blocks: int, block_size: int, n_slots: int) -> HybridCache:
         layers: list = []
@@ -218,7 +229,8 @@ class HybridModel(Projections):
         """A projection whose consumer reads plain rows (no split-K slabs)."""
         if self._pgemm_ok(x.shape[0], x.shape[1], w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
-        return ops.linear(x, w)
+        y = self._stream(0, x, w)
+        return ops.linear(x, w) if y is None else y
 
     def _slabs(self, tag, x, w, is_decode) -> torch.Tensor:
         """A projection whose consumer also reduces split-K slabs."""
@@ -304,9 +316,10 @@ class HybridModel(Projections):
     def logits(self, h: torch.Tensor, is_decode: bool = False) -> torch.Tensor:
         W = self.w["head"]
         cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
-        if cfg is not None and cfg[2] == 1:
+        z = self._stream(0, h, W)
+        if z is None and cfg is not None and cfg[2] == 1:
             z = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
-        else:
+        elif z is None:
             z = ops.linear(h, W)
         cap = self.cfg.logit_softcap
         return mops.softcap_(z, cap) if cap else z

@@ -223,7 +223,10 @@ class LlamaModel(Projections):
 
     def prepack_decode(self, max_batch: int) -> int:
         """Pack the decode projections for every batch bucket up to ``max_batch``;
-        returns the bytes packed (0: off / nothing on tgemm / over budget)."""
+        returns the bytes packed (0: off / over budget)."""
+        return self.pack_streams() + self._prepack_tiles(max_batch)
+
+    def _prepack_tiles(self, max_batch: int) -> int:
         self._packed = {}
         env = os.environ.get("OMNIA_TGEMM_PACK", "1")
         if env not in ("1", "force") or self.device.type != "cuda" or self.tp != 1 \
@@ -296,13 +299,7 @@ class LlamaModel(Projections):
             q = ops.pgemm(3, h, wqkv, positions=fb.positions, cos_sin=self.cos_sin,
                           k_cache=kv.k[li], v_cache=kv.v[li], slots=fb.slots, hq=self.hq,
                           hkv=self.hkv, block_size=kv.block_size)
-            q3 = q.view(T, self.hq, D)
-            if fb.num_decode:
-                o = self._mixed_attention(li, q3, fb, kv)
-            else:
-                o = ops.prefill_attention(q3, kv.k[li], kv.v[li], fb.block_tables,
-                                          fb.q_start_loc, fb.seq_lens, self.scale, fb.tile_seq,
-                                          fb.tile_q0)
+            o = self._attend(li, q.view(T, self.hq, D), fb, kv)
             return self._proj("o", o.view(T, self.hq * D), self.w["layers"][li]["o"], False)
         qkv = self._proj("qkv", h, wqkv, fb.is_decode)
         if fb.cp is not None:
@@ -322,18 +319,7 @@ class LlamaModel(Projections):
             v = qkv[:, (self.hq + self.hkv) * D:]
             ops.rope_kv(q, k, v, fb.positions, self.cos_sin, kv.k[li], kv.v[li], fb.slots,
                         self.hq, self.hkv, kv.block_size)
-        q3 = q.view(T, self.hq, D)
-        if fb.is_decode:
-            part, splits = self.decode_part(T, fb.block_tables.shape[1] * kv.block_size)
-            ws = self._decode_ws(T, fb.block_tables.shape[1], kv.block_size, h.device, part,
-                                 splits)
-            o = ops.decode_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.seq_lens,
-                                     self.scale, part_size=part, workspace=ws, splits=splits)
-        elif fb.num_decode:
-            o = self._mixed_attention(li, q3, fb, kv)
-        else:
-            o = ops.prefill_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.q_start_loc,
-                                      fb.seq_lens, self.scale, fb.tile_seq, fb.tile_q0)
+        o = self._attend(li, q.view(T, self.hq, D), fb, kv)
         return self._proj("o", o.view(T, self.hq * D), self.w["layers"][li]["o"], fb.is_decode)
 
     def _mixed_attention(self, li: int, q3: torch.Tensor, fb: ForwardBatch, kv: KVCache):
@@ -377,6 +363,19 @@ class LlamaModel(Projections):
                 batch * self.hkv * ((max_ctx + 2 * part - 1) // (2 * part)) >= 2048:
             part *= 2
         return part, 0
+
+    def _attend(self, li: int, q3: torch.Tensor, fb: ForwardBatch, kv: KVCache):
+        """Attention of a step's rotated queries over the pages."""
+        if fb.is_decode:
+            T, mb = q3.shape[0], fb.block_tables.shape[1]
+            part, splits = self.decode_part(T, mb * kv.block_size)
+            ws = self._decode_ws(T, mb, kv.block_size, q3.device, part, splits)
+            return ops.decode_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.seq_lens,
+                                        self.scale, part_size=part, workspace=ws, splits=splits)
+        if fb.num_decode:
+            return self._mixed_attention(li, q3, fb, kv)
+        return ops.prefill_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.q_start_loc,
+                                     fb.seq_lens, self.scale, fb.tile_seq, fb.tile_q0)
 
     def _decode_ws(self, B, max_blocks, bs, device, part, splits=0):
         key = (B, max_blocks, bs, str(device), part, splits)
@@ -428,22 +427,58 @@ class LlamaModel(Projections):
                       positions=fb.positions, cos_sin=self.cos_sin, k_cache=kv.k[li],
                       v_cache=kv.v[li], slots=fb.slots, hq=self.hq, hkv=self.hkv,
                       block_size=kv.block_size)
-            if fb.num_decode:
-                o = self._mixed_attention(li, q.view(T, self.hq, D), fb, kv)
-            else:
-                o = ops.prefill_attention(q.view(T, self.hq, D), kv.k[li], kv.v[li],
-                                          fb.block_tables, fb.q_start_loc, fb.seq_lens,
-                                          self.scale, fb.tile_seq, fb.tile_q0)
+            o = self._attend(li, q.view(T, self.hq, D), fb, kv)
             ops.pgemm(2, o.view(T, self.hq * D), layer["o"], out=h, ss_out=ss_mid)
             ops.pgemm(1, h, layer["gate_up"], out=act, ss_in=ss_mid, inv_d=inv_d, eps=eps)
             ops.pgemm(2, act, layer["down"], out=h, ss_out=ss_out)
             ss = ss_out  # the next QKV reads it before the next down overwrites it
         return h
 
-    def hidden_states(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
+    # ------------------------------------------------ a few rows (stream.hip)
+    def _use_stream(self, fb: ForwardBatch) -> bool:
+        """Steps of a few rows run a layer as four projections and attention: norms, RoPE and
+        KV write, SwiGLU and residual ride in the projections' kernels."""
         cfg = self.cfg
+        if fb.cp is not None or not self.fold_post_norm or cfg.head_dim != 128:
+            return False
+        T, layer = fb.input_ids.shape[0], self.w["layers"][0]
+        return all(self._stream_weight(T, layer[k], k == "gate_up") is not None
+                   for k in ("qkv", "o", "gate_up", "down"))
+
+    def _stream_residual(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
+        """Residual stream after the last layer (un-normalised) of a step of a few rows."""
+        cfg = self.cfg
+        T = fb.input_ids.shape[0]
+        norm = dict(inv_d=1.0 / cfg.hidden_size, eps=cfg.rms_eps)
+        h = self.embed(fb.input_ids, fb.ids_src, fb.tok_slots)
+        ss = ops.row_sumsq(h).view(T, 1)
+        mid, end = (ops.stream_sums(T, self.w["layers"][0][k], h.device) for k in ("o", "down"))
+        for li, layer in enumerate(self.w["layers"]):
+            q = self._stream(3, h, layer["qkv"], ss=ss, positions=fb.positions, cos_sin=self.cos_sin,
+                             k_cache=kv.k[li], v_cache=kv.v[li], slots=fb.slots, hq=self.hq,
+                             hkv=self.hkv, **norm)
+            o = self._attend(li, q.view(T, self.hq, cfg.head_dim), fb, kv)
+            self._stream(2, o.view(T, -1), layer["o"], out=h, ss=mid)
+            a = self._stream(1, h, layer["gate_up"], ss=mid, **norm)
+            self._stream(2, a, layer["down"], out=h, ss=end)
+            ss = end
+        return h
+
+    def _residual(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor | None:
+        """The un-normalised residual of a step on one of the fused layer paths, else None."""
         if self._use_fused(fb):
-            return ops.rmsnorm(self._fused_residual(fb, kv), self.w["final_norm"], cfg.rms_eps)
+            return self._fused_residual(fb, kv)
+        return self._stream_residual(fb, kv) if self._use_stream(fb) else None
+
+    def hidden_states(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
+        r = self._residual(fb, kv)
+        if r is not None:
+            return ops.rmsnorm(r, self.w["final_norm"], self.cfg.rms_eps)
+        return self._hidden_rows(fb, kv)
+
+    def _hidden_rows(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
+        """Final-normed rows by the unfused layer path."""
+        cfg = self.cfg
         self._min_rows = self.PGEMM_MIXED_MIN_ROWS if fb.num_decode else self.PGEMM_MIN_ROWS
         residual = self.embed(fb.input_ids, fb.ids_src, fb.tok_slots)
         h = ops.rmsnorm(residual, self.w["layers"][0]["in_norm"], cfg.rms_eps)
@@ -464,19 +499,19 @@ class LlamaModel(Projections):
         when the measured table lists an unsplit (bf16-out) config for it."""
         W = self.w["lm_head"]
         cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
-        if cfg is not None and cfg[2] == 1:
+        lg = self._stream(0, h, W)
+        if lg is None and cfg is not None and cfg[2] == 1:
             lg = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
-        else:
+        elif lg is None:
             lg = ops.linear(h, W)
         return pstate.tp_all_gather_lastdim(lg) if (self.tp > 1 and gather) else lg
 
     def forward(self, fb: ForwardBatch, kv: KVCache, gather: bool = True) -> torch.Tensor:
-        if self._use_fused(fb):
-            h = self._fused_residual(fb, kv).index_select(0, fb.logits_indices)
-            return self.logits(ops.rmsnorm(h, self.w["final_norm"], self.cfg.rms_eps), gather,
-                               False)
-        h = self.hidden_states(fb, kv)
+        r = self._residual(fb, kv)
+        h = self._hidden_rows(fb, kv) if r is None else r
         # decode rows are their own logits rows (logits_indices is the identity)
-        sel = h if fb.is_decode and fb.logits_indices.shape[0] == h.shape[0] else \
-            h.index_select(0, fb.logits_indices)
-        return self.logits(sel, gather, fb.is_decode)
+        if not (fb.is_decode and fb.logits_indices.shape[0] == h.shape[0]):
+            h = h.index_select(0, fb.logits_indices)
+        if r is not None:
+            h = ops.rmsnorm(h, self.w["final_norm"], self.cfg.rms_eps)
+        return self.logits(h, gather, fb.is_decode)

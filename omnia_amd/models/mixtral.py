@@ -85,7 +85,9 @@ class MixtralModel(LlamaModel):
             return moe(h, tokens=self.ep_tokens)
         return ops.moe(h, layer["router"], layer["experts_gate_up"], layer["experts_down"],
                        self.cfg.experts_per_token, self.cfg.num_experts, self.e_lo,
-                       graph_safe=self.graph_safe or h.shape[0] < 64)
+                       graph_safe=self.graph_safe or h.shape[0] < 64,
+                       streams=self.expert_streams(layer["experts_gate_up"],
+                                                   layer["experts_down"]))
 
     def forward(self, fb, kv, gather: bool = True):
         # decode batches are captured into hipGraphs: keep the MoE path sync-free

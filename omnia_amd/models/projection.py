@@ -51,6 +51,59 @@ class Projections:
     # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
 
+    # ---- a few rows (ops.stream): one launch a projection, with what follows in it
+    # copies of the projections in the order that kernel streams best, made before the KV
+    # pool is sized, while they fit this part of HBM
+    stream_budget_frac = 0.06
+    STREAM_KEYS = {"qkv", "o", "gate_up", "down", "up", "in", "uq", "experts_gate_up",
+                   "experts_down"}
+
+    def pack_streams(self) -> int:
+        """Lay the projection weights out for :func:`ops.stream`; returns the bytes (0: off, or
+        over budget)."""
+        self._streams: dict = {}
+        if self.device.type != "cuda" or self.dtype != torch.bfloat16 or self.tp != 1:
+            return 0
+        found: dict = {}
+
+        def walk(v):
+            for k, t in v.items() if isinstance(v, dict) else enumerate(v):
+                if isinstance(t, (dict, list, tuple)):
+                    walk(t)
+                elif k in self.STREAM_KEYS and isinstance(t, torch.Tensor) and \
+                        ops.stream_ok(1, t, True, gated=t.dim() == 3 or k == "gate_up"):
+                    found[t.data_ptr()] = t
+
+        walk(self.w["layers"])
+        total = sum(t.numel() * t.element_size() for t in found.values())
+        cap = torch.cuda.get_device_properties(self.device).total_memory * self.stream_budget_frac
+        if total > cap:
+            return 0
+        self._streams = {p: ops.stream_pack(t) for p, t in found.items()}
+        return total
+
+    def _stream_weight(self, M: int, w: torch.Tensor, gated: bool = False):
+        """(weight, packed) to run ``M`` rows of a projection on the streaming kernel, or None
+        for the other paths."""
+        if self.device.type != "cuda" or self.dtype != torch.bfloat16 or self.tp != 1 or \
+                M > ops.STREAM_MAX_M:
+            return None
+        t = getattr(self, "_streams", {}).get(w.data_ptr())
+        if not ops.stream_ok(M, w, t is not None, gated):
+            return None
+        return (w, False) if t is None else (t, True)
+
+    def expert_streams(self, up: torch.Tensor, down: torch.Tensor):
+        """Packed copies of a layer's expert weights, or None."""
+        packs = getattr(self, "_streams", {})
+        t = packs.get(up.data_ptr()), packs.get(down.data_ptr())
+        return None if t[0] is None or t[1] is None else t
+
+    def _stream(self, epi: int, x: torch.Tensor, w: torch.Tensor, **kw):
+        """:func:`ops.stream` of one projection, or None."""
+        s = self._stream_weight(x.shape[0], w, epi == 1)
+        return None if s is None else ops.stream(epi, x, s[0], packed=s[1], **kw)
+
     # Projections return either a bf16 tensor (library / gemm.hip path, not yet
     # TP-reduced) or :class:`Parts` (fp32 split-K slabs of the weight-streaming
     # kernel, wgemm.hip), which the NEXT kernel reduces while doing its own work:
@@ -113,6 +166,9 @@ class Projections:
             return RowPar(x, w)
         if self._pgemm_ok(M, K, w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
+        y = self._stream(0, x, w)
+        if y is not None:
+            return y
         cfg = self._wcfg(M, w.shape[0], K, 0, is_decode)
         if cfg is None:
             return ops.linear(x, w)

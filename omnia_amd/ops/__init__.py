@@ -9,6 +9,7 @@ the mock/CPU engine path).
 from __future__ import annotations
 
 import contextlib
+import functools
 import importlib
 import os
 import threading
@@ -459,6 +460,94 @@ def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tenso
     return out
 
 
+# ------------------------------------------------------ projections of a few rows (stream.hip)
+STREAM_MAX_M = 32  # with packed weights
+STREAM_ROW_MAJOR_M = 16
+STREAM_HEAD_ROWS = 65536
+_stream_on = os.environ.get("OMNIA_STREAM", "1") != "0"
+
+
+def stream_rows(w: torch.Tensor, packed: bool) -> int:
+    """Most rows ``x`` may have for :func:`stream` to be the better kernel for ``w``.
+
+    Its blocks each read all of x, so rows cost: in us at 1 / 16 / 32 rows, with the kernel
+    that takes over in brackets, 28672 x 4096 packed 38 / 42 / 47 (52 / 53 / 54), row-major
+    41 / 50 / 59; 4096 x 4096 packed 7.0 / 8.5 / 11.5 (15 / 15 / 13), row-major 8.7 / 10.8 /
+    13.7; 2048 x 2048 row-major 5.0 / 6.7 / 8.1 (11).  A row-major head of 128256 x 4096 takes
+    168 at 1 row, 188 at 8 and 205 at 16 (188 / 189 / 191)."""
+    if packed:
+        return STREAM_MAX_M
+    return 8 if w.shape[0] >= STREAM_HEAD_ROWS else STREAM_ROW_MAJOR_M
+
+
+def stream_ok(M: int, w: torch.Tensor, packed: bool, gated: bool = False) -> bool:
+    """Whether :func:`stream` covers, and is chosen for, ``M`` rows and this GPU weight."""
+    R, K = w.shape[-2:]
+    return (_stream_on and w.is_cuda and 1 <= M <= stream_rows(w, packed)
+            and w.dtype == torch.bfloat16
+            and K % 64 == 0 and R % (32 if gated else 16) == 0 and w.is_contiguous())
+
+
+@functools.lru_cache(maxsize=4096)
+def stream_fragments(M: int, rows: int) -> int:
+    """16-row weight fragments of a block (1, 2, 4).  More of them share the block's reads of x,
+    which cost about 0.3 of the weights' per 16 rows of x and fragment; fewer spread better
+    over 256 CUs as long as there are few blocks (4096 rows, one / two fragments: 7.0 / 7.7 us
+    at K = 4096; 6144 rows: 10.2 / 9.6, 384 blocks leaving half the CUs with twice the work)."""
+    best, cost = 1, float("inf")
+    for nw in (1, 2, 4):
+        if rows % (16 * nw):
+            break
+        rounds = rows / (16 * nw * 256)
+        c = (rounds if rounds > 1.6 else -(-rounds // 1)) * nw * (1.0 + 0.3 * M / 16 / nw)
+        if c < cost - 1e-9:
+            best, cost = nw, c
+    return best
+
+
+def stream_pack(w: torch.Tensor) -> torch.Tensor:
+    """``w`` [..., R, K] re-laid for :func:`stream` as [R / 16][K / 64][2][4][16][8] (k step, k
+    group, row, k), so that a wave reads one contiguous KB; returned with the shape of ``w``."""
+    R, K = w.shape[-2:]
+    if R % 16 or K % 64:
+        raise ValueError("stream_pack: whole 16-row, 64-column blocks")
+    t = w.reshape(-1, R // 16, 16, K // 64, 2, 4, 8).permute(0, 1, 3, 4, 5, 2, 6)
+    return t.contiguous().view(w.shape)
+
+
+def stream_sums(M: int, w: torch.Tensor, device) -> torch.Tensor:
+    """The ``ss`` an epi 2 :func:`stream` of ``M`` rows writes."""
+    return torch.empty(M, w.shape[0] // (16 * stream_fragments(M, w.shape[0])),
+                       dtype=torch.float32, device=device)
+
+
+def stream(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
+           packed: bool = False, ss: torch.Tensor | None = None, inv_d: float = 0.0,
+           eps: float = 0.0, bias=None, gelu: bool = False, positions=None, cos_sin=None,
+           k_cache=None, v_cache=None, slots=None, hq: int = 0, hkv: int = 0) -> torch.Tensor:
+    """``x @ w.T`` of up to 32 rows with a fused epilogue (``csrc/stream.hip``), GPU only.
+
+    ``ss`` (fp32 [M, n] partial sums of squares of the rows of ``x``) norms the rows first:
+    ``x * rsqrt(sum(ss) * inv_d + eps)`` in bf16, an RMSNorm whose weight is folded into ``w``.
+    epi 0: plain (+ ``bias``); 1: ``act(g + b) * (u + b)`` with ``w = [Wg; Wu]``, silu or, with
+    ``gelu``, its tanh form; 2: ``out`` is the residual, updated in place, and ``ss``
+    (:func:`stream_sums`) receives its rows' sums of squares; 3: QKV, as :func:`pgemm`'s.
+    ``packed``: ``w`` is from :func:`stream_pack`."""
+    M = x.shape[0]
+    N = w.shape[0] // 2 if epi == 1 else w.shape[0]
+    if out is None:
+        out = x.new_empty(M, hq * 128 if epi == 3 else N)
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < x.shape[1] or x.data_ptr() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+    if epi == 3 and checks.active(x):
+        checks.slots("stream qkv", slots, k_cache)
+    ss_in, ss_out = (None, ss) if epi == 2 else (ss, None)
+    kernels().stream_gemm(epi, out, x, w, stream_fragments(M, w.shape[0]), packed, ss_in, inv_d,
+                          eps, ss_out, bias, gelu, positions, cos_sin, k_cache, v_cache, slots,
+                          hq, hkv)
+    return out
+
+
 def row_sumsq(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """fp32 [M] sums of squares of the rows of a bf16 [M, d] matrix."""
     if out is None:
@@ -763,16 +852,35 @@ MOE_LIBRARY_ROWS = 1024  # mean rows/expert above which eager calls use hipBLASL
 MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
 
 
+def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
+                  packed: bool) -> bool:
+    """Whether ``n`` assignments to ``experts`` local experts run on the streaming kernel, in
+    16-row segments (a fuller expert's weights are read once per segment).
+
+    Both products, us at 1 / 4 / 8 / 16 / 32 / 64 tokens of 2 experts in 8, 2048 x 4096: 64-row
+    kernel 52 / 90 / 82 / 93 / 93 / 93, packed 25 / 63 / 58 / 72 / 74 / 95; 4096 x 14336: 193 /
+    383 / 470 / 472 / 475 / 477 and 111 / 315 / 418 / 419 / 431 / 602.  Row-major weights gain
+    only where most experts have no row: 29 for 52 and 133 for 193 at 1 token."""
+    return (_stream_on and w_up.dtype == torch.bfloat16 and w_up.is_cuda
+            and n <= (8 * experts if packed else (experts - 1) // 2)
+            and all(w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down)))
+
+
 def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=None,
-                 gelu: bool = False):
+                 gelu: bool = False, streams=None):
     """Grouped expert FFN over device-sorted assignments, no host sync: Y [T*k, d]
     (row t*k + j = slot j of token t, routing weight applied; other experts' rows
     unwritten).  ``bm`` 256: the 256x256 MFMA prefill tile; 64: moe.hip.  ``glu`` =
     (alpha, limit): clamped GLU experts whose INPUT takes the routing weight; ``gelu``:
-    ungated experts (``w_gu`` [E, I, d])."""
+    ungated experts (``w_gu`` [E, I, d]).  ``streams``: packed copies (:func:`stream_pack`) of
+    both weights, or None; few assignments run :func:`moe_stream_ok`'s kernel in place of
+    ``bm`` 64."""
     kk = kernels()
-    n = ids.numel()
-    mb = kk.moe_max_blocks(n, e_hi - e_lo, bm)
+    n, experts = ids.numel(), e_hi - e_lo
+    few = bm == 64 and moe_stream_ok(n, experts, w_gu, w_down, streams is not None)
+    if few:
+        bm = 16
+    mb = kk.moe_max_blocks(n, experts, bm)
     sorted_ids = torch.empty(mb * bm, dtype=torch.int32, device=x.device)
     blk = torch.empty(mb, dtype=torch.int32, device=x.device)
     nblk = torch.empty(1, dtype=torch.int32, device=x.device)
@@ -780,6 +888,16 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     act = torch.empty(mb * bm, w_down.shape[2], dtype=x.dtype, device=x.device)
     Y = torch.empty(n, x.shape[1], dtype=x.dtype, device=x.device)
     gemm = kk.pgemm_moe if bm == 256 else kk.moe_gemm
+    if few:
+        live = min(n, experts)  # experts whose weights are read, at most
+
+        def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
+            frags = min(2, stream_fragments(min(n, 16), w.shape[1] * live))
+            if streams is not None:
+                w = streams[mode == 1]
+            kk.stream_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, frags, streams is not None,
+                          alpha, limit)
+
     if glu is not None:
         gemm(2, act, x, w_gu, sorted_ids, blk, nblk, wts.view(-1), k, n, e_lo, *glu)
         gemm(1, Y, act, w_down, sorted_ids, blk, nblk, None, k, n, e_lo)
@@ -824,14 +942,15 @@ def moe_rows(rows: torch.Tensor, eids: torch.Tensor, w_gu: torch.Tensor, w_down:
 
 def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor,
         k: int, n_experts: int, e_lo: int = 0, renorm: bool = True,
-        graph_safe: bool = True) -> torch.Tensor:
+        graph_safe: bool = True, streams=None) -> torch.Tensor:
     """Top-k MoE FFN over the local experts ``[e_lo, e_lo + w_gu.shape[0])``.
 
     x [T, d] bf16, router [E, d], w_gu [E_loc, 2I, d] (gate ; up), w_down [E_loc, d, I].
     Returns the local experts' weighted contribution [T, d] (all-reduce over the
     EP group to complete it).  ``graph_safe`` keeps every shape static and the
     whole path on device (hipGraph decode); otherwise large batches run each
-    expert's GEMMs on hipBLASLt after one host sync on the expert counts."""
+    expert's GEMMs on hipBLASLt after one host sync on the expert counts.  ``streams``:
+    :func:`stream_pack` copies of both expert weights."""
     e_hi = e_lo + w_gu.shape[0]
     if not x.is_cuda:
         return ref.moe(x, router, w_gu, w_down, k, e_lo, renorm).to(x.dtype)
@@ -871,6 +990,6 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
         Y.index_copy_(0, order, ys * wts.view(-1).index_select(0, order)[:, None].to(x.dtype))
         kk.moe_combine(out, Y, ids, k, e_lo, e_hi)
         return out
-    Y = _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, 64)
+    Y = _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, 64, streams=streams)
     kk.moe_combine(out, Y, ids, k, e_lo, e_hi)
     return out

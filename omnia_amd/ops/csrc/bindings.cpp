@@ -120,6 +120,15 @@ int omnia_wgemm(int mode, void* out, const void* X, const void* W, int M, int N,
                 int nw, int nwaves, int ldo, hipStream_t s);
 int omnia_wgemm_wide(int mode, void* out, const void* X, const void* W, int M, int N, int K,
                      int S, int wt, int ldo, hipStream_t s);
+int omnia_stream(int epi, void* out, const void* x, const void* w, int M, int N, int K,
+                 int64_t ldx, int64_t ldo, int nw, int packed, const float* ss_in, int n_ss,
+                 float inv_d, float eps, float* ss_out, const float* bias, int gelu, const int* positions, const float* cos_sin,
+                 void* k_cache, void* v_cache, const int64_t* slots, int hq, int hkv, int page,
+                 hipStream_t s);
+int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
+                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
+                     int N, int topk, int n_assign, int e_lo, int max_blocks, int nw, int packed,
+                     float alpha, float limit, hipStream_t s);
 int omnia_dgemm(int mode, void* out, const void* X, const void* W, float* ws, int* cnt, int M,
                 int N, int K, int S, int wm, int wn, int ldo, int64_t ws_floats, int cnt_len,
                 hipStream_t s);
@@ -630,16 +639,16 @@ int64_t moe_max_blocks(int64_t n_assign, int64_t n_experts, int64_t bm) {
   return omnia_moe_max_blocks(n_assign, n_experts, bm);
 }
 
-// segments aligned to bm = sorted.numel() / blk_expert.numel() rows (64: moe_gemm,
-// 256: the pgemm_moe prefill tile)
+// segments aligned to bm = sorted.numel() / blk_expert.numel() rows (16: stream_moe,
+// 64: moe_gemm, 256: the pgemm_moe prefill tile)
 void moe_align(at::Tensor sorted, at::Tensor blk_expert, at::Tensor n_blocks, at::Tensor ids,
                int64_t E, int64_t e_lo, int64_t e_hi) {
   CHECK_GPU(ids); CHECK_I32(ids); CHECK_I32(sorted); CHECK_I32(blk_expert); CHECK_I32(n_blocks);
   const int n = ids.numel();
   const int mb = blk_expert.numel();
-  TORCH_CHECK(mb > 0 && (sorted.numel() == (int64_t)mb * 64 || sorted.numel() == (int64_t)mb * 256),
-              "sorted must hold max_blocks*64 (or *256) rows");
+  TORCH_CHECK(mb > 0 && sorted.numel() % mb == 0, "sorted must hold max_blocks segments");
   const int bm = (int)(sorted.numel() / mb);
+  TORCH_CHECK(bm == 16 || bm == 64 || bm == 256, "segments of 16, 64 or 256 rows");
   TORCH_CHECK(mb >= omnia_moe_max_blocks(n, e_hi - e_lo, bm), "blk_expert too small");
   TORCH_CHECK(E <= 256 && 0 <= e_lo && e_lo < e_hi && e_hi <= E, "expert range");
   CHECK_RC(omnia_moe_align(sorted.data_ptr<int>(), blk_expert.data_ptr<int>(),
@@ -741,6 +750,46 @@ void moe_gemm(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tens
                           n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N, topk,
                           n_assign, e_lo, mb, (float)alpha, (float)limit, cur_stream()),
            "moe_gemm");
+}
+
+// moe_gemm's modes for segments of 16 rows (stream.hip)
+void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
+                at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
+                int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
+                double alpha, double limit) {
+  CHECK_GPU(A); CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(out);
+  CHECK_I32(sorted); CHECK_I32(blk_expert); CHECK_I32(n_blocks);
+  TORCH_CHECK(mode >= 0 && mode <= 3, "mode");
+  TORCH_CHECK(A.is_contiguous() && W.is_contiguous() && out.is_contiguous(), "contiguous");
+  TORCH_CHECK(A.dim() == 2 && out.dim() == 2 && W.dim() == 3, "W [E_local, rows, K]");
+  for (const at::Tensor* t : {&W, &out, &sorted, &blk_expert, &n_blocks})
+    TORCH_CHECK(t->device() == A.device(), "same device");
+  const int K = W.size(2);
+  const int mb = blk_expert.numel();
+  constexpr int seg = 16;
+  TORCH_CHECK(sorted.numel() == (int64_t)mb * seg, "sorted must hold max_blocks*16 rows");
+  TORCH_CHECK(A.size(1) == K, "K mismatch");
+  if (route_w.has_value())
+    TORCH_CHECK(route_w->device() == A.device() && route_w->is_contiguous() &&
+                route_w->numel() == n_assign && route_w->scalar_type() == at::kFloat,
+                "route weights fp32 [T*k]");
+  int N;
+  if (mode != 1) {
+    TORCH_CHECK(mode == 3 || W.size(1) % 2 == 0, "gate_up rows even");
+    N = mode == 3 ? W.size(1) : W.size(1) / 2;
+    TORCH_CHECK(out.size(0) == (int64_t)mb * seg && out.size(1) == N, "act [max_blocks*seg, I]");
+    TORCH_CHECK(A.size(0) * topk == n_assign, "x rows * topk == n_assign");
+  } else {
+    N = W.size(1);
+    TORCH_CHECK(out.size(0) == n_assign && out.size(1) == N, "Y [T*k, d]");
+    TORCH_CHECK(A.size(0) == (int64_t)mb * seg, "act rows");
+  }
+  CHECK_RC(omnia_stream_moe((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(),
+                            sorted.data_ptr<int>(), blk_expert.data_ptr<int>(),
+                            n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N, topk,
+                            n_assign, e_lo, mb, (int)nw, packed, (float)alpha, (float)limit,
+                            cur_stream()),
+           "stream_moe");
 }
 
 void moe_combine(at::Tensor out, at::Tensor Y, at::Tensor ids, int64_t topk, int64_t e_lo,
@@ -939,6 +988,82 @@ void pgemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W,
                        out.stride(0), ssi, ssn, (float)inv_d, (float)eps, sso, pos, cs, kc, vc, sl,
                        (int)hq, (int)hkv, (int)block_size, bp, gelu, cur_stream()),
            "pgemm");
+}
+
+// projection of up to 32 rows (stream.hip); x rows may be strided
+void stream_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t nw, bool packed,
+                 c10::optional<at::Tensor> ss_in, double inv_d, double eps,
+                 c10::optional<at::Tensor> ss_out, c10::optional<at::Tensor> bias, bool gelu,
+                 c10::optional<at::Tensor> positions, c10::optional<at::Tensor> cos_sin,
+                 c10::optional<at::Tensor> k_cache, c10::optional<at::Tensor> v_cache,
+                 c10::optional<at::Tensor> slots, int64_t hq, int64_t hkv) {
+  CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W); CHECK_BF16(out);
+  TORCH_CHECK(epi >= 0 && epi <= 3, "epi");
+  TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && out.dim() == 2, "2-D operands");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1 && W.is_contiguous(), "contiguous rows, W");
+  TORCH_CHECK(x.device() == W.device() && x.device() == out.device(), "same device");
+  const int M = x.size(0), K = x.size(1);
+  TORCH_CHECK(W.size(1) == K, "K mismatch");
+  TORCH_CHECK(epi != 1 || W.size(0) % 2 == 0, "gate_up rows even");
+  const int N = epi == 1 ? W.size(0) / 2 : W.size(0);
+  TORCH_CHECK(out.size(0) == M && out.size(1) == (epi == 3 ? hq * 128 : N),
+              "out [M, N] (q [M, hq*128] for epi 3)");
+  const float* ssi = nullptr;
+  float* sso = nullptr;
+  int n_ss = 0;
+  if (ss_in.has_value() && ss_in->defined()) {
+    TORCH_CHECK(ss_in->scalar_type() == at::kFloat && ss_in->is_contiguous() &&
+                ss_in->dim() == 2 && ss_in->size(0) == M && ss_in->device() == x.device(),
+                "ss_in fp32 [M, n]");
+    ssi = ss_in->data_ptr<float>();
+    n_ss = ss_in->size(1);
+  }
+  if (epi == 2) {
+    TORCH_CHECK(ss_out.has_value() && ss_out->scalar_type() == at::kFloat &&
+                ss_out->is_contiguous() && ss_out->dim() == 2 && ss_out->size(0) == M &&
+                nw > 0 && ss_out->size(1) == N / (16 * nw) && ss_out->device() == x.device(),
+                "ss_out fp32 [M, N / (16 nw)]");
+    sso = ss_out->data_ptr<float>();
+  }
+  const float* bp = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(epi <= 1 && bias->device() == x.device() && bias->scalar_type() == at::kFloat &&
+                bias->is_contiguous() && bias->numel() == (epi == 1 ? 2 : 1) * N, "bias fp32");
+    bp = bias->data_ptr<float>();
+  }
+  const int* pos = nullptr;
+  const float* cs = nullptr;
+  void *kc = nullptr, *vc = nullptr;
+  const int64_t* sl = nullptr;
+  int page = 0;
+  if (epi == 3) {
+    TORCH_CHECK(positions.has_value() && cos_sin.has_value() && k_cache.has_value() &&
+                v_cache.has_value() && slots.has_value(), "epi 3 needs rope / cache operands");
+    TORCH_CHECK(positions->scalar_type() == at::kInt && positions->numel() == M &&
+                positions->is_contiguous(), "positions int32 [M]");
+    TORCH_CHECK(cos_sin->scalar_type() == at::kFloat && cos_sin->is_contiguous() &&
+                cos_sin->dim() == 2 && cos_sin->size(1) == 128, "cos_sin f32 [P, 128]");
+    TORCH_CHECK(slots->scalar_type() == at::kLong && slots->numel() == M && slots->is_contiguous(),
+                "slots int64 [M]");
+    CHECK_BF16(*k_cache); CHECK_BF16(*v_cache);
+    TORCH_CHECK(k_cache->dim() == 4 && k_cache->size(1) == hkv && k_cache->size(3) == 128 &&
+                k_cache->is_contiguous() && v_cache->is_contiguous() &&
+                v_cache->sizes() == k_cache->sizes(), "cache layout [NB, Hkv, BS, 128]");
+    for (const at::Tensor* t : {&*positions, &*cos_sin, &*k_cache, &*v_cache, &*slots})
+      TORCH_CHECK(t->device() == x.device(), "same device");
+    pos = positions->data_ptr<int>();
+    cs = cos_sin->data_ptr<float>();
+    kc = k_cache->data_ptr();
+    vc = v_cache->data_ptr();
+    sl = slots->data_ptr<int64_t>();
+    page = k_cache->size(2);
+  }
+  if (M == 0) return;
+  CHECK_RC(omnia_stream((int)epi, out.data_ptr(), x.data_ptr(), W.data_ptr(), M, N, K,
+                        x.stride(0), out.stride(0), (int)nw, packed, ssi, n_ss, (float)inv_d,
+                        (float)eps, sso, bp, gelu, pos, cs, kc, vc, sl, (int)hq, (int)hkv, page,
+                        cur_stream()),
+           "stream_gemm");
 }
 
 void pgemm_variant(int64_t variant, at::Tensor out, at::Tensor x, at::Tensor W) {
@@ -1971,6 +2096,8 @@ PYBIND11_MODULE(_omnia_kernels, m) {
         py::arg("limit") = 0.0);
   m.def("moe_combine", &moe_combine);
   m.def("dgemm", &dgemm);
+  m.def("stream_gemm", &stream_gemm);
+  m.def("stream_moe", &stream_moe);
   m.def("wgemm", &wgemm);
   m.def("wgemm_wide", &wgemm_wide);
   m.def("tgemm", &tgemm);

@@ -342,8 +342,8 @@ __global__ __launch_bounds__(256) void moe_route_f32_kernel(const float* __restr
 // ------------------------------------------------------------------ align
 // One 1024-thread workgroup.  n = T*k assignments.  sorted has max_blocks*BM
 // entries (n = padding sentinel), blk_expert max_blocks entries.
-// bm: the segment alignment = the grouped GEMM's row tile (64 here, 256 for the
-// 256x256 prefill tile of pgemm.hip EPI 5 / 6)
+// bm: the segment alignment = the grouped GEMM's row tile (64 here, 16 for a few rows
+// an expert, stream.hip, 256 for the 256x256 prefill tile of pgemm.hip EPI 5 / 6)
 __global__ __launch_bounds__(1024) void moe_align_kernel(int* __restrict__ sorted,
                                                          int* __restrict__ blk_expert,
                                                          int* __restrict__ n_blocks,
@@ -666,7 +666,7 @@ int omnia_moe_max_blocks(int n_assign, int n_experts, int bm) {
 int omnia_moe_align(int* sorted, int* blk_expert, int* n_blocks, const int* ids, int n, int E,
                     int e_lo, int e_hi, int max_blocks, int bm, hipStream_t s) {
   if (E > 256 || e_lo < 0 || e_hi > E || e_lo >= e_hi) return -1;
-  if (bm != 64 && bm != 256) return -2;
+  if (bm != 16 && bm != 64 && bm != 256) return -2;
   moe_align_kernel<<<1, 1024, 0, s>>>(sorted, blk_expert, n_blocks, ids, n, E, e_lo, e_hi,
                                       max_blocks, bm);
   return (int)hipGetLastError();

@@ -1,0 +1,187 @@
+"""Streaming projections of a few rows (``csrc/stream.hip``) against float64."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+from omnia_amd import ops
+from omnia_amd.ops import reference as ref
+
+U = 2.0 ** -8  # half an ulp of a bf16 result, relative
+
+
+def _mk(M, R, K, seed, lead=()):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(*lead, R, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    return x, w
+
+
+def _close(got, want, K, rounded=1):
+    """fp32 sums of K bf16 products of about 1 / sqrt(K) each, then ``rounded`` bf16 roundings."""
+    err = (got.double() - want).abs()
+    bound = rounded * U * want.abs() + 4 * K * 2.0 ** -24 * want.abs().clamp(min=1.0)
+    assert (err <= bound).all(), float((err - bound).max())
+
+
+def _weight(w, packed):
+    return ops.stream_pack(w) if packed else w
+
+
+def _normed(x, n=1):
+    """Partial sums of squares of the rows, and the rows as a norm kernel leaves them."""
+    ss = x.float().pow(2).view(x.shape[0], n, -1).sum(2).contiguous()
+    inv = torch.rsqrt(ss.sum(1, keepdim=True) / x.shape[1] + 1e-5)
+    return ss, (x.float() * inv).to(torch.bfloat16)
+
+
+def _close_normed(got, x, w, K, f=lambda h: h):
+    """A row's factor is good to an ulp of fp32, which may turn the bf16 rounding of an x here
+    and there: half an ulp each, in random directions."""
+    want = f(x.double() @ w.double().T)
+    err = (got.double() - want).abs()
+    bound = 2 * U * want.abs() + 16 * U * (x.double().abs().amax() * w.double().abs().amax()) + 1e-5
+    assert (err <= bound).all(), float((err - bound).max())
+    assert err.norm() <= 1.2 * U * want.norm()
+
+
+# rows around the 16-row fragments; K of one chunk, fewer chunks than waves, an odd number
+SIZES = [(1, 16, 64), (15, 48, 192), (16, 4096, 576), (17, 96, 1024), (31, 64, 4160), (32, 512, 640)]
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_plain_norm_and_residual(M, N, K, packed):
+    x, w = _mk(M, N, K, M + N + K)
+    want = x.double() @ w.double().T
+    wk, bias = _weight(w, packed), torch.randn(N, device="cuda")
+    _close(ops.stream(0, x, wk, packed=packed, bias=bias), want + bias.double(), K)
+    for n in (1, K // 64, K):  # one partial sum a row, some, more than 4 a lane
+        ss, xn = _normed(x, n)
+        got = ops.stream(0, x, wk, packed=packed, ss=ss, inv_d=1.0 / K, eps=1e-5)
+        _close_normed(got, xn, w, K)
+    res = torch.randn(M, N, device="cuda").to(torch.bfloat16)
+    old = res.clone()
+    ss = ops.stream_sums(M, w, "cuda")
+    out = ops.stream(2, x, wk, packed=packed, out=res, ss=ss)
+    assert out is res
+    # the projection in bf16 (a sum at the edge of a rounding may turn it by an ulp), then theirs
+    both = want.float().to(torch.bfloat16).double() + old.double()
+    err = (res.double() - both).abs()
+    assert (err <= U * both.abs() + 2 * U * want.abs() + 1e-6).all()
+    assert (err > U * both.abs()).sum() <= 2 + 0.01 * err.numel()
+    torch.testing.assert_close(ss.sum(1), res.float().pow(2).sum(1), rtol=1e-5, atol=1e-5)
+    # strided rows (columns of a wider matrix), and rows off the 16-byte grid
+    wide = torch.randn(M, K + 72, device="cuda").to(torch.bfloat16)
+    for off in (8, 3):
+        v = wide[:, off:off + K]
+        _close(ops.stream(0, v, wk, packed=packed), v.double() @ w.double().T, K)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_gated(M, N, K, gelu, packed):
+    x, w = _mk(M, 2 * N, K, M * N)
+    wk, b = _weight(w, packed), torch.randn(2 * N, device="cuda")
+    h = x.double() @ w.double().T
+
+    def act(v, u):
+        return (F.gelu(v, approximate="tanh") if gelu else F.silu(v)) * u
+
+    # v_exp_f32 and v_rcp_f32 are good to a few ulp of fp32: below the bf16 rounding
+    hb = h + b.double()
+    _close(ops.stream(1, x, wk, packed=packed, bias=b, gelu=gelu), act(*hb.chunk(2, 1)), 4 * K, 1.1)
+    ss, xn = _normed(x)
+    got = ops.stream(1, x, wk, packed=packed, gelu=gelu, ss=ss, inv_d=1.0 / K, eps=1e-5)
+    _close_normed(got, xn, w, K, lambda h: act(*h.chunk(2, 1)))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M,hq,hkv,K", [(1, 1, 1, 64), (5, 32, 8, 512), (16, 4, 2, 4096),
+                                        (32, 8, 1, 192), (25, 7, 1, 1024)])
+def test_qkv(M, hq, hkv, K, packed):
+    x, w = _mk(M, (hq + 2 * hkv) * 128, K, M + hq)
+    page, nb = 16, 6
+    cache = torch.zeros(2, nb, hkv, page, 128, device="cuda", dtype=torch.bfloat16)
+    slots = torch.randperm(nb * page, device="cuda")[:M].contiguous()
+    if M > 2:
+        slots[1] = -1
+    pos = torch.randint(0, 500, (M,), device="cuda", dtype=torch.int32)
+    cs = ref.rope_cos_sin(512, 128, 10000.0, device="cuda")
+    q = ops.stream(3, x, _weight(w, packed), packed=packed, positions=pos, cos_sin=cs,
+                   k_cache=cache[0], v_cache=cache[1], slots=slots, hq=hq, hkv=hkv)
+    h = (x.double() @ w.double().T).view(M, -1, 128)
+    c, s = (t.double()[:, None] for t in cs[pos.long()].chunk(2, 1))
+    a, b = h[..., :64], h[..., 64:]
+    r = torch.cat([a * c - b * s, b * c + a * s], -1)
+    lim = 2 * U * h.abs().amax()  # the projection's rounding, turned, and the result's
+    assert (q.view(M, hq, 128).double() - r[:, :hq]).abs().max() <= lim
+    want = torch.zeros_like(cache, dtype=torch.float64)
+    for m, at in enumerate(slots.tolist()):
+        if at >= 0:
+            want[0, at // page, :, at % page] = r[m, hq:hq + hkv]
+            want[1, at // page, :, at % page] = h[m, hq + hkv:]
+    assert (cache.double() - want).abs().max() <= lim
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("glu,gelu", [(None, False), ((1.702, 7.0), False), (None, True)])
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (5, 8, 2), (32, 8, 2), (3, 33, 1), (7, 4, 4)])
+def test_experts_match_the_64_row_kernels(T, E, k, glu, gelu, packed, monkeypatch):
+    """Segments of 16 rows, some experts without a row and some with two segments (every row
+    to expert 1): the same products as moe.hip's, summed in another order."""
+    d, ff = 192, 320
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    _, up = _mk(1, ff if gelu else 2 * ff, d, 3, (E,))
+    _, down = _mk(1, d, ff, 4, (E,))
+    x = torch.randn(T, d, generator=g, device="cuda").to(torch.bfloat16)
+    ids = torch.stack([torch.randperm(E, generator=g, device="cuda")[:k] for _ in range(T)]).int()
+    if T == 32:
+        ids[:, 0], ids[:, 1] = 1, 2
+    wts = torch.rand(T, k, generator=g, device="cuda")
+    args = (x, up, down, ids.contiguous(), wts, k, E, 0, E, 64, glu, gelu)
+    monkeypatch.setattr(ops, "moe_stream_ok", lambda *a: False)
+    want = ops._moe_grouped(*args).double()
+    monkeypatch.setattr(ops, "moe_stream_ok", lambda *a: True)
+    streams = (ops.stream_pack(up), ops.stream_pack(down)) if packed else None
+    got = ops._moe_grouped(*args, streams=streams).double()
+    # the activations may round apart by an ulp, and so may the results
+    assert (got - want).norm() <= 2 * U * want.norm()
+    assert ((got - want).abs() <= 4 * U * want.abs().clamp(min=want.pow(2).mean().sqrt())).all()
+
+
+def test_what_is_refused():
+    x, w = _mk(33, 64, 128, 1)
+    with pytest.raises(RuntimeError):
+        ops.stream(0, x, w)  # rows
+    with pytest.raises(RuntimeError):
+        ops.stream(0, x[:4, :96].contiguous(), w[:, :96].contiguous())  # whole 64-k chunks
+    with pytest.raises(RuntimeError):
+        ops.stream(0, x[:4], w[:40].contiguous())  # whole 16-row fragments
+    assert not ops.stream_ok(4, w[:40], False) and not ops.stream_ok(33, w, True)
+
+
+@pytest.mark.parametrize("rows,pack", [(1, True), (16, False), (23, True)])
+def test_llama_layers_match_the_unfused_path(rows, pack, monkeypatch):
+    """Decode steps of a small model: the four streamed projections a layer against separate
+    norm, RoPE, SwiGLU and residual kernels."""
+    from omnia_amd.engine.engine import EngineConfig, LLMEngine
+    from omnia_amd.engine.sampling_params import SamplingParams
+
+    def run(on):
+        monkeypatch.setattr(ops, "_stream_on", on)
+        eng = LLMEngine(EngineConfig(model="tiny-llama", max_batch=32, max_model_len=256, seed=4))
+        if not pack:
+            eng.model._streams = {}
+        eng.runner.enable_logit_tap()
+        p = SamplingParams(temperature=0.0, max_tokens=4, ignore_eos=True)
+        for i in range(rows):
+            eng.add_request([(7 * i + j) % 250 for j in range(5 + i % 3)], p)
+        eng.run_until_done()
+        return {s: r for ids, t in eng.runner.logit_tap[:1] for s, r in zip(ids, t)}
+
+    a, b = run(True), run(False)
+    for x, y in zip(a.values(), b.values()):
+        assert (x - y).norm() <= 0.02 * y.norm()
