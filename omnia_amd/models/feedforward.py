@@ -53,9 +53,9 @@ class DenseGLU:
         if m._pgemm_ok(M, K, N // 2, is_decode, 128) and (b is None or act == "silu"):
             return ops.pgemm(1, h, W, bias=b, gelu=act == "gelu_tanh")
         copy = w.get("gate_up_stream")
-        if ops.stream_ok(M, W, copy is not None, gated=True):
-            return ops.stream(1, h, W if copy is None else copy, packed=copy is not None, bias=b,
-                              gelu=act == "gelu_tanh")
+        if ops.stream_ok(M, W, gated=True):
+            return ops.few_rows(1, h, W if copy is None else copy, copy is not None, bias=b,
+                                gelu=act == "gelu_tanh")
         cfg = m._wcfg(M, N // 2, K, 1, is_decode)
         if cfg is not None:  # a tuned SwiGLU shape, as slabs (bias and activation follow)
             nw, nwaves, S = cfg

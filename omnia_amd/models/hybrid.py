@@ -229,7 +229,7 @@ class HybridModel(Projections):
         """A projection whose consumer reads plain rows (no split-K slabs)."""
         if self._pgemm_ok(x.shape[0], x.shape[1], w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
-        y = self._stream(0, x, w)
+        y = self._few(0, x, w)
         return ops.linear(x, w) if y is None else y
 
     def _slabs(self, tag, x, w, is_decode) -> torch.Tensor:
@@ -316,11 +316,11 @@ class HybridModel(Projections):
     def logits(self, h: torch.Tensor, is_decode: bool = False) -> torch.Tensor:
         W = self.w["head"]
         cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
-        z = self._stream(0, h, W)
-        if z is None and cfg is not None and cfg[2] == 1:
+        if cfg is not None and cfg[2] == 1:
             z = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
-        elif z is None:
-            z = ops.linear(h, W)
+        else:
+            z = self._few(0, h, W)
+            z = ops.linear(h, W) if z is None else z
         cap = self.cfg.logit_softcap
         return mops.softcap_(z, cap) if cap else z
 

@@ -275,7 +275,9 @@ class LlamaModel(Projections):
             return self._proj("down", ops.pgemm(1, h, layer["gate_up"]), layer["down"], False)
         cfg = self._wcfg(M, I2 // 2, K, 1, is_decode)
         if cfg is None:
-            a = ops.linear_silu(h, layer["gate_up"])  # SwiGLU fused into decode GEMMs
+            a = self._few(1, h, layer["gate_up"])
+            if a is None:
+                a = ops.linear_silu(h, layer["gate_up"])  # SwiGLU fused into decode GEMMs
         elif cfg[1] == ops.PGEMM_SPLIT and cfg[2] == 1:
             a = ops.pgemm(1, h, layer["gate_up"])  # mid-size step: the unsplit fused tile
         else:
@@ -301,7 +303,7 @@ class LlamaModel(Projections):
                           hkv=self.hkv, block_size=kv.block_size)
             o = self._attend(li, q.view(T, self.hq, D), fb, kv)
             return self._proj("o", o.view(T, self.hq * D), self.w["layers"][li]["o"], False)
-        qkv = self._proj("qkv", h, wqkv, fb.is_decode)
+        qkv = self._proj("qkv", h, wqkv, fb.is_decode, slabs=fb.cp is None)
         if fb.cp is not None:
             cp = fb.cp
             q = qkv[:, : self.hq * D]
@@ -442,7 +444,7 @@ class LlamaModel(Projections):
         if fb.cp is not None or not self.fold_post_norm or cfg.head_dim != 128:
             return False
         T, layer = fb.input_ids.shape[0], self.w["layers"][0]
-        return all(self._stream_weight(T, layer[k], k == "gate_up") is not None
+        return T <= ops.STREAM_MAX_M and all(self._stream_weight(T, layer[k], k == "gate_up") is not None
                    for k in ("qkv", "o", "gate_up", "down"))
 
     def _stream_residual(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
@@ -452,15 +454,20 @@ class LlamaModel(Projections):
         norm = dict(inv_d=1.0 / cfg.hidden_size, eps=cfg.rms_eps)
         h = self.embed(fb.input_ids, fb.ids_src, fb.tok_slots)
         ss = ops.row_sumsq(h).view(T, 1)
+
+        def stream(epi, x, w, **kw):
+            w, packed = self._stream_weight(T, w, epi == 1)
+            return ops.stream(epi, x, w, packed=packed, **kw)
+
         mid, end = (ops.stream_sums(T, self.w["layers"][0][k], h.device) for k in ("o", "down"))
         for li, layer in enumerate(self.w["layers"]):
-            q = self._stream(3, h, layer["qkv"], ss=ss, positions=fb.positions, cos_sin=self.cos_sin,
-                             k_cache=kv.k[li], v_cache=kv.v[li], slots=fb.slots, hq=self.hq,
-                             hkv=self.hkv, **norm)
+            q = stream(3, h, layer["qkv"], ss=ss, positions=fb.positions, cos_sin=self.cos_sin,
+                       k_cache=kv.k[li], v_cache=kv.v[li], slots=fb.slots, hq=self.hq,
+                       hkv=self.hkv, **norm)
             o = self._attend(li, q.view(T, self.hq, cfg.head_dim), fb, kv)
-            self._stream(2, o.view(T, -1), layer["o"], out=h, ss=mid)
-            a = self._stream(1, h, layer["gate_up"], ss=mid, **norm)
-            self._stream(2, a, layer["down"], out=h, ss=end)
+            stream(2, o.view(T, -1), layer["o"], out=h, ss=mid)
+            a = stream(1, h, layer["gate_up"], ss=mid, **norm)
+            stream(2, a, layer["down"], out=h, ss=end)
             ss = end
         return h
 
@@ -499,11 +506,11 @@ class LlamaModel(Projections):
         when the measured table lists an unsplit (bf16-out) config for it."""
         W = self.w["lm_head"]
         cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
-        lg = self._stream(0, h, W)
-        if lg is None and cfg is not None and cfg[2] == 1:
+        if cfg is not None and cfg[2] == 1:
             lg = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
-        elif lg is None:
-            lg = ops.linear(h, W)
+        else:
+            lg = self._few(0, h, W)
+            lg = ops.linear(h, W) if lg is None else lg
         return pstate.tp_all_gather_lastdim(lg) if (self.tp > 1 and gather) else lg
 
     def forward(self, fb: ForwardBatch, kv: KVCache, gather: bool = True) -> torch.Tensor:

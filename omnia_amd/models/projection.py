@@ -51,8 +51,8 @@ class Projections:
     # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
 
-    # ---- a few rows (ops.stream): one launch a projection, with what follows in it
-    # copies of the projections in the order that kernel streams best, made before the KV
+    # ---- a few rows (ops.stream, ops.panel)
+    # copies of the projections in the order those kernels stream best, made before the KV
     # pool is sized, while they fit this part of HBM
     stream_budget_frac = 0.06
     STREAM_KEYS = {"qkv", "o", "gate_up", "down", "up", "in", "uq", "experts_gate_up",
@@ -71,7 +71,7 @@ class Projections:
                 if isinstance(t, (dict, list, tuple)):
                     walk(t)
                 elif k in self.STREAM_KEYS and isinstance(t, torch.Tensor) and \
-                        ops.stream_ok(1, t, True, gated=t.dim() == 3 or k == "gate_up"):
+                        ops.stream_ok(1, t, gated=t.dim() == 3 or k == "gate_up"):
                     found[t.data_ptr()] = t
 
         walk(self.w["layers"])
@@ -83,14 +83,11 @@ class Projections:
         return total
 
     def _stream_weight(self, M: int, w: torch.Tensor, gated: bool = False):
-        """(weight, packed) to run ``M`` rows of a projection on the streaming kernel, or None
-        for the other paths."""
-        if self.device.type != "cuda" or self.dtype != torch.bfloat16 or self.tp != 1 or \
-                M > ops.STREAM_MAX_M:
+        """(weight, packed) to run ``M`` rows of a projection on the streaming or the panel
+        kernel, or None for the other paths."""
+        if self.device.type != "cuda" or self.tp != 1 or not ops.stream_ok(M, w, gated):
             return None
         t = getattr(self, "_streams", {}).get(w.data_ptr())
-        if not ops.stream_ok(M, w, t is not None, gated):
-            return None
         return (w, False) if t is None else (t, True)
 
     def expert_streams(self, up: torch.Tensor, down: torch.Tensor):
@@ -99,10 +96,11 @@ class Projections:
         t = packs.get(up.data_ptr()), packs.get(down.data_ptr())
         return None if t[0] is None or t[1] is None else t
 
-    def _stream(self, epi: int, x: torch.Tensor, w: torch.Tensor, **kw):
-        """:func:`ops.stream` of one projection, or None."""
+    def _few(self, epi: int, x: torch.Tensor, w: torch.Tensor, slabs: bool = False, **kw):
+        """A plain (epi 0) or gated (1) projection of up to 256 rows: its rows or, with ``slabs``,
+        perhaps its slabs; None for more rows and what the kernels do not cover."""
         s = self._stream_weight(x.shape[0], w, epi == 1)
-        return None if s is None else ops.stream(epi, x, s[0], packed=s[1], **kw)
+        return None if s is None else ops.few_rows(epi, x, *s, slabs=slabs, **kw)
 
     # Projections return either a bf16 tensor (library / gemm.hip path, not yet
     # TP-reduced) or :class:`Parts` (fp32 split-K slabs of the weight-streaming
@@ -111,6 +109,12 @@ class Projections:
     # splitk_add_rmsnorm (residual add + RMSNorm), gate_up parts -> splitk_swiglu.
     def _wcfg(self, M: int, N: int, K: int, mode: int, is_decode: bool):
         if self.device.type != "cuda" or self.dtype != torch.bfloat16:
+            return None
+        # up to 192 rows the streaming and panel kernels are ahead of all paths in the tables,
+        # from there on behind the tile GEMM (us at 192 / 256 rows, panel and table: 6144 x 4096
+        # 19.7 / 23.0 and 21.1 / 21.2; 28672 x 4096 58 / 71 and 65 / 67; 4096 x 14336 33 / 41 and
+        # 36 / 39; 4096 x 4096 16.1 / 19.7 and 14.5 / 16.3)
+        if M <= 192 and self.tp == 1 and ops.streams_on() and N % 16 == 0 and K % 64 == 0:
             return None
         if not is_decode:
             # mid-size steps below the prefill tile's row threshold: split-K on
@@ -159,18 +163,18 @@ class Projections:
             self._ws[key] = buf
         return buf
 
-    def _proj(self, tag, x: torch.Tensor, w: torch.Tensor, is_decode: bool):
-        """Plain projection: Parts on the weight-streaming path, else bf16."""
+    def _proj(self, tag, x: torch.Tensor, w: torch.Tensor, is_decode: bool, slabs: bool = True):
+        """Plain projection: Parts on the split-K paths (unless ``slabs`` is off), else bf16."""
         M, K = x.shape
         if tag in ("o", "down") and not is_decode and overlap.applies(M, x.device):
             return RowPar(x, w)
         if self._pgemm_ok(M, K, w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
-        y = self._stream(0, x, w)
-        if y is not None:
-            return y
-        cfg = self._wcfg(M, w.shape[0], K, 0, is_decode)
+        cfg = self._wcfg(M, w.shape[0], K, 0, is_decode) if slabs else None
         if cfg is None:
+            y = self._few(0, x, w, slabs)
+            if y is not None:
+                return y if y.dim() == 2 else Parts(y)
             return ops.linear(x, w)
         nw, nwaves, S = cfg
         return Parts(self._wgemm(2, x, w, S, nw, nwaves,

@@ -461,31 +461,36 @@ def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tenso
 
 
 # ------------------------------------------------------ projections of a few rows (stream.hip)
-STREAM_MAX_M = 32  # with packed weights
-STREAM_ROW_MAJOR_M = 16
-STREAM_HEAD_ROWS = 65536
+STREAM_MAX_M = 16
 _stream_on = os.environ.get("OMNIA_STREAM", "1") != "0"
 
 
-def stream_rows(w: torch.Tensor, packed: bool) -> int:
-    """Most rows ``x`` may have for :func:`stream` to be the better kernel for ``w``.
-
-    Its blocks each read all of x, so rows cost: in us at 1 / 16 / 32 rows, with the kernel
-    that takes over in brackets, 28672 x 4096 packed 38 / 42 / 47 (52 / 53 / 54), row-major
-    41 / 50 / 59; 4096 x 4096 packed 7.0 / 8.5 / 11.5 (15 / 15 / 13), row-major 8.7 / 10.8 /
-    13.7; 2048 x 2048 row-major 5.0 / 6.7 / 8.1 (11).  A row-major head of 128256 x 4096 takes
-    168 at 1 row, 188 at 8 and 205 at 16 (188 / 189 / 191)."""
-    if packed:
-        return STREAM_MAX_M
-    return 8 if w.shape[0] >= STREAM_HEAD_ROWS else STREAM_ROW_MAJOR_M
+def streams_on() -> bool:
+    return _stream_on
 
 
-def stream_ok(M: int, w: torch.Tensor, packed: bool, gated: bool = False) -> bool:
-    """Whether :func:`stream` covers, and is chosen for, ``M`` rows and this GPU weight."""
+def stream_ok(M: int, w: torch.Tensor, gated: bool = False) -> bool:
+    """Whether :func:`stream` and :func:`panel` cover ``M`` rows of this GPU weight
+    (:func:`few_rows` chooses)."""
     R, K = w.shape[-2:]
-    return (_stream_on and w.is_cuda and 1 <= M <= stream_rows(w, packed)
-            and w.dtype == torch.bfloat16
+    return (_stream_on and w.is_cuda and 1 <= M <= PANEL_MAX_M and w.dtype == torch.bfloat16
             and K % 64 == 0 and R % (32 if gated else 16) == 0 and w.is_contiguous())
+
+
+def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bool = False,
+             **kw) -> torch.Tensor:
+    """A plain (epi 0) or gated (1) projection of up to 256 rows on the better kernel.
+
+    Up to 16 rows of packed weights stream (us at 8 rows, stream / panel: 2048 x 2048 4.5 / 4.7,
+    4096 x 4096 7.7 / 8.8, 16384 x 2048 14.9 / 14.4), unless few long rows leave that kernel's
+    blocks few (2048 x 8192 10.7 / 8.7).  Row-major weights reach the streaming kernel in
+    pieces, the panel kernel in whole lines (14.5 / 9.0; 4096 x 4096 9.5 / 8.8).  More rows, panel
+    / library: 64 rows of 2048 x 8192 9.7 / 22.2, 192 of 16384 x 2048 (gated) 27 / 32 and the
+    activation kernel, 256 of 2048 x 8192 19 / 27, of 3072 x 1024 9.8 / 8.7."""
+    R, K = w.shape
+    if packed and x.shape[0] <= STREAM_MAX_M and not (slabs and R < 192 * 16 and K >= 4096):
+        return stream(epi, x, w, packed=True, **kw)
+    return panel(epi, x, w, packed=packed, slabs=slabs, **kw)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -525,7 +530,7 @@ def stream(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None 
            packed: bool = False, ss: torch.Tensor | None = None, inv_d: float = 0.0,
            eps: float = 0.0, bias=None, gelu: bool = False, positions=None, cos_sin=None,
            k_cache=None, v_cache=None, slots=None, hq: int = 0, hkv: int = 0) -> torch.Tensor:
-    """``x @ w.T`` of up to 32 rows with a fused epilogue (``csrc/stream.hip``), GPU only.
+    """``x @ w.T`` of up to 16 rows with a fused epilogue (``csrc/stream.hip``), GPU only.
 
     ``ss`` (fp32 [M, n] partial sums of squares of the rows of ``x``) norms the rows first:
     ``x * rsqrt(sum(ss) * inv_d + eps)`` in bf16, an RMSNorm whose weight is folded into ``w``.
@@ -545,6 +550,55 @@ def stream(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None 
     kernels().stream_gemm(epi, out, x, w, stream_fragments(M, w.shape[0]), packed, ss_in, inv_d,
                           eps, ss_out, bias, gelu, positions, cos_sin, k_cache, v_cache, slots,
                           hq, hkv)
+    return out
+
+
+# -------------------------------------------------- projections of some tens of rows (panel.hip)
+PANEL_MAX_M = 256
+
+
+def _panel_cost(bm: int, rows: int, K: int, wn: int, S: int) -> float:
+    """Modelled us of a panel GEMM of ``bm`` rows: a block takes in its weight rows and x at about
+    50 GB/s, the chip the weights at 6 TB/s; slabs are written and read once more."""
+    blocks = -(-(rows // 16) // wn) * S
+    rounds = blocks / 256 if blocks > 3 * 256 else -(-blocks // 256)
+    t = max(rounds * (16 * wn + bm) * (K / S) * 2 / 50e3, rows * K * 2 / 6.0e6)
+    return t + (S * bm * rows * 8 / 8e6 if S > 1 else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def panel_slices(rows: int, K: int) -> int:
+    """K slices of a panel GEMM whose consumer sums slabs, from the weight's size alone: a row's
+    result must not depend on the rows beside it.  Chosen for 96 rows (us at 64 rows and 1 / 2 /
+    4 / 8 slices: 4096 x 4096 14.9 / 11.3 / 9.6 / 9.8, 2048 x 8192 - / - / 13.4 / 9.7)."""
+    return min((_panel_cost(96, rows, K, wn, S), S) for wn in (4, 8)
+               for S in range(1, min(16, K // 64) + 1))[1]
+
+
+@functools.lru_cache(maxsize=8192)
+def panel_plan(M: int, rows: int, K: int, slabs: bool) -> tuple[int, int]:
+    """(waves a block, K slices) of a panel GEMM with ``rows`` weight rows."""
+    bm = next((b for b in (64, 128, 192) if M <= b), PANEL_MAX_M)
+    S = panel_slices(rows, K) if slabs else 1
+    return min((_panel_cost(bm, rows, K, wn, S), wn) for wn in (8, 4))[1], S
+
+
+def panel(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool = False, bias=None,
+          gelu: bool = False, slabs: bool = False) -> torch.Tensor:
+    """``x @ w.T`` of up to 256 rows (``csrc/panel.hip``), GPU only.  epi 0: plain, or with
+    ``slabs`` perhaps fp32 partial slabs [S, M, N] whose sum it is; 1: ``act(g + b) * (u + b)``
+    with ``w = [Wg; Wu]``, silu or, with ``gelu``, its tanh form.  ``packed``: ``w`` is from
+    :func:`stream_pack`."""
+    M, K = x.shape
+    N = w.shape[0] // 2 if epi == 1 else w.shape[0]
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < K or x.data_ptr() % 16:
+        x = x.clone(memory_format=torch.contiguous_format)
+    wn, S = panel_plan(M, w.shape[0], K, slabs and epi == 0)
+    if S > 1:
+        out, epi = torch.empty(S, M, N, dtype=torch.float32, device=x.device), 2
+    else:
+        out = x.new_empty(M, N)
+    kernels().panel_gemm(epi, out, x, w, wn, packed, bias, gelu)
     return out
 
 

@@ -125,6 +125,9 @@ int omnia_stream(int epi, void* out, const void* x, const void* w, int M, int N,
                  float inv_d, float eps, float* ss_out, const float* bias, int gelu, const int* positions, const float* cos_sin,
                  void* k_cache, void* v_cache, const int64_t* slots, int hq, int hkv, int page,
                  hipStream_t s);
+int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, int K, int S,
+                int64_t ldx, int64_t ldo, int wn, int packed, const float* bias, int gelu,
+                hipStream_t s);
 int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                      const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                      int N, int topk, int n_assign, int e_lo, int max_blocks, int nw, int packed,
@@ -990,7 +993,7 @@ void pgemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W,
            "pgemm");
 }
 
-// projection of up to 32 rows (stream.hip); x rows may be strided
+// projection of up to 16 rows (stream.hip); x rows may be strided
 void stream_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t nw, bool packed,
                  c10::optional<at::Tensor> ss_in, double inv_d, double eps,
                  c10::optional<at::Tensor> ss_out, c10::optional<at::Tensor> bias, bool gelu,
@@ -1064,6 +1067,39 @@ void stream_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_
                         (float)eps, sso, bp, gelu, pos, cs, kc, vc, sl, (int)hq, (int)hkv, page,
                         cur_stream()),
            "stream_gemm");
+}
+
+// projection of up to 256 rows (panel.hip); x rows may be strided.  epi 2: out = slabs [S, M, N]
+void panel_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t wn, bool packed,
+                c10::optional<at::Tensor> bias, bool gelu) {
+  CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W);
+  TORCH_CHECK(epi >= 0 && epi <= 2, "epi");
+  TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && out.dim() == (epi == 2 ? 3 : 2), "operand dims");
+  TORCH_CHECK(x.stride(1) == 1 && W.is_contiguous(), "contiguous rows, W");
+  TORCH_CHECK(x.device() == W.device() && x.device() == out.device(), "same device");
+  const int M = x.size(0), K = x.size(1);
+  TORCH_CHECK(W.size(1) == K, "K mismatch");
+  TORCH_CHECK(epi != 1 || W.size(0) % 2 == 0, "gate_up rows even");
+  const int N = epi == 1 ? W.size(0) / 2 : W.size(0);
+  if (epi == 2) {
+    TORCH_CHECK(out.scalar_type() == at::kFloat && out.is_contiguous() && out.size(1) == M &&
+                out.size(2) == N, "slabs fp32 [S, M, N]");
+  } else {
+    TORCH_CHECK(out.scalar_type() == at::kBFloat16 && out.stride(1) == 1 && out.size(0) == M &&
+                out.size(1) == N, "out bf16 [M, N]");
+  }
+  const float* bp = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(epi == 1 && bias->device() == x.device() && bias->scalar_type() == at::kFloat &&
+                bias->is_contiguous() && bias->numel() == 2 * N, "bias fp32 [2N] (epi 1)");
+    bp = bias->data_ptr<float>();
+  }
+  if (M == 0) return;
+  CHECK_RC(omnia_panel((int)epi, out.data_ptr(), x.data_ptr(), W.data_ptr(), M, N, K,
+                       epi == 2 ? (int)out.size(0) : 1, x.stride(0),
+                       epi == 2 ? (int64_t)N : out.stride(0),
+                       (int)wn, packed, bp, gelu, cur_stream()),
+           "panel_gemm");
 }
 
 void pgemm_variant(int64_t variant, at::Tensor out, at::Tensor x, at::Tensor W) {
@@ -2098,6 +2134,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("dgemm", &dgemm);
   m.def("stream_gemm", &stream_gemm);
   m.def("stream_moe", &stream_moe);
+  m.def("panel_gemm", &panel_gemm);
   m.def("wgemm", &wgemm);
   m.def("wgemm_wide", &wgemm_wide);
   m.def("tgemm", &tgemm);

@@ -1,0 +1,240 @@
+// Projections of some tens of rows on gfx950: out[M, N] = x[M, K] . W[N, K]^T for M <= 256, bf16
+// in, fp32 MFMA accumulate: decode batches, short prompts, the next message of a session.
+//
+// The weights are still read once and set the floor, but a block that read all of x for 16
+// weight rows of its own (stream.hip) would spend its intake on x.  So x is shared:
+//   * a block of WN waves holds x of 64 to 256 rows in LDS, shared by the waves, and 16 weight
+//     rows of its own for each; both are filled by LDS-DMA, 8 rows x 128 bytes an instruction
+//     (chunks XORed so that fragment reads have no bank conflicts; weights packed as for
+//     stream.hip, ops.stream_pack, are one KB in fragment order instead);
+//   * WN is 8, or 4 where few columns would leave CUs without a block; S blocks share a column
+//     tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
+//     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
+//     depend on how many rows the step has;
+//   * a ring of NS stages, of which NS - 1 stay in flight across the one raw barrier of a stage.
+//     Past the end the loads go to one line, so that every wait counts the same number of loads.
+//     The DMA is written as asm: hipcc, not knowing which stage a fragment read belongs to,
+//     otherwise waits for all of it before some of the reads.
+//   EPI 0  out = acc            EPI 1  out = act(g + b) * (u + b), W = [Wg; Wu]
+//   EPI 2  fp32 slabs [S][M][N]
+#include "common.h"
+
+using namespace omnia;
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ float4v mfma16(short8 a, short8 b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+struct PanelArgs {
+  void* out;
+  const bf16_t *x, *w;  // [M, ldx]; [N, K], EPI 1 [2N, K]
+  int M, N, K, S;
+  int64_t ldx, ldo;
+  const float* bias;  // EPI 1: [2N] or null
+  int gelu;
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst`` (m0,
+// which nothing else in this file uses).  NT: weights, read once (28672 x 4096 at 16 rows 47.0
+// -> 43.1 us row-major, 44.2 -> 39.9 packed)
+template <bool NT>
+__device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
+  const uint32_t at = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)dst);
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(at),
+                 "v"(src)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at),
+                 "v"(src)
+                 : "memory");
+}
+
+// stages of (16 mf + 16 wn) x 128 bytes: up to 80 KB, two blocks a CU, where that is 3 stages
+// or more (28672 x 4096 at 16 rows, 3 / 6 stages: 38.5 / 39.9 us), else up to 144 KB
+constexpr int stages(int mf, int wn) {
+  const int kb = 2 * (mf + wn), fit = (kb <= 26 ? 80 : 144) / kb;
+  return fit > 5 ? 5 : fit;
+}
+
+template <int MF, int WN, int EPI, bool PK>
+__global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
+  constexpr int BM = 16 * MF, NS = stages(MF, WN);
+  constexpr int XI = BM / (8 * WN);  // DMA instructions of a wave and stage for x
+  constexpr int L = XI + 2;          // loads of a wave and stage
+  static_assert(NS >= 3 && XI >= 1, "ring");
+  constexpr int XS = BM * 64, ST = XS + WN * 1024;  // a stage: x, then the waves' weights
+  __shared__ __attribute__((aligned(16))) bf16_t xs[NS][ST];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fq = lane >> 4;
+  const int units = EPI == 1 ? p.N >> 3 : p.N >> 4, tiles = (units + WN - 1) / WN;
+  const int bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int split = bid / tiles, tile = bid - split * tiles;
+  const int unit0 = tile * WN + wv, unit = unit0 < units ? unit0 : units - 1;
+  const int K = p.K, nch = K >> 6;
+  const int c0 = split * nch / p.S, n = (split + 1) * nch / p.S - c0;  // 64-k chunks: stages
+
+  // this wave's weights: row-major, rows 8h.. of the unit and 16-byte chunk lane & 7 of each;
+  // packed, lane 16q + r's chunk of step h
+  const bf16_t* wp[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    auto at = [&](int rr) -> int64_t {  // weight row of the unit's row rr
+      if constexpr (EPI == 1) return (rr < 8 ? 0 : (int64_t)p.N - 8) + (int64_t)unit * 8 + rr;
+      return (int64_t)unit * 16 + rr;
+    };
+    if constexpr (PK) {
+      const int64_t r = at(fr);
+      wp[h] = p.w + (r >> 4) * 16 * K + h * 512 + 128 * fq + 8 * (r & 15);
+    } else {
+      const int rr = 8 * h + (lane >> 3);
+      wp[h] = p.w + at(rr) * K + (((lane & 7) ^ (rr & 7)) << 3);
+    }
+  }
+  const bf16_t* xp[XI];  // DMA instruction i of this wave: 8 rows
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = (wv * XI + i) * 8 + (lane >> 3);
+    xp[i] = p.x + (int64_t)(r < p.M ? r : p.M - 1) * p.ldx + (((lane & 7) ^ (r & 7)) << 3);
+  }
+  auto issue = [&](bf16_t* dst, int s) {  // stage s into a slot
+    const bool in = s < n;
+    const int64_t c = c0 + s;
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+      dma16<false>(in ? xp[i] + c * 64 : p.x, dst + (wv * XI + i) * 512);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      dma16<true>(in ? wp[h] + c * (PK ? 1024 : 64) : p.x, dst + XS + wv * 1024 + h * 512);
+  };
+  float4v acc[MF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i) acc[i] = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const bf16_t* src) {
+    const bf16_t* wb = src + XS + wv * 1024;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int ch = ((4 * h + fq) ^ (fr & 7)) << 3;  // rows 16i + fr share their XOR
+      const short8 w =
+          *reinterpret_cast<const short8*>(PK ? wb + h * 512 + lane * 8 : wb + fr * 64 + ch);
+#pragma unroll
+      for (int i = 0; i < MF; ++i)
+        acc[i] = mfma16(*reinterpret_cast<const short8*>(src + (16 * i + fr) * 64 + ch), w, acc[i]);
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(xs[s], s);
+  int at = 0;
+  for (; at + NS < n; at += NS)
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      wait_vm<(NS - 2) * L>();  // this stage's loads of this wave
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(xs[(u + NS - 1) % NS], at + u + NS - 1);
+      compute(xs[u]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  // up to NS stages are left, the last of them perhaps not yet asked for
+#pragma unroll
+  for (int u = 0; u < NS; ++u)
+    if (at + u < n) {
+      if (u == 0 || u == NS - 1) {
+        wait_vm<0>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (u == 0 && at + NS == n) issue(xs[NS - 1], at + NS - 1);
+      compute(xs[u]);
+    }
+
+  // lane: rows 16i + 4fq + r, column fr
+  if (unit0 >= units) return;
+#pragma unroll
+  for (int i = 0; i < MF; ++i) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * i + 4 * fq + r;
+      float v = acc[i][r];
+      if constexpr (EPI == 1) {
+        float u = __shfl_xor(v, 8, 64);  // the up half, in the lanes of the gate half
+        const int col = unit * 8 + (fr & 7);
+        float g = v;
+        if (p.bias) {
+          g += p.bias[col];
+          u += p.bias[p.N + col];
+        }
+        if (fr < 8 && m < p.M)
+          reinterpret_cast<bf16_t*>(p.out)[m * p.ldo + col] =
+              f2bf((p.gelu ? gelu_tanh_(g) : siluf_(g)) * u);
+      } else if (m < p.M) {
+        const int64_t col = (int64_t)unit * 16 + fr;
+        if constexpr (EPI == 0)
+          reinterpret_cast<bf16_t*>(p.out)[m * p.ldo + col] = f2bf(v);
+        else
+          reinterpret_cast<float*>(p.out)[((int64_t)split * p.M + m) * p.N + col] = v;
+      }
+    }
+  }
+}
+
+template <int MF, int WN, int EPI>
+int launch(const PanelArgs& p, bool packed, hipStream_t s) {
+  const int units = EPI == 1 ? p.N / 8 : p.N / 16;
+  const int grid = (units + WN - 1) / WN * p.S;
+  if (packed)
+    panel_kernel<MF, WN, EPI, true><<<grid, 64 * WN, 0, s>>>(p);
+  else
+    panel_kernel<MF, WN, EPI, false><<<grid, 64 * WN, 0, s>>>(p);
+  return (int)hipGetLastError();
+}
+
+template <int WN, int EPI>
+int by_rows(const PanelArgs& p, bool packed, hipStream_t s) {
+  if (p.M <= 64) return launch<4, WN, EPI>(p, packed, s);
+  if (p.M <= 128) return launch<8, WN, EPI>(p, packed, s);
+  if (p.M <= 192) return launch<12, WN, EPI>(p, packed, s);
+  return launch<16, WN, EPI>(p, packed, s);
+}
+
+template <int EPI>
+int by_waves(const PanelArgs& p, int wn, bool packed, hipStream_t s) {
+  return wn == 8 ? by_rows<8, EPI>(p, packed, s) : by_rows<4, EPI>(p, packed, s);
+}
+
+}  // namespace
+
+extern "C" {
+
+// 0 on success, < 0 for what the kernel does not cover (checked before any launch).  wn: waves
+// a block (4, 8).
+int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, int K, int S,
+                int64_t ldx, int64_t ldo, int wn, int packed, const float* bias, int gelu,
+                hipStream_t s) {
+  if (epi < 0 || epi > 2) return -1;
+  if (M < 1 || M > 256) return -2;
+  if (K < 64 || K % 64 || ldx < K || ldx % 8) return -3;
+  if (S < 1 || S > 16 || S > K / 64 || (epi != 2 && S != 1)) return -4;
+  if (N < 16 || N % 16 || N > 1 << 24) return -5;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return -6;
+  if (bias && epi != 1) return -7;
+  if (wn != 4 && wn != 8) return -8;
+  const PanelArgs p{out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, S, ldx, ldo, bias, gelu};
+  if (epi == 0) return by_waves<0>(p, wn, packed, s);
+  if (epi == 1) return by_waves<1>(p, wn, packed, s);
+  return by_waves<2>(p, wn, packed, s);
+}
+
+}  // extern "C"

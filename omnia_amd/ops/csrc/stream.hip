@@ -1,4 +1,4 @@
-// Projections of a few rows on gfx950: out[M, N] = x[M, K] . W[N, K]^T for M <= 32, bf16 in,
+// Projections of a few rows on gfx950: out[M, N] = x[M, K] . W[N, K]^T for M <= 16, bf16 in,
 // fp32 MFMA accumulate, with the work that follows in the epilogue.
 //
 // At these sizes a projection reads its weights once and does little else, and a model step
@@ -7,15 +7,14 @@
 //   * A block of 8 waves owns 16 or 32 weight rows over the whole of K; the waves take turns
 //     at 64-k chunks, so together they read one contiguous KB of every row at a time, and meet
 //     once, in LDS, at the end.  No slabs, no second kernel, no atomics, a fixed order of sums.
-//   * Weights go from HBM to MFMA operand registers, 32 contiguous bytes a lane (the k order
-//     inside a chunk is the lanes'; x is read in the same order).  x comes from L2, as it is
-//     shared by all blocks.
+//   * Weights go from HBM to MFMA operand registers; x comes from L2, as it is shared by all
+//     blocks.
 //   * Row-major weights reach a CU in 64-byte pieces of 16 rows; PK weights (a copy laid out
 //     [row / 16][k / 64][k / 32][k / 8][row % 16][8], ops.stream_pack) as one KB a wave
 //     instruction: 28672 x 4096 at one row 40.9 us row-major, 37.9 packed; 4096 x 14336 24.5
 //     and 20.9.  Streaming loads (nt) help packed reads (41.7 -> 37.9) and hurt row-major ones.
-//   * A ring of D chunks a wave is in flight from the first instruction on: 48-64 KB a block,
-//     two blocks a CU.
+//   * A ring of D chunks a wave is in flight from the first instruction on: 64 KB of weights a
+//     block, two blocks a CU.
 //   * NORM: x is the residual, whose rows are RMS-normed (the norm's weight is folded into W)
 //     and rounded to bf16 as they become operands, as a norm kernel would: no launch, no pass.
 //     The rows' sums of squares come from the kernel that wrote the residual (EPI 2).
@@ -75,16 +74,12 @@ __device__ __forceinline__ float clamped_glu(float g, float u, float alpha, floa
   return g * sigmoidf_(alpha * g) * (u + 1.f);
 }
 
-// chunks in flight of MF + NW operand fragments, 8 registers each, and waves a SIMD they leave
-// room for
-constexpr int ring(int frags) { return frags <= 4 ? 4 : 3; }
-constexpr int waves(int frags) { return frags <= 3 ? 4 : 2; }
-
-template <int MF, int NW, int EPI, bool NORM, bool PK>
-__global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(StreamArgs p) {
-  constexpr int D = ring(MF + NW), F = 8 * NW;  // F: features of a paired block
-  __shared__ __attribute__((aligned(16))) float red[WAVES * MF * NW * 256];
-  __shared__ float rsl[NORM ? 16 * MF : 1];
+// D: chunks in flight of 1 + NW operand fragments, 8 registers each
+template <int NW, int EPI, bool NORM, bool PK>
+__global__ __launch_bounds__(64 * WAVES, NW <= 2 ? 4 : 2) void stream_kernel(StreamArgs p) {
+  constexpr int D = NW <= 2 ? 4 : 3, F = 8 * NW;  // F: features of a paired block
+  __shared__ __attribute__((aligned(16))) float red[WAVES * NW * 256];
+  __shared__ float rsl[NORM ? 16 : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4, unit = blockIdx.x;
@@ -108,29 +103,25 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
     return (int64_t)unit * 16 * NW + rr;
   };
   const bf16_t* wp[NW];
-  const bf16_t* xp[MF];
 #pragma unroll
   for (int j = 0; j < NW; ++j) {
     const int64_t r = wrow(16 * j + fr);
     wp[j] = wbase + (PK ? (r >> 4) * 16 * K + 128 * fq + 8 * (r & 15) : r * K + 8 * fq);
   }
-#pragma unroll
-  for (int i = 0; i < MF; ++i) {
-    int64_t row;
-    if constexpr (grouped(EPI) && EPI != 6) {
-      const int f = p.sorted[seg * 16 * MF + 16 * i + fr];
-      row = f < p.n_assign ? f / p.topk : 0;  // padding: any row, never written
-    } else if constexpr (EPI == 6) {
-      row = seg * 16 * MF + 16 * i + fr;
-    } else {
-      row = 16 * i + fr < p.M ? 16 * i + fr : p.M - 1;
-    }
-    xp[i] = p.x + row * p.ldx + 8 * fq;
+  int64_t xrow;
+  if constexpr (grouped(EPI) && EPI != 6) {
+    const int f = p.sorted[seg * 16 + fr];
+    xrow = f < p.n_assign ? f / p.topk : 0;  // padding: any row, never written
+  } else if constexpr (EPI == 6) {
+    xrow = seg * 16 + fr;
+  } else {
+    xrow = fr < p.M ? fr : p.M - 1;
   }
+  const bf16_t* xp = p.x + xrow * p.ldx + 8 * fq;
 
   // row sums of squares: requested before anything else, needed after the weights are on
   // their way
-  constexpr int RW = 2 * MF;  // rows of a wave
+  constexpr int RW = 16 / WAVES;  // rows of a wave
   float sv[NORM ? RW : 1][4];
   if constexpr (NORM) {
 #pragma unroll
@@ -146,7 +137,7 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
   }
 
   const int nch = K >> 6, n = (nch - wv + WAVES - 1) / WAVES;  // this wave's chunks
-  short8 wr[D][NW][2], xr[D][MF][2];
+  short8 wr[D][NW][2], xr[D][2];
   auto load = [&](auto& w, auto& x, int i) {
     const int c = wv + WAVES * i;
     const int64_t o = (int64_t)(c < nch ? c : nch - 1) * 64, ow = PK ? 16 * o : o;
@@ -158,34 +149,25 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
         w[j][h] = PK ? __builtin_nontemporal_load(v) : *v;
       }
 #pragma unroll
-    for (int i2 = 0; i2 < MF; ++i2)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        x[i2][h] = *reinterpret_cast<const short8*>(xp[i2] + o + 32 * h);
+    for (int h = 0; h < 2; ++h) x[h] = *reinterpret_cast<const short8*>(xp + o + 32 * h);
   };
-  float4v acc[MF][NW];
-  float rs[MF];
+  float4v acc[NW];
+  float rs = 1.f;
 #pragma unroll
-  for (int i = 0; i < MF; ++i) {
-    rs[i] = 1.f;
-#pragma unroll
-    for (int j = 0; j < NW; ++j) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
-  }
+  for (int j = 0; j < NW; ++j) acc[j] = {0.f, 0.f, 0.f, 0.f};
   auto compute = [&](auto& w, auto& x) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      short8 a = x[h];
+      if constexpr (NORM) {
+        bf16x8 y;
 #pragma unroll
-      for (int i = 0; i < MF; ++i) {
-        short8 a = x[i][h];
-        if constexpr (NORM) {
-          bf16x8 y;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) y[e] = (__bf16)(bf2f((uint16_t)a[e]) * rs[i]);
-          a = __builtin_bit_cast(short8, y);
-        }
-#pragma unroll
-        for (int j = 0; j < NW; ++j) acc[i][j] = mfma16(a, w[j][h], acc[i][j]);
+        for (int e = 0; e < 8; ++e) y[e] = (__bf16)(bf2f((uint16_t)a[e]) * rs);
+        a = __builtin_bit_cast(short8, y);
       }
+#pragma unroll
+      for (int j = 0; j < NW; ++j) acc[j] = mfma16(a, w[j][h], acc[j]);
+    }
   };
   // Loads are unconditional (past the end: the last chunk again) and stay where they are
   // written, so that every wait counts the loads behind it instead of draining them.
@@ -203,8 +185,7 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
       if (lane == 0) rsl[row] = rsqrtf(v * p.inv_d + p.eps);
     }
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < MF; ++i) rs[i] = rsl[16 * i + fr];
+    rs = rsl[fr];
   }
   int at = 0;
   for (; at + D < n; at += D)
@@ -218,30 +199,26 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
   for (int d = 0; d < D; ++d)
     if (at + d < n) compute(wr[d], xr[d]);
 
-  // ---- the waves' sums meet: lane holds rows 16i + 4fq + r of column 16j + fr
+  // ---- the waves' sums meet: lane holds rows 4fq + r of column 16j + fr
 #pragma unroll
-  for (int i = 0; i < MF; ++i) {
-#pragma unroll
-    for (int j = 0; j < NW; ++j)
-      *reinterpret_cast<float4v*>(red + ((wv * MF + i) * NW + j) * 256 + lane * 4) = acc[i][j];
-  }
+  for (int j = 0; j < NW; ++j)
+    *reinterpret_cast<float4v*>(red + (wv * NW + j) * 256 + lane * 4) = acc[j];
   __syncthreads();
-  // rows 16i + 4q + 0..3 of the block's weight row rr
-  auto total = [&](int i, int rr, int q) {
+  // rows 4q + 0..3 of the block's weight row rr
+  auto total = [&](int rr, int q) {
     float4v s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < WAVES; ++v)
-      s += *reinterpret_cast<const float4v*>(
-          red + ((v * MF + i) * NW + (rr >> 4)) * 256 + (q * 16 + (rr & 15)) * 4);
+      s += *reinterpret_cast<const float4v*>(red + (v * NW + (rr >> 4)) * 256 +
+                                             (q * 16 + (rr & 15)) * 4);
     return s;
   };
   constexpr int COLS = paired(EPI) ? F : 16 * NW;
   bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
-  for (int g = tid; g < MF * 4 * COLS; g += 64 * WAVES) {
-    const int c = g % COLS, q = (g / COLS) & 3, i = g / (4 * COLS);
-    const int row0 = 16 * i + 4 * q;
-    float4v a = total(i, c, q), b = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (paired(EPI)) b = total(i, F + c, q);
+  if (tid < 4 * COLS) {
+    const int c = tid % COLS, q = tid / COLS;
+    float4v a = total(c, q), b = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (paired(EPI)) b = total(F + c, q);
     float ba = 0.f, bb = 0.f;
     if constexpr (EPI == 0)
       if (p.bias) ba = p.bias[unit * COLS + c];
@@ -252,7 +229,7 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
       }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int m = row0 + r;
+      const int m = 4 * q + r;
       const int64_t col = (int64_t)unit * COLS + c;
       float va = a[r], vb = b[r];
       if constexpr (!grouped(EPI)) {
@@ -299,7 +276,7 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
           o[64] = f2bf(vb);
         }
       } else {
-        const int row = seg * 16 * MF + m, f = p.sorted[row];
+        const int row = seg * 16 + m, f = p.sorted[row];
         if (f >= p.n_assign) continue;
         if constexpr (EPI == 6) {
           out[f * p.ldo + col] = f2bf(p.route_w ? p.route_w[f] * va : va);
@@ -316,28 +293,23 @@ __global__ __launch_bounds__(64 * WAVES, waves(MF + NW)) void stream_kernel(Stre
   }
 }
 
-template <int MF, int NW, int EPI, bool NORM>
+template <int NW, int EPI, bool NORM>
 int launch(const StreamArgs& p, bool packed, int segs, hipStream_t s) {
   const int cols = paired(EPI) ? 8 * NW : 16 * NW;
   const int width = EPI == 3 ? (p.hq + 2 * p.hkv) * 64 : p.N;
   const dim3 grid(width / cols, segs);
   if (packed)
-    stream_kernel<MF, NW, EPI, NORM, true><<<grid, 64 * WAVES, 0, s>>>(p);
+    stream_kernel<NW, EPI, NORM, true><<<grid, 64 * WAVES, 0, s>>>(p);
   else
-    stream_kernel<MF, NW, EPI, NORM, false><<<grid, 64 * WAVES, 0, s>>>(p);
+    stream_kernel<NW, EPI, NORM, false><<<grid, 64 * WAVES, 0, s>>>(p);
   return (int)hipGetLastError();
 }
 
 template <int EPI, bool NORM>
-int by_size(const StreamArgs& p, int mf, int nw, bool packed, int segs, hipStream_t s) {
-#define OMNIA_ST(A, B) \
-  if (mf == A && nw == B) return launch<A, B, EPI, NORM>(p, packed, segs, s);
-  OMNIA_ST(1, 1) OMNIA_ST(1, 2) OMNIA_ST(1, 4)
-  if constexpr (!grouped(EPI)) {
-    OMNIA_ST(2, 1) OMNIA_ST(2, 2) OMNIA_ST(2, 4)
-  }
-#undef OMNIA_ST
-  return -20;
+int by_width(const StreamArgs& p, int nw, bool packed, int segs, hipStream_t s) {
+  if (nw == 1) return launch<1, EPI, NORM>(p, packed, segs, s);
+  if (nw == 2) return launch<2, EPI, NORM>(p, packed, segs, s);
+  return launch<4, EPI, NORM>(p, packed, segs, s);
 }
 
 }  // namespace
@@ -352,7 +324,7 @@ int omnia_stream(int epi, void* out, const void* x, const void* w, int M, int N,
                  void* k_cache, void* v_cache, const int64_t* slots, int hq, int hkv, int page,
                  hipStream_t s) {
   if (epi < 0 || epi > 3) return -1;
-  if (M < 1 || M > 32) return -2;
+  if (M < 1 || M > 16) return -2;
   if (K < 64 || K % 64 || ldx < K || ldx % 8) return -3;
   if (nw != 1 && nw != 2 && nw != 4) return -4;
   const int cols = epi == 1 ? 8 * nw : 16 * nw;
@@ -386,11 +358,10 @@ int omnia_stream(int epi, void* out, const void* x, const void* w, int M, int N,
   p.hq = hq;
   p.hkv = hkv;
   p.page = page;
-  const int mf = M <= 16 ? 1 : 2;
-  if (epi == 0) return norm ? by_size<0, true>(p, mf, nw, packed, 1, s) : by_size<0, false>(p, mf, nw, packed, 1, s);
-  if (epi == 1) return norm ? by_size<1, true>(p, mf, nw, packed, 1, s) : by_size<1, false>(p, mf, nw, packed, 1, s);
-  if (epi == 2) return by_size<2, false>(p, mf, nw, packed, 1, s);
-  return norm ? by_size<3, true>(p, mf, nw, packed, 1, s) : by_size<3, false>(p, mf, nw, packed, 1, s);
+  if (epi == 0) return norm ? by_width<0, true>(p, nw, packed, 1, s) : by_width<0, false>(p, nw, packed, 1, s);
+  if (epi == 1) return norm ? by_width<1, true>(p, nw, packed, 1, s) : by_width<1, false>(p, nw, packed, 1, s);
+  if (epi == 2) return by_width<2, false>(p, nw, packed, 1, s);
+  return norm ? by_width<3, true>(p, nw, packed, 1, s) : by_width<3, false>(p, nw, packed, 1, s);
 }
 
 // Grouped products of a few rows an expert: segments of 16 rows as omnia_moe_align makes them.
@@ -424,10 +395,10 @@ int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const in
   p.e_lo = e_lo;
   p.alpha = alpha;
   p.limit = limit;
-  if (mode == 0) return by_size<5, false>(p, 1, nw, packed, max_blocks, s);
-  if (mode == 1) return by_size<6, false>(p, 1, nw, packed, max_blocks, s);
-  if (mode == 2) return by_size<8, false>(p, 1, nw, packed, max_blocks, s);
-  return by_size<10, false>(p, 1, nw, packed, max_blocks, s);
+  if (mode == 0) return by_width<5, false>(p, nw, packed, max_blocks, s);
+  if (mode == 1) return by_width<6, false>(p, nw, packed, max_blocks, s);
+  if (mode == 2) return by_width<8, false>(p, nw, packed, max_blocks, s);
+  return by_width<10, false>(p, nw, packed, max_blocks, s);
 }
 
 }  // extern "C"

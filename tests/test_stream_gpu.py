@@ -1,4 +1,5 @@
-"""Streaming projections of a few rows (``csrc/stream.hip``) against float64."""
+"""Projections of a few rows (``csrc/stream.hip``) and of some tens (``csrc/panel.hip``)
+against float64."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -46,8 +47,8 @@ def _close_normed(got, x, w, K, f=lambda h: h):
     assert err.norm() <= 1.2 * U * want.norm()
 
 
-# rows around the 16-row fragments; K of one chunk, fewer chunks than waves, an odd number
-SIZES = [(1, 16, 64), (15, 48, 192), (16, 4096, 576), (17, 96, 1024), (31, 64, 4160), (32, 512, 640)]
+# one row to a fragment; K of one chunk, fewer chunks than waves, odd numbers of chunks
+SIZES = [(1, 16, 64), (15, 48, 192), (16, 4096, 576), (7, 96, 1024), (13, 64, 4160), (16, 512, 640)]
 
 
 @pytest.mark.parametrize("packed", [False, True])
@@ -100,7 +101,7 @@ def test_gated(M, N, K, gelu, packed):
 
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("M,hq,hkv,K", [(1, 1, 1, 64), (5, 32, 8, 512), (16, 4, 2, 4096),
-                                        (32, 8, 1, 192), (25, 7, 1, 1024)])
+                                        (12, 8, 1, 192), (9, 7, 1, 1024)])
 def test_qkv(M, hq, hkv, K, packed):
     x, w = _mk(M, (hq + 2 * hkv) * 128, K, M + hq)
     page, nb = 16, 6
@@ -153,20 +154,89 @@ def test_experts_match_the_64_row_kernels(T, E, k, glu, gelu, packed, monkeypatc
 
 
 def test_what_is_refused():
-    x, w = _mk(33, 64, 128, 1)
+    x, w = _mk(17, 64, 128, 1)
     with pytest.raises(RuntimeError):
         ops.stream(0, x, w)  # rows
     with pytest.raises(RuntimeError):
         ops.stream(0, x[:4, :96].contiguous(), w[:, :96].contiguous())  # whole 64-k chunks
     with pytest.raises(RuntimeError):
         ops.stream(0, x[:4], w[:40].contiguous())  # whole 16-row fragments
-    assert not ops.stream_ok(4, w[:40], False) and not ops.stream_ok(33, w, True)
+    assert not ops.stream_ok(4, w[:40]) and not ops.stream_ok(257, w)
+    x, _ = _mk(257, 64, 128, 1)
+    with pytest.raises(RuntimeError):
+        ops.panel(0, x, w)
+    with pytest.raises(RuntimeError):
+        ops.panel(0, x[:4], w[:40].contiguous())
 
 
-@pytest.mark.parametrize("rows,pack", [(1, True), (16, False), (23, True)])
+# rows around the tiles of 64 to 256; columns of fewer units than waves and of a remainder;
+# K of one chunk, of slices of unequal length and of fewer chunks than the ring has stages
+PANEL = [(1, 16, 64), (17, 48, 128), (63, 272, 576), (64, 2048, 8192), (65, 528, 1024),
+         (128, 64, 4160), (129, 4096, 640), (192, 80, 1088), (193, 64, 256), (256, 144, 2048)]
+
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M,N,K", PANEL)
+def test_panel_every_split(M, N, K, packed, monkeypatch):
+    x, w = _mk(M, N, K, M + N + K)
+    want, wk = x.double() @ w.double().T, _weight(w, packed)
+    for wn in (4, 8):
+        for S in {1, 2, 3, min(16, K // 64)}:
+            if S > K // 64:
+                continue
+            monkeypatch.setattr(ops, "panel_plan", lambda *a: (wn, S))
+            got = ops.panel(0, x, wk, packed=packed, slabs=True)
+            if S > 1:
+                assert got.shape == (S, M, N) and got.dtype == torch.float32
+                _close(got.sum(0), want, K, 0)
+            else:
+                _close(got, want, K)
+    monkeypatch.undo()
+    wide = torch.randn(M, K + 72, device="cuda").to(torch.bfloat16)
+    for off in (8, 3):  # strided rows, and rows off the 16-byte grid
+        v = wide[:, off:off + K]
+        _close(ops.panel(0, v, wk, packed=packed), v.double() @ w.double().T, K)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("M,N,K", PANEL)
+def test_panel_gated(M, N, K, gelu, packed, monkeypatch):
+    x, w = _mk(M, 2 * N, K, M * N)
+    b = torch.randn(2 * N, device="cuda")
+    hb = (x.double() @ w.double().T + b.double()).chunk(2, 1)
+    want = (F.gelu(hb[0], approximate="tanh") if gelu else F.silu(hb[0])) * hb[1]
+    for wn in (4, 8):
+        monkeypatch.setattr(ops, "panel_plan", lambda *a: (wn, 1))
+        got = ops.panel(1, x, _weight(w, packed), packed=packed, bias=b, gelu=gelu)
+        _close(got, want, 4 * K, 1.1)
+
+
+def test_panel_plans_fit_the_kernel():
+    """Whatever the size, a plan is one that the kernel covers, with slices that do not depend on
+    the rows."""
+    for rows in (16, 240, 4096, 8256, 128256):
+        for K in (64, 192, 1024, 14336):
+            plans = [ops.panel_plan(M, rows, K, True) for M in (1, 64, 65, 128, 129, 256)]
+            assert {wn for wn, _ in plans} <= {4, 8} and len({S for _, S in plans}) == 1
+            assert 1 <= plans[0][1] <= min(16, K // 64)
+            assert ops.panel_plan(100, rows, K, False)[1] == 1
+
+
+def test_panel_rows_do_not_depend_on_each_other():
+    """The same rows in steps of other sizes give the same bits, slabs included."""
+    x, w = _mk(256, 2048, 4096, 9)
+    for slabs in (False, True):
+        whole = ops.panel(0, x, w, slabs=slabs)
+        for M in (1, 20, 64, 100, 130):
+            assert torch.equal(ops.panel(0, x[:M], w, slabs=slabs), whole[..., :M, :])
+
+
+@pytest.mark.parametrize("rows,pack", [(1, True), (16, False), (23, True), (32, False)])
 def test_llama_layers_match_the_unfused_path(rows, pack, monkeypatch):
-    """Decode steps of a small model: the four streamed projections a layer against separate
-    norm, RoPE, SwiGLU and residual kernels."""
+    """Decode steps of a small model: the four streamed projections a layer, and the panel
+    kernel's, against the library's GEMMs with separate norm, RoPE, SwiGLU and residual kernels."""
     from omnia_amd.engine.engine import EngineConfig, LLMEngine
     from omnia_amd.engine.sampling_params import SamplingParams
 
