@@ -774,6 +774,25 @@ def prefill_tiles(q_lens: list[int], tile: int | None = None) -> tuple[list[int]
     return seqs, q0s
 
 
+@functools.lru_cache(maxsize=4096)
+def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int) -> int:
+    """Most key partitions of a 32-row query tile, for up to 512 blocks, two a CU (fewer where the
+    live length gives a partition less than 128 keys).  A block walks its 64-key tiles one after
+    the other, 1.35 us each; partitions shorten that walk but write and read fp32 partials, at
+    about 3 TB/s, and cost a launch (us at 1 / 2 / 4 / 8 partitions, 32 heads on 8: 77 rows on
+    4000 keys 89 / 53 / 34 / 28, on 1100 29 / 23 / 20 / 21, on 400 16.0 / 16.2 / 15.8 / 15.9;
+    512 on 3000 69 / 53 / 49 / 58, on 512 18 / 22 / 25 / 25)."""
+    group = hq // hkv
+    blocks = tiles * hq // (4 if group % 4 == 0 else 2 if group % 2 == 0 else 1)
+    walk = -(-max_keys // 64) * 1.35
+    best, cost = 1, walk
+    for P in range(2, min(16, 512 // max(blocks, 1), max_keys // 128) + 1):
+        c = walk / P + 5.0 + P * tiles * 32 * hq * 1024 / 3e6
+        if c < cost:
+            best, cost = P, c
+    return best
+
+
 def prefill_attention(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens, scale,
                       tile_seq=None, tile_q0=None, out=None, heads_per_wave: int = 0,
                       q_tile: int | None = None, lse=None, kv_lens=None):
@@ -795,9 +814,14 @@ def prefill_attention(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens, 
         if checks.active(q):
             checks.paged("prefill_attention", block_tables, seq_lens, k_cache,
                          q_start_loc.numel() - 1)
+        q_tile = q_tile or PREFILL_Q_TILE
+        parts = 1
+        if q_tile == 32 and lse is None and kv_lens is None:
+            parts = prefill_parts(tile_seq.numel(), q.shape[1], k_cache.shape[1],
+                                  block_tables.shape[1] * k_cache.shape[2])
         kernels().prefill_attention(out, q, k_cache, v_cache, block_tables, q_start_loc,
-                                    seq_lens, tile_seq, tile_q0, scale, heads_per_wave,
-                                    q_tile or PREFILL_Q_TILE, lse, kv_lens)
+                                    seq_lens, tile_seq, tile_q0, scale, heads_per_wave, q_tile,
+                                    lse, kv_lens, parts)
         return out
     if lse is not None or kv_lens is not None:
         r, l = ref.paged_attention_lse(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens,

@@ -234,11 +234,14 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(
   }
 }
 
-// grid: (B * Hq)   block: 128
-__global__ __launch_bounds__(128) void decode_reduce_kernel(
+// grid: (B * Hq)   block: 256.  Latency bound: a lane takes one partition's (m, l) of each 64 and
+// the four waves take every fourth partition's row, with the loads of several in flight (one
+// after the other, a 2000-key sequence in 32 partitions took 20.3 us with its attention, now 12.9).
+__global__ __launch_bounds__(256) void decode_reduce_kernel(
     bf16_t* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_ml,
     const int* __restrict__ seq_lens, int hq, int part_size, int max_parts, int split_t,
     int split_min, int bs) {
+  __shared__ float2 red[3][64];
   const int bh = blockIdx.x;
   const int b = bh / hq;
   const int len = seq_lens[b];
@@ -246,17 +249,48 @@ __global__ __launch_bounds__(128) void decode_reduce_kernel(
   const int pl = decode_part_len(len, part_size, split_t, split_min, bs);
   const int nparts = (len + pl - 1) / pl;
   if (nparts <= 1) return;
-  const float* ml = part_ml + (int64_t)bh * max_parts * 2;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const float2* ml = reinterpret_cast<const float2*>(part_ml) + (int64_t)bh * max_parts;
+  const float2* po =
+      reinterpret_cast<const float2*>(part_o) + (int64_t)bh * max_parts * (D / 2) + lane;
   float m = -INFINITY;
-  for (int p = 0; p < nparts; ++p) m = fmaxf(m, ml[2 * p]);
-  float tot = 0.f, acc = 0.f;
-  const int d = threadIdx.x;
-  for (int p = 0; p < nparts; ++p) {
-    const float wgt = exp2f(ml[2 * p] - m) * ml[2 * p + 1];
-    tot += wgt;
-    acc += wgt * part_o[((int64_t)bh * max_parts + p) * D + d];
+  for (int p = lane; p < nparts; p += 64) m = fmaxf(m, ml[p].x);
+  m = wave_max(m);
+  float tot = 0.f;
+  float2 acc = {0.f, 0.f};
+  for (int p0 = 0; p0 < nparts; p0 += 64) {
+    float wl = 0.f;
+    if (p0 + lane < nparts) {
+      const float2 v = ml[p0 + lane];
+      wl = exp2f(v.x - m) * v.y;
+    }
+    tot += wl;
+    const int n = min(64, nparts - p0);
+    for (int i0 = w; i0 < n; i0 += 32) {
+      float2 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = po[(int64_t)(p0 + min(i0 + 4 * u, n - 1)) * (D / 2)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float g = __shfl(wl, (i0 + 4 * u) & 63, 64);
+        if (i0 + 4 * u < n) {
+          acc.x += g * v[u].x;
+          acc.y += g * v[u].y;
+        }
+      }
+    }
   }
-  out[(int64_t)bh * D + d] = f2bf(acc / tot);
+  tot = wave_sum(tot);
+  if (w) red[w - 1][lane] = acc;
+  __syncthreads();
+  if (w) return;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    acc.x += red[i][lane].x;
+    acc.y += red[i][lane].y;
+  }
+  const uint32_t pk = pack_bf2(acc.x / tot, acc.y / tot);
+  reinterpret_cast<uint32_t*>(out)[(int64_t)bh * (D / 2) + lane] = pk;
 }
 
 // ============================================================== prefill
@@ -496,14 +530,27 @@ __device__ __forceinline__ int img(int row, int ch) {
   return row * 256 + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
-template <int BS, int HB>
+// Key partitions of a query tile with ``ntiles`` 64-key tiles, at most S, of at least kPartTiles
+// tiles each.
+constexpr int kPartTiles = 2;
+__device__ __forceinline__ int prefill_parts(int ntiles, int S) {
+  return max(1, min(S, ntiles / kPartTiles));
+}
+
+// SPLIT: gridDim.z blocks share a query tile's keys, decided from the live length, and write fp32
+// partials (O unnormalised [z][T][hq][D], max and sum [z][T][hq][2]) for prefill_merge_kernel; a
+// tile of one partition writes its result.  The walk over the keys is a serial chain of 1.35 us a
+// 64-key tile, which few query tiles leave most of the chip to wait for (3 tiles of 8 blocks on
+// 4000 keys: 89 us, 29 in 8 partitions; ops.prefill_parts).
+template <int BS, int HB, bool SPLIT>
 __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
     const bf16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ q_start_loc, const int* __restrict__ seq_lens,
     const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int hkv, int64_t q_stride,
     int64_t out_stride, float scale_log2, float* __restrict__ lse_out,
-    const int* __restrict__ kv_lens) {
+    const int* __restrict__ kv_lens, float* __restrict__ part_o, float2* __restrict__ part_ml,
+    int64_t part_rows) {
   // two K | V stages (separate objects, so the compiler sees that fragment reads
   // of one stage cannot alias the other stage's in-flight LDS-DMA): the next
   // tile is written while this one is still read, one barrier per tile
@@ -542,8 +589,15 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   const int last_row = min(q0 + 31, qlen - 1);
   const int klim = kv_lens ? kv_lens[s] : 0x7fffffff;
   const int kv_end = min(off + last_row + 1, klim);
-  const int ntiles = (kv_end + 63) / 64;
+  int t0 = 0, ntiles = (kv_end + 63) / 64, parts = 1;
   const int min_qpos = off + q0;
+  if constexpr (SPLIT) {
+    parts = prefill_parts(ntiles, gridDim.z);
+    const int z = blockIdx.z;
+    if (z >= parts) return;
+    t0 = ntiles * z / parts;
+    ntiles = ntiles * (z + 1) / parts;
+  }
 
   const int npg = min((kv_end + BS - 1) / BS, kMaxPages);
   for (int i = tid; i < npg; i += 64 * HB) pg_lds[i] = bt[i];
@@ -580,7 +634,8 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
     }
   };
 
-  float m_run = -INFINITY, l_run = 0.f;
+  // a row whose keys all lie before the partition keeps the finite start: its exponents are 0
+  float m_run = SPLIT ? -3.4028234e38f : -INFINITY, l_run = 0.f;
   float16v o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db)
@@ -594,8 +649,8 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
-  dma(0, B0{});
-  __syncthreads();  // vmcnt(0) + barrier: every wave's part of tile 0 landed
+  dma(t0, B0{});
+  __syncthreads();  // vmcnt(0) + barrier: every wave's part of the first tile landed
   // one tile on stage BUF while the next one's DMA fills the other stage; the
   // loop is unrolled by the two stages so every LDS address is a compile-time
   // offset from `lds` -- with a runtime stage index hipcc cannot tell the
@@ -689,11 +744,27 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
     }
     __syncthreads();  // tile t+1's DMA landed (vmcnt(0)) and tile t is read by all
   };
-  for (int t = 0; t < ntiles; t += 2) {
+  for (int t = t0; t < ntiles; t += 2) {
     body(t, B0{});
     if (t + 1 < ntiles) body(t + 1, B1{});
   }
 
+  if constexpr (SPLIT) {
+    if (parts > 1) {
+      if (row_ok) {
+        const int64_t row = (blockIdx.z * part_rows + qs + qr) * hq + h;
+        float4v* orow = reinterpret_cast<float4v*>(part_o + row * D);
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+            orow[db * 8 + 2 * m + hi] = float4v{o[db][4 * m], o[db][4 * m + 1],
+                                                o[db][4 * m + 2], o[db][4 * m + 3]};
+        if (hi == 0) part_ml[row] = float2{m_run, l_run};
+      }
+      return;
+    }
+  }
   if (row_ok) {
     const float inv = 1.f / l_run;
     bf16_t* orow = out + (int64_t)(qs + qr) * out_stride + h * D;
@@ -709,6 +780,38 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
     if (lse_out && hi == 0)
       lse_out[(int64_t)(qs + qr) * hq + h] = (m_run + log2f(l_run)) * 0.6931471805599453f;
   }
+}
+
+// grid: (hq, n_tiles, 4)   block: 256.  A block sums the partitions of 8 rows of one head, 32
+// lanes a row; rows with one partition have their result already.
+__global__ __launch_bounds__(256) void prefill_merge_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ part_o,
+    const float2* __restrict__ part_ml, const int* __restrict__ q_start_loc,
+    const int* __restrict__ seq_lens, const int* __restrict__ tile_seq,
+    const int* __restrict__ tile_q0, int S, int64_t part_rows, int64_t out_stride) {
+  const int hq = gridDim.x, h = blockIdx.x, tile = blockIdx.y;
+  const int s = tile_seq[tile], q0 = tile_q0[tile];
+  const int qs = q_start_loc[s], qlen = q_start_loc[s + 1] - qs;
+  const int kv_end = seq_lens[s] - qlen + min(q0 + 32, qlen);
+  const int parts = prefill_parts((kv_end + 63) / 64, S);
+  const int qr = q0 + blockIdx.z * 8 + (threadIdx.x >> 5), c = threadIdx.x & 31;
+  if (parts <= 1 || qr >= qlen) return;
+  const int64_t row = (int64_t)(qs + qr) * hq + h, step = part_rows * hq;
+  float m = -INFINITY;
+  for (int p = 0; p < parts; ++p) m = fmaxf(m, part_ml[p * step + row].x);
+  float l = 0.f;
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) {
+    const float2 v = part_ml[p * step + row];
+    const float g = __builtin_amdgcn_exp2f(v.x - m);
+    l += g * v.y;
+    acc += reinterpret_cast<const float4v*>(part_o + (p * step + row) * D)[c] * g;
+  }
+  uint2v pk;
+  pk[0] = pack_bf2(acc[0] / l, acc[1] / l);
+  pk[1] = pack_bf2(acc[2] / l, acc[3] / l);
+  *reinterpret_cast<uint2v*>(out + (int64_t)(qs + qr) * out_stride + h * D + 4 * c) = pk;
 }
 
 }  // namespace
@@ -778,7 +881,7 @@ int omnia_decode_attention(void* out, float* part_o, float* part_ml, const void*
 #undef OMNIA_DEC_NW
 #undef OMNIA_DEC_UG
   if (max_parts > 1)
-    decode_reduce_kernel<<<B * hq, 128, 0, s>>>((bf16_t*)out, part_o, part_ml, seq_lens, hq,
+    decode_reduce_kernel<<<B * hq, 256, 0, s>>>((bf16_t*)out, part_o, part_ml, seq_lens, hq,
                                                 part_size, max_parts, split_t, split_min,
                                                 block_size);
   return (int)hipGetLastError();
@@ -789,9 +892,11 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
                             const int* seq_lens, const int* tile_seq, const int* tile_q0,
                             int n_tiles, int hq, int hkv, int head_dim, int block_size,
                             int64_t q_stride, int64_t out_stride, float scale, int hp_req, int q_tile,
-                            float* lse_out, const int* kv_lens, hipStream_t s) {
+                            float* lse_out, const int* kv_lens, float* part_o, float* part_ml, int parts,
+                            int64_t part_rows, hipStream_t s) {
   if (head_dim != 128) return -1;
   if (hq % hkv) return -2;
+  if (parts > 1 && (q_tile != 32 || lse_out || kv_lens || !part_o || !part_ml)) return -8;
   if (n_tiles == 0) return 0;
   const float scale_log2 = scale * 1.4426950408889634f;
   // heads per wave (GQA packing) and waves per block (query tile = 16 * nw rows)
@@ -803,12 +908,17 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
   if (q_tile == 32) {
     // 32-row waves, HB heads of one KV head per block (prefill_attn32_kernel)
     const int hb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-    dim3 grid32(hq / hb, n_tiles), block32(64 * hb);
+    dim3 grid32(hq / hb, n_tiles, parts > 1 ? parts : 1), block32(64 * hb);
 #define OMNIA_PRE32(BB, HH)                                                                  \
-  prefill_attn32_kernel<BB, HH><<<grid32, block32, 0, s>>>(                                  \
+  do {                                                                                       \
+    if (parts > 1) OMNIA_PRE32_S(BB, HH, true);                                              \
+    else OMNIA_PRE32_S(BB, HH, false);                                                       \
+  } while (0)
+#define OMNIA_PRE32_S(BB, HH, SS)                                                            \
+  prefill_attn32_kernel<BB, HH, SS><<<grid32, block32, 0, s>>>(                              \
       (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache,        \
       block_tables, bt_stride, q_start_loc, seq_lens, tile_seq, tile_q0, hkv, q_stride,      \
-      out_stride, scale_log2, lse_out, kv_lens)
+      out_stride, scale_log2, lse_out, kv_lens, part_o, (float2*)part_ml, part_rows)
 #define OMNIA_PRE32_HB(BB)                 \
   if (hb == 4) OMNIA_PRE32(BB, 4);         \
   else if (hb == 2) OMNIA_PRE32(BB, 2);    \
@@ -819,6 +929,11 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
     else return -3;
 #undef OMNIA_PRE32_HB
 #undef OMNIA_PRE32
+#undef OMNIA_PRE32_S
+    if (parts > 1)
+      prefill_merge_kernel<<<dim3(hq, n_tiles, 4), 256, 0, s>>>(
+          (bf16_t*)out, part_o, (const float2*)part_ml, q_start_loc, seq_lens, tile_seq, tile_q0,
+          parts, part_rows, out_stride);
     return (int)hipGetLastError();
   }
   const int nw = q_tile / 16;

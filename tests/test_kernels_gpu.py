@@ -176,6 +176,75 @@ def test_prefill_attention(bs, hq, hkv, hp, qt):
     _close(out.cpu(), exp, 0.03, 0.02)
 
 
+def _attention64(q, kc, vc, bt, qlens, lens, scale):
+    """Paged attention in float64."""
+    out, r, bs, (hkv, hq) = [], 0, kc.shape[2], (kc.shape[1], q.shape[1])
+    for i, (n, ctx) in enumerate(zip(qlens, lens)):
+        pages = bt[i, : -(-ctx // bs)].long()
+        k, v = (c[pages].transpose(1, 2).reshape(-1, hkv, 128)[:ctx].double()
+                .repeat_interleave(hq // hkv, 1) for c in (kc, vc))
+        s = (q[r:r + n].double().transpose(0, 1) @ k.permute(1, 2, 0)) * scale
+        at = torch.arange(ctx, device=q.device)
+        s.masked_fill_(at[None] > (ctx - n + torch.arange(n, device=q.device))[:, None], -math.inf)
+        out.append((s.softmax(-1) @ v.transpose(0, 1)).transpose(0, 1))
+        r += n
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("parts", [2, 3, 16])
+@pytest.mark.parametrize("hq,hkv,bs", [(32, 8, 16), (16, 8, 32), (8, 8, 64)])
+def test_prefill_attention_in_key_partitions(parts, hq, hkv, bs):
+    """Partitions that no row of a tile, some rows (the causal edge inside the tile) and all rows
+    reach; contexts of one 64-key tile and of fewer tiles than partitions; ragged query tiles."""
+    torch.manual_seed(6)
+    specs = [(1, 0), (1, 127), (33, 96), (77, 1100), (40, 216), (5, 600)]
+    lens, qlens = [q + c for q, c in specs], [q for q, _ in specs]
+    nb_total = sum((n + bs - 1) // bs for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=6)
+    bt = _tables(lens, bs, nb_total)
+    q = torch.randn(sum(qlens), hq, 128, device=DEV, dtype=torch.bfloat16)
+    qsl = torch.tensor([0, *torch.tensor(qlens).cumsum(0)], dtype=torch.int32, device=DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    tiles = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in ops.prefill_tiles(qlens, 32)]
+    one, split = (torch.full_like(q, math.nan) for _ in range(2))
+    for out, p in ((one, 1), (split, parts)):
+        ops.kernels().prefill_attention(out, q, kc, vc, bt, qsl, sl, *tiles, 128 ** -0.5, 0, 32,
+                                        None, None, p)
+    exp = _attention64(q, kc, vc, bt, qlens, lens, 128 ** -0.5)
+    errs = [(o.double() - exp).norm().item() / exp.norm().item() for o in (one, split)]
+    # P is rounded to bf16 in both; the partials are fp32
+    assert errs[1] <= 1.05 * errs[0] + 1e-4, errs
+    _close(split.cpu(), exp.cpu(), 0.03, 0.02)
+
+
+def test_prefill_partitions_only_with_few_blocks():
+    assert ops.prefill_parts(3, 32, 8, 400) == 1 < ops.prefill_parts(3, 32, 8, 2000)
+    assert ops.prefill_parts(65, 32, 8, 100000) == 1  # 520 blocks
+    assert ops.prefill_parts(1, 32, 8, 100000) == 16
+    with pytest.raises(RuntimeError):  # partials of other tiles do not exist
+        q = torch.zeros(1, 8, 128, device=DEV, dtype=torch.bfloat16)
+        kc, vc = _make_cache(1, 8, 16)
+        i = torch.zeros(1, 1, dtype=torch.int32, device=DEV)
+        ops.kernels().prefill_attention(q, q, kc, vc, i, i[0], i[0], i[0], i[0], 1.0, 0, 64, None,
+                                        None, 2)
+
+
+@pytest.mark.parametrize("parts", [2, 5, 63, 64, 65, 130])
+def test_decode_attention_merge_of_many_partitions(parts):
+    torch.manual_seed(7)
+    lens, hq, hkv, bs = [64 * parts, 64 * parts - 63, 64], 8, 2, 16
+    nb_total = sum((n + bs - 1) // bs for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=7)
+    bt = _tables(lens, bs, nb_total)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(3, hq, 128, device=DEV, dtype=torch.bfloat16)
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=64)
+    exp = _attention64(q, kc, vc, bt, [1, 1, 1], lens, 128 ** -0.5)
+    # all sums are fp32: what is left is the result's rounding to bf16
+    err = (out.double() - exp).abs()
+    assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
