@@ -590,8 +590,13 @@ __global__ __launch_bounds__(256) void blocks_kernel(float* __restrict__ rec,
 // as ND accumulator tiles (key dimensions 16 j + 4 (lane >> 4) + r in register r).  The
 // accumulator layout serves as the B operand of the next product as it stands: k-step r
 // takes dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.
+// Bound by its serial chain: a block is 104 fp32 products of one wave (heads of 128), 1.4 us, and
+// a SIMD has one wave.  Vector instructions add to that, so registers hold 2 waves' worth (with
+// more, hipcc keeps S in the accumulators' file and moves it back and forth), offsets are made
+// once, and what is not a product goes between products.  16 heads of 128 with blocks_kernel,
+// 2048 rows of 8 sequences 371 -> 330 us, 333 of 3 68 -> 61.
 template <typename T, int ND>
-__global__ __launch_bounds__(256) void scan_blocks_kernel(
+__global__ __launch_bounds__(256, ND <= 8 ? 2 : 1) void scan_blocks_kernel(
     float* __restrict__ o, float* __restrict__ state, T* __restrict__ conv_state,
     const float* __restrict__ rec, const float* __restrict__ qn, const float* __restrict__ kn,
     const T* __restrict__ vc, const T* __restrict__ x, int64_t ldx, Rows rows, int KH, int H,
@@ -624,107 +629,174 @@ __global__ __launch_bounds__(256) void scan_blocks_kernel(
   float4v kreg[NL], qreg[NL];
   T vreg[4];
   float treg[2], greg;
-  const float* R = rec + ((int64_t)rec_base(rows.q_start, s) * H + h) * kRec + tid;
+  // Vector instructions do not run beside the fp32 products, so addresses are a uniform base and
+  // an offset made once.  Loads are unconditional, so that they all are in flight together: rows
+  // past the end re-read the last one (their u is 0 whatever k, q and v hold) and columns past
+  // the head re-read its last ones (zeroed when they are used).
+  const float* R = rec + ((int64_t)rec_base(rows.q_start, s) * H + h) * kRec;
   const int64_t kofs = ((int64_t)row0 * KH + kh) * Dp;
-  const T* vp = vc + ((int64_t)row0 * H + h) * V + min(col, V - 1);
+  const T* vp = vc + ((int64_t)row0 * H + h) * V;
   const int64_t kstep = (int64_t)16 * KH * Dp, vstep = (int64_t)16 * H * V;
-  // Loads are unconditional, so that they all are in flight together: rows past the end
-  // re-read the last one (their u is 0 whatever k, q and v hold) and columns past the
-  // head re-read its last ones (zeroed when they are used).
+  const int kd4 = tid % (DW / 4) * 4, vcol = min(col, V - 1);
+  uint32_t koff[NL], voff[4];
+  auto offsets = [&](int last) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      koff[i] = min((i * 256 + tid) / (DW / 4), last) * KH * Dp + min(kd4, Dp - 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) voff[r] = min(4 * g4 + r, last) * H * V + vcol;
+  };
   auto gload = [&](int bi) {
-    const int last = min(16, n - 16 * bi) - 1;
     const float* kb = kn + kofs + bi * kstep;
     const float* qb = qn + kofs + bi * kstep;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const int e = i * 256 + tid, tt = min(e / (DW / 4), last), d4 = (e % (DW / 4)) * 4;
-      const int a = tt * KH * Dp + min(d4, Dp - 4);
-      kreg[i] = *reinterpret_cast<const float4v*>(kb + a);
-      qreg[i] = *reinterpret_cast<const float4v*>(qb + a);
+      kreg[i] = *reinterpret_cast<const float4v*>(kb + koff[i]);
+      qreg[i] = *reinterpret_cast<const float4v*>(qb + koff[i]);
     }
     const T* vb = vp + bi * vstep;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) vreg[r] = vb[min(4 * g4 + r, last) * H * V];
+    for (int r = 0; r < 4; ++r) vreg[r] = vb[voff[r]];
     const float* rr = R + (int64_t)bi * H * kRec;
-    treg[0] = rr[0];
-    treg[1] = rr[256];
-    greg = rr[512 - (tid & ~31)];  // 32 values, read by every 32 threads
+    treg[0] = rr[(uint32_t)tid];
+    treg[1] = rr[256 + (uint32_t)tid];
+    greg = rr[512 + (uint32_t)(tid & 31)];
   };
-  auto lwrite = [&](Buf& b) {
+  auto lwrite_rows = [&](Buf& b) {  // k columns past Dp hold zeros from the start
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const int e = i * 256 + tid, tt = e / (DW / 4), d4 = (e % (DW / 4)) * 4;
-      const float4v z = {0.f, 0.f, 0.f, 0.f};
-      if (16 * DW / 4 % 256 == 0 || tt < 16) {
-        *reinterpret_cast<float4v*>(b.k + tt * KS + d4) = d4 < Dp ? kreg[i] : z;
-        *reinterpret_cast<float4v*>(b.q + tt * KS + d4) = d4 < Dp ? qreg[i] : z;
+      const int tt = (i * 256 + tid) / (DW / 4);
+      if (kd4 < Dp && (16 * DW / 4 % 256 == 0 || tt < 16)) {
+        *reinterpret_cast<float4v*>(b.k + tt * KS + kd4) = kreg[i];
+        *reinterpret_cast<float4v*>(b.q + tt * KS + kd4) = qreg[i];
       }
     }
+  };
+  auto lwrite_rest = [&](Buf& b) {
     b.t[(tid >> 4) * TS + (tid & 15)] = treg[0];
     b.p[(tid >> 4) * TS + (tid & 15)] = treg[1];
-    if (tid < 32) b.g[tid] = greg;
+    b.g[tid & 31] = greg;
   };
-  gload(0);
-  lwrite(buf[0]);
   const int nblk = (n + 15) / 16;
-  float* op = o + ((int64_t)(row0 + 4 * g4) * H + h) * Vs + col;
+  float* op = o + ((int64_t)row0 * H + h) * Vs;
+  const uint32_t ooff = 4 * g4 * H * Vs + col;
   const int64_t ostep = (int64_t)16 * H * Vs;
+  // Operands in registers ahead of their products (heads up to 128; wider ones read LDS as they
+  // go): k of the next block from the middle of this one, the rest from the top of the block.
+  constexpr bool PRE = ND <= 8;
+  float4v ka[PRE ? ND : 1], qa[PRE ? ND : 1];
+  float ku[4][PRE ? ND : 1];
+  auto rows_of = [&](const float* x, int j) {
+    return *reinterpret_cast<const float4v*>(x + c16 * KS + 16 * j + 4 * g4);
+  };
+  // LDS only: the loads of later blocks stay in flight
+  auto sync = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  float4v v, vnext;
+  auto values = [&] {
+    float4v t;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] = col < V ? ldf(&vreg[r]) : 0.f;
+    return t;
+  };
+  if (Dp < DW) {
+    for (int i = tid; i < 2 * (int)sizeof(Buf) / 4; i += 256)
+      reinterpret_cast<float*>(buf)[i] = 0.f;
+    __syncthreads();
+  }
+  offsets(min(16, n) - 1);
+  gload(0);
+  lwrite_rows(buf[0]);
+  lwrite_rest(buf[0]);
+  v = values();
+  if (nblk == 2) offsets(n - 17);
+  gload(min(1, nblk - 1));
+  sync();
+  if constexpr (PRE) {
+#pragma unroll
+    for (int j = 0; j < ND; ++j) ka[j] = rows_of(buf[0].k, j);
+  }
   for (int bi = 0; bi < nblk; ++bi) {
     const Buf& B = buf[bi & 1];
-    float4v v;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = col < V ? ldf(&vreg[r]) : 0.f;
-    // one barrier per block: this block's operands are complete, and every wave is done
-    // with the buffer the next one goes to
-    __syncthreads();
-    if (bi + 1 < nblk) gload(bi + 1);
-    // every operand of the block in registers ahead of the products (heads up to 128):
-    // the serial chain then never waits on LDS
-    constexpr bool PRE = ND <= 8;
-    float4v ka[PRE ? ND : 1], qa[PRE ? ND : 1];
-    float ku[4][PRE ? ND : 1];
-    if constexpr (PRE) {
-#pragma unroll
-      for (int j = 0; j < ND; ++j) {
-        ka[j] = *reinterpret_cast<const float4v*>(B.k + c16 * KS + 16 * j + 4 * g4);
-        qa[j] = *reinterpret_cast<const float4v*>(B.q + c16 * KS + 16 * j + 4 * g4);
+    Buf& N = buf[(bi + 1) & 1];
+    float4v G, E, ta, pa;
+    float G15;
+    // what the block does beside its products, in eight pieces: the next block's operands go to
+    // the buffer that every wave left before the last barrier, the loads of the one after it
+    // (past the end: the last block's once more) are issued, this block's other operands read
+    auto piece = [&](int i) {
+      if (i == 0) lwrite_rows(N);
+      if (i == 1) {
+        lwrite_rest(N);
+        vnext = values();
       }
-    }
-    const float4v G = *reinterpret_cast<const float4v*>(B.g + 4 * g4);
-    const float4v E = *reinterpret_cast<const float4v*>(B.g + 16 + 4 * g4);
-    const float G15 = B.g[15];
-    const float4v ta = *reinterpret_cast<const float4v*>(B.t + c16 * TS + 4 * g4);
-    const float4v pa = *reinterpret_cast<const float4v*>(B.p + c16 * TS + 4 * g4);
-    if constexpr (PRE) {
+      if (i == 2) {
+        const int b = min(bi + 2, nblk - 1);
+        if (b == nblk - 1) offsets(n - 16 * b - 1);
+        gload(b);
+      }
+      if (i == 3) {
+        G = *reinterpret_cast<const float4v*>(B.g + 4 * g4);
+        E = *reinterpret_cast<const float4v*>(B.g + 16 + 4 * g4);
+        G15 = B.g[15];
+        ta = *reinterpret_cast<const float4v*>(B.t + c16 * TS + 4 * g4);
+        pa = *reinterpret_cast<const float4v*>(B.p + c16 * TS + 4 * g4);
+        if constexpr (PRE) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+          for (int j = 0; j < ND; ++j) qa[j] = rows_of(B.q, j);
+        }
+      }
+      if constexpr (PRE) {
 #pragma unroll
-        for (int j = 0; j < ND; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + 16 * j + c16];
-    }
+        for (int r = 0; r < 4; ++r)
+          if (i == 4 + r) {
+#pragma unroll
+            for (int j = 0; j < ND; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + 16 * j + c16];
+          }
+      }
+    };
     float4v ks[2], qs[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) ks[c] = qs[c] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < ND; ++j) {
-      float4v a, b;
-      if constexpr (PRE) {
-        a = ka[j];
-        b = qa[j];
-      } else {
-        a = *reinterpret_cast<const float4v*>(B.k + c16 * KS + 16 * j + 4 * g4);
-        b = *reinterpret_cast<const float4v*>(B.q + c16 * KS + 16 * j + 4 * g4);
+      const float4v a = PRE ? ka[PRE ? j : 0] : rows_of(B.k, j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ks[r & 1] = mfma4(a[r], S[j][r], ks[r & 1]);
+      if constexpr (!PRE) {
+        const float4v b = rows_of(B.q, j);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qs[r & 1] = mfma4(b[r], S[j][r], qs[r & 1]);
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        ks[r & 1] = mfma4(a[r], S[j][r], ks[r & 1]);
-        qs[r & 1] = mfma4(b[r], S[j][r], qs[r & 1]);
-      }
+      for (int i = 0; i < 8; ++i)
+        if (i * ND / 8 == j) {
+          if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
+          piece(i);
+          if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
+        }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    const float4v res = v - G * (ks[0] + ks[1]);
-    float4v u = {0.f, 0.f, 0.f, 0.f}, ov = G * (qs[0] + qs[1]);
+    if constexpr (PRE) {
+      sync();
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u = mfma4(ta[r], res[r], u);
+      for (int j = 0; j < ND; ++j) ka[j] = rows_of(N.k, j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const float4v res = v - G * (ks[0] + ks[1]);
+    float4v u = {0.f, 0.f, 0.f, 0.f};
+    // the chain of u runs between the products with q, which do not need it
+#pragma unroll
+    for (int j = 0; j < ND; ++j) {
+      if constexpr (PRE) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qs[r & 1] = mfma4(qa[j][r], S[j][r], qs[r & 1]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r * ND / 4 == j) u = mfma4(ta[r], res[r], u);
+      if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
+    }
+    float4v ov = G * (qs[0] + qs[1]);
 #pragma unroll
     for (int j = 0; j < ND; ++j) S[j] *= G15;
     const float4v ue = u * E;
@@ -735,13 +807,19 @@ __global__ __launch_bounds__(256) void scan_blocks_kernel(
       for (int j = 0; j < ND; ++j)
         S[j] = mfma4(PRE ? ku[r][PRE ? j : 0] : B.k[(4 * g4 + r) * KS + 16 * j + c16], ue[r], S[j]);
     }
-    if (bi + 1 < nblk) lwrite(buf[(bi + 1) & 1]);
+    if constexpr (!PRE) sync();
     if (col < Vs) {
       const int m = n - 16 * bi;
+      if (m >= 16) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (4 * g4 + r < m) op[bi * ostep + r * H * Vs] = ov[r];
+        for (int r = 0; r < 4; ++r) (op + bi * ostep + r * H * Vs)[ooff] = ov[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * g4 + r < m) (op + bi * ostep + r * H * Vs)[ooff] = ov[r];
+      }
     }
+    v = vnext;
   }
   if (col < Vs) {
 #pragma unroll

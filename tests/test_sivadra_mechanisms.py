@@ -254,6 +254,22 @@ def test_delta_rule(spec, how, run):
 
 
 @pytest.mark.parametrize("run", RUNS)
+@pytest.mark.parametrize("dim,vdim", [(24, 20), (64, 64), (128, 72), (136, 40)])
+def test_delta_rule_around_whole_blocks_of_tokens(dim, vdim, run):
+    """One, two and more blocks of 16 tokens, whole and ragged, as first portions and after one;
+    heads that fill their 16-column tiles and heads that do not, up to 128 and wider."""
+    lens = [1, 15, 16, 17, 31, 32, 33, 48, 49, 80]
+    mixer, w, W, want = mixer_case("delta", dict(heads=2, kv_heads=1, dim=dim, vdim=vdim, conv=4),
+                                   32, run, 9)
+    g = gen(11)
+    hs = [rnd(n + 16, 32, g=g) for n in lens]
+    steps = [[(s, n) for s, n in enumerate(lens)], [(s, 16) for s in range(len(lens))]]
+    for h, y in zip(hs, run_mixer(mixer, w, hs, steps, 16, 12)):
+        assert rel(project_out(y, w), want(h)) < (LIMIT[run[1]] if run[1] == torch.float32
+                                                  else 0.04)
+
+
+@pytest.mark.parametrize("run", RUNS)
 @pytest.mark.parametrize("a_log,bias", [(4.0, 6.0), (-8.0, -4.0), (0.0, 0.0)])
 def test_delta_rule_extreme_decay(a_log, bias, run):
     """Decays that wipe the state every token, and ones that never forget."""
