@@ -348,21 +348,21 @@ class LlamaModel(Projections):
     def decode_part(self, batch: int, max_ctx: int) -> tuple[int, int]:
         """(partition length, splits) of the split-K decode attention.
 
-        With >= DECODE_SPLIT_PAIRS (sequence, kv head) pairs the pairs alone fill
-        the chip: partitions as long as possible (fewer partials to merge, no
-        merge kernel when one partition covers the context) while keeping
-        >= ~2048 workgroups.  With fewer pairs (small batches, one KV head per TP
-        rank) every live context is cut on the device into up to ``splits``
-        equal partitions (``ops.decode_attention``), so short contexts still
-        spread over the CUs; the captured graph needs no host-known length."""
+        With >= DECODE_SPLIT_PAIRS (sequence, kv head) pairs the pairs alone give every
+        CU a block: one partition up to 2048 keys, else partitions of 1024 (fewer starts
+        and partials, but ragged ends; us at 512 / 1024 / 2048 keys, 8 KV heads: 32
+        sequences of 1000 34 / 34 / 30, 128 of 1000 117 / 108 / 103, 64 of 2000 116 / 112
+        / 109, 40 of 3500 121 / 117 / 123).  With fewer pairs (small batches, one KV head
+        per TP rank) every live context is cut on the device into up to ``splits`` equal
+        partitions (``ops.decode_attention``), so short contexts still spread over the
+        CUs; the captured graph needs no host-known length."""
         pairs = batch * self.hkv
         if 0 < pairs < DECODE_SPLIT_PAIRS:
             splits = -(-DECODE_SPLIT_PAIRS // pairs)
             splits = max(1, min(splits, -(-max_ctx // ops.DECODE_SPLIT_MIN)))
             return self.decode_part_size, splits
         part = self.decode_part_size
-        while part < 2048 and part < max_ctx and \
-                batch * self.hkv * ((max_ctx + 2 * part - 1) // (2 * part)) >= 2048:
+        while part < (2048 if max_ctx <= 2048 else 1024) and part < max_ctx:
             part *= 2
         return part, 0
 

@@ -8,7 +8,7 @@
 // decode  : split-K ("flash-decoding") over partitions of the context, GQA
 //           group of G query heads per workgroup sharing one K/V stream;
 //           Q.K^T on the MFMA (16x16x32 bf16, heads padded to 16 columns),
-//           softmax in LDS, P.V on the VALU (8 dims per lane), partitions merged
+//           P.V on the VALU with P in fp32 (8 dims per lane), partitions merged
 //           by a second tiny kernel.
 // prefill : flash-attention over (cached prefix + new tokens) with causal
 //           offset, 64 query rows x 1 head per workgroup (16 rows per wave),
@@ -39,8 +39,8 @@ constexpr int D = 128;
 // page-aligned length -- decided on the device from the live length, so a graph
 // captured once splits every context evenly (a host-chosen fixed partition
 // leaves one workgroup per (sequence, kv head) at short contexts when the batch
-// has few such pairs, e.g. one Llama-3-70B TP=8 rank).  cap (the LDS score
-// tile) and BS divide each other's multiples: pl <= cap always.
+// has few such pairs, e.g. one Llama-3-70B TP=8 rank).  cap and BS divide each
+// other's multiples: pl <= cap always.
 __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, int split_min,
                                                int bs) {
   if (split_t <= 0) return cap;
@@ -50,29 +50,26 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
   return min(pl, cap);
 }
 
-// grid: (B, Hkv, max_parts)   block: 64 * NW (NW = 2 or 4 waves)
-// UG: 16-key groups whose K loads one wave issues before its first MFMA (and,
-// for UG > 1, the first V batch is issued ahead of the softmax) -- the memory-
-// level parallelism of one workgroup, which at short contexts (one workgroup
-// streams a whole ~600-token context) sets the kernel's speed, not HBM.
-// U: V rows (16 B per lane each) one wave keeps in flight under the P.V of the
-// previous batch -- the same parallelism for phase 3.
-template <int G, int BS, int UG, int NW, int U>
-__global__ __launch_bounds__(64 * NW) void decode_attn_kernel(
+// grid: (B, Hkv, max_parts)   block: 256.  Bound by the reads of K and V.  A wave goes through
+// every fourth 16-key group by itself, with its own running max: K and V of the next group are
+// loaded while this one's scores, softmax and P.V are computed, so that memory never waits for a
+// phase of the block, and the waves meet once at the end.  3 waves a SIMD: groups of 32 keys take
+// the registers of 2, and short contexts 50 us where these take 39; 4 spill.  us with scores,
+// softmax and P.V as phases of the block -> now (32 heads on 8; sequences x keys): 256 x 576
+// 127 -> 119 (5.1 TB/s), 128 x 1000 111 -> 104, 64 x 2000 115 -> 112, 32 x 1000 33.7 -> 29.3,
+// 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.
+constexpr int NW = 4;
+template <int G, int BS>
+__global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ seq_lens,
     int hkv, int64_t q_stride, int part_size, int max_parts, float scale_log2, int split_t,
     int split_min) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* stat = reinterpret_cast<float*>(smem);                    // [2*G] (padded to 16 floats)
-  float* scores = stat + 16;                                       // [G][part_size]
-  // [NW][G][D] wave partials of P.V: aliases `scores` (written after every wave's
-  // last scores read), so a workgroup holds one [G][part_size] score tile
-  float* red = scores;
-  int* pages = reinterpret_cast<int*>(scores + (G * part_size > NW * G * D ? G * part_size
-                                                                            : NW * G * D));
-
+  __shared__ __attribute__((aligned(16))) float pb[NW][16][G];  // a group's P, wave-private
+  __shared__ __attribute__((aligned(16))) float al[NW][G];
+  __shared__ __attribute__((aligned(16))) float red[NW][G][D];
+  __shared__ float ml[NW][G][2];
   const int b = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
   const int len = seq_lens[b];
   if (len <= 0) return;
@@ -81,145 +78,149 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(
   if (p0 >= len) return;
   const int n = min(pl, len - p0);
   const int nparts = (len + pl - 1) / pl;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int h0 = kvh * G;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h0 = kvh * G, c16 = lane & 15, g4 = lane >> 4;
+  const int* bt = block_tables + (int64_t)b * bt_stride + p0 / BS;
 
-  for (int i = tid; i < (n + BS - 1) / BS; i += 64 * NW)
-    pages[i] = block_tables[(int64_t)b * bt_stride + p0 / BS + i];
-
-  // Q^T as the MFMA B operand: column = head (l&15, only < G real), k = dims
+  // Q^T as the MFMA B operand: column = head (c16, only < G real), k = dims
   short8 qf[4];
   {
-    const int g = lane & 15;
-    const int hh = h0 + (g < G ? g : 0);
-    const bf16_t* qrow = q + (int64_t)b * q_stride + hh * D;
+    const bf16_t* qrow = q + (int64_t)b * q_stride + (h0 + (c16 < G ? c16 : 0)) * D;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      short8 v = *reinterpret_cast<const short8*>(qrow + kk * 32 + 8 * (lane >> 4));
-      if (g >= G) v = short8{0, 0, 0, 0, 0, 0, 0, 0};
+      short8 v = *reinterpret_cast<const short8*>(qrow + kk * 32 + 8 * g4);
+      if (c16 >= G) v = short8{0, 0, 0, 0, 0, 0, 0, 0};
       qf[kk] = v;
     }
   }
-  __syncthreads();
-
-  // ---- phase 1: scores. each wave takes 16-key groups round-robin, UG per
-  // pass with all their K loads in flight before the first MFMA (groups past
-  // the end re-read the last key: branch-free, hits in cache).
-  const int ngroups = (n + 15) / 16;
-  for (int grp0 = w; grp0 < ngroups; grp0 += NW * UG) {
-    short8 a[UG][4];
+  // K rows as the A operand (row = key c16 of the group); V: lane = (token g4 of 4, dims 8 c16
+  // ..).  A group lies in one page; rows past the end re-read the last one.
+  struct Group {
+    short8 k[4], v[4];
+  };
+  const int ngr = (n + 15) / 16, last = n - 1;
+  auto page = [&](int c) { return bt[min(c * 16, last) / BS]; };  // past the end: the last page
+  auto load = [&](Group& t, int c, int pg) {
+    const int k0 = min(c * 16, last & ~15), top = last - k0;
+    const int64_t base = (((int64_t)pg * hkv + kvh) * BS + k0 % BS) * D;
+    const bf16_t *kb = kc + base, *vb = vc + base;
+    const uint32_t ko = min(c16, top) * D + 8 * g4;
 #pragma unroll
-    for (int u = 0; u < UG; ++u) {
-      const int key = (grp0 + NW * u) * 16 + (lane & 15);  // this lane's A-row key
-      const int kk_ = min(key, n - 1);
-      const int tok = p0 + kk_;
-      const bf16_t* krow = kc + (((int64_t)pages[kk_ / BS] * hkv + kvh) * BS + (tok % BS)) * D;
+    for (int kk = 0; kk < 4; ++kk)
+      t.k[kk] = *reinterpret_cast<const short8*>(kb + ko + kk * 32);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
-        a[u][kk] = *reinterpret_cast<const short8*>(krow + kk * 32 + 8 * (lane >> 4));
-    }
-#pragma unroll
-    for (int u = 0; u < UG; ++u) {
-      const int grp = grp0 + NW * u;
-      if (grp >= ngroups) break;
-      float4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) acc = mfma16(a[u][kk], qf[kk], acc);
-      // acc[r] = S^T[key grp*16 + 4*(lane>>4) + r][head lane&15]
-      const int g = lane & 15;
-      if (g < G) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kidx = grp * 16 + 4 * (lane >> 4) + r;
-          if (kidx < n) scores[g * part_size + kidx] = acc[r] * scale_log2;
-        }
-      }
-    }
-  }
-  // first V batch of phase 3 in flight across the softmax (plain loads survive
-  // the barriers); lane = (token sub-index tg = lane>>4, dim chunk ch = lane&15)
-  const int tg = lane >> 4, ch = lane & 15;
-  short8 vv[U];
-  auto vload = [&](int base) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = min(base + u * 4 * NW + tg, n - 1);
-      const int tok = p0 + t;
-      vv[u] = *reinterpret_cast<const short8*>(
-          vc + (((int64_t)pages[t / BS] * hkv + kvh) * BS + (tok % BS)) * D + ch * 8);
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t vo = min(4 * i + g4, top) * D + 8 * c16;
+      t.v[i] = *reinterpret_cast<const short8*>(vb + vo);
     }
   };
-  if (UG > 1) vload(w * 4);
-  __syncthreads();
-
-  // ---- phase 2: softmax per head (wave w handles heads w, w+NW, ...)
-  for (int g = w; g < G; g += NW) {
-    float m = -INFINITY;
-    for (int i = lane; i < n; i += 64) m = fmaxf(m, scores[g * part_size + i]);
-    m = wave_max(m);
-    float s = 0.f;
-    for (int i = lane; i < n; i += 64) {
-      const float p = exp2f(scores[g * part_size + i] - m);
-      scores[g * part_size + i] = p;
-      s += p;
-    }
-    s = wave_sum(s);
-    if (lane == 0) {
-      stat[2 * g] = m;
-      stat[2 * g + 1] = s;
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 3: P.V. lane = (token sub-index tg = lane>>4, dim chunk ch = lane&15)
+  float m_run = -INFINITY, l_run = 0.f;  // of head c16
   float acc[G][8];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  for (int base = w * 4; base < n; base += 4 * NW * U) {
-    if (UG == 1) vload(base);
-    short8 cur[U];
+  auto compute = [&](const Group& t, int c) {
+    float4v sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < U; ++u) cur[u] = vv[u];
-    if (UG > 1) vload(base + 4 * NW * U);  // next batch (clamped past the end)
+    for (int kk = 0; kk < 4; ++kk) sc = mfma16(t.k[kk], qf[kk], sc);
+    // sc[r]: key 4 g4 + r of the group, head c16
+    const int top = n - c * 16 - 4 * g4;
+    float m = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int ti = base + u * 4 * NW + tg;
-      if (ti < n) {
+    for (int r = 0; r < 4; ++r) {
+      sc[r] = r < top ? sc[r] * scale_log2 : -INFINITY;
+      m = fmaxf(m, sc[r]);
+    }
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    // the maximum moves only when a head's grows by more than 2^8: P and its sums are fp32
+    const bool grow = m > m_run + 8.f;
+    const bool any = __builtin_amdgcn_ballot_w64(grow) != 0;
+    if (any) {
+      const float m_new = grow ? m : m_run;
+      const float a = exp2f(m_run - m_new);
+      l_run *= a;
+      m_run = m_new;
+      if (lane < G) al[w][lane] = a;
+    }
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float p = scores[g * part_size + ti];
+    for (int r = 0; r < 4; ++r) {
+      const float p = exp2f(sc[r] - m_run);
+      l_run += p;
+      if (c16 < G) pb[w][4 * g4 + r][c16] = p;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (any) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) acc[g][j] += p * bf2f((uint16_t)cur[u][j]);
-        }
+      for (int g = 0; g < G; ++g) {
+        const float a = al[w][g];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[g][j] *= a;
       }
     }
-  }
-  // reduce over the 4 token sub-lanes of the wave (tokens of wave w: w*4 + tg mod 4*NW)
 #pragma unroll
-  for (int g = 0; g < G; ++g)
+    for (int i = 0; i < 4; ++i) {
+      float p[G];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = acc[g][j];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      acc[g][j] = v;
+      for (int g = 0; g < G; ++g) p[g] = pb[w][4 * i + g4][g];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = bf2f((uint16_t)t.v[i][j]);
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][j] += p[g] * v;
+      }
     }
-  __syncthreads();  // every wave is done reading `scores`, which `red` overlays
-  if (tg == 0) {
+    __builtin_amdgcn_wave_barrier();
+  };
+  if (w < ngr) {
+    Group t0, t1;
+    load(t0, w, page(w));
+    int pg = page(w + NW);
+    for (int c = w; c < ngr; c += 2 * NW) {
+      load(t1, c + NW, pg);
+      pg = page(c + 2 * NW);
+      compute(t0, c);
+      load(t0, c + 2 * NW, pg);
+      pg = page(c + 3 * NW);
+      if (c + NW < ngr) compute(t1, c + NW);
+    }
+  }
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (lane < G) {
+    ml[w][lane][0] = m_run;
+    ml[w][lane][1] = l_run;
+  }
+  // over the 4 tokens of a V instruction: lane group g4 ends with two of the 8 dims, half of
+  // what a step leaves going to the other lanes
+  const bool hi = lane >= 32, mid = g4 & 1;
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+  for (int g = 0; g < G; ++g) {
+    float r[4], t[2];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) red[(w * G + g) * D + ch * 8 + j] = acc[g][j];
+    for (int j = 0; j < 4; ++j)
+      r[j] = (hi ? acc[g][4 + j] : acc[g][j]) + __shfl_xor(hi ? acc[g][j] : acc[g][4 + j], 32, 64);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      t[j] = (mid ? r[2 + j] : r[j]) + __shfl_xor(mid ? r[j] : r[2 + j], 16, 64);
+    *reinterpret_cast<float2*>(&red[w][g][c16 * 8 + g4 * 2]) = float2{t[0], t[1]};
   }
   __syncthreads();
   for (int i = tid; i < G * D; i += 64 * NW) {
     const int g = i / D, d = i % D;
-    float v = 0.f;
+    float m = ml[0][g][0];
 #pragma unroll
-    for (int wi = 0; wi < NW; ++wi) v += red[(wi * G + g) * D + d];
-    const float inv = 1.f / stat[2 * g + 1];
+    for (int wi = 1; wi < NW; ++wi) m = fmaxf(m, ml[wi][g][0]);
+    float v = 0.f, l = 0.f;
+#pragma unroll
+    for (int wi = 0; wi < NW; ++wi) {
+      const float e = exp2f(ml[wi][g][0] - m);
+      v += e * red[wi][g][d];
+      l += e * ml[wi][g][1];
+    }
+    const float inv = 1.f / l;
     const int h = h0 + g;
     if (nparts == 1) {
       out[((int64_t)b * gridDim.y * G + h) * D + d] = f2bf(v * inv);
@@ -227,8 +228,8 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(
       const int64_t slot = ((int64_t)b * gridDim.y * G + h) * max_parts + part;
       part_o[slot * D + d] = v * inv;
       if (d == 0) {
-        part_ml[slot * 2] = stat[2 * g];
-        part_ml[slot * 2 + 1] = stat[2 * g + 1];
+        part_ml[slot * 2] = m;
+        part_ml[slot * 2 + 1] = l;
       }
     }
   }
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(
 
 // grid: (B * Hq)   block: 256.  Latency bound: a lane takes one partition's (m, l) of each 64 and
 // the four waves take every fourth partition's row, with the loads of several in flight (one
-// after the other, a 2000-key sequence in 32 partitions took 20.3 us with its attention, now 12.9).
+// after the other, a 2000-key sequence in 32 partitions took 20.3 us with its attention, with this 12.9).
 __global__ __launch_bounds__(256) void decode_reduce_kernel(
     bf16_t* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_ml,
     const int* __restrict__ seq_lens, int hq, int part_size, int max_parts, int split_t,
@@ -831,41 +832,12 @@ int omnia_decode_attention(void* out, float* part_o, float* part_ml, const void*
   if (B == 0) return 0;
   const int G = hq / hkv;
   const float scale_log2 = scale * 1.4426950408889634f;
-  // OMNIA_DECODE_UG = 1 / 8 selects the single-group / 8-group K schedule
-  // (A/B measurements; read per call)
-  const char* ug_e = getenv("OMNIA_DECODE_UG");
-  const int ug = ug_e && atoi(ug_e) == 1 ? 1 : (ug_e && atoi(ug_e) == 8 ? 8 : 4);
-  // waves per workgroup: with many (sequence, kv head, partition) workgroups a
-  // 4-wave group (90+ VGPRs -> 5 groups per CU) leaves ~2048 groups in two
-  // uneven rounds; 2-wave groups keep every group of a 256-sequence batch
-  // resident at once (16 waves / CU, one score tile of LDS each) and stream
-  // the same bytes with the whole batch's loads in flight.  OMNIA_DECODE_NW
-  // = 2 / 4 forces one (A/B, and the numerics tests cover both; read per call).
-  const char* nw_e = getenv("OMNIA_DECODE_NW");
-  const int nw_env = nw_e ? atoi(nw_e) : 0;
-  const int64_t groups = (int64_t)B * hkv * max_parts;
-  const int nw = nw_env == 2 || nw_env == 4 ? nw_env : (groups >= 1024 ? 2 : 4);
-  // V rows in flight per lane in phase 3 (OMNIA_DECODE_U = 4 / 8, read per call)
-  const char* u_e = getenv("OMNIA_DECODE_U");
-  const int uv = u_e && atoi(u_e) == 8 ? 8 : 4;
-  dim3 grid(B, hkv, max_parts), block(64 * nw);
-  const size_t tile = (size_t)G * part_size > (size_t)nw * G * D ? (size_t)G * part_size
-                                                                  : (size_t)nw * G * D;
-  const size_t lds = 64 + tile * 4 + (part_size / block_size) * 4;
-#define OMNIA_DEC_UG(GG, BB, UU, NN, VV)                                                       \
-  decode_attn_kernel<GG, BB, UU, NN, VV><<<grid, block, lds, s>>>(                            \
-      (bf16_t*)out, part_o, part_ml, (const bf16_t*)q, (const bf16_t*)k_cache,               \
-      (const bf16_t*)v_cache, block_tables, bt_stride, seq_lens, hkv, q_stride, part_size,   \
+  dim3 grid(B, hkv, max_parts);
+#define OMNIA_DEC(GG, BB)                                                                      \
+  decode_attn_kernel<GG, BB><<<grid, 64 * NW, 0, s>>>(                                         \
+      (bf16_t*)out, part_o, part_ml, (const bf16_t*)q, (const bf16_t*)k_cache,                 \
+      (const bf16_t*)v_cache, block_tables, bt_stride, seq_lens, hkv, q_stride, part_size,     \
       max_parts, scale_log2, split_t, split_min)
-#define OMNIA_DEC_NW(GG, BB, UU, VV) \
-  do { if (nw == 2) OMNIA_DEC_UG(GG, BB, UU, 2, VV); else OMNIA_DEC_UG(GG, BB, UU, 4, VV); } while (0)
-#define OMNIA_DEC(GG, BB)                          \
-  do {                                             \
-    if (ug == 1) OMNIA_DEC_NW(GG, BB, 1, 4);       \
-    else if (ug == 8) OMNIA_DEC_NW(GG, BB, 8, 8);  \
-    else if (uv == 8) OMNIA_DEC_NW(GG, BB, 4, 8);  \
-    else OMNIA_DEC_NW(GG, BB, 4, 4);               \
-  } while (0)
 #define OMNIA_DEC_BS(GG)                                \
   if (block_size == 16) OMNIA_DEC(GG, 16);              \
   else if (block_size == 32) OMNIA_DEC(GG, 32);         \
@@ -878,8 +850,6 @@ int omnia_decode_attention(void* out, float* part_o, float* part_ml, const void*
   else return -4;
 #undef OMNIA_DEC_BS
 #undef OMNIA_DEC
-#undef OMNIA_DEC_NW
-#undef OMNIA_DEC_UG
   if (max_parts > 1)
     decode_reduce_kernel<<<B * hq, 256, 0, s>>>((bf16_t*)out, part_o, part_ml, seq_lens, hq,
                                                 part_size, max_parts, split_t, split_min,

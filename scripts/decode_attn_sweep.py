@@ -5,18 +5,14 @@ partition-merge kernel included.  The K+V stream (>= 545 MB) exceeds the
 256 MB Infinity Cache, so back-to-back runs read HBM (no flush kernel: its
 dirty lines would be written back under the measured kernel).
 
-    python scripts/decode_attn_sweep.py [--nw 2,4] [--parts 256,512,1024]
+    python scripts/decode_attn_sweep.py [--parts 256,512,1024]
     python scripts/decode_attn_sweep.py --batch 128 --hq 64   # Llama-3-70B, TP=1
     python scripts/decode_attn_sweep.py --hq 8 --hkv 1        # one Llama-3-70B TP=8 rank
 
 Rows ``mix`` draw every sequence's length uniformly from 513..640, as in a
 closed-loop wave (the partition split then varies per sequence).
-
-``--nw`` runs each shape with the 2- and the 4-wave workgroup
-(``OMNIA_DECODE_NW``, read per launch) and checks them against each other.
 """
 import argparse
-import os
 import sys
 import time
 
@@ -28,10 +24,7 @@ from omnia_amd import ops  # noqa: E402
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--nw", default="0")
     ap.add_argument("--parts", default="128,192,256,320,384,512,640,1024")
-    ap.add_argument("--u", default="4", help="V rows in flight per lane (OMNIA_DECODE_U); "
-                    "g8 = 8 K groups and 8 V rows (OMNIA_DECODE_UG=8)")
     ap.add_argument("--splits", default="0",
                     help="0 = fixed partitions of --parts keys; n > 0 = length-balanced "
                          "split into up to n partitions (--parts is then the cap)")
@@ -39,7 +32,6 @@ def main():
     ap.add_argument("--hq", type=int, default=32)
     ap.add_argument("--hkv", type=int, default=8, help="1 = a Llama-3-70B TP=8 shard")
     a = ap.parse_args()
-    nws = [int(x) for x in a.nw.split(",")]
     parts = [int(x) for x in a.parts.split(",")]
     torch.manual_seed(0)
     dev = "cuda"
@@ -57,7 +49,7 @@ def main():
     bt = perm.view(B, mb).contiguous()
     q = torch.randn(B, hq, D, device=dev, dtype=torch.bfloat16)
     scale = D ** -0.5
-    print(f"{'len':>5} {'part':>5} {'sp':>3} {'nw':>3} {'u':>2} {'us':>8} {'TB/s':>6}  err", flush=True)
+    print(f"{'len':>5} {'part':>5} {'sp':>3} {'us':>8} {'TB/s':>6}  err", flush=True)
     for L in (520, 576, 640, "mix"):
         if L == "mix":
             g = torch.Generator().manual_seed(1)
@@ -65,14 +57,7 @@ def main():
         else:
             sl = torch.full((B,), L, dtype=torch.int32, device=dev)
         ref = None
-        for part, nw, uv, sp in [(p, w, u, int(x)) for p in parts for w in nws
-                                 for u in a.u.split(",") for x in a.splits.split(",")]:
-            os.environ["OMNIA_DECODE_U"] = "8" if uv == "g8" else uv
-            os.environ["OMNIA_DECODE_UG"] = "8" if uv == "g8" else "4"
-            if nw:
-                os.environ["OMNIA_DECODE_NW"] = str(nw)
-            else:
-                os.environ.pop("OMNIA_DECODE_NW", None)
+        for part, sp in [(p, int(x)) for p in parts for x in a.splits.split(",")]:
             ws = ops.decode_workspace(B, hq, mb, BS, part, dev, sp)
             out = ops.decode_attention(q, kc, vc, bt, sl, scale, part_size=part, workspace=ws,
                                        splits=sp)
@@ -91,7 +76,7 @@ def main():
             ts.sort()
             us = ts[len(ts) // 2]
             nbytes = int(sl.sum().item()) * hkv * D * 2 * 2
-            print(f"{L!s:>5} {part:5d} {sp:3d} {nw:3d} {uv:>2} {us:8.1f} {nbytes / us / 1e6:6.2f}  {err:.2e}", flush=True)
+            print(f"{L!s:>5} {part:5d} {sp:3d} {us:8.1f} {nbytes / us / 1e6:6.2f}  {err:.2e}", flush=True)
     time.sleep(0.1)
 
 

@@ -245,6 +245,30 @@ def test_decode_attention_merge_of_many_partitions(parts):
     assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
 
 
+@pytest.mark.parametrize("hq,hkv,bs", [(4, 4, 16), (8, 4, 64), (32, 8, 16), (16, 2, 32)])
+def test_decode_attention_around_whole_key_groups(hq, hkv, bs):
+    """Waves with no, one and several 16-key groups, ragged last groups, scores whose maximum
+    keeps growing along the keys (the running maximum moves) and falls."""
+    torch.manual_seed(8)
+    lens = [1, 15, 16, 17, 48, 63, 64, 65, 127, 129, 1000]
+    nb_total = sum((n + bs - 1) // bs for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=8)
+    bt = _tables(lens, bs, nb_total)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(len(lens), hq, 128, device=DEV, dtype=torch.bfloat16)
+    q[:, ::2], kc[..., 0] = q[:, ::2].abs(), 0  # dimension 0 carries the slope
+    q[..., 0] = torch.where(torch.arange(hq, device=DEV) % 2 == 0, 16.0, -16.0)
+    for i, n in enumerate(lens):
+        for p in range(-(-n // bs)):
+            kc[bt[i, p].long(), :, :, 0] = (torch.arange(bs, device=DEV) + p * bs).bfloat16() / 8
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=1024)
+    exp = _attention64(q, kc, vc, bt, [1] * len(lens), lens, 128 ** -0.5)
+    # scores up to 250 carry an fp32 error of 250 * 2^-23 into the exponent; the rest is the
+    # result's rounding to bf16
+    err = (out.double() - exp).abs()
+    assert (err <= exp.abs() * 2.0 ** -8 + 2e-4 * vc.abs().max()).all(), err.max()
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
