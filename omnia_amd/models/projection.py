@@ -185,12 +185,14 @@ class Projections:
     def _pgemm_ok(self, M: int, K: int, N: int, is_decode: bool, tn: int = 256) -> bool:
         """A prefill-sized projection the hand 256x256 MFMA kernel covers (the
         unfused paths: TP shards, MoE attention, CP): K whole 128-k iterations,
-        N whole column tiles, and at least this forward's row threshold."""
+        N whole column tiles, and at least this forward's row threshold, or for a
+        gated one (tn 128) tiles that fill the chip."""
         # TP ranks rehearsed on ONE device (ipc transport) keep the library GEMMs:
         # a 256x256 tile's 132 KB of LDS cannot share a CU with the peers'
         # spinning all-reduce blocks, so a rank's GEMM can wait out their spin
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
+        rows = M >= self._min_rows or (tn == 128 and ops.gated_tile_fills(M, N))
         return (self.use_pgemm and not is_decode and self.device.type == "cuda"
                 and self.dtype == torch.bfloat16
-                and M >= self._min_rows and K % 128 == 0 and N % tn == 0
+                and rows and K % 128 == 0 and N % tn == 0
                 and (self.tp == 1 or pstate.ranks_per_device() == 1))

@@ -440,6 +440,17 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     return out
 
 
+def gated_tile_fills(M: int, N: int) -> bool:
+    """Whether the 256 x 128-feature tiles of a gated :func:`pgemm` of more rows than the panel
+    kernel takes are worth their rounds over 256 CUs: from three quarters of their work useful,
+    the activation in the epilogue makes up for the rest (useful part, us here / library and
+    activation kernel; 8192 features of 2048: 512 rows .50 48 / 42, 768 .75 51.5 / 52.7, 999 .98
+    55 / 67, 1536 .75 99 / 99, 2001 .98 108 / 124; 14336 of 4096: 320 .55 93 / 88, 512 .88 99 / 112,
+    768 .66 177 / 163, 999 .85 187 / 198)."""
+    rounds = -(-(-(-M // 256) * (N // 128)) // 256)
+    return M > PANEL_MAX_M and M * N > 0.75 * 256 * 256 * 128 * rounds
+
+
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
                  sched: int = 0) -> torch.Tensor:
     """fp16 split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the 256x256 MFMA tile

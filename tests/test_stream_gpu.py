@@ -255,3 +255,26 @@ def test_llama_layers_match_the_unfused_path(rows, pack, monkeypatch):
     a, b = run(True), run(False)
     for x, y in zip(a.values(), b.values()):
         assert (x - y).norm() <= 0.02 * y.norm()
+
+
+def test_gated_tiles_are_taken_where_they_fill_the_chip():
+    assert [m for m in (256, 512, 768, 769, 1024, 1025, 1536, 1537, 2048)
+            if ops.gated_tile_fills(m, 8192)] == [769, 1024, 1537, 2048]
+    assert [m for m in (320, 439, 440, 512, 513, 878, 879, 1024)
+            if ops.gated_tile_fills(m, 14336)] == [439, 440, 512, 878, 879, 1024]
+
+
+@pytest.mark.parametrize("M", [511, 512, 513])
+def test_gated_projection_on_both_sides_of_the_rule(M):
+    """32768 features: two rows of 256 tiles up to 512 rows, half-empty third ones after."""
+    from omnia_amd.models.projection import Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device("cuda"), torch.bfloat16, 1, {}
+
+    m, N, K = Model(), 32768, 128
+    assert m._pgemm_ok(M, K, N, False, 128) == (M <= 512)
+    assert not m._pgemm_ok(M, K, N, False) and not m._pgemm_ok(M, K, N, True, 128)
+    x, w = _mk(M, 2 * N, K, 5)
+    g, u = (x.double() @ w.double().t()).split(N, 1)
+    _close(ops.pgemm(1, x, w), F.silu(g) * u, K)
