@@ -933,11 +933,13 @@ def cosine_topk(q: torch.Tensor, m: torch.Tensor, k: int, valid: torch.Tensor | 
 # ------------------------------------------------------------- MoE (K14)
 MOE_LIBRARY_ROWS = 1024  # mean rows/expert above which eager calls use hipBLASLt per expert
 # mean rows per local expert from which the grouped GEMMs run on the 256x256
-# prefill tile (pgemm.hip EPI 5 / 6, 256-row expert segments); below it the
-# 64-row grouped kernels (moe.hip) waste less padding.  Both are graph-safe.
+# prefill tile (pgemm.hip EPI 5 / 6, 256-row expert segments); below it smaller
+# segments (moe_panel_rows) waste less padding.  All are graph-safe.
 # Both products, 64-row / 256-row: at 96 rows 164 / 204 us, at 128 213 / 208, at 512
 # 652 / 268 (8 experts of 2048 x 4096); at 96 174 / 190, at 128 202 / 193 (32 of 2048 x
-# 1024); wide experts cross earlier, at 64 803 / 791 (8 of 4096 x 14336)
+# 1024).  128-row / 256-row: at 128 141 / 199, at 160 173 / 201, at 256 245 / 208 (the first);
+# at 128 169 / 183, at 188 215 / 193 (the second); at 128 830 / 858, at 160 1069 / 869 (8 of
+# 4096 x 14336): it crosses between 128 and 230
 MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
 
 
@@ -955,6 +957,25 @@ def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor
             and all(w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down)))
 
 
+def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
+                   packed: bool) -> int:
+    """Segment rows of the panel kernel for ``n`` assignments to ``experts`` local experts, 0
+    where moe.hip's 64-row kernel does better.
+
+    From 56 rows an expert most would need two segments of 64, so the weights are read twice;
+    segments of 128 read them once (both products, us, 64-row kernel / 128-row segments at 64 / 100 / 128
+    rows: 8 experts of 2048 x 4096 122 / 156 / 196 and 109 / 114 / 141, of 4096 x 14336 798 / 1049
+    / 1296 and 547 / 588 / 830; 32 of 2048 x 1024 135 / 167 / 194 and 126 / 133 / 175).  Fewer rows
+    gain from whole-line reads of packed weights where K is long (8 to 32 rows, 64-row kernel /
+    64-row segments: 94 / 84, 494 / 445; 32 of 2048 x 1024 90 / 96)."""
+    if not (_stream_on and w_up.dtype == torch.bfloat16 and w_up.is_cuda and all(
+            w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down))):
+        return 0
+    if n >= 56 * experts:
+        return 128
+    return 64 if packed and min(w_up.shape[2], w_down.shape[2]) >= 2048 else 0
+
+
 def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=None,
                  gelu: bool = False, streams=None):
     """Grouped expert FFN over device-sorted assignments, no host sync: Y [T*k, d]
@@ -962,13 +983,17 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     unwritten).  ``bm`` 256: the 256x256 MFMA prefill tile; 64: moe.hip.  ``glu`` =
     (alpha, limit): clamped GLU experts whose INPUT takes the routing weight; ``gelu``:
     ungated experts (``w_gu`` [E, I, d]).  ``streams``: packed copies (:func:`stream_pack`) of
-    both weights, or None; few assignments run :func:`moe_stream_ok`'s kernel in place of
-    ``bm`` 64."""
+    both weights, or None; in place of ``bm`` 64, few assignments run :func:`moe_stream_ok`'s
+    kernel and others :func:`moe_panel_rows`'s."""
     kk = kernels()
     n, experts = ids.numel(), e_hi - e_lo
     few = bm == 64 and moe_stream_ok(n, experts, w_gu, w_down, streams is not None)
+    panel = 0
     if few:
         bm = 16
+    elif bm == 64:
+        panel = moe_panel_rows(n, experts, w_gu, w_down, streams is not None)
+        bm = panel or bm
     mb = kk.moe_max_blocks(n, experts, bm)
     sorted_ids = torch.empty(mb * bm, dtype=torch.int32, device=x.device)
     blk = torch.empty(mb, dtype=torch.int32, device=x.device)
@@ -986,6 +1011,16 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
                 w = streams[mode == 1]
             kk.stream_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, frags, streams is not None,
                           alpha, limit)
+
+    elif panel:
+        segs = experts * -(-5 * n // (4 * experts * panel))  # live ones, about
+
+        def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
+            wn = panel_plan(panel, w.shape[1] * segs, w.shape[2], False)[0]
+            if streams is not None:
+                w = streams[mode == 1]
+            kk.panel_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, wn, streams is not None,
+                         alpha, limit)
 
     if glu is not None:
         gemm(2, act, x, w_gu, sorted_ids, blk, nblk, wts.view(-1), k, n, e_lo, *glu)

@@ -133,6 +133,10 @@ int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const in
                      const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                      int N, int topk, int n_assign, int e_lo, int max_blocks, int nw, int packed,
                      float alpha, float limit, hipStream_t s);
+int omnia_panel_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
+                    const int* blk_expert, const int* n_blocks, const float* route_w, int K, int N,
+                    int topk, int n_assign, int e_lo, int max_blocks, int bm, int wn, int packed,
+                    float alpha, float limit, hipStream_t s);
 int omnia_dgemm(int mode, void* out, const void* X, const void* W, float* ws, int* cnt, int M,
                 int N, int K, int S, int wm, int wn, int ldo, int64_t ws_floats, int cnt_len,
                 hipStream_t s);
@@ -654,7 +658,7 @@ int64_t moe_max_blocks(int64_t n_assign, int64_t n_experts, int64_t bm) {
 }
 
 // segments aligned to bm = sorted.numel() / blk_expert.numel() rows (16: stream_moe,
-// 64: moe_gemm, 256: the pgemm_moe prefill tile)
+// 64 and 128: panel_moe, 64: moe_gemm, 256: the pgemm_moe prefill tile)
 void moe_align(at::Tensor sorted, at::Tensor blk_expert, at::Tensor n_blocks, at::Tensor ids,
                int64_t E, int64_t e_lo, int64_t e_hi) {
   CHECK_GPU(ids); CHECK_I32(ids); CHECK_I32(sorted); CHECK_I32(blk_expert); CHECK_I32(n_blocks);
@@ -662,7 +666,7 @@ void moe_align(at::Tensor sorted, at::Tensor blk_expert, at::Tensor n_blocks, at
   const int mb = blk_expert.numel();
   TORCH_CHECK(mb > 0 && sorted.numel() % mb == 0, "sorted must hold max_blocks segments");
   const int bm = (int)(sorted.numel() / mb);
-  TORCH_CHECK(bm == 16 || bm == 64 || bm == 256, "segments of 16, 64 or 256 rows");
+  TORCH_CHECK(bm == 16 || bm == 64 || bm == 128 || bm == 256, "segments of 16 to 256 rows");
   TORCH_CHECK(mb >= omnia_moe_max_blocks(n, e_hi - e_lo, bm), "blk_expert too small");
   TORCH_CHECK(E <= 256 && 0 <= e_lo && e_lo < e_hi && e_hi <= E, "expert range");
   CHECK_RC(omnia_moe_align(sorted.data_ptr<int>(), blk_expert.data_ptr<int>(),
@@ -767,7 +771,7 @@ void moe_gemm(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tens
 }
 
 // moe_gemm's modes for segments of 16 rows (stream.hip)
-void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
+static void few_moe(bool panel, int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
                 at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
                 int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
                 double alpha, double limit) {
@@ -780,8 +784,8 @@ void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Te
     TORCH_CHECK(t->device() == A.device(), "same device");
   const int K = W.size(2);
   const int mb = blk_expert.numel();
-  constexpr int seg = 16;
-  TORCH_CHECK(sorted.numel() == (int64_t)mb * seg, "sorted must hold max_blocks*16 rows");
+  const int seg = panel ? (int)(mb > 0 ? sorted.numel() / mb : 0) : 16;
+  TORCH_CHECK(sorted.numel() == (int64_t)mb * seg, "sorted must hold max_blocks segments");
   TORCH_CHECK(A.size(1) == K, "K mismatch");
   if (route_w.has_value())
     TORCH_CHECK(route_w->device() == A.device() && route_w->is_contiguous() &&
@@ -798,12 +802,32 @@ void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Te
     TORCH_CHECK(out.size(0) == n_assign && out.size(1) == N, "Y [T*k, d]");
     TORCH_CHECK(A.size(0) == (int64_t)mb * seg, "act rows");
   }
-  CHECK_RC(omnia_stream_moe((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(),
-                            sorted.data_ptr<int>(), blk_expert.data_ptr<int>(),
-                            n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N, topk,
-                            n_assign, e_lo, mb, (int)nw, packed, (float)alpha, (float)limit,
-                            cur_stream()),
-           "stream_moe");
+  const auto run = [&](auto f, auto... shape) {
+    return f((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(), sorted.data_ptr<int>(),
+             blk_expert.data_ptr<int>(), n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N,
+             (int)topk, (int)n_assign, (int)e_lo, mb, shape..., (int)packed, (float)alpha,
+             (float)limit, cur_stream());
+  };
+  const int rc = panel ? run(omnia_panel_moe, seg, (int)nw) : run(omnia_stream_moe, (int)nw);
+  CHECK_RC(rc, "grouped products of a few rows:");
+}
+
+// segments of 16 rows; nw: 16-row fragments of weights a block
+void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
+                at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
+                int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
+                double alpha, double limit) {
+  few_moe(false, mode, out, A, W, sorted, blk_expert, n_blocks, route_w, topk, n_assign, e_lo, nw,
+          packed, alpha, limit);
+}
+
+// segments of 64 or 128 rows; nw: waves a block
+void panel_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
+               at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
+               int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
+               double alpha, double limit) {
+  few_moe(true, mode, out, A, W, sorted, blk_expert, n_blocks, route_w, topk, n_assign, e_lo, nw,
+          packed, alpha, limit);
 }
 
 void moe_combine(at::Tensor out, at::Tensor Y, at::Tensor ids, int64_t topk, int64_t e_lo,
@@ -2146,6 +2170,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("stream_gemm", &stream_gemm);
   m.def("stream_moe", &stream_moe);
   m.def("panel_gemm", &panel_gemm);
+  m.def("panel_moe", &panel_moe);
   m.def("wgemm", &wgemm);
   m.def("wgemm_wide", &wgemm_wide);
   m.def("tgemm", &tgemm);

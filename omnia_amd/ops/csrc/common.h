@@ -46,6 +46,12 @@ __device__ __forceinline__ float sigmoidf_(float x) {
   return __builtin_amdgcn_rcpf(1.f + __expf(-x));
 }
 __device__ __forceinline__ float siluf_(float x) { return x * sigmoidf_(x); }
+// g = min(gate, limit), u = clamp(up, +-limit): g sigmoid(alpha g) (u + 1)
+__device__ __forceinline__ float clamped_glu(float g, float u, float alpha, float limit) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g * sigmoidf_(alpha * g) * (u + 1.f);
+}
 // gelu, tanh form: 0.5 x (1 + tanh(y)) = x sigmoid(2 y)
 __device__ __forceinline__ float gelu_tanh_(float x) {
   return x * sigmoidf_(1.5957691216057308f * (x + 0.044715f * x * x * x));

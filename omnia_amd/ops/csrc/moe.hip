@@ -666,7 +666,7 @@ int omnia_moe_max_blocks(int n_assign, int n_experts, int bm) {
 int omnia_moe_align(int* sorted, int* blk_expert, int* n_blocks, const int* ids, int n, int E,
                     int e_lo, int e_hi, int max_blocks, int bm, hipStream_t s) {
   if (E > 256 || e_lo < 0 || e_hi > E || e_lo >= e_hi) return -1;
-  if (bm != 16 && bm != 64 && bm != 256) return -2;
+  if (bm != 16 && bm != 64 && bm != 128 && bm != 256) return -2;
   moe_align_kernel<<<1, 1024, 0, s>>>(sorted, blk_expert, n_blocks, ids, n, E, e_lo, e_hi,
                                       max_blocks, bm);
   return (int)hipGetLastError();

@@ -17,6 +17,11 @@
 //     otherwise waits for all of it before some of the reads.
 //   EPI 0  out = acc            EPI 1  out = act(g + b) * (u + b), W = [Wg; Wu]
 //   EPI 2  fp32 slabs [S][M][N]
+// and of experts, whose rows are expert-sorted assignments in segments of 64 or 128 (a block
+// takes one segment; past the live ones it leaves):
+//   EPI 5  silu(g) * u of the assignments' token rows, in sorted order
+//   EPI 8  as 5, the routing weight on the input and a clamped GLU     EPI 10  gelu(up)
+//   EPI 6  rows in sorted order, out[assignment] = routing weight (if given) * acc
 #include "common.h"
 
 using namespace omnia;
@@ -37,7 +42,14 @@ struct PanelArgs {
   int64_t ldx, ldo;
   const float* bias;  // EPI 1: [2N] or null
   int gelu;
+  const int *sorted, *blk_expert, *n_blocks;  // experts
+  const float* route_w;
+  int topk, n_assign, e_lo;
+  float alpha, limit;
 };
+
+constexpr bool grouped(int epi) { return epi >= 5; }
+constexpr bool paired(int epi) { return epi == 1 || epi == 5 || epi == 8; }
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -79,8 +91,13 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
-  const int units = EPI == 1 ? p.N >> 3 : p.N >> 4, tiles = (units + WN - 1) / WN;
-  const int bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int units = paired(EPI) ? p.N >> 3 : p.N >> 4, tiles = (units + WN - 1) / WN;
+  const int bid = xcd_remap(blockIdx.x, gridDim.x), seg = blockIdx.y;
+  const bf16_t* W = p.w;
+  if constexpr (grouped(EPI)) {
+    if (seg >= *p.n_blocks) return;
+    W += (int64_t)(p.blk_expert[seg] - p.e_lo) * (paired(EPI) ? 2 * p.N : p.N) * p.K;
+  }
   const int split = bid / tiles, tile = bid - split * tiles;
   const int unit0 = tile * WN + wv, unit = unit0 < units ? unit0 : units - 1;
   const int K = p.K, nch = K >> 6;
@@ -92,22 +109,29 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     auto at = [&](int rr) -> int64_t {  // weight row of the unit's row rr
-      if constexpr (EPI == 1) return (rr < 8 ? 0 : (int64_t)p.N - 8) + (int64_t)unit * 8 + rr;
+      if constexpr (paired(EPI)) return (rr < 8 ? 0 : (int64_t)p.N - 8) + (int64_t)unit * 8 + rr;
       return (int64_t)unit * 16 + rr;
     };
     if constexpr (PK) {
       const int64_t r = at(fr);
-      wp[h] = p.w + (r >> 4) * 16 * K + h * 512 + 128 * fq + 8 * (r & 15);
+      wp[h] = W + (r >> 4) * 16 * K + h * 512 + 128 * fq + 8 * (r & 15);
     } else {
       const int rr = 8 * h + (lane >> 3);
-      wp[h] = p.w + at(rr) * K + (((lane & 7) ^ (rr & 7)) << 3);
+      wp[h] = W + at(rr) * K + (((lane & 7) ^ (rr & 7)) << 3);
     }
   }
   const bf16_t* xp[XI];  // DMA instruction i of this wave: 8 rows
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
     const int r = (wv * XI + i) * 8 + (lane >> 3);
-    xp[i] = p.x + (int64_t)(r < p.M ? r : p.M - 1) * p.ldx + (((lane & 7) ^ (r & 7)) << 3);
+    int64_t row = r < p.M ? r : p.M - 1;
+    if constexpr (EPI == 6) {
+      row = seg * BM + r;
+    } else if constexpr (grouped(EPI)) {  // the assignment's token (padding: the first one)
+      const int f = p.sorted[seg * BM + r];
+      row = f < p.n_assign ? f / p.topk : 0;
+    }
+    xp[i] = p.x + row * p.ldx + (((lane & 7) ^ (r & 7)) << 3);
   }
   auto issue = [&](bf16_t* dst, int s) {  // stage s into a slot
     const bool in = s < n;
@@ -167,33 +191,45 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 16 * i + 4 * fq + r;
-      float v = acc[i][r];
-      if constexpr (EPI == 1) {
-        float u = __shfl_xor(v, 8, 64);  // the up half, in the lanes of the gate half
-        const int col = unit * 8 + (fr & 7);
-        float g = v;
-        if (p.bias) {
-          g += p.bias[col];
-          u += p.bias[p.N + col];
+      float v = acc[i][r], u = 0.f;
+      if constexpr (paired(EPI)) u = __shfl_xor(v, 8, 64);  // the up half, to the gate half's lanes
+      const int64_t col = paired(EPI) ? (int64_t)unit * 8 + (fr & 7) : (int64_t)unit * 16 + fr;
+      if (paired(EPI) && fr >= 8) continue;
+      bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
+      if constexpr (grouped(EPI)) {
+        const int row = seg * BM + m, f = p.sorted[row];
+        if (f >= p.n_assign) continue;
+        if constexpr (EPI == 6) {
+          out[f * p.ldo + col] = f2bf(p.route_w ? p.route_w[f] * v : v);
+        } else if constexpr (EPI == 5) {
+          out[row * p.ldo + col] = f2bf(siluf_(v) * u);
+        } else if constexpr (EPI == 8) {
+          const float wt = p.route_w[f];
+          out[row * p.ldo + col] = f2bf(clamped_glu(wt * v, wt * u, p.alpha, p.limit));
+        } else {
+          out[row * p.ldo + col] = f2bf(gelu_erf16_(v));
         }
-        if (fr < 8 && m < p.M)
-          reinterpret_cast<bf16_t*>(p.out)[m * p.ldo + col] =
-              f2bf((p.gelu ? gelu_tanh_(g) : siluf_(g)) * u);
       } else if (m < p.M) {
-        const int64_t col = (int64_t)unit * 16 + fr;
-        if constexpr (EPI == 0)
-          reinterpret_cast<bf16_t*>(p.out)[m * p.ldo + col] = f2bf(v);
-        else
+        if constexpr (EPI == 1) {
+          if (p.bias) {
+            v += p.bias[col];
+            u += p.bias[p.N + col];
+          }
+          out[m * p.ldo + col] = f2bf((p.gelu ? gelu_tanh_(v) : siluf_(v)) * u);
+        } else if constexpr (EPI == 0) {
+          out[m * p.ldo + col] = f2bf(v);
+        } else {
           reinterpret_cast<float*>(p.out)[((int64_t)split * p.M + m) * p.N + col] = v;
+        }
       }
     }
   }
 }
 
 template <int MF, int WN, int EPI>
-int launch(const PanelArgs& p, bool packed, hipStream_t s) {
-  const int units = EPI == 1 ? p.N / 8 : p.N / 16;
-  const int grid = (units + WN - 1) / WN * p.S;
+int launch(const PanelArgs& p, bool packed, hipStream_t s, int segs = 1) {
+  const int units = paired(EPI) ? p.N / 8 : p.N / 16;
+  const dim3 grid((units + WN - 1) / WN * p.S, segs);
   if (packed)
     panel_kernel<MF, WN, EPI, true><<<grid, 64 * WN, 0, s>>>(p);
   else
@@ -214,6 +250,13 @@ int by_waves(const PanelArgs& p, int wn, bool packed, hipStream_t s) {
   return wn == 8 ? by_rows<8, EPI>(p, packed, s) : by_rows<4, EPI>(p, packed, s);
 }
 
+template <int EPI>
+int by_segment(const PanelArgs& p, int bm, int wn, bool packed, int segs, hipStream_t s) {
+  if (bm == 64)
+    return wn == 8 ? launch<4, 8, EPI>(p, packed, s, segs) : launch<4, 4, EPI>(p, packed, s, segs);
+  return wn == 8 ? launch<8, 8, EPI>(p, packed, s, segs) : launch<8, 4, EPI>(p, packed, s, segs);
+}
+
 }  // namespace
 
 extern "C" {
@@ -231,10 +274,35 @@ int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, 
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return -6;
   if (bias && epi != 1) return -7;
   if (wn != 4 && wn != 8) return -8;
-  const PanelArgs p{out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, S, ldx, ldo, bias, gelu};
+  const PanelArgs p{out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, S, ldx, ldo, bias, gelu,
+                    nullptr, nullptr, nullptr, nullptr, 1, 0, 0, 0.f, 0.f};
   if (epi == 0) return by_waves<0>(p, wn, packed, s);
   if (epi == 1) return by_waves<1>(p, wn, packed, s);
   return by_waves<2>(p, wn, packed, s);
+}
+
+// Grouped products over segments of bm (64, 128) rows as omnia_moe_align makes them.  Modes and
+// operands as omnia_moe_gemm.
+int omnia_panel_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
+                    const int* blk_expert, const int* n_blocks, const float* route_w, int K, int N,
+                    int topk, int n_assign, int e_lo, int max_blocks, int bm, int wn, int packed,
+                    float alpha, float limit, hipStream_t s) {
+  if (mode < 0 || mode > 3 || K < 64 || K % 64) return -1;
+  if (bm != 64 && bm != 128) return -2;
+  if (wn != 4 && wn != 8) return -3;
+  const int cols = mode == 0 || mode == 2 ? 8 : 16;
+  if (N < 16 || N % cols || (packed && N % 16) || N > 1 << 24) return -4;
+  if (mode == 2 && !route_w) return -5;
+  if (max_blocks == 0) return 0;
+  if (max_blocks > 65535 || topk < 1) return -6;
+  if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) return -7;
+  const PanelArgs p{out,    (const bf16_t*)A, (const bf16_t*)W, bm,       N,    K,        1,
+                    K,      N,                nullptr,          0,        sorted, blk_expert,
+                    n_blocks, route_w,        topk,             n_assign, e_lo, alpha,    limit};
+  if (mode == 0) return by_segment<5>(p, bm, wn, packed, max_blocks, s);
+  if (mode == 1) return by_segment<6>(p, bm, wn, packed, max_blocks, s);
+  if (mode == 2) return by_segment<8>(p, bm, wn, packed, max_blocks, s);
+  return by_segment<10>(p, bm, wn, packed, max_blocks, s);
 }
 
 }  // extern "C"

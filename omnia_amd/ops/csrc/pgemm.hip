@@ -129,13 +129,6 @@ __device__ __forceinline__ float16v mfma32(short8 a, short8 b, float16v c) {
 
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
 
-// g = min(gate, limit), u = clamp(up, +-limit): g sigmoid(alpha g) (u + 1)
-__device__ __forceinline__ float clamped_glu(float g, float u, float alpha, float limit) {
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g * __builtin_amdgcn_rcpf(1.f + __expf(-alpha * g)) * (u + 1.f);
-}
-
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");

@@ -68,12 +68,6 @@ constexpr bool gated(int epi) { return epi == 1 || epi == 5 || epi == 8; }
 constexpr bool paired(int epi) { return gated(epi) || epi == 3; }
 constexpr bool grouped(int epi) { return epi >= 5; }
 
-__device__ __forceinline__ float clamped_glu(float g, float u, float alpha, float limit) {
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return g * sigmoidf_(alpha * g) * (u + 1.f);
-}
-
 // D: chunks in flight of 1 + NW operand fragments, 8 registers each
 template <int NW, int EPI, bool NORM, bool PK>
 __global__ __launch_bounds__(64 * WAVES, NW <= 2 ? 4 : 2) void stream_kernel(StreamArgs p) {

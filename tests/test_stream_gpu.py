@@ -153,6 +153,48 @@ def test_experts_match_the_64_row_kernels(T, E, k, glu, gelu, packed, monkeypatc
     assert ((got - want).abs() <= 4 * U * want.abs().clamp(min=want.pow(2).mean().sqrt())).all()
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("glu,gelu", [(None, False), ((1.702, 7.0), False), (None, True)])
+@pytest.mark.parametrize("bm,T,E,k", [(64, 3, 8, 2), (64, 40, 4, 4), (128, 65, 1, 1),
+                                      (128, 129, 3, 1), (128, 300, 9, 2)])
+def test_experts_in_panel_segments(bm, T, E, k, glu, gelu, packed, monkeypatch):
+    """Segments of 64 and 128 rows: nearly empty, full and one row over (every row of an expert),
+    experts without a row, a column tile that is not whole: as the 64-row kernels above."""
+    d, ff = 224, 352
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    _, up = _mk(1, ff if gelu else 2 * ff, d, 3, (E,))
+    _, down = _mk(1, d, ff, 4, (E,))
+    up, down = (F.pad(t, (0, -t.shape[2] % 64)).contiguous() for t in (up, down))
+    ff = down.shape[2]
+    if not gelu:
+        up = up.view(E, 2, -1, up.shape[2])
+    up = F.pad(up, (0, 0, 0, ff - up.shape[-2])).reshape(E, -1, up.shape[-1]).contiguous()
+    down = F.pad(down, (0, 0, 0, up.shape[2] - d)).contiguous()
+    x = F.pad(torch.randn(T, d, generator=g, device="cuda"), (0, -d % 64)).to(torch.bfloat16)
+    ids = torch.stack([torch.randperm(E, generator=g, device="cuda")[:k] for _ in range(T)]).int()
+    if T == 129:
+        ids[:] = 1
+    wts = torch.rand(T, k, generator=g, device="cuda")
+    args = (x, up, down, ids.contiguous(), wts, k, E, 0, E, 64, glu, gelu)
+    monkeypatch.setattr(ops, "moe_stream_ok", lambda *a: False)
+    monkeypatch.setattr(ops, "moe_panel_rows", lambda *a: 0)
+    want = ops._moe_grouped(*args).double()
+    monkeypatch.setattr(ops, "moe_panel_rows", lambda *a: bm)
+    streams = (ops.stream_pack(up), ops.stream_pack(down)) if packed else None
+    got = ops._moe_grouped(*args, streams=streams).double()
+    assert (got - want).norm() <= 2 * U * want.norm()
+    assert ((got - want).abs() <= 4 * U * want.abs().clamp(min=want.pow(2).mean().sqrt())).all()
+
+
+def test_panel_segments_by_rows_an_expert():
+    up, down = (torch.empty(8, *s, dtype=torch.bfloat16, device="cuda")
+                for s in ((256, 2048), (2048, 2048)))
+    assert [ops.moe_panel_rows(n, 8, up, down, True) for n in (65, 447, 448)] == [64, 64, 128]
+    assert [ops.moe_panel_rows(n, 8, up, down, False) for n in (65, 447, 448)] == [0, 0, 128]
+    assert ops.moe_panel_rows(100, 8, up[..., :1024], down[:, :1024], True) == 0
+    assert ops.moe_panel_rows(448, 8, up.float(), down, True) == 0
+
+
 def test_what_is_refused():
     x, w = _mk(17, 64, 128, 1)
     with pytest.raises(RuntimeError):
