@@ -995,10 +995,13 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
         panel = moe_panel_rows(n, experts, w_gu, w_down, streams is not None)
         bm = panel or bm
     mb = kk.moe_max_blocks(n, experts, bm)
-    sorted_ids = torch.empty(mb * bm, dtype=torch.int32, device=x.device)
-    blk = torch.empty(mb, dtype=torch.int32, device=x.device)
+    # a wave of the streaming kernel sorts 64 assignments by itself, an expert a step
+    own = few and n <= 64 and experts <= 64
+    sorted_ids = torch.empty(0 if own else mb * bm, dtype=torch.int32, device=x.device)
+    blk = torch.empty(0 if own else mb, dtype=torch.int32, device=x.device)
     nblk = torch.empty(1, dtype=torch.int32, device=x.device)
-    kk.moe_align(sorted_ids, blk, nblk, ids, n_experts, e_lo, e_hi)
+    if not own:
+        kk.moe_align(sorted_ids, blk, nblk, ids, n_experts, e_lo, e_hi)
     act = torch.empty(mb * bm, w_down.shape[2], dtype=x.dtype, device=x.device)
     Y = torch.empty(n, x.shape[1], dtype=x.dtype, device=x.device)
     gemm = kk.pgemm_moe if bm == 256 else kk.moe_gemm
@@ -1010,7 +1013,7 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
             if streams is not None:
                 w = streams[mode == 1]
             kk.stream_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, frags, streams is not None,
-                          alpha, limit)
+                          alpha, limit, ids if own else None)
 
     elif panel:
         segs = experts * -(-5 * n // (4 * experts * panel))  # live ones, about

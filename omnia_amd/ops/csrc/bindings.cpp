@@ -129,8 +129,8 @@ int omnia_stream(int epi, void* out, const void* x, const void* w, int M, int N,
 int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, int K, int S,
                 int64_t ldx, int64_t ldo, int wn, int packed, const float* bias, int gelu,
                 hipStream_t s);
-int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
-                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
+int omnia_stream_moe(int mode, void* out, const void* A, const void* W, const int* ids, int e_hi,
+                     const int* sorted, const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                      int N, int topk, int n_assign, int e_lo, int max_blocks, int nw, int packed,
                      float alpha, float limit, hipStream_t s);
 int omnia_panel_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
@@ -774,7 +774,7 @@ void moe_gemm(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tens
 static void few_moe(bool panel, int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
                 at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
                 int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
-                double alpha, double limit) {
+                double alpha, double limit, const c10::optional<at::Tensor>& ids = {}) {
   CHECK_GPU(A); CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(out);
   CHECK_I32(sorted); CHECK_I32(blk_expert); CHECK_I32(n_blocks);
   TORCH_CHECK(mode >= 0 && mode <= 3, "mode");
@@ -783,9 +783,14 @@ static void few_moe(bool panel, int64_t mode, at::Tensor out, at::Tensor A, at::
   for (const at::Tensor* t : {&W, &out, &sorted, &blk_expert, &n_blocks})
     TORCH_CHECK(t->device() == A.device(), "same device");
   const int K = W.size(2);
-  const int mb = blk_expert.numel();
+  const int mb = ids ? (mode == 1 ? A : out).size(0) / 16 : blk_expert.numel();
+  if (ids) {
+    CHECK_I32((*ids));
+    TORCH_CHECK(ids->is_contiguous() && ids->device() == A.device() && ids->numel() == n_assign &&
+                n_assign <= 64, "ids of at most 64 assignments");
+  }
   const int seg = panel ? (int)(mb > 0 ? sorted.numel() / mb : 0) : 16;
-  TORCH_CHECK(sorted.numel() == (int64_t)mb * seg, "sorted must hold max_blocks segments");
+  TORCH_CHECK(ids || sorted.numel() == (int64_t)mb * seg, "sorted must hold max_blocks segments");
   TORCH_CHECK(A.size(1) == K, "K mismatch");
   if (route_w.has_value())
     TORCH_CHECK(route_w->device() == A.device() && route_w->is_contiguous() &&
@@ -802,23 +807,29 @@ static void few_moe(bool panel, int64_t mode, at::Tensor out, at::Tensor A, at::
     TORCH_CHECK(out.size(0) == n_assign && out.size(1) == N, "Y [T*k, d]");
     TORCH_CHECK(A.size(0) == (int64_t)mb * seg, "act rows");
   }
-  const auto run = [&](auto f, auto... shape) {
-    return f((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(), sorted.data_ptr<int>(),
-             blk_expert.data_ptr<int>(), n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N,
-             (int)topk, (int)n_assign, (int)e_lo, mb, shape..., (int)packed, (float)alpha,
-             (float)limit, cur_stream());
-  };
-  const int rc = panel ? run(omnia_panel_moe, seg, (int)nw) : run(omnia_stream_moe, (int)nw);
+  const int* so = ids ? nullptr : sorted.data_ptr<int>();
+  const int* bl = ids ? nullptr : blk_expert.data_ptr<int>();
+  const int* nb = ids ? nullptr : n_blocks.data_ptr<int>();
+  const float* rw = opt_ptr<float>(route_w);
+  const int rc =
+      panel ? omnia_panel_moe((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(), so, bl, nb,
+                              rw, K, N, (int)topk, (int)n_assign, (int)e_lo, mb, seg, (int)nw,
+                              packed, (float)alpha, (float)limit, cur_stream())
+            : omnia_stream_moe((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(),
+                               ids ? ids->data_ptr<int>() : nullptr, (int)(e_lo + W.size(0)), so,
+                               bl, nb, rw, K, N, (int)topk, (int)n_assign, (int)e_lo, mb, (int)nw,
+                               packed, (float)alpha, (float)limit, cur_stream());
   CHECK_RC(rc, "grouped products of a few rows:");
 }
 
-// segments of 16 rows; nw: 16-row fragments of weights a block
+// segments of 16 rows; nw: 16-row fragments of weights a block.  ids [n_assign <= 64]: the kernel
+// sorts them itself, and sorted, blk_expert and n_blocks are not read
 void stream_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
                 at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
                 int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,
-                double alpha, double limit) {
+                double alpha, double limit, c10::optional<at::Tensor> ids) {
   few_moe(false, mode, out, A, W, sorted, blk_expert, n_blocks, route_w, topk, n_assign, e_lo, nw,
-          packed, alpha, limit);
+          packed, alpha, limit, ids);
 }
 
 // segments of 64 or 128 rows; nw: waves a block

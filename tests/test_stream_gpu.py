@@ -153,6 +153,29 @@ def test_experts_match_the_64_row_kernels(T, E, k, glu, gelu, packed, monkeypatc
     assert ((got - want).abs() <= 4 * U * want.abs().clamp(min=want.pow(2).mean().sqrt())).all()
 
 
+@pytest.mark.parametrize("T,E,k,lo,hi", [(32, 8, 2, 2, 6), (64, 64, 1, 0, 64), (16, 5, 4, 4, 5),
+                                         (33, 8, 2, 0, 8), (6, 65, 2, 0, 65), (1, 4, 1, 0, 4)])
+def test_sorted_by_the_kernel_or_before(T, E, k, lo, hi, monkeypatch):
+    """Up to 64 assignments and experts the kernel sorts them itself: a shard's experts only, one
+    expert with every row, more of either, rows of every lane."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    _, up = _mk(1, 256, 128, 3, (hi - lo,))
+    _, down = _mk(1, 128, 128, 4, (hi - lo,))
+    x = torch.randn(T, 128, generator=g, device="cuda").to(torch.bfloat16)
+    ids = torch.stack([torch.randperm(E, generator=g, device="cuda")[:k] for _ in range(T)]).int()
+    if E == 5:
+        ids[:] = torch.arange(1, 5, device="cuda")
+    wts = torch.rand(T, k, generator=g, device="cuda")
+    local = ((ids >= lo) & (ids < hi)).view(-1)
+    args = (x, up, down, ids.contiguous(), wts, k, E, lo, hi, 64)
+    monkeypatch.setattr(ops, "moe_panel_rows", lambda *a: 0)
+    res = []
+    for few in (False, True):
+        monkeypatch.setattr(ops, "moe_stream_ok", lambda *a: few)
+        res.append(ops._moe_grouped(*args).double()[local])
+    assert (res[0] - res[1]).norm() <= 2 * U * res[0].norm()
+
+
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("glu,gelu", [(None, False), ((1.702, 7.0), False), (None, True)])
 @pytest.mark.parametrize("bm,T,E,k", [(64, 3, 8, 2), (64, 40, 4, 4), (128, 65, 1, 1),
