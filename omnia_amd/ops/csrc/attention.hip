@@ -568,7 +568,9 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = blockIdx.x * HB + w;
   const int kvh = blockIdx.x * HB / G;
-  const int tile = blockIdx.y;
+  // a sequence's last tiles, which see most keys, first: what is left for the end is short
+  // (4 x 1000 rows, 32 heads on 8, 71.2 -> 61.8 us; 8 x 2048 382 -> 373)
+  const int tile = gridDim.y - 1 - blockIdx.y;
   const int s = tile_seq[tile], q0 = tile_q0[tile];
   const int qs = q_start_loc[s], qlen = q_start_loc[s + 1] - qs;
   const int ctx = seq_lens[s];

@@ -81,7 +81,9 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
   // blocks of one key/value head are neighbours: (head block, tile, sub-tile)
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int sub = id & (HB - 1), rest = id >> p.hb_lg;
-  const int hblk = rest / p.n_tiles, tile = rest - hblk * p.n_tiles;
+  // a sequence's last tiles, which see most keys, first: what is left for the end is short
+  // (8 x 2048 rows, 16 heads, 225 -> 213 us)
+  const int hblk = rest / p.n_tiles, tile = p.n_tiles - 1 - (rest - hblk * p.n_tiles);
   const int s = p.tile_seq[tile];
   const int qs = p.q_start[s], qlen = p.q_start[s + 1] - qs;
   const int rows = 128 >> p.hb_lg;  // of this block: the tile has HB sub-tiles

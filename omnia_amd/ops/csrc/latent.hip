@@ -521,7 +521,9 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(
   __shared__ __attribute__((aligned(16))) bf16_t Kl[64 * KS];
   __shared__ __attribute__((aligned(16))) bf16_t Vl[VW * VS];
   const int id = xcd_remap(blockIdx.x, gridDim.x);  // a head's tiles share an XCD's L2
-  const int h = id / n_tiles, tl = id - h * n_tiles;
+  // a sequence's last tiles, which see most keys, first: what is left for the end is short
+  // (8 x 2048 rows, 16 heads, 225 -> 215 us)
+  const int h = id / n_tiles, tl = n_tiles - 1 - (id - h * n_tiles);
   const int s = tile_seq[tl], q0 = tile_q0[tl];
   const int qs = q_start[s], qlen = q_start[s + 1] - qs;
   const int off = seq_lens[s] - qlen, kf = kv_first[s], kst = kv_start[s];
