@@ -280,19 +280,32 @@ template <typename T>
 __device__ __forceinline__ void shift_conv(const T* __restrict__ x, int64_t ldx, T* cs, int row0,
                                            int n, bool fresh, int taps, int C, int c) {
   // oldest first; new entry i comes from row0 + n - (taps-1) + i, or from the old state
-  for (int i = 0; i < taps - 1; ++i) {
+  auto entry = [&](int i) -> T {
     const int r = n - (taps - 1) + i;  // relative to row0
-    T v;
-    if (r >= 0) v = x[(int64_t)(row0 + r) * ldx + c];
-    else if (fresh) v = (T)0;
-    else v = cs[(int64_t)(taps - 1 + r) * C + c];  // index >= i + n > i: not yet overwritten
-    cs[(int64_t)i * C + c] = v;
+    if (r >= 0) return x[(int64_t)(row0 + r) * ldx + c];
+    if (fresh) return (T)0;
+    return cs[(int64_t)(taps - 1 + r) * C + c];  // index >= i + n > i: not yet overwritten
+  };
+  if (taps <= 4) {  // all loads in flight together
+    T v[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < taps - 1) v[i] = entry(i);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < taps - 1) cs[(int64_t)i * C + c] = v[i];
+  } else {
+    for (int i = 0; i < taps - 1; ++i) cs[(int64_t)i * C + c] = entry(i);
   }
 }
 
 // ------------------------------------------------------------------ delta_step
 // grid (rows, H), 256 threads.  Thread (cg, rg): 4 state columns cg*4.., the rows
-// rg, rg + RG, ... kept in registers (NR of them).
+// rg, rg + RG, ... kept in registers (NR of them).  Bound by reading and writing the state, once
+// each and not again before the next token: past the caches (non-temporal), and with all else it
+// reads asked for before the first barrier.  us at 4 / 16 / 32 / 64 / 200 rows of 16 heads of 128,
+// before -> now: 8.7 / 11.7 / 22 / 39 / 101 -> 8.3 / 9.9 / 16 / 28 / 84 (5.0 TB/s; the loads
+// alone non-temporal 9.0 / 12.0 / 17.5 / 30 / 90).
 template <typename T, int NR>
 __global__ __launch_bounds__(256) void step_kernel(
     T* __restrict__ y, float* __restrict__ state, T* __restrict__ conv_state,
@@ -317,10 +330,14 @@ __global__ __launch_bounds__(256) void step_kernel(
   float* os = us + Vs;        // [Vs]
   float* scratch = os + Vs;   // [8]
   const int kh = h / (H / KH);
-  for (int i = tid; i < Dp; i += 256) {
-    ks[i] = kn[((int64_t)t * KH + kh) * Dp + i];
-    qs[i] = qn[((int64_t)t * KH + kh) * Dp + i];
-  }
+  const float* kr = kn + ((int64_t)t * KH + kh) * Dp;
+  const float* qr = qn + ((int64_t)t * KH + kh) * Dp;
+  const T* vr = vc + ((int64_t)t * H + h) * V;
+  const T* zr = x + (int64_t)t * ldx + C + h * V;
+  // a thread's first of each loop below over columns
+  const float lg = decay[(int64_t)t * H + h], bt = beta[(int64_t)t * H + h];
+  const int d0 = min(tid, Dp - 1), v0 = min(tid, V - 1);
+  const float k0 = kr[d0], q0 = qr[d0], vv0 = ldf(vr + v0), z0 = ldf(zr + v0), w0 = norm_w[v0];
   const int cg = tid % CG, rg = tid / CG;
   const bool act = rg < RG;
   float4v* S = reinterpret_cast<float4v*>(state + (((int64_t)slot * H + h) * D) * Vs) + cg;
@@ -328,10 +345,20 @@ __global__ __launch_bounds__(256) void step_kernel(
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int d = rg + i * RG;
-    reg[i] = (act && d < D && !fresh) ? S[(int64_t)d * CG] : float4v{0.f, 0.f, 0.f, 0.f};
+    reg[i] = (act && d < D && !fresh) ? __builtin_nontemporal_load(S + (int64_t)d * CG)
+                                      : float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  // this head's share of the convolution state (delta_prep has read it)
+  const int per = (C + H - 1) / H;
+  T* cs = conv_state + (int64_t)slot * (taps - 1) * C;
+  for (int c = h * per + tid; c < min(C, (h + 1) * per); c += 256)
+    shift_conv(x, ldx, cs, t, 1, fresh, taps, C, c);
+  for (int i = tid; i < Dp; i += 256) {
+    ks[i] = i < 256 ? k0 : kr[i];
+    qs[i] = i < 256 ? q0 : qr[i];
   }
   __syncthreads();
-  const float g = expf(decay[(int64_t)t * H + h]), bt = beta[(int64_t)t * H + h];
+  const float g = expf(lg);
   float4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
@@ -344,7 +371,7 @@ __global__ __launch_bounds__(256) void step_kernel(
   for (int j = tid; j < Vs; j += 256) {
     float sk = 0.f;
     for (int r = 0; r < RG; ++r) sk += red[r * Vs + j];
-    us[j] = j < V ? bt * (ldf(vc + ((int64_t)t * H + h) * V + j) - sk) : 0.f;
+    us[j] = j < V ? bt * ((j < 256 ? vv0 : ldf(vr + j)) - sk) : 0.f;
   }
   __syncthreads();
   acc = float4v{0.f, 0.f, 0.f, 0.f};
@@ -356,7 +383,7 @@ __global__ __launch_bounds__(256) void step_kernel(
       if (d < D) {
         reg[i] += u4 * ks[d];
         acc += reg[i] * qs[d];
-        S[(int64_t)d * CG] = reg[i];
+        __builtin_nontemporal_store(reg[i], S + (int64_t)d * CG);
       }
     }
     *reinterpret_cast<float4v*>(red + rg * Vs + cg * 4) = acc;
@@ -371,14 +398,10 @@ __global__ __launch_bounds__(256) void step_kernel(
   }
   ss = block_sum(ss, scratch);
   const float inv = 1.f / sqrtf(ss / (float)V + eps);
-  const T* zr = x + (int64_t)t * ldx + C + h * V;
-  for (int j = tid; j < Vp; j += 256)
-    stf(yr + j, j < V ? os[j] * inv * norm_w[j] * siluf_(ldf(zr + j)) : 0.f);
-  // this head's share of the convolution state (delta_prep has read it)
-  const int per = (C + H - 1) / H;
-  T* cs = conv_state + (int64_t)slot * (taps - 1) * C;
-  for (int c = h * per + tid; c < min(C, (h + 1) * per); c += 256)
-    shift_conv(x, ldx, cs, t, 1, fresh, taps, C, c);
+  for (int j = tid; j < Vp; j += 256) {
+    const float z = j < 256 || j >= V ? z0 : ldf(zr + j), nw = j < 256 || j >= V ? w0 : norm_w[j];
+    stf(yr + j, j < V ? os[j] * inv * nw * siluf_(z) : 0.f);
+  }
 }
 
 // ------------------------------------------------------------------ delta_scan
