@@ -116,13 +116,20 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
       t.v[i] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(vb + vo));
     }
   };
-  float m_run = -INFINITY, l_run = 0.f;  // of head c16
+  // of head c16; a finite start, so that keys whose scores are all -inf get exponents of -inf
+  float m_run = -3.4028234e38f, l_run = 0.f;
   float acc[G][8];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  auto compute = [&](const Group& t, int c) {
+  auto compute = [&](Group& t, int c) {
+    // rows past the end have P = 0, which leaves nothing of a V that is finite
+    if (n - c * 16 < 16) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (4 * i + g4 >= n - c * 16) t.v[i] = short8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
     float4v sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) sc = mfma16(t.k[kk], qf[kk], sc);

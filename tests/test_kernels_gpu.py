@@ -269,6 +269,30 @@ def test_decode_attention_around_whole_key_groups(hq, hkv, bs):
     assert (err <= exp.abs() * 2.0 ** -8 + 2e-4 * vc.abs().max()).all(), err.max()
 
 
+@pytest.mark.parametrize("n", [17, 33, 200, 1023])
+def test_decode_attention_with_infinite_scores_and_values(n):
+    """Keys whose scores are -inf weigh nothing, whichever groups of a wave they fill; an infinite
+    value of the last key reaches its own dimension only, with its sign."""
+    torch.manual_seed(9)
+    hq, hkv, bs = 8, 2, 16
+    kc, vc = _make_cache(-(-n // bs) + 1, hkv, bs, seed=9)
+    bt = _tables([n], bs, -(-n // bs) + 1)
+    sl = torch.tensor([n], dtype=torch.int32, device=DEV)
+    q = torch.rand(1, hq, 128, device=DEV).bfloat16() + 1
+    at = bt[0, :-2].long()
+    kc[at[:-1]] = -3e38  # sums of 128 such products overflow fp32
+    vc[at[-1], 0, (n - 1) % bs, 5] = math.inf
+    vc[at[-1], 1, (n - 1) % bs, 7] = -math.inf
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=1024).double()
+    exp = _attention64(q, kc, vc, bt, [1], [n], 128 ** -0.5)
+    assert torch.equal(out.isinf(), exp.isinf()) and exp.isinf().sum() == 8
+    assert torch.equal(out[exp.isinf()], exp[exp.isinf()])
+    rest = ~exp.isinf()
+    # all sums are fp32: what is left is the result's rounding to bf16
+    err = (out - exp).abs()[rest]
+    assert (err <= exp[rest].abs() * 2.0 ** -8 + 1e-4).all(), err.max()
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
