@@ -54,11 +54,14 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
 // every fourth 16-key group by itself, with its own running max: K and V of the next group are
 // loaded while this one's scores, softmax and P.V are computed, so that memory never waits for a
 // phase of the block, and the waves meet once at the end.  3 waves a SIMD: groups of 32 keys take
-// the registers of 2, and short contexts 50 us where these take 39; 4 spill.  K and V are read
-// once a step: past the caches (non-temporal).  us with scores, softmax and P.V as phases of the
-// block -> so -> and past the caches (32 heads on 8; sequences x keys): 256 x 576 127 -> 119 -> 111
-// (5.45 TB/s), 128 x 1000 111 -> 104 -> 97, 64 x 2000 115 -> 112 -> 105, 32 x 1000 33.7 -> 29.3
-// -> 26.3, 4 x 1000 15.3 -> 12.4 -> 12.0, 256 x 150 38.2 -> 37.0 -> 37.4.
+// the registers of 2, and short contexts 50 us where these take 39; 4 spill.  us with scores,
+// softmax and P.V as phases of the block -> now (32 heads on 8; sequences x keys): 256 x 576
+// 127 -> 119 (5.1 TB/s), 128 x 1000 111 -> 104, 64 x 2000 115 -> 112, 32 x 1000 33.7 -> 29.3,
+// 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  K and V go through the caches: sequences of one
+// prompt prefix share its pages, and of those a block finds what another has read.  Past the
+// caches (non-temporal) only what no sequence shares gains: 256 x 576 105 -> 103, 128 x 1000 94 ->
+// 84, 32 x 1000 27 -> 24, but 512 of 576 keys shared 59 -> 73, 896 of 1000 45 -> 64; choosing for
+// each block costs the registers of a wave.
 constexpr int NW = 4;
 template <int G, int BS>
 __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
@@ -109,11 +112,11 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
     const uint32_t ko = min(c16, top) * D + 8 * g4;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
-      t.k[kk] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(kb + ko + kk * 32));
+      t.k[kk] = *reinterpret_cast<const short8*>(kb + ko + kk * 32);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t vo = min(4 * i + g4, top) * D + 8 * c16;
-      t.v[i] = __builtin_nontemporal_load(reinterpret_cast<const short8*>(vb + vo));
+      t.v[i] = *reinterpret_cast<const short8*>(vb + vo);
     }
   };
   // of head c16; a finite start, so that keys whose scores are all -inf get exponents of -inf

@@ -8,6 +8,7 @@ dirty lines would be written back under the measured kernel).
     python scripts/decode_attn_sweep.py [--parts 256,512,1024]
     python scripts/decode_attn_sweep.py --batch 128 --hq 64   # Llama-3-70B, TP=1
     python scripts/decode_attn_sweep.py --hq 8 --hkv 1        # one Llama-3-70B TP=8 rank
+    python scripts/decode_attn_sweep.py --shared 512          # one prompt prefix for all
 
 Rows ``mix`` draw every sequence's length uniformly from 513..640, as in a
 closed-loop wave (the partition split then varies per sequence).
@@ -31,6 +32,8 @@ def main():
     ap.add_argument("--batch", type=int, default=256)
     ap.add_argument("--hq", type=int, default=32)
     ap.add_argument("--hkv", type=int, default=8, help="1 = a Llama-3-70B TP=8 shard")
+    ap.add_argument("--shared", type=int, default=0,
+                    help="keys at the start of every sequence whose pages are the same")
     a = ap.parse_args()
     parts = [int(x) for x in a.parts.split(",")]
     torch.manual_seed(0)
@@ -47,6 +50,7 @@ def main():
     kc, vc = kcs[0], vcs[0]
     perm = torch.randperm(nblk - 8, device=dev)[:B * mb].to(torch.int32)
     bt = perm.view(B, mb).contiguous()
+    bt[:, :a.shared // BS] = bt[0, :a.shared // BS]
     q = torch.randn(B, hq, D, device=dev, dtype=torch.bfloat16)
     scale = D ** -0.5
     print(f"{'len':>5} {'part':>5} {'sp':>3} {'us':>8} {'TB/s':>6}  err", flush=True)

@@ -293,6 +293,24 @@ def test_decode_attention_with_infinite_scores_and_values(n):
     assert (err <= exp[rest].abs() * 2.0 ** -8 + 1e-4).all(), err.max()
 
 
+@pytest.mark.parametrize("shared,splits", [(64, 0), (640, 0), (640, 8)])
+def test_decode_attention_on_shared_prefix_pages(shared, splits):
+    """Sequences of one prompt prefix read the same pages, whole partitions of them or parts."""
+    torch.manual_seed(10)
+    lens, hq, hkv, bs = [shared + n for n in (1, 7, 32, 200, 513)], 8, 2, 32
+    nb_total = sum(-(-n // bs) for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=10)
+    bt = _tables(lens, bs, nb_total)
+    bt[1:, :shared // bs] = bt[0, :shared // bs]
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(len(lens), hq, 128, device=DEV, dtype=torch.bfloat16)
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=512, splits=splits)
+    exp = _attention64(q, kc, vc, bt, [1] * len(lens), lens, 128 ** -0.5)
+    # all sums are fp32: what is left is the result's rounding to bf16
+    err = (out.double() - exp).abs()
+    assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
