@@ -945,8 +945,9 @@ MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
 
 def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
                   packed: bool) -> bool:
-    """Whether ``n`` assignments to ``experts`` local experts run on the streaming kernel, in
-    16-row segments (a fuller expert's weights are read once per segment).
+    """Whether ``n`` assignments to ``experts`` experts (all of them, where a shard holds some) run
+    on the streaming kernel, in 16-row segments (a fuller expert's weights are read once per
+    segment).
 
     Both products, us at 1 / 4 / 8 / 16 / 32 / 64 tokens of 2 experts in 8, 2048 x 4096: 64-row
     kernel 52 / 90 / 82 / 93 / 93 / 93, packed 25 / 63 / 58 / 72 / 74 / 95; 4096 x 14336: 193 /
@@ -959,8 +960,8 @@ def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor
 
 def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
                    packed: bool) -> int:
-    """Segment rows of the panel kernel for ``n`` assignments to ``experts`` local experts, 0
-    where moe.hip's 64-row kernel does better.
+    """Segment rows of the panel kernel for ``n`` assignments to ``experts`` experts (all of them,
+    where a shard holds some), 0 where moe.hip's 64-row kernel does better.
 
     From 56 rows an expert most would need two segments of 64, so the weights are read twice;
     segments of 128 read them once (both products, us, 64-row kernel / 128-row segments at 64 / 100 / 128
@@ -987,12 +988,12 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     kernel and others :func:`moe_panel_rows`'s."""
     kk = kernels()
     n, experts = ids.numel(), e_hi - e_lo
-    few = bm == 64 and moe_stream_ok(n, experts, w_gu, w_down, streams is not None)
+    few = bm == 64 and moe_stream_ok(n, n_experts, w_gu, w_down, streams is not None)
     panel = 0
     if few:
         bm = 16
     elif bm == 64:
-        panel = moe_panel_rows(n, experts, w_gu, w_down, streams is not None)
+        panel = moe_panel_rows(n, n_experts, w_gu, w_down, streams is not None)
         bm = panel or bm
     mb = kk.moe_max_blocks(n, experts, bm)
     # a wave of the streaming kernel sorts 64 assignments by itself, an expert a step
@@ -1006,7 +1007,8 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     Y = torch.empty(n, x.shape[1], dtype=x.dtype, device=x.device)
     gemm = kk.pgemm_moe if bm == 256 else kk.moe_gemm
     if few:
-        live = min(n, experts)  # experts whose weights are read, at most
+        # experts whose weights are read, of a shard's as many as of the rest
+        live = max(1, min(n, n_experts) * experts // n_experts)
 
         def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
             frags = min(2, stream_fragments(min(n, 16), w.shape[1] * live))
@@ -1016,7 +1018,7 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
                           alpha, limit, ids if own else None)
 
     elif panel:
-        segs = experts * -(-5 * n // (4 * experts * panel))  # live ones, about
+        segs = experts * -(-5 * n // (4 * n_experts * panel))  # live ones, about
 
         def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
             wn = panel_plan(panel, w.shape[1] * segs, w.shape[2], False)[0]
@@ -1091,7 +1093,7 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
     kk.moe_router_topk(ids, wts, x.contiguous(), router, k, renorm)
     out = torch.empty_like(x)
     d, inter = x.shape[1], w_down.shape[2]
-    if n >= MOE_TILE256_ROWS * (e_hi - e_lo) and d % 256 == 0 and inter % 128 == 0:
+    if n >= MOE_TILE256_ROWS * n_experts and d % 256 == 0 and inter % 128 == 0:
         # prefill-sized: the 256x256 MFMA tile, grouped by 256-row expert segments
         # (pgemm.hip EPI 5 / 6) -- hand kernels, graph-safe, no per-expert library
         # calls and no host sync

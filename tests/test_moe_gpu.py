@@ -96,7 +96,7 @@ def test_moe_tile256_prefill_matches_reference(T, d, I, E, k, e_lo, e_n):
     router, wgu, wd = _weights(E, d, I, g)
     x = (torch.randn(T, d, generator=g)).to(torch.bfloat16).cuda()
     wgu_l, wd_l = wgu[e_lo:e_lo + e_n].contiguous(), wd[e_lo:e_lo + e_n].contiguous()
-    assert T * k >= ops.MOE_TILE256_ROWS * e_n  # the 256-tile path is the one under test
+    assert T * k >= ops.MOE_TILE256_ROWS * E  # the 256-tile path is the one under test
     out = ops.moe(x, router, wgu_l, wd_l, k, E, e_lo, graph_safe=True)
     logits = torch.nn.functional.linear(x, router)
     rid, rw = ref.moe_route(logits.float().cpu(), k)
@@ -203,3 +203,32 @@ def test_router_topk_fused_matches_linear_then_topk(T, d, E, k):
     m = (ids.cpu() == rid).all(1)  # rows whose order no near-tie swapped
     assert m.float().mean().item() >= 0.9
     torch.testing.assert_close(w.cpu()[m], rw[m], atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("T,kernel", [(1, "stream_moe"), (64, "moe_gemm"), (300, "panel_moe"),
+                                      (2000, "pgemm_moe")])
+def test_a_shard_counts_its_rows_over_all_experts(T, kernel, monkeypatch):
+    """The kernel of a shard's experts follows the rows an expert has, which are those of all
+    assignments over all experts: one expert of eight takes the one that eight take."""
+    d, E, k = 256, 8, 2
+    g = torch.Generator().manual_seed(T)
+    router, wgu, wd = _weights(E, d, 256, g)
+    x = torch.randn(T, d, generator=g).to(torch.bfloat16).cuda()
+    used = []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(native, name)
+            if not name.endswith(("_moe", "moe_gemm")):
+                return f
+            return lambda *a: (used.append(name), f(*a))[1]
+
+    native = ops.kernels()
+    monkeypatch.setattr(ops, "kernels", Spy)
+    whole = ops.moe(x, router, wgu, wd, k, E).float()
+    of_whole, used[:] = set(used), []
+    parts = [ops.moe(x, router, wgu[e:e + 1].contiguous(), wd[e:e + 1].contiguous(), k, E, e)
+             for e in range(E)]
+    assert of_whole == set(used) == {kernel}
+    # the shards' sums round to bf16 one by one
+    torch.testing.assert_close(sum(p.float() for p in parts), whole, atol=2e-2, rtol=2e-2)
