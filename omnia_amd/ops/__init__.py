@@ -932,15 +932,23 @@ def cosine_topk(q: torch.Tensor, m: torch.Tensor, k: int, valid: torch.Tensor | 
 
 # ------------------------------------------------------------- MoE (K14)
 MOE_LIBRARY_ROWS = 1024  # mean rows/expert above which eager calls use hipBLASLt per expert
-# mean rows per local expert from which the grouped GEMMs run on the 256x256
-# prefill tile (pgemm.hip EPI 5 / 6, 256-row expert segments); below it smaller
-# segments (moe_panel_rows) waste less padding.  All are graph-safe.
-# Both products, 64-row / 256-row: at 96 rows 164 / 204 us, at 128 213 / 208, at 512
-# 652 / 268 (8 experts of 2048 x 4096); at 96 174 / 190, at 128 202 / 193 (32 of 2048 x
-# 1024).  128-row / 256-row: at 128 141 / 199, at 160 173 / 201, at 256 245 / 208 (the first);
-# at 128 169 / 183, at 188 215 / 193 (the second); at 128 830 / 858, at 160 1069 / 869 (8 of
-# 4096 x 14336): it crosses between 128 and 230
 MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
+
+
+def moe_tile_rows(experts: int, d: int) -> int:
+    """Mean rows an expert from which ``experts`` (a shard's own) run on the 256x256 prefill tile
+    (pgemm.hip EPI 5 / 6, 256-row segments); below it smaller segments (:func:`moe_panel_rows`)
+    waste less padding.
+
+    A segment costs the tile the same up to 256 rows and the panel kernel one step for each 128,
+    so the line lies near 128 rows where the tiles of the down product fill half the chip, and
+    where they do not, near 224.  Both products, us, 128-row segments (packed) / tile: 8 experts
+    of 4096 x 14336 (128 tiles) at 112 rows 604 / 842, at 128 877 / 846, at 150 1053 / 859; 8 of
+    2048 x 4096 (64 tiles) at 128 142 / 198, at 200 168 / 203, at 250 223 / 207; of 2048 x 3072 at
+    128 117 / 174, at 200 132 / 178, at 250 177 / 183; ungated of 2048 x 6144 at 140 163 / 252 (the
+    64-row kernel 230), at 200 165 / 257, at 260 236 / 258; 3 of 4096 x 7168 at 133 211 / 241, at
+    233 225 / 250, at 267 341 / 309."""
+    return max(MOE_TILE256_ROWS, 128 if experts * (d // 256) >= 128 else 224)
 
 
 def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
@@ -963,16 +971,18 @@ def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tenso
     """Segment rows of the panel kernel for ``n`` assignments to ``experts`` experts (all of them,
     where a shard holds some), 0 where moe.hip's 64-row kernel does better.
 
-    From 56 rows an expert most would need two segments of 64, so the weights are read twice;
-    segments of 128 read them once (both products, us, 64-row kernel / 128-row segments at 64 / 100 / 128
-    rows: 8 experts of 2048 x 4096 122 / 156 / 196 and 109 / 114 / 141, of 4096 x 14336 798 / 1049
-    / 1296 and 547 / 588 / 830; 32 of 2048 x 1024 135 / 167 / 194 and 126 / 133 / 175).  Fewer rows
-    gain from whole-line reads of packed weights where K is long (8 to 32 rows, 64-row kernel /
-    64-row segments: 94 / 84, 494 / 445; 32 of 2048 x 1024 90 / 96)."""
+    From 64 rows an expert most need two segments of 64, so the weights are read twice;
+    segments of 128 read them once (both products, us, 64-row kernel / 128-row segments, as they
+    are and packed, at 56 / 64 / 75 / 100 rows: 8 experts of 2048 x 4096 99 / 123 / 148 / 159, 119 /
+    120 / 123 / 126 and 106 / 105 / 108 / 113; of 4096 x 14336 567 / 752 / 971 / 1048, 584 / 593 /
+    604 / 634 and 538 / 544 / 564 / 600; of 2048 x 3072 78 / 99 / 112 / 117, 99 / 101 / 103 / 107 and
+    89 / 90 / 93 / 96).  Fewer rows gain from whole-line reads of packed weights where K is long (8
+    to 56 rows, 64-row kernel / 64-row segments: the first 94 / 82 to 99 / 92, the second 495 / 446
+    to 567 / 527, the third 75 / 70 to 78 / 80; 32 of 2048 x 1024 90 / 97)."""
     if not (_stream_on and w_up.dtype == torch.bfloat16 and w_up.is_cuda and all(
             w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down))):
         return 0
-    if n >= 56 * experts:
+    if n >= 64 * experts:
         return 128
     return 64 if packed and min(w_up.shape[2], w_down.shape[2]) >= 2048 else 0
 
@@ -1093,7 +1103,7 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
     kk.moe_router_topk(ids, wts, x.contiguous(), router, k, renorm)
     out = torch.empty_like(x)
     d, inter = x.shape[1], w_down.shape[2]
-    if n >= MOE_TILE256_ROWS * n_experts and d % 256 == 0 and inter % 128 == 0:
+    if n >= moe_tile_rows(e_hi - e_lo, d) * n_experts and d % 256 == 0 and inter % 128 == 0:
         # prefill-sized: the 256x256 MFMA tile, grouped by 256-row expert segments
         # (pgemm.hip EPI 5 / 6) -- hand kernels, graph-safe, no per-expert library
         # calls and no host sync

@@ -86,7 +86,8 @@ def test_moe_library_path_matches_grouped(monkeypatch):
     (2048, 512, 512, 8, 2, 0, 8),    # prefill-sized: 256x256-tile grouped GEMMs
     (2500, 256, 384, 8, 2, 0, 8),    # ragged expert segments, I not a multiple of 256
     (4096, 512, 256, 8, 2, 4, 4),    # expert-parallel shard: experts 4..7 only
-    (513, 256, 256, 8, 2, 0, 8),     # from 128 rows an expert, segments half full
+    (897, 256, 256, 8, 2, 0, 8),     # from 224 rows an expert, segments not full
+    (4097, 512, 128, 64, 2, 0, 64),  # from 128 where the down product has 128 tiles
 ])
 def test_moe_tile256_prefill_matches_reference(T, d, I, E, k, e_lo, e_n):
     """Large batches run the 256-row-segment grouped GEMMs (pgemm.hip EPI 5 / 6)
@@ -96,7 +97,7 @@ def test_moe_tile256_prefill_matches_reference(T, d, I, E, k, e_lo, e_n):
     router, wgu, wd = _weights(E, d, I, g)
     x = (torch.randn(T, d, generator=g)).to(torch.bfloat16).cuda()
     wgu_l, wd_l = wgu[e_lo:e_lo + e_n].contiguous(), wd[e_lo:e_lo + e_n].contiguous()
-    assert T * k >= ops.MOE_TILE256_ROWS * E  # the 256-tile path is the one under test
+    assert T * k >= ops.moe_tile_rows(e_n, d) * E  # the 256-tile path is the one under test
     out = ops.moe(x, router, wgu_l, wd_l, k, E, e_lo, graph_safe=True)
     logits = torch.nn.functional.linear(x, router)
     rid, rw = ref.moe_route(logits.float().cpu(), k)

@@ -209,13 +209,20 @@ def test_experts_in_panel_segments(bm, T, E, k, glu, gelu, packed, monkeypatch):
     assert ((got - want).abs() <= 4 * U * want.abs().clamp(min=want.pow(2).mean().sqrt())).all()
 
 
-def test_panel_segments_by_rows_an_expert():
+def test_segments_by_rows_an_expert():
+    """Segments grow with the rows an expert has, the 256-row tile last, and only weights that the
+    panel kernel covers take it."""
     up, down = (torch.empty(8, *s, dtype=torch.bfloat16, device="cuda")
                 for s in ((256, 2048), (2048, 2048)))
-    assert [ops.moe_panel_rows(n, 8, up, down, True) for n in (65, 447, 448)] == [64, 64, 128]
-    assert [ops.moe_panel_rows(n, 8, up, down, False) for n in (65, 447, 448)] == [0, 0, 128]
+    for packed in (False, True):
+        segs = [ops.moe_panel_rows(n, 8, up, down, packed) for n in range(65, 4096, 13)]
+        assert segs == sorted(segs) and set(segs) <= {0, 64, 128} and segs[-1] == 128
+        assert packed or 64 not in segs
     assert ops.moe_panel_rows(100, 8, up[..., :1024], down[:, :1024], True) == 0
-    assert ops.moe_panel_rows(448, 8, up.float(), down, True) == 0
+    assert ops.moe_panel_rows(1000, 8, up.float(), down, True) == 0
+    # a tile covers what 128-row segments begin with, and few tiles wait for fuller ones
+    assert ops.moe_panel_rows(8 * ops.moe_tile_rows(8, 4096) - 1, 8, up, down, False) == 128
+    assert ops.moe_tile_rows(8, 2048) > ops.moe_tile_rows(8, 4096) == ops.moe_tile_rows(64, 512)
 
 
 def test_what_is_refused():
