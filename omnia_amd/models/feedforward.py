@@ -50,7 +50,7 @@ class DenseGLU:
         m, W, b, act = self.model, w["gate_up"], w["gate_up_b"], self.spec.act
         M, K = h.shape
         N = W.shape[0]
-        if m._pgemm_ok(M, K, N // 2, is_decode, 128) and (b is None or act == "silu"):
+        if m._pgemm_ok(M, K, N // 2, is_decode, W) and (b is None or act == "silu"):
             return ops.pgemm(1, h, W, bias=b, gelu=act == "gelu_tanh")
         copy = w.get("gate_up_stream")
         if ops.stream_ok(M, W, gated=True):

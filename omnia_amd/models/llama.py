@@ -270,7 +270,7 @@ class LlamaModel(Projections):
     def mlp(self, layer: dict, h: torch.Tensor, is_decode: bool = False):
         M, K = h.shape
         I2 = layer["gate_up"].shape[0]
-        if self._pgemm_ok(M, K, I2 // 2, is_decode, 128):
+        if self._pgemm_ok(M, K, I2 // 2, is_decode, layer["gate_up"]):
             # gate_up + SwiGLU in the prefill kernel's epilogue (pgemm EPI 1)
             return self._proj("down", ops.pgemm(1, h, layer["gate_up"]), layer["down"], False)
         cfg = self._wcfg(M, I2 // 2, K, 1, is_decode)
@@ -456,7 +456,9 @@ class LlamaModel(Projections):
         ss = ops.row_sumsq(h).view(T, 1)
 
         def stream(epi, x, w, **kw):
-            w, packed = self._stream_weight(T, w, epi == 1)
+            # the first layer's are covered; another's may lie off the 16-byte grid
+            w, packed = self._stream_weight(T, w, epi == 1) or (
+                w.clone(memory_format=torch.contiguous_format), False)
             return ops.stream(epi, x, w, packed=packed, **kw)
 
         mid, end = (ops.stream_sums(T, self.w["layers"][0][k], h.device) for k in ("o", "down"))

@@ -182,16 +182,19 @@ class Projections:
 
     _min_rows = int(os.environ.get("OMNIA_PGEMM_MIN_ROWS", "2049"))  # this forward's threshold (mixed steps: the higher one)
 
-    def _pgemm_ok(self, M: int, K: int, N: int, is_decode: bool, tn: int = 256) -> bool:
+    def _pgemm_ok(self, M: int, K: int, N: int, is_decode: bool,
+                  gated: torch.Tensor | None = None) -> bool:
         """A prefill-sized projection the hand 256x256 MFMA kernel covers (the
         unfused paths: TP shards, MoE attention, CP): K whole 128-k iterations,
-        N whole column tiles, and at least this forward's row threshold, or for a
-        gated one (tn 128) tiles that fill the chip."""
+        N whole column tiles (``gated``: of a gate's and an up's half, N features
+        each of this weight), and at least this forward's row threshold, or for a
+        gated one tiles that fill the chip."""
         # TP ranks rehearsed on ONE device (ipc transport) keep the library GEMMs:
         # a 256x256 tile's 132 KB of LDS cannot share a CU with the peers'
         # spinning all-reduce blocks, so a rank's GEMM can wait out their spin
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
-        rows = M >= self._min_rows or (tn == 128 and ops.gated_tile_fills(M, N))
+        tn = 256 if gated is None else 128
+        rows = M >= self._min_rows or (tn == 128 and ops.gated_tile_fills(M, gated))
         return (self.use_pgemm and not is_decode and self.device.type == "cuda"
                 and self.dtype == torch.bfloat16
                 and rows and K % 128 == 0 and N % tn == 0

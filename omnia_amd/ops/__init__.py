@@ -440,15 +440,17 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     return out
 
 
-def gated_tile_fills(M: int, N: int) -> bool:
-    """Whether the 256 x 128-feature tiles of a gated :func:`pgemm` of more rows than the panel
-    kernel takes are worth their rounds over 256 CUs: from three quarters of their work useful,
+def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
+    """Whether a gated :func:`pgemm` of more rows than the panel kernel takes covers ``w`` = [Wg; Wu]
+    and its tiles of 256 rows x 128 features are worth their rounds over 256 CUs: from three quarters of their work useful,
     the activation in the epilogue makes up for the rest (useful part, us here / library and
     activation kernel; 8192 features of 2048: 512 rows .50 48 / 42, 768 .75 51.5 / 52.7, 999 .98
     55 / 67, 1536 .75 99 / 99, 2001 .98 108 / 124; 14336 of 4096: 320 .55 93 / 88, 512 .88 99 / 112,
     768 .66 177 / 163, 999 .85 187 / 198)."""
+    N = w.shape[0] // 2
     rounds = -(-(-(-M // 256) * (N // 128)) // 256)
-    return M > PANEL_MAX_M and M * N > 0.75 * 256 * 256 * 128 * rounds
+    return M > PANEL_MAX_M and M * N > 0.75 * 256 * 256 * 128 * rounds and \
+        w.is_contiguous() and _on_grid(w)
 
 
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
@@ -480,12 +482,18 @@ def streams_on() -> bool:
     return _stream_on
 
 
+def _on_grid(*ts: torch.Tensor) -> bool:
+    """Whether 16-byte loads of these tensors are aligned."""
+    return all(t.data_ptr() % 16 == 0 for t in ts)
+
+
 def stream_ok(M: int, w: torch.Tensor, gated: bool = False) -> bool:
     """Whether :func:`stream` and :func:`panel` cover ``M`` rows of this GPU weight
     (:func:`few_rows` chooses)."""
+    if not (_stream_on and 1 <= M <= PANEL_MAX_M and w.is_cuda and w.dtype == torch.bfloat16):
+        return False
     R, K = w.shape[-2:]
-    return (_stream_on and w.is_cuda and 1 <= M <= PANEL_MAX_M and w.dtype == torch.bfloat16
-            and K % 64 == 0 and R % (32 if gated else 16) == 0 and w.is_contiguous())
+    return K % 64 == 0 and R % (32 if gated else 16) == 0 and w.is_contiguous() and _on_grid(w)
 
 
 def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bool = False,
@@ -961,9 +969,15 @@ def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor
     kernel 52 / 90 / 82 / 93 / 93 / 93, packed 25 / 63 / 58 / 72 / 74 / 95; 4096 x 14336: 193 /
     383 / 470 / 472 / 475 / 477 and 111 / 315 / 418 / 419 / 431 / 602.  Row-major weights gain
     only where most experts have no row: 29 for 52 and 133 for 193 at 1 token."""
-    return (_stream_on and w_up.dtype == torch.bfloat16 and w_up.is_cuda
-            and n <= (8 * experts if packed else (experts - 1) // 2)
-            and all(w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down)))
+    return n <= (8 * experts if packed else (experts - 1) // 2) and _moe_few_ok(w_up, w_down)
+
+
+def _moe_few_ok(*ws: torch.Tensor) -> bool:
+    """Whether the streaming and panel kernels cover these expert weights: the shapes that
+    moe.hip takes, on the 16-byte grid."""
+    return (_stream_on and _on_grid(*ws) and all(
+        w.is_cuda and w.dtype == torch.bfloat16 and w.shape[1] % 64 == 0 and w.shape[2] % 64 == 0
+        for w in ws))
 
 
 def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
@@ -979,8 +993,7 @@ def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tenso
     89 / 90 / 93 / 96).  Fewer rows gain from whole-line reads of packed weights where K is long (8
     to 56 rows, 64-row kernel / 64-row segments: the first 94 / 82 to 99 / 92, the second 495 / 446
     to 567 / 527, the third 75 / 70 to 78 / 80; 32 of 2048 x 1024 90 / 97)."""
-    if not (_stream_on and w_up.dtype == torch.bfloat16 and w_up.is_cuda and all(
-            w.shape[1] % 32 == 0 and w.shape[2] % 64 == 0 for w in (w_up, w_down))):
+    if not _moe_few_ok(w_up, w_down):
         return 0
     if n >= 64 * experts:
         return 128
@@ -1005,6 +1018,8 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     elif bm == 64:
         panel = moe_panel_rows(n, n_experts, w_gu, w_down, streams is not None)
         bm = panel or bm
+    if bm != 64 and not _on_grid(x):  # moe.hip takes rows as they lie
+        x = x.clone()
     mb = kk.moe_max_blocks(n, experts, bm)
     # a wave of the streaming kernel sorts 64 assignments by itself, an expert a step
     own = few and n <= 64 and experts <= 64
@@ -1103,7 +1118,8 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
     kk.moe_router_topk(ids, wts, x.contiguous(), router, k, renorm)
     out = torch.empty_like(x)
     d, inter = x.shape[1], w_down.shape[2]
-    if n >= moe_tile_rows(e_hi - e_lo, d) * n_experts and d % 256 == 0 and inter % 128 == 0:
+    if n >= moe_tile_rows(e_hi - e_lo, d) * n_experts and d % 256 == 0 and \
+            inter % 128 == 0 and _on_grid(w_gu, w_down):
         # prefill-sized: the 256x256 MFMA tile, grouped by 256-row expert segments
         # (pgemm.hip EPI 5 / 6) -- hand kernels, graph-safe, no per-expert library
         # calls and no host sync

@@ -11,7 +11,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _moe_grouped, checks, kernels, moe_tile_rows
+from . import _moe_grouped, _on_grid, checks, kernels, moe_tile_rows
 from . import reference_mixers as ref
 
 
@@ -229,7 +229,7 @@ def experts(h, w: dict, spec):
                  spec.groups, spec.keep, bias)
     # column tiles of the 256-row prefill GEMM: 128 gate and up columns, or 256
     tile = h.dtype == torch.bfloat16 and d % 256 == 0 and \
-        T * k >= moe_tile_rows(spec.experts, d) * E and \
+        T * k >= moe_tile_rows(spec.experts, d) * E and _on_grid(w["up"], w["down"]) and \
         ff % (128 if spec.gated else 256) == 0
     y = _moe_grouped(h, w["up"], w["down"], ids, wts, k, E, 0, spec.experts, 256 if tile else 64,
                      (spec.alpha, spec.limit) if spec.expert == "clamped_glu" else None,

@@ -241,6 +241,82 @@ def test_what_is_refused():
         ops.panel(0, x[:4], w[:40].contiguous())
 
 
+def _off_grid(t, at=1):
+    """``t`` at an address ``at`` elements past the 16-byte grid."""
+    buf = torch.empty(t.numel() + at, dtype=t.dtype, device=t.device)
+    return buf[at:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("M", [1, 16, 40, 200])
+def test_weights_the_kernels_do_not_cover_take_the_library(M, strided):
+    """Off the 16-byte grid or strided: projections that ran before these kernels still run."""
+    from omnia_amd.models.projection import Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device("cuda"), torch.bfloat16, 1, {}
+
+    x, w = _mk(M, 64, 128, M)
+    v = F.pad(w, (0, 8))[:, :128] if strided else _off_grid(w)
+    assert not ops.stream_ok(M, v) and ops.stream_ok(M, w)
+    y = Model()._proj("o", x, v, True)
+    _close(y, x.double() @ w.double().T, 128)
+
+
+@pytest.mark.parametrize("key", ["qkv", "o", "gate_up", "down"])
+def test_a_layer_with_a_weight_off_the_grid(key):
+    """Steps of a few rows run, and give the same, where only a later layer's weight is so."""
+    from omnia_amd.models import build_model, resolve
+
+    out = []
+    for off in (False, True):
+        m = build_model(resolve("tiny-llama"), device="cuda", seed=3)
+        if off:
+            m.w["layers"][1][key] = _off_grid(m.w["layers"][1][key])
+        out.append(_step(m, 4))
+    assert torch.equal(*out)
+
+
+def _step(m, rows, past=40):
+    """Logits of a decode step of ``rows`` sequences."""
+    from omnia_amd.models import allocate_cache
+    from omnia_amd.models.llama import ForwardBatch
+
+    bs, per, g = 32, -(-(past + 1) // 32), torch.Generator(device="cuda").manual_seed(rows)
+    kv = allocate_cache(m, rows * per + 1, bs, "cuda", torch.bfloat16, rows + 1)
+    for t in kv.page_tensors():
+        t.normal_(generator=g)
+    bt = (torch.arange(rows * per, device="cuda", dtype=torch.int32) + 1).view(rows, per)
+
+    def full(n):
+        return torch.full((rows,), n, dtype=torch.int32, device="cuda")
+
+    ids = torch.randint(0, m.cfg.vocab_size, (rows,), generator=g, device="cuda").int()
+    fb = ForwardBatch(ids, full(past), bt[:, past // bs].long() * bs + past % bs, bt,
+                      full(past + 1), torch.arange(rows, device="cuda"), num_seqs=rows)
+    return m.forward(fb, kv).float()
+
+
+@pytest.mark.parametrize("T", [3, 40, 1000])
+def test_expert_rows_and_weights_off_the_grid(T):
+    """Rows are copied where a kernel reads 16 bytes at a time; weights stay with moe.hip, and so
+    do shapes that it refuses."""
+    E, d, k = 4, 256, 2
+    g = torch.Generator(device="cuda").manual_seed(T)
+    _, up = _mk(1, 256, d, 3, (E,))
+    _, down = _mk(1, d, 128, 4, (E,))
+    x = torch.randn(T, d, generator=g, device="cuda").to(torch.bfloat16)
+    router = torch.randn(E, d, generator=g, device="cuda").to(torch.bfloat16)
+    want = ops.moe(x, router, up, down, k, E)
+    assert torch.equal(ops.moe(_off_grid(x), router, up, down, k, E), want)
+    for ws in ((_off_grid(up), down), (up, _off_grid(down))):
+        assert not ops.moe_stream_ok(1, E, *ws, True) and not ops.moe_panel_rows(999, E, *ws, True)
+        got = ops.moe(x, router, *ws, k, E).double()
+        assert (got - want).norm() <= 2 * U * want.double().norm()
+    part = up[:, :224].contiguous(), F.pad(down[:, :, :112], (0, 16))
+    assert not ops.moe_stream_ok(1, E, *part, True) and not ops.moe_panel_rows(999, E, *part, True)
+
+
 # rows around the tiles of 64 to 256; columns of fewer units than waves and of a remainder;
 # K of one chunk, of slices of unequal length and of fewer chunks than the ring has stages
 PANEL = [(1, 16, 64), (17, 48, 128), (63, 272, 576), (64, 2048, 8192), (65, 528, 1024),
@@ -330,10 +406,17 @@ def test_llama_layers_match_the_unfused_path(rows, pack, monkeypatch):
 
 
 def test_gated_tiles_are_taken_where_they_fill_the_chip():
-    assert [m for m in (256, 512, 768, 769, 1024, 1025, 1536, 1537, 2048)
-            if ops.gated_tile_fills(m, 8192)] == [769, 1024, 1537, 2048]
-    assert [m for m in (320, 439, 440, 512, 513, 878, 879, 1024)
-            if ops.gated_tile_fills(m, 14336)] == [439, 440, 512, 878, 879, 1024]
+    """Only for more rows than the panel kernel takes, not where one row more leaves most of a
+    round empty, and only for weights that the tile covers."""
+    for N in (8192, 14336):
+        w = torch.empty(2 * N, 128, dtype=torch.bfloat16, device="cuda")
+        taken = [M for M in range(1, 2049) if ops.gated_tile_fills(M, w)]
+        assert min(taken) > ops.PANEL_MAX_M and 2048 in taken
+        for M in taken:  # a round of 256 tiles of 256 x 128, three quarters of it useful
+            tiles = -(-M // 256) * (N // 128)
+            assert M * N / (-(-tiles // 256) * 256 * 256 * 128) > 0.75
+        assert not ops.gated_tile_fills(2048, _off_grid(w))
+        assert not ops.gated_tile_fills(2048, F.pad(w, (0, 8))[:, :128])
 
 
 @pytest.mark.parametrize("M", [511, 512, 513])
@@ -345,8 +428,9 @@ def test_gated_projection_on_both_sides_of_the_rule(M):
         device, dtype, tp, _ws = torch.device("cuda"), torch.bfloat16, 1, {}
 
     m, N, K = Model(), 32768, 128
-    assert m._pgemm_ok(M, K, N, False, 128) == (M <= 512)
-    assert not m._pgemm_ok(M, K, N, False) and not m._pgemm_ok(M, K, N, True, 128)
     x, w = _mk(M, 2 * N, K, 5)
+    assert m._pgemm_ok(M, K, N, False, w) == (M <= 512)
+    assert not m._pgemm_ok(M, K, N, False) and not m._pgemm_ok(M, K, N, True, w)
+    assert not m._pgemm_ok(M, K, N, False, _off_grid(w))
     g, u = (x.double() @ w.double().t()).split(N, 1)
     _close(ops.pgemm(1, x, w), F.silu(g) * u, K)
