@@ -12,6 +12,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import mixers as mops
+from .projection import packed_copy, packed_experts
 
 
 def _up8(n: int) -> int:
@@ -52,8 +53,8 @@ class DenseGLU:
         N = W.shape[0]
         if m._pgemm_ok(M, K, N // 2, is_decode, W) and (b is None or act == "silu"):
             return ops.pgemm(1, h, W, bias=b, gelu=act == "gelu_tanh")
-        copy = w.get("gate_up_stream")
         if ops.stream_ok(M, W, gated=True):
+            copy = packed_copy(m, W)
             return ops.few_rows(1, h, W if copy is None else copy, copy is not None, bias=b,
                                 gelu=act == "gelu_tanh")
         cfg = m._wcfg(M, N // 2, K, 1, is_decode)
@@ -102,7 +103,8 @@ class Experts:
         return w
 
     def forward(self, w: dict, h: torch.Tensor, is_decode: bool) -> dict:
-        parts, ids, wts = mops.experts(h, w, self.spec)
+        parts, ids, wts = mops.experts(h, w, self.spec,
+                                       packed_experts(self.model, w["up"], w["down"]))
         out = {"m": parts, "slots": True}
         if self.spec.identity:
             out["identity"] = (ids, wts, h, self.spec.experts)

@@ -206,15 +206,8 @@ class HybridModel(Projections):
         return w
 
     def prepack_decode(self, max_batch: int) -> int:
-        """Lay projections out for small decode batches; returns the bytes.  Feed-forwards find
-        the copies of theirs beside the weights."""
-        n = self.pack_streams()
-        for w in self.w["layers"]:
-            for m in (w["mlp"], (w["mlp"] or {}).get("shared")):
-                for k in ("gate_up", "up", "down") if m else ():
-                    if k in m and m[k].data_ptr() in self._streams:
-                        m[k + "_stream"] = self._streams[m[k].data_ptr()]
-        return n
+        """Lay projections out for small decode batches; returns the bytes."""
+        return self.pack_streams()
 
     # ------------------------------------------------------------ cache
     def allocate_cache(self, num_blocks: int, block_size: int, n_slots: int) -> HybridCache:

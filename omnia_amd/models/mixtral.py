@@ -27,6 +27,7 @@ import torch
 from .. import ops
 from ..parallel import state as pstate
 from .llama import LlamaModel, _init
+from .projection import packed_experts
 
 
 class MixtralModel(LlamaModel):
@@ -86,8 +87,8 @@ class MixtralModel(LlamaModel):
         return ops.moe(h, layer["router"], layer["experts_gate_up"], layer["experts_down"],
                        self.cfg.experts_per_token, self.cfg.num_experts, self.e_lo,
                        graph_safe=self.graph_safe or h.shape[0] < 64,
-                       streams=self.expert_streams(layer["experts_gate_up"],
-                                                   layer["experts_down"]))
+                       streams=packed_experts(self, layer["experts_gate_up"],
+                                              layer["experts_down"]))
 
     def forward(self, fb, kv, gather: bool = True):
         # decode batches are captured into hipGraphs: keep the MoE path sync-free

@@ -36,6 +36,24 @@ class RowPar:
         self.x, self.w = x, w
 
 
+def _version(t: torch.Tensor) -> int:
+    """Counts in-place writes (inference tensors do not)."""
+    return 0 if t.is_inference() else t._version
+
+
+def packed_copy(model, w: torch.Tensor) -> torch.Tensor | None:
+    """The model's packed copy of a weight (``Projections.pack_streams``), while the weight is
+    what was copied."""
+    t, version, copy = getattr(model, "_streams", {}).get(w.data_ptr(), (None, None, None))
+    return copy if copy is not None and t.shape == w.shape and version == _version(w) else None
+
+
+def packed_experts(model, up: torch.Tensor, down: torch.Tensor):
+    """Packed copies of a layer's expert weights, or None."""
+    t = packed_copy(model, up), packed_copy(model, down)
+    return None if t[0] is None or t[1] is None else t
+
+
 class Projections:
     """Needs ``device``, ``dtype``, ``tp`` and ``_ws`` (workspace dict) on the model."""
 
@@ -58,10 +76,14 @@ class Projections:
     STREAM_KEYS = {"qkv", "o", "gate_up", "down", "up", "in", "uq", "experts_gate_up",
                    "experts_down"}
 
+    # address -> (weight, its version, copy): the weight is held, so that no other takes its
+    # address, and a copy counts only while the weight is what was copied
+    _streams: dict = {}
+
     def pack_streams(self) -> int:
         """Lay the projection weights out for :func:`ops.stream`; returns the bytes (0: off, or
-        over budget)."""
-        self._streams: dict = {}
+        over budget).  Weights replaced or written to afterwards run as they are."""
+        self._streams = {}
         if self.device.type != "cuda" or self.dtype != torch.bfloat16 or self.tp != 1:
             return 0
         found: dict = {}
@@ -79,7 +101,7 @@ class Projections:
         cap = torch.cuda.get_device_properties(self.device).total_memory * self.stream_budget_frac
         if total > cap:
             return 0
-        self._streams = {p: ops.stream_pack(t) for p, t in found.items()}
+        self._streams = {p: (t, _version(t), ops.stream_pack(t)) for p, t in found.items()}
         return total
 
     def _stream_weight(self, M: int, w: torch.Tensor, gated: bool = False):
@@ -87,14 +109,8 @@ class Projections:
         kernel, or None for the other paths."""
         if self.device.type != "cuda" or self.tp != 1 or not ops.stream_ok(M, w, gated):
             return None
-        t = getattr(self, "_streams", {}).get(w.data_ptr())
+        t = packed_copy(self, w)
         return (w, False) if t is None else (t, True)
-
-    def expert_streams(self, up: torch.Tensor, down: torch.Tensor):
-        """Packed copies of a layer's expert weights, or None."""
-        packs = getattr(self, "_streams", {})
-        t = packs.get(up.data_ptr()), packs.get(down.data_ptr())
-        return None if t[0] is None or t[1] is None else t
 
     def _few(self, epi: int, x: torch.Tensor, w: torch.Tensor, slabs: bool = False, **kw):
         """A plain (epi 0) or gated (1) projection of up to 256 rows: its rows or, with ``slabs``,

@@ -211,11 +211,11 @@ def softcap_(logits: torch.Tensor, cap: float) -> torch.Tensor:
 
 
 # -------------------------------------------------------------------- experts
-def experts(h, w: dict, spec):
+def experts(h, w: dict, spec, streams=None):
     """Routed experts: (parts [T, top, d], ids, weights), the parts summed by the residual
     kernel; those of identity experts (ids >= spec.experts) are not written.  The weights
-    are padded to whole tiles (``ff_pad``; d a multiple of 64); ``up_stream`` and
-    ``down_stream`` are copies by :func:`omnia_amd.ops.stream_pack`, if there."""
+    are padded to whole tiles (``ff_pad``; d a multiple of 64); ``streams``: copies of both by
+    :func:`omnia_amd.ops.stream_pack`, or None."""
     T, d = h.shape
     k, E, ff = spec.top, spec.outputs, w["down"].shape[2]
     corr, bias = w.get("correction"), w.get("router_b")
@@ -233,8 +233,7 @@ def experts(h, w: dict, spec):
         ff % (128 if spec.gated else 256) == 0
     y = _moe_grouped(h, w["up"], w["down"], ids, wts, k, E, 0, spec.experts, 256 if tile else 64,
                      (spec.alpha, spec.limit) if spec.expert == "clamped_glu" else None,
-                     not spec.gated,
-                     (w["up_stream"], w["down_stream"]) if "up_stream" in w else None)
+                     not spec.gated, streams)
     return y.view(T, k, d), ids, wts
 
 

@@ -294,7 +294,44 @@ def _step(m, rows, past=40):
     ids = torch.randint(0, m.cfg.vocab_size, (rows,), generator=g, device="cuda").int()
     fb = ForwardBatch(ids, full(past), bt[:, past // bs].long() * bs + past % bs, bt,
                       full(past + 1), torch.arange(rows, device="cuda"), num_seqs=rows)
+    if getattr(m, "stateful", False):
+        fb.state_slots = torch.arange(1, rows + 1, dtype=torch.int32, device="cuda")
     return m.forward(fb, kv).float()
+
+
+@pytest.mark.parametrize("write", [True, False])
+@pytest.mark.parametrize("rows", [3, 40])
+@pytest.mark.parametrize("name", ["tiny-llama", "tiny-mixtral", "tiny-sivadra", "tiny-sekazen"])
+def test_packed_copies_of_weights_that_change(name, rows, write):
+    """Weights written to, or replaced by others (which may take the old ones' addresses), are
+    what a step computes with from then on."""
+    from omnia_amd.models import build_model, resolve
+
+    def change(v):
+        for k in v if isinstance(v, dict) else range(len(v)):
+            t = v[k]
+            if isinstance(t, (dict, list)):
+                change(t)
+            elif k in type(m).STREAM_KEYS and isinstance(t, torch.Tensor):
+                new = t.flip(-1)
+                if write:
+                    t.copy_(new)
+                else:
+                    v[k] = None
+                    del t  # the last reference but the model's own
+                    v[k] = new.clone()
+
+    out = []
+    for pack in (True, False):
+        m = build_model(resolve(name), device="cuda", seed=3)
+        if pack:
+            assert m.prepack_decode(rows) > 0
+            before = _step(m, rows)
+        change(m.w["layers"])
+        out.append(_step(m, rows))
+    assert not torch.equal(before, out[1])
+    # the copies' products sum in another order than the weights' as they are
+    assert (out[0] - out[1]).norm() <= 0.02 * out[1].norm()
 
 
 @pytest.mark.parametrize("T", [3, 40, 1000])
