@@ -88,7 +88,8 @@ class MixtralModel(LlamaModel):
                        self.cfg.experts_per_token, self.cfg.num_experts, self.e_lo,
                        graph_safe=self.graph_safe or h.shape[0] < 64,
                        streams=packed_experts(self, layer["experts_gate_up"],
-                                              layer["experts_down"]))
+                                              layer["experts_down"]),
+                       shared_device=self.tp > 1 and pstate.ranks_per_device() > 1)
 
     def forward(self, fb, kv, gather: bool = True):
         # decode batches are captured into hipGraphs: keep the MoE path sync-free

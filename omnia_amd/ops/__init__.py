@@ -1001,21 +1001,21 @@ def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tenso
 
 
 def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=None,
-                 gelu: bool = False, streams=None):
+                 gelu: bool = False, streams=None, shared_device: bool = False):
     """Grouped expert FFN over device-sorted assignments, no host sync: Y [T*k, d]
     (row t*k + j = slot j of token t, routing weight applied; other experts' rows
     unwritten).  ``bm`` 256: the 256x256 MFMA prefill tile; 64: moe.hip.  ``glu`` =
     (alpha, limit): clamped GLU experts whose INPUT takes the routing weight; ``gelu``:
     ungated experts (``w_gu`` [E, I, d]).  ``streams``: packed copies (:func:`stream_pack`) of
     both weights, or None; in place of ``bm`` 64, few assignments run :func:`moe_stream_ok`'s
-    kernel and others :func:`moe_panel_rows`'s."""
+    kernel and others :func:`moe_panel_rows`'s (not with ``shared_device``)."""
     kk = kernels()
     n, experts = ids.numel(), e_hi - e_lo
     few = bm == 64 and moe_stream_ok(n, n_experts, w_gu, w_down, streams is not None)
     panel = 0
     if few:
         bm = 16
-    elif bm == 64:
+    elif bm == 64 and not shared_device:
         panel = moe_panel_rows(n, n_experts, w_gu, w_down, streams is not None)
         bm = panel or bm
     if bm != 64 and not _on_grid(x):  # moe.hip takes rows as they lie
@@ -1096,7 +1096,7 @@ def moe_rows(rows: torch.Tensor, eids: torch.Tensor, w_gu: torch.Tensor, w_down:
 
 def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor,
         k: int, n_experts: int, e_lo: int = 0, renorm: bool = True,
-        graph_safe: bool = True, streams=None) -> torch.Tensor:
+        graph_safe: bool = True, streams=None, shared_device: bool = False) -> torch.Tensor:
     """Top-k MoE FFN over the local experts ``[e_lo, e_lo + w_gu.shape[0])``.
 
     x [T, d] bf16, router [E, d], w_gu [E_loc, 2I, d] (gate ; up), w_down [E_loc, d, I].
@@ -1104,7 +1104,10 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
     EP group to complete it).  ``graph_safe`` keeps every shape static and the
     whole path on device (hipGraph decode); otherwise large batches run each
     expert's GEMMs on hipBLASLt after one host sync on the expert counts.  ``streams``:
-    :func:`stream_pack` copies of both expert weights."""
+    :func:`stream_pack` copies of both expert weights.  ``shared_device``: other ranks run on this
+    device, whose all-reduce blocks may spin until this rank's next: a block of the 256-row tile or
+    the panel kernel holds most of a CU's LDS, does not fit beside them and could wait out their
+    spin bound; the other kernels' blocks fit."""
     e_hi = e_lo + w_gu.shape[0]
     if not x.is_cuda:
         return ref.moe(x, router, w_gu, w_down, k, e_lo, renorm).to(x.dtype)
@@ -1119,7 +1122,7 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
     out = torch.empty_like(x)
     d, inter = x.shape[1], w_down.shape[2]
     if n >= moe_tile_rows(e_hi - e_lo, d) * n_experts and d % 256 == 0 and \
-            inter % 128 == 0 and _on_grid(w_gu, w_down):
+            inter % 128 == 0 and _on_grid(w_gu, w_down) and not shared_device:
         # prefill-sized: the 256x256 MFMA tile, grouped by 256-row expert segments
         # (pgemm.hip EPI 5 / 6) -- hand kernels, graph-safe, no per-expert library
         # calls and no host sync
@@ -1145,6 +1148,7 @@ def moe(x: torch.Tensor, router: torch.Tensor, w_gu: torch.Tensor, w_down: torch
         Y.index_copy_(0, order, ys * wts.view(-1).index_select(0, order)[:, None].to(x.dtype))
         kk.moe_combine(out, Y, ids, k, e_lo, e_hi)
         return out
-    Y = _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, 64, streams=streams)
+    Y = _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, 64, streams=streams,
+                     shared_device=shared_device)
     kk.moe_combine(out, Y, ids, k, e_lo, e_hi)
     return out

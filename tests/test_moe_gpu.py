@@ -206,6 +206,21 @@ def test_router_topk_fused_matches_linear_then_topk(T, d, E, k):
     torch.testing.assert_close(w.cpu()[m], rw[m], atol=1e-2, rtol=1e-2)
 
 
+def _spied(monkeypatch):
+    """Names of the expert kernels that run from here on."""
+    used, native = [], ops.kernels()
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(native, name)
+            if not name.endswith(("_moe", "moe_gemm")):
+                return f
+            return lambda *a: (used.append(name), f(*a))[1]
+
+    monkeypatch.setattr(ops, "kernels", Spy)
+    return used
+
+
 @pytest.mark.parametrize("T,kernel", [(1, "stream_moe"), (64, "moe_gemm"), (300, "panel_moe"),
                                       (2000, "pgemm_moe")])
 def test_a_shard_counts_its_rows_over_all_experts(T, kernel, monkeypatch):
@@ -215,17 +230,7 @@ def test_a_shard_counts_its_rows_over_all_experts(T, kernel, monkeypatch):
     g = torch.Generator().manual_seed(T)
     router, wgu, wd = _weights(E, d, 256, g)
     x = torch.randn(T, d, generator=g).to(torch.bfloat16).cuda()
-    used = []
-
-    class Spy:
-        def __getattr__(self, name):
-            f = getattr(native, name)
-            if not name.endswith(("_moe", "moe_gemm")):
-                return f
-            return lambda *a: (used.append(name), f(*a))[1]
-
-    native = ops.kernels()
-    monkeypatch.setattr(ops, "kernels", Spy)
+    used = _spied(monkeypatch)
     whole = ops.moe(x, router, wgu, wd, k, E).float()
     of_whole, used[:] = set(used), []
     parts = [ops.moe(x, router, wgu[e:e + 1].contiguous(), wd[e:e + 1].contiguous(), k, E, e)
@@ -233,3 +238,26 @@ def test_a_shard_counts_its_rows_over_all_experts(T, kernel, monkeypatch):
     assert of_whole == set(used) == {kernel}
     # the shards' sums round to bf16 one by one
     torch.testing.assert_close(sum(p.float() for p in parts), whole, atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("T,kernel", [(1, "stream_moe"), (300, "moe_gemm"), (2000, "moe_gemm")])
+def test_ranks_that_share_a_device_take_blocks_of_little_lds(T, kernel, monkeypatch):
+    """Ranks on one device spin in all-reduce blocks beside this rank's: no tile or panel blocks.
+    The model asks for it wherever its ranks share a device."""
+    from types import SimpleNamespace
+
+    from omnia_amd.models import mixtral
+
+    d, E, k = 256, 8, 2
+    g = torch.Generator().manual_seed(T)
+    router, wgu, wd = _weights(E, d, 256, g)
+    x = torch.randn(T, d, generator=g).to(torch.bfloat16).cuda()
+    want = ops.moe(x, router, wgu, wd, k, E).float()
+    used = _spied(monkeypatch)
+    monkeypatch.setattr(mixtral.pstate, "ranks_per_device", lambda: 2)
+    m = SimpleNamespace(ep_mode="tp", tp=2, e_lo=0, graph_safe=True,
+                        cfg=SimpleNamespace(experts_per_token=k, num_experts=E))
+    got = mixtral.MixtralModel.mlp(
+        m, {"router": router, "experts_gate_up": wgu, "experts_down": wd}, x).float()
+    assert set(used) == {kernel}
+    torch.testing.assert_close(got, want, atol=2e-2, rtol=2e-2)
