@@ -56,9 +56,8 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst`` (m0,
-// which nothing else in this file uses).  NT: weights, read once (28672 x 4096 at 16 rows 47.0
-// -> 43.1 us row-major, 44.2 -> 39.9 packed)
+// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst`` (in m0).
+// NT: weights, read once (28672 x 4096 at 16 rows 47.0 -> 43.1 us row-major, 44.2 -> 39.9 packed)
 template <bool NT>
 __device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
   const uint32_t at = __builtin_amdgcn_readfirstlane(
@@ -66,11 +65,11 @@ __device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
   if constexpr (NT)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(at),
                  "v"(src)
-                 : "memory");
+                 : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at),
                  "v"(src)
-                 : "memory");
+                 : "memory", "m0");
 }
 
 // stages of (16 mf + 16 wn) x 128 bytes: up to 80 KB, two blocks a CU, where that is 3 stages
