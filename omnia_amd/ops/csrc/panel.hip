@@ -56,8 +56,11 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst`` (in m0).
-// NT: weights, read once (28672 x 4096 at 16 rows 47.0 -> 43.1 us row-major, 44.2 -> 39.9 packed)
+// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst``, which the
+// load takes from m0.  hipcc reserves m0: it allocates no value to it (and warns that a clobber of
+// it is undefined), and sets it for each instruction of its own that reads it; this file's have
+// none (in the listing m0 is written by these lines alone).  NT: weights, read once (28672 x 4096
+// at 16 rows 47.0 -> 43.1 us row-major, 44.2 -> 39.9 packed)
 template <bool NT>
 __device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
   const uint32_t at = __builtin_amdgcn_readfirstlane(
@@ -65,11 +68,11 @@ __device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
   if constexpr (NT)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(at),
                  "v"(src)
-                 : "memory", "m0");
+                 : "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at),
                  "v"(src)
-                 : "memory", "m0");
+                 : "memory");
 }
 
 // stages of (16 mf + 16 wn) x 128 bytes: up to 80 KB, two blocks a CU, where that is 3 stages
