@@ -55,8 +55,9 @@ class DenseGLU:
             return ops.pgemm(1, h, W, bias=b, gelu=act == "gelu_tanh")
         if ops.stream_ok(M, W, gated=True):
             copy = packed_copy(m, W)
-            return ops.few_rows(1, h, W if copy is None else copy, copy is not None, bias=b,
-                                gelu=act == "gelu_tanh")
+            if ops.few_rows_pay(M, N, K, True, copy is not None, False):
+                return ops.few_rows(1, h, W if copy is None else copy, copy is not None, bias=b,
+                                    gelu=act == "gelu_tanh")
         cfg = m._wcfg(M, N // 2, K, 1, is_decode)
         if cfg is not None:  # a tuned SwiGLU shape, as slabs (bias and activation follow)
             nw, nwaves, S = cfg

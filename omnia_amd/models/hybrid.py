@@ -308,7 +308,7 @@ class HybridModel(Projections):
 
     def logits(self, h: torch.Tensor, is_decode: bool = False) -> torch.Tensor:
         W = self.w["head"]
-        cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
+        cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode, W, False)
         if cfg is not None and cfg[2] == 1:
             z = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
         else:

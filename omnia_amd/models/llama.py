@@ -273,7 +273,7 @@ class LlamaModel(Projections):
         if self._pgemm_ok(M, K, I2 // 2, is_decode, layer["gate_up"]):
             # gate_up + SwiGLU in the prefill kernel's epilogue (pgemm EPI 1)
             return self._proj("down", ops.pgemm(1, h, layer["gate_up"]), layer["down"], False)
-        cfg = self._wcfg(M, I2 // 2, K, 1, is_decode)
+        cfg = self._wcfg(M, I2 // 2, K, 1, is_decode, layer["gate_up"])
         if cfg is None:
             a = self._few(1, h, layer["gate_up"])
             if a is None:
@@ -444,8 +444,18 @@ class LlamaModel(Projections):
         if fb.cp is not None or not self.fold_post_norm or cfg.head_dim != 128:
             return False
         T, layer = fb.input_ids.shape[0], self.w["layers"][0]
-        return T <= ops.STREAM_MAX_M and all(self._stream_weight(T, layer[k], k == "gate_up") is not None
-                   for k in ("qkv", "o", "gate_up", "down"))
+        if T > ops.STREAM_MAX_M:
+            return False
+        ws = [self._stream_weight(T, layer[k], k == "gate_up")
+              for k in ("qkv", "o", "gate_up", "down")]
+        if not all(ws):
+            return False
+        # row-major weights reach that kernel in pieces: separate kernels on the panel take 0.76
+        # of a step of 16 rows at 8192 x 28672, 0.92 at 4096 x 14336, 0.86 at 2048 x 8192 and 0.92
+        # at 1024 x 4096 (captured), and 1.4 where an eager step of layers of 34 MB waits for its
+        # launches
+        return all(packed for _, packed in ws) or \
+            (not fb.is_decode and sum(w.numel() for w, _ in ws) <= 1 << 25)
 
     def _stream_residual(self, fb: ForwardBatch, kv: KVCache) -> torch.Tensor:
         """Residual stream after the last layer (un-normalised) of a step of a few rows."""
@@ -507,7 +517,7 @@ class LlamaModel(Projections):
         only the slice).  Decode batches use the weight-streaming tile kernel
         when the measured table lists an unsplit (bf16-out) config for it."""
         W = self.w["lm_head"]
-        cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode)
+        cfg = self._wcfg(h.shape[0], W.shape[0], h.shape[1], 0, is_decode, W, False)
         if cfg is not None and cfg[2] == 1:
             lg = ops.wgemm(0, h, W, 1, cfg[0], cfg[1])
         else:

@@ -115,22 +115,34 @@ class Projections:
     def _few(self, epi: int, x: torch.Tensor, w: torch.Tensor, slabs: bool = False, **kw):
         """A plain (epi 0) or gated (1) projection of up to 256 rows: its rows or, with ``slabs``,
         perhaps its slabs; None for more rows and what the kernels do not cover."""
-        s = self._stream_weight(x.shape[0], w, epi == 1)
+        s = self._few_weight(x.shape[0], w, epi == 1, slabs)
         return None if s is None else ops.few_rows(epi, x, *s, slabs=slabs, **kw)
+
+    def _few_weight(self, M: int, w: torch.Tensor, gated: bool, slabs: bool):
+        """:meth:`_stream_weight` where those kernels beat the other paths."""
+        if M > ops.PANEL_MAX_M:
+            return None
+        s = self._stream_weight(M, w, gated)
+        return s if s and ops.few_rows_pay(M, *w.shape, gated, s[1], slabs) else None
 
     # Projections return either a bf16 tensor (library / gemm.hip path, not yet
     # TP-reduced) or :class:`Parts` (fp32 split-K slabs of the weight-streaming
     # kernel, wgemm.hip), which the NEXT kernel reduces while doing its own work:
     # QKV parts -> splitk_rope_kv (RoPE + paged KV write), O / down parts ->
     # splitk_add_rmsnorm (residual add + RMSNorm), gate_up parts -> splitk_swiglu.
-    def _wcfg(self, M: int, N: int, K: int, mode: int, is_decode: bool):
+    def _wcfg(self, M: int, N: int, K: int, mode: int, is_decode: bool,
+              w: torch.Tensor | None = None, slabs: bool = True):
+        """The tables' entry for a projection, None where ``w`` runs on the few-row kernels or the
+        library."""
         if self.device.type != "cuda" or self.dtype != torch.bfloat16:
             return None
-        # up to 192 rows the streaming and panel kernels are ahead of all paths in the tables,
-        # from there on behind the tile GEMM (us at 192 / 256 rows, panel and table: 6144 x 4096
-        # 19.7 / 23.0 and 21.1 / 21.2; 28672 x 4096 58 / 71 and 65 / 67; 4096 x 14336 33 / 41 and
-        # 36 / 39; 4096 x 4096 16.1 / 19.7 and 14.5 / 16.3)
-        if M <= 192 and self.tp == 1 and ops.streams_on() and N % 16 == 0 and K % 64 == 0:
+        # up to 192 rows the few-row kernels come before the tables.  With the consumer's reads of
+        # the slabs, us at 64 / 128 / 192 rows, packed panel (fp32 slabs) and table (fp16 from 65
+        # rows on): 6144 x 4096 18 / 22 / 26 and 19 / 20 / 24; 4096 x 4096 14 / 19 / 25 and 18 /
+        # 17 / 19; 4096 x 14336 28 / 36 / 41 and 33 / 37 / 38; gated 28672 x 4096 44 / 53 / 56 and
+        # (library at 64, 128) 56 / 62 / 62.  Beyond, the tables by more: 256 rows 28 and 25, 28
+        # and 21, 49 and 45, 69 and 66
+        if M <= 192 and w is not None and self._few_weight(M, w, mode == 1, slabs):
             return None
         if not is_decode:
             # mid-size steps below the prefill tile's row threshold: split-K on
@@ -186,9 +198,10 @@ class Projections:
             return RowPar(x, w)
         if self._pgemm_ok(M, K, w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
-        cfg = self._wcfg(M, w.shape[0], K, 0, is_decode) if slabs else None
+        cfg = self._wcfg(M, w.shape[0], K, 0, is_decode, w) if slabs else None
         if cfg is None:
-            y = self._few(0, x, w, slabs)
+            # a gate and up that come here take the activation kernel as well: no slabs for it
+            y = self._few(0, x, w, slabs and not tag.endswith("gate_up"))
             if y is not None:
                 return y if y.dim() == 2 else Parts(y)
             return ops.linear(x, w)

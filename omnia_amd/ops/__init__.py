@@ -478,10 +478,6 @@ STREAM_MAX_M = 16
 _stream_on = os.environ.get("OMNIA_STREAM", "1") != "0"
 
 
-def streams_on() -> bool:
-    return _stream_on
-
-
 def _on_grid(*ts: torch.Tensor) -> bool:
     """Whether 16-byte loads of these tensors are aligned."""
     return all(t.data_ptr() % 16 == 0 for t in ts)
@@ -496,6 +492,35 @@ def stream_ok(M: int, w: torch.Tensor, gated: bool = False) -> bool:
     return K % 64 == 0 and R % (32 if gated else 16) == 0 and w.is_contiguous() and _on_grid(w)
 
 
+@functools.lru_cache(maxsize=8192)
+def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool) -> bool:
+    """Whether ``M`` rows of a weight [R, K] run on :func:`few_rows`' kernels rather than on the
+    library's (with the activation kernel, if gated).
+
+    In slices of K (``slabs``) a panel fills the chip and wins, but for many slabs' bytes (us with
+    the consumer's reads of them, panel / library: 2048 x 2048 at 64 / 256 rows 6.1 / 11.6, 14 /
+    11.7 and a launch less; 16512 x 4096 at 192 / 256 52 / 55, 64 / 58).  Unsliced, a block walks all of K
+    and takes longer the more rows it has, so few blocks lose: 2048 x 8192 at 32 rows 32 / 16;
+    4096 x 4096 at 64 20 / 15; 3072 x 1024 at 128 / 256 10 / 12, 16 / 12; 4096 x 2048 at 64 / 96
+    11 / 12, 16 / 13; 10304 x 2048 at 96 / 129 17 / 18, 22 / 17; gated of 4096 x 2048 at 64 / 65 /
+    256 13 / 14, 18 / 15, 33 / 16; 14336 x 4096 at 128 / 160 36 / 37, 44 / 41; 16384 x 2048 at 192
+    / 256 28 / 30, 34 / 33; 28672 x 4096 at 256 69 / 74.  Row-major weights of more than 0.7 GB,
+    which the library reads at 6 TB/s, only up to 32 rows: 57344 x 8192 at 32 / 64 / 256 rows
+    158 / 182, 182 / 161, 283 / 233; 128256 x 4096 at 32 / 64 / 128 167 / 169, 205 / 173, 224 /
+    193 (65536 x 4096, 0.54 GB, at 64 105 / 127)."""
+    if not packed and M > 32 and R * K > 3.5e8:
+        return False
+    if packed and M <= STREAM_MAX_M:
+        return True
+    if slabs and not gated and panel_slices(R, K) > 1:
+        return M <= 192 or R < 12288
+    if M <= 64:
+        return gated or K <= 2048 or R >= 12288
+    if M <= 128:
+        return R >= 8192 or (K <= 1024 and not gated)
+    return R >= (16384 if M <= 192 else 24576 if gated else 1 << 31)
+
+
 def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bool = False,
              **kw) -> torch.Tensor:
     """A plain (epi 0) or gated (1) projection of up to 256 rows on the better kernel.
@@ -503,9 +528,7 @@ def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bo
     Up to 16 rows of packed weights stream (us at 8 rows, stream / panel: 2048 x 2048 4.5 / 4.7,
     4096 x 4096 7.7 / 8.8, 16384 x 2048 14.9 / 14.4), unless few long rows leave that kernel's
     blocks few (2048 x 8192 10.7 / 8.7).  Row-major weights reach the streaming kernel in
-    pieces, the panel kernel in whole lines (14.5 / 9.0; 4096 x 4096 9.5 / 8.8).  More rows, panel
-    / library: 64 rows of 2048 x 8192 9.7 / 22.2, 192 of 16384 x 2048 (gated) 27 / 32 and the
-    activation kernel, 256 of 2048 x 8192 19 / 27, of 3072 x 1024 9.8 / 8.7."""
+    pieces, the panel kernel in whole lines (14.5 / 9.0; 4096 x 4096 9.5 / 8.8)."""
     R, K = w.shape
     if packed and x.shape[0] <= STREAM_MAX_M and not (slabs and R < 192 * 16 and K >= 4096):
         return stream(epi, x, w, packed=True, **kw)

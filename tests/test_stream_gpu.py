@@ -271,6 +271,7 @@ def test_a_layer_with_a_weight_off_the_grid(key):
     out = []
     for off in (False, True):
         m = build_model(resolve("tiny-llama"), device="cuda", seed=3)
+        assert m.prepack_decode(4) > 0
         if off:
             m.w["layers"][1][key] = _off_grid(m.w["layers"][1][key])
         out.append(_step(m, 4))
@@ -471,3 +472,34 @@ def test_gated_projection_on_both_sides_of_the_rule(M):
     assert not m._pgemm_ok(M, K, N, False, _off_grid(w))
     g, u = (x.double() @ w.double().t()).split(N, 1)
     _close(ops.pgemm(1, x, w), F.silu(g) * u, K)
+
+
+@pytest.mark.parametrize("M", [1, 16, 33, 64, 65, 128, 129, 192, 193, 256])
+def test_kernels_of_a_projection_by_its_rows(M):
+    """Whichever kernel the rows, the size and the layout choose, slabs or not, the product is the
+    same; unsliced walks of few blocks and large row-major weights stay with the library."""
+    from omnia_amd.models.projection import Parts, Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device("cuda"), torch.bfloat16, 1, {}
+
+    for R, K in ((64, 4096), (2048, 192), (8192, 64), (12288, 128), (24576, 64)):
+        x, w = _mk(M, R, K, M + R)
+        for packed in (False, True):
+            m = Model()
+            if packed:
+                m.w = {"layers": [{"o": w}]}
+                assert m.pack_streams() > 0
+            for slabs in (False, True):
+                y = m._proj("o", x, w, True, slabs)
+                assert slabs or not isinstance(y, Parts)
+                y = y.t.sum(0) if isinstance(y, Parts) else y
+                _close(y, x.double() @ w.double().T, K)
+            a = m._few(1, x, w)
+            if a is not None:
+                g, u = (x.double() @ w.double().T).chunk(2, 1)
+                _close(a, F.silu(g) * u, 4 * K, 1.1)
+    pay = ops.few_rows_pay
+    assert pay(M, 64, 4096, False, True, False) == (M <= 16)
+    assert pay(M, 57344, 8192, True, False, False) == (M <= 32)
+    assert pay(M, 2048, 8192, False, True, True) and pay(M, 28672, 4096, True, True, False)
