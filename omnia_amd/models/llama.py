@@ -26,7 +26,7 @@ from ..ops import reference as ref
 from ..parallel import overlap
 from ..parallel import state as pstate
 from .config import ModelConfig
-from .projection import Parts, Projections, RowPar
+from .projection import Parts, Projections, RowPar, version
 
 # decode attention: below this many (sequence, kv head) pairs a step splits every
 # live context on the device (``LlamaModel.decode_part``)
@@ -215,18 +215,21 @@ class LlamaModel(Projections):
     # ones ~6.0 TB/s; inside the full kernel, next to the x re-reads and the
     # MFMAs, the gain is 0-3 % per projection (profiles/r5/decode_gemm/); end to
     # end the closed-loop bench gains +0.8 % tok/s and -2 % TPOT, 3 of 3
-    # interleaved pairs (profiles/r6/bench/tgemm_pack/).  The copy (~14 GB for
-    # Llama-3-8B, 5 % of HBM) is built before the KV pool is sized, by default
-    # whenever it fits pack_budget_frac of HBM (70B TP=1 and MoE models: never);
+    # interleaved pairs (profiles/r6/bench/tgemm_pack/).  Only batches past the
+    # few-row kernels (193 to 256 rows) run it.  The copy is built before the KV
+    # pool is sized, by default whenever it and the few-row copies fit
+    # pack_budget_frac of HBM (70B TP=1 and MoE models: never);
     # OMNIA_TGEMM_PACK=0 turns it off.
-    pack_budget_frac = 0.10  # of the device's HBM
+    pack_budget_frac = 0.10  # of the device's HBM, copies for the few-row kernels included
 
     def prepack_decode(self, max_batch: int) -> int:
-        """Pack the decode projections for every batch bucket up to ``max_batch``;
-        returns the bytes packed (0: off / over budget)."""
-        return self.pack_streams() + self._prepack_tiles(max_batch)
+        """Pack the projections for the few-row kernels and, for the batches up to
+        ``max_batch`` that go on to tgemm, for that; returns the bytes packed (0: off /
+        over budget)."""
+        n = self.pack_streams()
+        return n + self._prepack_tiles(max_batch, n)
 
-    def _prepack_tiles(self, max_batch: int) -> int:
+    def _prepack_tiles(self, max_batch: int, packed: int) -> int:
         self._packed = {}
         env = os.environ.get("OMNIA_TGEMM_PACK", "1")
         if env not in ("1", "force") or self.device.type != "cuda" or self.tp != 1 \
@@ -234,22 +237,22 @@ class LlamaModel(Projections):
             return 0
         want = {}
         top = next((b for b in ops.WGEMM_BUCKETS if b >= max_batch), ops.WGEMM_BUCKETS[-1])
-        for b in (b for b in ops.WGEMM_BUCKETS if b <= top):
-            for layer in self.w["layers"]:
-                for key, mode in (("qkv", 0), ("o", 0), ("down", 0), ("gate_up", 1)):
-                    w = layer[key]
-                    N = w.shape[0] // 2 if mode == 1 else w.shape[0]
-                    cfg = ops.wgemm_config(b, N, w.shape[1], mode)
+        for layer in self.w["layers"]:
+            for key, mode in (("qkv", 0), ("o", 0), ("down", 0), ("gate_up", 1)):
+                w = layer[key]
+                N = w.shape[0] // 2 if mode == 1 else w.shape[0]
+                # the entries that some batch runs, which few rows do not
+                for cfg in {self._wcfg(M, N, w.shape[1], mode, True, w) for M in range(1, top + 1)}:
                     if cfg is None or cfg[1] >= 0 or (-1 - cfg[1]) & 2:
                         continue  # not tgemm, or its 32-k stage form
                     pmode = 1 if mode == 1 and cfg[2] == 1 else 0
                     want[(w.data_ptr(), cfg[0], pmode)] = w
         total = sum(w.numel() * w.element_size() for w in want.values())
         cap = torch.cuda.get_device_properties(self.device).total_memory * self.pack_budget_frac
-        if not want or (env != "force" and total > cap):
+        if not want or (env != "force" and packed + total > cap):
             return 0
         for (ptr, bn, pmode), w in want.items():
-            self._packed[(ptr, bn, pmode)] = ops.tgemm_pack(w, bn, pmode)
+            self._packed[(ptr, bn, pmode)] = w, version(w), ops.tgemm_pack(w, bn, pmode)
         return total
 
     # ------------------------------------------------------------ forward

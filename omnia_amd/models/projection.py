@@ -36,7 +36,7 @@ class RowPar:
         self.x, self.w = x, w
 
 
-def _version(t: torch.Tensor) -> int:
+def version(t: torch.Tensor) -> int:
     """Counts in-place writes (inference tensors do not)."""
     return 0 if t.is_inference() else t._version
 
@@ -44,8 +44,8 @@ def _version(t: torch.Tensor) -> int:
 def packed_copy(model, w: torch.Tensor) -> torch.Tensor | None:
     """The model's packed copy of a weight (``Projections.pack_streams``), while the weight is
     what was copied."""
-    t, version, copy = getattr(model, "_streams", {}).get(w.data_ptr(), (None, None, None))
-    return copy if copy is not None and t.shape == w.shape and version == _version(w) else None
+    t, at, copy = getattr(model, "_streams", {}).get(w.data_ptr(), (None, 0, None))
+    return copy if copy is not None and t.shape == w.shape and at == version(w) else None
 
 
 def packed_experts(model, up: torch.Tensor, down: torch.Tensor):
@@ -101,7 +101,7 @@ class Projections:
         cap = torch.cuda.get_device_properties(self.device).total_memory * self.stream_budget_frac
         if total > cap:
             return 0
-        self._streams = {p: (t, _version(t), ops.stream_pack(t)) for p, t in found.items()}
+        self._streams = {p: (t, version(t), ops.stream_pack(t)) for p, t in found.items()}
         return total
 
     def _stream_weight(self, M: int, w: torch.Tensor, gated: bool = False):
@@ -173,8 +173,8 @@ class Projections:
             mode = 3
         packed = getattr(self, "_packed", None)
         if packed and nwaves < 0:
-            wp = packed.get((w.data_ptr(), nw, 1 if mode == 1 else 0))
-            if wp is not None:
+            src, at, wp = packed.get((w.data_ptr(), nw, 1 if mode == 1 else 0), (None, 0, None))
+            if wp is not None and src.shape == w.shape and at == version(w):
                 return ops.tgemm(mode, x, wp, S, nw, (-1 - nwaves) | 8, out)
         if mode == 3:
             return ops.tgemm(3, x, w, S, nw, -1 - nwaves, out)

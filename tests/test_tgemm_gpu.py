@@ -197,6 +197,39 @@ def test_model_decode_on_packed_weights_is_bit_identical():
     assert torch.equal(got_mlp, ref_mlp) and torch.equal(got_qkv, ref_qkv)
 
 
+def test_every_tile_packed_copy_is_one_that_a_batch_reads():
+    """No copy for rows that the few-row kernels take, none past the HBM that both kinds of copies
+    share, and none read once its weight has changed."""
+    from omnia_amd.models import build_model
+    from omnia_amd.models.config import resolve
+
+    mc = resolve("llama-3-8b").replace(name="llama-3-8b-1l", num_layers=1, vocab_size=512)
+    m = build_model(mc, device=torch.device("cuda"), dtype=torch.bfloat16, seed=3)
+    layer = m.w["layers"][0]
+    size = {w.data_ptr(): w.numel() * 2 for w in layer.values()}
+    for top in (16, 64, 128, 192, 256):
+        n = m.prepack_decode(top)
+        read = set()
+        for key, mode in (("qkv", 0), ("o", 0), ("down", 0), ("gate_up", 1)):
+            w = layer[key]
+            N = w.shape[0] // (2 if mode else 1)
+            for M in range(1, top + 1):
+                cfg = m._wcfg(M, N, w.shape[1], mode, True, w)
+                if cfg is not None and cfg[1] < 0 and not (-1 - cfg[1]) & 2:
+                    read.add((w.data_ptr(), cfg[0], int(mode == 1 and cfg[2] == 1)))
+        assert set(m._packed) == read
+        assert n == sum(size[k[0]] for k in read) + sum(size[p] for p in m._streams)
+    assert read and len(m._streams) == 4
+    h = (torch.randn(256, mc.hidden_size, device="cuda") * 0.5).to(torch.bfloat16)
+    layer["qkv"].neg_()
+    got = m._proj("qkv", h, layer["qkv"], True).t.float().sum(0)
+    torch.testing.assert_close(got, h.float() @ layer["qkv"].float().t(), rtol=1e-2, atol=2e-2)
+    # room for the few-row copies and all but a byte of the others
+    total = torch.cuda.get_device_properties(0).total_memory
+    m.pack_budget_frac = (n - 1) / total
+    assert m.prepack_decode(256) == sum(size[p] for p in m._streams) and not m._packed
+
+
 def test_every_tgemm_table_entry_matches_fp32():
     """Every tile-kernel entry of the tuned decode table (the shapes the serving
     engine dispatches to it: Llama-3-8B, Llama-3-70B TP=1 / TP=8 shards) run as
