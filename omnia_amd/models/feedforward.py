@@ -12,7 +12,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import mixers as mops
-from .projection import packed_copy, packed_experts
+from .projection import few_weight, packed_experts
 
 
 def _up8(n: int) -> int:
@@ -53,11 +53,9 @@ class DenseGLU:
         N = W.shape[0]
         if m._pgemm_ok(M, K, N // 2, is_decode, W) and (b is None or act == "silu"):
             return ops.pgemm(1, h, W, bias=b, gelu=act == "gelu_tanh")
-        if ops.stream_ok(M, W, gated=True):
-            copy = packed_copy(m, W)
-            if ops.few_rows_pay(M, N, K, True, copy is not None, False):
-                return ops.few_rows(1, h, W if copy is None else copy, copy is not None, bias=b,
-                                    gelu=act == "gelu_tanh")
+        t = few_weight(m, M, W, True, False)
+        if t is not None:
+            return ops.few_rows(1, h, *t, bias=b, gelu=act == "gelu_tanh")
         cfg = m._wcfg(M, N // 2, K, 1, is_decode)
         if cfg is not None:  # a tuned SwiGLU shape, as slabs (bias and activation follow)
             nw, nwaves, S = cfg

@@ -278,7 +278,7 @@ class LlamaModel(Projections):
             return self._proj("down", ops.pgemm(1, h, layer["gate_up"]), layer["down"], False)
         cfg = self._wcfg(M, I2 // 2, K, 1, is_decode, layer["gate_up"])
         if cfg is None:
-            a = self._few(1, h, layer["gate_up"])
+            a = None if M > ops.PANEL_MAX_M else self._few(1, h, layer["gate_up"])
             if a is None:
                 a = ops.linear_silu(h, layer["gate_up"])  # SwiGLU fused into decode GEMMs
         elif cfg[1] == ops.PGEMM_SPLIT and cfg[2] == 1:

@@ -36,16 +36,37 @@ class RowPar:
         self.x, self.w = x, w
 
 
-def version(t: torch.Tensor) -> int:
-    """Counts in-place writes (inference tensors do not)."""
-    return 0 if t.is_inference() else t._version
+def version(t: torch.Tensor) -> int | None:
+    """Counts in-place writes (None: inference tensors do not)."""
+    return None if t.is_inference() else t._version
 
 
 def packed_copy(model, w: torch.Tensor) -> torch.Tensor | None:
     """The model's packed copy of a weight (``Projections.pack_streams``), while the weight is
     what was copied."""
-    t, at, copy = getattr(model, "_streams", {}).get(w.data_ptr(), (None, 0, None))
-    return copy if copy is not None and t.shape == w.shape and at == version(w) else None
+    streams = getattr(model, "_streams", None)
+    hit = streams.get(w.data_ptr()) if streams else None
+    if hit is None:
+        return None
+    t, at, copy = hit  # eager steps wait for this, so what is known is not asked for again
+    same = t is w or (t.shape == w.shape and t.dtype == w.dtype and w.is_contiguous())
+    return copy if same and (at is None or at == w._version) else None
+
+
+def few_weight(model, M: int, w: torch.Tensor, gated: bool, slabs: bool):
+    """(weight, packed) to run ``M`` rows of a projection on the few-row kernels where they beat
+    the other paths, else None."""
+    if not 1 <= M <= ops.PANEL_MAX_M or not ops.streams_on():
+        return None
+    copy = packed_copy(model, w)  # the kernels cover what has one
+    if copy is not None and M <= ops.STREAM_MAX_M:
+        return copy, True
+    if copy is None and not ops.stream_ok(M, w, gated):
+        return None
+    R, K = w.shape
+    if not ops.few_rows_pay(M, R, K, gated, copy is not None, slabs):
+        return None
+    return (w, False) if copy is None else (copy, True)
 
 
 def packed_experts(model, up: torch.Tensor, down: torch.Tensor):
@@ -105,9 +126,9 @@ class Projections:
         return total
 
     def _stream_weight(self, M: int, w: torch.Tensor, gated: bool = False):
-        """(weight, packed) to run ``M`` rows of a projection on the streaming or the panel
-        kernel, or None for the other paths."""
-        if self.device.type != "cuda" or self.tp != 1 or not ops.stream_ok(M, w, gated):
+        """(weight, packed) for a layer of the streaming kernel, or None where it does not cover
+        the weight."""
+        if self.tp != 1 or not ops.stream_ok(M, w, gated):
             return None
         t = packed_copy(self, w)
         return (w, False) if t is None else (t, True)
@@ -115,15 +136,10 @@ class Projections:
     def _few(self, epi: int, x: torch.Tensor, w: torch.Tensor, slabs: bool = False, **kw):
         """A plain (epi 0) or gated (1) projection of up to 256 rows: its rows or, with ``slabs``,
         perhaps its slabs; None for more rows and what the kernels do not cover."""
-        s = self._few_weight(x.shape[0], w, epi == 1, slabs)
-        return None if s is None else ops.few_rows(epi, x, *s, slabs=slabs, **kw)
-
-    def _few_weight(self, M: int, w: torch.Tensor, gated: bool, slabs: bool):
-        """:meth:`_stream_weight` where those kernels beat the other paths."""
-        if M > ops.PANEL_MAX_M:
+        if self.tp != 1:
             return None
-        s = self._stream_weight(M, w, gated)
-        return s if s and ops.few_rows_pay(M, *w.shape, gated, s[1], slabs) else None
+        t = few_weight(self, x.shape[0], w, epi == 1, slabs)
+        return None if t is None else ops.few_rows(epi, x, *t, slabs=slabs, **kw)
 
     # Projections return either a bf16 tensor (library / gemm.hip path, not yet
     # TP-reduced) or :class:`Parts` (fp32 split-K slabs of the weight-streaming
@@ -136,19 +152,20 @@ class Projections:
         library."""
         if self.device.type != "cuda" or self.dtype != torch.bfloat16:
             return None
+        if not is_decode:
+            # mid-size steps below the prefill tile's row threshold: split-K on
+            # the 256x256 tile where the table lists a win (ops.midm_config)
+            if self.tp == 1 and self.use_pgemm and M < self._min_rows:
+                return ops.midm_config(M, N, K, mode)
+            return None  # up to 256 rows among them
         # up to 192 rows the few-row kernels come before the tables.  With the consumer's reads of
         # the slabs, us at 64 / 128 / 192 rows, packed panel (fp32 slabs) and table (fp16 from 65
         # rows on): 6144 x 4096 18 / 22 / 26 and 19 / 20 / 24; 4096 x 4096 14 / 19 / 25 and 18 /
         # 17 / 19; 4096 x 14336 28 / 36 / 41 and 33 / 37 / 38; gated 28672 x 4096 44 / 53 / 56 and
         # (library at 64, 128) 56 / 62 / 62.  Beyond, the tables by more: 256 rows 28 and 25, 28
         # and 21, 49 and 45, 69 and 66
-        if M <= 192 and w is not None and self._few_weight(M, w, mode == 1, slabs):
-            return None
-        if not is_decode:
-            # mid-size steps below the prefill tile's row threshold: split-K on
-            # the 256x256 tile where the table lists a win (ops.midm_config)
-            if self.tp == 1 and self.use_pgemm and M < self._min_rows:
-                return ops.midm_config(M, N, K, mode)
+        if M <= 192 and w is not None and self.tp == 1 and \
+                few_weight(self, M, w, mode == 1, slabs):
             return None
         return ops.wgemm_config(M, N, K, mode)
 
@@ -174,7 +191,7 @@ class Projections:
         packed = getattr(self, "_packed", None)
         if packed and nwaves < 0:
             src, at, wp = packed.get((w.data_ptr(), nw, 1 if mode == 1 else 0), (None, 0, None))
-            if wp is not None and src.shape == w.shape and at == version(w):
+            if wp is not None and src.shape == w.shape and at in (None, w._version):
                 return ops.tgemm(mode, x, wp, S, nw, (-1 - nwaves) | 8, out)
         if mode == 3:
             return ops.tgemm(3, x, w, S, nw, -1 - nwaves, out)
@@ -201,7 +218,8 @@ class Projections:
         cfg = self._wcfg(M, w.shape[0], K, 0, is_decode, w) if slabs else None
         if cfg is None:
             # a gate and up that come here take the activation kernel as well: no slabs for it
-            y = self._few(0, x, w, slabs and not tag.endswith("gate_up"))
+            y = None if M > ops.PANEL_MAX_M else \
+                self._few(0, x, w, slabs and not tag.endswith("gate_up"))
             if y is not None:
                 return y if y.dim() == 2 else Parts(y)
             return ops.linear(x, w)
@@ -222,9 +240,8 @@ class Projections:
         # a 256x256 tile's 132 KB of LDS cannot share a CU with the peers'
         # spinning all-reduce blocks, so a rank's GEMM can wait out their spin
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
-        tn = 256 if gated is None else 128
-        rows = M >= self._min_rows or (tn == 128 and ops.gated_tile_fills(M, gated))
-        return (self.use_pgemm and not is_decode and self.device.type == "cuda"
-                and self.dtype == torch.bfloat16
-                and rows and K % 128 == 0 and N % tn == 0
+        return (self.use_pgemm and not is_decode and K % 128 == 0
+                and N % (256 if gated is None else 128) == 0
+                and (M >= self._min_rows or (gated is not None and ops.gated_tile_fills(M, gated)))
+                and self.device.type == "cuda" and self.dtype == torch.bfloat16
                 and (self.tp == 1 or pstate.ranks_per_device() == 1))

@@ -447,9 +447,11 @@ def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
     activation kernel; 8192 features of 2048: 512 rows .50 48 / 42, 768 .75 51.5 / 52.7, 999 .98
     55 / 67, 1536 .75 99 / 99, 2001 .98 108 / 124; 14336 of 4096: 320 .55 93 / 88, 512 .88 99 / 112,
     768 .66 177 / 163, 999 .85 187 / 198)."""
+    if M <= PANEL_MAX_M:
+        return False
     N = w.shape[0] // 2
     rounds = -(-(-(-M // 256) * (N // 128)) // 256)
-    return M > PANEL_MAX_M and M * N > 0.75 * 256 * 256 * 128 * rounds and \
+    return M * N > 0.75 * 256 * 256 * 128 * rounds and \
         w.is_contiguous() and _on_grid(w)
 
 
@@ -478,6 +480,10 @@ STREAM_MAX_M = 16
 _stream_on = os.environ.get("OMNIA_STREAM", "1") != "0"
 
 
+def streams_on() -> bool:
+    return _stream_on
+
+
 def _on_grid(*ts: torch.Tensor) -> bool:
     """Whether 16-byte loads of these tensors are aligned."""
     return all(t.data_ptr() % 16 == 0 for t in ts)
@@ -495,30 +501,36 @@ def stream_ok(M: int, w: torch.Tensor, gated: bool = False) -> bool:
 @functools.lru_cache(maxsize=8192)
 def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool) -> bool:
     """Whether ``M`` rows of a weight [R, K] run on :func:`few_rows`' kernels rather than on the
-    library's (with the activation kernel, if gated).
+    library's (with the activation kernel, if gated); up to 16 rows of packed ones always do.
 
-    In slices of K (``slabs``) a panel fills the chip and wins, but for many slabs' bytes (us with
-    the consumer's reads of them, panel / library: 2048 x 2048 at 64 / 256 rows 6.1 / 11.6, 14 /
-    11.7 and a launch less; 16512 x 4096 at 192 / 256 52 / 55, 64 / 58).  Unsliced, a block walks all of K
-    and takes longer the more rows it has, so few blocks lose: 2048 x 8192 at 32 rows 32 / 16;
-    4096 x 4096 at 64 20 / 15; 3072 x 1024 at 128 / 256 10 / 12, 16 / 12; 4096 x 2048 at 64 / 96
-    11 / 12, 16 / 13; 10304 x 2048 at 96 / 129 17 / 18, 22 / 17; gated of 4096 x 2048 at 64 / 65 /
-    256 13 / 14, 18 / 15, 33 / 16; 14336 x 4096 at 128 / 160 36 / 37, 44 / 41; 16384 x 2048 at 192
-    / 256 28 / 30, 34 / 33; 28672 x 4096 at 256 69 / 74.  Row-major weights of more than 0.7 GB,
-    which the library reads at 6 TB/s, only up to 32 rows: 57344 x 8192 at 32 / 64 / 256 rows
-    158 / 182, 182 / 161, 283 / 233; 128256 x 4096 at 32 / 64 / 128 167 / 169, 205 / 173, 224 /
-    193 (65536 x 4096, 0.54 GB, at 64 105 / 127)."""
+    In slices of K (``slabs``) a panel fills the chip and wins, but for the slabs' bytes at many
+    rows (us with the consumer's reads of them, panel / library: 2048 x 2048 at 64 / 192 / 256
+    rows 6.1 / 11.6, 12.2 / 12.0, 14 / 11.7; 4096 x 2048 at 193 / 256 15 / 13, 17 / 14; 2048 x
+    8192 at 256 23 / 27; 8256 x 2048 23 / 27; 16512 x 4096 at 192 / 256 52 / 55, 64 / 58).
+    Unsliced, a block walks all of K and takes longer the more rows it has, so few blocks lose:
+    2048 x 8192 at 32 rows 32 / 16; 4096 x 4096 at 64 20 / 15; 3072 x 1024 at 128 / 256 10 / 12,
+    16 / 12; 4096 x 2048 at 64 / 96 11 / 12, 16 / 13; 10304 x 2048 at 96 / 129 17 / 18, 22 / 17;
+    12352 x 2048 at 129 22 / 26; gated of 4096 x 2048 at 64 / 65 / 256 13 / 14, 18 / 15, 33 / 16;
+    14336 x 4096 at 128 / 160 36 / 37, 44 / 41; 16384 x 2048 at 192 / 256 28 / 30, 34 / 33; 28672
+    x 4096 at 256 69 / 74. Row-major weights of more than 0.7 GB, which the library reads at 6
+    TB/s, only up to 32 rows: 57344 x 8192 at 32 / 64 / 256 rows 158 / 182, 182 / 161, 283 / 233;
+    128256 x 4096 at 32 / 64 / 128 167 / 169, 205 / 173, 224 / 193 (65536 x 4096, 0.54 GB, at 64
+    105 / 127). Layers 1024 wide stay here by a little more: their eager steps wait for the host,
+    which these launches cost less (gated 8192 x 1024 at 160 / 256 17.0 / 16.3, 22 / 19, but a
+    step of 16 such layers of 200 rows 1.23 ms / 1.74)."""
     if not packed and M > 32 and R * K > 3.5e8:
         return False
-    if packed and M <= STREAM_MAX_M:
-        return True
     if slabs and not gated and panel_slices(R, K) > 1:
-        return M <= 192 or R < 12288
+        return M <= 192 or (R < 12288 and R * K > 1.4e7) or min(R, K) <= 1024
     if M <= 64:
         return gated or K <= 2048 or R >= 12288
+    if gated and K <= 1024:
+        return R >= 8192
     if M <= 128:
-        return R >= 8192 or (K <= 1024 and not gated)
-    return R >= (16384 if M <= 192 else 24576 if gated else 1 << 31)
+        return R >= 8192 or K <= 1024
+    if M <= 192:
+        return R >= (12288 if K <= 2048 else 16384)
+    return gated and R >= 24576
 
 
 def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bool = False,
@@ -992,15 +1004,20 @@ def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor
     kernel 52 / 90 / 82 / 93 / 93 / 93, packed 25 / 63 / 58 / 72 / 74 / 95; 4096 x 14336: 193 /
     383 / 470 / 472 / 475 / 477 and 111 / 315 / 418 / 419 / 431 / 602.  Row-major weights gain
     only where most experts have no row: 29 for 52 and 133 for 193 at 1 token."""
-    return n <= (8 * experts if packed else (experts - 1) // 2) and _moe_few_ok(w_up, w_down)
+    return n <= (8 * experts if packed else (experts - 1) // 2) and \
+        _moe_few_ok(packed, w_up, w_down)
 
 
-def _moe_few_ok(*ws: torch.Tensor) -> bool:
+def _moe_few_ok(packed: bool, *ws: torch.Tensor) -> bool:
     """Whether the streaming and panel kernels cover these expert weights: the shapes that
-    moe.hip takes, on the 16-byte grid."""
-    return (_stream_on and _on_grid(*ws) and all(
-        w.is_cuda and w.dtype == torch.bfloat16 and w.shape[1] % 64 == 0 and w.shape[2] % 64 == 0
-        for w in ws))
+    moe.hip takes, on the 16-byte grid (``packed``: the copies are)."""
+    if not _stream_on:
+        return False
+    for w in ws:
+        if w.shape[1] % 64 or w.shape[2] % 64 or \
+                not (packed or (w.is_cuda and w.dtype == torch.bfloat16 and _on_grid(w))):
+            return False
+    return True
 
 
 def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
@@ -1016,7 +1033,7 @@ def moe_panel_rows(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tenso
     89 / 90 / 93 / 96).  Fewer rows gain from whole-line reads of packed weights where K is long (8
     to 56 rows, 64-row kernel / 64-row segments: the first 94 / 82 to 99 / 92, the second 495 / 446
     to 567 / 527, the third 75 / 70 to 78 / 80; 32 of 2048 x 1024 90 / 97)."""
-    if not _moe_few_ok(w_up, w_down):
+    if not _moe_few_ok(packed, w_up, w_down):
         return 0
     if n >= 64 * experts:
         return 128
@@ -1066,7 +1083,10 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
                           alpha, limit, ids if own else None)
 
     elif panel:
-        segs = experts * -(-5 * n // (4 * n_experts * panel))  # live ones, about
+        # live ones, about: an expert may well have a third more rows than the mean (ungated of
+        # 2048 x 6144 at 102 rows, down product with 4 / 8 waves, routed evenly 59 / 71 us, to
+        # half of the experts more often 91 / 71)
+        segs = experts * -(-4 * n // (3 * n_experts * panel))
 
         def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
             wn = panel_plan(panel, w.shape[1] * segs, w.shape[2], False)[0]

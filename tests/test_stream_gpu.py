@@ -219,7 +219,7 @@ def test_segments_by_rows_an_expert():
         assert segs == sorted(segs) and set(segs) <= {0, 64, 128} and segs[-1] == 128
         assert packed or 64 not in segs
     assert ops.moe_panel_rows(100, 8, up[..., :1024], down[:, :1024], True) == 0
-    assert ops.moe_panel_rows(1000, 8, up.float(), down, True) == 0
+    assert ops.moe_panel_rows(1000, 8, up.float(), down, False) == 0
     # a tile covers what 128-row segments begin with, and few tiles wait for fuller ones
     assert ops.moe_panel_rows(8 * ops.moe_tile_rows(8, 4096) - 1, 8, up, down, False) == 128
     assert ops.moe_tile_rows(8, 2048) > ops.moe_tile_rows(8, 4096) == ops.moe_tile_rows(64, 512)
@@ -348,7 +348,7 @@ def test_expert_rows_and_weights_off_the_grid(T):
     want = ops.moe(x, router, up, down, k, E)
     assert torch.equal(ops.moe(_off_grid(x), router, up, down, k, E), want)
     for ws in ((_off_grid(up), down), (up, _off_grid(down))):
-        assert not ops.moe_stream_ok(1, E, *ws, True) and not ops.moe_panel_rows(999, E, *ws, True)
+        assert not ops.moe_stream_ok(1, E, *ws, False) and not ops.moe_panel_rows(999, E, *ws, False)
         got = ops.moe(x, router, *ws, k, E).double()
         assert (got - want).norm() <= 2 * U * want.double().norm()
     part = up[:, :224].contiguous(), F.pad(down[:, :, :112], (0, 16))
@@ -500,6 +500,6 @@ def test_kernels_of_a_projection_by_its_rows(M):
                 g, u = (x.double() @ w.double().T).chunk(2, 1)
                 _close(a, F.silu(g) * u, 4 * K, 1.1)
     pay = ops.few_rows_pay
-    assert pay(M, 64, 4096, False, True, False) == (M <= 16)
+    assert not pay(M, 64, 4096, False, True, False)
     assert pay(M, 57344, 8192, True, False, False) == (M <= 32)
     assert pay(M, 2048, 8192, False, True, True) and pay(M, 28672, 4096, True, True, False)
