@@ -87,7 +87,11 @@ class Projections:
     # mixed steps take the fused layer only from this many rows: at the open-loop
     # trickle (~256 decode rows + a few hundred prompt tokens) pgemm's 256x256
     # tiles leave most CUs idle, and the split decode / library path is 1.5x
-    # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms)
+    # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms).
+    # Neither threshold holds gated projections off the tile where it fills the
+    # chip (ops.gated_tile_fills): in mixed steps too that is the faster one (8 layers
+    # of 4096 x 14336, 256 decode rows and 190 / 256 prompt rows 3.29 / 3.38 ms with
+    # it, 3.37 / 3.45 without; 16 of 2048 x 8192, 256 and 650 5.85 and 6.08)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
 
     # ---- a few rows (ops.stream, ops.panel)
