@@ -353,12 +353,16 @@ class LlamaModel(Projections):
 
         With >= DECODE_SPLIT_PAIRS (sequence, kv head) pairs the pairs alone give every
         CU a block: one partition up to 2048 keys, else partitions of 1024 (fewer starts
-        and partials, but ragged ends; us at 512 / 1024 / 2048 keys, 8 KV heads: 32
-        sequences of 1000 34 / 34 / 30, 128 of 1000 117 / 108 / 103, 64 of 2000 116 / 112
-        / 109, 40 of 3500 121 / 117 / 123).  With fewer pairs (small batches, one KV head
-        per TP rank) every live context is cut on the device into up to ``splits`` equal
-        partitions (``ops.decode_attention``), so short contexts still spread over the
-        CUs; the captured graph needs no host-known length."""
+        and partials, but ragged ends).  us at 512 / 1024 / 2048 keys, 8 KV heads: 32
+        sequences of 1000 31 / 27 / 27, 128 of 1000 106 / 95 / 95, 64 of 2000 104 / 98 / 91,
+        40 of 3500 113 / 107 / 116; ragged from 100 to 2000 keys 32 sequences 39 / 38 / 33,
+        64 63 / 60 / 62, 128 119 / 117 / 114; 8 of 2000 among 248 of 500 242 / 227 / 214.
+        One of 2000 among 63 of 500 is bounded by its own walk: 48 / 52 / 58.
+
+        With fewer pairs (small batches, one KV head per TP rank) every live context is cut
+        on the device into up to ``splits`` equal partitions (``ops.decode_attention``), so
+        short contexts still spread over the CUs; the captured graph needs no host-known
+        length."""
         pairs = batch * self.hkv
         if 0 < pairs < DECODE_SPLIT_PAIRS:
             splits = -(-DECODE_SPLIT_PAIRS // pairs)
