@@ -102,16 +102,12 @@ def _tables(lens, bs, nb_total):
     return bt.to(DEV)
 
 
-@pytest.mark.parametrize("uv", ["4", "8", "g8"])
-@pytest.mark.parametrize("nw", ["2", "4"])
-@pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 8), (8, 8)])
-@pytest.mark.parametrize("bs", [16, 32])
-def test_decode_attention(hq, hkv, bs, nw, uv, monkeypatch):
-    # both workgroup shapes (2 / 4 waves; the launcher picks by grid size) and
-    # both V prefetch depths
-    monkeypatch.setenv("OMNIA_DECODE_NW", nw)
-    monkeypatch.setenv("OMNIA_DECODE_U", "8" if uv == "g8" else uv)
-    monkeypatch.setenv("OMNIA_DECODE_UG", "8" if uv == "g8" else "4")
+@pytest.mark.parametrize("part", [512, 1024, 2048])
+@pytest.mark.parametrize("hq,hkv", [(32, 8), (64, 8), (8, 8), (16, 8)])
+@pytest.mark.parametrize("bs", [16, 32, 64])
+def test_decode_attention(hq, hkv, bs, part):
+    """Groups of 1, 2, 4 and 8 query heads a KV head, every page size, the partition lengths that
+    the models choose; contexts of one and of several partitions."""
     torch.manual_seed(3)
     lens = [1, 17, 64, 513, 1500, 3000]
     B = len(lens)
@@ -121,7 +117,7 @@ def test_decode_attention(hq, hkv, bs, nw, uv, monkeypatch):
     sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
     q = torch.randn(B, hq, 128, device=DEV, dtype=torch.bfloat16)
     scale = 1 / math.sqrt(128)
-    out = ops.decode_attention(q, kc, vc, bt, sl, scale, part_size=512)
+    out = ops.decode_attention(q, kc, vc, bt, sl, scale, part_size=part)
     qsl = torch.arange(B + 1, dtype=torch.int32)
     exp = ref.paged_attention(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), qsl, sl.cpu(), scale)
     _close(out.cpu(), exp, 0.02, 0.02)

@@ -278,26 +278,51 @@ def test_a_layer_with_a_weight_off_the_grid(key):
     assert torch.equal(*out)
 
 
-def _step(m, rows, past=40):
-    """Logits of a decode step of ``rows`` sequences."""
+def _step(m, rows, past=40, decode=True, replays=0):
+    """Logits of a decode step of ``rows`` sequences, or of a prompt of as many tokens; with
+    ``replays`` those of every replay of its captured graph."""
     from omnia_amd.models import allocate_cache
     from omnia_amd.models.llama import ForwardBatch
 
+    def full(n, b=rows):
+        return torch.full((b,), n, dtype=torch.int32, device="cuda")
+
     bs, per, g = 32, -(-(past + 1) // 32), torch.Generator(device="cuda").manual_seed(rows)
-    kv = allocate_cache(m, rows * per + 1, bs, "cuda", torch.bfloat16, rows + 1)
+    kv = allocate_cache(m, rows * per + 4, bs, "cuda", torch.bfloat16, rows + 1)
     for t in kv.page_tensors():
         t.normal_(generator=g)
-    bt = (torch.arange(rows * per, device="cuda", dtype=torch.int32) + 1).view(rows, per)
-
-    def full(n):
-        return torch.full((rows,), n, dtype=torch.int32, device="cuda")
-
     ids = torch.randint(0, m.cfg.vocab_size, (rows,), generator=g, device="cuda").int()
-    fb = ForwardBatch(ids, full(past), bt[:, past // bs].long() * bs + past % bs, bt,
-                      full(past + 1), torch.arange(rows, device="cuda"), num_seqs=rows)
+    every = torch.arange(rows, device="cuda")
+    if decode:
+        bt = (torch.arange(rows * per, device="cuda", dtype=torch.int32) + 1).view(rows, per)
+        fb = ForwardBatch(ids, full(past), bt[:, past // bs].long() * bs + past % bs, bt,
+                          full(past + 1), every, num_seqs=rows)
+    else:
+        bt = torch.arange(1, 1 + -(-(past + rows) // bs), device="cuda", dtype=torch.int32)[None]
+        at = past + every
+        tiles = [torch.tensor(t, dtype=torch.int32, device="cuda")
+                 for t in ops.prefill_tiles([rows])]
+        fb = ForwardBatch(ids, at.int(), bt[0, at // bs].long() * bs + at % bs, bt,
+                          full(past + rows, 1), every, is_decode=False, num_seqs=1,
+                          q_start_loc=torch.tensor([0, rows], dtype=torch.int32, device="cuda"),
+                          tile_seq=tiles[0], tile_q0=tiles[1])
     if getattr(m, "stateful", False):
         fb.state_slots = torch.arange(1, rows + 1, dtype=torch.int32, device="cuda")
-    return m.forward(fb, kv).float()
+    if not replays:
+        return m.forward(fb, kv).float()
+    side, out = torch.cuda.Stream(), []
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        m.forward(fb, kv)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        logits = m.forward(fb, kv)
+    for _ in range(replays):
+        graph.replay()
+        out.append(logits.float())
+        torch.cuda.synchronize()
+    return out
 
 
 @pytest.mark.parametrize("write", [True, False])
@@ -419,28 +444,33 @@ def test_panel_rows_do_not_depend_on_each_other():
             assert torch.equal(ops.panel(0, x[:M], w, slabs=slabs), whole[..., :M, :])
 
 
-@pytest.mark.parametrize("rows,pack", [(1, True), (16, False), (23, True), (32, False)])
-def test_llama_layers_match_the_unfused_path(rows, pack, monkeypatch):
-    """Decode steps of a small model: the four streamed projections a layer, and the panel
-    kernel's, against the library's GEMMs with separate norm, RoPE, SwiGLU and residual kernels."""
-    from omnia_amd.engine.engine import EngineConfig, LLMEngine
-    from omnia_amd.engine.sampling_params import SamplingParams
+@pytest.mark.parametrize("decode", [True, False])
+@pytest.mark.parametrize("pack", [True, False])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 32])
+def test_llama_layers_match_the_unfused_path(rows, pack, decode, monkeypatch):
+    """Decode steps, captured too, and prompt steps of a small model: the four streamed
+    projections a layer (up to 16 rows of packed weights, or of small row-major ones in an eager
+    step) and the panel kernel's, against the library's GEMMs with separate norm, RoPE, SwiGLU
+    and residual kernels."""
+    from omnia_amd.models import build_model, resolve
 
-    def run(on):
-        monkeypatch.setattr(ops, "_stream_on", on)
-        eng = LLMEngine(EngineConfig(model="tiny-llama", max_batch=32, max_model_len=256, seed=4))
-        if not pack:
-            eng.model._streams = {}
-        eng.runner.enable_logit_tap()
-        p = SamplingParams(temperature=0.0, max_tokens=4, ignore_eos=True)
-        for i in range(rows):
-            eng.add_request([(7 * i + j) % 250 for j in range(5 + i % 3)], p)
-        eng.run_until_done()
-        return {s: r for ids, t in eng.runner.logit_tap[:1] for s, r in zip(ids, t)}
-
-    a, b = run(True), run(False)
-    for x, y in zip(a.values(), b.values()):
-        assert (x - y).norm() <= 0.02 * y.norm()
+    m = build_model(resolve("tiny-llama"), device="cuda", seed=4)
+    if pack:
+        assert m.prepack_decode(32) > 0
+    used, real = [], m._use_stream
+    monkeypatch.setattr(m, "_use_stream", lambda fb: used.append(real(fb)) or used[-1])
+    got = _step(m, rows, decode=decode)
+    assert used == [rows <= 16 and (pack or not decode)] and got.shape[0] == rows
+    monkeypatch.setattr(ops, "_stream_on", False)
+    want = _step(m, rows, decode=decode)
+    assert not used[-1]
+    # bf16 projections whose sums run in another order, through two layers
+    assert (got - want).norm() <= 0.02 * want.norm()
+    assert ((got - want).norm(dim=1) <= 0.03 * want.norm(dim=1)).all()
+    if decode:
+        monkeypatch.setattr(ops, "_stream_on", True)
+        for replay in _step(m, rows, replays=3):
+            assert torch.equal(replay, got)
 
 
 def test_gated_tiles_are_taken_where_they_fill_the_chip():
