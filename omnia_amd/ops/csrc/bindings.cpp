@@ -770,7 +770,7 @@ void moe_gemm(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tens
            "moe_gemm");
 }
 
-// moe_gemm's modes for segments of 16 rows (stream.hip)
+// moe_gemm's modes for segments of 16 rows (stream.hip), and with panel of 64 and 128 (panel.hip)
 static void few_moe(bool panel, int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
                 at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
                 int64_t topk, int64_t n_assign, int64_t e_lo, int64_t nw, bool packed,

@@ -613,11 +613,13 @@ __global__ __launch_bounds__(256) void blocks_kernel(float* __restrict__ rec,
 // as ND accumulator tiles (key dimensions 16 j + 4 (lane >> 4) + r in register r).  The
 // accumulator layout serves as the B operand of the next product as it stands: k-step r
 // takes dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.
-// Bound by its serial chain: a block is 104 fp32 products of one wave (heads of 128), 1.4 us, and
-// a SIMD has one wave.  Vector instructions add to that, so registers hold 2 waves' worth (with
-// more, hipcc keeps S in the accumulators' file and moves it back and forth), offsets are made
-// once, and what is not a product goes between products.  16 heads of 128 with blocks_kernel,
-// 2048 rows of 8 sequences 371 -> 330 us, 333 of 3 68 -> 61.
+// Bound by its serial chain: a block is 104 fp32 products of one wave (heads of 128), 1.4 of the
+// 3.0 us that it takes in a step, and a SIMD has one wave.  Vector instructions add to that, so
+// registers hold 2 waves' worth (with more, hipcc keeps S in the accumulators' file and moves it
+// back and forth), offsets are made once, and what is not a product goes between products.  16
+// heads of 128 in a model step, whose weights leave no operand in the caches: 2048 rows of 8
+// sequences 430 -> 381 us (blocks_kernel 66 beside it, as before), 333 of 3 65 -> 59.  Alone and
+// repeated, both kernels 371 -> 330 and 68 -> 61.
 template <typename T, int ND>
 __global__ __launch_bounds__(256, ND <= 8 ? 2 : 1) void scan_blocks_kernel(
     float* __restrict__ o, float* __restrict__ state, T* __restrict__ conv_state,

@@ -343,7 +343,8 @@ __global__ __launch_bounds__(256) void moe_route_f32_kernel(const float* __restr
 // One 1024-thread workgroup.  n = T*k assignments.  sorted has max_blocks*BM
 // entries (n = padding sentinel), blk_expert max_blocks entries.
 // bm: the segment alignment = the grouped GEMM's row tile (64 here, 16 for a few rows
-// an expert, stream.hip, 256 for the 256x256 prefill tile of pgemm.hip EPI 5 / 6)
+// an expert, stream.hip, 64 or 128 for some tens, panel.hip, 256 for the 256x256 prefill
+// tile of pgemm.hip EPI 5 / 6)
 __global__ __launch_bounds__(1024) void moe_align_kernel(int* __restrict__ sorted,
                                                          int* __restrict__ blk_expert,
                                                          int* __restrict__ n_blocks,
@@ -387,14 +388,11 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(int* __restrict__ sorte
 // (ds_read_b128 fragment reads are then conflict-free across the 16 rows).
 __device__ __forceinline__ int swz(int row, int ch) { return row * 64 + ((ch ^ (row & 7)) << 3); }
 
-// clamped GLU: g = min(gate, limit), u = clamp(up, +-limit): g sigmoid(alpha g) (u + 1)
-struct Glu {
+struct Glu {  // of the clamped GLU
   float alpha, limit;
 };
 __device__ __forceinline__ float clamped_glu(float g, float u, Glu c) {
-  g = fminf(g, c.limit);
-  u = fminf(fmaxf(u, -c.limit), c.limit);
-  return g * __builtin_amdgcn_rcpf(1.f + __expf(-c.alpha * g)) * (u + 1.f);
+  return omnia::clamped_glu(g, u, c.alpha, c.limit);
 }
 
 template <int MODE>

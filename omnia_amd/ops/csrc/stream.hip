@@ -4,17 +4,18 @@
 // At these sizes a projection reads its weights once and does little else, and a model step
 // is a chain of them: what counts is how fast a short read gets going, and how many launches
 // stand between two of them.
-//   * A block of 8 waves owns 16 or 32 weight rows over the whole of K; the waves take turns
-//     at 64-k chunks, so together they read one contiguous KB of every row at a time, and meet
-//     once, in LDS, at the end.  No slabs, no second kernel, no atomics, a fixed order of sums.
+//   * A block of 8 waves owns 16, 32 or 64 weight rows (NW = 1, 2, 4) over the whole of K; the
+//     waves take turns at 64-k chunks, so together they read one contiguous KB of every row at a
+//     time, and meet once, in LDS, at the end.  No slabs, no second kernel, no atomics, a fixed
+//     order of sums.
 //   * Weights go from HBM to MFMA operand registers; x comes from L2, as it is shared by all
 //     blocks.
 //   * Row-major weights reach a CU in 64-byte pieces of 16 rows; PK weights (a copy laid out
 //     [row / 16][k / 64][k / 32][k / 8][row % 16][8], ops.stream_pack) as one KB a wave
 //     instruction: 28672 x 4096 at one row 40.9 us row-major, 37.9 packed; 4096 x 14336 24.5
 //     and 20.9.  Streaming loads (nt) help packed reads (41.7 -> 37.9) and hurt row-major ones.
-//   * A ring of D chunks a wave is in flight from the first instruction on: 64 KB of weights a
-//     block, two blocks a CU.
+//   * A ring of D chunks a wave is in flight from the first instruction on: 64 or 128 KB of
+//     weights a block (NW = 1, 2) and two blocks a CU, or 192 KB (NW = 4) and one.
 //   * NORM: x is the residual, whose rows are RMS-normed (the norm's weight is folded into W)
 //     and rounded to bf16 as they become operands, as a norm kernel would: no launch, no pass.
 //     The rows' sums of squares come from the kernel that wrote the residual (EPI 2).
