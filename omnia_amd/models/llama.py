@@ -26,7 +26,7 @@ from ..ops import reference as ref
 from ..parallel import overlap
 from ..parallel import state as pstate
 from .config import ModelConfig
-from .projection import Parts, Projections, RowPar, version
+from .projection import Parts, Projections, RowPar, packed_copy, version
 
 # decode attention: below this many (sequence, kv head) pairs a step splits every
 # live context on the device (``LlamaModel.decode_part``)
@@ -235,14 +235,17 @@ class LlamaModel(Projections):
         if env not in ("1", "force") or self.device.type != "cuda" or self.tp != 1 \
                 or self.cfg.is_moe:
             return 0
-        want = {}
+        want, known = {}, {}
         top = next((b for b in ops.WGEMM_BUCKETS if b >= max_batch), ops.WGEMM_BUCKETS[-1])
         for layer in self.w["layers"]:
             for key, mode in (("qkv", 0), ("o", 0), ("down", 0), ("gate_up", 1)):
                 w = layer[key]
-                N = w.shape[0] // 2 if mode == 1 else w.shape[0]
-                # the entries that some batch runs, which few rows do not
-                for cfg in {self._wcfg(M, N, w.shape[1], mode, True, w) for M in range(1, top + 1)}:
+                kind = key, w.shape, packed_copy(self, w) is not None
+                if kind not in known:  # the entries that some batch runs, which few rows do not
+                    N = w.shape[0] // 2 if mode == 1 else w.shape[0]
+                    known[kind] = {self._wcfg(M, N, w.shape[1], mode, True, w)
+                                   for M in range(1, top + 1)}
+                for cfg in known[kind]:
                     if cfg is None or cfg[1] >= 0 or (-1 - cfg[1]) & 2:
                         continue  # not tgemm, or its 32-k stage form
                     pmode = 1 if mode == 1 and cfg[2] == 1 else 0
