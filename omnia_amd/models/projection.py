@@ -41,6 +41,13 @@ def version(t: torch.Tensor) -> int | None:
     return None if t.is_inference() else t._version
 
 
+def unchanged(w: torch.Tensor, t: torch.Tensor, at: int | None) -> bool:
+    """Whether ``w``, at the address of ``t``, is ``t`` as it was at version ``at``."""
+    # eager steps wait for this, so what is known is not asked for again
+    same = t is w or (t.shape == w.shape and t.dtype == w.dtype and w.is_contiguous())
+    return same and (at is None or at == w._version)
+
+
 def packed_copy(model, w: torch.Tensor) -> torch.Tensor | None:
     """The model's packed copy of a weight (``Projections.pack_streams``), while the weight is
     what was copied."""
@@ -48,9 +55,8 @@ def packed_copy(model, w: torch.Tensor) -> torch.Tensor | None:
     hit = streams.get(w.data_ptr()) if streams else None
     if hit is None:
         return None
-    t, at, copy = hit  # eager steps wait for this, so what is known is not asked for again
-    same = t is w or (t.shape == w.shape and t.dtype == w.dtype and w.is_contiguous())
-    return copy if same and (at is None or at == w._version) else None
+    t, at, copy = hit
+    return copy if unchanged(w, t, at) else None
 
 
 def few_weight(model, M: int, w: torch.Tensor, gated: bool, slabs: bool):
@@ -195,7 +201,7 @@ class Projections:
         packed = getattr(self, "_packed", None)
         if packed and nwaves < 0:
             src, at, wp = packed.get((w.data_ptr(), nw, 1 if mode == 1 else 0), (None, 0, None))
-            if wp is not None and src.shape == w.shape and at in (None, w._version):
+            if wp is not None and unchanged(w, src, at):
                 return ops.tgemm(mode, x, wp, S, nw, (-1 - nwaves) | 8, out)
         if mode == 3:
             return ops.tgemm(3, x, w, S, nw, -1 - nwaves, out)
