@@ -231,7 +231,8 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
       v += e * red[wi][g][d];
       l += e * ml[wi][g][1];
     }
-    const float inv = 1.f / l;
+    // a partition whose scores are all -inf weighs nothing among others
+    const float inv = l == 0.f && nparts > 1 ? 0.f : 1.f / l;
     const int h = h0 + g;
     if (nparts == 1) {
       out[((int64_t)b * gridDim.y * G + h) * D + d] = f2bf(v * inv);

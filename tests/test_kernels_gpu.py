@@ -265,10 +265,11 @@ def test_decode_attention_around_whole_key_groups(hq, hkv, bs):
     assert (err <= exp.abs() * 2.0 ** -8 + 2e-4 * vc.abs().max()).all(), err.max()
 
 
+@pytest.mark.parametrize("part", [128, 1024])
 @pytest.mark.parametrize("n", [17, 33, 200, 1023])
-def test_decode_attention_with_infinite_scores_and_values(n):
-    """Keys whose scores are -inf weigh nothing, whichever groups of a wave they fill; an infinite
-    value of the last key reaches its own dimension only, with its sign."""
+def test_decode_attention_with_infinite_scores_and_values(n, part):
+    """Keys whose scores are -inf weigh nothing, whichever groups of a wave or whole partitions
+    they fill; an infinite value of the last key reaches its own dimension only, with its sign."""
     torch.manual_seed(9)
     hq, hkv, bs = 8, 2, 16
     kc, vc = _make_cache(-(-n // bs) + 1, hkv, bs, seed=9)
@@ -279,7 +280,7 @@ def test_decode_attention_with_infinite_scores_and_values(n):
     kc[at[:-1]] = -3e38  # sums of 128 such products overflow fp32
     vc[at[-1], 0, (n - 1) % bs, 5] = math.inf
     vc[at[-1], 1, (n - 1) % bs, 7] = -math.inf
-    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=1024).double()
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=part).double()
     exp = _attention64(q, kc, vc, bt, [1], [n], 128 ** -0.5)
     assert torch.equal(out.isinf(), exp.isinf()) and exp.isinf().sum() == 8
     assert torch.equal(out[exp.isinf()], exp[exp.isinf()])
