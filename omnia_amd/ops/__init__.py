@@ -975,7 +975,8 @@ def cosine_topk(q: torch.Tensor, m: torch.Tensor, k: int, valid: torch.Tensor | 
 
 # ------------------------------------------------------------- MoE (K14)
 MOE_LIBRARY_ROWS = 1024  # mean rows/expert above which eager calls use hipBLASLt per expert
-MOE_TILE256_ROWS = int(os.environ.get("OMNIA_MOE_TILE256_ROWS", "128"))
+_rows = os.environ.get("OMNIA_MOE_TILE256_ROWS")
+MOE_TILE256_ROWS = int(_rows) if _rows else None  # None: by the tiles of the down product
 
 
 def moe_tile_rows(experts: int, d: int) -> int:
@@ -991,7 +992,9 @@ def moe_tile_rows(experts: int, d: int) -> int:
     128 117 / 174, at 200 132 / 178, at 250 177 / 183; ungated of 2048 x 6144 at 140 163 / 252 (the
     64-row kernel 230), at 200 165 / 257, at 260 236 / 258; 3 of 4096 x 7168 at 133 211 / 241, at
     233 225 / 250, at 267 341 / 309."""
-    return max(MOE_TILE256_ROWS, 128 if experts * (d // 256) >= 128 else 224)
+    if MOE_TILE256_ROWS is not None:
+        return MOE_TILE256_ROWS
+    return 128 if experts * (d // 256) >= 128 else 224
 
 
 def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
