@@ -503,10 +503,13 @@ def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool)
     """Whether ``M`` rows of a weight [R, K] run on :func:`few_rows`' kernels rather than on the
     library's (with the activation kernel, if gated); up to 16 rows of packed ones always do.
 
-    In slices of K (``slabs``) a panel fills the chip and wins, but for the slabs' bytes at many
-    rows (us with the consumer's reads of them, panel / library: 2048 x 2048 at 64 / 192 / 256
-    rows 6.1 / 11.6, 12.2 / 12.0, 14 / 11.7; 4096 x 2048 at 193 / 256 15 / 13, 17 / 14; 2048 x
-    8192 at 256 23 / 27; 8256 x 2048 23 / 27; 16512 x 4096 at 192 / 256 52 / 55, 64 / 58).
+    In slices of K (``slabs``) a panel fills the chip, and its sums reach the consumer in fp32,
+    where the library rounds them to bf16: steps of 193 to 256 rows through 16 layers of 2048 are
+    10 % closer to exact sums (error of the logits 0.0108, 0.0119 on the library).  So it is taken
+    even where the slabs' bytes cost a little more at many rows (us with the consumer's reads of
+    them, panel / library: 2048 x 2048 at 64 / 192 / 256 rows 6.1 / 11.6, 12.2 / 12.0, 14 / 11.7;
+    4096 x 2048 at 193 / 256 15 / 13, 17 / 14; 2048 x 8192 at 256 23 / 27; 8256 x 2048 23 / 27;
+    16512 x 4096 at 192 / 256 52 / 55, 64 / 58).
     Unsliced, a block walks all of K and takes longer the more rows it has, so few blocks lose:
     2048 x 8192 at 32 rows 32 / 16; 4096 x 4096 at 64 20 / 15; 3072 x 1024 at 128 / 256 10 / 12,
     16 / 12; 4096 x 2048 at 64 / 96 11 / 12, 16 / 13; 10304 x 2048 at 96 / 129 17 / 18, 22 / 17;
@@ -521,7 +524,7 @@ def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool)
     if not packed and M > 32 and R * K > 3.5e8:
         return False
     if slabs and not gated and panel_slices(R, K) > 1:
-        return M <= 192 or (R < 12288 and R * K > 1.4e7) or min(R, K) <= 1024
+        return True
     if M <= 64:
         return gated or K <= 2048 or R >= 12288
     if gated and K <= 1024:
@@ -530,7 +533,7 @@ def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool)
         return R >= 8192 or K <= 1024
     if M <= 192:
         return R >= (12288 if K <= 2048 else 16384)
-    return gated and R >= 24576
+    return gated and R >= 16384  # for fp32 into the activation, at what the library takes
 
 
 def few_rows(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool, slabs: bool = False,

@@ -532,4 +532,7 @@ def test_kernels_of_a_projection_by_its_rows(M):
     pay = ops.few_rows_pay
     assert not pay(M, 64, 4096, False, True, False)
     assert pay(M, 57344, 8192, True, False, False) == (M <= 32)
-    assert pay(M, 2048, 8192, False, True, True) and pay(M, 28672, 4096, True, True, False)
+    assert pay(M, 28672, 4096, True, True, False)
+    for R, K in ((2048, 2048), (2048, 8192), (4096, 4096)):  # whose slabs hand on fp32 sums
+        assert ops.panel_slices(R, K) > 1
+        assert pay(M, R, K, False, True, True) and pay(M, R, K, False, False, True)
