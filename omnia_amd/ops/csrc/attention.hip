@@ -59,9 +59,10 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
 // 127 -> 119 (5.1 TB/s), 128 x 1000 111 -> 104, 64 x 2000 115 -> 112, 32 x 1000 33.7 -> 29.3,
 // 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  K and V go through the caches: sequences of one
 // prompt prefix share its pages, and of those a block finds what another has read.  Past the
-// caches (non-temporal) only what no sequence shares gains: 256 x 576 105 -> 103, 128 x 1000 94 ->
-// 84, 32 x 1000 27 -> 24, but 512 of 576 keys shared 59 -> 73, 896 of 1000 45 -> 64; choosing for
-// each block costs the registers of a wave.
+// caches (non-temporal) only what no sequence shares gains: 256 x 576 105 -> 103 (in a step of 32
+// layers, whose weights pass through the caches too, 6 to 10 us of each: 8.86 -> 8.55 ms), 128 x
+// 1000 94 -> 84, 32 x 1000 27 -> 24, but 512 of 576 keys shared 59 -> 73, 896 of 1000 45 -> 64;
+// choosing for each block costs the registers of a wave.
 constexpr int NW = 4;
 template <int G, int BS>
 __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
