@@ -247,7 +247,7 @@ class Projections:
         each of this weight), and at least this forward's row threshold, or for a
         gated one tiles that fill the chip."""
         # TP ranks rehearsed on ONE device (ipc transport) keep the library GEMMs:
-        # a 256x256 tile's 132 KB of LDS cannot share a CU with the peers'
+        # a 256x256 tile's 160 KB of LDS cannot share a CU with the peers'
         # spinning all-reduce blocks, so a rank's GEMM can wait out their spin
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
         return (self.use_pgemm and not is_decode and K % 128 == 0

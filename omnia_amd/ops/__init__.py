@@ -45,7 +45,7 @@ def kernels():
 
             build(verbose=True)
             _ext = importlib.import_module("omnia_amd.ops._omnia_kernels")
-        # prefill GEMM main loop: 1 = 4-wave (one wave per SIMD), 0 = 8-wave ping-pong
+        # 0 or 1: named two main loops of the prefill GEMM, of which one is left
         sched = os.environ.get("OMNIA_PGEMM_SCHED")
         if sched is not None and hasattr(_ext, "pgemm_set_schedule"):
             _ext.pgemm_set_schedule(int(sched))
@@ -458,7 +458,7 @@ def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
                  sched: int = 0) -> torch.Tensor:
     """fp16 split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the 256x256 MFMA tile
-    (``csrc/pgemm.hip`` EPI 4; ``sched`` 0 / 1 = 8-wave / 4-wave main loop).  Each
+    (``csrc/pgemm.hip`` EPI 4; ``sched`` 0 or 1, of no effect).  Each
     slab is one K-slice's fp32 sum saturated to fp16; the splitk consumers reduce
     them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip)."""
     M, K = x.shape

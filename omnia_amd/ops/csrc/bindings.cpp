@@ -31,8 +31,6 @@ int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
                     float limit, hipStream_t s);
-int omnia_pgemm_variant(int variant, void* out, const void* X, const void* W, int M, int N,
-                        int K, hipStream_t s);
 int omnia_rmsnorm(void* out, const void* x, void* residual, const void* w, int rows, int d,
                   int64_t x_stride, int64_t out_stride, float eps, hipStream_t s);
 int omnia_rope_kv(void* q, void* k, const void* v, const int* positions, const float* cos_sin,
@@ -1148,18 +1146,8 @@ void panel_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t
            "panel_gemm");
 }
 
-void pgemm_variant(int64_t variant, at::Tensor out, at::Tensor x, at::Tensor W) {
-  CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W); CHECK_BF16(out);
-  TORCH_CHECK(x.is_contiguous() && W.is_contiguous() && out.is_contiguous(), "contiguous");
-  TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1) && out.size(0) == x.size(0) &&
-              out.size(1) == W.size(0), "shapes");
-  CHECK_RC(omnia_pgemm_variant((int)variant, out.data_ptr(), x.data_ptr(), W.data_ptr(),
-                               x.size(0), W.size(0), x.size(1), cur_stream()),
-           "pgemm_variant");
-}
-
 // split-K 256x256 MFMA GEMM (pgemm.hip EPI 4): parts fp16 [S, M, N] whose sum
-// over S is x @ W^T; sched 0 / 1 = 8-wave / 4-wave main loop
+// over S is x @ W^T; sched as pgemm_set_schedule's
 void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t sched) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W);
   TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1), "x [M, K], W [N, K]");
@@ -2187,7 +2175,6 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("tgemm", &tgemm);
   m.def("pgemm", &pgemm);
   m.def("row_sumsq", &row_sumsq);
-  m.def("pgemm_variant", &pgemm_variant);
   m.def("pgemm_splitk", &pgemm_splitk);
   m.def("pgemm_set_schedule", [](int64_t sched) {
     TORCH_CHECK(omnia_pgemm_set_schedule((int)sched) == 0, "pgemm schedule must be 0 or 1");

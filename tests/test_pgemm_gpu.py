@@ -263,3 +263,21 @@ def test_qkv_epilogue_tp_shard_heads(gen, schedule, hq, hkv):
     ref.write_kv(kw, vw, kk, vv, slots)
     assert _close(kc, kw, 2e-2)[0] and _close(vc, vw, 2e-2)[0]
     assert not _close(vc, kw, 2e-2)[0]  # k and v not swapped
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 256, 128), (255, 256, 256), (257, 512, 384),  # a row, a tile less and more than one
+    (1100, 768, 640), (2049, 512, 768),  # groups of 4 m-tiles and a rest; the ring's turns
+    (2100, 16384, 4224),  # more than 128 MB of weights: groups of 8 m-tiles and a rest
+])
+def test_tile_and_ring_edges(gen, M, N, K):
+    """Ragged rows, short and wrapping rings of K-tiles, both block orders: every element once,
+    nothing outside.  fp32 sums of K products rounded to bf16: 2^-8 of a value, and the same
+    again for values small beside their products' sum."""
+    x = _rand(M, K, gen=gen)
+    w = _rand(N, K, std=0.05, gen=gen)
+    whole = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.pgemm(0, x, w, out=whole[:M])
+    want = x.float() @ w.float().t()
+    assert ((whole[:M].float() - want).abs() <= 2 ** -8 * (want.abs() + K ** 0.5 * 0.05)).all()
+    assert (whole[M] == 7.0).all()
