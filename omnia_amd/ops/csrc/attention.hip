@@ -57,30 +57,38 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
 // the registers of 2, and short contexts 50 us where these take 39; 4 spill.  us with scores,
 // softmax and P.V as phases of the block -> now (32 heads on 8; sequences x keys): 256 x 576
 // 127 -> 119 (5.1 TB/s), 128 x 1000 111 -> 104, 64 x 2000 115 -> 112, 32 x 1000 33.7 -> 29.3,
-// 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  K and V go through the caches: sequences of one
-// prompt prefix share its pages, and of those a block finds what another has read.  Past the
-// caches (non-temporal) only what no sequence shares gains: 256 x 576 105 -> 103 (in a step of 32
-// layers, whose weights pass through the caches too, 6 to 10 us of each: 8.86 -> 8.55 ms), 128 x
-// 1000 94 -> 84, 32 x 1000 27 -> 24, but 512 of 576 keys shared 59 -> 73, 896 of 1000 45 -> 64;
-// choosing for each block costs the registers of a wave.
+// 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  Of
+// sequences that share the pages of a prompt prefix a block finds in the caches what another has
+// read; K and V that nobody shares go past them (non-temporal).  us through the caches and by
+// this rule: 256 x 576, ragged, 112 -> 107, 128 x 1000 101 -> 92, 64 x 2000 92 -> 81 (6.5 TB/s); 512
+// of 256 x 576 shared 58.3 -> 59.1 (past the caches 71), 896 of 128 x 1000 46.6 -> 47.5 (60); 256 x
+// 150, below it, 33 (past 35.5); 32 x 1000 29.4 -> 27.4, 960 shared 20.6 -> 21.3; 8 x 1000 in
+// partitions of 256 15.5 -> 14.7, 4 x 1000, of 128 and below it, 11.2 (past, with the look, 12.1).
 constexpr int NW = 4;
-template <int G, int BS>
-__global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
-    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
-    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ seq_lens,
-    int hkv, int64_t q_stride, int part_size, int max_parts, float scale_log2, int split_t,
-    int split_min) {
-  __shared__ __attribute__((aligned(16))) float pb[NW][16][G];  // a group's P, wave-private
-  __shared__ __attribute__((aligned(16))) float al[NW][G];
-  __shared__ __attribute__((aligned(16))) float red[NW][G][D];
-  __shared__ float ml[NW][G][2];
+template <int G>
+struct DecodeShared {
+  float pb[NW][16][G];  // a group's P, wave-private
+  float al[NW][G];
+  float red[NW][G][D];
+  float ml[NW][G][2];
+};
+
+// The whole work of a block, K and V past the caches or through them: two copies in the kernel,
+// with the registers of one (140; a choice at each load breaks the pipeline of loads, one around
+// the loop alone spills).
+template <int G, int BS, bool NT>
+__device__ __forceinline__ void decode_block(
+    DecodeShared<G>& sh, int len, int pl, bf16_t* __restrict__ out,
+    float* __restrict__ part_o, float* __restrict__ part_ml, const bf16_t* __restrict__ q,
+    const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+    const int* __restrict__ block_tables, int bt_stride, int hkv, int64_t q_stride, int max_parts,
+    float scale_log2) {
+  auto &pb = sh.pb;
+  auto &al = sh.al;
+  auto &red = sh.red;
+  auto &ml = sh.ml;
   const int b = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
-  const int len = seq_lens[b];
-  if (len <= 0) return;
-  const int pl = decode_part_len(len, part_size, split_t, split_min, BS);
   const int p0 = part * pl;
-  if (p0 >= len) return;
   const int n = min(pl, len - p0);
   const int nparts = (len + pl - 1) / pl;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -106,18 +114,21 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
   };
   const int ngr = (n + 15) / 16, last = n - 1;
   auto page = [&](int c) { return bt[min(c * 16, last) / BS]; };  // past the end: the last page
+  auto get = [](const bf16_t* p) {
+    const short8* s = reinterpret_cast<const short8*>(p);
+    return NT ? __builtin_nontemporal_load(s) : *s;
+  };
   auto load = [&](Group& t, int c, int pg) {
     const int k0 = min(c * 16, last & ~15), top = last - k0;
     const int64_t base = (((int64_t)pg * hkv + kvh) * BS + k0 % BS) * D;
     const bf16_t *kb = kc + base, *vb = vc + base;
     const uint32_t ko = min(c16, top) * D + 8 * g4;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-      t.k[kk] = *reinterpret_cast<const short8*>(kb + ko + kk * 32);
+    for (int kk = 0; kk < 4; ++kk) t.k[kk] = get(kb + ko + kk * 32);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t vo = min(4 * i + g4, top) * D + 8 * c16;
-      t.v[i] = *reinterpret_cast<const short8*>(vb + vo);
+      t.v[i] = get(vb + vo);
     }
   };
   // of head c16; a finite start, so that keys whose scores are all -inf get exponents of -inf
@@ -246,6 +257,39 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
       }
     }
   }
+}
+
+template <int G, int BS>
+__global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
+    bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ seq_lens,
+    int hkv, int64_t q_stride, int part_size, int max_parts, float scale_log2, int split_t,
+    int split_min) {
+  __shared__ __attribute__((aligned(16))) DecodeShared<G> sh;
+  const int b = blockIdx.x, part = blockIdx.z;
+  const int len = seq_lens[b];
+  if (len <= 0) return;
+  const int pl = decode_part_len(len, part_size, split_t, split_min, BS);
+  const int p0 = part * pl;
+  if (p0 >= len) return;
+  // past the caches: of a long sequence what none of the next 16 sequences has the page of, 64
+  // keys into the partition (a row's entries past its length may be anything: at worst the caches
+  // are used).  What shares less is read again for less than is gained
+  constexpr int LONG = 512;
+  if (len >= LONG && min(pl, len - p0) >= 192 && gridDim.x > 1) {
+    const int B = gridDim.x, d = min(1 + (int)(threadIdx.x & 15), B - 1);
+    const int* t = block_tables + min(p0 + 64, len - 1) / BS;
+    const bool same = t[(int64_t)(b + d < B ? b + d : b + d - B) * bt_stride] ==
+                      t[(int64_t)b * bt_stride];
+    if (__builtin_amdgcn_ballot_w64(same) == 0) {
+      decode_block<G, BS, true>(sh, len, pl, out, part_o, part_ml, q, kc, vc, block_tables,
+                                bt_stride, hkv, q_stride, max_parts, scale_log2);
+      return;
+    }
+  }
+  decode_block<G, BS, false>(sh, len, pl, out, part_o, part_ml, q, kc, vc, block_tables,
+                             bt_stride, hkv, q_stride, max_parts, scale_log2);
 }
 
 // grid: (B * Hq)   block: 256.  Latency bound: a lane takes one partition's (m, l) of each 64 and

@@ -308,6 +308,28 @@ def test_decode_attention_on_shared_prefix_pages(shared, splits):
     assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
 
 
+@pytest.mark.parametrize("hq,bs,part,splits", [(8, 32, 1024, 0), (16, 16, 512, 0), (8, 64, 512, 3)])
+@pytest.mark.parametrize("lens", [[700], [511, 512, 513], [640, 191, 705, 1030, 64] * 4])
+def test_decode_attention_past_and_through_the_caches(lens, hq, bs, part, splits):
+    """Long and short sequences and partitions, alone and beside others, every third sharing a
+    prefix with the next: both walks give the same sums."""
+    torch.manual_seed(13)
+    hkv, B = 2, len(lens)
+    nb_total = sum(-(-n // bs) for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=13)
+    bt = _tables(lens, bs, nb_total)
+    for i in range(0, B - 1, 3):
+        k = min(lens[i], lens[i + 1], 256) // bs
+        bt[i + 1, :k] = bt[i, :k]
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(B, hq, 128, device=DEV, dtype=torch.bfloat16)
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=part, splits=splits)
+    exp = _attention64(q, kc, vc, bt, [1] * B, lens, 128 ** -0.5)
+    # all sums are fp32: what is left is the result's rounding to bf16
+    err = (out.double() - exp).abs()
+    assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
