@@ -612,6 +612,7 @@ def stream(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None 
 
 # -------------------------------------------------- projections of some tens of rows (panel.hip)
 PANEL_MAX_M = 256
+PANEL_ROWS = (16, 32, 48, 64, 80, 96, 128, 160, 192, 224, PANEL_MAX_M)  # of a block
 
 
 def _panel_cost(bm: int, rows: int, K: int, wn: int, S: int) -> float:
@@ -635,9 +636,9 @@ def panel_slices(rows: int, K: int) -> int:
 @functools.lru_cache(maxsize=8192)
 def panel_plan(M: int, rows: int, K: int, slabs: bool) -> tuple[int, int]:
     """(waves a block, K slices) of a panel GEMM with ``rows`` weight rows."""
-    bm = next((b for b in (64, 128, 192) if M <= b), PANEL_MAX_M)
+    bm = next((b for b in PANEL_ROWS if M <= b), PANEL_MAX_M)
     S = panel_slices(rows, K) if slabs else 1
-    return min((_panel_cost(bm, rows, K, wn, S), wn) for wn in (8, 4))[1], S
+    return min((8, 4), key=lambda wn: _panel_cost(bm, rows, K, wn, S)), S
 
 
 def panel(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool = False, bias=None,

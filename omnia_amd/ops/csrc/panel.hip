@@ -3,10 +3,17 @@
 //
 // The weights are still read once and set the floor, but a block that read all of x for 16
 // weight rows of its own (stream.hip) would spend its intake on x.  So x is shared:
-//   * a block of WN waves holds x of 64 to 256 rows in LDS, shared by the waves, and 16 weight
+//   * a block of WN waves holds x of 16 to 256 rows in LDS, shared by the waves, and 16 weight
 //     rows of its own for each; both are filled by LDS-DMA, 8 rows x 128 bytes an instruction
 //     (chunks XORed so that fragment reads have no bank conflicts; weights packed as for
 //     stream.hip, ops.stream_pack, are one KB in fragment order instead);
+//   * every wave reads all of x from LDS, 128 KB a stage of 128 rows and 8 waves, so the rows of a
+//     block are few more than the step's: 16 apart up to 96, then 32.  us with heights of 64,
+//     128, 192 and 256 -> now: 4096 x 4096 at 20 / 77 / 150 rows 8.2 / 11.8 / 15.8 -> 7.6 / 10.0 /
+//     14.9, 6144 x 4096 at 77 15.6 -> 12.5, gated 28672 x 4096 at 20 / 77 / 224 49.6 / 53.7 / 71.8
+//     -> 46.0 / 50.0 / 65.1; 112 beside 128 is not worth its code.  Waves of two weight units read
+//     x half as often and were no faster (28672 x 4096 at 77 51.6, at 256 92): half as many waves
+//     issue the DMA;
 //   * WN is 8, or 4 where few columns would leave CUs without a block; S blocks share a column
 //     tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
 //     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
@@ -52,19 +59,22 @@ constexpr bool grouped(int epi) { return epi >= 5; }
 constexpr bool paired(int epi) { return epi == 1 || epi == 5 || epi == 8; }
 
 template <int N>
+struct Int {
+  static constexpr int value = N;
+};
+
+template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-// 16 bytes a lane from its global address to LDS, lane-linear from the wave's ``dst``, which the
-// load takes from m0.  hipcc reserves m0: it allocates no value to it (and warns that a clobber of
-// it is undefined), and sets it for each instruction of its own that reads it; this file's have
-// none (in the listing m0 is written by these lines alone).  NT: weights, read once (28672 x 4096
+// 16 bytes a lane from its global address to LDS, lane-linear from the wave's byte address ``at``,
+// which the load takes from m0.  hipcc reserves m0: it allocates no value to it (and warns that a
+// clobber of it is undefined), and sets it for each instruction of its own that reads it; this
+// file's have none (in the listing m0 is written by these lines alone).  NT: weights, read once (28672 x 4096
 // at 16 rows 47.0 -> 43.1 us row-major, 44.2 -> 39.9 packed)
 template <bool NT>
-__device__ __forceinline__ void dma16(const void* src, const bf16_t* dst) {
-  const uint32_t at = __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)dst);
+__device__ __forceinline__ void dma16(const void* src, uint32_t at) {
   if constexpr (NT)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(at),
                  "v"(src)
@@ -85,9 +95,10 @@ constexpr int stages(int mf, int wn) {
 template <int MF, int WN, int EPI, bool PK>
 __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
   constexpr int BM = 16 * MF, NS = stages(MF, WN);
-  constexpr int XI = BM / (8 * WN);  // DMA instructions of a wave and stage for x
-  constexpr int L = XI + 2;          // loads of a wave and stage
-  static_assert(NS >= 3 && XI >= 1, "ring");
+  // DMA instructions of a wave and stage for x: XI, of the last XW waves XI - 1
+  constexpr int XI = (2 * MF + WN - 1) / WN, XW = XI * WN - 2 * MF;
+  constexpr int L = XI + 2;  // loads of a wave and stage
+  static_assert(NS >= 3, "ring");
   constexpr int XS = BM * 64, ST = XS + WN * 1024;  // a stage: x, then the waves' weights
   __shared__ __attribute__((aligned(16))) bf16_t xs[NS][ST];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -102,6 +113,7 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
   }
   const int split = bid / tiles, tile = bid - split * tiles;
   const int unit0 = tile * WN + wv, unit = unit0 < units ? unit0 : units - 1;
+  const bool full = XW == 0 || wv < WN - XW;
   const int K = p.K, nch = K >> 6;
   const int c0 = split * nch / p.S, n = (split + 1) * nch / p.S - c0;  // 64-k chunks: stages
 
@@ -125,7 +137,11 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
   const bf16_t* xp[XI];  // DMA instruction i of this wave: 8 rows
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
-    const int r = (wv * XI + i) * 8 + (lane >> 3);
+    const int r = (wv + i * WN) * 8 + (lane >> 3);
+    if (!full && i == XI - 1) {
+      xp[i] = p.x;
+      continue;
+    }
     int64_t row = r < p.M ? r : p.M - 1;
     if constexpr (EPI == 6) {
       row = seg * BM + r;
@@ -135,15 +151,27 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
     }
     xp[i] = p.x + row * p.ldx + (((lane & 7) ^ (r & 7)) << 3);
   }
-  auto issue = [&](bf16_t* dst, int s) {  // stage s into a slot
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) bf16_t*)&xs[0][0]);
+  auto issue = [&](int slot, int s) {  // stage s into a slot
+    const uint32_t dst = lds0 + slot * ST * 2;
     const bool in = s < n;
     const int64_t c = c0 + s;
 #pragma unroll
     for (int i = 0; i < XI; ++i)
-      dma16<false>(in ? xp[i] + c * 64 : p.x, dst + (wv * XI + i) * 512);
+      if (full || i < XI - 1)
+        dma16<false>(in ? xp[i] + c * 64 : p.x, dst + (wv + i * WN) * 1024);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      dma16<true>(in ? wp[h] + c * (PK ? 1024 : 64) : p.x, dst + XS + wv * 1024 + h * 512);
+      dma16<true>(in ? wp[h] + c * (PK ? 1024 : 64) : p.x, dst + XS * 2 + wv * 2048 + h * 1024);
+  };
+  auto landed = [&](auto left) {  // this wave's loads but those of the newest ``left`` stages
+    if (full)
+      wait_vm<decltype(left)::value * L>();
+    else
+      wait_vm<decltype(left)::value * (L - 1)>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
   };
   float4v acc[MF];
 #pragma unroll
@@ -161,30 +189,45 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
     }
   };
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s) issue(xs[s], s);
+  for (int s = 0; s < NS - 1; ++s) issue(s, s);
   int at = 0;
   for (; at + NS < n; at += NS)
 #pragma unroll
     for (int u = 0; u < NS; ++u) {
-      wait_vm<(NS - 2) * L>();  // this stage's loads of this wave
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue(xs[(u + NS - 1) % NS], at + u + NS - 1);
+      landed(Int<NS - 2>());
+      issue((u + NS - 1) % NS, at + u + NS - 1);
       compute(xs[u]);
       __builtin_amdgcn_sched_barrier(0);
     }
-  // up to NS stages are left, the last of them perhaps not yet asked for
-#pragma unroll
-  for (int u = 0; u < NS; ++u)
-    if (at + u < n) {
-      if (u == 0 || u == NS - 1) {
-        wait_vm<0>();
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+  // up to NS stages are left, the last of them perhaps not yet asked for; each is waited for by
+  // itself, since a slice may be a dozen stages (6144 x 4096 in 5 slices at 150 / 256 rows, with
+  // one wait for what is left, 19.9 / 22.3 us, now 16.2 / 20.4)
+  const bool more = at + NS == n;
+  auto last = [&](auto i) {
+    constexpr int u = decltype(i)::value;
+    if constexpr (u < NS) {
+      if (at + u >= n) return;
+      if constexpr (u == 0) {
+        landed(Int<NS - 2>());
+        if (more) issue(NS - 1, at + NS - 1);
+      } else if constexpr (u == NS - 1) {
+        landed(Int<0>());
+      } else {
+        if (more)
+          landed(Int<NS - 1 - u>());
+        else
+          landed(Int<NS - 2 - u>());
       }
-      if (u == 0 && at + NS == n) issue(xs[NS - 1], at + NS - 1);
       compute(xs[u]);
+      __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  last(Int<0>());
+  last(Int<1>());
+  last(Int<2>());
+  last(Int<3>());
+  last(Int<4>());
+  wait_vm<0>();  // loads past the end: none may land in the LDS of a block that follows
 
   // lane: rows 16i + 4fq + r, column fr
   if (unit0 >= units) return;
@@ -241,10 +284,19 @@ int launch(const PanelArgs& p, bool packed, hipStream_t s, int segs = 1) {
 
 template <int WN, int EPI>
 int by_rows(const PanelArgs& p, bool packed, hipStream_t s) {
-  if (p.M <= 64) return launch<4, WN, EPI>(p, packed, s);
-  if (p.M <= 128) return launch<8, WN, EPI>(p, packed, s);
-  if (p.M <= 192) return launch<12, WN, EPI>(p, packed, s);
-  return launch<16, WN, EPI>(p, packed, s);
+  switch ((p.M + 15) / 16) {
+    case 1: return launch<1, WN, EPI>(p, packed, s);
+    case 2: return launch<2, WN, EPI>(p, packed, s);
+    case 3: return launch<3, WN, EPI>(p, packed, s);
+    case 4: return launch<4, WN, EPI>(p, packed, s);
+    case 5: return launch<5, WN, EPI>(p, packed, s);
+    case 6: return launch<6, WN, EPI>(p, packed, s);
+    case 7: case 8: return launch<8, WN, EPI>(p, packed, s);
+    case 9: case 10: return launch<10, WN, EPI>(p, packed, s);
+    case 11: case 12: return launch<12, WN, EPI>(p, packed, s);
+    case 13: case 14: return launch<14, WN, EPI>(p, packed, s);
+    default: return launch<16, WN, EPI>(p, packed, s);
+  }
 }
 
 template <int EPI>

@@ -424,6 +424,19 @@ def test_panel_gated(M, N, K, gelu, packed, monkeypatch):
         _close(got, want, 4 * K, 1.1)
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M", [16, 32, 33, 48, 80, 81, 96, 97, 144, 160, 161, 208, 224, 225, 240])
+def test_panel_every_height(M, packed, monkeypatch):
+    """Blocks of every height, also those whose waves load unlike parts of x, over K from fewer
+    chunks than the ring has stages to two rounds of it."""
+    for chunks in range(1, 11):
+        x, w = _mk(M, 208, 64 * chunks, M + chunks)
+        want, wk = x.double() @ w.double().T, _weight(w, packed)
+        for wn in (4, 8):
+            monkeypatch.setattr(ops, "panel_plan", lambda *a: (wn, 1))
+            _close(ops.panel(0, x, wk, packed=packed), want, 64 * chunks)
+
+
 def test_panel_plans_fit_the_kernel():
     """Whatever the size, a plan is one that the kernel covers, with slices that do not depend on
     the rows."""
