@@ -223,7 +223,7 @@ class HybridModel(Projections):
         if self._pgemm_ok(x.shape[0], x.shape[1], w.shape[0], is_decode):
             return ops.pgemm(0, x, w)
         y = self._few(0, x, w)
-        return ops.linear(x, w) if y is None else y
+        return self._mid(x, w, is_decode, False) if y is None else y
 
     def _slabs(self, tag, x, w, is_decode) -> torch.Tensor:
         """A projection whose consumer also reduces split-K slabs."""

@@ -95,7 +95,7 @@ class Projections:
     # tiles leave most CUs idle, and the split decode / library path is 1.5x
     # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms).
     # Neither threshold holds gated projections off the tile where it fills the
-    # chip (ops.gated_tile_fills): in mixed steps too that is the faster one (8 layers
+    # chip (ops.gated_tile_pays): in mixed steps too that is the faster one (8 layers
     # of 4096 x 14336, 256 decode rows and 190 / 256 prompt rows 3.29 / 3.38 ms with
     # it, 3.37 / 3.45 without; 16 of 2048 x 8192, 256 and 650 5.85 and 6.08)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
@@ -195,7 +195,7 @@ class Projections:
         """ops.wgemm, on the tile-packed copy of ``w`` when one exists for this
         tgemm config; split-K slabs in fp16 on the tile GEMM (``out``'s dtype)."""
         if nwaves == ops.PGEMM_SPLIT:
-            return ops.pgemm_splitk(x, w, S, out)
+            return ops.pgemm_splitk(x, w, S, out, cols=nw)
         if nwaves < 0 and mode == 2 and out is not None and out.dtype == torch.float16:
             mode = 3
         packed = getattr(self, "_packed", None)
@@ -232,10 +232,25 @@ class Projections:
                 self._few(0, x, w, slabs and not tag.endswith("gate_up"))
             if y is not None:
                 return y if y.dim() == 2 else Parts(y)
-            return ops.linear(x, w)
+            return self._mid(x, w, is_decode, slabs and not tag.endswith("gate_up"))
         nw, nwaves, S = cfg
         return Parts(self._wgemm(2, x, w, S, nw, nwaves,
                                  out=self._parts(tag, S, M, w.shape[0], self._slab_dtype(nwaves))))
+
+    def _mid(self, x: torch.Tensor, w: torch.Tensor, is_decode: bool, slabs: bool):
+        """More rows than the few-row kernels take and fewer than ``_pgemm_ok`` asks for: the
+        prefill tile where it fills the chip, whole or in slices of K (fp32 :class:`Parts`), else
+        the library."""
+        M, K = x.shape
+        if M > ops.PANEL_MAX_M and self.tp == 1 and ops._on_grid(x, w) and \
+                self._pgemm_covers(K, w.shape[0], is_decode):
+            if ops.plain_tile_fills(M, w):
+                return ops.pgemm(0, x, w)
+            S = ops.tile_slices(M, w.shape[0], K) if slabs and w.is_contiguous() else 0
+            if S:
+                return Parts(ops.pgemm_splitk(
+                    x, w, S, torch.empty(S, M, w.shape[0], device=x.device), cols=128))
+        return ops.linear(x, w)
 
     _min_rows = int(os.environ.get("OMNIA_PGEMM_MIN_ROWS", "2049"))  # this forward's threshold (mixed steps: the higher one)
 
@@ -246,12 +261,15 @@ class Projections:
         N whole column tiles (``gated``: of a gate's and an up's half, N features
         each of this weight), and at least this forward's row threshold, or for a
         gated one tiles that fill the chip."""
+        return (self._pgemm_covers(K, N if gated is None else 2 * N, is_decode)
+                and N % (256 if gated is None else 128) == 0
+                and (M >= self._min_rows or (gated is not None and ops.gated_tile_pays(M, gated))))
+
+    def _pgemm_covers(self, K: int, R: int, is_decode: bool) -> bool:
         # TP ranks rehearsed on ONE device (ipc transport) keep the library GEMMs:
         # a 256x256 tile's 160 KB of LDS cannot share a CU with the peers'
         # spinning all-reduce blocks, so a rank's GEMM can wait out their spin
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
-        return (self.use_pgemm and not is_decode and K % 128 == 0
-                and N % (256 if gated is None else 128) == 0
-                and (M >= self._min_rows or (gated is not None and ops.gated_tile_fills(M, gated)))
+        return (self.use_pgemm and not is_decode and K % 128 == 0 and R % 128 == 0
                 and self.device.type == "cuda" and self.dtype == torch.bfloat16
                 and (self.tp == 1 or pstate.ranks_per_device() == 1))

@@ -270,7 +270,7 @@ _midm_on = os.environ.get("OMNIA_MIDM", "1") != "0"
 
 def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | None:
     """Mid-size projections (M = 257..4096 rows: open-loop mixed steps, which
-    the unsplit 256x256 prefill tile under-fills): ``(256, PGEMM_SPLIT, S)``
+    the unsplit 256x256 prefill tile under-fills): ``(columns of a tile, PGEMM_SPLIT, S)``
     when ``ops/tuned/midm_mi355x.json`` lists a split-K win of the 256x256 tile
     (+ its slab consumer) over the library path for this shape's M bucket
     (``scripts/midm_sweep.py``), else None (library GEMM)."""
@@ -287,7 +287,12 @@ def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | Non
                 _midm_table = {k: int(v) for k, v in json.load(f).items()}
     b = next(x for x in MIDM_BUCKETS if M <= x)
     S = _midm_table.get(f"{mode}:{b}:{N}:{K}")
-    return (256, PGEMM_SPLIT, S) if S else None
+    if not S:
+        return None
+    # short slices cost more in slabs than the narrow tile's second read of x: as many blocks in
+    # half the slices (us with the consumer's reads, before / after: 4096 x 4096 at 512 rows 32.4
+    # / 28.2, 768 38.1 / 38.0, 999 43.9 / 40.7; not 4096 x 14336: at 512 60.0 / 62.8)
+    return (128, PGEMM_SPLIT, S // 2) if S >= 4 and K <= 4096 else (256, PGEMM_SPLIT, S)
 
 
 def wgemm(mode: int, x: torch.Tensor, w: torch.Tensor, splits: int = 1, nw: int = 2,
@@ -300,7 +305,7 @@ def wgemm(mode: int, x: torch.Tensor, w: torch.Tensor, splits: int = 1, nw: int 
     if nwaves == PGEMM_SPLIT:  # table code for the 256x256 split-K tile (pgemm.hip EPI 4)
         if mode not in (2, 3):
             raise ValueError("the pgemm split-K table entry produces fp16 slabs (mode 2/3)")
-        return pgemm_splitk(x, w, splits, out)
+        return pgemm_splitk(x, w, splits, out, cols=nw)
     if nwaves == 0:  # table code for the wide-batch kernel: nw = 32-col tiles per wave
         return wgemm_wide(mode, x, w, splits, nw, out)
     if nwaves < 0:  # table code for the full-batch tile kernel: nw = weight rows per block,
@@ -392,7 +397,7 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
           ss_in: torch.Tensor | None = None, inv_d: float = 0.0, eps: float = 0.0,
           ss_out: torch.Tensor | None = None, positions=None, cos_sin=None, k_cache=None,
           v_cache=None, slots=None, hq: int = 0, hkv: int = 0, block_size: int = 0,
-          bias: torch.Tensor | None = None, gelu: bool = False):
+          bias: torch.Tensor | None = None, gelu: bool = False, cols: int = 0):
     """Prefill GEMM ``x @ w.T`` with a fused epilogue (``csrc/pgemm.hip``).
 
     ``ss_in`` ([M, n] fp32 partial row sums of squares of ``x``) scales row r by
@@ -403,7 +408,8 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     2: ``out`` is the residual, updated in place (out += GEMM)
     with ``ss_out[r, t]`` = sum of squares of its new 256-column slice t;
     3: QKV -> RoPE'd q in ``out`` [M, hq*128], RoPE'd k and v written to the
-    paged caches at ``slots``."""
+    paged caches at ``slots``.  ``cols``: weight rows of a tile, 256 or (epi 0, 1) 128, to the
+    same bits; 0: :func:`tile_cols`."""
     M, K = x.shape
     N = w.shape[0] // 2 if epi == 1 else w.shape[0]
     if out is None:
@@ -411,8 +417,10 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     if x.is_cuda:
         if epi == 3 and checks.active(x):
             checks.slots("pgemm qkv", slots, k_cache)
+        if not cols and epi <= 1:
+            cols = tile_cols(M, w.shape[0])
         kernels().pgemm(epi, out, x.contiguous(), w, ss_in, inv_d, eps, ss_out, positions,
-                        cos_sin, k_cache, v_cache, slots, hq, hkv, block_size, bias, gelu)
+                        cos_sin, k_cache, v_cache, slots, hq, hkv, block_size, bias, gelu, cols)
         return out
     h = x.float() @ w.float().t()
     if bias is not None:
@@ -440,10 +448,32 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     return out
 
 
+def _tile_rounds(M: int, R: int, cols: int) -> int:
+    return -(-(-(-M // 256) * (R // cols)) // 256)
+
+
+@functools.lru_cache(maxsize=8192)
+def tile_cols(M: int, R: int) -> int:
+    """Columns of :func:`pgemm`'s tile for ``M`` rows and ``R`` weight rows: 128 where that fills
+    the rounds over 256 CUs better, by more than its second read of x.  A round of narrow tiles
+    takes 0.57 to 0.6 of a wide one's (us wide / narrow and their rounds: gated 16384 x 2048 at 300
+    rows 43.8 / 31.2 (1, 1), 600 45.6 / 54.4 (1, 2), 1536 92.5 / 87.0 (2, 3), 2001 103 / 120 (2,
+    4); 28672 x 4096 at 600 165 / 149 (2, 3), 1280 253 / 266 (3, 5); plain 4096 x 2048 at 2001
+    42.6 / 30.6 (1, 1))."""
+    narrow = R % 256 == 0 and 0.6 * _tile_rounds(M, R, 128) < 0.97 * _tile_rounds(M, R, 256)
+    return 128 if narrow else 256
+
+
+def _tiles_useful(M: int, R: int) -> float:
+    """Part of the work of :func:`pgemm`'s rounds that is not padding."""
+    cols = tile_cols(M, R)
+    return M * R / (256 * 256 * cols * _tile_rounds(M, R, cols))
+
+
 def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
     """Whether a gated :func:`pgemm` of more rows than the panel kernel takes covers ``w`` = [Wg; Wu]
-    and its tiles of 256 rows x 128 features are worth their rounds over 256 CUs: from three quarters of their work useful,
-    the activation in the epilogue makes up for the rest (useful part, us here / library and
+    and its wide tiles (128 features) are worth their rounds over 256 CUs: from three quarters of
+    their work useful, the activation in the epilogue makes up for the rest (useful part, us here / library and
     activation kernel; 8192 features of 2048: 512 rows .50 48 / 42, 768 .75 51.5 / 52.7, 999 .98
     55 / 67, 1536 .75 99 / 99, 2001 .98 108 / 124; 14336 of 4096: 320 .55 93 / 88, 512 .88 99 / 112,
     768 .66 177 / 163, 999 .85 187 / 198)."""
@@ -455,23 +485,67 @@ def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
         w.is_contiguous() and _on_grid(w)
 
 
+def gated_tile_pays(M: int, w: torch.Tensor) -> bool:
+    """:func:`gated_tile_fills` of the wide tile or, by the same line, of the narrow one where
+    :func:`tile_cols` takes that (us, here / library and activation kernel: 8192 features of 2048 at
+    300 rows .59 useful 31.2 / 35.1, 512 1.0 32.8 / 40.9, 1280 .83 82.7 / 84.2; 14336 of 4096 at
+    600 .68 149 / 139, 768 .88 162 / 158)."""
+    return gated_tile_fills(M, w) or (
+        M > PANEL_MAX_M and tile_cols(M, w.shape[0]) == 128 and
+        _tiles_useful(M, w.shape[0]) > 0.75 and w.is_contiguous() and _on_grid(w))
+
+
+def plain_tile_fills(M: int, w: torch.Tensor) -> bool:
+    """Whether an ungated :func:`pgemm` of more rows than the panel kernel takes covers ``w`` and
+    beats the library: from nine tenths of its tiles' work useful (useful part, us here /
+    library: 4096 x 2048 at 1536 rows .75 28.9 / 29.3, 2001 .98 30.6 / 34.6; 4096 x 4096 at 1536 .75
+    52.0 / 51.6, 2001 .98 55 / 60; 4096 x 14336 at 1536 .75 180 / 176, 2001 .98 194 / 204; 2048 x
+    2048 at 2001 .49 27.1 / 23.8)."""
+    if M <= PANEL_MAX_M or w.dim() != 2:
+        return False
+    R, K = w.shape
+    return K % 128 == 0 and R % 256 == 0 and _tiles_useful(M, R) > 0.9 and \
+        w.is_contiguous() and _on_grid(w)
+
+
+@functools.lru_cache(maxsize=8192)
+def tile_slices(M: int, R: int, K: int) -> int:
+    """K slices in which :func:`pgemm_splitk`'s narrow tile runs ``M`` rows of a weight [R, K] into
+    fp32 slabs, where that and the consumer's reads of them take less than the library and its
+    rows; 0 where not.  By what both take (us): a tile 0.67 for 64 of K and 5 besides, slabs written
+    at 3.6 TB/s and read at 7, as many slices as 256 CUs take at once; the library 9, 1.9 for 1000
+    of K and its products at 1.35 PFLOP/s.  With a margin, since its kernels change with every size
+    (us with the consumer, library / here, rows of 2048 x 8192: 257 40.7 / 31.4, 512 41.9 / 35.0,
+    768 50.5 / 43.2, 999 62.5 / 48.9, 1536 71.2 / 71.9 not taken, 2001 88.7 / 77.4; 4096 x 8192:
+    512 61 / 51, 768 71 / 73 not taken; 2048 x 16384: 999 101 / 73; 2048 x 4096: 257 27.6 / 24.3,
+    999 37.4 / 36.2 not taken)."""
+    if M <= PANEL_MAX_M or M > 2048 or R % 128 or K % 128:
+        return 0
+    tiles, best = -(-M // 256) * (R // 128), (0.9 * (9.0 + 1.9e-3 * K + 2 * M * R * K / 1.35e9), 0)
+    for S in range(2, 17):
+        if tiles * S <= 256 and K % (128 * S) == 0:
+            t = 5.0 + 0.67 * K / 64 / S + M * R * (4 * S / 3.6e6 + (4 * S - 2) / 7e6)
+            best = min(best, (t, S))
+    return best[1]
+
+
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
-                 sched: int = 0) -> torch.Tensor:
-    """fp16 split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the 256x256 MFMA tile
-    (``csrc/pgemm.hip`` EPI 4; ``sched`` 0 or 1, of no effect).  Each
-    slab is one K-slice's fp32 sum saturated to fp16; the splitk consumers reduce
-    them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip)."""
+                 sched: int = 0, cols: int = 0) -> torch.Tensor:
+    """Split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the MFMA tile of 256 rows and ``cols``
+    (128, else 256) columns (``csrc/pgemm.hip`` EPI 4; ``sched`` 0 or 1, of no effect).  Each
+    slab is one K-slice's fp32 sum, saturated to fp16 unless ``out`` is fp32; the splitk consumers
+    reduce them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip)."""
     M, K = x.shape
     N = w.shape[0]
     if out is None:
         out = torch.empty(splits, M, N, dtype=torch.float16, device=x.device)
     if x.is_cuda:
-        kernels().pgemm_splitk(out, x.contiguous(), w, sched)
+        kernels().pgemm_splitk(out, x.contiguous(), w, sched, 128 if cols == 128 else 256)
         return out
     ks = K // splits
     for s in range(splits):
         r = x[:, s * ks:(s + 1) * ks].float() @ w[:, s * ks:(s + 1) * ks].float().t()
-        out[s].copy_(r.clamp(-65504.0, 65504.0).to(out.dtype))
+        out[s].copy_(r if out.dtype == torch.float32 else r.clamp(-65504.0, 65504.0))
     return out
 
 

@@ -17,7 +17,7 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
                 const float* ss_in, int ss_in_n, float inv_d, float eps, float* ss_out,
                 const int* positions, const float* cos_sin, void* k_cache, void* v_cache,
                 const int64_t* slots, int hq, int hkv, int block_size, const float* bias,
-                int gelu, hipStream_t s);
+                int gelu, int cols, hipStream_t s);
 int omnia_row_sumsq(float* ss, const void* x, int rows, int d, int64_t stride, hipStream_t s);
 int omnia_ar_alltoall(void* out, const void* in, void* const* regions, int* epochs, int* err,
                       int64_t chunk, int64_t slot_bytes, int rank, int world, hipStream_t s);
@@ -26,7 +26,7 @@ int omnia_ar_sendrecv(void* out, const void* in, void* const* regions, int* epoc
                       hipStream_t s);
 int omnia_pgemm_set_schedule(int sched);
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int sched, hipStream_t s);
+                       int sched, int cols, int f32, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
@@ -970,7 +970,8 @@ void pgemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W,
            c10::optional<at::Tensor> ss_out, c10::optional<at::Tensor> positions,
            c10::optional<at::Tensor> cos_sin, c10::optional<at::Tensor> k_cache,
            c10::optional<at::Tensor> v_cache, c10::optional<at::Tensor> slots, int64_t hq,
-           int64_t hkv, int64_t block_size, c10::optional<at::Tensor> bias, bool gelu) {
+           int64_t hkv, int64_t block_size, c10::optional<at::Tensor> bias, bool gelu,
+           int64_t cols) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W); CHECK_BF16(out);
   TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && out.dim() == 2, "2-D operands");
   TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "contiguous x / W");
@@ -1033,7 +1034,7 @@ void pgemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W,
   if (M == 0) return;
   CHECK_RC(omnia_pgemm((int)epi, out.data_ptr(), x.data_ptr(), W.data_ptr(), M, N, K,
                        out.stride(0), ssi, ssn, (float)inv_d, (float)eps, sso, pos, cs, kc, vc, sl,
-                       (int)hq, (int)hkv, (int)block_size, bp, gelu, cur_stream()),
+                       (int)hq, (int)hkv, (int)block_size, bp, gelu, (int)cols, cur_stream()),
            "pgemm");
 }
 
@@ -1146,18 +1147,20 @@ void panel_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t
            "panel_gemm");
 }
 
-// split-K 256x256 MFMA GEMM (pgemm.hip EPI 4): parts fp16 [S, M, N] whose sum
-// over S is x @ W^T; sched as pgemm_set_schedule's
-void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t sched) {
+// split-K MFMA GEMM (pgemm.hip EPI 4, 11): parts fp16 or fp32 [S, M, N] whose sum
+// over S is x @ W^T; sched as pgemm_set_schedule's; cols of a tile: 128, 256 (0)
+void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t sched, int64_t cols) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W);
   TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1), "x [M, K], W [N, K]");
   TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "contiguous x / W");
-  TORCH_CHECK(parts.scalar_type() == at::kHalf && parts.is_contiguous() && parts.dim() == 3 &&
-              parts.size(1) == x.size(0) && parts.size(2) == W.size(0), "parts fp16 [S, M, N]");
+  const bool f32 = parts.scalar_type() == at::kFloat;
+  TORCH_CHECK((f32 || parts.scalar_type() == at::kHalf) && parts.is_contiguous() &&
+              parts.dim() == 3 && parts.size(1) == x.size(0) && parts.size(2) == W.size(0),
+              "parts fp16 or fp32 [S, M, N]");
   TORCH_CHECK(x.device() == W.device() && x.device() == parts.device(), "same device");
   if (x.size(0) == 0) return;
   CHECK_RC(omnia_pgemm_splitk(parts.data_ptr(), x.data_ptr(), W.data_ptr(), x.size(0), W.size(0),
-                              x.size(1), parts.size(0), (int)sched, cur_stream()),
+                              x.size(1), parts.size(0), (int)sched, (int)cols, f32, cur_stream()),
            "pgemm_splitk");
 }
 

@@ -1,7 +1,6 @@
 // Prefill GEMM with fused epilogues on gfx950:  out = X[M, K] . W[N, K]^T  for
 // prefill chunks (M = hundreds to 16K rows), bf16 operands, fp32 MFMA accumulate.
-// SURVEY §2.4 K3 (QKV), K4/K5 (RoPE + paged KV write), K8 (O), K9 (SwiGLU),
-// K10 (down), K2 (residual add + RMSNorm).
+// QKV (with RoPE and the paged KV write), O, SwiGLU, down (with the residual add).
 //
 // Main loop: a 256x256 tile by four waves, 2 x 2, one a SIMD, 128 x 128 of the tile each (256
 // fp32 accumulators a lane, in AGPRs), in K-tiles of 64:
@@ -27,6 +26,11 @@
 // Normal values, us before (eight waves, one K-tile ahead) and now, 16384 rows: 4096 x 4096
 // 382 / 361, 4096 x 14336 1344 / 1270, 28672 x 4096 2698 / 2574 (1.50 PF/s), 6144 x 4096 578 /
 // 554, 2048 x 2048 110 / 100.
+// The narrow tile (NF 4: 128 columns, a wave 128 x 64, K-tiles of three halves in a ring of nine) is
+// for steps of some hundred rows, whose wide tiles leave CUs without one: a round of them takes
+// 0.57 to 0.6 of a wide round, bound by what a CU takes in (48 KB in 0.67 us, where the wide
+// tile's 64 KB in 1.09 are at the rate of its products).  us wide / narrow: gated 16384 x 2048 at 512
+// rows 45.5 / 32.8, 4096 x 2048 at 2001 42.6 / 30.6; in 4 slices 2048 x 8192 at 999 45.8 / 33.4.
 // Epilogues (W is the product's first operand, so a lane holds four neighbouring columns of a
 // row; lanes exchange pairs and store 16 bytes, 64 a row and instruction, past LDS):
 //   EPI 0  out = rs[r] * acc                                  (plain / row-scaled)
@@ -47,6 +51,7 @@
 //          fp32 sum, saturated to fp16, into slab ks of out[S][M][N]; the splitk.hip
 //          consumers reduce the slabs (decode projections at M <= 256: one m-tile,
 //          the K split fills the chip that N / 256 column tiles alone cannot)
+//   EPI 11 EPI 4 with the sums as they are, slabs in fp32
 // where rs[r] = rsqrt(sum_t ss_in[r][t] / d + eps): with the RMSNorm weight folded
 // into W (W' = W * diag(w), models/llama.py fold_norms), RMSNorm(h) @ W^T ==
 // rs * (h @ W'^T), so the normalisation rides the consumer's epilogue and the
@@ -65,7 +70,8 @@ typedef float float2v __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 64;
 constexpr int HALF = 128 * BK;  // bf16 elements of a half-tile (16 KB)
-constexpr int RING = 10 * HALF;
+// NF: 16-column fragments of a wave; a block's tile is 256 rows x 32 NF columns
+constexpr int ring(int nf) { return (nf == 8 ? 10 : 9) * HALF; }
 
 struct PArgs {
   void* out;            // EPI 0/1: bf16 [M, ldo]; EPI 2: residual bf16 [M, ldo]; EPI 3: q [M, ldo]
@@ -98,6 +104,8 @@ struct PArgs {
 constexpr bool gated(int epi) {
   return epi == 1 || epi == 5 || epi == 7 || epi == 8 || epi == 9;
 }
+// slabs of K-slices
+constexpr bool sliced(int epi) { return epi == 4 || epi == 11; }
 // rows are expert-sorted assignments
 constexpr bool grouped(int epi) { return epi == 5 || epi == 6 || epi == 8 || epi == 10; }
 // A rows are token rows gathered by assignment
@@ -183,21 +191,22 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-template <int EPI>
+template <int EPI, int NF = 8>
 __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
+  constexpr int RING = ring(NF), KT = 2 + NF / 4;  // half-tiles of a K-tile
   __shared__ __attribute__((aligned(1024))) bf16_t lds[RING];
-  constexpr int TN = gated(EPI) ? 128 : 256;  // output columns per block tile
+  constexpr int TN = gated(EPI) ? 16 * NF : 32 * NF;  // output columns per block tile
   constexpr bool MOE = grouped(EPI), GATHER = gathered(EPI);
-  // EPI 4: the K-slices are extra "m-tiles" of the L2 grouping below (blocks of
+  // sliced: the K-slices are extra "m-tiles" of the L2 grouping below (blocks of
   // one slice share its x slice, blocks of one column tile its W rows)
-  const int S = EPI == 4 ? p.splits : 1;
+  const int S = sliced(EPI) ? p.splits : 1;
   // MoE: the grid is sized for the worst-case segment count (graph-safe, no host sync); the
   // live tiles are spread over the XCDs, the other blocks leave
   const int ntn = p.N / TN, mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8, mtn = mtn1 * S;
   const int tiles = MOE ? mtn * ntn : gridDim.x;
   if (MOE && blockIdx.x >= tiles) return;
   const int bid = xcd_remap(blockIdx.x, tiles);
-  const int gm = (int64_t)ntn * p.K > (1 << 18) ? 8 : 4;  // 128 MB of W (256 rows a tile)
+  const int gm = (int64_t)ntn * NF * p.K > (1 << 21) ? 8 : 4;  // 128 MB of W (32 NF rows a tile)
   const int per_group = gm * ntn;
   const int grp = bid / per_group, gm0 = grp * gm;
   const int gsz = mtn - gm0 < gm ? mtn - gm0 : gm;
@@ -224,8 +233,12 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     base[h] = (const char*)(p.X + (int64_t)m0 * K + kbase);
-    base[2 + h] = (const char*)(Wb + ((gated(EPI) ? (int64_t)h * p.N + (int64_t)nt * 128
-                                                  : (int64_t)nt * 256 + h * 128)) * K);
+    if constexpr (NF == 8)
+      base[2 + h] = (const char*)(Wb + ((gated(EPI) ? (int64_t)h * p.N + (int64_t)nt * 128
+                                                    : (int64_t)nt * 256 + h * 128)) * K);
+    else  // one half-tile: gated, 64 rows of the gate's half and (waves 2, 3) 64 of the up's
+      base[2] = (const char*)(Wb + (gated(EPI) ? (int64_t)nt * 64 + (w >> 1) * ((int64_t)p.N - 64)
+                                               : (int64_t)nt * 128) * K);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 32 * w + 8 * i + (lane >> 3);
@@ -242,11 +255,11 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
     }
   }
 
-  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10
+  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10, or (3t + h) mod 9
   const uint32_t dst0 =
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)lds + 32 * w * 128;
-  auto step4 = [&](int s) __attribute__((always_inline)) {  // a K-tile on
-    return s + 4 * HALF >= RING ? s + 4 * HALF - RING : s + 4 * HALF;
+  auto next = [&](int s) __attribute__((always_inline)) {  // a K-tile on
+    return s + KT * HALF >= RING ? s + KT * HALF - RING : s + KT * HALF;
   };
   int da = 0, db = 2 * HALF, ka = 0, kb = 0;  // slots and K-tiles to ask for next
   uint32_t qa = 0, qb = 0;                    // of the DMAs under way: LDS address, sources
@@ -259,14 +272,14 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
     pa[0] = base[0] + koff;
     pa[1] = base[1] + koff;
     ka = ka + 1 < nk ? ka + 1 : nk - 1;
-    da = step4(da);
+    da = next(da);
   };
   auto set_b = [&]() __attribute__((always_inline)) {
     qb = dst0 + db * 2;
     pb[0] = base[2] + (int64_t)kb * (BK * 2);
-    pb[1] = base[3] + (int64_t)kb * (BK * 2);
+    if constexpr (NF == 8) pb[1] = base[3] + (int64_t)kb * (BK * 2);
     kb = kb + 1 < nk ? kb + 1 : nk - 1;
-    db = step4(db);
+    db = next(db);
   };
   auto dma_a = [&](int d) __attribute__((always_inline)) {
     const int h = d >> 2, i = d & 3, off = h * HALF * 2 + i * 1024;
@@ -276,62 +289,66 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   auto dma_b = [&](int d) __attribute__((always_inline)) {
     dma16(vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb, (d >> 2) * HALF * 2 + (d & 3) * 1024);
   };
-  // K-tiles 0 and 1, and A of 2
+  // K-tiles 0 and 1, and A of 2 (NF 4: all of it)
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
     set_a();
 #pragma unroll
     for (int d = 0; d < 8; ++d) dma_a(d);
-    if (t < 2) {
+    if (t < 2 || NF == 4) {
       set_b();
 #pragma unroll
-      for (int d = 0; d < 8; ++d) dma_b(d);
+      for (int d = 0; d < NF; ++d) dma_b(d);
     }
   }
 
   // ---- fragments: A rows wr*128 + 16m + fr; B rows of half wc, or (gated) rows wc*64 + 16n + fr
-  // of the gate's half for n < 4 and of the up's for n >= 4; k chunk 4s + fq of step s
+  // of the gate's half for n < 4 and of the up's for n >= 4 (NF 4: the same in quarters); k chunk
+  // 4s + fq of step s
+  constexpr int NG = NF / 2;  // gate fragments of a wave
+  constexpr int WCOL = (gated(EPI) ? NG : NF) * 16;
   const bf16_t *fa[2], *fb[2];
-  int ra = wr * HALF, rb = gated(EPI) ? 2 * HALF : (2 + wc) * HALF;
+  int ra = wr * HALF, rb = gated(EPI) || NF == 4 ? 2 * HALF : (2 + wc) * HALF;
   auto set_r = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int at = fr * BK + (((4 * s + fq) ^ (fr & 7)) << 3);
       fa[s] = lds + ra + at;
-      fb[s] = lds + rb + at + (gated(EPI) ? wc * 64 * BK : 0);
+      fb[s] = lds + rb + at + (gated(EPI) || NF == 4 ? wc * WCOL * BK : 0);
     }
-    ra = step4(ra);
-    rb = step4(rb);
+    ra = next(ra);
+    rb = next(rb);
   };
   set_r();
-  short8 fx[2][8], fw[2][8];
-  auto read = [&](int set, int s, int j) __attribute__((always_inline)) {  // x 0, w 0..7, x 1..7
-    if (j == 0 || j > 8) {
-      const int m = j ? j - 8 : 0;
+  short8 fx[2][8], fw[2][NF];
+  auto read = [&](int set, int s, int j) __attribute__((always_inline)) {  // x 0, all w, x 1..7
+    if (j == 0 || j > NF) {
+      const int m = j ? j - NF : 0;
       fx[set][m] = *reinterpret_cast<const short8*>(fa[s] + m * 16 * BK);
     } else {
-      const int n = j - 1, at = gated(EPI) ? (n >> 2) * HALF + (n & 3) * 16 * BK : n * 16 * BK;
+      const int n = j - 1;
+      const int at = gated(EPI) ? n / NG * NG * 32 * BK + n % NG * 16 * BK : n * 16 * BK;
       fw[set][n] = *reinterpret_cast<const short8*>(fb[s] + at);
     }
   };
 
-  float4v acc[8][8];  // [m][n]: rows 16m + fr, columns 16n + 4fq + j
+  float4v acc[8][NF];  // [m][n]: rows 16m + fr, columns 16n + 4fq + j
   // accumulators settle: a product may be behind them, a read or write of theirs before them
   auto pin = [&]() __attribute__((always_inline)) {
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 64; ++i) asm volatile("" : "+a"(acc[i >> 3][i & 7]));
+    for (int i = 0; i < 8 * NF; ++i) asm volatile("" : "+a"(acc[i / NF][i % NF]));
     asm volatile("s_nop 15" ::: "memory");
   };
 #pragma unroll
   for (int m = 0; m < 8; ++m)
 #pragma unroll
-    for (int n = 0; n < 8; ++n) acc[m][n] = {0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NF; ++n) acc[m][n] = {0.f, 0.f, 0.f, 0.f};
   pin();
 
   // this thread's row scale, ready before the loop
   constexpr bool ROUTED = EPI == 6 || EPI == 8;
-  constexpr bool UNSCALED = EPI == 2 || EPI == 7 || EPI == 9 || EPI == 10;
+  constexpr bool UNSCALED = EPI == 2 || EPI == 11 || EPI == 7 || EPI == 9 || EPI == 10;
   const bool scaled = ROUTED || (!UNSCALED && p.ss_in != nullptr);
   float own = 1.f;
   if constexpr (ROUTED) {  // the assignment's routing weight
@@ -351,7 +368,7 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   }
 
   auto product = [&](int set, int j, int d) __attribute__((always_inline)) {  // d: DMA or -1
-    const int m = j >> 3, n = (m & 1) ? 7 - (j & 7) : j & 7;
+    const int m = j / NF, n = (m & 1) ? NF - 1 - j % NF : j % NF;
     if (d < 0) {
       mfma16(acc[m][n], fw[set][n], fx[set][m]);
     } else if (d < 8) {
@@ -365,34 +382,45 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
         mfma16_dma(acc[m][n], fw[set][n], fx[set][m], vo[h][i], pa[h], qa, off);
     }
   };
-  // Step s of K-tile t: 64 products of 32 k.  FREE: every wave has read the K-tile (its last
-  // fragments are asked for by product 30 of step 0); its slots take B of t + 2, then, behind
-  // LAND, A of t + 3.  LAND: the 16 loads younger than B of t + 1 (A of t + 2, B of t + 2) may
-  // be under way, K-tile t + 1 is there, and its first fragments are read.
-  constexpr int FREE = 36, LAND = 12;
+  // Step s of K-tile t: 8 NF products of 32 k.  FREE: every wave has read the K-tile (its last
+  // fragments are asked for by product 30 of step 0, NF 4: 22); its slots take B of t + 2, then,
+  // behind LAND, A of t + 3 (NF 4: B and A of t + 3).  LAND: the loads younger than K-tile t + 1
+  // may be under way (NF 8: A and B of t + 2; NF 4: all of t + 2, 5 of t + 3), K-tile t + 1 is
+  // there, and its first fragments are read.
+  constexpr int P = 8 * NF, FREE = NF == 8 ? 36 : 26, LAND = NF == 8 ? 12 : 6;
+  constexpr int YOUNGER = NF == 8 ? 16 : 17;
+  // the DMA behind product j: B's are 0 to NF - 1, A's 8 to 15; -1: none
+  auto dma_at = [](int s, int j) constexpr {
+    if (NF == 8) {
+      if (s == 0 && j >= FREE && (j - FREE) % 3 == 0 && (j - FREE) / 3 < 8) return (j - FREE) / 3;
+      if (s == 1 && j > LAND && (j - LAND) % 6 == 3 && (j - LAND) / 6 < 8)
+        return 8 + (j - LAND) / 6;
+    } else {
+      if (s == 0 && j >= FREE && (j - FREE) % 2 == 0) return (j - FREE) / 2;  // B 0 to 2
+      if (s == 1 && j % 3 == 1 && j < 27) return j == 1 ? 3 : 8 + j / 3 - 1;
+    }
+    return -1;
+  };
   auto step = [&](auto SC) __attribute__((always_inline)) {
     constexpr int s = decltype(SC)::value;
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
+    for (int j = 0; j < P; ++j) {
       if (s == 0 && j == FREE) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
       if (s == 1 && j == LAND) {
-        wait_vm<16>();
+        wait_vm<YOUNGER>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
-      int d = -1;
-      if (s == 0 && j >= FREE && (j - FREE) % 3 == 0 && (j - FREE) / 3 < 8) d = (j - FREE) / 3;
-      if (s == 1 && j > LAND && (j - LAND) % 6 == 3 && (j - LAND) / 6 < 8) d = 8 + (j - LAND) / 6;
-      product(s, j, d);
-      if (s == 0 && !(j & 1) && j < 32) read(1, 1, j >> 1);
-      if (s == 1 && !(j & 1) && j >= LAND && j < LAND + 32) read(0, 0, (j - LAND) >> 1);
+      product(s, j, dma_at(s, j));
+      if (s == 0 && !(j & 1) && j < 2 * (8 + NF)) read(1, 1, j >> 1);
+      if (s == 1 && !(j & 1) && j >= LAND && j < LAND + 2 * (8 + NF)) read(0, 0, (j - LAND) >> 1);
       // addresses of what comes next, between products that hide them
-      if (s == 0 && j == 33) set_b();
-      if (s == 0 && j == 48) set_r();
+      if (s == 0 && j == FREE - 3) set_b();
+      if (s == 0 && j == (NF == 8 ? 48 : 29)) set_r();
       if (s == 1 && j == 2) set_a();
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -401,7 +429,7 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 16; ++j) read(0, 0, j);
+  for (int j = 0; j < 8 + NF; ++j) read(0, 0, j);
   for (int t = 0; t < nk; ++t) {
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
@@ -426,12 +454,12 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   }
   bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
   if constexpr (gated(EPI)) {
-    // gate (n < 4) and up (n + 4) of features nt*128 + wc*64 + 16n + 4fq + j in one lane
-    const int f0 = nt * 128 + wc * 64;
-    float4v bg[4], bu[4];
+    // gate (n < NG) and up (n + NG) of features nt*TN + wc*WCOL + 16n + 4fq + j in one lane
+    const int f0 = nt * TN + wc * WCOL;
+    float4v bg[NG], bu[NG];
     if constexpr (EPI == 7)
 #pragma unroll
-      for (int n = 0; n < 4; ++n)
+      for (int n = 0; n < NG; ++n)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           bg[n][j] = p.bias[f0 + 16 * n + 4 * fq + j];
@@ -440,10 +468,10 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
       const int r = row0 + 16 * m;
-      float4v v[4];
+      float4v v[NG];
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        float4v g = acc[m][n], u = acc[m][n + 4];
+      for (int n = 0; n < NG; ++n) {
+        float4v g = acc[m][n], u = acc[m][n + NG];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if constexpr (EPI == 7)
@@ -458,8 +486,9 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
       }
       if (r < Mt) {
         bf16_t* o = out + (int64_t)(m0 + r) * p.ldo + f0 + ccol;
-        *reinterpret_cast<uint4v*>(o) = chunk<EPI>(v[0], v[1]);
-        *reinterpret_cast<uint4v*>(o + 32) = chunk<EPI>(v[2], v[3]);
+#pragma unroll
+        for (int n = 0; n < NG; n += 2)
+          *reinterpret_cast<uint4v*>(o + 16 * n) = chunk<EPI>(v[n], v[n + 1]);
       }
     }
   } else if constexpr (EPI == 2) {
@@ -556,6 +585,16 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
         *reinterpret_cast<uint4v*>(d + 96) = v3;
       }
     }
+  } else if constexpr (EPI == 11) {
+    float* slab = reinterpret_cast<float*>(p.out) + (int64_t)ks * p.M * p.N + nt * TN + wc * WCOL;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int r = row0 + 16 * m;
+      if (r < Mt)
+#pragma unroll
+        for (int n = 0; n < NF; ++n)
+          *reinterpret_cast<float4v*>(slab + (int64_t)(m0 + r) * p.N + 16 * n + 4 * fq) = acc[m][n];
+    }
   } else {
     if constexpr (EPI == 4) out += (int64_t)ks * p.M * p.N;
 #pragma unroll
@@ -567,9 +606,9 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
         orow = p.sorted[m0 + r];
         live = orow < p.n_assign;
       }
-      bf16_t* o = out + orow * p.ldo + (int64_t)nt * 256 + wc * 128 + ccol;
+      bf16_t* o = out + orow * p.ldo + (int64_t)nt * TN + wc * WCOL + ccol;
 #pragma unroll
-      for (int n = 0; n < 8; n += 2) {
+      for (int n = 0; n < NF; n += 2) {
         float4v c = acc[m][n], d = acc[m][n + 1];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -616,7 +655,7 @@ extern "C" {
 // (checked BEFORE any launch).
 int omnia_pgemm_set_schedule(int sched);
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int sched, hipStream_t s);
+                       int sched, int cols, int f32, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
@@ -629,13 +668,16 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
                 const float* ss_in, int ss_in_n, float inv_d, float eps, float* ss_out,
                 const int* positions, const float* cos_sin, void* k_cache, void* v_cache,
                 const int64_t* slots, int hq, int hkv, int block_size, const float* bias,
-                int gelu, hipStream_t s) {
+                int gelu, int cols, hipStream_t s) {
   if (epi < 0 || epi > 3) return -1;
+  if (cols && cols != 128 && cols != 256) return -16;
+  const bool narrow = cols == 128;
+  if (narrow && epi > 1) return -16;
   if (bias && (epi != 1 || ss_in)) return -14;
   if (gelu && (epi != 1 || ss_in || bias)) return -15;
   if (M < 1) return -2;
   if (K <= 0 || K % (2 * BK)) return -3;  // whole iterations of two K-tiles
-  const int tn = epi == 1 ? 128 : 256;
+  const int tn = (epi == 1 ? 128 : 256) >> (narrow ? 1 : 0);
   if (N <= 0 || N % tn) return -4;
   if ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
        reinterpret_cast<uintptr_t>(out)) & 15)
@@ -659,39 +701,52 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
           ss_out, positions, cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache, slots, hq, hkv,
           block_size, 1, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, bias};
   const dim3 grid((unsigned)blocks);
-  if (bias) {
-    pgemm_kernel<7><<<grid, 256, 0, s>>>(a);
-    return (int)hipGetLastError();
-  }
-  if (gelu) {
-    pgemm_kernel<9><<<grid, 256, 0, s>>>(a);
-    return (int)hipGetLastError();
-  }
+#define OMNIA_PGEMM(EPI)                                       \
+  do {                                                         \
+    if (narrow)                                                \
+      pgemm_kernel<EPI, 4><<<grid, 256, 0, s>>>(a);            \
+    else                                                       \
+      pgemm_kernel<EPI, 8><<<grid, 256, 0, s>>>(a);            \
+    return (int)hipGetLastError();                             \
+  } while (0)
+  if (bias) OMNIA_PGEMM(7);
+  if (gelu) OMNIA_PGEMM(9);
   switch (epi) {
-    case 0: pgemm_kernel<0><<<grid, 256, 0, s>>>(a); break;
-    case 1: pgemm_kernel<1><<<grid, 256, 0, s>>>(a); break;
+    case 0: OMNIA_PGEMM(0);
+    case 1: OMNIA_PGEMM(1);
+#undef OMNIA_PGEMM
     case 2: pgemm_kernel<2><<<grid, 256, 0, s>>>(a); break;
     default: pgemm_kernel<3><<<grid, 256, 0, s>>>(a); break;
   }
   return (int)hipGetLastError();
 }
 
-// split-K GEMM: parts[S][M][N] fp16, sum over s of parts[s] = X . W^T (EPI 4).
-// `sched` as omnia_pgemm_set_schedule's.
+// split-K GEMM: parts[S][M][N] fp16 or fp32, sum over s of parts[s] = X . W^T (EPI 4, 11).
+// `sched` as omnia_pgemm_set_schedule's; cols: of a tile, 128 or 256 (0).
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int sched, hipStream_t s) {
+                       int sched, int cols, int f32, hipStream_t s) {
+  if (cols && cols != 128 && cols != 256) return -16;
+  const int tn = cols == 128 ? 128 : 256;
   if (M < 1 || S < 1 || S > 16) return -1;
   if (K <= 0 || K % S || (K / S) % (2 * BK)) return -3;
-  if (N <= 0 || N % 256) return -4;
+  if (N <= 0 || N % tn) return -4;
   if ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
        reinterpret_cast<uintptr_t>(parts)) & 15)
     return -5;
-  const int64_t blocks = (int64_t)((M + 255) / 256) * (N / 256) * S;
+  const int64_t blocks = (int64_t)((M + 255) / 256) * (N / tn) * S;
   if (blocks > (1 << 30)) return -13;
   PArgs a{parts, (const bf16_t*)X, (const bf16_t*)W, M, N, K, N, nullptr, 0, 0.f, 0.f, nullptr,
           nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, S, nullptr, nullptr, nullptr,
           nullptr, 0, 0, 0};
-  pgemm_kernel<4><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
+  const dim3 grid((unsigned)blocks);
+  if (f32 && tn == 128)
+    pgemm_kernel<11, 4><<<grid, 256, 0, s>>>(a);
+  else if (f32)
+    pgemm_kernel<11><<<grid, 256, 0, s>>>(a);
+  else if (tn == 128)
+    pgemm_kernel<4, 4><<<grid, 256, 0, s>>>(a);
+  else
+    pgemm_kernel<4><<<grid, 256, 0, s>>>(a);
   return (int)hipGetLastError();
 }
 

@@ -31,3 +31,26 @@ def test_bucket_mapping_and_boundaries():
 def test_kill_switch(monkeypatch):
     monkeypatch.setattr(ops, "_midm_on", False)
     assert ops.midm_config(600, 4096, 14336, 0) is None
+
+
+def test_slices_of_the_narrow_tile_fit_the_kernel():
+    """Whole K-tile pairs in every slice, one round of blocks, only between the few-row kernels and
+    the prefill rows, and only where it takes a tenth less than the library by their models."""
+    taken = 0
+    for M in (1, 256, 257, 512, 999, 2001, 2048, 2049, 5000):
+        for R in (128, 256, 1000, 2048, 4096, 16384):
+            for K in (128, 1000, 2048, 4096, 8192, 14336, 16384):
+                S = ops.tile_slices(M, R, K)
+                if S:
+                    taken += 1
+                    assert 256 < M <= 2048 and R % 128 == 0 and K % (128 * S) == 0
+                    assert S > 1 and -(-M // 256) * (R // 128) * S <= 256
+    assert taken and ops.tile_slices(999, 2048, 8192) == 4 and not ops.tile_slices(999, 2048, 2048)
+
+
+def test_tile_width():
+    """Narrow where one round of it does, or three for two wide ones; never for rows that leave no
+    whole wide tiles, which the kernel refuses."""
+    assert ops.tile_cols(512, 16384) == 128 and ops.tile_cols(999, 16384) == 256
+    assert ops.tile_cols(600, 28672) == 128 and ops.tile_cols(16384, 28672) == 256
+    assert ops.tile_cols(512, 16384 - 128) == 256

@@ -281,3 +281,41 @@ def test_tile_and_ring_edges(gen, M, N, K):
     want = x.float() @ w.float().t()
     assert ((whole[:M].float() - want).abs() <= 2 ** -8 * (want.abs() + K ** 0.5 * 0.05)).all()
     assert (whole[M] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (255, 768, 256), (257, 256, 384),
+                                   (513, 512, 1152), (300, 128, 512)])
+def test_narrow_tile(gen, M, N, K):
+    """The tile of 128 columns walks K as the wide one does: the same bits, of every epilogue and
+    from fewer K-tiles than its ring has to three rounds of it."""
+    x = _rand(M, K, gen=gen)
+    w = _rand(N, K, std=0.05, gen=gen)
+    ss = torch.rand(M, 3, device=DEV, generator=gen) * K
+    if N % 256 == 0:
+        for kw in (dict(epi=0), dict(epi=0, ss_in=ss, inv_d=1.0 / K, eps=1e-5), dict(epi=1),
+                   dict(epi=1, ss_in=ss, inv_d=1.0 / K, eps=1e-5), dict(epi=1, gelu=True),
+                   dict(epi=1, bias=torch.randn(N, device=DEV, generator=gen))):
+            assert torch.equal(ops.pgemm(x=x, w=w, cols=128, **kw),
+                               ops.pgemm(x=x, w=w, cols=256, **kw))
+    want = x.double() @ w.double().t()
+    for S in (1, 2, 3):
+        if K % (128 * S):
+            continue
+        half = ops.pgemm_splitk(x, w, S, cols=128)
+        if N % 256 == 0:
+            assert torch.equal(half, ops.pgemm_splitk(x, w, S, cols=256))
+        for cols in (128, 256) if N % 256 == 0 else (128,):
+            parts = torch.empty(S, M, N, device=DEV)
+            ops.pgemm_splitk(x, w, S, parts, cols=cols)
+            # fp32 sums of K exact products: K roundings of at most 2^-24 of the sum of magnitudes
+            bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+            assert ((parts.double().sum(0) - want).abs() <= bound).all()
+            assert torch.equal(parts.half(), half)
+
+
+def test_narrow_tile_refuses(gen):
+    x, w = _rand(4, 128, gen=gen), _rand(192, 128, gen=gen)
+    for call in (lambda: ops.pgemm(0, x, w, cols=128), lambda: ops.pgemm(0, x, w[:128], cols=64),
+                 lambda: ops.pgemm(0, x, w[:128]), lambda: ops.pgemm_splitk(x, w, 1, cols=128)):
+        with pytest.raises(RuntimeError):
+            call()
