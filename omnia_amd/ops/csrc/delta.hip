@@ -116,9 +116,11 @@ __global__ __launch_bounds__(256) void prep_kernel(
 }
 
 // Fast path (taps <= 4, head sizes up to 64 * VEC * NE, even when VEC = 2): a wave takes
-// a run of TR consecutive rows of one unit.  The raw inputs of the run are loaded up
-// front, the convolution slides over them in registers, and a sequence that starts
-// inside the run (or the run's own start) reloads the taps - 1 inputs before it.
+// a run of TR consecutive rows of one unit: 8, which reads 11 rows for 8, or of few rows 4, since
+// their time is the chain of a run (us in runs of 16 / 8 / 4, 16 heads of 128: 100 rows 15.1 / 9.3 /
+// 6.6, 999 17.8 / 12.9 / 12.3, 2000 21.5 / 19.0 / 22.4, 16384 141 / 134 / 165).  The raw inputs of
+// the run are loaded up front, the convolution slides over them in registers, and a sequence that
+// starts inside the run (or the run's own start) reloads the taps - 1 inputs before it.
 template <typename T, int VEC>
 struct Vec;
 template <>
@@ -920,10 +922,11 @@ int prep(float* qn, float* kn, void* vc, float* decay, float* beta, const void* 
         a_log, dt_bias, r, T_, KH, H, D, Dp, V);                                                \
     return (int)hipGetLastError();                                                              \
   } while (0)
-#define OMNIA_PREP_R(VEC, NE, TAPS)                 \
-  do {                                              \
-    if (r.q_start) OMNIA_PREP(VEC, NE, TAPS, 16 / NE);    \
-    else OMNIA_PREP(VEC, NE, TAPS, 1);              \
+#define OMNIA_PREP_R(VEC, NE, TAPS)                           \
+  do {                                                        \
+    if (r.q_start && T_ > 1200) OMNIA_PREP(VEC, NE, TAPS, 8); \
+    else if (r.q_start) OMNIA_PREP(VEC, NE, TAPS, 4);         \
+    else OMNIA_PREP(VEC, NE, TAPS, 1);                        \
   } while (0)
 #define OMNIA_PREP_T(VEC, NE)                  \
   do {                                         \

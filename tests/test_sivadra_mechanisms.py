@@ -16,6 +16,7 @@ from omnia_amd.models.layers import (LatentAttentionSpec, RotarySpec, YarnSpec, 
                                      _delta, _latent_attention)
 from omnia_amd.models.llama import ForwardBatch  # noqa: E402
 from omnia_amd.models.mixers import GatedDelta, LatentAttention, rotary_table  # noqa: E402
+from omnia_amd import ops  # noqa: E402
 from omnia_amd.ops import mixers as mops  # noqa: E402
 
 GPU = pytest.mark.gpu
@@ -251,6 +252,37 @@ def test_delta_rule(spec, how, run):
         # the recurrence amplifies the bf16 rounding of its inputs
         assert rel(project_out(y, w), want(h)) < (LIMIT[run[1]] if run[1] == torch.float32
                                                   else 0.04)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,vdim", [(64, 32), (128, 128), (160, 96)])
+def test_delta_prep_runs(dim, vdim):
+    """Many rows go in runs of 8, few in runs of 4: the same bits, wherever sequences start."""
+    lens = [1, 7, 8, 9, 3, 4, 5, 600, 331, 240, 2]
+    KH, H, taps, T = 2, 4, 4, sum(lens)
+    assert T > 1200
+    C, dev, g = 2 * KH * dim + H * vdim, "cuda", gen(5)
+    x = rnd(T, C + H * vdim + 2 * H, g=g).to(dev, torch.bfloat16)
+    cw, conv = (rnd(*n, g=g).to(dev, torch.bfloat16) for n in ((C, taps), (len(lens), taps - 1, C)))
+    al, db = rnd(H, g=g).to(dev).float(), rnd(H, g=g).to(dev).float()
+
+    def prep(some):
+        a, n = sum(lens[:some[0]]), [lens[i] for i in some]
+        t = sum(n)
+        out = (torch.empty(t, KH, dim, device=dev), torch.empty(t, KH, dim, device=dev),
+               torch.empty(t, H * vdim, dtype=torch.bfloat16, device=dev),
+               torch.empty(t, H, device=dev), torch.empty(t, H, device=dev))
+        pos = torch.cat([torch.arange(i % 2, i % 2 + lens[i]) for i in some]).int().to(dev)
+        start = torch.tensor([sum(n[:i]) for i in range(len(n) + 1)], dtype=torch.int32)
+        ops.kernels().delta_prep(*out, x[a:a + t], cw, conv, al, db, start.to(dev), pos,
+                                 torch.tensor(some, dtype=torch.int32, device=dev), KH, H, dim, dim,
+                                 vdim, taps)
+        return out
+
+    whole = prep(list(range(len(lens))))
+    parts = [prep(list(range(8))), prep([8, 9, 10])]
+    for w, p in zip(whole, zip(*parts)):
+        assert torch.equal(w, torch.cat(p))
 
 
 @pytest.mark.parametrize("run", RUNS)
