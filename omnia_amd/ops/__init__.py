@@ -1075,6 +1075,16 @@ def moe_tile_rows(experts: int, d: int) -> int:
     return 128 if experts * (d // 256) >= 128 else 224
 
 
+def down_tile_cols(n: int, n_experts: int, experts: int, d: int) -> int:
+    """Columns of the down product's tile for ``n`` assignments to ``n_experts`` experts, of which
+    ``experts`` are here: 128 where the narrow tiles of the segments to be expected, half of an
+    expert's last one empty, are one round of 256 CUs (us wide / narrow and narrow tiles, 8 experts
+    of 2048 x 4096: 600 tokens of two 84 / 61 (128), 1600 85 / 63 (256), 2001 88 / 112 (272); 8 of
+    4096 x 14336: 600 313 / 261 (256), 1001 319 / 432 (320))."""
+    segments = n * experts / n_experts / 256 + experts / 2
+    return 128 if d % 256 == 0 and segments * (d // 128) <= 256 else 256
+
+
 def moe_stream_ok(n: int, experts: int, w_up: torch.Tensor, w_down: torch.Tensor,
                   packed: bool) -> bool:
     """Whether ``n`` assignments to ``experts`` experts (all of them, where a shard holds some) run
@@ -1152,6 +1162,12 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
     act = torch.empty(mb * bm, w_down.shape[2], dtype=x.dtype, device=x.device)
     Y = torch.empty(n, x.shape[1], dtype=x.dtype, device=x.device)
     gemm = kk.pgemm_moe if bm == 256 else kk.moe_gemm
+    if bm == 256 and down_tile_cols(n, n_experts, experts, w_down.shape[1]) == 128:
+
+        def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
+            kk.pgemm_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha, limit,
+                         128 if mode == 1 else 256)
+
     if few:
         # experts whose weights are read, of a shard's as many as of the rest
         live = max(1, min(n, n_experts) * experts // n_experts)

@@ -30,7 +30,7 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
-                    float limit, hipStream_t s);
+                    float limit, int cols, hipStream_t s);
 int omnia_rmsnorm(void* out, const void* x, void* residual, const void* w, int rows, int d,
                   int64_t x_stride, int64_t out_stride, float eps, hipStream_t s);
 int omnia_rope_kv(void* q, void* k, const void* v, const int* positions, const float* cos_sin,
@@ -675,7 +675,8 @@ void moe_align(at::Tensor sorted, at::Tensor blk_expert, at::Tensor n_blocks, at
 // the 256x256-tile grouped MoE GEMMs (pgemm.hip EPI 5 / 6) over 256-row segments
 void pgemm_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Tensor sorted,
                at::Tensor blk_expert, at::Tensor n_blocks, c10::optional<at::Tensor> route_w,
-               int64_t topk, int64_t n_assign, int64_t e_lo, double alpha, double limit) {
+               int64_t topk, int64_t n_assign, int64_t e_lo, double alpha, double limit,
+               int64_t cols) {
   CHECK_GPU(A); CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(out);
   CHECK_I32(sorted); CHECK_I32(blk_expert); CHECK_I32(n_blocks);
   if (route_w.has_value())
@@ -701,7 +702,7 @@ void pgemm_moe(int64_t mode, at::Tensor out, at::Tensor A, at::Tensor W, at::Ten
   CHECK_RC(omnia_pgemm_moe((int)mode, out.data_ptr(), A.data_ptr(), W.data_ptr(),
                            sorted.data_ptr<int>(), blk_expert.data_ptr<int>(),
                            n_blocks.data_ptr<int>(), opt_ptr<float>(route_w), K, N, topk,
-                           n_assign, e_lo, mb, (float)alpha, (float)limit, cur_stream()),
+                           n_assign, e_lo, mb, (float)alpha, (float)limit, (int)cols, cur_stream()),
            "pgemm_moe");
 }
 
@@ -2158,7 +2159,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("pgemm_moe", &pgemm_moe, py::arg("mode"), py::arg("out"), py::arg("A"), py::arg("W"),
         py::arg("sorted"), py::arg("blk_expert"), py::arg("n_blocks"), py::arg("route_w"),
         py::arg("topk"), py::arg("n_assign"), py::arg("e_lo"), py::arg("alpha") = 0.0,
-        py::arg("limit") = 0.0);
+        py::arg("limit") = 0.0, py::arg("cols") = 0);
   m.def("moe_route", &moe_route, py::arg("ids"), py::arg("wts"), py::arg("x"), py::arg("router"),
         py::arg("k"), py::arg("sigmoid"), py::arg("renorm"), py::arg("corr") = py::none(),
         py::arg("groups") = 1, py::arg("keep") = 1, py::arg("bias") = py::none());

@@ -70,8 +70,9 @@ typedef float float2v __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 64;
 constexpr int HALF = 128 * BK;  // bf16 elements of a half-tile (16 KB)
-// NF: 16-column fragments of a wave; a block's tile is 256 rows x 32 NF columns
-constexpr int ring(int nf) { return (nf == 8 ? 10 : 9) * HALF; }
+// A block's tile: 256 x 256, narrow 256 x 128, flat 128 x 256 (four waves side by side)
+enum Shape { WIDE, NARROW, FLAT };
+constexpr int ring(int shape) { return (shape == WIDE ? 10 : 9) * HALF; }
 
 struct PArgs {
   void* out;            // EPI 0/1: bf16 [M, ldo]; EPI 2: residual bf16 [M, ldo]; EPI 3: q [M, ldo]
@@ -191,38 +192,27 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-template <int EPI, int NF = 8>
-__global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
-  constexpr int RING = ring(NF), KT = 2 + NF / 4;  // half-tiles of a K-tile
-  __shared__ __attribute__((aligned(1024))) bf16_t lds[RING];
-  constexpr int TN = gated(EPI) ? 16 * NF : 32 * NF;  // output columns per block tile
-  constexpr bool MOE = grouped(EPI), GATHER = gathered(EPI);
-  // sliced: the K-slices are extra "m-tiles" of the L2 grouping below (blocks of
-  // one slice share its x slice, blocks of one column tile its W rows)
-  const int S = sliced(EPI) ? p.splits : 1;
-  // MoE: the grid is sized for the worst-case segment count (graph-safe, no host sync); the
-  // live tiles are spread over the XCDs, the other blocks leave
-  const int ntn = p.N / TN, mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8, mtn = mtn1 * S;
-  const int tiles = MOE ? mtn * ntn : gridDim.x;
-  if (MOE && blockIdx.x >= tiles) return;
-  const int bid = xcd_remap(blockIdx.x, tiles);
-  const int gm = (int64_t)ntn * NF * p.K > (1 << 21) ? 8 : 4;  // 128 MB of W (32 NF rows a tile)
-  const int per_group = gm * ntn;
-  const int grp = bid / per_group, gm0 = grp * gm;
-  const int gsz = mtn - gm0 < gm ? mtn - gm0 : gm;
-  const int idx = bid - grp * per_group;
-  const int vmt = gm0 + idx % gsz, nt = idx / gsz;
-  const int ks = vmt / mtn1, mt = vmt - ks * mtn1;
+// Tile (mt, nt) of K-slice ks
+template <int EPI, int SHAPE>
+__device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, int mt, int nt,
+                                     int ks) {
+  constexpr int NF = SHAPE == WIDE ? 8 : 4;  // 16-column fragments of a wave
+  constexpr int KT = SHAPE == WIDE ? 4 : 3;  // half-tiles of a K-tile: NA of x, then NB of W
+  constexpr int NA = SHAPE == FLAT ? 1 : 2, NB = KT - NA, RING = ring(SHAPE);
+  constexpr int TN = gated(EPI) ? 64 * NB : 128 * NB;  // output columns per block tile
+  constexpr bool GATHER = gathered(EPI);
+  const int S = sliced(EPI) ? p.splits : 1, ntn = p.N / TN;
+  // (flat: grouped only, the first rows of a segment of 256)
   const int m0 = mt << 8, Mt = p.M - m0 < 256 ? p.M - m0 : 256;
   const int K = p.K, nk = K / S / BK;
   const int64_t kbase = (int64_t)ks * (K / S);
   const bf16_t* Wb = p.W + kbase;
-  if constexpr (MOE)
+  if constexpr (grouped(EPI))
     Wb += (int64_t)(p.blk_expert[mt] - p.e_lo) * (gated(EPI) ? 2 * p.N : p.N) * K;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = w >> 1, wc = w & 1;
+  const int wr = SHAPE == FLAT ? 0 : w >> 1, wc = SHAPE == FLAT ? w : w & 1;
   const int fr = lane & 15, fq = lane >> 4;
 
   // ---- DMA sources: instruction i of wave w fills half-tile rows 32w + 8i + lane/8, LDS chunk
@@ -233,7 +223,7 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     base[h] = (const char*)(p.X + (int64_t)m0 * K + kbase);
-    if constexpr (NF == 8)
+    if constexpr (SHAPE != NARROW)
       base[2 + h] = (const char*)(Wb + ((gated(EPI) ? (int64_t)h * p.N + (int64_t)nt * 128
                                                     : (int64_t)nt * 256 + h * 128)) * K);
     else  // one half-tile: gated, 64 rows of the gate's half and (waves 2, 3) 64 of the up's
@@ -244,6 +234,7 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
       const int r = 32 * w + 8 * i + (lane >> 3);
       const uint32_t ch = ((lane & 7) ^ (r & 7)) << 4;
       vo[2 + h][i] = (uint32_t)r * (uint32_t)K * 2u + ch;
+      if (h == 1 && NA == 1) continue;
       int ar = h * 128 + r;
       if constexpr (GATHER) {  // the assignment's token row (padding: row 0)
         const int f = p.sorted[m0 + ar];
@@ -255,13 +246,13 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
     }
   }
 
-  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10, or (3t + h) mod 9
+  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10 (narrow, flat: (3t + h) mod 9)
   const uint32_t dst0 =
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)lds + 32 * w * 128;
   auto next = [&](int s) __attribute__((always_inline)) {  // a K-tile on
     return s + KT * HALF >= RING ? s + KT * HALF - RING : s + KT * HALF;
   };
-  int da = 0, db = 2 * HALF, ka = 0, kb = 0;  // slots and K-tiles to ask for next
+  int da = 0, db = NA * HALF, ka = 0, kb = 0;  // slots and K-tiles to ask for next
   uint32_t qa = 0, qb = 0;                    // of the DMAs under way: LDS address, sources
   const char *pa[2], *pb[2];
   int64_t koff = 0;
@@ -270,14 +261,14 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
     qa = dst0 + da * 2;
     koff = (int64_t)ka * (BK * 2);
     pa[0] = base[0] + koff;
-    pa[1] = base[1] + koff;
+    if constexpr (NA == 2) pa[1] = base[1] + koff;
     ka = ka + 1 < nk ? ka + 1 : nk - 1;
     da = next(da);
   };
   auto set_b = [&]() __attribute__((always_inline)) {
     qb = dst0 + db * 2;
     pb[0] = base[2] + (int64_t)kb * (BK * 2);
-    if constexpr (NF == 8) pb[1] = base[3] + (int64_t)kb * (BK * 2);
+    if constexpr (NB == 2) pb[1] = base[3] + (int64_t)kb * (BK * 2);
     kb = kb + 1 < nk ? kb + 1 : nk - 1;
     db = next(db);
   };
@@ -289,32 +280,31 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   auto dma_b = [&](int d) __attribute__((always_inline)) {
     dma16(vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb, (d >> 2) * HALF * 2 + (d & 3) * 1024);
   };
-  // K-tiles 0 and 1, and A of 2 (NF 4: all of it)
+  // K-tiles 0 and 1, and A of 2 (narrow, flat: all of it)
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
     set_a();
 #pragma unroll
-    for (int d = 0; d < 8; ++d) dma_a(d);
-    if (t < 2 || NF == 4) {
+    for (int d = 0; d < 4 * NA; ++d) dma_a(d);
+    if (t < 2 || SHAPE != WIDE) {
       set_b();
 #pragma unroll
-      for (int d = 0; d < NF; ++d) dma_b(d);
+      for (int d = 0; d < 4 * NB; ++d) dma_b(d);
     }
   }
 
-  // ---- fragments: A rows wr*128 + 16m + fr; B rows of half wc, or (gated) rows wc*64 + 16n + fr
-  // of the gate's half for n < 4 and of the up's for n >= 4 (NF 4: the same in quarters); k chunk
-  // 4s + fq of step s
-  constexpr int NG = NF / 2;  // gate fragments of a wave
+  // ---- fragments: A rows wr*128 + 16m + fr; B's columns wc*WCOL + 16n + fr, gated those of the
+  // gate's part for n < NG and of the up's, GU columns on, for the rest; k chunk 4s + fq of step s
+  constexpr int NG = NF / 2, GU = 64 * NB;
   constexpr int WCOL = (gated(EPI) ? NG : NF) * 16;
   const bf16_t *fa[2], *fb[2];
-  int ra = wr * HALF, rb = gated(EPI) || NF == 4 ? 2 * HALF : (2 + wc) * HALF;
+  int ra = wr * HALF, rb = NA * HALF;
   auto set_r = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int at = fr * BK + (((4 * s + fq) ^ (fr & 7)) << 3);
       fa[s] = lds + ra + at;
-      fb[s] = lds + rb + at + (gated(EPI) || NF == 4 ? wc * WCOL * BK : 0);
+      fb[s] = lds + rb + wc * WCOL * BK + at;
     }
     ra = next(ra);
     rb = next(rb);
@@ -327,7 +317,7 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
       fx[set][m] = *reinterpret_cast<const short8*>(fa[s] + m * 16 * BK);
     } else {
       const int n = j - 1;
-      const int at = gated(EPI) ? n / NG * NG * 32 * BK + n % NG * 16 * BK : n * 16 * BK;
+      const int at = gated(EPI) ? n / NG * GU * BK + n % NG * 16 * BK : n * 16 * BK;
       fw[set][n] = *reinterpret_cast<const short8*>(fb[s] + at);
     }
   };
@@ -389,15 +379,17 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   // there, and its first fragments are read.
   constexpr int P = 8 * NF, FREE = NF == 8 ? 36 : 26, LAND = NF == 8 ? 12 : 6;
   constexpr int YOUNGER = NF == 8 ? 16 : 17;
-  // the DMA behind product j: B's are 0 to NF - 1, A's 8 to 15; -1: none
+  // the DMA behind product j: B's are 0 to 4 NB - 1, A's from 8 on; -1: none
   auto dma_at = [](int s, int j) constexpr {
     if (NF == 8) {
       if (s == 0 && j >= FREE && (j - FREE) % 3 == 0 && (j - FREE) / 3 < 8) return (j - FREE) / 3;
       if (s == 1 && j > LAND && (j - LAND) % 6 == 3 && (j - LAND) / 6 < 8)
         return 8 + (j - LAND) / 6;
     } else {
-      if (s == 0 && j >= FREE && (j - FREE) % 2 == 0) return (j - FREE) / 2;  // B 0 to 2
-      if (s == 1 && j % 3 == 1 && j < 27) return j == 1 ? 3 : 8 + j / 3 - 1;
+      int q = -1;
+      if (s == 0 && j >= FREE && (j - FREE) % 2 == 0) q = (j - FREE) / 2;  // 0 to 2
+      if (s == 1 && j % 3 == 1 && j < 27) q = 3 + j / 3;
+      return q < 4 * NB ? q : 8 + q - 4 * NB;
     }
     return -1;
   };
@@ -627,6 +619,87 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   }
 }
 
+template <int EPI, int SHAPE = WIDE>
+__global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
+  __shared__ __attribute__((aligned(1024))) bf16_t lds[ring(SHAPE)];
+  constexpr int TN = (gated(EPI) ? 128 : 256) / (SHAPE == NARROW ? 2 : 1);
+  constexpr bool MOE = grouped(EPI);
+  // sliced: the K-slices are extra "m-tiles" of the L2 grouping below (blocks of
+  // one slice share its x slice, blocks of one column tile its W rows)
+  const int S = sliced(EPI) ? p.splits : 1;
+  // MoE: the grid is sized for the worst-case segment count (graph-safe, no host sync); the
+  // live tiles are spread over the XCDs, the other blocks leave
+  constexpr int WORDS = 4;
+  const int lane = threadIdx.x & 63, most = p.M >> 8;
+  bool light = false, ordered = MOE && SHAPE == WIDE && most <= 64 * WORDS && gridDim.x <= 9 * 256;
+  int half[WORDS];  // assignment 128 of segments 64 i + lane, asked for beside their number
+  if constexpr (MOE && SHAPE == WIDE)
+    if (ordered)
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i)
+        if (64 * i < most)
+          half[i] = p.sorted[(int64_t)min(64 * i + lane, most - 1) * 256 + 128];
+  const int ntn = p.N / TN, mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8;
+  int first = 0, tiles = MOE ? mtn1 * ntn : gridDim.x, mtn = mtn1 * S;
+  if (MOE && blockIdx.x >= tiles) return;
+  // An expert's last segment may have 128 rows or fewer: light, half a tile.  All others come first,
+  // so that the last round is of light ones (us before / now, 8 experts of 2048 x 4096: up at 1600
+  // tokens of two 136 / 117, 3000 208 / 193, down at 8192 263 / 239, 16384 458 / 421).  Up to 9 rounds:
+  // finding them takes 1 us a tile (up at 16384, 16.5 rounds, 893 / 905); not where they are few and
+  // the last round is short as it is, since apart from their expert's others they read its weights
+  // once more (up at 2001, one of 17, 157 / 163, in a step 160 / 168).
+  uint64_t pick[WORDS];
+  if constexpr (MOE && SHAPE == WIDE) {
+    if (ordered) {
+      int full = 0;
+      uint64_t heavy[WORDS];
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i) {
+        heavy[i] = 64 * i < most
+                       ? __builtin_amdgcn_ballot_w64(64 * i + lane < mtn1 && half[i] < p.n_assign)
+                       : 0;
+        full += __popcll(heavy[i]);
+      }
+      ordered = p.K >= 4096 || 10 * (mtn1 - full) >= mtn1 || mtn1 * ntn >= 3 * 256;
+      light = ordered && blockIdx.x >= full * ntn;
+      first = light ? full * ntn : 0;
+      if (ordered) mtn = light ? mtn1 - full : full;
+      tiles = mtn * ntn;
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i)
+        pick[i] = light ? __builtin_amdgcn_ballot_w64(64 * i + lane < mtn1) & ~heavy[i] : heavy[i];
+    }
+  }
+  const int bid = xcd_remap(blockIdx.x - first, tiles);
+  const int64_t w_rows = gated(EPI) ? 2 * p.N : p.N;
+  const int gm = w_rows * p.K > (1 << 26) ? 8 : 4;  // 128 MB of W
+  const int per_group = gm * ntn;
+  const int grp = bid / per_group, gm0 = grp * gm;
+  const int gsz = mtn - gm0 < gm ? mtn - gm0 : gm;
+  const int idx = bid - grp * per_group;
+  const int vmt = gm0 + idx % gsz, nt = idx / gsz;
+  const int ks = vmt / mtn1;
+  int mt = vmt - ks * mtn1;
+  if constexpr (MOE && SHAPE == WIDE) {
+    if (ordered) {  // the mt-th of the picked segments
+      int before = 0, seg = 0;
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i) {
+        const int rank = before + __popcll(pick[i] & ((1ull << lane) - 1));
+        const uint64_t hit = __builtin_amdgcn_ballot_w64((pick[i] >> lane & 1) && rank == mt);
+        if (hit) seg = 64 * i + __builtin_ctzll(hit);
+        before += __popcll(pick[i]);
+      }
+      mt = seg;
+    }
+    if (light) {
+      tile<EPI, FLAT>(p, lds, mt, nt, 0);
+      return;
+    }
+  }
+  tile<EPI, SHAPE>(p, lds, mt, nt, ks);
+}
+
 // one workgroup (256 threads) per row: ss[r] = sum(x[r]^2) (layer-0 input of the
 // folded-norm prefill path: the embedding rows have no producer epilogue)
 __global__ __launch_bounds__(256) void row_sumsq_kernel(float* __restrict__ ss,
@@ -659,7 +732,7 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
-                    float limit, hipStream_t s);
+                    float limit, int cols, hipStream_t s);
 
 // 0 and 1 named two main loops; one is left
 int omnia_pgemm_set_schedule(int sched) { return sched < 0 || sched > 1 ? -1 : 0; }
@@ -704,9 +777,9 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
 #define OMNIA_PGEMM(EPI)                                       \
   do {                                                         \
     if (narrow)                                                \
-      pgemm_kernel<EPI, 4><<<grid, 256, 0, s>>>(a);            \
+      pgemm_kernel<EPI, NARROW><<<grid, 256, 0, s>>>(a);            \
     else                                                       \
-      pgemm_kernel<EPI, 8><<<grid, 256, 0, s>>>(a);            \
+      pgemm_kernel<EPI, WIDE><<<grid, 256, 0, s>>>(a);            \
     return (int)hipGetLastError();                             \
   } while (0)
   if (bias) OMNIA_PGEMM(7);
@@ -740,11 +813,11 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
           nullptr, 0, 0, 0};
   const dim3 grid((unsigned)blocks);
   if (f32 && tn == 128)
-    pgemm_kernel<11, 4><<<grid, 256, 0, s>>>(a);
+    pgemm_kernel<11, NARROW><<<grid, 256, 0, s>>>(a);
   else if (f32)
     pgemm_kernel<11><<<grid, 256, 0, s>>>(a);
   else if (tn == 128)
-    pgemm_kernel<4, 4><<<grid, 256, 0, s>>>(a);
+    pgemm_kernel<4, NARROW><<<grid, 256, 0, s>>>(a);
   else
     pgemm_kernel<4><<<grid, 256, 0, s>>>(a);
   return (int)hipGetLastError();
@@ -759,9 +832,11 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
-                    float limit, hipStream_t s) {
+                    float limit, int cols, hipStream_t s) {
   if (mode < 0 || mode > 3 || max_blocks < 0 || topk < 1) return -1;
-  const int tn = mode == 0 || mode == 2 ? 128 : 256;
+  if (cols && cols != 128 && cols != 256) return -16;
+  const bool narrow = cols == 128;
+  const int tn = (mode == 0 || mode == 2 ? 128 : 256) >> (narrow ? 1 : 0);
   if (K <= 0 || K % (2 * BK)) return -3;
   if (N <= 0 || N % tn) return -4;
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W) |
@@ -774,15 +849,20 @@ int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int
   PArgs a{out, (const bf16_t*)A, (const bf16_t*)W, max_blocks * 256, N, K, N, nullptr, 0, 0.f,
           0.f, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 1, sorted,
           blk_expert, n_blocks, route_w, topk, n_assign, e_lo, nullptr, alpha, limit};
-  if (mode == 0)
-    pgemm_kernel<5><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
-  else if (mode == 2)
-    pgemm_kernel<8><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
-  else if (mode == 3)
-    pgemm_kernel<10><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
-  else
-    pgemm_kernel<6><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
-  return (int)hipGetLastError();
+  const dim3 grid((unsigned)blocks);
+#define OMNIA_PGEMM(EPI)                            \
+  do {                                              \
+    if (narrow)                                     \
+      pgemm_kernel<EPI, NARROW><<<grid, 256, 0, s>>>(a); \
+    else                                            \
+      pgemm_kernel<EPI, WIDE><<<grid, 256, 0, s>>>(a); \
+    return (int)hipGetLastError();                  \
+  } while (0)
+  if (mode == 0) OMNIA_PGEMM(5);
+  if (mode == 1) OMNIA_PGEMM(6);
+  if (mode == 2) OMNIA_PGEMM(8);
+  OMNIA_PGEMM(10);
+#undef OMNIA_PGEMM
 }
 
 int omnia_row_sumsq(float* ss, const void* x, int rows, int d, int64_t stride, hipStream_t s) {

@@ -261,3 +261,51 @@ def test_ranks_that_share_a_device_take_blocks_of_little_lds(T, kernel, monkeypa
         m, {"router": router, "experts_gate_up": wgu, "experts_down": wd}, x).float()
     assert set(used) == {kernel}
     torch.testing.assert_close(got, want, atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("E,rows", [
+    (20, [1, 127, 128, 129, 255, 256, 257, 300, 383, 384, 385, 512, 513, 0, 2, 0, 130, 640, 3, 250]),
+    (9, [300, 300, 300, 300, 300, 300, 300, 300, 300]),  # an expert's last segment: 44 rows
+    (4, [90, 120, 7, 128]),                              # light segments alone
+    (4, [256, 512, 256, 200]),                           # none
+    (100, [40 + 3 * e for e in range(100)]),             # more than a word of segments
+    (200, [200 + e for e in range(200)])])               # more than are put in order
+def test_segments_of_few_rows(E, rows):
+    """Segments of 128 rows or fewer run as half a tile behind the others: the bits of the narrow
+    tile, which knows no such segments, in every product."""
+    kk, dev, d, I = ops.kernels(), "cuda", 256, 384
+    g = torch.Generator().manual_seed(E)
+    n = sum(rows)
+    ids = torch.arange(E).repeat_interleave(torch.tensor(rows))[torch.randperm(n, generator=g)]
+    ids = ids.int().view(n, 1).to(dev)
+    x = torch.randn(n, d, generator=g).to(torch.bfloat16).to(dev)
+    up = (torch.randn(E, 2 * I, d, generator=g) * 0.05).to(torch.bfloat16).to(dev)
+    down = (torch.randn(E, d, I, generator=g) * 0.05).to(torch.bfloat16).to(dev)
+    wts = torch.rand(n, generator=g).to(dev)
+    mb = kk.moe_max_blocks(n, E, 256)
+    order = torch.empty(mb * 256, dtype=torch.int32, device=dev)
+    blk = torch.empty(mb, dtype=torch.int32, device=dev)
+    nb = torch.empty(1, dtype=torch.int32, device=dev)
+    kk.moe_align(order, blk, nb, ids, E, 0, E)
+    live = (order < n) & (torch.arange(mb * 256, device=dev) < nb * 256)
+    for mode, w, rw in ((0, up, None), (2, up, wts), (3, up[:, :I].contiguous(), None)):
+        acts = []
+        for cols in (256, 128):
+            if w.shape[1] // (1 if mode == 3 else 2) % (cols // (1 if mode == 3 else 2)):
+                continue
+            act = torch.zeros(mb * 256, w.shape[1] // (1 if mode == 3 else 2), device=dev,
+                              dtype=torch.bfloat16)
+            kk.pgemm_moe(mode, act, x, w, order, blk, nb, rw, 1, n, 0, 1.702, 7.0, cols)
+            acts.append(act[live])
+        assert len(acts) == 1 or torch.equal(*acts)
+        if mode != 0:
+            continue
+        y = torch.empty(2, n, d, device=dev, dtype=torch.bfloat16)
+        for i, cols in enumerate((256, 128)):
+            kk.pgemm_moe(1, y[i], act, down, order, blk, nb, wts, 1, n, 0, 0.0, 0.0, cols)
+        assert torch.equal(y[0], y[1])
+        for e in set(range(E)) if E <= 20 else {0, E // 2, E - 1}:
+            of = ids.view(-1) == e
+            a, b = (x[of].float() @ up[e].float().t()).split(I, 1)
+            want = (torch.nn.functional.silu(a) * b) @ down[e].float().t() * wts[of, None]
+            torch.testing.assert_close(y[0][of].float(), want, atol=2e-2, rtol=2e-2)
