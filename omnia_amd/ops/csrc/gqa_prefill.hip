@@ -17,6 +17,7 @@
 // fp32 as it is, and neither a running maximum nor a rescaling is needed.  A tile is then
 // worked on in halves of 32 keys, its biases are a table of distances in LDS, and the
 // denominator sums the same rounded P as the output.
+#include <algorithm>
 #include <type_traits>
 
 #include "mask.h"
@@ -67,15 +68,20 @@ struct Args {
 
 // KEEP: windows hold the sequence's first p.mask.keep keys as well.  SHAPE: scores are plain
 // (0), capped or biased (1), capped and biased within bounds (2)
-template <int DK, int DV, bool KEEP, int SHAPE>
-__global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Args p) {
+// KS 2: two such groups of waves, on every other key tile each, whose maxima, sums and outputs are
+// joined through LDS in fp32: where there are few blocks, they last as long as the longest walk over
+// the keys, 1.85 us a tile with one wave a SIMD and 2.8 for two tiles with two.
+template <int DK, int DV, bool KEEP, int SHAPE, int KS>
+__global__ __launch_bounds__(256 * KS, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Args p) {
   // two K | V stages as separate objects: reads of one cannot alias the DMA into the other
-  __shared__ __attribute__((aligned(16))) char st0[128 * (DK + DV)];
-  __shared__ __attribute__((aligned(16))) char st1[128 * (DK + DV)];
+  constexpr int STAGE = 128 * (DK + DV);
+  __shared__ __attribute__((aligned(16))) char st0[STAGE * KS];
+  __shared__ __attribute__((aligned(16))) char st1[STAGE * KS];
   constexpr int kMaxPages = 1024;  // pages of the visible range staged in LDS
   __shared__ int pg_lds[kMaxPages];
   // SHAPE 2: per wave, cap - bias of the 95 distances between its rows and a tile's keys
-  __shared__ float dist_lds[SHAPE == 2 ? 4 : 1][96];
+  __shared__ float dist_lds[SHAPE == 2 ? 4 * KS : 1][96];
+  __shared__ float joined[KS == 2 ? 8 : 1][64];  // maximum and sum of the second group's lanes
 
   const int HB = 1 << p.hb_lg, group = p.H / p.G;
   // blocks of one key/value head are neighbours: (head block, tile, sub-tile)
@@ -90,7 +96,8 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
   const int b0 = p.tile_q0[tile] + sub * rows;
   if (b0 >= qlen) return;
   const int off = p.seq_lens[s] - qlen;  // position of the portion's first row
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, ql = lane & 31, hi = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, ql = lane & 31, hi = lane >> 5;
+  const int w = (tid >> 6) & 3, part = KS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
   const int h = hblk * HB + (w & (HB - 1)), kvh = hblk * HB / group;
   const int* bt = p.block_tables + (int64_t)s * p.bt_stride;
   const int BS = 1 << p.page_lg, pmask = BS - 1;
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
   const int nkp = ((tk << 6) + BS - 1) >> p.page_lg;
   const int pg0 = (t0 << 6) >> p.page_lg;
   const int npg = min(nkp + ((kv_end - 1) >> p.page_lg) - pg0 + 1, kMaxPages);
-  for (int i = tid; i < npg; i += 256) pg_lds[i] = bt[i < nkp ? i : pg0 + i - nkp];
+  for (int i = tid; i < npg; i += 256 * KS) pg_lds[i] = bt[i < nkp ? i : pg0 + i - nkp];
   __syncthreads();
 
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -142,7 +149,7 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
                                        (lds_ptr_t)(dst + (w * N + i) * 1024), 16, 0, 0);
   };
   auto dma = [&](int t, auto BUF) {
-    char* st = decltype(BUF)::value ? st1 : st0;
+    char* st = (decltype(BUF)::value ? st1 : st0) + part * STAGE;
     dma1(t, std::integral_constant<int, DK>{}, p.kc, st);
     dma1(t, std::integral_constant<int, DV>{}, p.vc, st + 128 * DK);
   };
@@ -151,8 +158,8 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
   const float r2 = SHAPE && p.score.r1 ? p.score.r2[h] : 0.f;
   const float to2 = SHAPE ? 1.f : p.score.mul;  // the tile's scores to base 2
   const float sink = p.sinks ? p.sinks[h] * 1.4426950408889634f : -1e30f;
-  float m_run = sink;
-  float l_run = p.sinks && SHAPE != 2 ? 1.f : 0.f;
+  float m_run = part ? -1e30f : sink;  // the sink is the first group's
+  float l_run = p.sinks && SHAPE != 2 && !part ? 1.f : 0.f;
   float16v o[DV / 32];
 #pragma unroll
   for (int d = 0; d < DV / 32; ++d)
@@ -164,13 +171,13 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
-  dma(tile_of(0), B0{});
+  if (part < nt) dma(tile_of(part), B0{});
   __syncthreads();
   auto body = [&](int j, auto BUF) {
     constexpr int buf = decltype(BUF)::value;
     const int t = tile_of(j);
-    if (j + 1 < nt) dma(tile_of(j + 1), std::integral_constant<int, 1 - buf>{});
-    const char* Kl = buf ? st1 : st0;
+    if (j + KS < nt) dma(tile_of(j + KS), std::integral_constant<int, 1 - buf>{});
+    const char* Kl = (buf ? st1 : st0) + part * STAGE;
     const char* Vl = Kl + 128 * DK;
     const int k0 = t * 64;
     // S^T of 32 keys
@@ -200,10 +207,10 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
       }
     };
     // wave-uniform: some row sees some key
-    const bool seen = k0 <= wmax && (k0 + 63 >= lo_min || (KEEP && k0 < keep));
+    const bool seen = (KS == 1 || j < nt) && k0 <= wmax && (k0 + 63 >= lo_min || (KEEP && k0 < keep));
     if (SHAPE == 2 && seen) {
       // entry t: distance (first row + 31) - (first key) - t; keys ahead of a row are masked
-      float* dist = dist_lds[w];
+      float* dist = dist_lds[4 * part + w];
       const int far = off + q0 + 31 - k0;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -328,12 +335,36 @@ __global__ __launch_bounds__(256, DK + DV <= 256 ? 2 : 1) void prefill_kernel(Ar
     }
     __syncthreads();  // the next tile landed and this one is read by all waves
   };
-  for (int j = 0; j < nt; j += 2) {
-    body(j, B0{});
-    if (j + 1 < nt) body(j + 1, B1{});
+  for (int j = 0; j < nt; j += 2 * KS) {
+    body(j + part, B0{});
+    if (j + KS < nt) body(j + KS + part, B1{});
   }
   if constexpr (SHAPE == 2)
-    l_run += __shfl_xor(l_run, 32, 64) + (p.sinks ? __builtin_amdgcn_exp2f(sink) : 0.f);
+    l_run += __shfl_xor(l_run, 32, 64) + (p.sinks && !part ? __builtin_amdgcn_exp2f(sink) : 0.f);
+  if constexpr (KS == 2) {
+    static_assert(DV <= DK, "the second group's sums fill a stage");
+    float4v* sums = reinterpret_cast<float4v*>(st0) + (int64_t)w * (DV / 8) * 64 + lane;
+    if (part) {
+#pragma unroll
+      for (int i = 0; i < DV / 8; ++i)
+        sums[64 * i] = float4v{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1],
+                               o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+      joined[w][lane] = m_run;
+      joined[4 + w][lane] = l_run;
+    }
+    __syncthreads();
+    if (part) return;
+    const float m = SHAPE == 2 ? m_run : joined[w][lane], top = fmaxf(m_run, m);
+    const float mine = __builtin_amdgcn_exp2f(m_run - top), other = __builtin_amdgcn_exp2f(m - top);
+    l_run = l_run * mine + joined[4 + w][lane] * other;
+#pragma unroll
+    for (int i = 0; i < DV / 8; ++i) {
+      const float4v v = sums[64 * i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[i >> 2][4 * (i & 3) + r] = o[i >> 2][4 * (i & 3) + r] * mine + v[r] * other;
+    }
+  }
   if (row_ok) {
     const float inv = (p.gate ? p.gate[(int64_t)(qs + qr) * p.H + h] : 1.f) / l_run;
     bf16_t* orow = p.out + ((int64_t)(qs + qr) * p.H + h) * DV;
@@ -371,25 +402,38 @@ int omnia_gqa_prefill(void* out, const void* q, const void* kc, const void* vc,
          q_start, seq_lens, tile_seq, tile_q0, sinks, gate, bt_stride, n_tiles, H, G, hb_lg,
          page_lg, mask, Score2(score)};
   const bool keep = mask.window > 0 && mask.chunk == 0 && mask.keep > 0;
-#define OMNIA_GQ(K, V)                                                  \
-  if (Dp == K && Vp == V) {                                             \
-    if (!score.plain() && keep)                                         \
-      prefill_kernel<K, V, true, 1><<<n_tiles * H, 256, 0, s>>>(a);     \
-    else if (bounded)                                                   \
-      prefill_kernel<K, V, false, 2><<<n_tiles * H, 256, 0, s>>>(a);    \
-    else if (!score.plain())                                            \
-      prefill_kernel<K, V, false, 1><<<n_tiles * H, 256, 0, s>>>(a);    \
-    else if (keep)                                                      \
-      prefill_kernel<K, V, true, 0><<<n_tiles * H, 256, 0, s>>>(a);     \
-    else                                                                \
-      prefill_kernel<K, V, false, 0><<<n_tiles * H, 256, 0, s>>>(a);    \
-    return (int)hipGetLastError();                                      \
+  // two groups of waves where few blocks wait for the longest walk: one a CU, from 5 tiles of keys,
+  // or two a CU, from 32 (us with one / two, 16 heads of 128: 77 rows 8.1 / 9.4, behind 1900 keys 59 /
+  // 43, 300 14.6 / 13.4, 1001 33.9 / 26.3, 2001 60.7 / 45.4, window 1024 36.8 / 29.5; 384 to 512
+  // blocks: 3000 rows 93 / 64, window 1024 46 / 54, 8 x 333 22 / 27, 2 x 2048 85 / 58; 2048 blocks
+  // 208 / 218)
+  const int keys = mask.most((int)std::min<int64_t>((int64_t)bt_stride << page_lg, 1 << 30));
+  const int64_t blocks = (int64_t)n_tiles * H;
+  const bool twice = blocks <= 256 ? keys >= 320 : blocks <= 512 && keys >= 2048;
+#define OMNIA_GQS(K, V, KEEP, SHAPE)                                                      \
+  do {                                                                                    \
+    if constexpr (K == V && K <= 128)                                                     \
+      if (twice) {                                                                        \
+        prefill_kernel<K, V, KEEP, SHAPE, 2><<<n_tiles * H, 512, 0, s>>>(a);              \
+        return (int)hipGetLastError();                                                    \
+      }                                                                                   \
+    prefill_kernel<K, V, KEEP, SHAPE, 1><<<n_tiles * H, 256, 0, s>>>(a);                  \
+    return (int)hipGetLastError();                                                        \
+  } while (0)
+#define OMNIA_GQ(K, V)                                      \
+  if (Dp == K && Vp == V) {                                 \
+    if (!score.plain() && keep) OMNIA_GQS(K, V, true, 1);   \
+    if (bounded) OMNIA_GQS(K, V, false, 2);                 \
+    if (!score.plain()) OMNIA_GQS(K, V, false, 1);          \
+    if (keep) OMNIA_GQS(K, V, true, 0);                     \
+    OMNIA_GQS(K, V, false, 0);                              \
   }
 #define OMNIA_GQV(K) \
   OMNIA_GQ(K, 32) OMNIA_GQ(K, 64) OMNIA_GQ(K, 96) OMNIA_GQ(K, 128) OMNIA_GQ(K, 192) OMNIA_GQ(K, 256)
   OMNIA_GQV(32) OMNIA_GQV(64) OMNIA_GQV(96) OMNIA_GQV(128) OMNIA_GQV(192) OMNIA_GQV(256)
 #undef OMNIA_GQV
 #undef OMNIA_GQ
+#undef OMNIA_GQS
   return -3;
 }
 

@@ -408,6 +408,55 @@ def test_long_contexts(page):
             assert rel(d[i], want[i][-1]) < 0.012
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,G", [(128, 2), (64, 4), (32, 1)])
+@pytest.mark.parametrize("kind", ["full", "window", "keep", "chunk", "cap", "bounded", "keep cap"])
+def test_prefill_by_two_groups_of_waves(kind, D, G):
+    """Blocks whose keys two groups share (tables of many pages) against those of one (few), and
+    both against exact sums: from one tile of keys to uneven numbers of them, sequences with a past
+    among them."""
+    H, page, g = 4, 16, gen(15)
+    lens, nq = [1, 64, 65, 128, 129, 193, 290, 300, 250], [1, 64, 65, 128, 129, 193, 290, 5, 200]
+    window = 0 if kind in ("full", "chunk", "cap", "bounded") else 70
+    capped = "cap" in kind or kind == "bounded"
+    spec = AttentionSpec(H, G, D, D, 0.2, RotarySpec(8, 1e4), window,
+                         sink="" if kind == "bounded" else "learned",
+                         keep_first=33 if "keep" in kind else 0, chunk=96 if kind == "chunk" else 0,
+                         softcap=20.0 if capped else 0.0)
+    dist = torch.rand(2, H, generator=g) * 0.3 if capped else None
+    sinks = None if kind == "bounded" else torch.randn(H, generator=g)
+    gate = torch.rand(sum(nq), H, generator=g)
+    pages = [torch.randn(180, G, page, D, generator=g).to(torch.bfloat16) for _ in range(2)]
+    free = iter((1 + torch.randperm(179, generator=g)).tolist())
+    width = 19
+    bt = torch.tensor([[next(free) if i < -(-n // page) else 0 for i in range(width)]
+                       for n in lens], dtype=torch.int32)
+    q = torch.randn(sum(nq), H * D, generator=g).to(torch.bfloat16)
+    start = torch.tensor([0] + nq).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(n - m, n) for n, m in zip(lens, nq)]).to(torch.int32)
+    ts, t0 = prefill_tiles(nq, 128)
+    want = mops.gqa_attend(q.float(), [p.float() for p in pages], bt, start, pos, spec, sinks,
+                           dist=dist, gate=gate)
+
+    def cuda(t):
+        return None if t is None else t.cuda()
+
+    def ints(v):
+        return torch.tensor(v, dtype=torch.int32, device="cuda")
+
+    got = []
+    for w in (width, 40):  # 304 keys of a table at most, or 640
+        fb = ForwardBatch(None, cuda(pos), None, cuda(torch.nn.functional.pad(bt, (0, w - width))),
+                          ints(lens), None, is_decode=False, q_start_loc=cuda(start),
+                          tile_seq=ints(ts), tile_q0=ints(t0))
+        got.append(mops.gqa_prefill(cuda(q), [cuda(p) for p in pages], fb, spec, cuda(sinks),
+                                    dist=cuda(dist), gate=cuda(gate), bounded=kind == "bounded"))
+    for o in got:
+        assert torch.isfinite(o).all() and rel(o.double().cpu(), want.double()) < 0.006
+    # the same sums but for the roundings of P, 2^-9 each, and of the result
+    assert rel(got[1].double(), got[0].double()) < 0.004
+
+
 # ---------------------------------------------------------------- experts
 def expert_weights(E, d, ff, g, scale=1.0):
     W = {"router": rnd(E, d, g=g, scale=d ** -0.5)}
