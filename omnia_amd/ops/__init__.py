@@ -910,16 +910,21 @@ def prefill_tiles(q_lens: list[int], tile: int | None = None) -> tuple[list[int]
 def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int) -> int:
     """Most key partitions of a 32-row query tile, for up to 512 blocks, two a CU (fewer where the
     live length gives a partition less than 128 keys).  A block walks its 64-key tiles one after
-    the other, 1.35 us each; partitions shorten that walk but write and read fp32 partials, at
-    about 3 TB/s, and cost a launch (us at 1 / 2 / 4 / 8 partitions, 32 heads on 8: 77 rows on
-    4000 keys 89 / 53 / 34 / 28, on 1100 29 / 23 / 20 / 21, on 400 16.0 / 16.2 / 15.8 / 15.9;
-    512 on 3000 69 / 53 / 49 / 58, on 512 18 / 22 / 25 / 25)."""
+    the other, 1.35 us each, or, with two groups of waves where blocks are one a CU, 0.975;
+    partitions shorten that walk but write and read fp32 partials, at about 3 TB/s, and cost a
+    launch (us at 1 / 2 / 4 / 8 partitions, 32 heads on 8: 77 rows on 4000 keys 64 / 43 / 30 / 27, on
+    1100 26 / 22 / 20 / 21, on 400 16 / 17 / 17 / 17; 200 on 2200 40 / 33 / 29 / 33; 512 on 3500 59 /
+    53 / 56 / 64, on 512 15.9 / 22 / 25 / 25; 1001 on 4000 77 / 96)."""
     group = hq // hkv
     blocks = tiles * hq // (4 if group % 4 == 0 else 2 if group % 2 == 0 else 1)
-    walk = -(-max_keys // 64) * 1.35
-    best, cost = 1, walk
+
+    def walk(P):
+        t = -(-max_keys // 64) / P
+        return min(1.35 * t, 0.975 * t + 1.5) if blocks * P <= 256 else 1.35 * t
+
+    best, cost = 1, walk(1)
     for P in range(2, min(16, 512 // max(blocks, 1), max_keys // 128) + 1):
-        c = walk / P + 5.0 + P * tiles * 32 * hq * 1024 / 3e6
+        c = walk(P) + 5.0 + P * tiles * 32 * hq * 1024 / 3e6
         if c < cost:
             best, cost = P, c
     return best

@@ -600,8 +600,10 @@ __device__ __forceinline__ int prefill_parts(int ntiles, int S) {
 // tile of one partition writes its result.  The walk over the keys is a serial chain of 1.35 us a
 // 64-key tile, which few query tiles leave most of the chip to wait for (3 tiles of 8 blocks on
 // 4000 keys: 89 us, 29 in 8 partitions; ops.prefill_parts).
-template <int BS, int HB, bool SPLIT>
-__global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kernel(
+// KS 2: two groups of HB waves, on every other key tile each, joined through LDS in fp32: two tiles
+// in 1.95 us.
+template <int BS, int HB, bool SPLIT, int KS>
+__global__ __launch_bounds__(64 * HB * KS, HB == 4 ? 2 : 1) void prefill_attn32_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
     const bf16_t* __restrict__ vc, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ q_start_loc, const int* __restrict__ seq_lens,
@@ -612,17 +614,20 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   // two K | V stages (separate objects, so the compiler sees that fragment reads
   // of one stage cannot alias the other stage's in-flight LDS-DMA): the next
   // tile is written while this one is still read, one barrier per tile
-  __shared__ __attribute__((aligned(16))) char st0[2 * 64 * 256];
-  __shared__ __attribute__((aligned(16))) char st1[2 * 64 * 256];
+  constexpr int STAGE = 2 * 64 * 256;
+  __shared__ __attribute__((aligned(16))) char st0[STAGE * KS];
+  __shared__ __attribute__((aligned(16))) char st1[STAGE * KS];
   // the sequence's page indices for the first kMaxPages pages, staged once: a K/V
   // prefetch is then ONE global load deep instead of a page-table load followed
   // by the data load it feeds
   constexpr int kMaxPages = 1024;
   __shared__ int pg_lds[kMaxPages];
+  __shared__ float joined[KS == 2 ? 2 * HB : 1][64];  // maximum and sum of the second group's lanes
 
   const int hq = gridDim.x * HB;
   const int G = hq / hkv;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & (HB - 1);
+  const int group = KS == 2 ? __builtin_amdgcn_readfirstlane(tid / (64 * HB)) : 0;
   const int h = blockIdx.x * HB + w;
   const int kvh = blockIdx.x * HB / G;
   // a sequence's last tiles, which see most keys, first: what is left for the end is short
@@ -660,7 +665,7 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   }
 
   const int npg = min((kv_end + BS - 1) / BS, kMaxPages);
-  for (int i = tid; i < npg; i += 64 * HB) pg_lds[i] = bt[i];
+  for (int i = tid; i < npg; i += 64 * HB * KS) pg_lds[i] = bt[i];
   __syncthreads();
 
   // K / V tiles go global -> LDS by LDS-DMA (16 B per lane, 4 rows x 256 B per
@@ -670,7 +675,7 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   constexpr int NCH = 16 / HB;  // wave instructions per wave per 64-key tensor tile
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   auto dma = [&](int t, auto BUF) {
-    char* Kl = decltype(BUF)::value ? st1 : st0;
+    char* Kl = (decltype(BUF)::value ? st1 : st0) + group * STAGE;
     char* Vl = Kl + 64 * 256;
     int page[NCH];  // all page lookups before the first DMA issue
 #pragma unroll
@@ -695,7 +700,7 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   };
 
   // a row whose keys all lie before the partition keeps the finite start: its exponents are 0
-  float m_run = SPLIT ? -3.4028234e38f : -INFINITY, l_run = 0.f;
+  float m_run = SPLIT || KS == 2 ? -3.4028234e38f : -INFINITY, l_run = 0.f;
   float16v o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db)
@@ -709,7 +714,7 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
-  dma(t0, B0{});
+  if (KS == 1 || t0 + group < ntiles) dma(t0 + group, B0{});
   __syncthreads();  // vmcnt(0) + barrier: every wave's part of the first tile landed
   // one tile on stage BUF while the next one's DMA fills the other stage; the
   // loop is unrolled by the two stages so every LDS address is a compile-time
@@ -719,10 +724,14 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
   auto body = [&](int t, auto BUF) {
     constexpr int buf = decltype(BUF)::value;
     // the other stage was last read in tile t-1, before the previous barrier
-    if (t + 1 < ntiles) dma(t + 1, std::integral_constant<int, 1 - buf>{});
-    const char* Kl = buf ? st1 : st0;
+    if (t + KS < ntiles) dma(t + KS, std::integral_constant<int, 1 - buf>{});
+    const char* Kl = (buf ? st1 : st0) + group * STAGE;
     const char* Vl = Kl + 64 * 256;
     const int k0 = t * 64;
+    if (KS == 2 && t >= ntiles) {  // the other group has one tile more
+      __syncthreads();
+      return;
+    }
     float16v sacc[2];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -804,9 +813,33 @@ __global__ __launch_bounds__(64 * HB, HB == 4 ? 2 : 1) void prefill_attn32_kerne
     }
     __syncthreads();  // tile t+1's DMA landed (vmcnt(0)) and tile t is read by all
   };
-  for (int t = t0; t < ntiles; t += 2) {
-    body(t, B0{});
-    if (t + 1 < ntiles) body(t + 1, B1{});
+  for (int t = t0; t < ntiles; t += 2 * KS) {
+    body(t + group, B0{});
+    if (t + KS < ntiles) body(t + KS + group, B1{});
+  }
+  if constexpr (KS == 2) {
+    float4v* sums = reinterpret_cast<float4v*>(st0) + w * 16 * 64 + lane;
+    if (group) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        sums[64 * i] = float4v{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1],
+                               o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+      joined[w][lane] = m_run;
+      joined[HB + w][lane] = l_run;
+    }
+    __syncthreads();
+    if (group) return;
+    const float m = joined[w][lane], top = fmaxf(m_run, m);
+    const float mine = __builtin_amdgcn_exp2f(m_run - top), other = __builtin_amdgcn_exp2f(m - top);
+    m_run = top;
+    l_run = l_run * mine + joined[HB + w][lane] * other;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float4v v = sums[64 * i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[i >> 2][4 * (i & 3) + r] = o[i >> 2][4 * (i & 3) + r] * mine + v[r] * other;
+    }
   }
 
   if constexpr (SPLIT) {
@@ -937,14 +970,24 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
   if (q_tile == 32) {
     // 32-row waves, HB heads of one KV head per block (prefill_attn32_kernel)
     const int hb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
-    dim3 grid32(hq / hb, n_tiles, parts > 1 ? parts : 1), block32(64 * hb);
+    const dim3 grid32(hq / hb, n_tiles, parts > 1 ? parts : 1);
+    // two groups where few blocks wait for the longest walk: one a CU from 6 tiles of keys on, two a
+    // CU from 15 (us with one / two, 32 heads on 8: 300 rows 12.4 / 12.5, 512 16.8 / 15.9, 1001 28.4 /
+    // 24.0, behind 3000 keys 93 / 77, 3 x 333 14.9 / 16.9, 4 x 512 27.6 / 29.7, 2 x 1000 42.6 / 34.0,
+    // 2001 57 / 50, 32 x 512 140 / 198)
+    const int64_t blocks = (int64_t)(hq / hb) * n_tiles * (parts > 1 ? parts : 1);
+    const int64_t keys = (int64_t)bt_stride * block_size / (parts > 1 ? parts : 1);
+    const bool twice = !kv_lens && !lse_out &&
+                       (blocks <= 256 ? keys >= 360 : blocks <= 512 && parts <= 1 && keys >= 900);
 #define OMNIA_PRE32(BB, HH)                                                                  \
   do {                                                                                       \
-    if (parts > 1) OMNIA_PRE32_S(BB, HH, true);                                              \
-    else OMNIA_PRE32_S(BB, HH, false);                                                       \
+    if (parts > 1 && twice) OMNIA_PRE32_S(BB, HH, true, 2);                                  \
+    else if (parts > 1) OMNIA_PRE32_S(BB, HH, true, 1);                                      \
+    else if (twice) OMNIA_PRE32_S(BB, HH, false, 2);                                         \
+    else OMNIA_PRE32_S(BB, HH, false, 1);                                                    \
   } while (0)
-#define OMNIA_PRE32_S(BB, HH, SS)                                                            \
-  prefill_attn32_kernel<BB, HH, SS><<<grid32, block32, 0, s>>>(                              \
+#define OMNIA_PRE32_S(BB, HH, SS, KK)                                                        \
+  prefill_attn32_kernel<BB, HH, SS, KK><<<grid32, KK * 64 * HH, 0, s>>>(                     \
       (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache,        \
       block_tables, bt_stride, q_start_loc, seq_lens, tile_seq, tile_q0, hkv, q_stride,      \
       out_stride, scale_log2, lse_out, kv_lens, part_o, (float2*)part_ml, part_rows)

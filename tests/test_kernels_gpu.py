@@ -213,6 +213,34 @@ def test_prefill_attention_in_key_partitions(parts, hq, hkv, bs):
     _close(split.cpu(), exp.cpu(), 0.03, 0.02)
 
 
+@pytest.mark.parametrize("hq,hkv,bs", [(32, 8, 16), (16, 8, 32), (8, 8, 64)])
+@pytest.mark.parametrize("parts", [1, 2])
+def test_prefill_attention_by_two_groups_of_waves(parts, hq, hkv, bs):
+    """Tables of few pages are walked by one group of waves, those of more (here behind the same
+    ones, not reached) by two: from one tile of keys to uneven numbers of them."""
+    torch.manual_seed(8)
+    specs = [(1, 0), (64, 0), (33, 32), (1, 128), (40, 153), (129, 0), (97, 160), (9, 290)]
+    lens, qlens = [q + c for q, c in specs], [q for q, _ in specs]
+    nb_total = sum((n + bs - 1) // bs for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=8)
+    bt = _tables(lens, bs, nb_total)[:, : -(-max(lens) // bs)].contiguous()
+    assert bt.shape[1] * bs < 360
+    wide = torch.zeros(len(lens), 1024 // bs, dtype=torch.int32, device=DEV)
+    wide[:, : bt.shape[1]] = bt
+    q = torch.randn(sum(qlens), hq, 128, device=DEV, dtype=torch.bfloat16)
+    qsl = torch.tensor([0, *torch.tensor(qlens).cumsum(0)], dtype=torch.int32, device=DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    tiles = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in ops.prefill_tiles(qlens, 32)]
+    one, two = (torch.full_like(q, math.nan) for _ in range(2))
+    for out, table in ((one, bt), (two, wide)):
+        ops.kernels().prefill_attention(out, q, kc, vc, table, qsl, sl, *tiles, 128 ** -0.5, 0, 32,
+                                        None, None, parts)
+    exp = _attention64(q, kc, vc, bt, qlens, lens, 128 ** -0.5)
+    errs = [(o.double() - exp).norm().item() / exp.norm().item() for o in (one, two)]
+    assert errs[1] <= 1.05 * errs[0] + 1e-4, errs
+    _close(two.cpu(), exp.cpu(), 0.03, 0.02)
+
+
 def test_prefill_partitions_only_with_few_blocks():
     assert ops.prefill_parts(3, 32, 8, 400) == 1 < ops.prefill_parts(3, 32, 8, 2000)
     assert ops.prefill_parts(65, 32, 8, 100000) == 1  # 520 blocks
