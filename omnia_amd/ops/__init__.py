@@ -709,10 +709,18 @@ def panel_slices(rows: int, K: int) -> int:
 
 @functools.lru_cache(maxsize=8192)
 def panel_plan(M: int, rows: int, K: int, slabs: bool) -> tuple[int, int]:
-    """(waves a block, K slices) of a panel GEMM with ``rows`` weight rows."""
+    """(waves a block, K slices) of a panel GEMM with ``rows`` weight rows.  Unsliced, two waves
+    while their blocks are one a CU (us at 32 / 64 / 128 rows, 4 / 2 waves: 6400 x 2048 9.3 / 7.9,
+    11.5 / 9.9, 16.9 / 15.4; gated 8192 x 2048 10.5 / 8.9, 13.3 / 11.4, 19.9 / 17.8; but 12352 x
+    2048 10.7 / 12.5, 12.9 / 15.0, 18.0 / 21.8).  Where 8 and 4 both wait for the weights, 4 up to
+    16 rows (a row-major 128256 x 4096 at 1 row, 8 / 4: 164 / 157; above, packed and gated 28672 x
+    4096 at 32: 39.7 / 40.5, at 64 42.1 / 47.6)."""
+    if not slabs and rows <= 2 * 16 * 256:
+        return 2, 1
     bm = next((b for b in PANEL_ROWS if M <= b), PANEL_MAX_M)
     S = panel_slices(rows, K) if slabs else 1
-    return min((8, 4), key=lambda wn: _panel_cost(bm, rows, K, wn, S)), S
+    waves = (4, 8) if bm == 16 and not slabs else (8, 4)  # the first of equals
+    return min(waves, key=lambda wn: _panel_cost(bm, rows, K, wn, S)), S
 
 
 def panel(epi: int, x: torch.Tensor, w: torch.Tensor, packed: bool = False, bias=None,
@@ -1191,7 +1199,7 @@ def _moe_grouped(x, w_gu, w_down, ids, wts, k, n_experts, e_lo, e_hi, bm, glu=No
         segs = experts * -(-4 * n // (3 * n_experts * panel))
 
         def gemm(mode, out, A, w, so, bl, nb, rw, k, n, e0, alpha=0.0, limit=0.0):
-            wn = panel_plan(panel, w.shape[1] * segs, w.shape[2], False)[0]
+            wn = max(4, panel_plan(panel, w.shape[1] * segs, w.shape[2], False)[0])
             if streams is not None:
                 w = streams[mode == 1]
             kk.panel_moe(mode, out, A, w, so, bl, nb, rw, k, n, e0, wn, streams is not None,

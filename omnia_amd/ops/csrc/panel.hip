@@ -14,8 +14,8 @@
 //     -> 46.0 / 50.0 / 65.1; 112 beside 128 is not worth its code.  Waves of two weight units read
 //     x half as often and were no faster (28672 x 4096 at 77 51.6, at 256 92): half as many waves
 //     issue the DMA;
-//   * WN is 8, or 4 where few columns would leave CUs without a block; S blocks share a column
-//     tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
+//   * WN is 8, or 4 where few columns would leave CUs without a block, unsliced 2 while its blocks
+//     are one a CU; S blocks share a column tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
 //     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
 //     depend on how many rows the step has;
 //   * a ring of NS stages, of which NS - 1 stay in flight across the one raw barrier of a stage.
@@ -301,6 +301,8 @@ int by_rows(const PanelArgs& p, bool packed, hipStream_t s) {
 
 template <int EPI>
 int by_waves(const PanelArgs& p, int wn, bool packed, hipStream_t s) {
+  if constexpr (EPI != 2)
+    if (wn == 2) return by_rows<2, EPI>(p, packed, s);
   return wn == 8 ? by_rows<8, EPI>(p, packed, s) : by_rows<4, EPI>(p, packed, s);
 }
 
@@ -316,7 +318,7 @@ int by_segment(const PanelArgs& p, int bm, int wn, bool packed, int segs, hipStr
 extern "C" {
 
 // 0 on success, < 0 for what the kernel does not cover (checked before any launch).  wn: waves
-// a block (4, 8).
+// a block (4, 8; epi 0 and 1: 2).
 int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, int K, int S,
                 int64_t ldx, int64_t ldo, int wn, int packed, const float* bias, int gelu,
                 hipStream_t s) {
@@ -327,7 +329,7 @@ int omnia_panel(int epi, void* out, const void* x, const void* w, int M, int N, 
   if (N < 16 || N % 16 || N > 1 << 24) return -5;
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return -6;
   if (bias && epi != 1) return -7;
-  if (wn != 4 && wn != 8) return -8;
+  if (wn != 4 && wn != 8 && (wn != 2 || epi == 2)) return -8;
   const PanelArgs p{out, (const bf16_t*)x, (const bf16_t*)w, M, N, K, S, ldx, ldo, bias, gelu,
                     nullptr, nullptr, nullptr, nullptr, 1, 0, 0, 0.f, 0.f};
   if (epi == 0) return by_waves<0>(p, wn, packed, s);

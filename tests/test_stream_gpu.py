@@ -432,9 +432,12 @@ def test_panel_every_height(M, packed, monkeypatch):
     for chunks in range(1, 11):
         x, w = _mk(M, 208, 64 * chunks, M + chunks)
         want, wk = x.double() @ w.double().T, _weight(w, packed)
-        for wn in (4, 8):
+        got = []
+        for wn in (2, 4, 8):
             monkeypatch.setattr(ops, "panel_plan", lambda *a: (wn, 1))
-            _close(ops.panel(0, x, wk, packed=packed), want, 64 * chunks)
+            got.append(ops.panel(0, x, wk, packed=packed))
+            _close(got[-1], want, 64 * chunks)
+            assert torch.equal(got[-1], got[0])
 
 
 def test_panel_plans_fit_the_kernel():
