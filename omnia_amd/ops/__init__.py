@@ -585,15 +585,16 @@ def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool)
     4096 x 2048 at 193 / 256 15 / 13, 17 / 14; 2048 x 8192 at 256 23 / 27; 8256 x 2048 23 / 27;
     16512 x 4096 at 192 / 256 52 / 55, 64 / 58).
     Unsliced, a block walks all of K and takes longer the more rows it has, so few blocks lose:
-    2048 x 8192 at 32 rows 32 / 16; 4096 x 4096 at 64 20 / 15; 3072 x 1024 at 128 / 256 10 / 12,
-    16 / 12; 4096 x 2048 at 64 / 96 11 / 12, 16 / 13; 10304 x 2048 at 96 / 129 17 / 18, 22 / 17;
-    12352 x 2048 at 129 22 / 26; gated of 4096 x 2048 at 64 / 65 / 256 13 / 14, 18 / 15, 33 / 16;
-    14336 x 4096 at 128 / 160 36 / 37, 44 / 41; 16384 x 2048 at 192 / 256 28 / 30, 34 / 33; 28672
-    x 4096 at 256 69 / 74. Row-major weights of more than 0.7 GB, which the library reads at 6
+    2048 x 8192 at 32 rows 32 / 16; 4096 x 4096 at 64 17 / 15; 3072 x 1024 at 128 / 256 9.5 / 12,
+    17 / 12; 4096 x 2048 at 80 / 96 / 128 11.1 / 12.5, 12.7 / 13.4, 15.2 / 14.7; 1664 x 2048 at 96
+    12.6 / 11.2; 10304 x 2048 at 160 / 192 / 256 21 / 24, 23.5 / 25.2, 29 / 27; 8192 x 2048 at 160
+    18.3 / 17.6; gated of 4096 x 2048 at 96 / 128 / 256 14.3 / 15.7, 17.4 / 17.5, 32 / 16; 4096 x
+    1024 at 128 / 160 / 192 11.6 / 14.6, 14.0 / 15.2, 16.6 / 15.6; 14336 x 4096 at 128 / 160 36 /
+    38, 42 / 42; 16384 x 2048 at 192 / 256 29 / 30, 36 / 34; 28672 x 4096 at 256 76 / 81. Row-major weights of more than 0.7 GB, which the library reads at 6
     TB/s, only up to 32 rows: 57344 x 8192 at 32 / 64 / 256 rows 158 / 182, 182 / 161, 283 / 233;
     128256 x 4096 at 32 / 64 / 128 167 / 169, 205 / 173, 224 / 193 (65536 x 4096, 0.54 GB, at 64
     105 / 127). Layers 1024 wide stay here by a little more: their eager steps wait for the host,
-    which these launches cost less (gated 8192 x 1024 at 160 / 256 17.0 / 16.3, 22 / 19, but a
+    which these launches cost less (gated 8192 x 1024 at 160 / 256 14.1 / 16.3, 21 / 19, but a
     step of 16 such layers of 200 rows 1.23 ms / 1.74)."""
     if not packed and M > 32 and R * K > 3.5e8:
         return False
@@ -602,11 +603,13 @@ def few_rows_pay(M: int, R: int, K: int, gated: bool, packed: bool, slabs: bool)
     if M <= 64:
         return gated or K <= 2048 or R >= 12288
     if gated and K <= 1024:
-        return R >= 8192
+        return R >= (4096 if M <= 160 else 8192)
+    if M <= 96 and 2048 >= K and R >= 4096:
+        return True
     if M <= 128:
         return R >= 8192 or K <= 1024
     if M <= 192:
-        return R >= (12288 if K <= 2048 else 16384)
+        return R >= (10240 if K <= 2048 else 16384)
     return gated and R >= 16384  # for fp32 into the activation, at what the library takes
 
 
