@@ -440,6 +440,24 @@ def test_panel_every_height(M, packed, monkeypatch):
             assert torch.equal(got[-1], got[0])
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("M,R,K", [(1, 32, 64), (17, 96, 192), (64, 160, 640), (81, 8192, 128),
+                                   (129, 96, 1088), (256, 416, 2048)])
+def test_panel_gated_in_blocks_of_two_waves(M, R, K, packed, monkeypatch):
+    """The bits of blocks of four waves, blocks without all of their rows included; never slabs."""
+    x, w = _mk(M, R, K, M + R + K)
+    wk, b = _weight(w, packed), torch.randn(R, device="cuda")
+    assert ops.panel_plan(M, R, K, False) == (2, 1)
+    got = ops.panel(1, x, wk, packed=packed, bias=b)
+    monkeypatch.setattr(ops, "panel_plan", lambda *a: (4, 1))
+    assert torch.equal(got, ops.panel(1, x, wk, packed=packed, bias=b))
+    g, u = (x.double() @ w.double().T + b.double()).chunk(2, 1)
+    _close(got, F.silu(g) * u, 4 * K, 1.1)
+    with pytest.raises(RuntimeError):
+        ops.kernels().panel_gemm(2, x.new_empty(1, M, R, dtype=torch.float32), x, wk, 2, packed,
+                                 None, False)
+
+
 def test_panel_plans_fit_the_kernel():
     """Whatever the size, a plan is one that the kernel covers, with slices that do not depend on
     the rows."""
