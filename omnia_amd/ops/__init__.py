@@ -270,7 +270,7 @@ _midm_on = os.environ.get("OMNIA_MIDM", "1") != "0"
 
 def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | None:
     """Mid-size projections (M = 257..4096 rows: open-loop mixed steps, which
-    the unsplit 256x256 prefill tile under-fills): ``(columns of a tile, PGEMM_SPLIT, S)``
+    the unsplit 256x256 prefill tile under-fills): ``(256, PGEMM_SPLIT, S)``
     when ``ops/tuned/midm_mi355x.json`` lists a split-K win of the 256x256 tile
     (+ its slab consumer) over the library path for this shape's M bucket
     (``scripts/midm_sweep.py``), else None (library GEMM)."""
@@ -287,12 +287,7 @@ def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | Non
                 _midm_table = {k: int(v) for k, v in json.load(f).items()}
     b = next(x for x in MIDM_BUCKETS if M <= x)
     S = _midm_table.get(f"{mode}:{b}:{N}:{K}")
-    if not S:
-        return None
-    # short slices cost more in slabs than the narrow tile's second read of x: as many blocks in
-    # half the slices (us with the consumer's reads, before / after: 4096 x 4096 at 512 rows 32.4
-    # / 28.2, 768 38.1 / 38.0, 999 43.9 / 40.7; not 4096 x 14336: at 512 60.0 / 62.8)
-    return (128, PGEMM_SPLIT, S // 2) if S >= 4 and K <= 4096 else (256, PGEMM_SPLIT, S)
+    return (256, PGEMM_SPLIT, S) if S else None
 
 
 def wgemm(mode: int, x: torch.Tensor, w: torch.Tensor, splits: int = 1, nw: int = 2,

@@ -28,6 +28,14 @@ def test_bucket_mapping_and_boundaries():
     assert ops.midm_config(700, 1234, 4096, 0) is None  # unknown shape
 
 
+def test_slices_are_the_tables():
+    """No fewer fp16 slabs than the table says: each would saturate at less of the row's sum."""
+    p = os.path.join(os.path.dirname(ops.__file__), "tuned", "midm_mi355x.json")
+    for k, S in json.load(open(p)).items():
+        mode, b, N, K = (int(x) for x in k.split(":"))
+        assert ops.midm_config(b, N, K, mode) == (256, ops.PGEMM_SPLIT, S)
+
+
 def test_kill_switch(monkeypatch):
     monkeypatch.setattr(ops, "_midm_on", False)
     assert ops.midm_config(600, 4096, 14336, 0) is None

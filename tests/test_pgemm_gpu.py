@@ -214,6 +214,19 @@ def test_splitk_saturates_fp16(gen, schedule):
     assert (parts[:, :, N // 2:] == 65504).all() and (parts[:, :, : N // 2] == -65504).all()
 
 
+def test_mid_size_slabs_hold_large_sums():
+    """A step of 512 rows, whose projection of 4096 the table cuts in 8: the slabs hold a row's sum
+    of 393216, 49152 each."""
+    from omnia_amd.models.projection import Parts, Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device(DEV), torch.bfloat16, 1, {}
+
+    x = torch.full((512, 4096), 16.0, dtype=torch.bfloat16, device=DEV)
+    y = Model()._proj("o", x, torch.full((4096, 4096), 6.0, dtype=torch.bfloat16, device=DEV), False)
+    assert isinstance(y, Parts) and (y.t.float().sum(0) == 96 * 4096).all()
+
+
 def test_splitk_feeds_consumer(gen, schedule):
     """pgemm split-K slabs through splitk_swiglu == SwiGLU of the fp32 product."""
     M, F, K, S = 256, 512, 2048, 4
