@@ -97,7 +97,10 @@ __global__ __launch_bounds__(256 * KS, DK + DV <= 256 ? 2 : 1) void prefill_kern
   if (b0 >= qlen) return;
   const int off = p.seq_lens[s] - qlen;  // position of the portion's first row
   const int tid = threadIdx.x, lane = tid & 63, ql = lane & 31, hi = lane >> 5;
-  const int w = (tid >> 6) & 3, part = KS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+  // the wave's number as a scalar, and all that follows from it: heads of 128 need no scratch so (24
+  // bytes a lane without, 8 x 2048 rows and 16 heads 207 us / 191)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
+  const int part = KS == 1 ? 0 : wave >> 2;
   const int h = hblk * HB + (w & (HB - 1)), kvh = hblk * HB / group;
   const int* bt = p.block_tables + (int64_t)s * p.bt_stride;
   const int BS = 1 << p.page_lg, pmask = BS - 1;
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(256 * KS, DK + DV <= 256 ? 2 : 1) void prefill_kern
 
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
-  if (part < nt) dma(tile_of(part), B0{});
+  if (KS == 1 || part < nt) dma(tile_of(part), B0{});
   __syncthreads();
   auto body = [&](int j, auto BUF) {
     constexpr int buf = decltype(BUF)::value;
