@@ -348,7 +348,7 @@ class LlamaModel(Projections):
         if T > Bd:
             ops.prefill_attention(q3[Bd:], kv.k[li], kv.v[li], fb.block_tables,
                                   fb.q_start_loc, fb.seq_lens, self.scale, fb.tile_seq,
-                                  fb.tile_q0, out=o[Bd:])
+                                  fb.tile_q0, out=o[Bd:], shared_device=self._shared_device())
         return o
 
     def decode_part(self, batch: int, max_ctx: int) -> tuple[int, int]:
@@ -387,7 +387,8 @@ class LlamaModel(Projections):
         if fb.num_decode:
             return self._mixed_attention(li, q3, fb, kv)
         return ops.prefill_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.q_start_loc,
-                                     fb.seq_lens, self.scale, fb.tile_seq, fb.tile_q0)
+                                     fb.seq_lens, self.scale, fb.tile_seq, fb.tile_q0,
+                                     shared_device=self._shared_device())
 
     def _decode_ws(self, B, max_blocks, bs, device, part, splits=0):
         key = (B, max_blocks, bs, str(device), part, splits)

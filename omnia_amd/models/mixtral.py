@@ -89,7 +89,7 @@ class MixtralModel(LlamaModel):
                        graph_safe=self.graph_safe or h.shape[0] < 64,
                        streams=packed_experts(self, layer["experts_gate_up"],
                                               layer["experts_down"]),
-                       shared_device=self.tp > 1 and pstate.ranks_per_device() > 1)
+                       shared_device=self._shared_device())
 
     def forward(self, fb, kv, gather: bool = True):
         # decode batches are captured into hipGraphs: keep the MoE path sync-free

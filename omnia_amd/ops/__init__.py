@@ -913,7 +913,7 @@ def prefill_tiles(q_lens: list[int], tile: int | None = None) -> tuple[list[int]
 
 
 @functools.lru_cache(maxsize=4096)
-def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int) -> int:
+def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int, one_group: bool = False) -> int:
     """Most key partitions of a 32-row query tile, for up to 512 blocks, two a CU (fewer where the
     live length gives a partition less than 128 keys).  A block walks its 64-key tiles one after
     the other, 1.35 us each, or, with two groups of waves where blocks are one a CU, 0.975;
@@ -926,7 +926,7 @@ def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int) -> int:
 
     def walk(P):
         t = -(-max_keys // 64) / P
-        return min(1.35 * t, 0.975 * t + 1.5) if blocks * P <= 256 else 1.35 * t
+        return min(1.35 * t, 0.975 * t + 1.5) if blocks * P <= 256 and not one_group else 1.35 * t
 
     best, cost = 1, walk(1)
     for P in range(2, min(16, 512 // max(blocks, 1), max_keys // 128) + 1):
@@ -938,7 +938,8 @@ def prefill_parts(tiles: int, hq: int, hkv: int, max_keys: int) -> int:
 
 def prefill_attention(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens, scale,
                       tile_seq=None, tile_q0=None, out=None, heads_per_wave: int = 0,
-                      q_tile: int | None = None, lse=None, kv_lens=None):
+                      q_tile: int | None = None, lse=None, kv_lens=None,
+                      shared_device: bool = False):
     """q: [T, Hq, D] new tokens of several sequences (varlen, causal w/ cached prefix).
 
     ``lse`` (fp32 [T, Hq], optional) receives each row's natural-log sum of
@@ -946,7 +947,9 @@ def prefill_attention(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens, 
     with.  ``kv_lens`` (int32 [B], optional) caps the visible keys of sequence
     ``s`` at ``kv_lens[s]`` on top of the causal bound, so a K/V block that lies
     wholly before the queries is attended in full: ``seq_lens = kv_len + qlen``
-    puts the queries after every key."""
+    puts the queries after every key.  ``shared_device``: other ranks run on this device, whose
+    all-reduce blocks may spin until this rank's next: blocks of two groups of waves hold all of a
+    CU's registers, do not fit beside them and could wait out their spin bound."""
     if q.is_cuda:
         if tile_seq is None:
             qsl = q_start_loc.cpu().tolist()
@@ -961,10 +964,10 @@ def prefill_attention(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens, 
         parts = 1
         if q_tile == 32 and lse is None and kv_lens is None:
             parts = prefill_parts(tile_seq.numel(), q.shape[1], k_cache.shape[1],
-                                  block_tables.shape[1] * k_cache.shape[2])
+                                  block_tables.shape[1] * k_cache.shape[2], shared_device)
         kernels().prefill_attention(out, q, k_cache, v_cache, block_tables, q_start_loc,
                                     seq_lens, tile_seq, tile_q0, scale, heads_per_wave, q_tile,
-                                    lse, kv_lens, parts)
+                                    lse, kv_lens, parts, shared_device)
         return out
     if lse is not None or kv_lens is not None:
         r, l = ref.paged_attention_lse(q, k_cache, v_cache, block_tables, q_start_loc, seq_lens,

@@ -52,7 +52,8 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
                             int n_tiles, int hq, int hkv, int head_dim, int block_size,
                             int64_t q_stride, int64_t out_stride, float scale, int hp,
                             int q_tile, float* lse_out, const int* kv_lens, float* part_o,
-                            float* part_ml, int parts, int64_t part_rows, hipStream_t s);
+                            float* part_ml, int parts, int64_t part_rows, int one_group,
+                            hipStream_t s);
 int omnia_apply_token_mask(void* logits, int logits_is_bf16, int rows, int64_t row_stride,
                            int vocab, const uint32_t* mask, int words, hipStream_t s);
 int omnia_sample(int* out_tok, float* out_logprob, const void* logits, int logits_is_bf16,
@@ -387,7 +388,7 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache, at::Ten
                        at::Tensor block_tables, at::Tensor q_start_loc, at::Tensor seq_lens,
                        at::Tensor tile_seq, at::Tensor tile_q0, double scale, int64_t hp,
                        int64_t q_tile, c10::optional<at::Tensor> lse,
-                       c10::optional<at::Tensor> kv_lens, int64_t parts) {
+                       c10::optional<at::Tensor> kv_lens, int64_t parts, bool one_group) {
   CHECK_GPU(q); CHECK_BF16(q); CHECK_BF16(out); CHECK_BF16(k_cache);
   CHECK_I32(block_tables); CHECK_I32(q_start_loc); CHECK_I32(seq_lens); CHECK_I32(tile_seq);
   CHECK_I32(tile_q0);
@@ -425,7 +426,7 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache, at::Ten
                                    tile_q0.data_ptr<int>(), tile_seq.numel(), q.size(1), hkv, D,
                                    bs, q.stride(0), out.stride(0), (float)scale, (int)hp,
                                    (int)q_tile, lse_p, kvl_p, po, pml, (int)parts, q.size(0),
-                                   cur_stream()),
+                                   one_group, cur_stream()),
            "prefill_attention");
 }
 
@@ -2144,7 +2145,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"), py::arg("q_start_loc"),
         py::arg("seq_lens"), py::arg("tile_seq"), py::arg("tile_q0"), py::arg("scale"),
         py::arg("hp") = 0, py::arg("q_tile") = 64, py::arg("lse") = py::none(),
-        py::arg("kv_lens") = py::none(), py::arg("parts") = 1);
+        py::arg("kv_lens") = py::none(), py::arg("parts") = 1, py::arg("one_group") = false);
   m.def("sample", &sample, py::arg("out_tok"), py::arg("out_logprob"), py::arg("logits"),
         py::arg("temperature"), py::arg("top_k"), py::arg("top_p"), py::arg("seeds"),
         py::arg("steps"), py::arg("counts"), py::arg("freq_pen"), py::arg("pres_pen"),

@@ -241,6 +241,24 @@ def test_prefill_attention_by_two_groups_of_waves(parts, hq, hkv, bs):
     _close(two.cpu(), exp.cpu(), 0.03, 0.02)
 
 
+def test_prefill_attention_of_ranks_that_share_a_device():
+    """Where two groups of waves would share a walk over the keys, such ranks keep to one: the bits
+    of one group, whose blocks leave half of a CU's registers to the peers' all-reduce."""
+    torch.manual_seed(9)
+    kc, vc = _make_cache(40, 2, 32, seed=9)
+    bt = _tables([500], 32, 40)
+    q = torch.randn(200, 8, 128, device=DEV, dtype=torch.bfloat16)
+    qsl, sl = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in ([0, 200], [500]))
+    tiles = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in ops.prefill_tiles([200], 32)]
+    args = (q, kc, vc, bt, qsl, sl, 128 ** -0.5, *tiles)
+    parts = ops.prefill_parts(tiles[0].numel(), 8, 2, bt.shape[1] * 32, True)
+    one = torch.empty_like(q)
+    ops.kernels().prefill_attention(one, *args[:6], *tiles, 128 ** -0.5, 0, 32, None, None, parts,
+                                    True)
+    assert not torch.equal(ops.prefill_attention(*args), one)
+    assert torch.equal(ops.prefill_attention(*args, shared_device=True), one)
+
+
 def test_prefill_partitions_only_with_few_blocks():
     assert ops.prefill_parts(3, 32, 8, 400) == 1 < ops.prefill_parts(3, 32, 8, 2000)
     assert ops.prefill_parts(65, 32, 8, 100000) == 1  # 520 blocks
