@@ -955,7 +955,7 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
                             int n_tiles, int hq, int hkv, int head_dim, int block_size,
                             int64_t q_stride, int64_t out_stride, float scale, int hp_req, int q_tile,
                             float* lse_out, const int* kv_lens, float* part_o, float* part_ml, int parts,
-                            int64_t part_rows, int one_group, hipStream_t s) {
+                            int64_t part_rows, int n_seqs, int one_group, hipStream_t s) {
   if (head_dim != 128) return -1;
   if (hq % hkv) return -2;
   if (parts > 1 && (q_tile != 32 || lse_out || kv_lens || !part_o || !part_ml)) return -8;
@@ -972,13 +972,19 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
     const int hb = G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
     const dim3 grid32(hq / hb, n_tiles, parts > 1 ? parts : 1);
     // two groups where few blocks wait for the longest walk: one a CU from 6 tiles of keys on, two a
-    // CU from 15 (us with one / two, 32 heads on 8: 300 rows 12.4 / 12.5, 512 16.8 / 15.9, 1001 28.4 /
-    // 24.0, behind 3000 keys 93 / 77, 3 x 333 14.9 / 16.9, 4 x 512 27.6 / 29.7, 2 x 1000 42.6 / 34.0,
-    // 2001 57 / 50, 32 x 512 140 / 198).  one_group: never; two fill a CU's registers and most of its LDS
+    // CU from 15 where portions are so long (768 rows in the mean) that their walks differ: two groups
+    // fill the CU and its blocks come one after the other (us with one / two, 32 heads on 8: 300
+    // rows 12.4 / 12.5, 512 16.8 / 15.9, 1001 28.4 / 24.0, behind 3000 keys 93 / 77, 3 x 333 14.9 /
+    // 16.9, 4 x 512 27.6 / 29.7, 2 x 1000 41.7 / 32.7, behind 3000 keys 147 / 135, 2001 55.8 / 48.8,
+    // 32 x 512 140 / 198; behind 512 to 1500 keys 4 x 512 46.8 / 48.4, 8 x 256 46.8 / 50.3, 16 x 100 64
+    // / 70; 32 heads on 16, 8 x 100 behind 1000 41.2 / 46.2).  one_group: never, since two fill a
+    // CU's registers and most of its LDS
     const int64_t blocks = (int64_t)(hq / hb) * n_tiles * (parts > 1 ? parts : 1);
     const int64_t keys = (int64_t)bt_stride * block_size / (parts > 1 ? parts : 1);
     const bool twice = !one_group && !kv_lens && !lse_out &&
-                       (blocks <= 256 ? keys >= 360 : blocks <= 512 && parts <= 1 && keys >= 900);
+                       (blocks <= 256 ? keys >= 360
+                                      : blocks <= 512 && parts <= 1 && keys >= 900 &&
+                                            part_rows >= (int64_t)768 * n_seqs);
 #define OMNIA_PRE32(BB, HH)                                                                  \
   do {                                                                                       \
     if (parts > 1 && twice) OMNIA_PRE32_S(BB, HH, true, 2);                                  \

@@ -52,8 +52,8 @@ int omnia_prefill_attention(void* out, const void* q, const void* k_cache, const
                             int n_tiles, int hq, int hkv, int head_dim, int block_size,
                             int64_t q_stride, int64_t out_stride, float scale, int hp,
                             int q_tile, float* lse_out, const int* kv_lens, float* part_o,
-                            float* part_ml, int parts, int64_t part_rows, int one_group,
-                            hipStream_t s);
+                            float* part_ml, int parts, int64_t part_rows, int n_seqs,
+                            int one_group, hipStream_t s);
 int omnia_apply_token_mask(void* logits, int logits_is_bf16, int rows, int64_t row_stride,
                            int vocab, const uint32_t* mask, int words, hipStream_t s);
 int omnia_sample(int* out_tok, float* out_logprob, const void* logits, int logits_is_bf16,
@@ -426,7 +426,7 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache, at::Ten
                                    tile_q0.data_ptr<int>(), tile_seq.numel(), q.size(1), hkv, D,
                                    bs, q.stride(0), out.stride(0), (float)scale, (int)hp,
                                    (int)q_tile, lse_p, kvl_p, po, pml, (int)parts, q.size(0),
-                                   one_group, cur_stream()),
+                                   seq_lens.numel(), one_group, cur_stream()),
            "prefill_attention");
 }
 

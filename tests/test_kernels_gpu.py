@@ -259,6 +259,29 @@ def test_prefill_attention_of_ranks_that_share_a_device():
     assert torch.equal(ops.prefill_attention(*args, shared_device=True), one)
 
 
+@pytest.mark.parametrize("news,past,two", [([100] * 8, 1000, False), ([512] * 4, 512, False),
+                                           ([1000] * 2, 0, True), ([100] * 2, 1000, True)])
+def test_prompt_attention_of_walks_alike_by_one_group(news, past, two):
+    """Two blocks a CU are of two groups only where the walks over the keys differ, one a CU are
+    whatever they walk."""
+    torch.manual_seed(10)
+    hkv, hq = (16, 32) if past == 1000 else (8, 32)
+    lens = [n + past for n in news]
+    nb_total = sum(-(-n // 32) for n in lens) + 8
+    kc, vc = _make_cache(nb_total, hkv, 32, seed=10)
+    bt = _tables(lens, 32, nb_total)
+    q = torch.randn(sum(news), hq, 128, device=DEV, dtype=torch.bfloat16)
+    qsl = torch.tensor([0, *torch.tensor(news).cumsum(0)], dtype=torch.int32, device=DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    tiles = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in ops.prefill_tiles(news, 32)]
+    got = []
+    for one_group in (False, True):
+        got.append(torch.empty_like(q))
+        ops.kernels().prefill_attention(got[-1], q, kc, vc, bt, qsl, sl, *tiles, 128 ** -0.5, 0, 32,
+                                        None, None, 1, one_group)
+    assert torch.equal(*got) != two
+
+
 def test_prefill_partitions_only_with_few_blocks():
     assert ops.prefill_parts(3, 32, 8, 400) == 1 < ops.prefill_parts(3, 32, 8, 2000)
     assert ops.prefill_parts(65, 32, 8, 100000) == 1  # 520 blocks
