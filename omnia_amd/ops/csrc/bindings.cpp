@@ -216,7 +216,8 @@ int omnia_gqa_prefill(void* out, const void* q, const void* kc, const void* vc,
                       const int* block_tables, int bt_stride, const int* q_start,
                       const int* seq_lens, const int* tile_seq, const int* tile_q0, int n_tiles,
                       int page, int H, int G, int Dp, int Vp, Mask mask, Score score,
-                      const float* sinks, const float* gate, int bounded, hipStream_t s);
+                      const float* sinks, const float* gate, int bounded, int64_t rows, int n_seqs,
+                      hipStream_t s);
 int omnia_joined_residual(void* h1, void* h2, int f32, float* x, int fresh, int rows, int d,
                           const void* am, int at, int aS, int64_t arow, int64_t apart,
                           const void* bm, int bS, int64_t brow, int64_t bpart, const void* cm,
@@ -2096,7 +2097,8 @@ void gqa_prefill(at::Tensor out, at::Tensor q, at::Tensor k, at::Tensor v, at::T
                              veci(tile_seq, nt, "tile_seq"), veci(tile_q0, nt, "tile_q0"), nt,
                              s.page, H, s.G, s.Dp, s.Vp, mask_of(mask),
                              score_of(scale, cap, dist, H), opt_ptr<float>(sinks),
-                             opt_vecf(gate, q.size(0) * H, "gate"), bounded, cur_stream()),
+                             opt_vecf(gate, q.size(0) * H, "gate"), bounded, q.size(0), nseq,
+                             cur_stream()),
            "gqa_prefill");
 }
 

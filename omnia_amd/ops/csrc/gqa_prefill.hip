@@ -392,7 +392,8 @@ int omnia_gqa_prefill(void* out, const void* q, const void* kc, const void* vc,
                       const int* block_tables, int bt_stride, const int* q_start,
                       const int* seq_lens, const int* tile_seq, const int* tile_q0, int n_tiles,
                       int page, int H, int G, int Dp, int Vp, Mask mask, Score score,
-                      const float* sinks, const float* gate, int bounded, hipStream_t s) {
+                      const float* sinks, const float* gate, int bounded, int64_t rows, int n_seqs,
+                      hipStream_t s) {
   if (G < 1 || H % G || !mask.ok() || !score.ok()) return -1;
   if (bounded && (!(score.cap > 0.f && score.cap <= 40.f) || !score.r1)) return -5;
   int page_lg = 0;
@@ -406,13 +407,17 @@ int omnia_gqa_prefill(void* out, const void* q, const void* kc, const void* vc,
          page_lg, mask, Score2(score)};
   const bool keep = mask.window > 0 && mask.chunk == 0 && mask.keep > 0;
   // two groups of waves where few blocks wait for the longest walk: one a CU, from 5 tiles of keys,
-  // or two a CU, from 32 (us with one / two, 16 heads of 128: 77 rows 8.1 / 9.4, behind 1900 keys 59 /
-  // 43, 300 14.6 / 13.4, 1001 33.9 / 26.3, 2001 60.7 / 45.4, window 1024 36.8 / 29.5; 384 to 512
-  // blocks: 3000 rows 93 / 64, window 1024 46 / 54, 8 x 333 22 / 27, 2 x 2048 85 / 58; 2048 blocks
-  // 208 / 218)
+  // or two a CU, from 32 tiles where portions are so long (1024 rows in the mean) that their walks
+  // differ, or where two such blocks fit a CU (us with one / two, 16 heads of 128: 77 rows 8.9 / 9.5,
+  // 300 13.4 / 12.7, 2001 55 / 43.5, window 1024 33.3 / 27.9, 2 x 1000 behind 4000 keys 134 / 101; 384
+  // to 512 blocks: 3000 rows 82 / 59.5, window 1024 41 / 50, 8 x 333 20 / 25, 2 x 2048 76 / 55, behind
+  // 2000 keys 150 / 128; 8 x 512 behind 2000 106 / 112, 32 x 128 98 / 117, of heads of 32 46 / 39; 2048
+  // blocks 208 / 218)
   const int keys = mask.most((int)std::min<int64_t>((int64_t)bt_stride << page_lg, 1 << 30));
   const int64_t blocks = (int64_t)n_tiles * H;
-  const bool twice = blocks <= 256 ? keys >= 320 : blocks <= 512 && keys >= 2048;
+  const bool twice = blocks <= 256 ? keys >= 320
+                                   : blocks <= 512 && keys >= 2048 &&
+                                         (rows >= (int64_t)1024 * n_seqs || Dp <= 32);
 #define OMNIA_GQS(K, V, KEEP, SHAPE)                                                      \
   do {                                                                                    \
     if constexpr (K == V && K <= 128)                                                     \

@@ -457,6 +457,29 @@ def test_prefill_by_two_groups_of_waves(kind, D, G):
     assert rel(got[1].double(), got[0].double()) < 0.004
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,two", [(128, False), (64, False), (32, True)])
+def test_prefill_of_walks_alike_by_one_group(D, two):
+    """512 blocks whose walks are alike take one group of waves, as 1024 do: the same bits.  Where
+    two blocks of two groups fit a CU, they take two."""
+    H, G, page, g = 16, 2, 32, gen(16)
+    spec = AttentionSpec(H, G, D, D, 0.2, RotarySpec(8, 1e4))
+    pages = [torch.randn(67, G, page, D, generator=g).to("cuda", torch.bfloat16) for _ in range(2)]
+    q = torch.randn(64 * 128, H * D, generator=g).to("cuda", torch.bfloat16)
+
+    def run(n):
+        def ints(v):
+            return torch.tensor(v, dtype=torch.int32, device="cuda")
+
+        ts, t0 = prefill_tiles([128] * n, 128)
+        fb = ForwardBatch(None, None, None, ints([list(range(67))] * n), ints([2128] * n), None,
+                          is_decode=False, q_start_loc=ints([128 * i for i in range(n + 1)]),
+                          tile_seq=ints(ts), tile_q0=ints(t0))
+        return mops.gqa_prefill(q[:128 * n], pages, fb, spec, None)
+
+    assert torch.equal(run(32), run(64)[:32 * 128]) != two
+
+
 # ---------------------------------------------------------------- experts
 def expert_weights(E, d, ff, g, scale=1.0):
     W = {"router": rnd(E, d, g=g, scale=d ** -0.5)}
