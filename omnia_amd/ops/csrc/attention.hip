@@ -60,10 +60,11 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
 // 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  Of
 // sequences that share the pages of a prompt prefix a block finds in the caches what another has
 // read; K and V that nobody shares go past them (non-temporal).  us through the caches and by
-// this rule: 256 x 576, ragged, 112 -> 107, 128 x 1000 101 -> 92, 64 x 2000 92 -> 81 (6.5 TB/s); 512
-// of 256 x 576 shared 58.3 -> 59.1 (past the caches 71), 896 of 128 x 1000 46.6 -> 47.5 (60); 256 x
-// 150, below it, 33 (past 35.5); 32 x 1000 29.4 -> 27.4, 960 shared 20.6 -> 21.3; 8 x 1000 in
-// partitions of 256 15.5 -> 14.7, 4 x 1000, of 128 and below it, 11.2 (past, with the look, 12.1).
+// this rule: 256 x 576 107 -> 102.5, 128 x 1000 93.6 -> 81.8, 64 x 2000 91 -> 80, 512 x 600 212 ->
+// 200; 512 of 256 x 576 shared by all 55.2 -> 55, by sequences 32 apart 54 -> 55.9 (past the caches
+// 76), 896 of 128 x 1000 44.8 -> 44.4 and 45 -> 46.7 (59, 66); 256 x 150, below it, 33 (past 35.5);
+// 32 x 1000 in a step 29.4 -> 27.4, 8 x 1000 in partitions of 256 15.5 -> 14.7, 4 x 1000, of 128 and
+// below it, 11.2 (past, with the look, 12.1).
 constexpr int NW = 4;
 template <int G>
 struct DecodeShared {
@@ -273,16 +274,21 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
   const int pl = decode_part_len(len, part_size, split_t, split_min, BS);
   const int p0 = part * pl;
   if (p0 >= len) return;
-  // past the caches: of a long sequence what none of the next 16 sequences has the page of, 64
-  // keys into the partition (a row's entries past its length may be anything: at worst the caches
-  // are used).  What shares less is read again for less than is gained
+  // past the caches: of a long sequence what no other has the page of, 64 keys into the partition (a
+  // row's entries past its length may be anything: at worst the caches are used).  What shares less
+  // is read again for less than is gained.  Sharers may be anywhere in the batch, so the block's
+  // threads look at all of it, a row each; up to 64 rows every wave for itself, without a barrier
   constexpr int LONG = 512;
   if (len >= LONG && min(pl, len - p0) >= 192 && gridDim.x > 1) {
-    const int B = gridDim.x, d = min(1 + (int)(threadIdx.x & 15), B - 1);
-    const int* t = block_tables + min(p0 + 64, len - 1) / BS;
-    const bool same = t[(int64_t)(b + d < B ? b + d : b + d - B) * bt_stride] ==
-                      t[(int64_t)b * bt_stride];
-    if (__builtin_amdgcn_ballot_w64(same) == 0) {
+    const int B = gridDim.x, *t = block_tables + min(p0 + 64, len - 1) / BS;
+    const int own = t[(int64_t)b * bt_stride];
+    bool same = false;
+    for (int i = B <= 64 ? threadIdx.x & 63 : threadIdx.x; i < B; i += 128 * NW) {
+      const int j = min(i + 64 * NW, B - 1);
+      const int x = t[(int64_t)i * bt_stride], y = t[(int64_t)j * bt_stride];
+      same |= (x == own && i != b) || (y == own && j != b);
+    }
+    if (B <= 64 ? __builtin_amdgcn_ballot_w64(same) == 0 : !__syncthreads_or(same)) {
       decode_block<G, BS, true>(sh, len, pl, out, part_o, part_ml, q, kc, vc, block_tables,
                                 bt_stride, hkv, q_stride, max_parts, scale_log2);
       return;

@@ -399,6 +399,40 @@ def test_decode_attention_past_and_through_the_caches(lens, hq, bs, part, splits
     assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
 
 
+def test_decode_attention_finds_sharers_far_apart():
+    """Prompt prefixes shared by sequences 32 rows apart: the sums are right, and the shared pages go
+    through the caches as those of neighbours do (past them 1.4 times as long)."""
+    torch.manual_seed(14)
+    B, hq, hkv, bs, shared, n = 256, 32, 8, 32, 512, 576
+    own = -(-n // bs) - shared // bs
+    nb = 32 * (shared // bs) + B * own
+    kc, vc = (torch.randn(nb, hkv, bs, 128, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(B, hq, 128, device=DEV, dtype=torch.bfloat16)
+    sl = torch.full((B,), n, dtype=torch.int32, device=DEV)
+    rows = torch.arange(B)
+
+    def table(group):
+        pre = group[:, None] * (shared // bs) + torch.arange(shared // bs)
+        tail = 32 * (shared // bs) + rows[:, None] * own + torch.arange(own)
+        return torch.cat([pre, tail], 1).int().to(DEV)
+
+    best, tables = {}, {"apart": table(rows % 32), "all": table(rows * 0)}
+    for _ in range(12):
+        for name, bt in tables.items():
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=1024)
+            b.record()
+            torch.cuda.synchronize()
+            best[name] = min(best.get(name, 1e9), a.elapsed_time(b))
+            if name == "apart":
+                got = out[::37]
+    exp = _attention64(q[::37], kc, vc, tables["apart"][::37], [1] * 7, [n] * 7, 128 ** -0.5)
+    assert ((got.double() - exp).abs() <= exp.abs() * 2.0 ** -8 + 1e-4).all()
+    assert best["apart"] < 1.2 * best["all"], best
+
+
 def test_sample_greedy_matches_argmax():
     logits = torch.randn(7, 128256, device=DEV)
     temp = torch.zeros(7, device=DEV)
