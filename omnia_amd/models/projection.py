@@ -179,15 +179,13 @@ class Projections:
             return None
         return ops.wgemm_config(M, N, K, mode)
 
-    # split-K slabs of the tile GEMM in fp16 (tgemm mode 3): half the slab bytes
+    # split-K slabs of the tile GEMMs in fp16 (tgemm mode 3, pgemm): half the slab bytes
     # the producer writes and the consumer (splitk.hip) reads; each slab is one
     # K-slice's fp32 sum rounded to 11 bits, finer than the bf16 rounding of the
     # projection output itself.  OMNIA_SPLITK_FP32=1 keeps fp32 slabs.
     splitk_half = os.environ.get("OMNIA_SPLITK_FP32", "0") != "1"
 
     def _slab_dtype(self, nwaves: int) -> torch.dtype:
-        if nwaves == ops.PGEMM_SPLIT:
-            return torch.float16  # the 256x256 split-K tile writes fp16 slabs only
         return torch.float16 if (self.splitk_half and nwaves < 0) else torch.float32
 
     def _wgemm(self, mode: int, x: torch.Tensor, w: torch.Tensor, S: int, nw: int, nwaves: int,

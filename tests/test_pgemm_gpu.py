@@ -227,6 +227,20 @@ def test_mid_size_slabs_hold_large_sums():
     assert isinstance(y, Parts) and (y.t.float().sum(0) == 96 * 4096).all()
 
 
+def test_slabs_of_the_split_tile_in_fp32():
+    """OMNIA_SPLITK_FP32=1 on it too: sums past fp16's range."""
+    from omnia_amd.models.projection import Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device(DEV), torch.bfloat16, 1, {}
+        splitk_half = False
+
+    x = torch.full((512, 4096), 16.0, dtype=torch.bfloat16, device=DEV)
+    w = torch.full((4096, 4096), 96.0, dtype=torch.bfloat16, device=DEV)
+    y = Model()._proj("o", x, w, False)
+    assert y.t.dtype == torch.float32 and (y.t.sum(0) == 1536 * 4096).all()
+
+
 def test_splitk_feeds_consumer(gen, schedule):
     """pgemm split-K slabs through splitk_swiglu == SwiGLU of the fp32 product."""
     M, F, K, S = 256, 512, 2048, 4
