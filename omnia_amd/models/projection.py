@@ -246,8 +246,8 @@ class Projections:
                 return ops.pgemm(0, x, w)
             S = ops.tile_slices(M, w.shape[0], K) if slabs and w.is_contiguous() else 0
             if S:
-                return Parts(ops.pgemm_splitk(
-                    x, w, S, torch.empty(S, M, w.shape[0], device=x.device), cols=128))
+                out = torch.empty(S, M, w.shape[0], dtype=torch.float32, device=x.device)
+                return Parts(ops.pgemm_splitk(x, w, S, out, cols=128))
         return ops.linear(x, w)
 
     _min_rows = int(os.environ.get("OMNIA_PGEMM_MIN_ROWS", "2049"))  # this forward's threshold (mixed steps: the higher one)

@@ -241,6 +241,26 @@ def test_slabs_of_the_split_tile_in_fp32():
     assert y.t.dtype == torch.float32 and (y.t.sum(0) == 1536 * 4096).all()
 
 
+def test_slices_of_the_narrow_tile_whatever_torchs_default_type(gen):
+    """Their slabs are fp32, not of the type that new tensors have by default."""
+    from omnia_amd.models.projection import Parts, Projections
+
+    class Model(Projections):
+        device, dtype, tp, _ws = torch.device(DEV), torch.bfloat16, 1, {}
+
+    x, w = _rand(300, 8192, gen=gen), _rand(2048, 8192, std=0.05, gen=gen)
+    want = x.double() @ w.double().t()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        y = Model()._proj("down", x, w, False)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    assert isinstance(y, Parts) and y.t.dtype == torch.float32
+    # fp32 sums of K exact products: K roundings of at most 2^-24 of the sum of magnitudes
+    bound = 8192 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((y.t.double().sum(0) - want).abs() <= bound).all()
+
+
 def test_splitk_feeds_consumer(gen, schedule):
     """pgemm split-K slabs through splitk_swiglu == SwiGLU of the fp32 product."""
     M, F, K, S = 256, 512, 2048, 4
