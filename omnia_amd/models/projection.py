@@ -94,10 +94,15 @@ class Projections:
     # trickle (~256 decode rows + a few hundred prompt tokens) pgemm's 256x256
     # tiles leave most CUs idle, and the split decode / library path is 1.5x
     # faster per step (profiles/r5/mixed_open_loop/: p50 TPOT 14.9 vs 22.9 ms).
-    # Neither threshold holds gated projections off the tile where it fills the
-    # chip (ops.gated_tile_pays): in mixed steps too that is the faster one (8 layers
-    # of 4096 x 14336, 256 decode rows and 190 / 256 prompt rows 3.29 / 3.38 ms with
-    # it, 3.37 / 3.45 without; 16 of 2048 x 8192, 256 and 650 5.85 and 6.08)
+    # Neither threshold holds projections off the tile where it fills the chip
+    # (ops.gated_tile_pays, ops.plain_tile_fills), nor long-K ones off its slices
+    # (ops.tile_slices; OMNIA_MIDM=0 does): in mixed steps too that is the faster
+    # way (gated: 8 layers of 4096 x 14336, 256 decode rows and 190 / 256 prompt
+    # rows 3.29 / 3.38 ms with it, 3.37 / 3.45 without; 16 of 2048 x 8192, 256 and
+    # 650 5.85 and 6.08.  Plain and sliced: 8 layers of 4096 x 14336, 256 and 1280 /
+    # 2800 / 3700 6.00 / 10.46 / 12.56, without 6.01 / 10.44 / 12.74; 16 of 2048 x
+    # 8192, 256 and 650 / 1792 / 3700 4.46 / 6.32 / 10.54, without 4.60 / 6.45 /
+    # 10.68)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
 
     # ---- a few rows (ops.stream, ops.panel)
@@ -244,7 +249,9 @@ class Projections:
                 self._pgemm_covers(K, w.shape[0], is_decode):
             if ops.plain_tile_fills(M, w):
                 return ops.pgemm(0, x, w)
-            S = ops.tile_slices(M, w.shape[0], K) if slabs and w.is_contiguous() else 0
+            S = 0
+            if slabs and ops.midm_on() and w.is_contiguous():
+                S = ops.tile_slices(M, w.shape[0], K)
             if S:
                 out = torch.empty(S, M, w.shape[0], dtype=torch.float32, device=x.device)
                 return Parts(ops.pgemm_splitk(x, w, S, out, cols=128))

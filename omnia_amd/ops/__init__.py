@@ -268,6 +268,10 @@ _midm_table: dict | None = None
 _midm_on = os.environ.get("OMNIA_MIDM", "1") != "0"
 
 
+def midm_on() -> bool:
+    return _midm_on
+
+
 def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | None:
     """Mid-size projections (M = 257..4096 rows: open-loop mixed steps, which
     the unsplit 256x256 prefill tile under-fills): ``(256, PGEMM_SPLIT, S)``
