@@ -26,7 +26,8 @@ from ..ops import reference as ref
 from ..parallel import overlap
 from ..parallel import state as pstate
 from .config import ModelConfig
-from .projection import Parts, Projections, RowPar, packed_copy, version
+from .projection import (Parts, Projections, RowPar, packed_copy, shared_device,
+                         version)
 
 # decode attention: below this many (sequence, kv head) pairs a step splits every
 # live context on the device (``LlamaModel.decode_part``)
@@ -348,7 +349,7 @@ class LlamaModel(Projections):
         if T > Bd:
             ops.prefill_attention(q3[Bd:], kv.k[li], kv.v[li], fb.block_tables,
                                   fb.q_start_loc, fb.seq_lens, self.scale, fb.tile_seq,
-                                  fb.tile_q0, out=o[Bd:], shared_device=self._shared_device())
+                                  fb.tile_q0, out=o[Bd:], shared_device=shared_device(self))
         return o
 
     def decode_part(self, batch: int, max_ctx: int) -> tuple[int, int]:
@@ -388,7 +389,7 @@ class LlamaModel(Projections):
             return self._mixed_attention(li, q3, fb, kv)
         return ops.prefill_attention(q3, kv.k[li], kv.v[li], fb.block_tables, fb.q_start_loc,
                                      fb.seq_lens, self.scale, fb.tile_seq, fb.tile_q0,
-                                     shared_device=self._shared_device())
+                                     shared_device=shared_device(self))
 
     def _decode_ws(self, B, max_blocks, bs, device, part, splits=0):
         key = (B, max_blocks, bs, str(device), part, splits)

@@ -27,7 +27,7 @@ import torch
 from .. import ops
 from ..parallel import state as pstate
 from .llama import LlamaModel, _init
-from .projection import packed_experts
+from .projection import packed_experts, shared_device
 
 
 class MixtralModel(LlamaModel):
@@ -89,7 +89,7 @@ class MixtralModel(LlamaModel):
                        graph_safe=self.graph_safe or h.shape[0] < 64,
                        streams=packed_experts(self, layer["experts_gate_up"],
                                               layer["experts_down"]),
-                       shared_device=self._shared_device())
+                       shared_device=shared_device(self))
 
     def forward(self, fb, kv, gather: bool = True):
         # decode batches are captured into hipGraphs: keep the MoE path sync-free

@@ -81,6 +81,11 @@ def packed_experts(model, up: torch.Tensor, down: torch.Tensor):
     return None if t[0] is None or t[1] is None else t
 
 
+def shared_device(model) -> bool:
+    """Whether other ranks, whose all-reduce blocks may spin, run on this one's device."""
+    return model.tp > 1 and pstate.ranks_per_device() > 1
+
+
 class Projections:
     """Needs ``device``, ``dtype``, ``tp`` and ``_ws`` (workspace dict) on the model."""
 
@@ -270,10 +275,6 @@ class Projections:
                 and N % (256 if gated is None else 128) == 0
                 and (M >= self._min_rows or (gated is not None and ops.gated_tile_pays(M, gated))))
 
-    def _shared_device(self) -> bool:
-        """Whether other ranks, whose all-reduce blocks may spin, run on this one's device."""
-        return self.tp > 1 and pstate.ranks_per_device() > 1
-
     def _pgemm_covers(self, K: int, R: int, is_decode: bool) -> bool:
         # TP ranks rehearsed on ONE device (ipc transport) keep the library GEMMs:
         # a 256x256 tile's 160 KB of LDS cannot share a CU with the peers'
@@ -281,4 +282,4 @@ class Projections:
         # bound (the comm.hip error flag) -- real TP has one rank per GPU
         return (self.use_pgemm and not is_decode and K % 128 == 0 and R % 128 == 0
                 and self.device.type == "cuda" and self.dtype == torch.bfloat16
-                and not self._shared_device())
+                and not shared_device(self))
