@@ -632,26 +632,38 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   constexpr int WORDS = 4;
   const int lane = threadIdx.x & 63, most = p.M >> 8;
   bool light = false, ordered = MOE && SHAPE == WIDE && most <= 64 * WORDS && gridDim.x <= 9 * 256;
-  int half[WORDS];  // assignment 128 of segments 64 i + lane, asked for beside their number
+  // of segments 64 i + lane, asked for beside their number: assignment 128, and whether the segment
+  // before is of the same expert
+  int half[WORDS], expert[WORDS], last[WORDS];
   if constexpr (MOE && SHAPE == WIDE)
     if (ordered)
 #pragma unroll
       for (int i = 0; i < WORDS; ++i)
-        if (64 * i < most)
-          half[i] = p.sorted[(int64_t)min(64 * i + lane, most - 1) * 256 + 128];
+        if (64 * i < most) {
+          const int s = min(64 * i + lane, most - 1);
+          half[i] = p.sorted[(int64_t)s * 256 + 128];
+          expert[i] = p.blk_expert[s];
+          last[i] = p.blk_expert[s ? s - 1 : 0];
+        }
   const int ntn = p.N / TN, mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8;
   int first = 0, tiles = MOE ? mtn1 * ntn : gridDim.x, mtn = mtn1 * S;
   if (MOE && blockIdx.x >= tiles) return;
   // An expert's last segment may have 128 rows or fewer: light, half a tile.  All others come first,
   // so that the last round is of light ones (us before / now, 8 experts of 2048 x 4096: up at 1600
-  // tokens of two 136 / 117, 3000 208 / 193, down at 8192 263 / 239, 16384 458 / 421).  Up to 9 rounds:
-  // finding them takes 1 us a tile (up at 16384, 16.5 rounds, 893 / 905); not where they are few and
-  // the last round is short as it is, since apart from their expert's others they read its weights
-  // once more (up at 2001, one of 17, 157 / 163, in a step 160 / 168).
+  // tokens of two 136 / 115, 3000 203 / 189, down at 8192 262 / 234, 16384 458 / 421).  Up to 9 rounds:
+  // finding them takes 1 us a tile (up at 16384, 16.5 rounds, 893 / 905).
+  // Apart from their expert's others they read its weights once more: not from more than a fifth of
+  // all on (us without / with: up of 8 x 4096 x 4096 at 2400 tokens of two, 8 of 24 segments, 304 /
+  // 383; 8 x 2048 x 6144 at 1300, 8 of 16, 165 / 189; 64 x 2048 x 1024 at 3000 of six, 59 of 123, 226 /
+  // 281; 2 of 10 113 / 106, 200 / 198 and, of 4096 x 14336, 545 / 520), but where all tiles are one
+  // round (down of 8 x 2048 x 4096 at 1300, 8 of 16, 87 / 77; of 16 x 2048 x 2048 at 2400, 16 of 32,
+  // 58.5 / 51).  Nor where they are few, rounds are few and a tile is soon done (up at 2001, one of
+  // 17, 155 / 158; but K = 4096, up of 8 x 4096 x 4096 at 1600, one of 16, 250 / 219, down at 4096,
+  // three of 35, 268 / 254).  Over 160 such products the rule takes 0.7 % longer than the better of both.
   uint64_t pick[WORDS];
   if constexpr (MOE && SHAPE == WIDE) {
     if (ordered) {
-      int full = 0;
+      int full = 0, apart = 0;  // heavy segments, and light ones whose expert has a heavy one
       uint64_t heavy[WORDS];
 #pragma unroll
       for (int i = 0; i < WORDS; ++i) {
@@ -659,8 +671,14 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
                        ? __builtin_amdgcn_ballot_w64(64 * i + lane < mtn1 && half[i] < p.n_assign)
                        : 0;
         full += __popcll(heavy[i]);
+        if (64 * i < most)
+          apart += __popcll(__builtin_amdgcn_ballot_w64(
+              64 * i + lane > 0 && 64 * i + lane < mtn1 && half[i] >= p.n_assign &&
+              expert[i] == last[i]));
       }
-      ordered = p.K >= 4096 || 10 * (mtn1 - full) >= mtn1 || mtn1 * ntn >= 3 * 256;
+      ordered = mtn1 * ntn <= 256 ||
+                (5 * apart <= mtn1 &&
+                 (p.K >= 4096 || 10 * (mtn1 - full) >= mtn1 || mtn1 * ntn >= 3 * 256));
       light = ordered && blockIdx.x >= full * ntn;
       first = light ? full * ntn : 0;
       if (ordered) mtn = light ? mtn1 - full : full;

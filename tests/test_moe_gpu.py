@@ -309,3 +309,35 @@ def test_segments_of_few_rows(E, rows):
             a, b = (x[of].float() @ up[e].float().t()).split(I, 1)
             want = (torch.nn.functional.silu(a) * b) @ down[e].float().t() * wts[of, None]
             torch.testing.assert_close(y[0][of].float(), want, atol=2e-2, rtol=2e-2)
+
+
+def test_segments_of_few_rows_take_no_longer_than_full_ones():
+    """Apart from their expert's others, light segments read its weights once more, so many of them
+    stay where they are: 8 light segments of 24 against 24 full ones (1.26 times as long apart)."""
+    kk, dev, E, d, I = ops.kernels(), "cuda", 8, 4096, 4096
+    up = [torch.randn(E, 2 * I, d, device=dev, dtype=torch.bfloat16) * 0.02 for _ in range(2)]
+    runs = {}
+    for rows in (600, 768):
+        n = E * rows
+        ids = torch.arange(E, dtype=torch.int32, device=dev).repeat(rows).view(n, 1)
+        x = torch.randn(n, d, device=dev).to(torch.bfloat16)
+        mb = kk.moe_max_blocks(n, E, 256)
+        order = torch.empty(mb * 256, dtype=torch.int32, device=dev)
+        blk = torch.empty(mb, dtype=torch.int32, device=dev)
+        nb = torch.empty(1, dtype=torch.int32, device=dev)
+        kk.moe_align(order, blk, nb, ids, E, 0, E)
+        assert nb.item() == 24
+        act = torch.empty(mb * 256, I, device=dev, dtype=torch.bfloat16)
+        runs[rows] = lambda w, a=(x, order, blk, nb, n, act): kk.pgemm_moe(
+            0, a[5], a[0], w, *a[1:4], None, 1, a[4], 0)
+    best = {}
+    for _ in range(12):
+        for rows, run in runs.items():
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for w in up * 3:
+                run(w)
+            b.record()
+            torch.cuda.synchronize()
+            best[rows] = min(best.get(rows, 1e9), a.elapsed_time(b))
+    assert best[600] < 1.1 * best[768], best
