@@ -116,11 +116,13 @@ __global__ __launch_bounds__(256) void prep_kernel(
 }
 
 // Fast path (taps <= 4, head sizes up to 64 * VEC * NE, even when VEC = 2): a wave takes
-// a run of TR consecutive rows of one unit: 8, which reads 11 rows for 8, or of few rows 4, since
-// their time is the chain of a run (us in runs of 16 / 8 / 4, 16 heads of 128: 100 rows 15.1 / 9.3 /
-// 6.6, 999 17.8 / 12.9 / 12.3, 2000 21.5 / 19.0 / 22.4, 16384 141 / 134 / 165).  The raw inputs of
-// the run are loaded up front, the convolution slides over them in registers, and a sequence that
-// starts inside the run (or the run's own start) reloads the taps - 1 inputs before it.
+// a run of TR consecutive rows of one unit: 8, which reads 11 rows for 8, or 4 while the chip holds
+// the waves of all of them at once (32 a CU), since the time is then the chain of a run (us in runs of
+// 16 / 8 / 4, 32 units of 128 channels: 100 rows 13.5 / 8.8 / 6.3, 999 17.8 / 12.8 / 11.9, 1300 19.8 /
+// 15.1 / 17.1, 8000 69 / 66 / 80; 64 units: 333 16.0 / 11.2 / 9.4, 600 19.3 / 14.1 / 15.9, 999 21.2 / 20.0 /
+// 22.1; 128 units: 200 17.8 / 12.3 / 11.0, 333 20.0 / 15.4 / 17.0; 8 units: 4000 18 / 13 / 12.5).  The
+// raw inputs of the run are loaded up front, the convolution slides over them in registers, and a
+// sequence that starts inside the run (or the run's own start) reloads the taps - 1 inputs before it.
 template <typename T, int VEC>
 struct Vec;
 template <>
@@ -915,6 +917,7 @@ int prep(float* qn, float* kn, void* vc, float* decay, float* beta, const void* 
          Rows r, int T_, int KH, int H, int D, int Dp, int V, int taps, hipStream_t s) {
   const int big = D > V ? D : V, vec = (D % 2 || V % 2) ? 1 : 2, ne = (big + 64 * vec - 1) / (64 * vec);
   const unsigned uy = (2 * KH + H + 1 + 3) / 4;
+  const bool chain = (int64_t)T_ * (2 * KH + H) <= 4 * 32 * 256;  // runs of 4 at once
 #define OMNIA_PREP(VEC, NE, TAPS, TR)                                                           \
   do {                                                                                          \
     prep_run_kernel<T, VEC, NE, TAPS, TR><<<dim3((T_ + (TR) - 1) / (TR), uy), 256, 0, s>>>(         \
@@ -924,7 +927,7 @@ int prep(float* qn, float* kn, void* vc, float* decay, float* beta, const void* 
   } while (0)
 #define OMNIA_PREP_R(VEC, NE, TAPS)                           \
   do {                                                        \
-    if (r.q_start && T_ > 1200) OMNIA_PREP(VEC, NE, TAPS, 8); \
+    if (r.q_start && !chain) OMNIA_PREP(VEC, NE, TAPS, 8);    \
     else if (r.q_start) OMNIA_PREP(VEC, NE, TAPS, 4);         \
     else OMNIA_PREP(VEC, NE, TAPS, 1);                        \
   } while (0)

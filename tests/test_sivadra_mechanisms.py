@@ -259,8 +259,9 @@ def test_delta_rule(spec, how, run):
 def test_delta_prep_runs(dim, vdim):
     """Many rows go in runs of 8, few in runs of 4: the same bits, wherever sequences start."""
     lens = [1, 7, 8, 9, 3, 4, 5, 600, 331, 240, 2]
-    KH, H, taps, T = 2, 4, 4, sum(lens)
-    assert T > 1200
+    KH, H, taps, T = 8, 16, 4, sum(lens)
+    at_once = 4 * 32 * 256 // (2 * KH + H)  # rows up to which runs of 4 are
+    assert sum(lens[:8]) <= at_once < T
     C, dev, g = 2 * KH * dim + H * vdim, "cuda", gen(5)
     x = rnd(T, C + H * vdim + 2 * H, g=g).to(dev, torch.bfloat16)
     cw, conv = (rnd(*n, g=g).to(dev, torch.bfloat16) for n in ((C, taps), (len(lens), taps - 1, C)))
