@@ -45,10 +45,6 @@ def kernels():
 
             build(verbose=True)
             _ext = importlib.import_module("omnia_amd.ops._omnia_kernels")
-        # 0 or 1: named two main loops of the prefill GEMM, of which one is left
-        sched = os.environ.get("OMNIA_PGEMM_SCHED")
-        if sched is not None and hasattr(_ext, "pgemm_set_schedule"):
-            _ext.pgemm_set_schedule(int(sched))
     return _ext
 
 
@@ -529,9 +525,9 @@ def tile_slices(M: int, R: int, K: int) -> int:
 
 
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
-                 sched: int = 0, cols: int = 0) -> torch.Tensor:
+                 cols: int = 0) -> torch.Tensor:
     """Split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the MFMA tile of 256 rows and ``cols``
-    (128, else 256) columns (``csrc/pgemm.hip`` EPI 4; ``sched`` 0 or 1, of no effect).  Each
+    (128, else 256) columns (``csrc/pgemm.hip`` EPI 4, 11).  Each
     slab is one K-slice's fp32 sum, saturated to fp16 unless ``out`` is fp32; the splitk consumers
     reduce them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip)."""
     M, K = x.shape
@@ -539,7 +535,7 @@ def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tenso
     if out is None:
         out = torch.empty(splits, M, N, dtype=torch.float16, device=x.device)
     if x.is_cuda:
-        kernels().pgemm_splitk(out, x.contiguous(), w, sched, 128 if cols == 128 else 256)
+        kernels().pgemm_splitk(out, x.contiguous(), w, 128 if cols == 128 else 256)
         return out
     ks = K // splits
     for s in range(splits):

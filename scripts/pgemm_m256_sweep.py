@@ -102,28 +102,26 @@ def main():
                             p = ops.wgemm(2, x, nxt(), S, bn, nwv, out=parts)
                         consume(p)
                 out[f"table:{cfg}"] = timeit(fn)
-            for sched in (0, 1):
-                for S in (1, 2, 3, 4, 6, 7, 8, 12, 14, 16):
-                    if K % S or (K // S) % 128:
-                        continue
-                    nblk = (N // 256) * S
-                    if nblk > 2048:
-                        continue
-                    parts = torch.empty(S, M, N, device=dev, dtype=torch.float16)
-                    ops.pgemm_splitk(x, ws[0], S, parts, sched)
-                    torch.cuda.synchronize()
-                    err = (parts.float().sum(0) - exact).abs().max().item() / scale
-                    if err > 2e-2:
-                        print(f"  BAD {name} M{M} S{S} sched{sched} rel err {err:.3g}", flush=True)
-                        out[f"pgemm:s{sched}:S{S}:BAD"] = err
-                        continue
+            for S in (1, 2, 3, 4, 6, 7, 8, 12, 14, 16):
+                if K % S or (K // S) % 128:
+                    continue
+                nblk = (N // 256) * S
+                if nblk > 2048:
+                    continue
+                parts = torch.empty(S, M, N, device=dev, dtype=torch.float16)
+                ops.pgemm_splitk(x, ws[0], S, parts)
+                torch.cuda.synchronize()
+                err = (parts.float().sum(0) - exact).abs().max().item() / scale
+                if err > 2e-2:
+                    print(f"  BAD {name} M{M} S{S} rel err {err:.3g}", flush=True)
+                    out[f"pgemm:S{S}:BAD"] = err
+                    continue
 
-                    def fn(S=S, sched=sched, parts=parts):
-                        consume(ops.pgemm_splitk(x, nxt(), S, parts, sched))
-                    out[f"pgemm:s{sched}:S{S}"] = timeit(fn)
-                    out[f"pgemm:s{sched}:S{S}:noconsumer"] = timeit(
-                        lambda S=S, sched=sched, parts=parts: ops.pgemm_splitk(x, nxt(), S, parts,
-                                                                               sched))
+                def fn(S=S, parts=parts):
+                    consume(ops.pgemm_splitk(x, nxt(), S, parts))
+                out[f"pgemm:S{S}"] = timeit(fn)
+                out[f"pgemm:S{S}:noconsumer"] = timeit(
+                    lambda S=S, parts=parts: ops.pgemm_splitk(x, nxt(), S, parts))
             if name == "gate_up" and M > 0:  # the fused-SwiGLU prefill tile, unsplit
                 act = torch.empty(M, I, device=dev, dtype=torch.bfloat16)
                 out["pgemm:epi1"] = timeit(lambda: ops.pgemm(1, x, nxt(), out=act))

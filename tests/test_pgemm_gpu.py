@@ -24,17 +24,6 @@ def _close(got, want, tol):
     return err <= tol * scale, err / max(scale, 1e-30)
 
 
-@pytest.fixture(autouse=True, params=[0, 1], ids=["8wave", "4wave"])
-def schedule(request):
-    """Every check runs on both main loops: the 8-wave ping-pong and the 4-wave
-    one-wave-per-SIMD schedule (same epilogues)."""
-    if not torch.cuda.is_available():
-        pytest.skip("no GPU")
-    ops.kernels().pgemm_set_schedule(request.param)
-    yield request.param
-    ops.kernels().pgemm_set_schedule(0)
-
-
 @pytest.fixture(scope="module")
 def gen():
     if not torch.cuda.is_available():
@@ -153,41 +142,38 @@ def test_rejects_bad_shapes(gen):
         ops.pgemm(0, x, w, out=torch.empty(256, 256, dtype=torch.bfloat16, device=DEV))
 
 
-@pytest.mark.parametrize("epi", [0, 1, 2])
-def test_schedules_are_bit_identical(gen, schedule, epi):
-    """Both main loops accumulate every output element over K in the same order
-    with the same instruction: identical bits, ragged M included."""
-    M, K = 777, 1024
-    N = 512
-    x = _rand(M, K, gen=gen)
+@pytest.mark.parametrize("epi,cols", [(0, 128), (0, 256), (1, 128), (1, 256), (2, 256)])
+def test_a_rows_bits_are_its_own(gen, epi, cols):
+    """A row's result does not depend on how many rows the step has, on where in the step it lies, or
+    on the run."""
+    K, N = 1024, 512
+    x = _rand(777, K, gen=gen)
     w = _rand(2 * N if epi == 1 else N, K, std=0.05, gen=gen)
-    ss = torch.rand(M, 2, device=DEV, generator=gen) * K
-    outs = []
-    for sched in (0, 1):
-        ops.kernels().pgemm_set_schedule(sched)
+    ss = torch.rand(777, 2, device=DEV, generator=gen) * K
+    res = _rand(777, N, gen=gen)
+
+    def run(a, b):
         if epi == 2:
-            o = _rand(M, N, gen=torch.Generator(device=DEV).manual_seed(5))
-            sso = torch.zeros(M, N // 256, device=DEV)
-            ops.pgemm(2, x, w, out=o, ss_out=sso)
-            outs.append((o, sso))
-        else:
-            o = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
-            ops.pgemm(epi, x, w, out=o, ss_in=ss, inv_d=1.0 / K, eps=1e-5)
-            outs.append((o,))
-    ops.kernels().pgemm_set_schedule(schedule)
-    for a, b in zip(*outs):
-        assert torch.equal(a, b)
+            o, sso = res[a:b].clone(), torch.zeros(b - a, N // 256, device=DEV)
+            ops.pgemm(2, x[a:b], w, out=o, ss_out=sso)
+            return o, sso
+        return (ops.pgemm(epi, x[a:b], w, ss_in=ss[a:b], inv_d=1.0 / K, eps=1e-5, cols=cols),)
+
+    whole = run(0, 777)
+    for a, b in ((0, 777), (0, 1), (255, 258), (300, 777)):
+        for got, want in zip(run(a, b), whole):
+            assert torch.equal(got, want[a:b])
 
 
 @pytest.mark.parametrize("M,N,K,S", [(256, 512, 1024, 4), (192, 768, 2048, 8), (77, 256, 512, 2),
                                      (300, 512, 896, 7)])
-def test_splitk_slabs(gen, schedule, M, N, K, S):
+def test_splitk_slabs(gen, M, N, K, S):
     """EPI 4: fp16 slab s holds x[:, Ks] @ w[:, Ks]^T of K-slice s; decode sizes
     (one m-tile, ragged) and prefill sizes (two m-tiles) against fp32 matmuls."""
     x = _rand(M, K, gen=gen)
     w = _rand(N, K, std=0.05, gen=gen)
     parts = torch.full((S, M, N), float("nan"), dtype=torch.float16, device=DEV)
-    ops.pgemm_splitk(x, w, S, parts, schedule)
+    ops.pgemm_splitk(x, w, S, parts)
     ks = K // S
     for s in range(S):
         want = x[:, s * ks:(s + 1) * ks].float() @ w[:, s * ks:(s + 1) * ks].float().t()
@@ -201,15 +187,15 @@ def test_splitk_slabs(gen, schedule, M, N, K, S):
     assert not _close(parts[S - 1], want0, 2e-3)[0]
 
 
-def test_splitk_saturates_fp16(gen, schedule):
+def test_splitk_saturates_fp16(gen):
     """A K-slice partial beyond the fp16 range saturates to +-65504 (finite), so
-    the consumer never sees inf / NaN (unclamped casts)."""
+    the consumer never sees inf / NaN."""
     M, N, K, S = 256, 256, 512, 2
     x = torch.full((M, K), 16.0, dtype=torch.bfloat16, device=DEV)
     w = torch.full((N, K), 16.0, dtype=torch.bfloat16, device=DEV)  # partial = 256*256 = 65536
     w[: N // 2] = -16.0
     parts = torch.empty(S, M, N, dtype=torch.float16, device=DEV)
-    ops.pgemm_splitk(x, w, S, parts, schedule)
+    ops.pgemm_splitk(x, w, S, parts)
     assert torch.isfinite(parts).all()
     assert (parts[:, :, N // 2:] == 65504).all() and (parts[:, :, : N // 2] == -65504).all()
 
@@ -261,12 +247,12 @@ def test_slices_of_the_narrow_tile_whatever_torchs_default_type(gen):
     assert ((y.t.double().sum(0) - want).abs() <= bound).all()
 
 
-def test_splitk_feeds_consumer(gen, schedule):
+def test_splitk_feeds_consumer(gen):
     """pgemm split-K slabs through splitk_swiglu == SwiGLU of the fp32 product."""
     M, F, K, S = 256, 512, 2048, 4
     x = _rand(M, K, gen=gen)
     w = _rand(2 * F, K, std=0.05, gen=gen)
-    act = ops.splitk_swiglu(ops.pgemm_splitk(x, w, S, sched=schedule))
+    act = ops.splitk_swiglu(ops.pgemm_splitk(x, w, S))
     h = (x.float() @ w.float().t()).to(torch.bfloat16).float()
     want = torch.nn.functional.silu(h[:, :F]) * h[:, F:]
     ok, e = _close(act, want, 2e-2)
@@ -278,12 +264,12 @@ def test_splitk_rejects_bad_split(gen):
     w = _rand(256, 1024, gen=gen)
     with pytest.raises(RuntimeError):  # K / S = 341.33
         ops.pgemm_splitk(x, w, 3)
-    with pytest.raises(RuntimeError):  # K / S = 64: not whole iterations of two K-tiles
+    with pytest.raises(RuntimeError):  # K / S = 64: an odd number of K-tiles
         ops.pgemm_splitk(x, w, 16)
 
 
 @pytest.mark.parametrize("hq,hkv", [(8, 1), (4, 1), (6, 1)])
-def test_qkv_epilogue_tp_shard_heads(gen, schedule, hq, hkv):
+def test_qkv_epilogue_tp_shard_heads(gen, hq, hkv):
     """TP shards' QKV: one KV head per rank (Llama-3-70B at TP=8: hq 8, hkv 1 ->
     10 heads = 5 tiles) -- 256-column tiles straddle the q / k / v boundaries;
     the per-head epilogue still routes q, k and v correctly."""
