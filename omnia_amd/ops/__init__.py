@@ -492,15 +492,17 @@ def gated_tile_pays(M: int, w: torch.Tensor) -> bool:
 
 def plain_tile_fills(M: int, w: torch.Tensor) -> bool:
     """Whether an ungated :func:`pgemm` of more rows than the panel kernel takes covers ``w`` and
-    beats the library: from nine tenths of its tiles' work useful (useful part, us here /
-    library: 4096 x 2048 at 1536 rows .75 28.9 / 29.3, 2001 .98 30.6 / 34.6; 4096 x 4096 at 1536 .75
-    52.0 / 51.6, 2001 .98 55 / 60; 4096 x 14336 at 1536 .75 180 / 176, 2001 .98 194 / 204; 2048 x
-    2048 at 2001 .49 27.1 / 23.8)."""
+    beats the library: one round of narrow tiles with nine tenths of their work useful (useful part,
+    us here / library: 4096 x 2048 at 1536 rows .75 28.9 / 29.3, 2001 .98 30.6 / 34.6; 4096 x 4096 at
+    1536 .75 52.0 / 51.6, 2001 .98 55 / 60; 4096 x 14336 at 1536 .75 180 / 176, 2001 .98 194 / 204;
+    2048 x 2048 at 2001 .49 27.1 / 23.8).  Over 28 such sizes the library takes 1.02 to 1.14 as long;
+    over 32 of three narrow rounds .86 to 1.6, most of them less (15360 x 5120 at 1448 rows 216 /
+    192), over 18 of one wide round .95 to 1.04."""
     if M <= PANEL_MAX_M or w.dim() != 2:
         return False
     R, K = w.shape
     return K % 128 == 0 and R % 256 == 0 and _tiles_useful(M, R) > 0.9 and \
-        w.is_contiguous() and _on_grid(w)
+        tile_cols(M, R) == 128 and _tile_rounds(M, R, 128) == 1 and w.is_contiguous() and _on_grid(w)
 
 
 @functools.lru_cache(maxsize=8192)

@@ -84,6 +84,17 @@ def test_gated_projections_on_both_sides_of_the_rule(M, N, K, pays):
     assert not Model()._pgemm_ok(M, K, N, True, w)
 
 
+@pytest.mark.parametrize("M,R,K,fills", [
+    (1843, 4096, 2048, False), (1844, 4096, 2048, True), (2048, 4096, 2048, True),  # .9 of a round
+    (2049, 4096, 2048, False),                                           # nine rows of tiles
+    (1024, 8192, 1024, True), (1024, 8192 + 128, 1024, False), (1024, 8192, 1024 + 64, False),
+    (1449, 16128, 11392, False), (1014, 23808, 1024, False),             # three narrow rounds
+    (1001, 15872, 14208, False), (2048, 8192, 2048, False)])             # one wide one
+def test_plain_projections_on_both_sides_of_the_rule(M, R, K, fills):
+    w = torch.empty(R, K, dtype=torch.bfloat16, device="meta")
+    assert ops.plain_tile_fills(M, w) == fills
+
+
 def test_down_tile_cols():
     """Narrow while the segments to be expected are one round of narrow tiles, half of each expert's
     last one empty; of a shard's experts, their part of the assignments."""
