@@ -104,10 +104,8 @@ class Projections:
     # (ops.tile_slices; OMNIA_MIDM=0 does): in mixed steps too that is the faster
     # way (gated: 8 layers of 4096 x 14336, 256 decode rows and 190 / 256 prompt
     # rows 3.29 / 3.38 ms with it, 3.37 / 3.45 without; 16 of 2048 x 8192, 256 and
-    # 650 5.85 and 6.08.  Plain and sliced: 8 layers of 4096 x 14336, 256 and 1280 /
-    # 2800 / 3700 6.00 / 10.46 / 12.56, without 6.01 / 10.44 / 12.74; 16 of 2048 x
-    # 8192, 256 and 650 / 1792 / 3700 4.46 / 6.32 / 10.54, without 4.60 / 6.45 /
-    # 10.68)
+    # 650 5.85 and 6.08.  Plain and sliced: 16 of 2048 x 8192, 256 and 250 / 650 /
+    # 1792 / 3700 3.65 / 4.39 / 6.23 / 10.30, without 3.73 / 4.49 / 6.34 / 10.44)
     PGEMM_MIXED_MIN_ROWS = int(os.environ.get("OMNIA_PGEMM_MIXED_MIN_ROWS", "4096"))
 
     # ---- a few rows (ops.stream, ops.panel)

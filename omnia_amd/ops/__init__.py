@@ -515,8 +515,11 @@ def tile_slices(M: int, R: int, K: int) -> int:
     (us with the consumer, library / here, rows of 2048 x 8192: 257 40.7 / 31.4, 512 41.9 / 35.0,
     768 50.5 / 43.2, 999 62.5 / 48.9, 1536 71.2 / 71.9 not taken, 2001 88.7 / 77.4; 4096 x 8192:
     512 61 / 51, 768 71 / 73 not taken; 2048 x 16384: 999 101 / 73; 2048 x 4096: 257 27.6 / 24.3,
-    999 37.4 / 36.2 not taken)."""
-    if M <= PANEL_MAX_M or M > 2048 or R % 128 or K % 128:
+    999 37.4 / 36.2 not taken).  That model of the library is one of 2048 rows of weights and more;
+    of fewer it is faster up to K of some 5000 (1280 x 2304 at 308 rows 13.0 / 18.7, 1024 x 4608 at 432
+    18.3 / 23.1, 1536 x 5120 at 257 21.9 / 24.3, but 1024 x 6144 at 257 23.4 / 21.4, 8192 at 400 28.1 /
+    25.0)."""
+    if M <= PANEL_MAX_M or M > 2048 or R % 128 or K % 128 or (R < 2048 and K < 6144):
         return 0
     tiles, best = -(-M // 256) * (R // 128), (0.9 * (9.0 + 1.9e-3 * K + 2 * M * R * K / 1.35e9), 0)
     for S in range(2, 17):

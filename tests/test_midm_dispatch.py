@@ -46,13 +46,14 @@ def test_slices_of_the_narrow_tile_fit_the_kernel():
     the prefill rows, and only where it takes a tenth less than the library by their models."""
     taken = 0
     for M in (1, 256, 257, 512, 999, 2001, 2048, 2049, 5000):
-        for R in (128, 256, 1000, 2048, 4096, 16384):
-            for K in (128, 1000, 2048, 4096, 8192, 14336, 16384):
+        for R in (128, 256, 1000, 1024, 1536, 2048, 4096, 16384):
+            for K in (128, 1000, 2048, 4096, 5120, 6144, 8192, 14336, 16384):
                 S = ops.tile_slices(M, R, K)
                 if S:
                     taken += 1
                     assert 256 < M <= 2048 and R % 128 == 0 and K % (128 * S) == 0
                     assert S > 1 and -(-M // 256) * (R // 128) * S <= 256
+                    assert R >= 2048 or K >= 6144  # below, the library is faster
     assert taken and ops.tile_slices(999, 2048, 8192) == 4 and not ops.tile_slices(999, 2048, 2048)
 
 
