@@ -59,12 +59,13 @@ __device__ __forceinline__ int decode_part_len(int len, int cap, int split_t, in
 // 127 -> 119 (5.1 TB/s), 128 x 1000 111 -> 104, 64 x 2000 115 -> 112, 32 x 1000 33.7 -> 29.3,
 // 4 x 1000 15.3 -> 12.4, 256 x 150 38.2 -> 37.0.  Of
 // sequences that share the pages of a prompt prefix a block finds in the caches what another has
-// read; K and V that nobody shares go past them (non-temporal).  us through the caches and by
-// this rule: 256 x 576 107 -> 102.5, 128 x 1000 93.6 -> 81.8, 64 x 2000 91 -> 80, 512 x 600 212 ->
-// 200; 512 of 256 x 576 shared by all 55.2 -> 55, by sequences 32 apart 54 -> 55.9 (past the caches
-// 76), 896 of 128 x 1000 44.8 -> 44.4 and 45 -> 46.7 (59, 66); 256 x 150, below it, 33 (past 35.5);
-// 32 x 1000 in a step 29.4 -> 27.4, 8 x 1000 in partitions of 256 15.5 -> 14.7, 4 x 1000, of 128 and
-// below it, 11.2 (past, with the look, 12.1).
+// read; K and V that nobody shares go past them (non-temporal) where many long sequences make
+// bandwidth the bound.  us through the caches and past them, out of 1.2 GB and more: 256 x 576 109 /
+// 106, 256 x 768 148 / 131, 128 x 1000 96 / 86, 64 x 2000 96 / 85, 32 x 1000 26.2 / 23.9; lengths
+// from half up to 600 64 x 27.2 / 28.6, to 800 33.7 / 33.7, to 1000 43.6 / 40.8; in partitions 16 x
+// 1500 27.3 / 27.2, 8 x 900 13.2 / 13.6.  By the rule: 512 of 256 x 576 shared by all 55.2 -> 55, by
+// sequences 32 apart 54 -> 55.9 (past the caches 76), 896 of 128 x 1000 44.8 -> 44.4 and 45 -> 46.7
+// (59, 66).
 constexpr int NW = 4;
 template <int G>
 struct DecodeShared {
@@ -274,21 +275,38 @@ __global__ __launch_bounds__(64 * NW, G < 8 ? 3 : 2) void decode_attn_kernel(
   const int pl = decode_part_len(len, part_size, split_t, split_min, BS);
   const int p0 = part * pl;
   if (p0 >= len) return;
-  // past the caches: of a long sequence what no other has the page of, 64 keys into the partition (a
-  // row's entries past its length may be anything: at worst the caches are used).  What shares less
-  // is read again for less than is gained.  Sharers may be anywhere in the batch, so the block's
-  // threads look at all of it, a row each; up to 64 rows every wave for itself, without a barrier
+  // Past the caches, where bandwidth is the bound: blocks enough without partitions, two thirds of
+  // the sequences long (few long ones are waited for, and such loads come later), and of a long one
+  // what no other has the page of, 64 keys into the partition (a row's entries past its length may
+  // be anything: at worst the caches are used).  What shares less is read again for less than is
+  // gained.  Sharers may be anywhere in the batch, so the block's threads look at all of it, a row
+  // each; up to 64 rows every wave for itself, without a barrier
   constexpr int LONG = 512;
-  if (len >= LONG && min(pl, len - p0) >= 192 && gridDim.x > 1) {
-    const int B = gridDim.x, *t = block_tables + min(p0 + 64, len - 1) / BS;
+  const int B = gridDim.x;
+  if (len >= LONG && min(pl, len - p0) >= 192 && B * gridDim.y >= 256) {
+    const bool alone = B <= 64;
+    const int me = alone ? threadIdx.x & 63 : threadIdx.x, step = alone ? 64 : 64 * NW;
+    const int* t = block_tables + min(p0 + 64, len - 1) / BS;
     const int own = t[(int64_t)b * bt_stride];
-    bool same = false;
-    for (int i = B <= 64 ? threadIdx.x & 63 : threadIdx.x; i < B; i += 128 * NW) {
-      const int j = min(i + 64 * NW, B - 1);
-      const int x = t[(int64_t)i * bt_stride], y = t[(int64_t)j * bt_stride];
-      same |= (x == own && i != b) || (y == own && j != b);
+    int votes = 0;
+    uint64_t same = 0;
+#pragma unroll 2
+    for (int i0 = 0; i0 < B; i0 += step) {
+      const int i = min(i0 + me, B - 1), n = i0 + me < B ? seq_lens[i] : 0;
+      same |= __builtin_amdgcn_ballot_w64(t[(int64_t)i * bt_stride] == own && i != b);
+      votes += __popcll(__builtin_amdgcn_ballot_w64(n >= LONG)) -
+               2 * __popcll(__builtin_amdgcn_ballot_w64(n > 0 && n < LONG));
     }
-    if (B <= 64 ? __builtin_amdgcn_ballot_w64(same) == 0 : !__syncthreads_or(same)) {
+    if (same) votes = -(1 << 28);
+    if (!alone) {
+      __shared__ int look[NW];
+      if ((threadIdx.x & 63) == 0) look[threadIdx.x >> 6] = votes;
+      __syncthreads();
+      votes = 0;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) votes += look[i];
+    }
+    if (votes >= 0) {
       decode_block<G, BS, true>(sh, len, pl, out, part_o, part_ml, q, kc, vc, block_tables,
                                 bt_stride, hkv, q_stride, max_parts, scale_log2);
       return;

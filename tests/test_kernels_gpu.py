@@ -399,6 +399,34 @@ def test_decode_attention_past_and_through_the_caches(lens, hq, bs, part, splits
     assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
 
 
+@pytest.mark.parametrize("B,hkv,hq", [(64, 4, 4), (64, 4, 32), (65, 4, 16), (128, 2, 8), (300, 1, 2)])
+@pytest.mark.parametrize("short", [0, 0.25, 0.5])
+def test_decode_attention_of_batches_past_the_caches(B, hkv, hq, short):
+    """Blocks enough without partitions: where two thirds of the sequences are long, long ones that
+    share no page go past the caches, looked for by a wave up to 64 rows and by the block beyond;
+    empty rows are none."""
+    torch.manual_seed(15)
+    bs, g = 32, torch.Generator().manual_seed(B)
+    lens = torch.randint(512, 900, (B,), generator=g)
+    lens[torch.rand(B, generator=g) < short] = 70
+    lens[3::17] = 0
+    n = [int(x) for x in lens]
+    nb_total = sum(-(-x // bs) for x in n) + 8
+    kc, vc = _make_cache(nb_total, hkv, bs, seed=15)
+    bt = _tables([max(x, 1) for x in n], bs, nb_total + B)
+    bt %= nb_total
+    for i in range(0, B - 40, 9):  # 40 rows apart
+        k = min(n[i], n[i + 40], 256) // bs
+        bt[i + 40, :k] = bt[i, :k]
+    sl = lens.int().to(DEV)
+    q = torch.randn(B, hq, 128, device=DEV, dtype=torch.bfloat16)
+    out = ops.decode_attention(q, kc, vc, bt, sl, 128 ** -0.5, part_size=1024)
+    live = (sl > 0).nonzero().view(-1)
+    exp = _attention64(q[live], kc, vc, bt[live], [1] * len(live), [x for x in n if x], 128 ** -0.5)
+    err = (out[live].double() - exp).abs()
+    assert (err <= exp.abs() * 2.0 ** -8 + 1e-4).all(), err.max()
+
+
 def test_decode_attention_finds_sharers_far_apart():
     """Prompt prefixes shared by sequences 32 rows apart: the sums are right, and the shared pages go
     through the caches as those of neighbours do (past them 1.4 times as long)."""
