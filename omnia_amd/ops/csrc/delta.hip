@@ -613,256 +613,305 @@ __global__ __launch_bounds__(256) void blocks_kernel(float* __restrict__ rec,
   }
 }
 
-// grid (ceil(Vs / 64), H, nseq), 4 waves: wave w owns state columns 64 x + 16 w + ..15
-// as ND accumulator tiles (key dimensions 16 j + 4 (lane >> 4) + r in register r).  The
-// accumulator layout serves as the B operand of the next product as it stands: k-step r
-// takes dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.
-// Bound by its serial chain: a block is 104 fp32 products of one wave (heads of 128), 1.4 of the
-// 3.0 us that it takes in a step, and a SIMD has one wave.  Vector instructions add to that, so
-// registers hold 2 waves' worth (with more, hipcc keeps S in the accumulators' file and moves it
-// back and forth), offsets are made once, and what is not a product goes between products.  16
-// heads of 128 in a model step, whose weights leave no operand in the caches: 2048 rows of 8
-// sequences 430 -> 381 us (blocks_kernel 66 beside it, as before), 333 of 3 65 -> 59.  Alone and
-// repeated, both kernels 371 -> 330 and 68 -> 61.
-template <typename T, int ND>
-__global__ __launch_bounds__(256, ND <= 8 ? 2 : 1) void scan_blocks_kernel(
+// Rows of a tensor as a buffer: reads past ``bytes`` give 0, writes there do nothing.
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+constexpr uint32_t kOut = 0x80000000u;  // a lane's offset past every buffer
+
+__device__ __forceinline__ Rsrc buffer(const void* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ float4v load4(Rsrc b, uint32_t off) {
+  return __builtin_bit_cast(float4v, (uint4v)__builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
+}
+__device__ __forceinline__ float load1(Rsrc b, uint32_t off) {
+  return __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(b, off, 0, 0));
+}
+__device__ __forceinline__ void store1(float v, Rsrc b, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), b, off, 0, 0);
+}
+
+template <int N>
+struct Int {
+  static constexpr int value = N;
+};
+
+// One block's operands in LDS.
+template <int ND, int CW>
+struct ScanBuf {
+  static constexpr int KS = 16 * ND + 4, TS = 20;
+  float k[16 * KS], q[16 * KS], t[16 * TS], p[16 * TS], g[32], v[16 * CW * TS];
+};
+// Two of them: the compute waves read all of a block's between two barriers, while the next
+// block's are written over what they read before.  ks, os: parts of K S and of the output.
+template <int ND, int NW, int CW>
+struct ScanShared {
+  ScanBuf<ND, CW> buf[2];
+  float4v ks[2][CW][NW][64], os[2][CW][NW][64];
+};
+
+// grid (ceil(Vs / (16 CW)) x H, nseq), CW x NW waves that multiply and 4 that move operands and
+// outputs.  The former own 16 state columns each (cw) and share the key dimensions: wave w of NW has
+// NJ = ND / NW accumulator tiles (key dimensions 16 (w NJ + j) + 4 (lane >> 4) + r in register r).
+// The accumulator layout serves as the B operand of the next product as it stands: k-step r takes
+// dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.  Their parts of K S
+// meet in LDS, added by all in one order, so that all hold the same u; parts of the output are
+// added by the moving waves, a block later.
+// Bound by the serial chain of a block where few blocks run: K S, the exchange, T', K^T U, 20 of a
+// wave's 29 fp32 products (13.3 ns each) and the latencies between them.  A wave issues an
+// instruction in about 5 clocks and none beside its own products, so whatever is not on the chain
+// is another wave's work: with the staging in the multiplying waves the 16 heads of 4000 rows below
+// took 262 us, with operands straight from global memory 282.  Where the chip is full, fp32
+// products and vector instructions share one unit: 112 products a block of 32 columns, 1.5 of 2.1 us.
+// us with blocks_kernel (heads of 128), one wave a 16 columns and all of their key dimensions ->
+// now: 16 heads, 77 rows 23 -> 14, 4000 547 -> 184, 1000 and 1500 216 -> 86, 333 of 3 61 -> 38, 60
+// of 16 37 -> 36, 512 of 32 315 -> 318, 2048 of 8 356 -> 327; 32 heads, 333 of 3 67 -> 60.
+template <typename T, int ND, int NW, int CW>
+__global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan_blocks_kernel(
     float* __restrict__ o, float* __restrict__ state, T* __restrict__ conv_state,
     const float* __restrict__ rec, const float* __restrict__ qn, const float* __restrict__ kn,
     const T* __restrict__ vc, const T* __restrict__ x, int64_t ldx, Rows rows, int KH, int H,
     int D, int Dp, int V, int Vs, int taps) {
-  constexpr int DW = 16 * ND, KS = DW + 4, TS = 20;
-  constexpr int NL = (16 * DW / 4 + 255) / 256;  // float4 per thread of one operand block
-  // one block's operands; two of them, so the next block is written while this is read
-  struct Buf {
-    float k[16 * KS], q[16 * KS], t[16 * TS], p[16 * TS], g[32];
-  };
-  __shared__ __attribute__((aligned(16))) Buf buf[2];
-  const int h = blockIdx.y, s = blockIdx.z, tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6, c16 = lane & 15, g4 = lane >> 4;
-  const int col = blockIdx.x * 64 + 16 * w + c16;
+  constexpr int NJ = ND / NW, PR = 4 / NW, CN = NW * CW;
+  using Buf = ScanBuf<ND, CW>;
+  constexpr int KS = Buf::KS, TS = Buf::TS;
+  static_assert(NJ * NW == ND && (NW == 2 || NW == 4), "tiles of a wave");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  ScanShared<ND, NW, CW>& sh = *reinterpret_cast<ScanShared<ND, NW, CW>*>(lds);
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // neighbours, which read the same keys and queries, on one XCD
+  const int nx = (Vs + 16 * CW - 1) / (16 * CW), bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int bx = bid % nx, h = bid / nx, s = blockIdx.y;
   const int row0 = rows.q_start[s], n = rows.q_start[s + 1] - row0;
   const int slot = rows.slots[s];
   if (n <= 0 || slot < 0) return;
   const bool fresh = rows.positions[row0] == 0;
-  const int C = 2 * KH * D + H * V, kh = h / (H / KH);
-  float* Sg = state + (((int64_t)slot * H + h) * D) * Vs + col;
-  float4v S[ND];
-#pragma unroll
-  for (int j = 0; j < ND; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = 16 * j + 4 * g4 + r;
-      S[j][r] = (!fresh && d < D && col < Vs) ? Sg[(int64_t)d * Vs] : 0.f;
-    }
-  // this thread's share of a block: element e of [16][DW / 4] float4s
-  float4v kreg[NL], qreg[NL];
-  T vreg[4];
-  float treg[2], greg;
-  // Vector instructions do not run beside the fp32 products, so addresses are a uniform base and
-  // an offset made once.  Loads are unconditional, so that they all are in flight together: rows
-  // past the end re-read the last one (their u is 0 whatever k, q and v hold) and columns past
-  // the head re-read its last ones (zeroed when they are used).
-  const float* R = rec + ((int64_t)rec_base(rows.q_start, s) * H + h) * kRec;
-  const int64_t kofs = ((int64_t)row0 * KH + kh) * Dp;
-  const T* vp = vc + ((int64_t)row0 * H + h) * V;
-  const int64_t kstep = (int64_t)16 * KH * Dp, vstep = (int64_t)16 * H * V;
-  const int kd4 = tid % (DW / 4) * 4, vcol = min(col, V - 1);
-  uint32_t koff[NL], voff[4];
-  auto offsets = [&](int last) {
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
-      koff[i] = min((i * 256 + tid) / (DW / 4), last) * KH * Dp + min(kd4, Dp - 4);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) voff[r] = min(4 * g4 + r, last) * H * V + vcol;
-  };
-  auto gload = [&](int bi) {
-    const float* kb = kn + kofs + bi * kstep;
-    const float* qb = qn + kofs + bi * kstep;
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      kreg[i] = *reinterpret_cast<const float4v*>(kb + koff[i]);
-      qreg[i] = *reinterpret_cast<const float4v*>(qb + koff[i]);
-    }
-    const T* vb = vp + bi * vstep;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) vreg[r] = vb[voff[r]];
-    const float* rr = R + (int64_t)bi * H * kRec;
-    treg[0] = rr[(uint32_t)tid];
-    treg[1] = rr[256 + (uint32_t)tid];
-    greg = rr[512 + (uint32_t)(tid & 31)];
-  };
-  auto lwrite_rows = [&](Buf& b) {  // k columns past Dp hold zeros from the start
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int tt = (i * 256 + tid) / (DW / 4);
-      if (kd4 < Dp && (16 * DW / 4 % 256 == 0 || tt < 16)) {
-        *reinterpret_cast<float4v*>(b.k + tt * KS + kd4) = kreg[i];
-        *reinterpret_cast<float4v*>(b.q + tt * KS + kd4) = qreg[i];
-      }
-    }
-  };
-  auto lwrite_rest = [&](Buf& b) {
-    b.t[(tid >> 4) * TS + (tid & 15)] = treg[0];
-    b.p[(tid >> 4) * TS + (tid & 15)] = treg[1];
-    b.g[tid & 31] = greg;
-  };
   const int nblk = (n + 15) / 16;
-  float* op = o + ((int64_t)row0 * H + h) * Vs;
-  const uint32_t ooff = 4 * g4 * H * Vs + col;
-  const int64_t ostep = (int64_t)16 * H * Vs;
-  // Operands in registers ahead of their products (heads up to 128; wider ones read LDS as they
-  // go): k of the next block from the middle of this one, the rest from the top of the block.
-  constexpr bool PRE = ND <= 8;
-  float4v ka[PRE ? ND : 1], qa[PRE ? ND : 1];
-  float ku[4][PRE ? ND : 1];
-  auto rows_of = [&](const float* x, int j) {
-    return *reinterpret_cast<const float4v*>(x + c16 * KS + 16 * j + 4 * g4);
-  };
   // LDS only: the loads of later blocks stay in flight
   auto sync = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  float4v v, vnext;
-  auto values = [&] {
-    float4v t;
+
+  if (wv >= CN) {  // ---- the waves that move operands and outputs
+    const int tid = threadIdx.x - 64 * CN, kh = h / (H / KH);
+    constexpr int DW = 16 * ND, KT = DW / 4, NL = (16 * KT + 255) / 256;
+    const int kbytes = KH * Dp * 4, vbytes = H * V * (int)sizeof(T), obytes = H * Vs * 4;
+    // A thread's share of a block, in registers from two blocks before it is written to LDS: rows
+    // of k and q, values of v, of T' and P, G or E.  Rows past the end, dimensions past Dp and
+    // columns past V read as 0, and so does all of a block past the last.
+    struct Stage {
+      float4v k[NL], q[NL];
+      float t, p, g;
+      T v[CW];
+    } st[2];
+    const bool krow = 16 * KT >= 256 || tid < 16 * KT;
+    const int kd4 = tid % KT * 4, tok = tid >> 4;
+    const uint32_t koff = kd4 < Dp && krow ? tid / KT * kbytes + kd4 * 4 : kOut;
+    uint32_t voff[CW], ooff[CW];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) t[r] = col < V ? ldf(&vreg[r]) : 0.f;
-    return t;
-  };
-  if (Dp < DW) {
-    for (int i = tid; i < 2 * (int)sizeof(Buf) / 4; i += 256)
-      reinterpret_cast<float*>(buf)[i] = 0.f;
-    __syncthreads();
-  }
-  offsets(min(16, n) - 1);
-  gload(0);
-  lwrite_rows(buf[0]);
-  lwrite_rest(buf[0]);
-  v = values();
-  if (nblk == 2) offsets(n - 17);
-  gload(min(1, nblk - 1));
-  sync();
-  if constexpr (PRE) {
+    for (int c = 0; c < CW; ++c) {
+      const int col = (bx * CW + c) * 16 + c16;
+      voff[c] = col < V ? tok * vbytes + col * (int)sizeof(T) : kOut;
+      ooff[c] = col < Vs ? tok * obytes + col * 4 : kOut;
+    }
+    // a block's rows, from a head's first of them: what the block's lanes may touch
+    auto rows_of = [&](const void* base, int bi, int stride) {
+      const int m = min(16, n - 16 * bi);
+      return buffer(reinterpret_cast<const char*>(base) + (int64_t)16 * bi * stride,
+                    m > 0 ? m * stride : 0);
+    };
+    const float* kb = kn + ((int64_t)row0 * KH + kh) * Dp;
+    const float* qb = qn + ((int64_t)row0 * KH + kh) * Dp;
+    const T* vb = vc + ((int64_t)row0 * H + h) * V;
+    const float* rb = rec + ((int64_t)rec_base(rows.q_start, s) * H + h) * kRec;
+    float* ob = o + ((int64_t)row0 * H + h) * Vs;
+    auto gload = [&](Stage& t, int bi) {
+      const Rsrc K = rows_of(kb, bi, kbytes), Q = rows_of(qb, bi, kbytes);
+      const Rsrc Vb = rows_of(vb, bi, vbytes);
+      const Rsrc R = buffer(rb + (int64_t)bi * H * kRec, bi < nblk ? kRec * 4 : 0);
 #pragma unroll
-    for (int j = 0; j < ND; ++j) ka[j] = rows_of(buf[0].k, j);
-  }
-  for (int bi = 0; bi < nblk; ++bi) {
-    const Buf& B = buf[bi & 1];
-    Buf& N = buf[(bi + 1) & 1];
-    float4v G, E, ta, pa;
-    float G15;
-    // what the block does beside its products, in eight pieces: the next block's operands go to
-    // the buffer that every wave left before the last barrier, the loads of the one after it
-    // (past the end: the last block's once more) are issued, this block's other operands read
-    auto piece = [&](int i) {
-      if (i == 0) lwrite_rows(N);
-      if (i == 1) {
-        lwrite_rest(N);
-        vnext = values();
+      for (int i = 0; i < NL; ++i) {
+        t.k[i] = load4(K, koff + i * (256 / KT) * kbytes);
+        t.q[i] = load4(Q, koff + i * (256 / KT) * kbytes);
       }
-      if (i == 2) {
-        const int b = min(bi + 2, nblk - 1);
-        if (b == nblk - 1) offsets(n - 16 * b - 1);
-        gload(b);
-      }
-      if (i == 3) {
-        G = *reinterpret_cast<const float4v*>(B.g + 4 * g4);
-        E = *reinterpret_cast<const float4v*>(B.g + 16 + 4 * g4);
-        G15 = B.g[15];
-        ta = *reinterpret_cast<const float4v*>(B.t + c16 * TS + 4 * g4);
-        pa = *reinterpret_cast<const float4v*>(B.p + c16 * TS + 4 * g4);
-        if constexpr (PRE) {
 #pragma unroll
-          for (int j = 0; j < ND; ++j) qa[j] = rows_of(B.q, j);
+      for (int c = 0; c < CW; ++c) {
+        if constexpr (sizeof(T) == 2)
+          t.v[c] = __builtin_amdgcn_raw_buffer_load_b16(Vb, voff[c], 0, 0);
+        else
+          t.v[c] = load1(Vb, voff[c]);
+      }
+      t.t = load1(R, tid * 4);
+      t.p = load1(R, 1024 + tid * 4);
+      t.g = load1(R, 2048 + (tid & 31) * 4);
+    };
+    auto lwrite = [&](const Stage& t, Buf& b) {
+      if (krow) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+          const int at = (i * (256 / KT) + tid / KT) * KS + kd4;
+          *reinterpret_cast<float4v*>(b.k + at) = t.k[i];
+          *reinterpret_cast<float4v*>(b.q + at) = t.q[i];
         }
       }
-      if constexpr (PRE) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (i == 4 + r) {
+      for (int c = 0; c < CW; ++c) b.v[(16 * c + c16) * TS + tok] = ldf(&t.v[c]);
+      b.t[tok * TS + c16] = t.t;
+      b.p[tok * TS + c16] = t.p;
+      b.g[tid & 31] = t.g;
+    };
+    auto store = [&](int bi) {
+      const Rsrc O = rows_of(ob, bi, obytes);
 #pragma unroll
-            for (int j = 0; j < ND; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + 16 * j + c16];
-          }
+      for (int c = 0; c < CW; ++c) {
+        float y = sh.os[bi & 1][c][0][16 * (tok >> 2) + c16][tok & 3];
+#pragma unroll
+        for (int i = 1; i < NW; ++i) y += sh.os[bi & 1][c][i][16 * (tok >> 2) + c16][tok & 3];
+        store1(y, O, ooff[c]);
       }
     };
-    float4v ks[2], qs[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) ks[c] = qs[c] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < ND; ++j) {
-      const float4v a = PRE ? ka[PRE ? j : 0] : rows_of(B.k, j);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ks[r & 1] = mfma4(a[r], S[j][r], ks[r & 1]);
-      if constexpr (!PRE) {
-        const float4v b = rows_of(B.q, j);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) qs[r & 1] = mfma4(b[r], S[j][r], qs[r & 1]);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i * ND / 8 == j) {
-          if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
-          piece(i);
-          if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    if constexpr (PRE) {
+    auto phase = [&](Stage& t, int bi) {
+      lwrite(t, sh.buf[(bi + 1) & 1]);
+      gload(t, bi + 3);
+      if (bi > 1) store(bi - 2);
       sync();
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < ND; ++j) ka[j] = rows_of(N.k, j);
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    gload(st[0], 0);
+    gload(st[1], 1);
+    lwrite(st[0], sh.buf[0]);
+    gload(st[0], 2);
+    sync();
+    int bi = 0;
+#pragma clang loop unroll(disable)
+    for (; bi + 1 < nblk; bi += 2) {
+      phase(st[1], bi);
+      phase(st[0], bi + 1);
     }
-    const float4v res = v - G * (ks[0] + ks[1]);
+    if (bi < nblk) phase(st[1], bi);
+    if (nblk > 1) store(nblk - 2);
+    sync();
+    store(nblk - 1);
+    const int C = 2 * KH * D + H * V, nb = nx * H, b = bx * H + h, per = (C + nb - 1) / nb;
+    T* cs = conv_state + (int64_t)slot * (taps - 1) * C;
+    for (int c = b * per + tid; c < min(C, (b + 1) * per); c += 256)
+      shift_conv(x, ldx, cs, row0, n, fresh, taps, C, c);
+    return;
+  }
+
+  // ---- the waves that multiply: 16 columns (cw) and ND / NW tiles of key dimensions (w) each
+  const int cw = wv / NW, w = wv % NW, d0 = 16 * NJ * w, col = (bx * CW + cw) * 16 + c16;
+  // the state of this head: past its columns and rows reads are 0 and writes dropped
+  const Rsrc Sb = buffer(state + ((int64_t)slot * H + h) * D * Vs, D * Vs * 4);
+  auto soff = [&](int j, int r) {
+    return col < Vs ? (uint32_t)(((d0 + 4 * g4 + 16 * j + r) * Vs + col) * 4) : kOut;
+  };
+  float4v S[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[j][r] = fresh ? 0.f : load1(Sb, soff(j, r));
+  // operands of a block: k from behind the barrier before it, the rest before its own
+  float4v ka[NJ], qa[NJ], ta, G, E, v;
+  float ku[4][NJ], pa[PR];
+  auto keys = [&](const Buf& b) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      ka[j] = *reinterpret_cast<const float4v*>(b.k + c16 * KS + d0 + 16 * j + 4 * g4);
+  };
+  auto block = [&](auto odd) {
+    constexpr int P = decltype(odd)::value;
+    const Buf& B = sh.buf[P];
+    float4v ks = {0.f, 0.f, 0.f, 0.f}, qs = ks, parts[NW];
+    auto qstep = [&](int i) { qs = mfma4(qa[i >> 2][i & 3], S[i >> 2][i & 3], qs); };
+#pragma unroll
+    for (int i = 0; i < 4 * NJ; ++i) {
+      ks = mfma4(ka[i >> 2][i & 3], S[i >> 2][i & 3], ks);
+      if (i == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          qa[j] = *reinterpret_cast<const float4v*>(B.q + c16 * KS + d0 + 16 * j + 4 * g4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i == 1) {
+        G = *reinterpret_cast<const float4v*>(B.g + 4 * g4);
+        v = *reinterpret_cast<const float4v*>(B.v + (16 * cw + c16) * TS + 4 * g4);
+        ta = *reinterpret_cast<const float4v*>(B.t + c16 * TS + 4 * g4);
+        E = *reinterpret_cast<const float4v*>(B.g + 16 + 4 * g4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i == 2) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + d0 + 16 * j + c16];
+#pragma unroll
+        for (int k = 0; k < PR; ++k) pa[k] = B.p[c16 * TS + 4 * g4 + NW * k + w];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // half of the products with q while the parts of K S go out, the others while they come in
+    constexpr int Q0 = 2 * NJ, Q1 = 3 * NJ;
+    sh.ks[P][cw][w][lane] = ks;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < Q0; ++i) qstep(i);
+    __builtin_amdgcn_sched_barrier(0);
+    sync();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) parts[i] = sh.ks[P][cw][i][lane];
+    keys(sh.buf[1 - P]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = Q0; i < Q1; ++i) qstep(i);
+    __builtin_amdgcn_sched_barrier(0);
+    ks = parts[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) ks += parts[i];
+    const float4v res = v - G * ks;
     float4v u = {0.f, 0.f, 0.f, 0.f};
     // the chain of u runs between the products with q, which do not need it
 #pragma unroll
-    for (int j = 0; j < ND; ++j) {
-      if constexpr (PRE) {
+    for (int r = 0; r < 4; ++r) {
+      u = mfma4(ta[r], res[r], u);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) qs[r & 1] = mfma4(qa[j][r], S[j][r], qs[r & 1]);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (r * ND / 4 == j) u = mfma4(ta[r], res[r], u);
-      if constexpr (PRE) __builtin_amdgcn_sched_barrier(0);
+      for (int i = Q1; i < 4 * NJ; ++i)
+        if ((i - Q1) * 4 / NJ == r) qstep(i);
     }
-    float4v ov = G * (qs[0] + qs[1]);
+    // exp(c_15), the last of the 16 tokens'
+    const float G3 = G[3], G15 = __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, G3), 48));
 #pragma unroll
-    for (int j = 0; j < ND; ++j) S[j] *= G15;
+    for (int j = 0; j < NJ; ++j) S[j] *= G15;
     const float4v ue = u * E;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ov = mfma4(pa[r], u[r], ov);
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int j = 0; j < ND; ++j)
-        S[j] = mfma4(PRE ? ku[r][PRE ? j : 0] : B.k[(4 * g4 + r) * KS + 16 * j + c16], ue[r], S[j]);
+      for (int j = 0; j < NJ; ++j) S[j] = mfma4(ku[r][j], ue[r], S[j]);
+    qs *= G;
+#pragma unroll
+    for (int i = 0; i < PR; ++i) {
+      float t = u[NW * i];
+#pragma unroll
+      for (int k = 1; k < NW; ++k) t = w == k ? u[NW * i + k] : t;
+      qs = mfma4(pa[i], t, qs);
     }
-    if constexpr (!PRE) sync();
-    if (col < Vs) {
-      const int m = n - 16 * bi;
-      if (m >= 16) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) (op + bi * ostep + r * H * Vs)[ooff] = ov[r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (4 * g4 + r < m) (op + bi * ostep + r * H * Vs)[ooff] = ov[r];
-      }
-    }
-    v = vnext;
+    sh.os[P][cw][w][lane] = qs;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  sync();
+  keys(sh.buf[0]);
+  int bi = 0;
+#pragma clang loop unroll(disable)
+  for (; bi + 1 < nblk; bi += 2) {
+    block(Int<0>());
+    block(Int<1>());
   }
-  if (col < Vs) {
+  if (bi < nblk) block(Int<0>());
+  sync();
 #pragma unroll
-    for (int j = 0; j < ND; ++j)
+  for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = 16 * j + 4 * g4 + r;
-        if (d < D) Sg[(int64_t)d * Vs] = S[j][r];
-      }
-  }
-  const int nb = gridDim.x * H, b = blockIdx.x * H + h, per = (C + nb - 1) / nb;
-  T* cs = conv_state + (int64_t)slot * (taps - 1) * C;
-  for (int c = b * per + tid; c < min(C, (b + 1) * per); c += 256)
-    shift_conv(x, ldx, cs, row0, n, fresh, taps, C, c);
+    for (int r = 0; r < 4; ++r) store1(S[j][r], Sb, soff(j, r));
 }
 
 // ------------------------------------------------------------------ delta_norm
@@ -973,18 +1022,30 @@ template <typename T>
 int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, const float* kn,
          const void* vc, const float* decay, const float* beta, const void* x, int64_t ldx, Rows r,
          int n_rows, int KH, int H, int D, int Dp, int V, int Vs, int taps, hipStream_t s) {
-  const dim3 bgrid(n_rows / 16 + r.nseq, (H + 3) / 4), sgrid((Vs + 63) / 64, H, r.nseq);
+  const dim3 bgrid(n_rows / 16 + r.nseq, (H + 3) / 4);
+  // One column group a block, its key dimensions over 4 waves, while those blocks are one a CU: the
+  // chain of a block is what the step waits for.  Beyond, two groups of 2 waves (us, one / two: 256
+  // blocks 86 / 118, 384 39 / 38, 768 60 / 60, 1024 105 / 90 and 368 / 327).
+  const bool few = (int64_t)((Vs + 15) / 16) * H * r.nseq <= 256;
+#define OMNIA_SPLIT(ND, NW, CW)                                                                   \
+  scan_blocks_kernel<T, ND, NW, CW>                                                               \
+      <<<dim3((Vs + 16 * CW - 1) / (16 * CW) * H, r.nseq), 64 * (NW * CW + 4),                    \
+         sizeof(ScanShared<ND, NW, CW>), s>>>(o, state, (T*)conv_state, rec, qn, kn,              \
+                                              (const T*)vc, (const T*)x, ldx, r, KH, H, D, Dp, V, \
+                                              Vs, taps)
 #define OMNIA_SCANB(ND)                                                                         \
   if (D <= 16 * ND) {                                                                           \
     blocks_kernel<ND><<<bgrid, 256, 0, s>>>(rec, qn, kn, decay, beta, r.q_start, r.nseq, KH, H, \
                                             Dp);                                                \
-    scan_blocks_kernel<T, ND><<<sgrid, 256, 0, s>>>(o, state, (T*)conv_state, rec, qn, kn,      \
-                                                    (const T*)vc, (const T*)x, ldx, r, KH, H,   \
-                                                    D, Dp, V, Vs, taps);                        \
+    if (few)                                                                                    \
+      OMNIA_SPLIT(ND, (ND < 4 ? 2 : 4), 1);                                                     \
+    else                                                                                        \
+      OMNIA_SPLIT(ND, 2, 2);                                                                    \
     return (int)hipGetLastError();                                                              \
   }
   OMNIA_SCANB(2) OMNIA_SCANB(4) OMNIA_SCANB(8) OMNIA_SCANB(16)
 #undef OMNIA_SCANB
+#undef OMNIA_SPLIT
   const dim3 grid((Vs + 15) / 16, H, r.nseq);
 #define OMNIA_SCAN(N)                                                                           \
   if (D <= 64 * N) {                                                                            \
