@@ -179,6 +179,11 @@ int omnia_delta_step(void* y, float* state, void* conv_state, const float* qn, c
                      int64_t ldx, const float* norm_w, const int* positions, const int* slots,
                      int T, int KH, int H, int D, int Dp, int V, int Vs, int Vp, int taps,
                      float eps, hipStream_t s);
+int omnia_delta_step_conv(void* y, float* state, void* conv_state, const void* x, int f32,
+                          int64_t ldx, const void* conv_w, const float* a_log,
+                          const float* dt_bias, const float* norm_w, const int* positions,
+                          const int* slots, int T, int KH, int H, int D, int V, int Vs, int Vp,
+                          int taps, float eps, hipStream_t s);
 int64_t omnia_delta_records(int n_rows, int nseq, int H);
 int omnia_delta_scan(float* o, float* state, void* conv_state, float* rec, const float* qn,
                      const float* kn, const void* vc, const float* decay, const float* beta,
@@ -1757,6 +1762,28 @@ void delta_step(at::Tensor y, at::Tensor state, at::Tensor conv_state, at::Tenso
                             Dp, V, Vs, Vp, taps, (float)eps, cur_stream()), "delta_step");
 }
 
+// delta_prep and delta_step of decode rows in one launch; false: sizes that need the two
+bool delta_step_conv(at::Tensor y, at::Tensor state, at::Tensor conv_state, at::Tensor x,
+                     at::Tensor conv_w, at::Tensor a_log, at::Tensor dt_bias, at::Tensor norm_w,
+                     at::Tensor positions, at::Tensor slots, int64_t KH, int64_t H, int64_t D,
+                     int64_t V, int64_t Vp, int64_t taps, double eps) {
+  const int f32 = is_f32(x, "x");
+  const int64_t T = positions.numel(), C = 2 * KH * D + H * V, Vs = state.size(-1);
+  TORCH_CHECK(slots.numel() == T, "decode: one slot per row");
+  const int64_t ld = rows2(x, T, C + H * V + 2 * H, "x");
+  check_state(state, conv_state, x, H, D, Vs, taps, C);
+  like(conv_w, x, C * taps, "conv_w");
+  like(y, x, T * H * Vp, "y");
+  const int rc = omnia_delta_step_conv(
+      y.data_ptr(), state.data_ptr<float>(), conv_state.data_ptr(), x.data_ptr(), f32, ld,
+      conv_w.data_ptr(), vecf(a_log, H, "a_log"), vecf(dt_bias, H, "dt_bias"),
+      vecf(norm_w, V, "norm_w"), veci(positions, T, "positions"), veci(slots, T, "slots"), T, KH, H,
+      D, V, Vs, Vp, taps, (float)eps, cur_stream());
+  if (rc == -3) return false;
+  CHECK_RC(rc, "delta_step_conv");
+  return true;
+}
+
 void delta_scan(at::Tensor o, at::Tensor state, at::Tensor conv_state, at::Tensor rec, at::Tensor qn,
                 at::Tensor kn, at::Tensor vc, at::Tensor decay, at::Tensor beta, at::Tensor x,
                 at::Tensor q_start, at::Tensor positions, at::Tensor slots, int64_t KH, int64_t H,
@@ -2125,6 +2152,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("lightning_scratch", &omnia_lightning_scratch);
   m.def("delta_prep", &delta_prep);
   m.def("delta_step", &delta_step);
+  m.def("delta_step_conv", &delta_step_conv);
   m.def("delta_scan", &delta_scan);
   m.def("delta_norm", &delta_norm);
   m.def("latent_prep", &latent_prep);

@@ -408,6 +408,159 @@ __global__ __launch_bounds__(256) void step_kernel(
   }
 }
 
+// delta_prep and delta_step in one launch: a block of 256 threads a head has all R heads of a key
+// head of a row, so that the convolution inputs it reads are its own to shift.  Waves 0 and 1 make q
+// and k, 2 .. R + 1 the heads' v, 128 channels each, while the state's loads are under way; the rest
+// is step_kernel's.  Saves the launch and the round trip of q, k and v: us of both kernels -> this
+// one, 8 key heads of two heads of 128, states out of 1 GB, 1 / 8 / 32 / 64 / 96 / 192 / 256 rows
+// 10.9 / 11.3 / 19.0 / 31.4 / 44.6 / 83 / 107 -> 8.7 / 11.0 / 16.2 / 27.2 / 42.9 / 79.7 / 102.
+template <typename T, int NR, int R>
+__global__ __launch_bounds__(256 * R) void step_conv_kernel(
+    T* __restrict__ y, float* __restrict__ state, T* __restrict__ conv_state,
+    const T* __restrict__ x, int64_t ldx, const T* __restrict__ conv_w,
+    const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+    const float* __restrict__ norm_w, Rows rows, int KH, int D, int V, int Vs, int Vp, int taps,
+    float eps) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int t = blockIdx.x, kh = blockIdx.y, tid = threadIdx.x & 255, lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), own = wv >> 2;
+  const int H = KH * R, h = kh * R + own;  // this thread's head
+  const int slot = rows.slots[t];
+  T* yr = y + ((int64_t)t * H + h) * Vp;
+  if (slot < 0) {
+    for (int i = tid; i < Vp; i += 256) stf(yr + i, 0.f);
+    return;
+  }
+  const bool fresh = rows.positions[t] == 0;
+  const int C = 2 * KH * D + H * V, CG = Vs / 4, RG = 256 / CG;
+  float* qs = sm;                      // [128]
+  float* ks = qs + 128;                // [128]
+  float* vs = ks + 128 + own * 128;    // [R][128]
+  float* scratch = ks + 128 * (R + 1);  // [4 R]
+  float* red = scratch + 4 * R + own * (RG + 2) * Vs;  // [RG][Vs] of each head, and
+  float* us = red + RG * Vs;                           // [Vs]
+  float* os = us + Vs;                                 // [Vs]
+  const T* xr = x + (int64_t)t * ldx;
+
+  // ---- convolution inputs and weights of two channels a lane; oldest input first
+  const bool conv = wv < R + 2, isv = wv >= 2;
+  const int n = isv ? V : D, i0 = 2 * lane;
+  const int c0 = (isv ? 2 * KH * D + (kh * R + wv - 2) * V : wv * KH * D + kh * D) + i0;
+  T* cs = conv_state + (int64_t)slot * (taps - 1) * C + c0;
+  float in[2] = {0.f, 0.f}, hist[3][2], cw[2][4];
+  const bool lives = conv && i0 < n;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    hist[j][0] = hist[j][1] = 0.f;
+    if (lives && j < taps - 1 && !fresh) Vec<T, 2>::ld(hist[j], cs + (int64_t)j * C);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      cw[v][j] = lives && j < taps ? ldf(conv_w + (int64_t)(c0 + v) * taps + j) : 0.f;
+  if (lives) Vec<T, 2>::ld(in, xr + c0);
+  const float bx = ldf(xr + C + H * V + h), ax = ldf(xr + C + H * V + H + h);
+  const float dt = dt_bias[h], al = a_log[h];
+  const T* zr = xr + C + h * V;
+  const int v0 = min(tid, V - 1);
+  const float z0 = ldf(zr + v0), w0 = norm_w[v0];
+
+  const int cg = tid % CG, rg = tid / CG;
+  const bool act = rg < RG;
+  float4v* S = reinterpret_cast<float4v*>(state + (((int64_t)slot * H + h) * D) * Vs) + cg;
+  float4v reg[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int d = rg + i * RG;
+    reg[i] = (act && d < D && !fresh) ? __builtin_nontemporal_load(S + (int64_t)d * CG)
+                                      : float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  if (conv) {
+    float a[2], ss = 0.f;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      a[v] = in[v] * (taps == 4 ? cw[v][3] : taps == 3 ? cw[v][2] : cw[v][1]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (j < taps - 1) a[v] += hist[j][v] * cw[v][j];
+      a[v] = siluf_(a[v]);
+      ss += a[v] * a[v];
+    }
+    if (isv) {
+      T r[2];  // as delta_prep stores them
+      stf(r, a[0]);
+      stf(r + 1, a[1]);
+      float* o = ks + 128 * (wv - 1) + i0;
+      if (i0 < n) o[0] = ldf(r), o[1] = ldf(r + 1);
+    } else {
+      ss = row_sum16(ss);
+      ss += __shfl_xor(ss, 16, 64);
+      ss += __shfl_xor(ss, 32, 64);
+      float inv = 1.f / sqrtf(ss + 1e-6f);
+      if (wv == 0) inv *= 1.f / sqrtf((float)D);
+      float* o = qs + 128 * wv + i0;
+      if (i0 < n) o[0] = a[0] * inv, o[1] = a[1] * inv;
+    }
+    if (lives) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (j < taps - 1) Vec<T, 2>::st(cs + (int64_t)j * C, j < taps - 2 ? hist[j < 2 ? j + 1 : 2] : in);
+    }
+  }
+  const float z = ax + dt, sp = z > 20.f ? z : log1pf(expf(z));
+  const float g = expf(-expf(al) * sp), bt = sigmoidf_(bx);
+  __syncthreads();
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int d = rg + i * RG;
+    reg[i] *= g;
+    if (d < D) acc += reg[i] * ks[d];
+  }
+  if (act) *reinterpret_cast<float4v*>(red + rg * Vs + cg * 4) = acc;
+  __syncthreads();
+  for (int j = tid; j < Vs; j += 256) {
+    float sk = 0.f;
+    for (int r = 0; r < RG; ++r) sk += red[r * Vs + j];
+    us[j] = j < V ? bt * (vs[j] - sk) : 0.f;
+  }
+  __syncthreads();
+  acc = float4v{0.f, 0.f, 0.f, 0.f};
+  if (act) {
+    const float4v u4 = *reinterpret_cast<const float4v*>(us + cg * 4);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int d = rg + i * RG;
+      if (d < D) {
+        reg[i] += u4 * ks[d];
+        acc += reg[i] * qs[d];
+        __builtin_nontemporal_store(reg[i], S + (int64_t)d * CG);
+      }
+    }
+    *reinterpret_cast<float4v*>(red + rg * Vs + cg * 4) = acc;
+  }
+  __syncthreads();
+  float ss = 0.f;
+  for (int j = tid; j < Vs; j += 256) {
+    float o = 0.f;
+    for (int r = 0; r < RG; ++r) o += red[r * Vs + j];
+    os[j] = o;
+    if (j < V) ss += o * o;
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) scratch[wv] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ss += scratch[4 * own + i];
+  const float inv = 1.f / sqrtf(ss / (float)V + eps);
+  for (int j = tid; j < Vp; j += 256) {
+    const float zj = j < 256 || j >= V ? z0 : ldf(zr + j), nw = j < 256 || j >= V ? w0 : norm_w[j];
+    stf(yr + j, j < V ? os[j] * inv * nw * siluf_(zj) : 0.f);
+  }
+}
+
 // ------------------------------------------------------------------ delta_scan
 // grid (ceil(Vs / 16), H, nseq), 256 threads: wave w, lane l -> state column
 // blockIdx.x*16 + 4w + (l >> 4); lane l & 15 holds the key dimensions
@@ -1018,6 +1171,33 @@ int step(void* y, float* state, void* conv_state, const float* qn, const float* 
   return -5;
 }
 
+// -3: not covered (the two kernels above cover all)
+template <typename T>
+int step_conv(void* y, float* state, void* conv_state, const void* x, int64_t ldx,
+              const void* conv_w, const float* a_log, const float* dt_bias, const float* norm_w,
+              Rows r, int T_, int KH, int H, int D, int V, int Vs, int Vp, int taps, float eps,
+              hipStream_t s) {
+  const int CG = Vs / 4, RG = 256 / CG, nr = (D + RG - 1) / RG, R = H / KH;
+  if (D > 128 || V > 128 || D % 2 || V % 2 || taps < 2 || taps > 4 || nr > 16) return -3;
+  // blocks of several heads read and write in step with one another: in two rounds of the chip (four
+  // heads a CU) that costs what the launch does (112 / 128 / 144 rows, two kernels and one: 49.8 /
+  // 53.3 / 65.1 and 49.8 / 54.4 / 63.1)
+  const int64_t heads = (int64_t)T_ * H;
+  if (R > 1 && heads > 1664 && heads <= 2176) return -3;
+  const size_t lds = (size_t)(256 + 132 * R + R * (RG + 2) * Vs) * 4;
+#define OMNIA_STEP(N, RR)                                                                      \
+  if (R == RR && nr <= N) {                                                                    \
+    step_conv_kernel<T, N, RR><<<dim3(T_, KH), 256 * RR, lds, s>>>(                            \
+        (T*)y, state, (T*)conv_state, (const T*)x, ldx, (const T*)conv_w, a_log, dt_bias,      \
+        norm_w, r, KH, D, V, Vs, Vp, taps, eps);                                               \
+    return (int)hipGetLastError();                                                             \
+  }
+  OMNIA_STEP(4, 1) OMNIA_STEP(16, 1) OMNIA_STEP(4, 2) OMNIA_STEP(16, 2) OMNIA_STEP(4, 4)
+  OMNIA_STEP(16, 4)
+#undef OMNIA_STEP
+  return -3;
+}
+
 template <typename T>
 int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, const float* kn,
          const void* vc, const float* decay, const float* beta, const void* x, int64_t ldx, Rows r,
@@ -1092,6 +1272,23 @@ int omnia_delta_step(void* y, float* state, void* conv_state, const float* qn, c
                        D, Dp, V, Vs, Vp, taps, eps, s);
   return step<bf16_t>(y, state, conv_state, qn, kn, vc, decay, beta, x, ldx, norm_w, r, T, KH, H,
                       D, Dp, V, Vs, Vp, taps, eps, s);
+}
+
+// omnia_delta_prep and omnia_delta_step of decode rows in one launch; -3 where it does not cover the
+// sizes (checked before any launch)
+int omnia_delta_step_conv(void* y, float* state, void* conv_state, const void* x, int f32,
+                          int64_t ldx, const void* conv_w, const float* a_log,
+                          const float* dt_bias, const float* norm_w, const int* positions,
+                          const int* slots, int T, int KH, int H, int D, int V, int Vs, int Vp,
+                          int taps, float eps, hipStream_t s) {
+  if (KH < 1 || H % KH || Vs % 4 || Vs < V || Vp < V) return -1;
+  if (T == 0) return 0;
+  const Rows r{nullptr, T, positions, slots};
+  if (f32)
+    return step_conv<float>(y, state, conv_state, x, ldx, conv_w, a_log, dt_bias, norm_w, r, T, KH,
+                            H, D, V, Vs, Vp, taps, eps, s);
+  return step_conv<bf16_t>(y, state, conv_state, x, ldx, conv_w, a_log, dt_bias, norm_w, r, T, KH,
+                           H, D, V, Vs, Vp, taps, eps, s);
 }
 
 // floats of the block records of n_rows rows in nseq sequences

@@ -262,12 +262,16 @@ def delta_rule(x, w: dict, spec, state, conv_state, q_start, positions, slots, e
     kk, dev = kernels(), x.device
     if checks.active(x):
         checks.state_slots("delta_rule", slots, state)
+    y = torch.empty(T, H * Vp, dtype=x.dtype, device=dev) if out is None else out
+    if q_start is None and kk.delta_step_conv(y, state, conv_state, x, w["conv"], w["a_log"],
+                                              w["dt_bias"], w["norm"], positions, slots, KH, H, D,
+                                              V, Vp, taps, eps):
+        return y
     qn = torch.empty(T, KH, Dp, dtype=torch.float32, device=dev)
     kn = torch.empty_like(qn)
     vc = torch.empty(T, H * V, dtype=x.dtype, device=dev)
     decay = torch.empty(T, H, dtype=torch.float32, device=dev)
     beta = torch.empty_like(decay)
-    y = torch.empty(T, H * Vp, dtype=x.dtype, device=dev) if out is None else out
     kk.delta_prep(qn, kn, vc, decay, beta, x, w["conv"], conv_state, w["a_log"], w["dt_bias"],
                   q_start, positions, slots, KH, H, D, Dp, V, taps)
     if q_start is None:
