@@ -23,6 +23,13 @@
 //     share W column tiles and X row tiles in its L2: 4 where W stays in the 256 MB Infinity
 //     Cache, else 8 (16384 rows of 4096 x 14336 GM 4 / 8: 1270 / 1301 us; of 28672 x 4096
 //     2605 / 2574).
+// What is left of a tile is its ends: 3 to 4 thousand clocks until its first K-tiles are there and
+// 6 to 8 thousand of its epilogue, of a K-tile's 2.3.  One wave a SIMD issues an instruction in about
+// 5 clocks, so the accumulators start with the first products' results (256 writes fewer), rows
+// without a scale are not multiplied by one (256), a bias is there when it is needed, and the stores
+// of a row stand together.  us before / now, tiles of 4 rounds: 4096 rows of 16384 x 256 54.7 / 50.2, x
+// 2048 206 / 201, gated with bias 203 / 200, x 4096 377 / 373; of one round 53.2 / 51.5.  The other
+// K-tiles' DMAs between the first one's products: no gain.
 // Normal values, us before (eight waves, one K-tile ahead) and now, 16384 rows: 4096 x 4096
 // 382 / 361, 4096 x 14336 1344 / 1270, 28672 x 4096 2698 / 2574 (1.50 PF/s), 6144 x 4096 578 /
 // 554, 2048 x 2048 110 / 100.
@@ -118,6 +125,10 @@ __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcp
 // that overwrite an operand (it is read at issue)
 __device__ __forceinline__ void mfma16(float4v& acc, short8 a, short8 b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// acc = a . b
+__device__ __forceinline__ void mfma16_first(float4v& acc, short8 a, short8 b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
 }
 // ... and behind it a DMA of 16 bytes a lane to LDS address ``at`` + OFF (lane-linear)
 __device__ __forceinline__ void mfma16_dma(float4v& acc, short8 a, short8 b, uint32_t voff,
@@ -215,6 +226,21 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   const int wr = SHAPE == FLAT ? 0 : w >> 1, wc = SHAPE == FLAT ? w : w & 1;
   const int fr = lane & 15, fq = lane >> 4;
 
+  // ---- a bias is asked for before the DMAs, which are counted
+  constexpr int NG = NF / 2, GU = 64 * NB;
+  constexpr int WCOL = (gated(EPI) ? NG : NF) * 16;
+  const int f0 = nt * TN + wc * WCOL;
+  float4v bg[NG], bu[NG];
+  if constexpr (EPI == 7) {
+#pragma unroll
+    for (int n = 0; n < NG; ++n)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        bg[n][j] = p.bias[f0 + 16 * n + 4 * fq + j];
+        bu[n][j] = p.bias[p.N + f0 + 16 * n + 4 * fq + j];
+      }
+  }
+
   // ---- DMA sources: instruction i of wave w fills half-tile rows 32w + 8i + lane/8, LDS chunk
   // lane%8 <- global chunk (lane%8) ^ (row & 7)
   const char* base[4];  // A0 A1 B0 B1
@@ -295,8 +321,6 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
 
   // ---- fragments: A rows wr*128 + 16m + fr; B's columns wc*WCOL + 16n + fr, gated those of the
   // gate's part for n < NG and of the up's, GU columns on, for the rest; k chunk 4s + fq of step s
-  constexpr int NG = NF / 2, GU = 64 * NB;
-  constexpr int WCOL = (gated(EPI) ? NG : NF) * 16;
   const bf16_t *fa[2], *fb[2];
   int ra = wr * HALF, rb = NA * HALF;
   auto set_r = [&]() __attribute__((always_inline)) {
@@ -330,15 +354,10 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     for (int i = 0; i < 8 * NF; ++i) asm volatile("" : "+a"(acc[i / NF][i % NF]));
     asm volatile("s_nop 15" ::: "memory");
   };
-#pragma unroll
-  for (int m = 0; m < 8; ++m)
-#pragma unroll
-    for (int n = 0; n < NF; ++n) acc[m][n] = {0.f, 0.f, 0.f, 0.f};
-  pin();
 
   // this thread's row scale, ready before the loop
   constexpr bool ROUTED = EPI == 6 || EPI == 8;
-  constexpr bool UNSCALED = EPI == 2 || EPI == 11 || EPI == 7 || EPI == 9 || EPI == 10;
+  constexpr bool UNSCALED = EPI == 2 || sliced(EPI) || EPI == 5 || EPI == 7 || EPI == 9 || EPI == 10;
   const bool scaled = ROUTED || (!UNSCALED && p.ss_in != nullptr);
   float own = 1.f;
   if constexpr (ROUTED) {  // the assignment's routing weight
@@ -357,9 +376,13 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     own = __builtin_amdgcn_rsqf(t * p.inv_d + p.eps);
   }
 
-  auto product = [&](int set, int j, int d) __attribute__((always_inline)) {  // d: DMA or -1
+  // d: DMA or -1; first: the accumulator's first product
+  auto product = [&](int set, int j, int d, bool first) __attribute__((always_inline)) {
     const int m = j / NF, n = (m & 1) ? NF - 1 - j % NF : j % NF;
-    if (d < 0) {
+    if (first) {
+      mfma16_first(acc[m][n], fw[set][n], fx[set][m]);
+      if (d >= 0) dma_b(d);
+    } else if (d < 0) {
       mfma16(acc[m][n], fw[set][n], fx[set][m]);
     } else if (d < 8) {
       mfma16_dma(acc[m][n], fw[set][n], fx[set][m], vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb,
@@ -393,7 +416,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     }
     return -1;
   };
-  auto step = [&](auto SC) __attribute__((always_inline)) {
+  auto step = [&](auto SC, auto FIRST) __attribute__((always_inline)) {
     constexpr int s = decltype(SC)::value;
 #pragma unroll
     for (int j = 0; j < P; ++j) {
@@ -407,7 +430,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
-      product(s, j, dma_at(s, j));
+      product(s, j, dma_at(s, j), decltype(FIRST)::value);
       if (s == 0 && !(j & 1) && j < 2 * (8 + NF)) read(1, 1, j >> 1);
       if (s == 1 && !(j & 1) && j >= LAND && j < LAND + 2 * (8 + NF)) read(0, 0, (j - LAND) >> 1);
       // addresses of what comes next, between products that hide them
@@ -422,10 +445,12 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < 8 + NF; ++j) read(0, 0, j);
-  for (int t = 0; t < nk; ++t) {
-    step(std::integral_constant<int, 0>{});
-    step(std::integral_constant<int, 1>{});
+  step(std::integral_constant<int, 0>{}, std::true_type{});
+  for (int t = 1; t < nk; ++t) {
+    step(std::integral_constant<int, 1>{}, std::false_type{});
+    step(std::integral_constant<int, 0>{}, std::false_type{});
   }
+  step(std::integral_constant<int, 1>{}, std::false_type{});
   pin();
   wait_vm<0>();  // the reloads past the end land before LDS is used again, or left
 
@@ -435,35 +460,46 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   const int row0 = wr * 128 + fr, ccol = 16 * (fq & 1) + 8 * (fq >> 1);
   float* scratch = reinterpret_cast<float*>(lds);
   float rs[8];
-#pragma unroll
-  for (int m = 0; m < 8; ++m) rs[m] = 1.f;
   if (scaled) {
     __syncthreads();
     scratch[tid] = own;
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < 8; ++m) rs[m] = scratch[row0 + 16 * m];
+  } else if constexpr (EPI == 3) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) rs[m] = 1.f;
   }
+  // a wave issues an instruction in 5 clocks: 256 fewer where rows have no scale
+  auto rows = [&](auto put) __attribute__((always_inline)) {
+    if (scaled) {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) put(std::true_type{}, m);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 8; ++m) put(std::false_type{}, m);
+    }
+  };
+  // (the asm keeps hipcc from reading all accumulators ahead of that branch, for both sides)
+  auto sums = [&](auto SCALED, int m, int n) __attribute__((always_inline)) {
+    float4v v = acc[m][n];
+    if constexpr (decltype(SCALED)::value) {
+      asm volatile("; scaled" : "+v"(v));
+      v *= rs[m];
+    } else {
+      asm volatile("; plain" : "+v"(v));
+    }
+    return v;
+  };
   bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
   if constexpr (gated(EPI)) {
     // gate (n < NG) and up (n + NG) of features nt*TN + wc*WCOL + 16n + 4fq + j in one lane
-    const int f0 = nt * TN + wc * WCOL;
-    float4v bg[NG], bu[NG];
-    if constexpr (EPI == 7)
-#pragma unroll
-      for (int n = 0; n < NG; ++n)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          bg[n][j] = p.bias[f0 + 16 * n + 4 * fq + j];
-          bu[n][j] = p.bias[p.N + f0 + 16 * n + 4 * fq + j];
-        }
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
+    rows([&](auto SCALED, int m) __attribute__((always_inline)) {
       const int r = row0 + 16 * m;
       float4v v[NG];
 #pragma unroll
       for (int n = 0; n < NG; ++n) {
-        float4v g = acc[m][n], u = acc[m][n + NG];
+        const float4v g = sums(SCALED, m, n), u = sums(SCALED, m, n + NG);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if constexpr (EPI == 7)
@@ -471,18 +507,20 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
           else if constexpr (EPI == 9)
             v[n][j] = gelu_tanh_(g[j]) * u[j];
           else if constexpr (EPI == 8)
-            v[n][j] = clamped_glu(g[j] * rs[m], u[j] * rs[m], p.glu_alpha, p.glu_limit);
+            v[n][j] = clamped_glu(g[j], u[j], p.glu_alpha, p.glu_limit);
           else
-            v[n][j] = silu(g[j] * rs[m]) * (u[j] * rs[m]);
+            v[n][j] = silu(g[j]) * u[j];
         }
       }
+      uint4v c[NG / 2];
+#pragma unroll
+      for (int n = 0; n < NG; n += 2) c[n / 2] = chunk<EPI>(v[n], v[n + 1]);
       if (r < Mt) {
         bf16_t* o = out + (int64_t)(m0 + r) * p.ldo + f0 + ccol;
 #pragma unroll
-        for (int n = 0; n < NG; n += 2)
-          *reinterpret_cast<uint4v*>(o + 16 * n) = chunk<EPI>(v[n], v[n + 1]);
+        for (int n = 0; n < NG; n += 2) *reinterpret_cast<uint4v*>(o + 16 * n) = c[n / 2];
       }
-    }
+    });
   } else if constexpr (EPI == 2) {
     // residual += tile; the sums of squares of a row's 16-byte chunks meet in pairs: of the two
     // waves, then of a lane, then of its four lanes
@@ -589,8 +627,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     }
   } else {
     if constexpr (EPI == 4) out += (int64_t)ks * p.M * p.N;
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
+    rows([&](auto SCALED, int m) __attribute__((always_inline)) {
       const int r = row0 + 16 * m;
       int64_t orow = m0 + r;
       bool live = r < Mt;
@@ -599,23 +636,24 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
         live = orow < p.n_assign;
       }
       bf16_t* o = out + orow * p.ldo + (int64_t)nt * TN + wc * WCOL + ccol;
+      uint4v v[NF / 2];
 #pragma unroll
       for (int n = 0; n < NF; n += 2) {
-        float4v c = acc[m][n], d = acc[m][n + 1];
+        float4v c = sums(SCALED, m, n), d = sums(SCALED, m, n + 1);
+        if constexpr (EPI == 10) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if constexpr (EPI == 10) {
+          for (int j = 0; j < 4; ++j) {
             c[j] = gelu_erf16_(c[j]);
             d[j] = gelu_erf16_(d[j]);
-          } else {
-            c[j] *= rs[m];
-            d[j] *= rs[m];
           }
         }
-        const uint4v v = chunk<EPI>(c, d);
-        if (live) *reinterpret_cast<uint4v*>(o + 16 * n) = v;
+        v[n / 2] = chunk<EPI>(c, d);
       }
-    }
+      if (live) {
+#pragma unroll
+        for (int n = 0; n < NF; n += 2) *reinterpret_cast<uint4v*>(o + 16 * n) = v[n / 2];
+      }
+    });
   }
 }
 
