@@ -92,8 +92,15 @@ constexpr int stages(int mf, int wn) {
   return fit > 5 ? 5 : fit;
 }
 
+// What the first loads need comes as arguments of their own: 14 words that are in registers when a
+// wave starts (a struct is loaded from memory).
 template <int MF, int WN, int EPI, bool PK>
-__global__ __launch_bounds__(64 * WN, 1) void panel_kernel(PanelArgs p) {
+__global__ __launch_bounds__(64 * WN, 1) void panel_kernel(const bf16_t* x, const bf16_t* w,
+                                                           int64_t ldx, const int* n_blocks,
+                                                           const int* blk_expert, int M, int N,
+                                                           int K_, int S, PanelArgs p) {
+  p.x = x, p.w = w, p.ldx = ldx, p.n_blocks = n_blocks, p.blk_expert = blk_expert;
+  p.M = M, p.N = N, p.K = K_, p.S = S;
   constexpr int BM = 16 * MF, NS = stages(MF, WN);
   // DMA instructions of a wave and stage for x: XI, of the last XW waves XI - 1
   constexpr int XI = (2 * MF + WN - 1) / WN, XW = XI * WN - 2 * MF;
@@ -275,10 +282,14 @@ template <int MF, int WN, int EPI>
 int launch(const PanelArgs& p, bool packed, hipStream_t s, int segs = 1) {
   const int units = paired(EPI) ? p.N / 8 : p.N / 16;
   const dim3 grid((units + WN - 1) / WN * p.S, segs);
+#define OMNIA_PANEL(PK)                                                                       \
+  panel_kernel<MF, WN, EPI, PK><<<grid, 64 * WN, 0, s>>>(p.x, p.w, p.ldx, p.n_blocks,         \
+                                                         p.blk_expert, p.M, p.N, p.K, p.S, p)
   if (packed)
-    panel_kernel<MF, WN, EPI, true><<<grid, 64 * WN, 0, s>>>(p);
+    OMNIA_PANEL(true);
   else
-    panel_kernel<MF, WN, EPI, false><<<grid, 64 * WN, 0, s>>>(p);
+    OMNIA_PANEL(false);
+#undef OMNIA_PANEL
   return (int)hipGetLastError();
 }
 

@@ -657,8 +657,15 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   }
 }
 
-template <int EPI, int SHAPE = WIDE>
-__global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
+// What the first loads need comes as arguments of their own: 14 words that are in registers when a
+// wave starts (a struct is loaded from memory).
+template <int EPI, int SHAPE>
+__global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf16_t* W, int M,
+                                                       int N, int K, int splits,
+                                                       const int* n_blocks, const int* blk_expert,
+                                                       const int* sorted, PArgs p) {
+  p.X = X, p.W = W, p.M = M, p.N = N, p.K = K, p.splits = splits;
+  p.n_blocks = n_blocks, p.blk_expert = blk_expert, p.sorted = sorted;
   __shared__ __attribute__((aligned(1024))) bf16_t lds[ring(SHAPE)];
   constexpr int TN = (gated(EPI) ? 128 : 256) / (SHAPE == NARROW ? 2 : 1);
   constexpr bool MOE = grouped(EPI);
@@ -756,6 +763,12 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(PArgs p) {
   tile<EPI, SHAPE>(p, lds, mt, nt, ks);
 }
 
+template <int EPI, int SHAPE>
+void launch(const PArgs& a, dim3 grid, hipStream_t s) {
+  pgemm_kernel<EPI, SHAPE><<<grid, 256, 0, s>>>(a.X, a.W, a.M, a.N, a.K, a.splits, a.n_blocks,
+                                                a.blk_expert, a.sorted, a);
+}
+
 // one workgroup (256 threads) per row: ss[r] = sum(x[r]^2) (layer-0 input of the
 // folded-norm prefill path: the embedding rows have no producer epilogue)
 __global__ __launch_bounds__(256) void row_sumsq_kernel(float* __restrict__ ss,
@@ -829,9 +842,9 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
 #define OMNIA_PGEMM(EPI)                                       \
   do {                                                         \
     if (narrow)                                                \
-      pgemm_kernel<EPI, NARROW><<<grid, 256, 0, s>>>(a);            \
+      launch<EPI, NARROW>(a, grid, s);            \
     else                                                       \
-      pgemm_kernel<EPI, WIDE><<<grid, 256, 0, s>>>(a);            \
+      launch<EPI, WIDE>(a, grid, s);            \
     return (int)hipGetLastError();                             \
   } while (0)
   if (bias) OMNIA_PGEMM(7);
@@ -840,8 +853,8 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
     case 0: OMNIA_PGEMM(0);
     case 1: OMNIA_PGEMM(1);
 #undef OMNIA_PGEMM
-    case 2: pgemm_kernel<2><<<grid, 256, 0, s>>>(a); break;
-    default: pgemm_kernel<3><<<grid, 256, 0, s>>>(a); break;
+    case 2: launch<2, WIDE>(a, grid, s); break;
+    default: launch<3, WIDE>(a, grid, s); break;
   }
   return (int)hipGetLastError();
 }
@@ -865,13 +878,13 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
           nullptr, 0, 0, 0};
   const dim3 grid((unsigned)blocks);
   if (f32 && tn == 128)
-    pgemm_kernel<11, NARROW><<<grid, 256, 0, s>>>(a);
+    launch<11, NARROW>(a, grid, s);
   else if (f32)
-    pgemm_kernel<11><<<grid, 256, 0, s>>>(a);
+    launch<11, WIDE>(a, grid, s);
   else if (tn == 128)
-    pgemm_kernel<4, NARROW><<<grid, 256, 0, s>>>(a);
+    launch<4, NARROW>(a, grid, s);
   else
-    pgemm_kernel<4><<<grid, 256, 0, s>>>(a);
+    launch<4, WIDE>(a, grid, s);
   return (int)hipGetLastError();
 }
 
@@ -907,9 +920,9 @@ int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int
 #define OMNIA_PGEMM(EPI)                            \
   do {                                              \
     if (narrow)                                     \
-      pgemm_kernel<EPI, NARROW><<<grid, 256, 0, s>>>(a); \
+      launch<EPI, NARROW>(a, grid, s); \
     else                                            \
-      pgemm_kernel<EPI, WIDE><<<grid, 256, 0, s>>>(a); \
+      launch<EPI, WIDE>(a, grid, s); \
     return (int)hipGetLastError();                  \
   } while (0)
   if (mode == 0) OMNIA_PGEMM(5);

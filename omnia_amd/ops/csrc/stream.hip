@@ -71,9 +71,21 @@ constexpr bool gated(int epi) { return epi == 1 || epi == 5 || epi == 8; }
 constexpr bool paired(int epi) { return gated(epi) || epi == 3; }
 constexpr bool grouped(int epi) { return epi >= 5; }
 
-// D: chunks in flight of 1 + NW operand fragments, 8 registers each
+// D: chunks in flight of 1 + NW operand fragments, 8 registers each.  What the first loads need
+// comes as arguments of their own, 14 words that are in registers when a wave starts (a struct is
+// loaded from memory): i0 .. of experts e_lo, e_hi, n_assign and topk, else M and n_ss.
 template <int NW, int EPI, bool NORM, bool PK>
-__global__ __launch_bounds__(64 * WAVES, NW <= 2 ? 4 : 2) void stream_kernel(StreamArgs p) {
+__global__ __launch_bounds__(64 * WAVES, NW <= 2 ? 4 : 2) void stream_kernel(
+    const bf16_t* x, const bf16_t* w, int64_t ldx, const void* first, int N, int K_, int i0, int i1,
+    int i2, int i3, StreamArgs p) {
+  p.x = x, p.w = w, p.ldx = ldx, p.N = N, p.K = K_;
+  if constexpr (grouped(EPI)) {
+    p.ids = reinterpret_cast<const int*>(first);
+    p.e_lo = i0, p.e_hi = i1, p.n_assign = i2, p.topk = i3;
+  } else {
+    p.ss_in = reinterpret_cast<const float*>(first);
+    p.M = i0, p.n_ss = i1;
+  }
   constexpr int D = NW <= 2 ? 4 : 3, F = 8 * NW;  // F: features of a paired block
   __shared__ __attribute__((aligned(16))) float red[WAVES * NW * 256];
   __shared__ float rsl[NORM ? 16 : 1];
@@ -317,10 +329,17 @@ int launch(const StreamArgs& p, bool packed, int segs, hipStream_t s) {
   const int cols = paired(EPI) ? 8 * NW : 16 * NW;
   const int width = EPI == 3 ? (p.hq + 2 * p.hkv) * 64 : p.N;
   const dim3 grid(width / cols, segs);
+  constexpr bool E = grouped(EPI);
+  const void* first = E ? (const void*)p.ids : (const void*)p.ss_in;
+#define OMNIA_STREAM(PK)                                                                          \
+  stream_kernel<NW, EPI, NORM, PK><<<grid, 64 * WAVES, 0, s>>>(                                   \
+      p.x, p.w, p.ldx, first, p.N, p.K, E ? p.e_lo : p.M, E ? p.e_hi : p.n_ss,                    \
+      E ? p.n_assign : 0, E ? p.topk : 0, p)
   if (packed)
-    stream_kernel<NW, EPI, NORM, true><<<grid, 64 * WAVES, 0, s>>>(p);
+    OMNIA_STREAM(true);
   else
-    stream_kernel<NW, EPI, NORM, false><<<grid, 64 * WAVES, 0, s>>>(p);
+    OMNIA_STREAM(false);
+#undef OMNIA_STREAM
   return (int)hipGetLastError();
 }
 
