@@ -101,9 +101,13 @@ class Experts:
             w["shared"] = self.shared.pack(lambda n: get("shared." + n), d)
         return w
 
-    def forward(self, w: dict, h: torch.Tensor, is_decode: bool) -> dict:
+    def routing(self, w: dict) -> mops.Routing:
+        return mops.Routing(w, self.spec)
+
+    def forward(self, w: dict, h: torch.Tensor, is_decode: bool,
+                route: mops.Routing | None = None) -> dict:
         parts, ids, wts = mops.experts(h, w, self.spec,
-                                       packed_experts(self.model, w["up"], w["down"]))
+                                       packed_experts(self.model, w["up"], w["down"]), route)
         out = {"m": parts, "slots": True}
         if self.spec.identity:
             out["identity"] = (ids, wts, h, self.spec.experts)

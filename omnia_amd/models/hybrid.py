@@ -35,7 +35,7 @@ from ..ops import mixers as mops
 from ..parallel import state as pstate
 from ..parallel.overlap import side_stream
 from .config import ModelConfig
-from .feedforward import MLPS
+from .feedforward import MLPS, Experts
 from .layers import tensor_shapes
 from .mixers import MIXERS, rotary_table
 from .projection import Parts, Projections
@@ -297,11 +297,12 @@ class HybridModel(Projections):
                                self.w["embed_norm"], ws[0]["pre1"], fb.ids_src, fb.tok_slots)
         for i, (w, mixer, mlp) in enumerate(zip(ws, self.mixers, self.mlps)):
             after = ws[i + 1]["pre1"] if i + 1 < len(ws) else self.w["final_norm"]
+            route = {"route": mlp.routing(w["mlp"])} if isinstance(mlp, Experts) else {}
             h = mops.norm_residual(x, post=w["post1"], pre=w["pre2"] if mlp else after, dtype=dt,
-                                   **mixer.sublayer(w["mix"], h, fb, kv.layers[i]))
+                                   **mixer.sublayer(w["mix"], h, fb, kv.layers[i]), **route)
             if mlp:
                 h = mops.norm_residual(x, post=w["post2"], pre=after, dtype=dt,
-                                       **mlp.forward(w["mlp"], h, dec))
+                                       **mlp.forward(w["mlp"], h, dec, **route))
             if trace is not None:
                 trace.append(x[:, :self.cfg.hidden_size].clone())
         return h

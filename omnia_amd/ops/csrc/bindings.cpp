@@ -199,7 +199,8 @@ int omnia_rms_embed(void* h, float* x, const int* ids, const void* table, int f3
 int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int S,
                        int64_t row_stride, int64_t part_stride, int rows, int d,
                        const float* bias, const float* w_post, const float* w_pre, float inv_n, float eps,
-                       hipStream_t s);
+                       const void* router, int* ids, float* wts, int E, int k, int sigmoid, int renorm,
+                       const float* corr, int groups, int keep, const float* rbias, hipStream_t s);
 int omnia_softcap(void* z, int f32, int64_t n, float cap, hipStream_t s);
 int omnia_gqa_prep(void* q, void* kc, void* vc, int f32, const void* x, int ptype, int S,
                    int64_t slab, int64_t ldx, const float* wq, const float* wk,
@@ -1979,16 +1980,38 @@ void rms_embed(at::Tensor h, at::Tensor x, at::Tensor ids, at::Tensor table, int
                            opt_ptr<int>(tok_slots), cur_stream()), "rms_embed");
 }
 
-void rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bias,
-                  at::Tensor w_post, OptT w_pre, double inv_n, double eps) {
+// With a router [E, d] the rows' experts too, as moe_route; false: sizes that need it (nothing ran)
+bool rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bias,
+                  at::Tensor w_post, OptT w_pre, double inv_n, double eps, OptT router, OptT ids,
+                  OptT wts, int64_t k, bool sigmoid, bool renorm, OptT corr, int64_t groups,
+                  int64_t keep, OptT rbias) {
   const int f32 = is_f32(h, "h");
   const ResidParts p = resid_parts(m, slots);
   const int64_t d = p.d;
   like(h, h, p.M * d, "h");
-  CHECK_RC(omnia_rms_residual(h.data_ptr(), f32, outf(x, p.M * d, "x"), m.data_ptr(), p.type, p.S,
-                              p.row, p.part, p.M, d, opt_vecf(bias, d, "bias"),
-                              vecf(w_post, d, "w_post"), opt_vecf(w_pre, d, "w_pre"),
-                              (float)inv_n, (float)eps, cur_stream()), "rms_residual");
+  const bool route = router.has_value() && router->defined();
+  int64_t E = 0;
+  if (route) {
+    TORCH_CHECK(router->is_cuda() && router->scalar_type() == h.scalar_type() &&
+                router->is_contiguous() && router->dim() == 2 && router->size(1) == d,
+                "router [E, d]");
+    E = router->size(0);
+    if (reinterpret_cast<uintptr_t>(router->data_ptr()) & 7) return false;
+    TORCH_CHECK(ids.has_value() && wts.has_value() && ids->is_cuda() && wts->is_cuda() &&
+                ids->scalar_type() == at::kInt && wts->scalar_type() == at::kFloat &&
+                ids->numel() == p.M * k && wts->numel() == p.M * k && ids->is_contiguous() &&
+                wts->is_contiguous(), "ids / wts [M, k]");
+  }
+  const int rc = omnia_rms_residual(
+      h.data_ptr(), f32, outf(x, p.M * d, "x"), m.data_ptr(), p.type, p.S, p.row, p.part, p.M, d,
+      opt_vecf(bias, d, "bias"), vecf(w_post, d, "w_post"), opt_vecf(w_pre, d, "w_pre"),
+      (float)inv_n, (float)eps, route ? router->data_ptr() : nullptr,
+      route ? ids->data_ptr<int>() : nullptr, route ? wts->data_ptr<float>() : nullptr, E, k,
+      sigmoid, renorm, opt_vecf(corr, E, "correction"), groups, keep,
+      opt_vecf(rbias, E, "router bias"), cur_stream());
+  if (route && rc == -3) return false;
+  CHECK_RC(rc, "rms_residual");
+  return true;
 }
 
 void softcap(at::Tensor z, double cap) {
@@ -2135,7 +2158,12 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("rmsnorm", &rmsnorm);
   m.def("tanh_norm_embed", &tanh_norm_embed);
   m.def("rms_embed", &rms_embed);
-  m.def("rms_residual", &rms_residual);
+  m.def("rms_residual", &rms_residual, py::arg("h"), py::arg("x"), py::arg("m"), py::arg("slots"),
+        py::arg("bias"), py::arg("w_post"), py::arg("w_pre"), py::arg("inv_n"), py::arg("eps"),
+        py::arg("router") = py::none(), py::arg("ids") = py::none(), py::arg("wts") = py::none(),
+        py::arg("k") = 0, py::arg("sigmoid") = false, py::arg("renorm") = false,
+        py::arg("corr") = py::none(), py::arg("groups") = 1, py::arg("keep") = 1,
+        py::arg("rbias") = py::none());
   m.def("softcap", &softcap);
   m.def("gqa_prep", &gqa_prep);
   m.def("gqa_attend", &gqa_attend);

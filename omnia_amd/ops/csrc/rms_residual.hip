@@ -13,7 +13,7 @@
 // One workgroup per row; a thread keeps its columns in registers between the statistic
 // and the update.  Few rows (decode): 1024 threads a row, so that a row's loads are all
 // in flight at once.
-#include "common.h"
+#include "route.h"
 
 using namespace omnia;
 
@@ -98,14 +98,64 @@ __global__ __launch_bounds__(NT) void embed_kernel(T* __restrict__ h, float* __r
   }
 }
 
-template <typename T, typename P, int NT, int NC>
+// Router logits of a row for up to EP experts, in the block that has the row: saves a launch of 5.5 us
+// a sparse layer for about 1 us here.  The router's columns are loaded ahead of everything else; a
+// wave adds a column's EP products over its lanes in EP - 1 + log2(64 / EP) exchanges, half of the
+// values it still has going to the other lanes each time.
+template <int EP>
+struct Logits {
+  short4v w[EP];
+  __device__ __forceinline__ void load(const bf16_t* router, int E, int d, int c) {
+#pragma unroll
+    for (int e = 0; e < EP; ++e)
+      w[e] = c < d && e < E ? *reinterpret_cast<const short4v*>(router + (int64_t)e * d + c)
+                            : short4v{0, 0, 0, 0};
+  }
+  // v: the row's values as the experts read them.  part [waves][EP]; ends with row z[0 .. E - 1]
+  template <int NT>
+  __device__ __forceinline__ void row(float4v v, float (*part)[EP], float* z) const {
+    const int lane = threadIdx.x & 63;
+    float s[EP];
+#pragma unroll
+    for (int e = 0; e < EP; ++e) {
+      s[e] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[e] += v[j] * bf2f((uint16_t)w[e][j]);
+    }
+    int at = 0;  // the value that this lane ends with
+#pragma unroll
+    for (int n = EP / 2, bit = 1; n >= 1; n /= 2, bit *= 2) {
+      const bool up = lane & bit;
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+        s[i] = (up ? s[i + n] : s[i]) + __shfl_xor(up ? s[i] : s[i + n], bit, 64);
+      at += up ? n : 0;
+    }
+#pragma unroll
+    for (int o = EP; o < 64; o *= 2) s[0] += __shfl_xor(s[0], o, 64);
+    if (lane < EP) part[threadIdx.x >> 6][at] = s[0];
+    __syncthreads();
+    if (threadIdx.x < EP) {
+      float a = 0.f;
+      for (int i = 0; i < NT / 64; ++i) a += part[i][threadIdx.x];
+      z[threadIdx.x] = a;
+    }
+  }
+};
+
+// EP: experts of a route behind the row (0: none)
+template <typename T, typename P, int NT, int NC, int EP>
 __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* __restrict__ x,
                                                        const P* __restrict__ m, int S,
                                                        int64_t row_stride, int64_t part_stride,
                                                        int d, const float* __restrict__ bias,
-                                                       Norm post, Norm pre) {
+                                                       Norm post, Norm pre,
+                                                       const bf16_t* __restrict__ router,
+                                                       Route route) {
   __shared__ float scratch[NT / 64];
   const int64_t t = blockIdx.x;
+  Logits<EP ? EP : 1> logits;
+  if constexpr (EP > 0) logits.load(router, route.E, d, threadIdx.x * 4);
   const P* mr = m + t * row_stride;
   float* xr = x + t * d;
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
@@ -144,6 +194,19 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
   for (int i = 0; i < NC; ++i) {
     const int c = (threadIdx.x + i * NT) * 4;
     if (c < d) store4(h + t * d + c, v[i]);
+  }
+  if constexpr (EP > 0) {
+    static_assert(NC == 1 && sizeof(T) == 2, "columns of a thread");
+    __shared__ float part[NT / 64][EP];
+    __shared__ float z[16];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[0][j] = bf2f(f2bf(v[0][j]));  // what h holds
+    logits.template row<NT>(v[0], part, z);
+    if (threadIdx.x < 16) {  // one wave: its LDS in order
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      choose<16, 1>(z, threadIdx.x, t, route);
+    }
   }
 }
 
@@ -201,19 +264,41 @@ int omnia_rms_embed(void* h, float* x, const int* ids, const void* table, int f3
   return (int)hipGetLastError();
 }
 
-// ptype: storage of `m` -- 0 bf16, 1 fp32, 2 fp16 (slabs)
+// ptype: storage of `m` -- 0 bf16, 1 fp32, 2 fp16 (slabs).  router: null, or [E, d] bf16: the rows'
+// experts as omnia_moe_route chooses them; -3 where that kernel has to
 int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int S,
                        int64_t row_stride, int64_t part_stride, int rows, int d,
                        const float* bias, const float* w_post, const float* w_pre, float inv_n, float eps,
+                       const void* router, int* ids, float* wts, int E, int k, int sigmoid, int renorm,
+                       const float* corr, int groups, int keep, const float* rbias,
                        hipStream_t s) {
   if (d % 4 || d < 4 || d > 16384 || S < 1 || row_stride % 4 || part_stride % 4 || !w_post)
     return -1;
   if (f32 && ptype != 1) return -2;
   if (rows == 0) return 0;
   const Norm post{w_post, inv_n, eps}, pre{w_pre, inv_n, eps};
-#define OMNIA_RR(TT, PP, NT, N)                                                                 \
-  residual_kernel<TT, PP, NT, N><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride,    \
-                                                  part_stride, d, bias, post, pre)
+  const Route route{ids, wts, corr, rbias, E, k, sigmoid, renorm, groups, keep};
+#define OMNIA_RE(TT, PP, NT, N, EP)                                                             \
+  residual_kernel<TT, PP, NT, N, EP><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride, \
+                                                         part_stride, d, bias, post, pre,       \
+                                                         (const bf16_t*)router, route)
+  if (router) {
+    // rows of one chunk of 4 columns a thread, up to 512 of them: beyond, a kernel that reads the
+    // router once for 16 rows
+    if (f32 || rows > 512 || d > 4096 || d % 32 || E < 1 || E > 16 || k < 1 || k > E) return -3;
+    if (groups < 1 || E % groups || keep < 1 || keep > groups || k > keep * (E / groups)) return -4;
+#define OMNIA_RT(EP)                                           \
+  do {                                                         \
+    if (ptype == 0) OMNIA_RE(bf16_t, bf16_t, 1024, 1, EP);     \
+    else if (ptype == 1) OMNIA_RE(bf16_t, float, 1024, 1, EP); \
+    else OMNIA_RE(bf16_t, _Float16, 1024, 1, EP);              \
+  } while (0)
+    if (E <= 8) OMNIA_RT(8);
+    else OMNIA_RT(16);
+#undef OMNIA_RT
+    return (int)hipGetLastError();
+  }
+#define OMNIA_RR(TT, PP, NT, N) OMNIA_RE(TT, PP, NT, N, 0)
 #define OMNIA_RRN(NT, N)                                       \
   do {                                                      \
     if (f32) OMNIA_RR(float, float, NT, N);                     \
@@ -224,6 +309,7 @@ int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int
   OMNIA_NC(OMNIA_RRN);
 #undef OMNIA_RRN
 #undef OMNIA_RR
+#undef OMNIA_RE
   return (int)hipGetLastError();
 }
 

@@ -100,14 +100,44 @@ def rms_embed(ids, table, vocab: int, emb: RMSNorm, pre: RMSNorm | None, src=Non
     return x, (x if pre is None else ref.rms_norm(x, pre)).to(table.dtype)
 
 
+# widths beyond and up to which, and rows up to which, the residual kernel takes a thread for 4 columns
+# and routes a row beside (see rms_residual.hip)
+ROUTE_ROWS = 1024, 4096, 512
+
+
+class Routing:
+    """What a step's rows are routed by (an expert feed-forward's tensors and spec); ``ids`` and
+    ``wts`` [M, top], once a kernel ahead of the experts has chosen them."""
+
+    __slots__ = ("w", "spec", "ids", "wts")
+
+    def __init__(self, w: dict, spec):
+        self.w, self.spec, self.ids, self.wts = w, spec, None, None
+
+    def empty(self, rows: int, device):
+        k = self.spec.top
+        return (torch.empty(rows, k, dtype=torch.int32, device=device),
+                torch.empty(rows, k, dtype=torch.float32, device=device))
+
+
 def rms_residual(x, m, post: RMSNorm, pre: RMSNorm | None, dtype, bias=None,
-                 slots: bool = False):
+                 slots: bool = False, route: Routing | None = None):
     """In place ``x += post(m + bias)``; returns ``pre(x)``, or x itself, in ``dtype``.  ``m``: a
-    projection [M, d], its split-K slabs [S, M, d], or (``slots``) parts [M, S, d]."""
+    projection [M, d], its split-K slabs [S, M, d], or (``slots``) parts [M, S, d].  ``route``: the
+    rows' experts as well, on the GPU for few rows and experts."""
     if x.is_cuda:
         h = torch.empty(x.shape, dtype=dtype, device=x.device)
-        kernels().rms_residual(h, x, m, slots, bias, post.w, None if pre is None else pre.w,
-                               post.inv_n, post.eps)
+        args = (h, x, m, slots, bias, post.w, None if pre is None else pre.w, post.inv_n, post.eps)
+        if route is not None and ROUTE_ROWS[0] < x.shape[1] <= ROUTE_ROWS[1] and \
+                x.shape[0] <= ROUTE_ROWS[2] and dtype == torch.bfloat16:
+            s, w = route.spec, route.w
+            ids, wts = route.empty(x.shape[0], x.device)
+            if kernels().rms_residual(*args, w["router"], ids, wts, s.top, s.score == "sigmoid",
+                                      s.renorm, w.get("correction"), s.groups, s.keep,
+                                      w.get("router_b")):
+                route.ids, route.wts = ids, wts
+                return h
+        kernels().rms_residual(*args)
         return h
     v = m.float().sum(1) if slots else ref.slab_sum(m)
     if bias is not None:
@@ -189,7 +219,7 @@ def joined_residual(x, parts, pres, dtype, enter: PassInput | None = None, fresh
 
 
 def norm_residual(x, m=None, post=None, pre=None, dtype=None, bias=None, slots: bool = False,
-                  identity=None, branches=None):
+                  identity=None, branches=None, route: Routing | None = None):
     """What follows a sublayer, of either norm kind (see the functions above)."""
     if branches is not None:
         if post is not None:
@@ -199,7 +229,7 @@ def norm_residual(x, m=None, post=None, pre=None, dtype=None, bias=None, slots: 
         return tanh_norm_residual(x, m, post, pre, dtype, bias, slots, identity)
     if post is None or identity is not None:
         raise ValueError("RMS residual steps need a post-norm and no identity parts")
-    return rms_residual(x, m, post, pre, dtype, bias, slots)
+    return rms_residual(x, m, post, pre, dtype, bias, slots, route)
 
 
 def softcap_(logits: torch.Tensor, cap: float) -> torch.Tensor:
@@ -211,22 +241,23 @@ def softcap_(logits: torch.Tensor, cap: float) -> torch.Tensor:
 
 
 # -------------------------------------------------------------------- experts
-def experts(h, w: dict, spec, streams=None):
+def experts(h, w: dict, spec, streams=None, route: Routing | None = None):
     """Routed experts: (parts [T, top, d], ids, weights), the parts summed by the residual
     kernel; those of identity experts (ids >= spec.experts) are not written.  The weights
     are padded to whole tiles (``ff_pad``; d a multiple of 64); ``streams``: copies of both by
-    :func:`omnia_amd.ops.stream_pack`, or None."""
+    :func:`omnia_amd.ops.stream_pack`, or None; ``route``: the rows' experts, if chosen before."""
     T, d = h.shape
     k, E, ff = spec.top, spec.outputs, w["down"].shape[2]
     corr, bias = w.get("correction"), w.get("router_b")
     if not h.is_cuda:
         ids, wts = ref.route(h, w["router"], spec, corr, bias)
         return ref.experts(h, ids, wts, w["up"], w["down"], spec), ids, wts
-    kk = kernels()
-    ids = torch.empty(T, k, dtype=torch.int32, device=h.device)
-    wts = torch.empty(T, k, dtype=torch.float32, device=h.device)
-    kk.moe_route(ids, wts, h, w["router"], k, spec.score == "sigmoid", spec.renorm, corr,
-                 spec.groups, spec.keep, bias)
+    if route is not None and route.ids is not None:
+        ids, wts = route.ids, route.wts
+    else:
+        ids, wts = Routing(w, spec).empty(T, h.device)
+        kernels().moe_route(ids, wts, h, w["router"], k, spec.score == "sigmoid", spec.renorm,
+                            corr, spec.groups, spec.keep, bias)
     # column tiles of the 256-row prefill GEMM: 128 gate and up columns, or 256
     tile = h.dtype == torch.bfloat16 and d % 256 == 0 and \
         T * k >= moe_tile_rows(spec.experts, d) * E and _on_grid(w["up"], w["down"]) and \
