@@ -185,6 +185,11 @@ int omnia_delta_step_conv(void* y, float* state, void* conv_state, const void* x
                           const int* slots, int T, int KH, int H, int D, int V, int Vs, int Vp,
                           int taps, float eps, hipStream_t s);
 int64_t omnia_delta_records(int n_rows, int nseq, int H);
+int omnia_delta_prep_blocks(float* rec, float* qn, float* kn, void* vc, const void* x, int f32,
+                            int64_t ldx, const void* conv_w, const void* conv_state,
+                            const float* a_log, const float* dt_bias, const int* q_start, int nseq,
+                            const int* positions, const int* slots, int T, int KH, int H, int D,
+                            int Dp, int V, int taps, hipStream_t s);
 int omnia_delta_scan(float* o, float* state, void* conv_state, float* rec, const float* qn,
                      const float* kn, const void* vc, const float* decay, const float* beta,
                      const void* x, int f32, int64_t ldx, const int* q_start, int nseq,
@@ -1785,8 +1790,35 @@ bool delta_step_conv(at::Tensor y, at::Tensor state, at::Tensor conv_state, at::
   return true;
 }
 
+// delta_prep of sequences' rows and the block records of delta_scan in one launch; false: sizes that
+// need delta_prep
+bool delta_prep_blocks(at::Tensor rec, at::Tensor qn, at::Tensor kn, at::Tensor vc, at::Tensor x,
+                       at::Tensor conv_w, at::Tensor conv_state, at::Tensor a_log,
+                       at::Tensor dt_bias, at::Tensor q_start, at::Tensor positions,
+                       at::Tensor slots, int64_t KH, int64_t H, int64_t D, int64_t Dp, int64_t V,
+                       int64_t taps) {
+  const int f32 = is_f32(x, "x");
+  const int64_t T = positions.numel(), C = 2 * KH * D + H * V, nseq = slots.numel();
+  const int64_t ld = rows2(x, T, C + H * V + 2 * H, "x");
+  like(conv_w, x, C * taps, "conv_w");
+  like(vc, x, T * H * V, "vc");
+  TORCH_CHECK(conv_state.is_contiguous() && conv_state.scalar_type() == x.scalar_type() &&
+              conv_state.dim() == 3 && conv_state.size(1) == taps - 1 && conv_state.size(2) == C,
+              "conv_state [slots, taps-1, C]");
+  const int rc = omnia_delta_prep_blocks(
+      outf(rec, omnia_delta_records(T, nseq, H), "rec"), outf(qn, T * KH * Dp, "qn"),
+      outf(kn, T * KH * Dp, "kn"), vc.data_ptr(), x.data_ptr(), f32, ld, conv_w.data_ptr(),
+      conv_state.data_ptr(), vecf(a_log, H, "a_log"), vecf(dt_bias, H, "dt_bias"),
+      veci(q_start, nseq + 1, "q_start"), nseq, veci(positions, T, "positions"),
+      veci(slots, nseq, "slots"), T, KH, H, D, Dp, V, taps, cur_stream());
+  if (rc == -3) return false;
+  CHECK_RC(rc, "delta_prep_blocks");
+  return true;
+}
+
+// decay and beta None: rec holds the records (delta_prep_blocks)
 void delta_scan(at::Tensor o, at::Tensor state, at::Tensor conv_state, at::Tensor rec, at::Tensor qn,
-                at::Tensor kn, at::Tensor vc, at::Tensor decay, at::Tensor beta, at::Tensor x,
+                at::Tensor kn, at::Tensor vc, OptT decay, OptT beta, at::Tensor x,
                 at::Tensor q_start, at::Tensor positions, at::Tensor slots, int64_t KH, int64_t H,
                 int64_t D, int64_t Dp, int64_t V, int64_t taps) {
   const int f32 = is_f32(x, "x");
@@ -1794,11 +1826,13 @@ void delta_scan(at::Tensor o, at::Tensor state, at::Tensor conv_state, at::Tenso
   const int64_t ld = rows2(x, T, C + H * V + 2 * H, "x"), nseq = slots.numel();
   check_state(state, conv_state, x, H, D, Vs, taps, C);
   like(vc, x, T * H * V, "vc");
+  TORCH_CHECK(decay.has_value() == beta.has_value(), "decay and beta, or neither");
   CHECK_RC(omnia_delta_scan(outf(o, T * H * Vs, "o"), state.data_ptr<float>(),
                             conv_state.data_ptr(),
                             outf(rec, omnia_delta_records(T, nseq, H), "rec"),
                             vecf(qn, T * KH * Dp, "qn"), vecf(kn, T * KH * Dp, "kn"), vc.data_ptr(),
-                            vecf(decay, T * H, "decay"), vecf(beta, T * H, "beta"), x.data_ptr(),
+                            decay ? vecf(*decay, T * H, "decay") : nullptr,
+                            beta ? vecf(*beta, T * H, "beta") : nullptr, x.data_ptr(),
                             f32, ld, veci(q_start, nseq + 1, "q_start"), nseq,
                             veci(positions, T, "positions"), veci(slots, nseq, "slots"), T, KH, H,
                             D, Dp, V, Vs, taps, cur_stream()), "delta_scan");
@@ -2181,6 +2215,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("delta_prep", &delta_prep);
   m.def("delta_step", &delta_step);
   m.def("delta_step_conv", &delta_step_conv);
+  m.def("delta_prep_blocks", &delta_prep_blocks);
   m.def("delta_scan", &delta_scan);
   m.def("delta_norm", &delta_norm);
   m.def("latent_prep", &latent_prep);

@@ -7,7 +7,8 @@
 // unit vectors per head.  One fused input projection feeds it, a row of
 //     [q (KH*D) | k (KH*D) | v (H*V) | z (H*V) | b (H) | a (H)]     (row stride ldx).
 //
-//   delta_prep   convolutions, unit norms, decay and step size of every token
+//   delta_prep   convolutions, unit norms, decay and step size of every token (few rows of
+//                sequences: delta_prep_blocks, with the blocks' systems of delta_scan)
 //   delta_step   decode: one token per sequence -- state update, per-head RMS norm and
 //                the silu(z) output gate in one launch, one workgroup per (row, head)
 //   delta_scan   prefill: each sequence's new tokens in blocks of 16, the state in MFMA
@@ -687,6 +688,48 @@ __device__ __forceinline__ float4v mfma4(float a, float b, float4v c) {
 // first record of sequence s: leaves room for every earlier sequence's ragged block
 __device__ __forceinline__ int rec_base(const int* q_start, int s) { return q_start[s] / 16 + s; }
 
+// A block's record, by one wave, from its products k.k and q.k (lane: column c16, rows 4 g4 ..) and
+// token c16's log decay and step size; Ls: LDS of this wave
+__device__ __forceinline__ void record(float* __restrict__ R, float4v kk, float4v qk, float c,
+                                       float bt, float (*Ls)[20]) {
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    const float up = __shfl_up(c, o, 16);
+    if (c16 >= o) c += up;
+  }
+  // lane: column i = c16, rows t = 4 g4 + r
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = 4 * g4 + r;
+    const float ct = __shfl(c, t, 16), btt = __shfl(bt, t, 16);
+    const float e = c16 <= t ? expf(ct - c) : 0.f;
+    Ls[t][c16] = c16 < t ? btt * e * kk[r] : 0.f;
+    R[256 + t * 16 + c16] = e * qk[r];
+  }
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS writes
+  float T[16];  // column c16 of the inverse, by forward substitution
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    float a = t == c16 ? 1.f : 0.f;
+#pragma unroll
+    for (int i = 0; i < t; i += 4) {
+      const float4v l = *reinterpret_cast<const float4v*>(&Ls[t][i]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (i + r < t) a -= l[r] * T[i + r];
+    }
+    T[t] = a;
+  }
+  if (g4 == 0) {
+#pragma unroll
+    for (int t = 0; t < 16; ++t) R[t * 16 + c16] = T[t] * bt;
+    R[512 + c16] = expf(c);
+    R[528 + c16] = expf(__shfl(c, 15, 16) - c);
+  }
+}
+
 // grid (records, ceil(H / 4)): one wave per (block, head)
 template <int ND>
 __global__ __launch_bounds__(256) void blocks_kernel(float* __restrict__ rec,
@@ -726,44 +769,134 @@ __global__ __launch_bounds__(256) void blocks_kernel(float* __restrict__ rec,
       qk = mfma4(b[r], a[r], qk);
     }
   }
-  const float bt = in ? beta[row * H + h] : 0.f;
-  float c = in ? decay[row * H + h] : 0.f;
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-    const float up = __shfl_up(c, o, 16);
-    if (c16 >= o) c += up;
+  record(rec + ((int64_t)id * H + h) * kRec, kk, qk, in ? decay[row * H + h] : 0.f,
+         in ? beta[row * H + h] : 0.f, Ls[w]);
+}
+
+// delta_prep and blocks_kernel in one launch: a block makes the 16 tokens of a record for one key head
+// and its R heads.  Four waves a unit (q, k, each head's v), four tokens each, whose inputs are loaded
+// up front; normed q and k go to memory for the scan and to LDS, from which wave r makes head r's
+// record.  D, V <= 128.  Bound by the chain of its loads and of the record's substitution; what it saves
+// is a launch and the way of q and k through memory (figures at its rule).
+template <typename T, int TAPS, int R>
+__global__ __launch_bounds__(256 * (2 + R)) void prep_blocks_kernel(
+    float* __restrict__ rec, float* __restrict__ qn, float* __restrict__ kn, T* __restrict__ vc,
+    const T* __restrict__ x, int64_t ldx, const T* __restrict__ conv_w,
+    const T* __restrict__ conv_state, const float* __restrict__ a_log,
+    const float* __restrict__ dt_bias, Rows rows, int KH, int D, int Dp, int V) {
+  constexpr int TR = 4, LS = 132;
+  __shared__ __attribute__((aligned(16))) float qk[2][16][LS];
+  __shared__ __attribute__((aligned(16))) float Ls[R][16][20];
+  __shared__ float gates[2][R][16];
+  const int id = blockIdx.x, kh = blockIdx.y, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = w >> 2;
+  int lo = 0, hi = rows.nseq - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (rec_base(rows.q_start, mid) <= id) lo = mid; else hi = mid - 1;
   }
-  float* R = rec + ((int64_t)id * H + h) * kRec;
-  // lane: column i = c16, rows t = 4 g4 + r
+  const int row0 = rows.q_start[lo], first = row0 + (id - rec_base(rows.q_start, lo)) * 16;
+  const int m = min(16, rows.q_start[lo + 1] - first);
+  if (m <= 0) return;  // the whole block
+  const int H = KH * R, C = 2 * KH * D + H * V;
+  const bool isv = u >= 2;
+  const int n = isv ? V : D, i = 2 * lane, r0 = TR * (w & 3), nt = min(TR, m - r0), t0 = first + r0;
+  const int c0 = (isv ? 2 * KH * D + (kh * R + u - 2) * V : (u * KH + kh) * D) + i;
+  const bool lives = i < n;
+  float wt[2][TAPS], in[TR][2], hist[TAPS - 1][2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int t = 4 * g4 + r;
-    const float ct = __shfl(c, t, 16), btt = __shfl(bt, t, 16);
-    const float e = c16 <= t ? expf(ct - c) : 0.f;
-    Ls[w][t][c16] = c16 < t ? btt * e * kk[r] : 0.f;
-    R[256 + t * 16 + c16] = e * qk[r];
+  for (int r = 0; r < TR; ++r) {
+    in[r][0] = in[r][1] = 0.f;
+    if (lives && r < nt) Vec<T, 2>::ld(in[r], x + (int64_t)(t0 + r) * ldx + c0);
   }
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS writes
-  float T[16];  // column c16 of the inverse, by forward substitution
 #pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    float a = t == c16 ? 1.f : 0.f;
+  for (int v = 0; v < 2 * TAPS; v += 2) {
+    float t2[2] = {0.f, 0.f};
+    if (lives) Vec<T, 2>::ld(t2, conv_w + (int64_t)c0 * TAPS + v);
+    wt[v / TAPS][v % TAPS] = t2[0];
+    wt[(v + 1) / TAPS][(v + 1) % TAPS] = t2[1];
+  }
 #pragma unroll
-    for (int i = 0; i < t; i += 4) {
-      const float4v l = *reinterpret_cast<const float4v*>(&Ls[w][t][i]);
+  for (int j = 0; j < TAPS - 1; ++j) hist[j][0] = hist[j][1] = 0.f;
+  if (t0 - row0 >= TAPS - 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (i + r < t) a -= l[r] * T[i + r];
+    for (int j = 0; j < TAPS - 1; ++j)
+      if (lives && nt > 0) Vec<T, 2>::ld(hist[j], x + (int64_t)(t0 - (TAPS - 1 - j)) * ldx + c0);
+  } else {  // inputs before the sequence's new tokens
+    const int slot = rows.slots[lo];
+    const bool fresh = slot < 0 || rows.positions[row0] == 0;
+    const T* cs = conv_state + (int64_t)(slot < 0 ? 0 : slot) * (TAPS - 1) * C;
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int r = t0 - (TAPS - 1 - j);
+      const T* src = r >= row0 ? x + (int64_t)r * ldx : cs + (int64_t)(TAPS - 1 - (row0 - r)) * C;
+      if (lives && (r >= row0 || !fresh)) Vec<T, 2>::ld(hist[j], src + c0);
     }
-    T[t] = a;
   }
-  if (g4 == 0) {
+  if (w == 8 && lane < 16 * R) {
+    const int tt = lane & 15, h = kh * R + (lane >> 4);
+    float dec = 0.f, bt = 0.f;
+    if (tt < m) {
+      const T* xr = x + (int64_t)(first + tt) * ldx + C + H * V;
+      bt = sigmoidf_(ldf(xr + h));
+      const float z = ldf(xr + H + h) + dt_bias[h];
+      const float sp = z > 20.f ? z : log1pf(expf(z));
+      dec = -expf(a_log[h]) * sp;
+    }
+    gates[0][lane >> 4][tt] = dec;
+    gates[1][lane >> 4][tt] = bt;
+  }
 #pragma unroll
-    for (int t = 0; t < 16; ++t) R[t * 16 + c16] = T[t] * bt;
-    R[512 + c16] = expf(c);
-    R[528 + c16] = expf(__shfl(c, 15, 16) - c);
+  for (int r = 0; r < TR; ++r) {
+    float y[2], ss = 0.f;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      float a = in[r][v] * wt[v][TAPS - 1];
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) a += hist[j][v] * wt[v][j];
+      a = siluf_(a);
+      y[v] = a;
+      ss += a * a;
+#pragma unroll
+      for (int j = 0; j + 1 < TAPS - 1; ++j) hist[j][v] = hist[j + 1][v];
+      hist[TAPS - 2][v] = in[r][v];
+    }
+    if (isv) {
+      if (lives && r < nt)
+        Vec<T, 2>::st(vc + (int64_t)(t0 + r) * H * V + (c0 - 2 * KH * D), y);
+      continue;
+    }
+    ss = row_sum16(ss);
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    float inv = 1.f / sqrtf(ss + 1e-6f);
+    if (u == 0) inv *= 1.f / sqrtf((float)D);
+    y[0] = r < nt ? y[0] * inv : 0.f;  // columns past D are zeros by their inputs
+    y[1] = r < nt ? y[1] * inv : 0.f;
+    Vec<float, 2>::st(&qk[u][r0 + r][i], y);
+    if (r < nt) {
+      float* o = (u == 0 ? qn : kn) + ((int64_t)(t0 + r) * KH + kh) * Dp;
+      if (lives) Vec<float, 2>::st(o + i, y);
+      for (int j = n + lane; j < Dp; j += 64) o[j] = 0.f;
+    }
   }
+  __syncthreads();
+  if (w >= R) return;
+  const int c16 = lane & 15, g4 = lane >> 4;
+  float4v kk = {0.f, 0.f, 0.f, 0.f}, pk = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (16 * j >= Dp) break;
+    const float4v b = *reinterpret_cast<const float4v*>(&qk[0][c16][16 * j + 4 * g4]);
+    const float4v a = *reinterpret_cast<const float4v*>(&qk[1][c16][16 * j + 4 * g4]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      kk = mfma4(a[r], a[r], kk);
+      pk = mfma4(b[r], a[r], pk);
+    }
+  }
+  record(rec + ((int64_t)id * H + kh * R + w) * kRec, kk, pk, gates[0][w][c16], gates[1][w][c16],
+         Ls[w]);
 }
 
 // Rows of a tensor as a buffer: reads past ``bytes`` give 0, writes there do nothing.
@@ -1150,6 +1283,32 @@ int prep(float* qn, float* kn, void* vc, float* decay, float* beta, const void* 
   return (int)hipGetLastError();
 }
 
+// -3: not covered (delta_prep, and blocks_kernel at the scan, cover all)
+template <typename T>
+int prep_blocks(float* rec, float* qn, float* kn, void* vc, const void* x, int64_t ldx,
+                const void* conv_w, const void* conv_state, const float* a_log,
+                const float* dt_bias, Rows r, int T_, int KH, int H, int D, int Dp, int V, int taps,
+                hipStream_t s) {
+  if (D > 128 || V > 128 || D % 2 || V % 2 || Dp > 128) return -3;
+  const dim3 grid(T_ / 16 + r.nseq, KH);
+  // While the chip holds about all waves at once (8192): beyond, most of a block's waves wait for the
+  // few that make its records (us of prep, records and scan, two launches before the scan / one: 8 key
+  // heads of two of 128, 20 rows 16.4 / 13.0, 200 25.6 / 21.4, 3 x 333 (8320 waves) 48.0 / 43.5, 2000
+  // (16128) 111.5 / 111.9, 8 x 1000 192 / 202; of one, 3 x 333 (6240) 38.4 / 32.0, 2000 (12096) 109.7 /
+  // 109.9, 8 x 512 75.6 / 82.0; 2 of two, 8 x 512 (8448) 50.5 / 44.0, 8 x 1000 (16256) 74.8 / 72.2)
+  if ((int64_t)grid.x * KH * 4 * (2 + H / KH) > 10240) return -3;
+#define OMNIA_PB(TAPS, R)                                                                         \
+  if (taps == TAPS && H == R * KH) {                                                              \
+    prep_blocks_kernel<T, TAPS, R><<<grid, 256 * (2 + R), 0, s>>>(                                \
+        rec, qn, kn, (T*)vc, (const T*)x, ldx, (const T*)conv_w, (const T*)conv_state, a_log,     \
+        dt_bias, r, KH, D, Dp, V);                                                                \
+    return (int)hipGetLastError();                                                                \
+  }
+  OMNIA_PB(2, 1) OMNIA_PB(3, 1) OMNIA_PB(4, 1) OMNIA_PB(2, 2) OMNIA_PB(3, 2) OMNIA_PB(4, 2)
+#undef OMNIA_PB
+  return -3;
+}
+
 template <typename T>
 int step(void* y, float* state, void* conv_state, const float* qn, const float* kn, const void* vc,
          const float* decay, const float* beta, const void* x, int64_t ldx, const float* norm_w,
@@ -1215,8 +1374,9 @@ int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, 
                                               Vs, taps)
 #define OMNIA_SCANB(ND)                                                                         \
   if (D <= 16 * ND) {                                                                           \
-    blocks_kernel<ND><<<bgrid, 256, 0, s>>>(rec, qn, kn, decay, beta, r.q_start, r.nseq, KH, H, \
-                                            Dp);                                                \
+    if (decay)                                                                                  \
+      blocks_kernel<ND><<<bgrid, 256, 0, s>>>(rec, qn, kn, decay, beta, r.q_start, r.nseq, KH,  \
+                                              H, Dp);                                           \
     if (few)                                                                                    \
       OMNIA_SPLIT(ND, (ND < 4 ? 2 : 4), 1);                                                     \
     else                                                                                        \
@@ -1226,6 +1386,7 @@ int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, 
   OMNIA_SCANB(2) OMNIA_SCANB(4) OMNIA_SCANB(8) OMNIA_SCANB(16)
 #undef OMNIA_SCANB
 #undef OMNIA_SPLIT
+  if (!decay) return -5;
   const dim3 grid((Vs + 15) / 16, H, r.nseq);
 #define OMNIA_SCAN(N)                                                                           \
   if (D <= 64 * N) {                                                                            \
@@ -1291,11 +1452,30 @@ int omnia_delta_step_conv(void* y, float* state, void* conv_state, const void* x
                            H, D, V, Vs, Vp, taps, eps, s);
 }
 
+// omnia_delta_prep of sequences' rows, and the block records of omnia_delta_scan, in one launch; -3
+// where it does not cover the sizes (checked before any launch)
+int omnia_delta_prep_blocks(float* rec, float* qn, float* kn, void* vc, const void* x, int f32,
+                            int64_t ldx, const void* conv_w, const void* conv_state,
+                            const float* a_log, const float* dt_bias, const int* q_start, int nseq,
+                            const int* positions, const int* slots, int T, int KH, int H, int D,
+                            int Dp, int V, int taps, hipStream_t s) {
+  if (taps < 1 || KH < 1 || H % KH || Dp % 4 || Dp < D) return -1;
+  if (KH > 65535) return -2;
+  if (T == 0 || nseq == 0) return 0;
+  const Rows r{q_start, nseq, positions, slots};
+  if (f32)
+    return prep_blocks<float>(rec, qn, kn, vc, x, ldx, conv_w, conv_state, a_log, dt_bias, r, T, KH,
+                              H, D, Dp, V, taps, s);
+  return prep_blocks<bf16_t>(rec, qn, kn, vc, x, ldx, conv_w, conv_state, a_log, dt_bias, r, T, KH,
+                             H, D, Dp, V, taps, s);
+}
+
 // floats of the block records of n_rows rows in nseq sequences
 int64_t omnia_delta_records(int n_rows, int nseq, int H) {
   return (int64_t)(n_rows / 16 + nseq) * H * kRec;
 }
 
+// decay and beta null: rec holds the records (omnia_delta_prep_blocks)
 int omnia_delta_scan(float* o, float* state, void* conv_state, float* rec, const float* qn,
                      const float* kn, const void* vc, const float* decay, const float* beta,
                      const void* x, int f32, int64_t ldx, const int* q_start, int nseq,

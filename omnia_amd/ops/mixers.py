@@ -301,16 +301,21 @@ def delta_rule(x, w: dict, spec, state, conv_state, q_start, positions, slots, e
     qn = torch.empty(T, KH, Dp, dtype=torch.float32, device=dev)
     kn = torch.empty_like(qn)
     vc = torch.empty(T, H * V, dtype=x.dtype, device=dev)
-    decay = torch.empty(T, H, dtype=torch.float32, device=dev)
-    beta = torch.empty_like(decay)
-    kk.delta_prep(qn, kn, vc, decay, beta, x, w["conv"], conv_state, w["a_log"], w["dt_bias"],
-                  q_start, positions, slots, KH, H, D, Dp, V, taps)
+    rec = decay = beta = None
+    if q_start is not None:
+        rec = torch.empty(kk.delta_records(T, slots.numel(), H), dtype=torch.float32, device=dev)
+    if rec is None or not kk.delta_prep_blocks(rec, qn, kn, vc, x, w["conv"], conv_state,
+                                               w["a_log"], w["dt_bias"], q_start, positions, slots,
+                                               KH, H, D, Dp, V, taps):
+        decay = torch.empty(T, H, dtype=torch.float32, device=dev)
+        beta = torch.empty_like(decay)
+        kk.delta_prep(qn, kn, vc, decay, beta, x, w["conv"], conv_state, w["a_log"], w["dt_bias"],
+                      q_start, positions, slots, KH, H, D, Dp, V, taps)
     if q_start is None:
         kk.delta_step(y, state, conv_state, qn, kn, vc, decay, beta, x, w["norm"], positions,
                       slots, KH, H, D, Dp, V, Vp, taps, eps)
         return y
     o = torch.empty(T, H, Vs, dtype=torch.float32, device=dev)
-    rec = torch.empty(kk.delta_records(T, slots.numel(), H), dtype=torch.float32, device=dev)
     kk.delta_scan(o, state, conv_state, rec, qn, kn, vc, decay, beta, x, q_start, positions, slots, KH,
                   H, D, Dp, V, taps)
     kk.delta_norm(y, o, x, C, w["norm"], H, V, Vs, Vp, eps)
