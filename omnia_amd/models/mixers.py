@@ -127,12 +127,16 @@ class LatentAttention(Mixer):
     def _decode(self, w, q, gate, pages, bt, positions, out):
         s = self.spec
         qa = mops.latent_absorb(q, w["uk_absorb"], s, positions, self.table)
+        parts = None
         if self.mfma_decode and pages.shape[1] & (pages.shape[1] - 1) == 0:
-            o = mops.latent_decode(qa, pages, bt, positions, s,
-                                   self.splits(q.shape[0], bt.shape[1] * pages.shape[1]))
+            n = self.splits(q.shape[0], bt.shape[1] * pages.shape[1])
+            merge = n == 1 or not mops.latent_expands_parts(s)
+            o = mops.latent_decode(qa, pages, bt, positions, s, n, merge)
+            if not merge:
+                o, parts = o
         else:
             o = mops.latent_attend(qa, pages, bt, None, positions, s)
-        return mops.latent_expand(o, w["uv"], s, gate, out)
+        return mops.latent_expand(o, w["uv"], s, gate, out, parts)
 
     def _prefill(self, w, q, gate, pages, fb, positions, out):
         s = self.spec

@@ -253,6 +253,10 @@ int omnia_latent_decode_covers(int Cp, int Lp);
 int omnia_latent_decode(void* out, float* part_o, float* part_ml, const void* q, const void* cache,
                         const int* block_tables, int bt_stride, const int* positions, int T,
                         int page, int H, int Cp, int Lp, int window, float scale, int splits,
+                        int merge, hipStream_t s);
+int omnia_latent_expand(void* out, int64_t ldo, int ho, const void* o, const float* part_o,
+                        const float* part_ml, const void* W, const void* gate, int64_t ldg,
+                        const int* positions, int T, int H, int N, int K, int window, int splits,
                         hipStream_t s);
 int omnia_latent_gather(void* c, void* kr, const void* cache, const int* block_tables,
                         int bt_stride, const int* kv_start, const int* kv_first,
@@ -1933,7 +1937,7 @@ void latent_attend(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor bl
 
 void latent_decode(at::Tensor out, OptT part_o, OptT part_ml, at::Tensor q, at::Tensor cache,
                    at::Tensor block_tables, at::Tensor positions, int64_t H, int64_t Cp,
-                   int64_t window, double scale, int64_t splits) {
+                   int64_t window, double scale, int64_t splits, bool merge) {
   CHECK_GPU(q); CHECK_BF16(q);
   check_latent(cache, q);
   const int64_t T = positions.numel(), Lp = cache.size(2);
@@ -1951,7 +1955,28 @@ void latent_decode(at::Tensor out, OptT part_o, OptT part_ml, at::Tensor q, at::
   CHECK_RC(omnia_latent_decode(out.data_ptr(), po, pm, q.data_ptr(), cache.data_ptr(),
                                tables(block_tables, T), block_tables.stride(0),
                                veci(positions, T, "positions"), T, cache.size(1), H, Cp, Lp,
-                               window, (float)scale, splits, cur_stream()), "latent_decode");
+                               window, (float)scale, splits, merge, cur_stream()),
+           "latent_decode");
+}
+
+// latents of latent_decode without its merge -> gated head outputs
+void latent_expand(at::Tensor out, int64_t ho, at::Tensor o, OptT part_o, OptT part_ml,
+                   at::Tensor W, at::Tensor gate, at::Tensor positions, int64_t window,
+                   int64_t splits) {
+  CHECK_GPU(o); CHECK_BF16(o); CHECK_BF16(out); CHECK_BF16(gate);
+  TORCH_CHECK(W.dim() == 3, "W [H, N, K]");
+  const int64_t T = positions.numel(), H = W.size(0), N = W.size(1), K = W.size(2);
+  like(W, o, W.numel(), "W");
+  like(o, o, T * H * K, "o");
+  const int64_t ldo = rows2(out, T, H * ho, "out"), ldg = rows2(gate, T, H, "gate");
+  if (splits > 1)
+    TORCH_CHECK(part_o.has_value() && part_ml.has_value() && part_o->scalar_type() == at::kFloat &&
+                part_o->numel() >= T * H * splits * K && part_ml->scalar_type() == at::kFloat &&
+                part_ml->numel() >= T * H * splits * 2, "partials for splits > 1");
+  CHECK_RC(omnia_latent_expand(out.data_ptr(), ldo, ho, o.data_ptr(), opt_ptr<float>(part_o),
+                               opt_ptr<float>(part_ml), W.data_ptr(), gate.data_ptr(), ldg,
+                               veci(positions, T, "positions"), T, H, N, K, window, splits,
+                               cur_stream()), "latent_expand");
 }
 
 void latent_gather(at::Tensor c, at::Tensor kr, at::Tensor cache, at::Tensor block_tables,
@@ -2222,7 +2247,11 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("latent_rotate", &latent_rotate);
   m.def("latent_heads", &latent_heads);
   m.def("latent_attend", &latent_attend);
-  m.def("latent_decode", &latent_decode);
+  m.def("latent_decode", &latent_decode, py::arg("out"), py::arg("part_o"), py::arg("part_ml"),
+        py::arg("q"), py::arg("cache"), py::arg("block_tables"), py::arg("positions"),
+        py::arg("H"), py::arg("Cp"), py::arg("window"), py::arg("scale"), py::arg("splits"),
+        py::arg("merge") = true);
+  m.def("latent_expand", &latent_expand);
   m.def("latent_gather", &latent_gather);
   m.def("latent_prefill", &latent_prefill);
   m.def("delta_records", &omnia_delta_records);

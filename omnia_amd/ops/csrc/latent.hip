@@ -12,6 +12,7 @@
 //   latent_attend   generic attention over absorbed queries (any size, bf16 or fp32)
 //   latent_decode   decode on MFMA: absorbed queries, all heads of a row share each
 //                   staged page tile, split over the window, + latent_merge
+//   latent_expand   decode: latent_merge and the expansion of W_uv in one launch
 //   latent_gather   cached rows of each sequence's visible range -> dense [Tk] rows
 //   latent_prefill  prefill on MFMA: expanded per-head keys and (transposed) values of
 //                   the gathered range, online softmax, window mask, output gate
@@ -45,7 +46,8 @@ __device__ __forceinline__ int find_seq(const int* q_start, int nseq, int t) {
 }
 
 // ----------------------------------------------------------------- latent_prep
-// one workgroup per token; cos_sin: [positions][R] fp32 = (cos[R/2] | sin[R/2])
+// one workgroup per token, bound by the latency of its loads, so all of a thread's are under way
+// before the first sum (64 rows of 768 + 512 + 64 4.3 -> 3.6 us); cos_sin: [positions][R] fp32 = (cos[R/2] | sin[R/2])
 template <typename T>
 __global__ __launch_bounds__(256) void prep_kernel(
     T* __restrict__ cq, T* __restrict__ cache, const T* __restrict__ x, int64_t ldx,
@@ -58,27 +60,63 @@ __global__ __launch_bounds__(256) void prep_kernel(
   const T* xc = xq + Qp;
   const T* xr = xc + Cp;
   const int64_t slot = slots[t];
-  float sq = 0.f, sc = 0.f;
-  for (int i = tid; i < Q; i += 256) {
+  const float* cs = cos_sin + (int64_t)positions[t] * R;
+  const int half = R / 2;
+  // a thread's first NV of each, all asked for before the first is waited for
+  constexpr int NV = 4;
+  float vq[NV], vc[NV], gq[NV], gc[NV], sq = 0.f, sc = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = tid + 256 * j;
+    vq[j] = vc[j] = gq[j] = gc[j] = 0.f;
+    if (i < Q) vq[j] = ldf(xq + i), gq[j] = wq[i];
+    if (i < C) vc[j] = ldf(xc + i), gc[j] = wc[i];
+  }
+  float u0 = 0.f, v0 = 0.f, c0 = 0.f, s0 = 0.f;
+  if (slot >= 0 && tid < half)
+    u0 = ldf(xr + tid), v0 = ldf(xr + half + tid), c0 = cs[tid], s0 = cs[half + tid];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    sq += vq[j] * vq[j];
+    sc += vc[j] * vc[j];
+  }
+  for (int i = tid + 256 * NV; i < Q; i += 256) {
     const float v = ldf(xq + i);
     sq += v * v;
   }
-  for (int i = tid; i < C; i += 256) {
+  for (int i = tid + 256 * NV; i < C; i += 256) {
     const float v = ldf(xc + i);
     sc += v * v;
   }
-  sq = block_sum(sq, scratch);
-  sc = block_sum(sc, scratch);
+  sq = wave_sum(sq);
+  sc = wave_sum(sc);
+  if ((tid & 63) == 0) {
+    scratch[tid >> 6] = sq;
+    scratch[4 + (tid >> 6)] = sc;
+  }
+  __syncthreads();
+  sq = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
+  sc = ((scratch[4] + scratch[5]) + scratch[6]) + scratch[7];
   const float iq = 1.f / sqrtf(sq / (float)Q + eps), ic = 1.f / sqrtf(sc / (float)C + eps);
-  for (int i = tid; i < Qp; i += 256)
-    stf(cq + (int64_t)t * Qp + i, i < Q ? ldf(xq + i) * iq * wq[i] : 0.f);
+  T* cr = cq + (int64_t)t * Qp;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = tid + 256 * j;
+    if (i < Qp) stf(cr + i, vq[j] * iq * gq[j]);
+  }
+  for (int i = tid + 256 * NV; i < Qp; i += 256) stf(cr + i, i < Q ? ldf(xq + i) * iq * wq[i] : 0.f);
   if (slot < 0) return;
   T* row = cache + slot * Lp;
-  for (int i = tid; i < C; i += 256) stf(row + i, ldf(xc + i) * ic * wc[i]);
-  const float* cs = cos_sin + (int64_t)positions[t] * R;
-  const int half = R / 2;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int i = tid + 256 * j;
+    if (i < C) stf(row + i, vc[j] * ic * gc[j]);
+  }
+  for (int i = tid + 256 * NV; i < C; i += 256) stf(row + i, ldf(xc + i) * ic * wc[i]);
   for (int i = tid; i < half; i += 256) {
-    const float u = ldf(xr + i), v = ldf(xr + half + i), c = cs[i], s = cs[half + i];
+    const bool own = i < 256;
+    const float u = own ? u0 : ldf(xr + i), v = own ? v0 : ldf(xr + half + i);
+    const float c = own ? c0 : cs[i], s = own ? s0 : cs[half + i];
     stf(row + Cp + i, u * c - v * s);
     stf(row + Cp + half + i, v * c + u * s);
   }
@@ -142,15 +180,34 @@ __global__ __launch_bounds__(256) void heads_kernel(T* __restrict__ out, int64_t
   }
 }
 
-// MFMA form (bf16): grid (ceil(N/64), H, ceil(T/16)), one wave: 16 rows x 64 columns,
-// operands straight from L2 (K is a head dimension or the latent: a few hundred),
-// four k-steps of loads in flight.  K % 32 == 0.
+// MFMA form (bf16): grid (ceil(N/64), and one for the rotated part, H, ceil(T/16)), one wave: 16 rows
+// x 64 columns, operands straight from L2 (K is a head dimension or the latent: a few hundred),
+// four k-steps of loads in flight.  K % 32 == 0.  The rotated part is a chain of small loads: in the
+// block of the first columns, behind their products, absorbing took 2.7 / 5.5 / 10.2 / 19.6 us at 1 / 64 /
+// 256 / 600 rows of 16 heads of 128 -> 512, in blocks of its own 2.6 / 4.2 / 7.7 / 16.4.
 __global__ __launch_bounds__(64) void heads_mfma_kernel(
     bf16_t* __restrict__ out, int64_t ldo, int ho, const bf16_t* __restrict__ x, int64_t ldx,
     int hx, const bf16_t* __restrict__ W, int T, int N, int K, const bf16_t* __restrict__ gate,
     int64_t ldg, Rot rot) {
   const int lane = threadIdx.x;
   const int h = blockIdx.y, n0 = blockIdx.x * 64, r0 = blockIdx.z * 16;
+  if (n0 >= N) {  // the last of a row of blocks: the rotated part
+    const int half = rot.R / 2, nr = min(16, T - r0);
+#pragma unroll 4
+    for (int e = lane; e < nr * half; e += 64) {
+      const int row = r0 + e / half, i = e % half;
+      const float* cs = rot.cos_sin + (int64_t)rot.positions[row] * rot.R;
+      const bf16_t* xr = x + (int64_t)row * ldx + h * hx + rot.rotx;
+      bf16_t* orow = out + (int64_t)row * ldo + h * ho + N;
+      const float u = ldf(xr + i), v = ldf(xr + half + i), c = cs[i], s = cs[half + i];
+      stf(orow + i, u * c - v * s);
+      stf(orow + half + i, v * c + u * s);
+    }
+    const int pad = rot.Rp + rot.tail - rot.R;
+    for (int e = lane; e < nr * pad; e += 64)
+      stf(out + (int64_t)(r0 + e / pad) * ldo + h * ho + N + rot.R + e % pad, 0.f);
+    return;
+  }
   const int fr = lane & 15, fq = lane >> 4;
   const int ra = min(r0 + fr, T - 1);
   const bf16_t* xa = x + (int64_t)ra * ldx + h * hx + 8 * fq;
@@ -189,20 +246,88 @@ __global__ __launch_bounds__(64) void heads_mfma_kernel(
       if (n < N) stf(out + (int64_t)row * ldo + h * ho + n, acc[j][r] * g);
     }
   }
-  if (rot.positions && blockIdx.x == 0) {
-    const int half = rot.R / 2, nr = min(16, T - r0);
-    for (int e = lane; e < nr * half; e += 64) {
-      const int row = r0 + e / half, i = e % half;
-      const float* cs = rot.cos_sin + (int64_t)rot.positions[row] * rot.R;
-      const bf16_t* xr = x + (int64_t)row * ldx + h * hx + rot.rotx;
-      bf16_t* orow = out + (int64_t)row * ldo + h * ho + N;
-      const float u = ldf(xr + i), v = ldf(xr + half + i), c = cs[i], s = cs[half + i];
-      stf(orow + i, u * c - v * s);
-      stf(orow + half + i, v * c + u * s);
+}
+
+// Parts of a row's keys on the device (live length), equal and 64-aligned: keys of a part.
+__device__ __forceinline__ int part_len(int n, int splits) {
+  return ((n + splits - 1) / splits + 63) / 64 * 64;
+}
+
+// latent_decode's merge and the expansion of W_uv in one launch: grid (H, ceil(T / RB)), 8 waves, RB
+// rows of a head (4, 8 or 16 of the product's 16: few rows spread over the CUs).  Wave w multiplies the
+// columns 16 w ..; its weights, all of K, are under way while the waves merge the rows' parts into LDS,
+// 256 latent columns a wave and turn.  Bound by the latency of those loads; each of the launches that it
+// stands for had one.  us of decode with merge and expansion, before / now, 16 heads of 512 -> 128, rows x
+// keys (parts): 1 x 1024 (8) 20.6 / 18.1, 4 x 4000 (32) 25.3 / 25.0, 64 x 1024 (8) 32.0 / 28.4, 256 x 1024
+// (2) 71.4 / 65.3.  Where rows have one part there is nothing to merge, and the two stay (600 x 200 53.7 /
+// 56.5, 256 x 100 22.4 / 22.0).
+__global__ __launch_bounds__(512) void expand_kernel(
+    bf16_t* __restrict__ out, int64_t ldo, int ho, const bf16_t* __restrict__ o,
+    const float* __restrict__ part_o, const float* __restrict__ part_ml,
+    const bf16_t* __restrict__ W, const bf16_t* __restrict__ gate, int64_t ldg,
+    const int* __restrict__ positions, int T, int H, int N, int K, int window, int splits, int RB) {
+  constexpr int KS = 16;  // k-steps of 32: K <= 512
+  __shared__ __attribute__((aligned(16))) bf16_t xs[16][32 * KS + 8];
+  const int h = blockIdx.x, r0 = blockIdx.y * RB, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fq = lane >> 4;
+  const int n = 16 * w + fr;
+  short8 b[KS];
+  if (16 * w < N) {
+    const bf16_t* wb = W + ((int64_t)h * N + min(n, N - 1)) * K + 8 * fq;
+#pragma unroll
+    for (int u = 0; u < KS; ++u)
+      if (32 * u < K) b[u] = *reinterpret_cast<const short8*>(wb + 32 * u);
+  }
+  float g[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    g[r] = sigmoidf_(ldf(gate + (int64_t)min(r0 + 4 * fq + r, T - 1) * ldg + h));
+  const int segs = (K + 255) / 256;
+  for (int q = w; q < RB * segs; q += 8) {  // wave-uniform
+    const int row = r0 + q / segs, c = q % segs * 256 + 4 * lane;
+    if (row >= T) break;
+    const int64_t bh = (int64_t)row * H + h;
+    const int pos = positions[row], lo = window > 0 ? max(0, pos - window + 1) : 0;
+    const int keys = max(pos + 1 - lo, 1), pl = part_len(keys, splits), np = (keys + pl - 1) / pl;
+    uint2v k = {0, 0};
+    if (np <= 1) {
+      if (c < K) k = *reinterpret_cast<const uint2v*>(o + bh * K + c);
+    } else {
+      const float* ml = part_ml + (bh * splits + min(lane, np - 1)) * 2;
+      const float m = lane < np ? ml[0] : -INFINITY, l = lane < np ? ml[1] : 0.f;
+      const float* po = part_o + bh * splits * K + min(c, K - 4);
+      float4v a = {0.f, 0.f, 0.f, 0.f};
+      float wt = 0.f;
+      for (int p0 = 0; p0 < np; p0 += 8) {
+        float4v v[8];
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+          v[p] = *reinterpret_cast<const float4v*>(po + (int64_t)min(p0 + p, np - 1) * K);
+        if (p0 == 0) {
+          wt = exp2f(m - wave_max(m)) * l;
+          wt = wt / wave_sum(wt);
+        }
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+          if (p0 + p < np) a += v[p] * __shfl(wt, p0 + p, 64);
+      }
+      k[0] = pack_bf2(a[0], a[1]);
+      k[1] = pack_bf2(a[2], a[3]);
     }
-    const int pad = rot.Rp + rot.tail - rot.R;
-    for (int e = lane; e < nr * pad; e += 64)
-      stf(out + (int64_t)(r0 + e / pad) * ldo + h * ho + N + rot.R + e % pad, 0.f);
+    if (c < K) *reinterpret_cast<uint2v*>(&xs[row - r0][c]) = k;
+  }
+  __syncthreads();
+  if (16 * w >= N) return;
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < KS; ++u)  // rows of xs past RB: of products that are not stored
+    if (32 * u < K)
+      acc = mfma16(*reinterpret_cast<const short8*>(&xs[fr][32 * u + 8 * fq]), b[u], acc);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = 4 * fq + r;
+    if (i < RB && r0 + i < T && n < N)
+      stf(out + (int64_t)(r0 + i) * ldo + h * ho + n, acc[r] * g[r]);
   }
 }
 
@@ -266,11 +391,6 @@ __global__ __launch_bounds__(256) void attend_kernel(
 //   P V  wave w owns latent column tiles w, w+4, ...; V^T fragments by
 //        ds_read_b64_tr_b16 from the row-major tile, the keys of the k-step permuted the
 //        same way on the P side
-// A row's keys are cut into equal 64-aligned parts on the device (live length).
-__device__ __forceinline__ int part_len(int n, int splits) {
-  return ((n + splits - 1) / splits + 63) / 64 * 64;
-}
-
 template <int HT, int LW>
 __global__ __launch_bounds__(256, 2) void decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -719,7 +839,7 @@ int omnia_latent_heads(void* out, int f32, int64_t ldo, int ho, const void* x, i
   if (K % 32 || ldx % 8 || hx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15)) return -3;
   const int mt = (T + 15) / 16;
   if (mt > 65535) return -4;
-  heads_mfma_kernel<<<dim3((N + 63) / 64, H, mt), 64, 0, s>>>(
+  heads_mfma_kernel<<<dim3((N + 63) / 64 + (positions ? 1 : 0), H, mt), 64, 0, s>>>(
       (bf16_t*)out, ldo, ho, (const bf16_t*)x, ldx, hx, (const bf16_t*)W, T, N, K,
       (const bf16_t*)gate, ldg, rot);
   return (int)hipGetLastError();
@@ -757,7 +877,7 @@ int omnia_latent_decode_covers(int Cp, int Lp) {
 int omnia_latent_decode(void* out, float* part_o, float* part_ml, const void* q, const void* cache,
                         const int* block_tables, int bt_stride, const int* positions, int T,
                         int page, int H, int Cp, int Lp, int window, float scale, int splits,
-                        hipStream_t s) {
+                        int merge, hipStream_t s) {
   if (!omnia_latent_decode_covers(Cp, Lp) || splits < 1 || splits > 64) return -1;
   if (page < 1 || (page & (page - 1))) return -2;
   if (T == 0) return 0;
@@ -782,9 +902,30 @@ int omnia_latent_decode(void* out, float* part_o, float* part_ml, const void* q,
   OMNIA_LATENT_WIDTHS(OMNIA_LW)
 #undef OMNIA_LW
 #undef OMNIA_LD
-  if (splits > 1)
+  if (splits > 1 && merge)
     merge_kernel<<<T * H, 128, 0, s>>>((bf16_t*)out, part_o, part_ml, positions, H, Cp, window,
                                        splits);
+  return (int)hipGetLastError();
+}
+
+// the merge of omnia_latent_decode (not yet merged) and omnia_latent_heads with W [H, N, K] of its
+// latents o [T, H, K], in one launch
+int omnia_latent_expand(void* out, int64_t ldo, int ho, const void* o, const float* part_o,
+                        const float* part_ml, const void* W, const void* gate, int64_t ldg,
+                        const int* positions, int T, int H, int N, int K, int window, int splits,
+                        hipStream_t s) {
+  if (K % 32 || K < 32 || K > 512 || N < 1 || N > 128 || ho < N) return -1;
+  if (splits < 1 || splits > 64 || (splits > 1 && (!part_o || !part_ml)) || !gate) return -2;
+  if (((uintptr_t)o | (uintptr_t)W | (uintptr_t)part_o) & 15) return -3;
+  if (T == 0) return 0;
+  // rows a block: blocks of about one a CU
+  const int64_t heads = (int64_t)T * H;
+  const int rb = heads > 8 * 256 ? 16 : heads > 4 * 256 ? 8 : 4;
+  const int64_t gy = (T + rb - 1) / rb;
+  if (gy > 65535) return -4;
+  expand_kernel<<<dim3(H, (unsigned)gy), 512, 0, s>>>(
+      (bf16_t*)out, ldo, ho, (const bf16_t*)o, part_o, part_ml, (const bf16_t*)W,
+      (const bf16_t*)gate, ldg, positions, T, H, N, K, window, splits, rb);
   return (int)hipGetLastError();
 }
 

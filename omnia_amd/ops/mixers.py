@@ -9,6 +9,8 @@ GPU tensors (bf16 or fp32) run the HIP kernels and nothing else; CPU tensors run
 :mod:`omnia_amd.ops.reference_mixers`."""
 from __future__ import annotations
 
+from typing import NamedTuple
+
 import torch
 
 from . import _moe_grouped, _on_grid, checks, kernels, moe_tile_rows
@@ -384,10 +386,15 @@ def latent_absorb(q, w_uk, spec, positions, cos_sin):
     return out
 
 
-def latent_expand(o, w_uv, spec, gate, out=None):
-    """Attended latents [T, H * latent_pad] -> gated head outputs [T, H * v_pad]."""
+def latent_expand(o, w_uv, spec, gate, out=None, parts=None):
+    """Attended latents [T, H * latent_pad] -> gated head outputs [T, H * v_pad].  ``parts``: those
+    of :func:`latent_decode`, which are merged here."""
     if out is None:
         out = torch.empty(o.shape[0], spec.heads * spec.v_pad, dtype=o.dtype, device=o.device)
+    if parts is not None:
+        kernels().latent_expand(out, spec.v_pad, o, parts.o, parts.ml, w_uv, gate, parts.positions,
+                                spec.window, parts.splits)
+        return out
     args = (out, spec.v_pad, o, spec.latent_pad, w_uv, gate, None, None, 0, 0, 0)
     (kernels().latent_heads if o.is_cuda else ref.latent_heads)(*args)
     return out
@@ -410,8 +417,22 @@ def latent_decode_covers(spec) -> bool:
     return bool(kernels().latent_decode_covers(spec.latent_pad, spec.padded_cache_width))
 
 
-def latent_decode(q, cache, block_tables, positions, spec, splits: int):
-    """MFMA decode over absorbed queries, each row's keys in up to ``splits`` parts."""
+class LatentParts(NamedTuple):
+    """Partial sums of :func:`latent_decode` (None: one part a row)."""
+    o: torch.Tensor | None
+    ml: torch.Tensor | None
+    positions: torch.Tensor
+    splits: int
+
+
+def latent_expands_parts(spec) -> bool:
+    """Whether one kernel merges parts of this size and expands them."""
+    return spec.latent_pad % 32 == 0 and spec.latent_pad <= 512 and spec.v_pad <= 128
+
+
+def latent_decode(q, cache, block_tables, positions, spec, splits: int, merge: bool = True):
+    """MFMA decode over absorbed queries, each row's keys in up to ``splits`` parts.  ``merge``
+    False: (latents, :class:`LatentParts`) for :func:`latent_expand`."""
     T, H, Cp = positions.numel(), spec.heads, spec.latent_pad
     out = torch.empty(T, H * Cp, dtype=q.dtype, device=q.device)
     po = pm = None
@@ -419,8 +440,8 @@ def latent_decode(q, cache, block_tables, positions, spec, splits: int):
         po = torch.empty(T * H * splits * Cp, dtype=torch.float32, device=q.device)
         pm = torch.empty(T * H * splits * 2, dtype=torch.float32, device=q.device)
     kernels().latent_decode(out, po, pm, q, cache, block_tables, positions, H, Cp, spec.window,
-                            spec.scale, splits)
-    return out
+                            spec.scale, splits, merge)
+    return out if merge else (out, LatentParts(po, pm, positions, splits))
 
 
 def latent_gather(cache, block_tables, kv_start, kv_first, seq_lens, rows: int, spec):
