@@ -1336,8 +1336,9 @@ int step_conv(void* y, float* state, void* conv_state, const void* x, int64_t ld
               const void* conv_w, const float* a_log, const float* dt_bias, const float* norm_w,
               Rows r, int T_, int KH, int H, int D, int V, int Vs, int Vp, int taps, float eps,
               hipStream_t s) {
+  if (D > 128 || V > 128 || D % 2 || V % 2 || taps < 2 || taps > 4 || Vs / 4 > 256) return -3;
   const int CG = Vs / 4, RG = 256 / CG, nr = (D + RG - 1) / RG, R = H / KH;
-  if (D > 128 || V > 128 || D % 2 || V % 2 || taps < 2 || taps > 4 || nr > 16) return -3;
+  if (nr > 16) return -3;
   // blocks of several heads read and write in step with one another: in two rounds of the chip (four
   // heads a CU) that costs what the launch does (112 / 128 / 144 rows, two kernels and one: 49.8 /
   // 53.3 / 65.1 and 49.8 / 54.4 / 63.1)
@@ -1424,7 +1425,8 @@ int omnia_delta_step(void* y, float* state, void* conv_state, const float* qn, c
                      int64_t ldx, const float* norm_w, const int* positions, const int* slots,
                      int T, int KH, int H, int D, int Dp, int V, int Vs, int Vp, int taps,
                      float eps, hipStream_t s) {
-  if (taps < 1 || KH < 1 || H % KH || Dp % 4 || Dp < D || Vs % 4 || Vs < V || Vp < V) return -1;
+  if (taps < 1 || KH < 1 || H % KH || Dp % 4 || Dp < D || Vs < 4 || Vs % 4 || Vs < V || Vp < V)
+    return -1;
   if (Vs / 4 > 256) return -2;
   if (T == 0) return 0;
   const Rows r{nullptr, T, positions, slots};
@@ -1442,7 +1444,7 @@ int omnia_delta_step_conv(void* y, float* state, void* conv_state, const void* x
                           const float* dt_bias, const float* norm_w, const int* positions,
                           const int* slots, int T, int KH, int H, int D, int V, int Vs, int Vp,
                           int taps, float eps, hipStream_t s) {
-  if (KH < 1 || H % KH || Vs % 4 || Vs < V || Vp < V) return -1;
+  if (KH < 1 || H % KH || Vs < 4 || Vs % 4 || Vs < V || Vp < V) return -1;
   if (T == 0) return 0;
   const Rows r{nullptr, T, positions, slots};
   if (f32)

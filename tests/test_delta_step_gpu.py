@@ -57,7 +57,7 @@ def test_step(T, D, V, KH, H, taps, dtype):
 
 @pytest.mark.parametrize("T,D,V,KH,H,taps", [
     (1, 130, 64, 1, 1, 4), (1, 64, 130, 1, 1, 4), (1, 63, 64, 1, 1, 4), (1, 64, 64, 1, 3, 4),
-    (1, 64, 64, 1, 1, 5), (120, 64, 64, 8, 16, 4)])
+    (1, 64, 64, 1, 1, 5), (1, 64, 1028, 1, 1, 4), (120, 64, 64, 8, 16, 4)])
 def test_sizes_left_to_the_two_kernels(T, D, V, KH, H, taps):
     k, dev = ops.kernels(), "cuda"
     C, Vs, Vp = 2 * KH * D + H * V, -(-V // 4) * 4, -(-V // 8) * 8
