@@ -1299,6 +1299,7 @@ int prep_blocks(float* rec, float* qn, float* kn, void* vc, const void* x, int64
   if ((int64_t)grid.x * KH * 4 * (2 + H / KH) > 10240) return -3;
 #define OMNIA_PB(TAPS, R)                                                                         \
   if (taps == TAPS && H == R * KH) {                                                              \
+    if (T_ == 0 || r.nseq == 0) return 0;                                                         \
     prep_blocks_kernel<T, TAPS, R><<<grid, 256 * (2 + R), 0, s>>>(                                \
         rec, qn, kn, (T*)vc, (const T*)x, ldx, (const T*)conv_w, (const T*)conv_state, a_log,     \
         dt_bias, r, KH, D, Dp, V);                                                                \
@@ -1463,7 +1464,6 @@ int omnia_delta_prep_blocks(float* rec, float* qn, float* kn, void* vc, const vo
                             int Dp, int V, int taps, hipStream_t s) {
   if (taps < 1 || KH < 1 || H % KH || Dp % 4 || Dp < D) return -1;
   if (KH > 65535) return -2;
-  if (T == 0 || nseq == 0) return 0;
   const Rows r{q_start, nseq, positions, slots};
   if (f32)
     return prep_blocks<float>(rec, qn, kn, vc, x, ldx, conv_w, conv_state, a_log, dt_bias, r, T, KH,

@@ -45,3 +45,16 @@ def step_conv(T, KH, H, D, V, Vs, taps=4):
                                        (64, 0, 0, -1)])
 def test_step_of_wide_states(D, V, Vs, rc):
     assert step_conv(1, 1, 1, D, V, Vs) == rc
+
+
+def prep_blocks(T, nseq, KH, H, D, V, taps=4):
+    return call("omnia_delta_prep_blocks", P, P, P, P, P, ("i", 0), ("l", 4096), P, P, P, P, P,
+                ("i", nseq), P, P, *ints(T, KH, H, D, -(-D // 4) * 4, V, taps), P)
+
+
+# no rows or no sequences: done only where rows of these sizes would be (the scan then expects records)
+@pytest.mark.parametrize("T,nseq", [(0, 3), (0, 0)])
+@pytest.mark.parametrize("D,KH,H,taps,rc", [(320, 1, 1, 4, -3), (64, 1, 4, 4, -3), (64, 1, 1, 5, -3),
+                                            (64, 1, 2, 4, 0)])
+def test_preparation_of_no_rows(T, nseq, D, KH, H, taps, rc):
+    assert prep_blocks(T, nseq, KH, H, D, 64, taps) == rc
