@@ -1339,12 +1339,19 @@ int step_conv(void* y, float* state, void* conv_state, const void* x, int64_t ld
               hipStream_t s) {
   if (D > 128 || V > 128 || D % 2 || V % 2 || taps < 2 || taps > 4 || Vs / 4 > 256) return -3;
   const int CG = Vs / 4, RG = 256 / CG, nr = (D + RG - 1) / RG, R = H / KH;
-  if (nr > 16) return -3;
-  // blocks of several heads read and write in step with one another: in two rounds of the chip (four
-  // heads a CU) that costs what the launch does (112 / 128 / 144 rows, two kernels and one: 49.8 /
-  // 53.3 / 65.1 and 49.8 / 54.4 / 63.1)
+  // One or two heads a key head.  Four were blocks of 1024 threads, one a CU, each with the states of
+  // four heads: slower than the two kernels until the chip is full and again past it (us, two / one, 4
+  // key heads of four heads of 128: 1 row 10.9 / 13.6, 8 11.4 / 14.9, 32 19.0 / 18.5, 64 31.2 / 27.1, 72
+  // 35.6 / 39.3, 128 52.5 / 51.5, 136 60.7 / 63.6, 256 105.0 / 102.5).
+  if (nr > 16 || R > 2) return -3;
+  // Of states of half that size (8 rows a thread) a CU holds 7 blocks of step_kernel, and 3 of 512
+  // threads here, 6 heads: two kernels while all heads are on the chip at once there and not here (8 key
+  // heads of two heads of 128 x 64, 104 rows 25.0 / 26.9, 112 26.7 / 27.9; 96 24.3 / 23.2, 120 30.6 /
+  // 29.2).  Elsewhere a CU holds as many heads of both, and the rounds of the two kernels are not a
+  // reason: of 128 x 128, 112 / 120 / 128 / 136 rows 49.4 / 52.4 / 53.1 / 61.1 and 49.5 / 51.7 / 53.8 /
+  // 60.0, of one head a key head 51.7 / 54.0 / 54.6 / 63.9 and 52.2 / 55.7 / 55.9 / 61.4.
   const int64_t heads = (int64_t)T_ * H;
-  if (R > 1 && heads > 1664 && heads <= 2176) return -3;
+  if (R == 2 && nr > 4 && nr <= 8 && heads > 6 * 256 && heads <= 7 * 256) return -3;
   const size_t lds = (size_t)(256 + 132 * R + R * (RG + 2) * Vs) * 4;
 #define OMNIA_STEP(N, RR)                                                                      \
   if (R == RR && nr <= N) {                                                                    \
@@ -1353,8 +1360,8 @@ int step_conv(void* y, float* state, void* conv_state, const void* x, int64_t ld
         norm_w, r, KH, D, V, Vs, Vp, taps, eps);                                               \
     return (int)hipGetLastError();                                                             \
   }
-  OMNIA_STEP(4, 1) OMNIA_STEP(16, 1) OMNIA_STEP(4, 2) OMNIA_STEP(16, 2) OMNIA_STEP(4, 4)
-  OMNIA_STEP(16, 4)
+  OMNIA_STEP(4, 1) OMNIA_STEP(8, 1) OMNIA_STEP(16, 1) OMNIA_STEP(4, 2) OMNIA_STEP(8, 2)
+  OMNIA_STEP(16, 2)
 #undef OMNIA_STEP
   return -3;
 }

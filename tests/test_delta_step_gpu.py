@@ -7,12 +7,12 @@ from omnia_amd import ops
 pytestmark = pytest.mark.gpu
 
 
-# one, two and four heads a key head; widths under, at and off a wave's 128 channels; rows that
-# start anew and padded ones (slot -1), strided input rows
+# one and two heads a key head; widths under, at and off a wave's 128 channels, states of 4, 8 and 16
+# rows a thread; rows that start anew and padded ones (slot -1), strided input rows
 @pytest.mark.parametrize("T", [1, 5, 64])
 @pytest.mark.parametrize("D,V,KH,H,taps", [(128, 128, 8, 16, 4), (128, 128, 2, 2, 4),
-                                           (20, 30, 1, 4, 3), (64, 128, 2, 4, 2),
-                                           (126, 6, 1, 1, 4), (128, 124, 1, 4, 4)])
+                                           (20, 30, 1, 2, 3), (64, 128, 2, 4, 2), (96, 80, 2, 2, 3),
+                                           (126, 6, 1, 1, 4), (128, 124, 1, 2, 4)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_step(T, D, V, KH, H, taps, dtype):
     k, dev = ops.kernels(), "cuda"
@@ -57,7 +57,8 @@ def test_step(T, D, V, KH, H, taps, dtype):
 
 @pytest.mark.parametrize("T,D,V,KH,H,taps", [
     (1, 130, 64, 1, 1, 4), (1, 64, 130, 1, 1, 4), (1, 63, 64, 1, 1, 4), (1, 64, 64, 1, 3, 4),
-    (1, 64, 64, 1, 1, 5), (1, 64, 1028, 1, 1, 4), (120, 64, 64, 8, 16, 4)])
+    (1, 64, 64, 1, 1, 5), (1, 64, 1028, 1, 1, 4), (1, 20, 30, 1, 4, 3), (64, 128, 124, 1, 4, 4),
+    (97, 128, 64, 8, 16, 4), (112, 64, 128, 8, 16, 4)])
 def test_sizes_left_to_the_two_kernels(T, D, V, KH, H, taps):
     k, dev = ops.kernels(), "cuda"
     C, Vs, Vp = 2 * KH * D + H * V, -(-V // 4) * 4, -(-V // 8) * 8
