@@ -1291,12 +1291,18 @@ int prep_blocks(float* rec, float* qn, float* kn, void* vc, const void* x, int64
                 hipStream_t s) {
   if (D > 128 || V > 128 || D % 2 || V % 2 || Dp > 128) return -3;
   const dim3 grid(T_ / 16 + r.nseq, KH);
-  // While the chip holds about all waves at once (8192): beyond, most of a block's waves wait for the
-  // few that make its records (us of prep, records and scan, two launches before the scan / one: 8 key
-  // heads of two of 128, 20 rows 16.4 / 13.0, 200 25.6 / 21.4, 3 x 333 (8320 waves) 48.0 / 43.5, 2000
-  // (16128) 111.5 / 111.9, 8 x 1000 192 / 202; of one, 3 x 333 (6240) 38.4 / 32.0, 2000 (12096) 109.7 /
-  // 109.9, 8 x 512 75.6 / 82.0; 2 of two, 8 x 512 (8448) 50.5 / 44.0, 8 x 1000 (16256) 74.8 / 72.2)
-  if ((int64_t)grid.x * KH * 4 * (2 + H / KH) > 10240) return -3;
+  // A CU holds two blocks (threads): while all of them, 512, are there at once, most of a block's waves
+  // wait for the few that make its records at no one's cost.  A second round still pays for up to 640
+  // where nearly all blocks have a record: of many short sequences up to half have none, and delta_prep is
+  // fast on their few rows.  us of preparation, records and scan, two launches before the scan / one, 8 key
+  // heads of two of 128: 20 rows 16.4 / 13.0, 200 25.7 / 21.8, 56 x 2 (504 blocks) 54.3 / 51.9, 22 x 31 (512)
+  // 43.3 / 39.5, 32 x 16 (512) 40.4 / 39.6; 3 x 333 (520) 49.3 / 45.7, 8 x 120 (544) 44.1 / 40.6, 8 x 136
+  // (608) 48.3 / 46.2, 1200 (608) 77.6 / 77.5; not taken: 33 x 16 (528) 43.7 / 46.9, 60 x 2 (536) 56.6 / 59.1,
+  // 24 x 31 (560) 45.0 / 45.2, 40 x 16 (640) 47.7 / 50.9, 2000 (1008) 111.5 / 111.9, 8 x 1000 192 / 202.  Of
+  // one head a key head: 3 x 333 39.3 / 34.4, 32 x 16 29.4 / 27.6, 1200 75.6 / 74.1; not taken: 33 x 16 31.6 /
+  // 33.5, 20 x 48 37.1 / 37.8, 2000 109.7 / 109.9.  Of heads of 64: 3 x 333 32.1 / 28.1; 33 x 16 25.3 / 28.2.
+  const int64_t blocks = (int64_t)grid.x * KH;
+  if (blocks > 640 || (blocks > 512 && 4 * r.nseq > T_ / 16)) return -3;
 #define OMNIA_PB(TAPS, R)                                                                         \
   if (taps == TAPS && H == R * KH) {                                                              \
     if (T_ == 0 || r.nseq == 0) return 0;                                                         \

@@ -29,7 +29,8 @@ def inputs(lens, D, V, KH, H, taps, dtype):
 
 # ends inside, at and past a record and its runs of four, sequences shorter than the taps, none;
 # widths under, at and off a wave's 128 channels; strided input rows
-@pytest.mark.parametrize("lens", [[1], [16, 4, 21], [2, 0, 47, 3, 64, 1], [333] * 3])
+@pytest.mark.parametrize("lens", [[1], [16, 4, 21], [2, 0, 47, 3, 64, 1], [333] * 3,
+                                  [16] * 32, [1264]])
 @pytest.mark.parametrize("D,V,KH,H,taps", [(128, 128, 8, 16, 4), (128, 96, 2, 2, 4), (20, 30, 1, 2, 3),
                                            (64, 128, 2, 4, 2), (126, 6, 1, 1, 4)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

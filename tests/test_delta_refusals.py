@@ -63,3 +63,11 @@ def test_preparation_of_no_rows():
     got = results("omnia_delta_prep_blocks",
                   [prep_blocks(0, nseq, *s) for nseq in (3, 0) for s in sizes])
     assert got == [-3, -3, -3, 0] * 2
+
+
+def test_preparation_in_two_rounds():
+    """-3 past two blocks a CU where many sequences are short, and past 640 blocks."""
+    sizes = [(33 * 16, 33), (2 * 60, 60), (24 * 31, 24), (1264 + 16, 1), (8 * 1000, 8)]
+    got = results("omnia_delta_prep_blocks", [prep_blocks(T, n, 8, R * 8, 128, 128, 4)
+                                              for R in (1, 2) for T, n in sizes])
+    assert got == [-3] * 10
