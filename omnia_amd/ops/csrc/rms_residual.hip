@@ -98,22 +98,25 @@ __global__ __launch_bounds__(NT) void embed_kernel(T* __restrict__ h, float* __r
   }
 }
 
-// Router logits of a row for up to EP experts, in the block that has the row: saves a launch of 5.5 us
-// a sparse layer for about 1 us here.  The router's columns are loaded ahead of everything else; a
-// wave adds a column's EP products over its lanes in EP - 1 + log2(64 / EP) exchanges, half of the
-// values it still has going to the other lanes each time.
+// Router logits of a row for up to EP experts, in the block that has the row: saves a launch.  The
+// router's columns are loaded ahead of everything else; a wave adds a column's EP products over its lanes
+// in EP - 1 + log2(64 / EP) exchanges, half of the values it still has going to the other lanes each
+// time.  Bound by the chain of loads, exchanges and the choice (figures at its rule).
 template <int EP>
 struct Logits {
   short4v w[EP];
   __device__ __forceinline__ void load(const bf16_t* router, int E, int d, int c) {
+    // all at once, from valid places: columns past d are zeroed at their use, experts past E repeat the
+    // last one and are not read
+    const int at = min(c, d - 4);
 #pragma unroll
     for (int e = 0; e < EP; ++e)
-      w[e] = c < d && e < E ? *reinterpret_cast<const short4v*>(router + (int64_t)e * d + c)
-                            : short4v{0, 0, 0, 0};
+      w[e] = *reinterpret_cast<const short4v*>(router + (int64_t)min(e, E - 1) * d + at);
   }
-  // v: the row's values as the experts read them.  part [waves][EP]; ends with row z[0 .. E - 1]
+  // v: the row's values as the experts read them (live: columns of the row).  part [waves][EP]; ends
+  // with row z[0 .. E - 1]
   template <int NT>
-  __device__ __forceinline__ void row(float4v v, float (*part)[EP], float* z) const {
+  __device__ __forceinline__ void row(float4v v, bool live, float (*part)[EP], float* z) const {
     const int lane = threadIdx.x & 63;
     float s[EP];
 #pragma unroll
@@ -121,14 +124,19 @@ struct Logits {
       s[e] = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[e] += v[j] * bf2f((uint16_t)w[e][j]);
+      s[e] = live ? s[e] : 0.f;
     }
     int at = 0;  // the value that this lane ends with
 #pragma unroll
     for (int n = EP / 2, bit = 1; n >= 1; n /= 2, bit *= 2) {
       const bool up = lane & bit;
 #pragma unroll
-      for (int i = 0; i < n; ++i)
-        s[i] = (up ? s[i + n] : s[i]) + __shfl_xor(up ? s[i] : s[i + n], bit, 64);
+      for (int i = 0; i < n; ++i) {
+        // (the asm keeps hipcc from making the choice one of an index, a comparison for every value)
+        float lo = s[i], hi = s[i + n];
+        asm("" : "+v"(lo), "+v"(hi));
+        s[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, bit, 64);
+      }
       at += up ? n : 0;
     }
 #pragma unroll
@@ -201,7 +209,7 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
     __shared__ float z[16];
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[0][j] = bf2f(f2bf(v[0][j]));  // what h holds
-    logits.template row<NT>(v[0], part, z);
+    logits.template row<NT>(v[0], threadIdx.x * 4 < d, part, z);
     if (threadIdx.x < 16) {  // one wave: its LDS in order
       __builtin_amdgcn_wave_barrier();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -283,9 +291,17 @@ int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int
                                                          part_stride, d, bias, post, pre,       \
                                                          (const bf16_t*)router, route)
   if (router) {
-    // rows of one chunk of 4 columns a thread, up to 512 of them: beyond, a kernel that reads the
-    // router once for 16 rows
+    // Rows of one chunk of 4 columns a thread.  Every row's block reads the router, where the kernel that
+    // only routes reads it once for 16 rows; blocks past 256 wait for a second round of the chip, which
+    // of more than 8 experts pays from 2048 columns.  us of residual step and routing, two launches / one, 8
+    // experts: 1056 columns 1 / 64 / 256 / 264 / 512 rows 5.6 / 7.4 / 7.9 / 8.2 / 8.8 and 5.3 / 5.8 / 6.1 / 7.7
+    // / 8.3, 2048 6.6 / 8.8 / 9.6 / 10.1 / 11.1 and 5.4 / 5.8 / 6.4 / 8.2 / 8.9, 4096 8.6 / 12.2 / 13.4 / 14.1
+    // / 15.7 and 6.0 / 6.5 / 7.4 / 9.4 / 10.6; 16 experts: 1056 5.9 / 7.6 / 8.0 / 8.4 / 9.1 and 6.8 / 7.2 / 7.7
+    // / 10.2 / 10.9 (8 rows 7.1 both), 1536 6.9 / 8.8 / 9.3 / 9.8 / 10.6 and 6.8 / 7.2 / 7.8 / 10.3 / 11.1, 2048
+    // 7.4 / 9.7 / 10.4 / 10.9 / 11.9 and 6.9 / 7.4 / 8.0 / 10.6 / 11.4, 4096 9.9 / 13.6 / 14.8 / 15.5 / 17.1 and
+    // 7.5 / 8.1 / 9.2 / 12.1 / 13.2.  Slabs and slots the same within 0.5.
     if (f32 || rows > 512 || d > 4096 || d % 32 || E < 1 || E > 16 || k < 1 || k > E) return -3;
+    if (E > 8 && rows > 256 && d < 2048) return -3;
     if (groups < 1 || E % groups || keep < 1 || keep > groups || k > keep * (E / groups)) return -4;
 #define OMNIA_RT(EP)                                           \
   do {                                                         \
