@@ -201,6 +201,7 @@ int omnia_delta_norm(void* y, const float* o, const void* x, int f32, int64_t ld
 int omnia_rms_embed(void* h, float* x, const int* ids, const void* table, int f32, int T, int d,
                     int vocab, const float* we, const float* wp, float inv_n, float eps,
                     const int64_t* src, const int* tok_slots, hipStream_t s);
+int omnia_rms_residual_routes(int64_t rows, int64_t d, int64_t E);
 int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int S,
                        int64_t row_stride, int64_t part_stride, int rows, int d,
                        const float* bias, const float* w_post, const float* w_pre, float inv_n, float eps,
@@ -2039,7 +2040,8 @@ void rms_embed(at::Tensor h, at::Tensor x, at::Tensor ids, at::Tensor table, int
                            opt_ptr<int>(tok_slots), cur_stream()), "rms_embed");
 }
 
-// With a router [E, d] the rows' experts too, as moe_route; false: sizes that need it (nothing ran)
+// With a router [E, d] the rows' experts too, as moe_route, for the sizes of rms_residual_routes; false:
+// a router off the 8-byte grid, which needs moe_route (nothing ran)
 bool rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bias,
                   at::Tensor w_post, OptT w_pre, double inv_n, double eps, OptT router, OptT ids,
                   OptT wts, int64_t k, bool sigmoid, bool renorm, OptT corr, int64_t groups,
@@ -2068,7 +2070,6 @@ bool rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bia
       route ? ids->data_ptr<int>() : nullptr, route ? wts->data_ptr<float>() : nullptr, E, k,
       sigmoid, renorm, opt_vecf(corr, E, "correction"), groups, keep,
       opt_vecf(rbias, E, "router bias"), cur_stream());
-  if (route && rc == -3) return false;
   CHECK_RC(rc, "rms_residual");
   return true;
 }
@@ -2217,6 +2218,9 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("rmsnorm", &rmsnorm);
   m.def("tanh_norm_embed", &tanh_norm_embed);
   m.def("rms_embed", &rms_embed);
+  m.def("rms_residual_routes", [](int64_t rows, int64_t d, int64_t E) {
+    return omnia_rms_residual_routes(rows, d, E) != 0;
+  });
   m.def("rms_residual", &rms_residual, py::arg("h"), py::arg("x"), py::arg("m"), py::arg("slots"),
         py::arg("bias"), py::arg("w_post"), py::arg("w_pre"), py::arg("inv_n"), py::arg("eps"),
         py::arg("router") = py::none(), py::arg("ids") = py::none(), py::arg("wts") = py::none(),

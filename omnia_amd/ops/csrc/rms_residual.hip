@@ -272,6 +272,21 @@ int omnia_rms_embed(void* h, float* x, const int* ids, const void* table, int f3
   return (int)hipGetLastError();
 }
 
+// Whether omnia_rms_residual takes a router of E experts along: rows of one chunk of 4 columns for each of
+// 1024 threads.  Every row's block reads the router, where the kernel that only routes reads it once for
+// 16 rows; blocks past 256 wait for a second round of the chip, which of more than 8 experts pays from 2048
+// columns.  us of residual step and routing, two launches / one, 8
+// experts: 1056 columns 1 / 64 / 256 / 264 / 512 rows 5.6 / 7.4 / 7.9 / 8.2 / 8.8 and 5.3 / 5.8 / 6.1 / 7.7
+// / 8.3, 2048 6.6 / 8.8 / 9.6 / 10.1 / 11.1 and 5.4 / 5.8 / 6.4 / 8.2 / 8.9, 4096 8.6 / 12.2 / 13.4 / 14.1
+// / 15.7 and 6.0 / 6.5 / 7.4 / 9.4 / 10.6; 16 experts: 1056 5.9 / 7.6 / 8.0 / 8.4 / 9.1 and 6.8 / 7.2 / 7.7
+// / 10.2 / 10.9 (8 rows 7.1 both), 1536 6.9 / 8.8 / 9.3 / 9.8 / 10.6 and 6.8 / 7.2 / 7.8 / 10.3 / 11.1, 2048
+// 7.4 / 9.7 / 10.4 / 10.9 / 11.9 and 6.9 / 7.4 / 8.0 / 10.6 / 11.4, 4096 9.9 / 13.6 / 14.8 / 15.5 / 17.1 and
+// 7.5 / 8.1 / 9.2 / 12.1 / 13.2.  Slabs and slots the same within 0.5.
+int omnia_rms_residual_routes(int64_t rows, int64_t d, int64_t E) {
+  if (E < 1 || E > 16 || rows > 512 || d <= 1024 || d > 4096 || d % 32) return 0;
+  return E <= 8 || rows <= 256 || d >= 2048;
+}
+
 // ptype: storage of `m` -- 0 bf16, 1 fp32, 2 fp16 (slabs).  router: null, or [E, d] bf16: the rows'
 // experts as omnia_moe_route chooses them; -3 where that kernel has to
 int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int S,
@@ -291,17 +306,7 @@ int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int
                                                          part_stride, d, bias, post, pre,       \
                                                          (const bf16_t*)router, route)
   if (router) {
-    // Rows of one chunk of 4 columns a thread.  Every row's block reads the router, where the kernel that
-    // only routes reads it once for 16 rows; blocks past 256 wait for a second round of the chip, which
-    // of more than 8 experts pays from 2048 columns.  us of residual step and routing, two launches / one, 8
-    // experts: 1056 columns 1 / 64 / 256 / 264 / 512 rows 5.6 / 7.4 / 7.9 / 8.2 / 8.8 and 5.3 / 5.8 / 6.1 / 7.7
-    // / 8.3, 2048 6.6 / 8.8 / 9.6 / 10.1 / 11.1 and 5.4 / 5.8 / 6.4 / 8.2 / 8.9, 4096 8.6 / 12.2 / 13.4 / 14.1
-    // / 15.7 and 6.0 / 6.5 / 7.4 / 9.4 / 10.6; 16 experts: 1056 5.9 / 7.6 / 8.0 / 8.4 / 9.1 and 6.8 / 7.2 / 7.7
-    // / 10.2 / 10.9 (8 rows 7.1 both), 1536 6.9 / 8.8 / 9.3 / 9.8 / 10.6 and 6.8 / 7.2 / 7.8 / 10.3 / 11.1, 2048
-    // 7.4 / 9.7 / 10.4 / 10.9 / 11.9 and 6.9 / 7.4 / 8.0 / 10.6 / 11.4, 4096 9.9 / 13.6 / 14.8 / 15.5 / 17.1 and
-    // 7.5 / 8.1 / 9.2 / 12.1 / 13.2.  Slabs and slots the same within 0.5.
-    if (f32 || rows > 512 || d > 4096 || d % 32 || E < 1 || E > 16 || k < 1 || k > E) return -3;
-    if (E > 8 && rows > 256 && d < 2048) return -3;
+    if (f32 || !omnia_rms_residual_routes(rows, d, E) || k < 1 || k > E) return -3;
     if (groups < 1 || E % groups || keep < 1 || keep > groups || k > keep * (E / groups)) return -4;
 #define OMNIA_RT(EP)                                           \
   do {                                                         \

@@ -102,11 +102,6 @@ def rms_embed(ids, table, vocab: int, emb: RMSNorm, pre: RMSNorm | None, src=Non
     return x, (x if pre is None else ref.rms_norm(x, pre)).to(table.dtype)
 
 
-# widths beyond and up to which, and rows up to which, the residual kernel takes a thread for 4 columns
-# and routes a row beside (see rms_residual.hip)
-ROUTE_ROWS = 1024, 4096, 512
-
-
 class Routing:
     """What a step's rows are routed by (an expert feed-forward's tensors and spec); ``ids`` and
     ``wts`` [M, top], once a kernel ahead of the experts has chosen them."""
@@ -130,8 +125,8 @@ def rms_residual(x, m, post: RMSNorm, pre: RMSNorm | None, dtype, bias=None,
     if x.is_cuda:
         h = torch.empty(x.shape, dtype=dtype, device=x.device)
         args = (h, x, m, slots, bias, post.w, None if pre is None else pre.w, post.inv_n, post.eps)
-        if route is not None and ROUTE_ROWS[0] < x.shape[1] <= ROUTE_ROWS[1] and \
-                x.shape[0] <= ROUTE_ROWS[2] and dtype == torch.bfloat16:
+        if route is not None and dtype == torch.bfloat16 and \
+                kernels().rms_residual_routes(*x.shape, route.w["router"].shape[0]):
             s, w = route.spec, route.w
             ids, wts = route.empty(x.shape[0], x.device)
             if kernels().rms_residual(*args, w["router"], ids, wts, s.top, s.score == "sigmoid",
