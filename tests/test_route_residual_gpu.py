@@ -60,3 +60,39 @@ def test_sizes_left_to_the_router(rows, d, E):
     x, m = torch.zeros(rows, d, device=dev), torch.ones(rows, d, dtype=bf, device=dev)
     h = mops.rms_residual(x, m, post, None, bf, route=route)
     assert route.ids is None and bool((h == 1).all()) and bool((x - 1).abs().max() < 1e-4)
+
+
+# what a residual step sums (ptype and parts of the kernel): fp32 and fp16 slabs, a row's slots, a plain
+# fp32 projection; rows of infinities and NaN choose as the kernel that only routes
+@pytest.mark.parametrize("rows,d", [(5, 1056), (33, 2080)])
+@pytest.mark.parametrize("E,k", [(8, 2), (7, 3), (16, 4)])
+@pytest.mark.parametrize("kind", ["fp32", "fp32 slabs", "fp16 slabs", "slots"])
+def test_route_of_parts(rows, d, E, k, kind):
+    dev, bf = "cuda", torch.bfloat16
+    g = torch.Generator().manual_seed(d + E)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g)
+
+    m = {"fp32": lambda: rnd(rows, d), "fp32 slabs": lambda: rnd(3, rows, d),
+         "fp16 slabs": lambda: rnd(4, rows, d).half(), "slots": lambda: rnd(rows, 2, d).to(bf)}[kind]()
+    m, x0 = m.to(dev), rnd(rows, d).to(dev)
+    x0[1, 17], x0[2, d - 1], x0[3, 4] = float("inf"), -float("inf"), float("nan")
+    w = {"router": (rnd(E, d) * d ** -0.5).to(bf).to(dev)}
+    spec = SimpleNamespace(top=k, score="sigmoid", renorm=False, groups=1, keep=1)
+    post = mops.RMSNorm((rnd(d) * 0.1 + 1.0).to(dev), d, 1e-5)
+    x1, x2, route = x0.clone(), x0.clone(), mops.Routing(w, spec)
+    h1 = mops.rms_residual(x1, m, post, None, bf, slots=kind == "slots", route=route)
+    h2 = mops.rms_residual(x2, m, post, None, bf, slots=kind == "slots")
+    assert route.ids is not None
+    for a, b in ((x1, x2), (h1, h2)):
+        assert torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
+    ids, wts = route.empty(rows, dev)
+    ops.kernels().moe_route(ids, wts, h2, w["router"], k, True, False, None, 1, 1, None)
+    odd = slice(1, 4)
+    assert torch.equal(route.ids[odd], ids[odd])
+    assert torch.equal(route.wts[odd].nan_to_num(nan=7.0), wts[odd].nan_to_num(nan=7.0))
+    # elsewhere fp32 sums of d products in two orders, as above
+    rest = torch.tensor([i for i in range(rows) if i not in (1, 2, 3)], device=dev)
+    close = (route.wts - wts).abs().amax(1) <= 2e-5
+    assert bool(((route.ids == ids).all(1) & close)[rest].float().mean() >= 0.99)
