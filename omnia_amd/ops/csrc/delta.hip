@@ -942,7 +942,9 @@ struct ScanShared {
 // The accumulator layout serves as the B operand of the next product as it stands: k-step r takes
 // dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.  Their parts of K S
 // meet in LDS, added by all in one order, so that all hold the same u; parts of the output are
-// added by the moving waves, a block later.
+// added by the moving waves, a block later.  A wave that has twice the tiles keeps two sums, so that the
+// order of additions, and with it every bit of a sequence's results, is that of four waves (one sum a wave
+// of two was 1 % faster where the chip is full: 16 heads of 128, 2048 rows of 8 285 -> 288 us).
 // Bound by the serial chain of a block where few blocks run: K S, the exchange, T', K^T U, 20 of a
 // wave's 29 fp32 products (13.3 ns each) and the latencies between them.  A wave issues an
 // instruction in about 5 clocks and none beside its own products, so whatever is not on the chain
@@ -958,7 +960,9 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
     const float* __restrict__ rec, const float* __restrict__ qn, const float* __restrict__ kn,
     const T* __restrict__ vc, const T* __restrict__ x, int64_t ldx, Rows rows, int KH, int H,
     int D, int Dp, int V, int Vs, int taps) {
-  constexpr int NJ = ND / NW, PR = 4 / NW, CN = NW * CW;
+  // NS sums of a wave, of JS tiles each: four in all (two, of the narrowest heads) whatever NW, added in
+  // pairs, so that a sequence's results do not depend on the shape that its step takes
+  constexpr int NJ = ND / NW, PR = 4 / NW, CN = NW * CW, NS = ND >= 4 ? PR : 1, JS = NJ / NS;
   using Buf = ScanBuf<ND, CW>;
   constexpr int KS = Buf::KS, TS = Buf::TS;
   static_assert(NJ * NW == ND && (NW == 2 || NW == 4), "tiles of a wave");
@@ -1049,10 +1053,10 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
       const Rsrc O = rows_of(ob, bi, obytes);
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
-        float y = sh.os[bi & 1][c][0][16 * (tok >> 2) + c16][tok & 3];
+        float y[NW];
 #pragma unroll
-        for (int i = 1; i < NW; ++i) y += sh.os[bi & 1][c][i][16 * (tok >> 2) + c16][tok & 3];
-        store1(y, O, ooff[c]);
+        for (int i = 0; i < NW; ++i) y[i] = sh.os[bi & 1][c][i][16 * (tok >> 2) + c16][tok & 3];
+        store1(NW == 2 ? y[0] + y[1] : (y[0] + y[1]) + (y[NW - 2] + y[NW - 1]), O, ooff[c]);
       }
     };
     auto phase = [&](Stage& t, int bi) {
@@ -1106,11 +1110,19 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
   auto block = [&](auto odd) {
     constexpr int P = decltype(odd)::value;
     const Buf& B = sh.buf[P];
-    float4v ks = {0.f, 0.f, 0.f, 0.f}, qs = ks, parts[NW];
-    auto qstep = [&](int i) { qs = mfma4(qa[i >> 2][i & 3], S[i >> 2][i & 3], qs); };
+    float4v ks[NS], qs[NS], parts[NW];
+#pragma unroll
+    for (int a = 0; a < NS; ++a) ks[a] = qs[a] = float4v{0.f, 0.f, 0.f, 0.f};
+    // product i is one of sum i % NS
+    auto tile = [](int i) { return i % NS * JS + (i / NS >> 2); };
+    auto qstep = [&](int i) {
+      const int j = tile(i), r = i / NS & 3;
+      qs[i % NS] = mfma4(qa[j][r], S[j][r], qs[i % NS]);
+    };
 #pragma unroll
     for (int i = 0; i < 4 * NJ; ++i) {
-      ks = mfma4(ka[i >> 2][i & 3], S[i >> 2][i & 3], ks);
+      const int tj = tile(i), tr = i / NS & 3;
+      ks[i % NS] = mfma4(ka[tj][tr], S[tj][tr], ks[i % NS]);
       if (i == 0) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1131,13 +1143,13 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
 #pragma unroll
           for (int j = 0; j < NJ; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + d0 + 16 * j + c16];
 #pragma unroll
-        for (int k = 0; k < PR; ++k) pa[k] = B.p[c16 * TS + 4 * g4 + NW * k + w];
+        for (int k = 0; k < PR; ++k) pa[k] = B.p[c16 * TS + 4 * g4 + PR * w + k];
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     // half of the products with q while the parts of K S go out, the others while they come in
     constexpr int Q0 = 2 * NJ, Q1 = 3 * NJ;
-    sh.ks[P][cw][w][lane] = ks;
+    sh.ks[P][cw][w][lane] = NS == 2 ? ks[0] + ks[NS - 1] : ks[0];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < Q0; ++i) qstep(i);
@@ -1150,10 +1162,9 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
 #pragma unroll
     for (int i = Q0; i < Q1; ++i) qstep(i);
     __builtin_amdgcn_sched_barrier(0);
-    ks = parts[0];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) ks += parts[i];
-    const float4v res = v - G * ks;
+    const float4v sum = NW == 2 ? parts[0] + parts[1]
+                                : (parts[0] + parts[1]) + (parts[NW - 2] + parts[NW - 1]);
+    const float4v res = v - G * sum;
     float4v u = {0.f, 0.f, 0.f, 0.f};
     // the chain of u runs between the products with q, which do not need it
 #pragma unroll
@@ -1173,15 +1184,16 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int j = 0; j < NJ; ++j) S[j] = mfma4(ku[r][j], ue[r], S[j]);
-    qs *= G;
 #pragma unroll
-    for (int i = 0; i < PR; ++i) {
-      float t = u[NW * i];
+    for (int a = 0; a < NS; ++a) qs[a] *= G;
 #pragma unroll
-      for (int k = 1; k < NW; ++k) t = w == k ? u[NW * i + k] : t;
-      qs = mfma4(pa[i], t, qs);
+    for (int i = 0; i < PR; ++i) {  // token PR w + i of a lane's four
+      float t = u[i];
+#pragma unroll
+      for (int k = 1; k < NW; ++k) t = w == k ? u[PR * k + i] : t;
+      qs[i % NS] = mfma4(pa[i], t, qs[i % NS]);
     }
-    sh.os[P][cw][w][lane] = qs;
+    sh.os[P][cw][w][lane] = NS == 2 ? qs[0] + qs[NS - 1] : qs[0];
     __builtin_amdgcn_sched_barrier(0);
   };
   sync();

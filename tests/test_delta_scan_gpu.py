@@ -73,3 +73,40 @@ def test_scan(D, V, H, KH, lens, dtype):
         old = torch.zeros(taps - 1, C, dtype=dtype) if i == B - 1 else conv[slots[i]]
         full = torch.cat([old, x[starts[i]:starts[i + 1], :C]])
         assert torch.equal(cv[slots[i]], full[-(taps - 1):])
+
+
+# the shape that a step takes (few sequences: one group of columns, four waves; many: two of two)
+# changes no bit of a sequence's outputs and state
+@pytest.mark.parametrize("D,V,H,KH", [(24, 40, 6, 3), (64, 64, 16, 8), (96, 80, 8, 8),
+                                      (128, 128, 16, 8), (200, 128, 8, 8)])
+def test_sequences_beside_change_nothing(D, V, H, KH):
+    k, dev = ops.kernels(), "cuda"
+    n, taps, C = 77, 4, 2 * KH * D + H * V
+
+    def run(B):
+        g = torch.Generator().manual_seed(D)
+
+        def rnd(*shape):
+            return torch.randn(*shape, generator=g)
+
+        def all_rows(t):
+            return t.to(dev).repeat(B, *[1] * (t.dim() - 1))
+
+        qn = torch.nn.functional.normalize(rnd(n, KH, D), dim=-1) * D ** -0.5
+        kn = torch.nn.functional.normalize(rnd(n, KH, D), dim=-1)
+        v, decay, beta = rnd(n, H * V), -torch.exp(rnd(n, H) * 0.5 - 2.0), torch.sigmoid(rnd(n, H))
+        state, x = rnd(1, H, D, V) * 0.1, rnd(n, C + H * V + 2 * H)
+        qn, kn, v, decay, beta, state, x = map(all_rows, (qn, kn, v, decay, beta, state, x))
+        state = state.contiguous()
+        conv = torch.zeros(B, taps - 1, C, device=dev)
+        starts = (torch.arange(B + 1) * n).int().to(dev)
+        pos = torch.arange(5, 5 + n).repeat(B).int().to(dev)
+        o = torch.empty(n * B, H, V, device=dev)
+        rec = torch.empty(k.delta_records(n * B, B, H), device=dev)
+        k.delta_scan(o, state, conv, rec, qn, kn, v, decay, beta, x, starts, pos,
+                     torch.arange(B, dtype=torch.int32, device=dev), KH, H, D, D, V, taps)
+        return o, state
+
+    (o1, s1), (o, s) = run(1), run(40)
+    assert torch.equal(o.view(40, n, H, V), o1[None].expand(40, -1, -1, -1))
+    assert torch.equal(s, s1.expand_as(s))
