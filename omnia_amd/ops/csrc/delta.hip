@@ -937,7 +937,7 @@ struct ScanShared {
 };
 
 // grid (ceil(Vs / (16 CW)) x H, nseq), CW x NW waves that multiply and 4 that move operands and
-// outputs.  The former own 16 state columns each (cw) and share the key dimensions: wave w of NW has
+// outputs.  The former own 16 state columns each (cw) and share the key dimensions: wave w of NW (1, 2 or 4) has
 // NJ = ND / NW accumulator tiles (key dimensions 16 (w NJ + j) + 4 (lane >> 4) + r in register r).
 // The accumulator layout serves as the B operand of the next product as it stands: k-step r takes
 // dimension (token) 4 (lane >> 4) + r, and the A side is read in that order.  Their parts of K S
@@ -950,22 +950,35 @@ struct ScanShared {
 // instruction in about 5 clocks and none beside its own products, so whatever is not on the chain
 // is another wave's work: with the staging in the multiplying waves the 16 heads of 4000 rows below
 // took 262 us, with operands straight from global memory 282.  Where the chip is full, fp32
-// products and vector instructions share one unit: 112 products a block of 32 columns, 1.5 of 2.1 us.
-// us with blocks_kernel (heads of 128), one wave a 16 columns and all of their key dimensions ->
-// now: 16 heads, 77 rows 23 -> 14, 4000 547 -> 184, 1000 and 1500 216 -> 86, 333 of 3 61 -> 38, 60
-// of 16 37 -> 36, 512 of 32 315 -> 318, 2048 of 8 356 -> 327; 32 heads, 333 of 3 67 -> 60.
+// products and vector instructions share one unit: of heads of 128, a wave of two has 54 products (16 each
+// of K S, Q S and K^T U, 4 of T', 2 of P U) and a SIMD 108, of its two blocks: 1.44 of the 2.1 us that a
+// block of 32 columns takes.
+// us with blocks_kernel, one wave a 16 columns and all of their key dimensions -> now, heads of 128: 16 heads,
+// 77 rows 23 -> 14, 1000 146 -> 52, 4000 547 -> 184, 333 of 3 61 -> 36, 60 of 16 36 -> 33, 512 of 32 298 ->
+// 290, 2048 of 8 330 -> 288; 32 heads, 333 of 3 64 -> 55, 2048 of 8 583 -> 577;
+// 8 heads of 256 x 128, 333 of 3 114 -> 39, 512 of 32 400 -> 336; heads of 64: at their rule in scan.
 template <typename T, int ND, int NW, int CW>
-__global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan_blocks_kernel(
+__global__
+__launch_bounds__(64 * (NW * CW + 4), ND <= 4 || ND / NW <= 2 ? 4 : 2) void scan_blocks_kernel(
     float* __restrict__ o, float* __restrict__ state, T* __restrict__ conv_state,
     const float* __restrict__ rec, const float* __restrict__ qn, const float* __restrict__ kn,
     const T* __restrict__ vc, const T* __restrict__ x, int64_t ldx, Rows rows, int KH, int H,
     int D, int Dp, int V, int Vs, int taps) {
   // NS sums of a wave, of JS tiles each: four in all (two, of the narrowest heads) whatever NW, added in
   // pairs, so that a sequence's results do not depend on the shape that its step takes
-  constexpr int NJ = ND / NW, PR = 4 / NW, CN = NW * CW, NS = ND >= 4 ? PR : 1, JS = NJ / NS;
+  constexpr int NJ = ND / NW, PR = 4 / NW, CN = NW * CW, NS = ND >= 4 ? PR : 2 / NW, JS = NJ / NS;
+  // of the sums of a wave, and of those of the waves
+  auto pairs = [](auto const& a, auto n) {
+    if constexpr (decltype(n)::value == 1)
+      return a[0];
+    else if constexpr (decltype(n)::value == 2)
+      return a[0] + a[1];
+    else
+      return (a[0] + a[1]) + (a[2] + a[3]);
+  };
   using Buf = ScanBuf<ND, CW>;
   constexpr int KS = Buf::KS, TS = Buf::TS;
-  static_assert(NJ * NW == ND && (NW == 2 || NW == 4), "tiles of a wave");
+  static_assert(NJ * NW == ND && (NW == 1 || NW == 2 || NW == 4), "tiles of a wave");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   ScanShared<ND, NW, CW>& sh = *reinterpret_cast<ScanShared<ND, NW, CW>*>(lds);
   const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
@@ -1056,7 +1069,7 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
         float y[NW];
 #pragma unroll
         for (int i = 0; i < NW; ++i) y[i] = sh.os[bi & 1][c][i][16 * (tok >> 2) + c16][tok & 3];
-        store1(NW == 2 ? y[0] + y[1] : (y[0] + y[1]) + (y[NW - 2] + y[NW - 1]), O, ooff[c]);
+        store1(pairs(y, Int<NW>()), O, ooff[c]);
       }
     };
     auto phase = [&](Stage& t, int bi) {
@@ -1099,7 +1112,8 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[j][r] = fresh ? 0.f : load1(Sb, soff(j, r));
-  // operands of a block: k from behind the barrier before it, the rest before its own
+  // operands of a block: k from behind the barrier before it, the rest before its own (one wave reads each
+  // into the registers of the one before, 128 in all, of which a CU holds 2 blocks)
   float4v ka[NJ], qa[NJ], ta, G, E, v;
   float ku[4][NJ], pa[PR];
   auto keys = [&](const Buf& b) {
@@ -1107,10 +1121,18 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
     for (int j = 0; j < NJ; ++j)
       ka[j] = *reinterpret_cast<const float4v*>(b.k + c16 * KS + d0 + 16 * j + 4 * g4);
   };
+  auto updates = [&](const Buf& b) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) ku[r][j] = b.k[(4 * g4 + r) * KS + d0 + 16 * j + c16];
+#pragma unroll
+    for (int k = 0; k < PR; ++k) pa[k] = b.p[c16 * TS + 4 * g4 + PR * w + k];
+  };
   auto block = [&](auto odd) {
     constexpr int P = decltype(odd)::value;
     const Buf& B = sh.buf[P];
-    float4v ks[NS], qs[NS], parts[NW];
+    float4v ks[NS], qs[NS], parts[NW], sum;
 #pragma unroll
     for (int a = 0; a < NS; ++a) ks[a] = qs[a] = float4v{0.f, 0.f, 0.f, 0.f};
     // product i is one of sum i % NS
@@ -1137,33 +1159,33 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
         E = *reinterpret_cast<const float4v*>(B.g + 16 + 4 * g4);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (i == 2) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) ku[r][j] = B.k[(4 * g4 + r) * KS + d0 + 16 * j + c16];
-#pragma unroll
-        for (int k = 0; k < PR; ++k) pa[k] = B.p[c16 * TS + 4 * g4 + PR * w + k];
+      if (NW > 1 && i == 2) {
+        updates(B);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     // half of the products with q while the parts of K S go out, the others while they come in
     constexpr int Q0 = 2 * NJ, Q1 = 3 * NJ;
-    sh.ks[P][cw][w][lane] = NS == 2 ? ks[0] + ks[NS - 1] : ks[0];
+    sum = pairs(ks, Int<NS>());
+    if constexpr (NW > 1)
+      sh.ks[P][cw][w][lane] = sum;
+    else
+      updates(B);  // (registers of ka)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < Q0; ++i) qstep(i);
     __builtin_amdgcn_sched_barrier(0);
     sync();
+    if constexpr (NW > 1) {
 #pragma unroll
-    for (int i = 0; i < NW; ++i) parts[i] = sh.ks[P][cw][i][lane];
-    keys(sh.buf[1 - P]);
+      for (int i = 0; i < NW; ++i) parts[i] = sh.ks[P][cw][i][lane];
+      keys(sh.buf[1 - P]);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = Q0; i < Q1; ++i) qstep(i);
     __builtin_amdgcn_sched_barrier(0);
-    const float4v sum = NW == 2 ? parts[0] + parts[1]
-                                : (parts[0] + parts[1]) + (parts[NW - 2] + parts[NW - 1]);
+    if constexpr (NW > 1) sum = pairs(parts, Int<NW>());
     const float4v res = v - G * sum;
     float4v u = {0.f, 0.f, 0.f, 0.f};
     // the chain of u runs between the products with q, which do not need it
@@ -1173,6 +1195,11 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
 #pragma unroll
       for (int i = Q1; i < 4 * NJ; ++i)
         if ((i - Q1) * 4 / NJ == r) qstep(i);
+    }
+    if constexpr (NW == 1) {
+      __builtin_amdgcn_sched_barrier(0);
+      keys(sh.buf[1 - P]);  // (registers of qa)
+      __builtin_amdgcn_sched_barrier(0);
     }
     // exp(c_15), the last of the 16 tokens'
     const float G3 = G[3], G15 = __builtin_bit_cast(
@@ -1191,9 +1218,9 @@ __global__ __launch_bounds__(64 * (NW * CW + 4), ND / NW <= 2 ? 4 : 2) void scan
       float t = u[i];
 #pragma unroll
       for (int k = 1; k < NW; ++k) t = w == k ? u[PR * k + i] : t;
-      qs[i % NS] = mfma4(pa[i], t, qs[i % NS]);
+      qs[i * NS / PR] = mfma4(pa[i], t, qs[i * NS / PR]);
     }
-    sh.os[P][cw][w][lane] = NS == 2 ? qs[0] + qs[NS - 1] : qs[0];
+    sh.os[P][cw][w][lane] = pairs(qs, Int<NS>());
     __builtin_amdgcn_sched_barrier(0);
   };
   sync();
@@ -1392,7 +1419,13 @@ int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, 
   // One column group a block, its key dimensions over 4 waves, while those blocks are one a CU: the
   // chain of a block is what the step waits for.  Beyond, two groups of 2 waves (us, one / two: 256
   // blocks 86 / 118, 384 39 / 38, 768 60 / 60, 1024 105 / 90 and 368 / 327).
-  const bool few = (int64_t)((Vs + 15) / 16) * H * r.nseq <= 256;
+  // Heads of up to 64, four groups a block, once those are one a CU: a wave a group takes all of the key
+  // dimensions, so that a column has fewer products and movers, and two blocks a CU wait for one another
+  // (us, two of 2 / four of 1, heads of 64 x 64: 512 groups 39.2 / 49.8, 1024 60 / 57 and 217 / 209, 2048
+  // 110 / 97, 8192 439 / 390, 64 sequences of 2 tokens 23.2 / 18.2, of 32 heads 38.1 / 31.3; of 32 x 64,
+  // 2048 76 / 67, 4096 149 / 133).
+  const int64_t groups = (int64_t)((Vs + 15) / 16) * H * r.nseq;
+  const bool few = groups <= 256, narrow = groups >= 1024 && (Vs + 15) / 16 % 4 == 0;
 #define OMNIA_SPLIT(ND, NW, CW)                                                                   \
   scan_blocks_kernel<T, ND, NW, CW>                                                               \
       <<<dim3((Vs + 16 * CW - 1) / (16 * CW) * H, r.nseq), 64 * (NW * CW + 4),                    \
@@ -1406,6 +1439,8 @@ int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, 
                                               H, Dp);                                           \
     if (few)                                                                                    \
       OMNIA_SPLIT(ND, (ND < 4 ? 2 : 4), 1);                                                     \
+    else if (ND <= 4 && narrow)                                                                 \
+      OMNIA_SPLIT(ND, (ND <= 4 ? 1 : 2), (ND <= 4 ? 4 : 2));                                    \
     else                                                                                        \
       OMNIA_SPLIT(ND, 2, 2);                                                                    \
     return (int)hipGetLastError();                                                              \

@@ -20,11 +20,12 @@ def exact(qn, kn, v, decay, beta, S, starts, H):
     return out, S
 
 
-# few sequences: one group of 16 columns a block; many: two.  Widths in every padding of the key
-# dimensions, odd value widths, groups of columns that end inside a block
+# few sequences: one group of 16 columns a block; many: two, of up to 64 key dimensions four.  Widths
+# in every padding of the key dimensions, odd value widths, groups of columns that end inside a block
 @pytest.mark.parametrize("lens", [[1], [16], [15, 33, 64, 1], [47, 32] + [2] * 120])
 @pytest.mark.parametrize("D,V,H,KH", [(128, 128, 4, 2), (20, 29, 2, 1), (32, 16, 2, 2),
-                                      (64, 40, 3, 1), (96, 72, 2, 1), (200, 48, 2, 1)])
+                                      (64, 40, 3, 1), (96, 72, 2, 1), (200, 48, 2, 1),
+                                      (40, 61, 4, 2), (64, 64, 4, 4), (32, 128, 2, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_scan(D, V, H, KH, lens, dtype):
     k = ops.kernels()
@@ -77,7 +78,7 @@ def test_scan(D, V, H, KH, lens, dtype):
 
 # the shape that a step takes (few sequences: one group of columns, four waves; many: two of two)
 # changes no bit of a sequence's outputs and state
-@pytest.mark.parametrize("D,V,H,KH", [(24, 40, 6, 3), (64, 64, 16, 8), (96, 80, 8, 8),
+@pytest.mark.parametrize("D,V,H,KH", [(24, 40, 6, 3), (24, 64, 8, 4), (64, 64, 16, 8), (96, 80, 8, 8),
                                       (128, 128, 16, 8), (200, 128, 8, 8)])
 def test_sequences_beside_change_nothing(D, V, H, KH):
     k, dev = ops.kernels(), "cuda"
