@@ -1419,13 +1419,15 @@ int scan(float* o, float* state, void* conv_state, float* rec, const float* qn, 
   // One column group a block, its key dimensions over 4 waves, while those blocks are one a CU: the
   // chain of a block is what the step waits for.  Beyond, two groups of 2 waves (us, one / two: 256
   // blocks 86 / 118, 384 39 / 38, 768 60 / 60, 1024 105 / 90 and 368 / 327).
-  // Heads of up to 64, four groups a block, once those are one a CU: a wave a group takes all of the key
-  // dimensions, so that a column has fewer products and movers, and two blocks a CU wait for one another
-  // (us, two of 2 / four of 1, heads of 64 x 64: 512 groups 39.2 / 49.8, 1024 60 / 57 and 217 / 209, 2048
-  // 110 / 97, 8192 439 / 390, 64 sequences of 2 tokens 23.2 / 18.2, of 32 heads 38.1 / 31.3; of 32 x 64,
-  // 2048 76 / 67, 4096 149 / 133).
-  const int64_t groups = (int64_t)((Vs + 15) / 16) * H * r.nseq;
-  const bool few = groups <= 256, narrow = groups >= 1024 && (Vs + 15) / 16 % 4 == 0;
+  // Heads of up to 64, four groups a block, once those are one a CU and leave no more of their groups empty
+  // than blocks of two: a wave a group takes all of the key dimensions, so that a column has fewer products
+  // and movers, and two blocks a CU wait for one another (us, two of 2 / four of 1, heads of 64 x 64: 512
+  // groups 39.2 / 49.8, 1024 60 / 57 and 217 / 209, 2048 110 / 97, 8192 439 / 390, 64 sequences of 2 tokens
+  // 23.2 / 18.2, of 32 heads 38.1 / 31.3; of 64 x 48, 6144 414 / 373; of 32 x 64, 2048 76 / 67, 4096 149 / 133;
+  // of 24 x 40, 64 sequences of 2 tokens of 32 heads 27.8 / 24.1, where the kernel before took 22.6).
+  const int g = (Vs + 15) / 16;
+  const int64_t heads = (int64_t)H * r.nseq;
+  const bool few = g * heads <= 256, narrow = (g + 3) / 4 * heads >= 256 && (g % 4 == 0 || g % 4 == 3);
 #define OMNIA_SPLIT(ND, NW, CW)                                                                   \
   scan_blocks_kernel<T, ND, NW, CW>                                                               \
       <<<dim3((Vs + 16 * CW - 1) / (16 * CW) * H, r.nseq), 64 * (NW * CW + 4),                    \
