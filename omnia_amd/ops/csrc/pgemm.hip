@@ -226,7 +226,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   const int wr = SHAPE == FLAT ? 0 : w >> 1, wc = SHAPE == FLAT ? w : w & 1;
   const int fr = lane & 15, fq = lane >> 4;
 
-  // ---- a bias is asked for before the DMAs, which are counted
+  // ---- a bias, and the rows' places in the output, are asked for before the DMAs, which are counted
   constexpr int NG = NF / 2, GU = 64 * NB;
   constexpr int WCOL = (gated(EPI) ? NG : NF) * 16;
   const int f0 = nt * TN + wc * WCOL;
@@ -239,6 +239,11 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
         bg[n][j] = p.bias[f0 + 16 * n + 4 * fq + j];
         bu[n][j] = p.bias[p.N + f0 + 16 * n + 4 * fq + j];
       }
+  }
+  int place[8];
+  if constexpr (EPI == 6) {
+#pragma unroll
+    for (int m = 0; m < 8; ++m) place[m] = p.sorted[m0 + wr * 128 + 16 * m + fr];
   }
 
   // ---- DMA sources: instruction i of wave w fills half-tile rows 32w + 8i + lane/8, LDS chunk
@@ -416,12 +421,22 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     }
     return -1;
   };
+  // Every fragment asked for is there, and hipcc knows it and puts no waits of its own before the
+  // products.  Of those, 26 a K-tile where the first K-tile stands before the loop, and 16 where the loop
+  // began with zeroed sums; a wave issues each in 5 clocks (16384 rows, us with 16 / 26 / 3: residual
+  // products 861 / 868 / 858, experts' down with places loaded a row at a time 443 / 456, ahead 441).
+  auto wait_lds = [] __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  };
   auto step = [&](auto SC, auto FIRST) __attribute__((always_inline)) {
     constexpr int s = decltype(SC)::value;
+    if (s == 0) wait_lds();
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       if (s == 0 && j == FREE) {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        wait_lds();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -446,11 +461,11 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
 #pragma unroll
   for (int j = 0; j < 8 + NF; ++j) read(0, 0, j);
   step(std::integral_constant<int, 0>{}, std::true_type{});
-  for (int t = 1; t < nk; ++t) {
-    step(std::integral_constant<int, 1>{}, std::false_type{});
-    step(std::integral_constant<int, 0>{}, std::false_type{});
-  }
   step(std::integral_constant<int, 1>{}, std::false_type{});
+  for (int t = 1; t < nk; ++t) {
+    step(std::integral_constant<int, 0>{}, std::false_type{});
+    step(std::integral_constant<int, 1>{}, std::false_type{});
+  }
   pin();
   wait_vm<0>();  // the reloads past the end land before LDS is used again, or left
 
@@ -632,7 +647,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
       int64_t orow = m0 + r;
       bool live = r < Mt;
       if constexpr (EPI == 6) {  // to the assignment's row
-        orow = p.sorted[m0 + r];
+        orow = place[m];
         live = orow < p.n_assign;
       }
       bf16_t* o = out + orow * p.ldo + (int64_t)nt * TN + wc * WCOL + ccol;
