@@ -2041,7 +2041,7 @@ void rms_embed(at::Tensor h, at::Tensor x, at::Tensor ids, at::Tensor table, int
 }
 
 // With a router [E, d] the rows' experts too, as moe_route, for the sizes of rms_residual_routes; false:
-// a router off the 8-byte grid, which needs moe_route (nothing ran)
+// a router off the 16-byte grid, which needs moe_route (nothing ran)
 bool rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bias,
                   at::Tensor w_post, OptT w_pre, double inv_n, double eps, OptT router, OptT ids,
                   OptT wts, int64_t k, bool sigmoid, bool renorm, OptT corr, int64_t groups,
@@ -2057,7 +2057,7 @@ bool rms_residual(at::Tensor h, at::Tensor x, at::Tensor m, bool slots, OptT bia
                 router->is_contiguous() && router->dim() == 2 && router->size(1) == d,
                 "router [E, d]");
     E = router->size(0);
-    if (reinterpret_cast<uintptr_t>(router->data_ptr()) & 7) return false;
+    if (reinterpret_cast<uintptr_t>(router->data_ptr()) & 15) return false;
     TORCH_CHECK(ids.has_value() && wts.has_value() && ids->is_cuda() && wts->is_cuda() &&
                 ids->scalar_type() == at::kInt && wts->scalar_type() == at::kFloat &&
                 ids->numel() == p.M * k && wts->numel() == p.M * k && ids->is_contiguous() &&

@@ -9,8 +9,10 @@
 //
 //   delta_prep   convolutions, unit norms, decay and step size of every token (few rows of
 //                sequences: delta_prep_blocks, with the blocks' systems of delta_scan)
-//   delta_step   decode: one token per sequence -- state update, per-head RMS norm and
-//                the silu(z) output gate in one launch, one workgroup per (row, head)
+//   delta_step_conv  decode, one token per sequence, of one or two heads a key head: convolutions,
+//                norms, state update, per-head RMS norm and the silu(z) output gate in one launch,
+//                one workgroup per (row, key head)
+//   delta_step   decode of other sizes: the same behind delta_prep, one workgroup per (row, head)
 //   delta_scan   prefill: each sequence's new tokens in blocks of 16, the state in MFMA
 //                accumulators (delta_blocks first solves every block's 16 x 16 system);
 //                key dimensions past 256 take a token-by-token scan instead
@@ -20,7 +22,8 @@
 // last taps-1 projection rows (oldest first, in the storage type).  A sequence whose
 // first row of this launch is at position 0 starts from zeros, whatever its slot held:
 // slots are never cleared.  A negative slot (padded graph row) reads and writes nothing.
-// delta_prep only READS conv_state; the step / scan launch that follows it shifts it.
+// delta_prep only READS conv_state; the step / scan launch that follows it shifts it.  delta_step_conv
+// reads and shifts the channels of its own heads.
 // Everything that enters the recurrence is fp32; decays are carried as logarithms.
 #include "common.h"
 

@@ -26,13 +26,6 @@ using namespace omnia;
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ float4v mfma16(short8 a, short8 b, float4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 constexpr int BM = 64;  // rows per grouped-GEMM block (and alignment of expert segments)
 
 // ------------------------------------------------------------------ top-k

@@ -98,61 +98,49 @@ __global__ __launch_bounds__(NT) void embed_kernel(T* __restrict__ h, float* __r
   }
 }
 
-// Router logits of a row for up to EP experts, in the block that has the row: saves a launch.  The
-// router's columns are loaded ahead of everything else; a wave adds a column's EP products over its lanes
-// in EP - 1 + log2(64 / EP) exchanges, half of the values it still has going to the other lanes each
-// time.  Bound by the chain of loads, exchanges and the choice (figures at its rule).
-template <int EP>
+// Router logits of a row for up to 16 experts, in the block that has the row: saves a launch.  Waves 0 to
+// 7 take a part of the columns each, of up to NK steps of 32: experts are the columns of a product whose 16
+// rows are all this one, so that the sums are those of moe_route_kernel, bit for bit, and a row's experts do
+// not depend on how many rows its step has.  The router's values are asked for ahead of everything else.
+// Bound by the chain of loads, products and the choice (figures at its rule).
+template <int NK>
 struct Logits {
-  short4v w[EP];
-  __device__ __forceinline__ void load(const bf16_t* router, int E, int d, int c) {
-    // all at once, from valid places: columns past d are zeroed at their use, experts past E repeat the
-    // last one and are not read
-    const int at = min(c, d - 4);
+  short8 w[NK];
+  int k0, n;  // first step of this wave, and steps
+  __device__ __forceinline__ Logits(const bf16_t* router, int E, int d) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int nk = d / 32, per = (nk + 7) / 8;
+    k0 = wave * per;
+    n = wave < 8 ? min(nk - k0, per) : 0;
+    const bf16_t* r = router + (int64_t)min(lane & 15, E - 1) * d + 8 * (lane >> 4);
+    if (n > 0) {
 #pragma unroll
-    for (int e = 0; e < EP; ++e)
-      w[e] = *reinterpret_cast<const short4v*>(router + (int64_t)min(e, E - 1) * d + at);
+      for (int u = 0; u < NK; ++u)  // past the end: the last
+        w[u] = *reinterpret_cast<const short8*>(r + 32 * (k0 + min(u, n - 1)));
+    }
   }
-  // v: the row's values as the experts read them (live: columns of the row).  part [waves][EP]; ends
-  // with row z[0 .. E - 1]
-  template <int NT>
-  __device__ __forceinline__ void row(float4v v, bool live, float (*part)[EP], float* z) const {
+  // row: the values as the experts read them, in LDS; a wave's sums in part [wave][expert]
+  __device__ __forceinline__ void sums(const bf16_t* row, float (*part)[16]) const {
     const int lane = threadIdx.x & 63;
-    float s[EP];
+    float4v acc = {0.f, 0.f, 0.f, 0.f};
+    if (n > 0) {
+      const bf16_t* r = row + 32 * k0 + 8 * (lane >> 4);
 #pragma unroll
-    for (int e = 0; e < EP; ++e) {
-      s[e] = 0.f;
+      for (int i = 0; i < NK; i += 8) {
+        short8 x[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s[e] += v[j] * bf2f((uint16_t)w[e][j]);
-      s[e] = live ? s[e] : 0.f;
-    }
-    int at = 0;  // the value that this lane ends with
+        for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const short8*>(r + 32 * min(i + u, n - 1));
 #pragma unroll
-    for (int n = EP / 2, bit = 1; n >= 1; n /= 2, bit *= 2) {
-      const bool up = lane & bit;
-#pragma unroll
-      for (int i = 0; i < n; ++i) {
-        // (the asm keeps hipcc from making the choice one of an index, a comparison for every value)
-        float lo = s[i], hi = s[i + n];
-        asm("" : "+v"(lo), "+v"(hi));
-        s[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, bit, 64);
+        for (int u = 0; u < 8; ++u)
+          if (i + u < n) acc = mfma16(x[u], w[i + u], acc);
       }
-      at += up ? n : 0;
     }
-#pragma unroll
-    for (int o = EP; o < 64; o *= 2) s[0] += __shfl_xor(s[0], o, 64);
-    if (lane < EP) part[threadIdx.x >> 6][at] = s[0];
-    __syncthreads();
-    if (threadIdx.x < EP) {
-      float a = 0.f;
-      for (int i = 0; i < NT / 64; ++i) a += part[i][threadIdx.x];
-      z[threadIdx.x] = a;
-    }
+    if (threadIdx.x < 512 && lane < 16) part[threadIdx.x >> 6][lane] = acc[0];
   }
 };
 
-// EP: experts of a route behind the row (0: none)
-template <typename T, typename P, int NT, int NC, int EP>
+// NK: of a route behind the row (see Logits; 0: none)
+template <typename T, typename P, int NT, int NC, int NK>
 __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* __restrict__ x,
                                                        const P* __restrict__ m, int S,
                                                        int64_t row_stride, int64_t part_stride,
@@ -162,8 +150,10 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
                                                        Route route) {
   __shared__ float scratch[NT / 64];
   const int64_t t = blockIdx.x;
-  Logits<EP ? EP : 1> logits;
-  if constexpr (EP > 0) logits.load(router, route.E, d, threadIdx.x * 4);
+  [[maybe_unused]] const auto logits = [&] {
+    if constexpr (NK > 0) return Logits<NK>(router, route.E, d);
+    else return 0;
+  }();
   const P* mr = m + t * row_stride;
   float* xr = x + t * d;
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
@@ -203,14 +193,20 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
     const int c = (threadIdx.x + i * NT) * 4;
     if (c < d) store4(h + t * d + c, v[i]);
   }
-  if constexpr (EP > 0) {
-    static_assert(NC == 1 && sizeof(T) == 2, "columns of a thread");
-    __shared__ float part[NT / 64][EP];
-    __shared__ float z[16];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[0][j] = bf2f(f2bf(v[0][j]));  // what h holds
-    logits.template row<NT>(v[0], threadIdx.x * 4 < d, part, z);
+  if constexpr (NK > 0) {
+    static_assert(NC == 1 && NT == 1024 && sizeof(T) == 2, "columns of a thread");
+    __shared__ __attribute__((aligned(16))) bf16_t row[4 * NT];
+    __shared__ float part[8][16], z[16];
+    const int c = threadIdx.x * 4;
+    if (c < d) store4(row + c, v[0]);
+    __syncthreads();
+    logits.sums(row, part);
+    __syncthreads();
     if (threadIdx.x < 16) {  // one wave: its LDS in order
+      float a = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) a += part[i][threadIdx.x];
+      z[threadIdx.x] = a;
       __builtin_amdgcn_wave_barrier();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       choose<16, 1>(z, threadIdx.x, t, route);
@@ -301,20 +297,20 @@ int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int
   if (rows == 0) return 0;
   const Norm post{w_post, inv_n, eps}, pre{w_pre, inv_n, eps};
   const Route route{ids, wts, corr, rbias, E, k, sigmoid, renorm, groups, keep};
-#define OMNIA_RE(TT, PP, NT, N, EP)                                                             \
-  residual_kernel<TT, PP, NT, N, EP><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride, \
+#define OMNIA_RE(TT, PP, NT, N, NK)                                                             \
+  residual_kernel<TT, PP, NT, N, NK><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride, \
                                                          part_stride, d, bias, post, pre,       \
                                                          (const bf16_t*)router, route)
   if (router) {
     if (f32 || !omnia_rms_residual_routes(rows, d, E) || k < 1 || k > E) return -3;
     if (groups < 1 || E % groups || keep < 1 || keep > groups || k > keep * (E / groups)) return -4;
-#define OMNIA_RT(EP)                                           \
+#define OMNIA_RT(NK)                                           \
   do {                                                         \
-    if (ptype == 0) OMNIA_RE(bf16_t, bf16_t, 1024, 1, EP);     \
-    else if (ptype == 1) OMNIA_RE(bf16_t, float, 1024, 1, EP); \
-    else OMNIA_RE(bf16_t, _Float16, 1024, 1, EP);              \
+    if (ptype == 0) OMNIA_RE(bf16_t, bf16_t, 1024, 1, NK);     \
+    else if (ptype == 1) OMNIA_RE(bf16_t, float, 1024, 1, NK); \
+    else OMNIA_RE(bf16_t, _Float16, 1024, 1, NK);              \
   } while (0)
-    if (E <= 8) OMNIA_RT(8);
+    if (d <= 2048) OMNIA_RT(8);
     else OMNIA_RT(16);
 #undef OMNIA_RT
     return (int)hipGetLastError();

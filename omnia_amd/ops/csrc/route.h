@@ -5,6 +5,13 @@
 
 namespace omnia {
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ float4v mfma16(short8 a, short8 b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 // Router for any score function: logits z[e] = x . router[e] (+ bias[e]) stay in fp32;
 // weights are sigmoid(z) or softmax(z), renormalised over the chosen ones if asked.  The k
 // largest choice scores are chosen: z, or with a correction score + correction (weights stay

@@ -10,8 +10,8 @@ from omnia_amd.ops import mixers as mops
 pytestmark = pytest.mark.gpu
 
 
-# widths where the last threads have no columns and where all have; counts of experts around the
-# kernel's two; every kind of choice; a row of NaN
+# widths where the last threads have no columns and where all have; counts of experts up to the
+# kernel's 16; every kind of choice; a row of NaN
 @pytest.mark.parametrize("rows,d", [(1, 1056), (8, 2048), (77, 4096), (512, 2080)])
 @pytest.mark.parametrize("E,k,score,renorm,groups,keep,extra", [
     (8, 2, "sigmoid", False, 1, 1, False), (6, 2, "softmax", True, 1, 1, True),
@@ -41,11 +41,8 @@ def test_route(rows, d, E, k, score, renorm, groups, keep, extra):
     ids, wts = route.empty(rows, dev)
     ops.kernels().moe_route(ids, wts, h2, w["router"], k, score == "sigmoid", renorm,
                             w.get("correction"), groups, keep, w.get("router_b"))
-    # fp32 sums of d products in two orders: some 2^-24 sqrt(d) of logits of about one.  Where the
-    # choice lies that close, either is right
-    close = (route.wts - wts).abs().amax(1) <= 2e-5
-    same = (route.ids == ids).all(1)
-    assert bool((same & close)[torch.arange(rows, device=dev) != 3].float().mean() >= 0.99)
+    # the sums of both kernels are the same, so that experts do not depend on a step's count of rows
+    assert torch.equal(route.ids, ids) and torch.equal(route.wts, wts)
     assert int(route.ids.min()) >= 0 and int(route.ids.max()) < E
     assert all(len(set(r)) == k for r in route.ids.tolist())
 
@@ -89,10 +86,5 @@ def test_route_of_parts(rows, d, E, k, kind):
         assert torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
     ids, wts = route.empty(rows, dev)
     ops.kernels().moe_route(ids, wts, h2, w["router"], k, True, False, None, 1, 1, None)
-    odd = slice(1, 4)
-    assert torch.equal(route.ids[odd], ids[odd])
-    assert torch.equal(route.wts[odd].nan_to_num(nan=7.0), wts[odd].nan_to_num(nan=7.0))
-    # elsewhere fp32 sums of d products in two orders, as above
-    rest = torch.tensor([i for i in range(rows) if i not in (1, 2, 3)], device=dev)
-    close = (route.wts - wts).abs().amax(1) <= 2e-5
-    assert bool(((route.ids == ids).all(1) & close)[rest].float().mean() >= 0.99)
+    assert torch.equal(route.ids, ids)
+    assert torch.equal(route.wts.nan_to_num(nan=7.0), wts.nan_to_num(nan=7.0))
