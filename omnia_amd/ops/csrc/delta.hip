@@ -119,6 +119,13 @@ __global__ __launch_bounds__(256) void prep_kernel(
   for (int i = n + lane; i < Dp; i += 64) qk[i] = 0.f;
 }
 
+// A tap more of a convolution: oldest input, newest, those between.  Fused by name: of the first two
+// products hipcc fuses either, and not the same in every kernel, so that fp32 rows differed by which kernel
+// their step took.
+__device__ __forceinline__ float conv_add(float a, float in, float w) {
+  return __builtin_fmaf(in, w, a);
+}
+
 // Fast path (taps <= 4, head sizes up to 64 * VEC * NE, even when VEC = 2): a wave takes
 // a run of TR consecutive rows of one unit: 8, which reads 11 rows for 8, or 4 while the chip holds
 // the waves of all of them at once (32 a CU), since the time is then the chain of a run (us in runs of
@@ -246,9 +253,10 @@ __global__ __launch_bounds__(256) void prep_run_kernel(
     for (int e = 0; e < NE; ++e)
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
-        float a = in[r][e][v] * w[e][v][TAPS - 1];
+        float a = (TAPS > 1 ? hist[0][e][v] : in[r][e][v]) * w[e][v][0];
+        if (TAPS > 1) a = conv_add(a, in[r][e][v], w[e][v][TAPS - 1]);
 #pragma unroll
-        for (int j = 0; j < TAPS - 1; ++j) a += hist[j][e][v] * w[e][v][j];
+        for (int j = 1; j < TAPS - 1; ++j) a = conv_add(a, hist[j][e][v], w[e][v][j]);
         a = siluf_(a);
         y[e][v] = a;
         ss += a * a;
@@ -484,10 +492,11 @@ __global__ __launch_bounds__(256 * R) void step_conv_kernel(
     float a[2], ss = 0.f;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
-      a[v] = in[v] * (taps == 4 ? cw[v][3] : taps == 3 ? cw[v][2] : cw[v][1]);
+      a[v] = conv_add(hist[0][v] * cw[v][0], in[v],
+                      taps == 4 ? cw[v][3] : taps == 3 ? cw[v][2] : cw[v][1]);
 #pragma unroll
-      for (int j = 0; j < 3; ++j)
-        if (j < taps - 1) a[v] += hist[j][v] * cw[v][j];
+      for (int j = 1; j < 3; ++j)
+        if (j < taps - 1) a[v] = conv_add(a[v], hist[j][v], cw[v][j]);
       a[v] = siluf_(a[v]);
       ss += a[v] * a[v];
     }
@@ -854,9 +863,9 @@ __global__ __launch_bounds__(256 * (2 + R)) void prep_blocks_kernel(
     float y[2], ss = 0.f;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
-      float a = in[r][v] * wt[v][TAPS - 1];
+      float a = conv_add(hist[0][v] * wt[v][0], in[r][v], wt[v][TAPS - 1]);
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) a += hist[j][v] * wt[v][j];
+      for (int j = 1; j < TAPS - 1; ++j) a = conv_add(a, hist[j][v], wt[v][j]);
       a = siluf_(a);
       y[v] = a;
       ss += a * a;
