@@ -99,19 +99,22 @@ __global__ __launch_bounds__(NT) void embed_kernel(T* __restrict__ h, float* __r
 }
 
 // Router logits of a row for up to 16 experts, in the block that has the row: saves a launch.  Waves 0 to
-// 7 take a part of the columns each, of up to NK steps of 32: experts are the columns of a product whose 16
-// rows are all this one, so that the sums are those of moe_route_kernel, bit for bit, and a row's experts do
-// not depend on how many rows its step has.  The router's values are asked for ahead of everything else.
-// Bound by the chain of loads, products and the choice (figures at its rule).
-template <int NK>
+// 7 take a part of the columns each, up to 8 steps of 32 of it, and past 2048 columns waves 8 to 15 the
+// rest from where those ended: experts are the columns of a product whose 16 rows are all this one, so that
+// the sums are those of moe_route_kernel, bit for bit, and a row's experts do not depend on how many rows
+// its step has.  The router's values are asked for behind the row's parts, and arrive during the norms (ahead
+// of the parts 0.7 us more), at most 8 steps a wave, so that two blocks share a CU (16 steps in 8 waves, one
+// block: 264 rows of 16 experts of 4096 columns 16.4 us, now 12.6).  Bound by the chain of loads, sums,
+// products and the choice (figures at its rule).
 struct Logits {
+  static constexpr int NK = 8;
   short8 w[NK];
   int k0, n;  // first step of this wave, and steps
   __device__ __forceinline__ Logits(const bf16_t* router, int E, int d) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int nk = d / 32, per = (nk + 7) / 8;
-    k0 = wave * per;
-    n = wave < 8 ? min(nk - k0, per) : 0;
+    const int nk = d / 32, per = (nk + 7) / 8, first = (wave & 7) * per, skip = wave < 8 ? 0 : NK;
+    k0 = first + skip;
+    n = min(min(nk - first, per) - skip, NK);
     const bf16_t* r = router + (int64_t)min(lane & 15, E - 1) * d + 8 * (lane >> 4);
     if (n > 0) {
 #pragma unroll
@@ -119,41 +122,47 @@ struct Logits {
         w[u] = *reinterpret_cast<const short8*>(r + 32 * (k0 + min(u, n - 1)));
     }
   }
-  // row: the values as the experts read them, in LDS; a wave's sums in part [wave][expert]
-  __device__ __forceinline__ void sums(const bf16_t* row, float (*part)[16]) const {
-    const int lane = threadIdx.x & 63;
-    float4v acc = {0.f, 0.f, 0.f, 0.f};
-    if (n > 0) {
-      const bf16_t* r = row + 32 * k0 + 8 * (lane >> 4);
+  // row: the values as the experts read them, in LDS; acc: the sums so far
+  __device__ __forceinline__ void products(float4v& acc, const bf16_t* row) const {
+    const bf16_t* r = row + 32 * k0 + 8 * ((threadIdx.x & 63) >> 4);
 #pragma unroll
-      for (int i = 0; i < NK; i += 8) {
-        short8 x[8];
+    for (int i = 0; i < NK; i += 4) {
+      short8 x[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const short8*>(r + 32 * min(i + u, n - 1));
+      for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const short8*>(r + 32 * min(i + u, n - 1));
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (i + u < n) acc = mfma16(x[u], w[i + u], acc);
-      }
+      for (int u = 0; u < 4; ++u)
+        if (i + u < n) acc = mfma16(x[u], w[i + u], acc);
     }
-    if (threadIdx.x < 512 && lane < 16) part[threadIdx.x >> 6][lane] = acc[0];
+  }
+  // part [part][expert]; ends with a barrier
+  __device__ __forceinline__ void sums(const bf16_t* row, int d, float (*part)[16]) const {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float* mine = &part[wave & 7][lane & 15];
+    float4v acc = {0.f, 0.f, 0.f, 0.f};
+    if (wave < 8) {
+      if (n > 0) products(acc, row);
+      if (lane < 16) *mine = acc[0];
+    }
+    __syncthreads();
+    if (d <= 32 * 8 * NK) return;
+    if (wave >= 8 && n > 0) {
+      acc = float4v{*mine, *mine, *mine, *mine};  // rows alike
+      products(acc, row);
+      if (lane < 16) *mine = acc[0];
+    }
+    __syncthreads();
   }
 };
 
-// NK: of a route behind the row (see Logits; 0: none)
-template <typename T, typename P, int NT, int NC, int NK>
-__global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* __restrict__ x,
-                                                       const P* __restrict__ m, int S,
-                                                       int64_t row_stride, int64_t part_stride,
-                                                       int d, const float* __restrict__ bias,
-                                                       Norm post, Norm pre,
-                                                       const bf16_t* __restrict__ router,
-                                                       Route route) {
+// ROUTE: the row's experts behind it
+template <typename T, typename P, int NT, int NC, bool ROUTE>
+__global__ __launch_bounds__(NT, ROUTE ? 8 : 1) void residual_kernel(
+    T* __restrict__ h, float* __restrict__ x, const P* __restrict__ m, int S, int64_t row_stride,
+    int64_t part_stride, int d, const float* __restrict__ bias, Norm post, Norm pre,
+    const bf16_t* __restrict__ router, Route route) {
   __shared__ float scratch[NT / 64];
   const int64_t t = blockIdx.x;
-  [[maybe_unused]] const auto logits = [&] {
-    if constexpr (NK > 0) return Logits<NK>(router, route.E, d);
-    else return 0;
-  }();
   const P* mr = m + t * row_stride;
   float* xr = x + t * d;
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
@@ -178,6 +187,10 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
       }
     }
   }
+  [[maybe_unused]] const auto logits = [&] {
+    if constexpr (ROUTE) return Logits(router, route.E, d);
+    else return 0;
+  }();
   norm_row<NT, NC>(v, d, post, scratch);
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
@@ -193,15 +206,14 @@ __global__ __launch_bounds__(NT) void residual_kernel(T* __restrict__ h, float* 
     const int c = (threadIdx.x + i * NT) * 4;
     if (c < d) store4(h + t * d + c, v[i]);
   }
-  if constexpr (NK > 0) {
+  if constexpr (ROUTE) {
     static_assert(NC == 1 && NT == 1024 && sizeof(T) == 2, "columns of a thread");
     __shared__ __attribute__((aligned(16))) bf16_t row[4 * NT];
     __shared__ float part[8][16], z[16];
     const int c = threadIdx.x * 4;
     if (c < d) store4(row + c, v[0]);
     __syncthreads();
-    logits.sums(row, part);
-    __syncthreads();
+    logits.sums(row, d, part);
     if (threadIdx.x < 16) {  // one wave: its LDS in order
       float a = 0.f;
 #pragma unroll
@@ -269,18 +281,16 @@ int omnia_rms_embed(void* h, float* x, const int* ids, const void* table, int f3
 }
 
 // Whether omnia_rms_residual takes a router of E experts along: rows of one chunk of 4 columns for each of
-// 1024 threads.  Every row's block reads the router, where the kernel that only routes reads it once for
-// 16 rows; blocks past 256 wait for a second round of the chip, which of more than 8 experts pays from 2048
-// columns.  us of residual step and routing, two launches / one, 8
-// experts: 1056 columns 1 / 64 / 256 / 264 / 512 rows 5.6 / 7.4 / 7.9 / 8.2 / 8.8 and 5.3 / 5.8 / 6.1 / 7.7
-// / 8.3, 2048 6.6 / 8.8 / 9.6 / 10.1 / 11.1 and 5.4 / 5.8 / 6.4 / 8.2 / 8.9, 4096 8.6 / 12.2 / 13.4 / 14.1
-// / 15.7 and 6.0 / 6.5 / 7.4 / 9.4 / 10.6; 16 experts: 1056 5.9 / 7.6 / 8.0 / 8.4 / 9.1 and 6.8 / 7.2 / 7.7
-// / 10.2 / 10.9 (8 rows 7.1 both), 1536 6.9 / 8.8 / 9.3 / 9.8 / 10.6 and 6.8 / 7.2 / 7.8 / 10.3 / 11.1, 2048
-// 7.4 / 9.7 / 10.4 / 10.9 / 11.9 and 6.9 / 7.4 / 8.0 / 10.6 / 11.4, 4096 9.9 / 13.6 / 14.8 / 15.5 / 17.1 and
-// 7.5 / 8.1 / 9.2 / 12.1 / 13.2.  Slabs and slots the same within 0.5.
+// 1024 threads, as many as have such blocks.  Every row's block reads the router, where the kernel that only
+// routes reads it once for 16 rows.  us of residual step and routing, two launches / one, at 1 / 64 / 256 /
+// 264 / 512 rows, 8 experts: 1056 columns 5.2 / 6.7 / 7.2 / 7.7 / 8.3 and 4.1 / 4.6 / 4.8 / 5.9 / 6.4, 2048
+// 6.1 / 8.3 / 9.0 / 9.6 / 10.5 and 4.4 / 4.8 / 5.3 / 6.6 / 7.4, 4096 8.0 / 11.5 / 12.9 / 13.3 / 15.1 and 6.1 /
+// 6.5 / 7.3 / 10.1 / 11.3; 16 experts: 1056 5.5 / 7.0 / 7.4 / 7.9 / 8.5 and 4.5 / 4.9 / 5.3 / 6.3 / 6.8, 2048
+// 7.0 / 9.1 / 9.8 / 10.4 / 11.3 and 5.2 / 5.7 / 6.1 / 8.0 / 8.7, 4096 9.4 / 13.1 / 14.3 / 14.8 / 16.7 and 7.5 /
+// 8.1 / 8.7 / 12.6 / 13.9; of three fp32 slabs, 16 experts of 4096 9.7 / 13.2 / 14.6 / 15.4 / 18.2 and 8.3 /
+// 8.7 / 9.5 / 13.7 / 15.9.
 int omnia_rms_residual_routes(int64_t rows, int64_t d, int64_t E) {
-  if (E < 1 || E > 16 || rows > 512 || d <= 1024 || d > 4096 || d % 32) return 0;
-  return E <= 8 || rows <= 256 || d >= 2048;
+  return E >= 1 && E <= 16 && rows <= 512 && d > 1024 && d <= 4096 && d % 32 == 0;
 }
 
 // ptype: storage of `m` -- 0 bf16, 1 fp32, 2 fp16 (slabs).  router: null, or [E, d] bf16: the rows'
@@ -297,25 +307,19 @@ int omnia_rms_residual(void* h, int f32, float* x, const void* m, int ptype, int
   if (rows == 0) return 0;
   const Norm post{w_post, inv_n, eps}, pre{w_pre, inv_n, eps};
   const Route route{ids, wts, corr, rbias, E, k, sigmoid, renorm, groups, keep};
-#define OMNIA_RE(TT, PP, NT, N, NK)                                                             \
-  residual_kernel<TT, PP, NT, N, NK><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride, \
+#define OMNIA_RE(TT, PP, NT, N, ROUTE)                                                           \
+  residual_kernel<TT, PP, NT, N, ROUTE><<<rows, NT, 0, s>>>((TT*)h, x, (const PP*)m, S, row_stride, \
                                                          part_stride, d, bias, post, pre,       \
                                                          (const bf16_t*)router, route)
   if (router) {
     if (f32 || !omnia_rms_residual_routes(rows, d, E) || k < 1 || k > E) return -3;
     if (groups < 1 || E % groups || keep < 1 || keep > groups || k > keep * (E / groups)) return -4;
-#define OMNIA_RT(NK)                                           \
-  do {                                                         \
-    if (ptype == 0) OMNIA_RE(bf16_t, bf16_t, 1024, 1, NK);     \
-    else if (ptype == 1) OMNIA_RE(bf16_t, float, 1024, 1, NK); \
-    else OMNIA_RE(bf16_t, _Float16, 1024, 1, NK);              \
-  } while (0)
-    if (d <= 2048) OMNIA_RT(8);
-    else OMNIA_RT(16);
-#undef OMNIA_RT
+    if (ptype == 0) OMNIA_RE(bf16_t, bf16_t, 1024, 1, true);
+    else if (ptype == 1) OMNIA_RE(bf16_t, float, 1024, 1, true);
+    else OMNIA_RE(bf16_t, _Float16, 1024, 1, true);
     return (int)hipGetLastError();
   }
-#define OMNIA_RR(TT, PP, NT, N) OMNIA_RE(TT, PP, NT, N, 0)
+#define OMNIA_RR(TT, PP, NT, N) OMNIA_RE(TT, PP, NT, N, false)
 #define OMNIA_RRN(NT, N)                                       \
   do {                                                      \
     if (f32) OMNIA_RR(float, float, NT, N);                     \
