@@ -956,19 +956,19 @@ struct ScanShared {
 // meet in LDS, added by all in one order, so that all hold the same u; parts of the output are
 // added by the moving waves, a block later.  A wave that has twice the tiles keeps two sums, so that the
 // order of additions, and with it every bit of a sequence's results, is that of four waves (one sum a wave
-// of two was 1 % faster where the chip is full: 16 heads of 128, 2048 rows of 8 285 -> 288 us).
+// of two was 1 % faster where the chip is full: 16 heads of 128, 2048 rows of 8 351 -> 354 us).
 // Bound by the serial chain of a block where few blocks run: K S, the exchange, T', K^T U, 20 of a
 // wave's 29 fp32 products (13.3 ns each) and the latencies between them.  A wave issues an
 // instruction in about 5 clocks and none beside its own products, so whatever is not on the chain
 // is another wave's work: with the staging in the multiplying waves the 16 heads of 4000 rows below
 // took 262 us, with operands straight from global memory 282.  Where the chip is full, fp32
 // products and vector instructions share one unit: of heads of 128, a wave of two has 54 products (16 each
-// of K S, Q S and K^T U, 4 of T', 2 of P U) and a SIMD 108, of its two blocks: 1.44 of the 2.1 us that a
+// of K S, Q S and K^T U, 4 of T', 2 of P U) and a SIMD 108, of its two blocks: 1.44 of the 2.4 us that a
 // block of 32 columns takes.
 // us with blocks_kernel, one wave a 16 columns and all of their key dimensions -> now, heads of 128: 16 heads,
-// 77 rows 23 -> 14, 1000 146 -> 52, 4000 547 -> 184, 333 of 3 61 -> 36, 60 of 16 36 -> 33, 512 of 32 298 ->
-// 290, 2048 of 8 330 -> 288; 32 heads, 333 of 3 64 -> 55, 2048 of 8 583 -> 577;
-// 8 heads of 256 x 128, 333 of 3 114 -> 39, 512 of 32 400 -> 336; heads of 64: at their rule in scan.
+// 77 rows 23 -> 14, 1000 151 -> 56, 4000 550 -> 190, 333 of 3 63 -> 38, 60 of 16 38 -> 36, 512 of 32 336 ->
+// 336, 2048 of 8 392 -> 354; 32 heads, 333 of 3 68 -> 61, 8192 1168 -> 437, 2048 of 8 686 -> 689; 8 heads of
+// 256 x 128, 333 of 3 116 -> 41, 512 of 32 430 -> 368; heads of 64: at their rule in scan.
 template <typename T, int ND, int NW, int CW>
 __global__
 __launch_bounds__(64 * (NW * CW + 4), ND <= 4 || ND / NW <= 2 ? 4 : 2) void scan_blocks_kernel(
