@@ -18,6 +18,17 @@
 //     are one a CU; S blocks share a column tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
 //     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
 //     depend on how many rows the step has;
+//   * rows of a weight are a power of two of bytes apart, or nearly, and blocks walk them in step, so
+//     at any time all would ask a few memory channels for their 128 bytes of every row.  Blocks of
+//     row-major weights of 64 MB and more therefore take the chunks of a power of two each in another
+//     order: by the number of its eight weight units, whatever the waves and rows, so that bits do not
+//     depend on them, and its bits reversed, so that blocks that run together are far apart.  us, in
+//     order / apart: gated 28672 x 4096 at 32 / 77 / 128 rows 45.2 / 36.8, 49.3 / 42.0, 54.4 / 49.4;
+//     gated 22016 x 4096 38.0 / 32.1, 42.7 / 39.6, 49.3 / 47.0; 4096 x 14336 25.8 / 20.6, 28.6 / 24.6,
+//     31.9 / 28.6; gated 16384 x 2048 15.8 / 12.6, 18.6 / 16.5, 22.9 / 21.7; 32768 x 2048 32.0 / 22.9,
+//     32.8 / 24.3, 34.6 / 28.6.  Smaller ones have little to gain and may lose (8192 x 2048 gated at 32
+//     9.6 / 9.2, 4096 x 4096 7.9 / 8.8), packed ones, 2 KB a chunk and unit, as well (28672 x 4096 40.3
+//     / 47.1);
 //   * a ring of NS stages, of which NS - 1 stay in flight across the one raw barrier of a stage.
 //     Past the end the loads go to one line, so that every wait counts the same number of loads.
 //     The DMA is written as asm: hipcc, not knowing which stage a fragment read belongs to,
@@ -123,6 +134,10 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(const bf16_t* x, cons
   const bool full = XW == 0 || wv < WN - XW;
   const int K = p.K, nch = K >> 6;
   const int c0 = split * nch / p.S, n = (split + 1) * nch / p.S - c0;  // 64-k chunks: stages
+  // stage s of this block is chunk s ^ turn of its slice, by its weights' place alone
+  int turn = 0;
+  if (!PK && !grouped(EPI) && (int64_t)p.N * K >= (paired(EPI) ? 1 << 24 : 1 << 25))
+    turn = (int)(__builtin_bitreverse32(tile * WN >> 3) >> 26) & ((n & -n) - 1);
 
   // this wave's weights: row-major, rows 8h.. of the unit and 16-byte chunk lane & 7 of each;
   // packed, lane 16q + r's chunk of step h
@@ -163,7 +178,7 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(const bf16_t* x, cons
   auto issue = [&](int slot, int s) {  // stage s into a slot
     const uint32_t dst = lds0 + slot * ST * 2;
     const bool in = s < n;
-    const int64_t c = c0 + s;
+    const int64_t c = c0 + (s ^ turn);
 #pragma unroll
     for (int i = 0; i < XI; ++i)
       if (full || i < XI - 1)

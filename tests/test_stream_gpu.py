@@ -458,6 +458,29 @@ def test_panel_gated_in_blocks_of_two_waves(M, R, K, packed, monkeypatch):
                                  None, False)
 
 
+@pytest.mark.parametrize("gated,R,K", [(False, 32784, 1024), (False, 32768, 1088), (False, 2048, 16448),
+                                       (True, 16416, 2112), (True, 16384, 2048)])
+def test_panel_of_weights_whose_chunks_are_taken_apart(gated, R, K):
+    """Row-major weights of 64 MB and more: of every chunk once, also where their number is odd, has
+    a small power of two or more than 64, in slices too; a row's bits are the same whatever the rows
+    beside it and in blocks of other waves."""
+    x, w = _mk(200, R, K, R + K)
+    whole = ops.panel(int(gated), x, w, slabs=not gated)
+    y = whole.sum(0) if whole.dim() == 3 else whole
+    want = x.double() @ w.double().T
+    if gated:
+        g, u = want.chunk(2, 1)
+        want = F.silu(g) * u
+    _close(y, want, 4 * K, 1.1)
+    for M in (1, 33, 100):
+        assert torch.equal(ops.panel(int(gated), x[:M], w, slabs=not gated), whole[..., :M, :])
+    if whole.dim() == 2:
+        out = [torch.empty_like(whole) for _ in range(3)]
+        for o, wn in zip(out, (2, 4, 8)):
+            ops.kernels().panel_gemm(int(gated), o, x, w, wn, False, None, False)
+            assert torch.equal(o, whole)
+
+
 def test_panel_plans_fit_the_kernel():
     """Whatever the size, a plan is one that the kernel covers, with slices that do not depend on
     the rows."""
