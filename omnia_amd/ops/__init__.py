@@ -404,7 +404,8 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     with ``ss_out[r, t]`` = sum of squares of its new 256-column slice t;
     3: QKV -> RoPE'd q in ``out`` [M, hq*128], RoPE'd k and v written to the
     paged caches at ``slots``.  ``cols``: weight rows of a tile, 256 or (epi 0, 1) 128, to the
-    same bits; 0: :func:`tile_cols`."""
+    same bits; of 256, a last round's are cut in two where that fills the chip better.  0: 128 where
+    all tiles are one round of that, which the kernel of both has 0.4 us more to find, else 256."""
     M, K = x.shape
     N = w.shape[0] // 2 if epi == 1 else w.shape[0]
     if out is None:
@@ -412,8 +413,9 @@ def pgemm(epi: int, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None =
     if x.is_cuda:
         if epi == 3 and checks.active(x):
             checks.slots("pgemm qkv", slots, k_cache)
-        if not cols and epi <= 1:
-            cols = tile_cols(M, w.shape[0])
+        if not cols and epi <= 1 and tile_cols(M, w.shape[0]) == 128 and \
+                _tile_rounds(M, w.shape[0], 128) == 1:
+            cols = 128
         kernels().pgemm(epi, out, x.contiguous(), w, ss_in, inv_d, eps, ss_out, positions,
                         cos_sin, k_cache, v_cache, slots, hq, hkv, block_size, bias, gelu, cols)
         return out
@@ -449,7 +451,7 @@ def _tile_rounds(M: int, R: int, cols: int) -> int:
 
 @functools.lru_cache(maxsize=8192)
 def tile_cols(M: int, R: int) -> int:
-    """Columns of :func:`pgemm`'s tile for ``M`` rows and ``R`` weight rows: 128 where that fills
+    """Columns of a tile for ``M`` rows and ``R`` weight rows, were all alike: 128 where that fills
     the rounds over 256 CUs better, by more than its second read of x.  A round of narrow tiles
     takes 0.57 to 0.6 of a wide one's (us wide / narrow and their rounds: gated 16384 x 2048 at 300
     rows 43.8 / 31.2 (1, 1), 600 45.6 / 54.4 (1, 2), 1536 92.5 / 87.0 (2, 3), 2001 103 / 120 (2,
@@ -463,6 +465,12 @@ def _tiles_useful(M: int, R: int) -> float:
     """Part of the work of :func:`pgemm`'s rounds that is not padding."""
     cols = tile_cols(M, R)
     return M * R / (256 * 256 * cols * _tile_rounds(M, R, cols))
+
+
+def _cut_rounds(tiles: int) -> float:
+    """Rounds over 256 CUs that wide tiles take where those of the last are cut in two if they fill
+    half of it or less."""
+    return tiles // 256 + (0.0, 0.6, 1.0)[(tiles % 256 > 0) + (tiles % 256 > 128)]
 
 
 def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
@@ -483,11 +491,18 @@ def gated_tile_fills(M: int, w: torch.Tensor) -> bool:
 def gated_tile_pays(M: int, w: torch.Tensor) -> bool:
     """:func:`gated_tile_fills` of the wide tile or, by the same line, of the narrow one where
     :func:`tile_cols` takes that (us, here / library and activation kernel: 8192 features of 2048 at
-    300 rows .59 useful 31.2 / 35.1, 512 1.0 32.8 / 40.9, 1280 .83 82.7 / 84.2; 14336 of 4096 at
-    600 .68 149 / 139, 768 .88 162 / 158)."""
-    return gated_tile_fills(M, w) or (
-        M > PANEL_MAX_M and tile_cols(M, w.shape[0]) == 128 and
-        _tiles_useful(M, w.shape[0]) > 0.75 and w.is_contiguous() and _on_grid(w))
+    300 rows .59 useful 31.2 / 35.1, 512 1.0 32.8 / 40.9); of more than a round of wide tiles, whose
+    last ones are cut in two, from .67 of :func:`_cut_rounds` useful (14336 of 4096 at 600 .64 144 / 144,
+    800 .68 180 / 187, 1100 .72 229 / 242, 1280 .84 235 / 258, 1700 .81 310 / 348; 8192 of 2048 at
+    1100 .67 72 / 84, 1280 .78 74.3 / 86.7)."""
+    R = w.shape[0]
+    if gated_tile_fills(M, w):
+        return True
+    if M <= PANEL_MAX_M or R % 256 or not (w.is_contiguous() and _on_grid(w)):
+        return False
+    tiles = -(-M // 256) * (R // 256)
+    return (tile_cols(M, R) == 128 and _tiles_useful(M, R) > 0.75) or \
+        (tiles > 256 and M * R > 0.67 * 256 ** 3 * _cut_rounds(tiles))
 
 
 def plain_tile_fills(M: int, w: torch.Tensor) -> bool:

@@ -116,6 +116,14 @@ constexpr bool gated(int epi) {
 constexpr bool sliced(int epi) { return epi == 4 || epi == 11; }
 // rows are expert-sorted assignments
 constexpr bool grouped(int epi) { return epi == 5 || epi == 6 || epi == 8 || epi == 10; }
+// wide tiles may be cut in two narrow ones
+constexpr bool cuts(int epi) { return epi != 2 && epi != 3 && !sliced(epi); }
+// Of ``wide`` tiles with ``light`` half ones behind them, how many of the last round over 256 CUs to
+// cut in two.
+__host__ __device__ constexpr int cut_tiles(int wide, int light) {
+  const int last = wide & 255;
+  return 2 * last + light <= 256 ? last : 0;
+}
 // A rows are token rows gathered by assignment
 constexpr bool gathered(int epi) { return epi == 5 || epi == 8 || epi == 10; }
 
@@ -201,6 +209,25 @@ __device__ __forceinline__ uint4v chunk(float4v c, float4v d) {
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// scale of row i of a tile from row m0, of which Mt are live
+template <int EPI>
+__device__ __forceinline__ float row_scale(const PArgs& p, int m0, int Mt, int i) {
+  if constexpr (EPI == 6 || EPI == 8) {  // the assignment's routing weight
+    const int f = p.sorted[m0 + i];
+    return f >= p.n_assign ? 0.f : p.route_w ? p.route_w[f] : 1.f;
+  }
+  const float* s = p.ss_in + (int64_t)(m0 + (i < Mt ? i : Mt - 1)) * p.ss_in_n;
+  float t = 0.f;
+  for (int k = 0; k < p.ss_in_n; k += 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = s[k + j < p.ss_in_n ? k + j : k];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t += k + j < p.ss_in_n ? v[j] : 0.f;
+  }
+  return __builtin_amdgcn_rsqf(t * p.inv_d + p.eps);
 }
 
 // Tile (mt, nt) of K-slice ks
@@ -364,22 +391,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   constexpr bool ROUTED = EPI == 6 || EPI == 8;
   constexpr bool UNSCALED = EPI == 2 || sliced(EPI) || EPI == 5 || EPI == 7 || EPI == 9 || EPI == 10;
   const bool scaled = ROUTED || (!UNSCALED && p.ss_in != nullptr);
-  float own = 1.f;
-  if constexpr (ROUTED) {  // the assignment's routing weight
-    const int f = p.sorted[m0 + tid];
-    own = f >= p.n_assign ? 0.f : p.route_w ? p.route_w[f] : 1.f;
-  } else if (scaled) {
-    const float* s = p.ss_in + (int64_t)(m0 + (tid < Mt ? tid : Mt - 1)) * p.ss_in_n;
-    float t = 0.f;
-    for (int i = 0; i < p.ss_in_n; i += 8) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = s[i + j < p.ss_in_n ? i + j : i];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) t += i + j < p.ss_in_n ? v[j] : 0.f;
-    }
-    own = __builtin_amdgcn_rsqf(t * p.inv_d + p.eps);
-  }
+  const float own = scaled ? row_scale<EPI>(p, m0, Mt, tid) : 1.f;
 
   // d: DMA or -1; first: the accumulator's first product
   auto product = [&](int set, int j, int d, bool first) __attribute__((always_inline)) {
@@ -683,15 +695,15 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
   p.n_blocks = n_blocks, p.blk_expert = blk_expert, p.sorted = sorted;
   __shared__ __attribute__((aligned(1024))) bf16_t lds[ring(SHAPE)];
   constexpr int TN = (gated(EPI) ? 128 : 256) / (SHAPE == NARROW ? 2 : 1);
-  constexpr bool MOE = grouped(EPI);
+  constexpr bool MOE = grouped(EPI), CUT = SHAPE == WIDE && cuts(EPI);
   // sliced: the K-slices are extra "m-tiles" of the L2 grouping below (blocks of
   // one slice share its x slice, blocks of one column tile its W rows)
   const int S = sliced(EPI) ? p.splits : 1;
   // MoE: the grid is sized for the worst-case segment count (graph-safe, no host sync); the
   // live tiles are spread over the XCDs, the other blocks leave
   constexpr int WORDS = 4;
-  const int lane = threadIdx.x & 63, most = p.M >> 8;
-  bool light = false, ordered = MOE && SHAPE == WIDE && most <= 64 * WORDS && gridDim.x <= 9 * 256;
+  const int lane = threadIdx.x & 63, most = p.M >> 8, ntn = p.N / TN;
+  bool light = false, ordered = MOE && SHAPE == WIDE && most <= 64 * WORDS && most * ntn <= 9 * 256;
   // of segments 64 i + lane, asked for beside their number: assignment 128, and whether the segment
   // before is of the same expert
   int half[WORDS], expert[WORDS], last[WORDS];
@@ -705,9 +717,8 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
           expert[i] = p.blk_expert[s];
           last[i] = p.blk_expert[s ? s - 1 : 0];
         }
-  const int ntn = p.N / TN, mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8;
-  int first = 0, tiles = MOE ? mtn1 * ntn : gridDim.x, mtn = mtn1 * S;
-  if (MOE && blockIdx.x >= tiles) return;
+  const int mtn1 = MOE ? *p.n_blocks : (p.M + 255) >> 8;
+  int heavy_m = mtn1 * S, light_m = 0;  // m-tiles
   // An expert's last segment may have 128 rows or fewer: light, half a tile.  All others come first,
   // so that the last round is of light ones (us before / now, 8 experts of 2048 x 4096: up at 1600
   // tokens of two 136 / 115, 3000 203 / 189, down at 8192 262 / 234, 16384 458 / 421).  Up to 9 rounds:
@@ -716,8 +727,8 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
   // all on (us without / with: up of 8 x 4096 x 4096 at 2400 tokens of two, 8 of 24 segments, 304 /
   // 383; 8 x 2048 x 6144 at 1300, 8 of 16, 165 / 189; 64 x 2048 x 1024 at 3000 of six, 59 of 123, 226 /
   // 281; 2 of 10 113 / 106, 200 / 198 and, of 4096 x 14336, 545 / 520), but where all tiles are one
-  // round (down of 8 x 2048 x 4096 at 1300, 8 of 16, 87 / 77; of 16 x 2048 x 2048 at 2400, 16 of 32,
-  // 58.5 / 51).  Nor where they are few, rounds are few and a tile is soon done (up at 2001, one of
+  // round and, cut, are not (down of 16 x 2048 x 2048 at 2400, 16 of 32, 58.5 / 51; of 8 x 2048 x 4096
+  // at 1000, 4 of 12, all of them cut 60, light ones half as high 63).  Nor where they are few, rounds are few and a tile is soon done (up at 2001, one of
   // 17, 155 / 158; but K = 4096, up of 8 x 4096 x 4096 at 1600, one of 16, 250 / 219, down at 4096,
   // three of 35, 268 / 254).  Over 160 such products the rule takes 0.7 % longer than the better of both.
   uint64_t pick[WORDS];
@@ -736,19 +747,39 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
               64 * i + lane > 0 && 64 * i + lane < mtn1 && half[i] >= p.n_assign &&
               expert[i] == last[i]));
       }
-      ordered = mtn1 * ntn <= 256 ||
-                (5 * apart <= mtn1 &&
-                 (p.K >= 4096 || 10 * (mtn1 - full) >= mtn1 || mtn1 * ntn >= 3 * 256));
-      light = ordered && blockIdx.x >= full * ntn;
-      first = light ? full * ntn : 0;
-      if (ordered) mtn = light ? mtn1 - full : full;
-      tiles = mtn * ntn;
+      ordered = mtn1 * ntn > 128 &&
+                (mtn1 * ntn <= 256 ||
+                 (5 * apart <= mtn1 &&
+                  (p.K >= 4096 || 10 * (mtn1 - full) >= mtn1 || mtn1 * ntn >= 3 * 256)));
+      if (ordered) heavy_m = full, light_m = mtn1 - full;
 #pragma unroll
-      for (int i = 0; i < WORDS; ++i)
-        pick[i] = light ? __builtin_amdgcn_ballot_w64(64 * i + lane < mtn1) & ~heavy[i] : heavy[i];
+      for (int i = 0; i < WORDS; ++i) pick[i] = heavy[i];
     }
   }
-  const int bid = xcd_remap(blockIdx.x - first, tiles);
+  // Wide tiles of a last round that they fill by half or less, with the light ones behind them, are cut
+  // in two: two narrow tiles on two CUs take 0.6 of a wide one's time, to the same bits.  us before / now:
+  // gated 28672 x 4096 at 600 / 1300 / 2001 rows 168 / 148, 253 / 235, 351 / 329, 16384 x 2048 at 1300 84.1
+  // / 77.6; plain 6144 x 4096 at 2600 139 / 126, 2048 x 2048 at 10000 79 / 69; 8 experts of 2048 x 4096, up
+  // at 1000 tokens of two 111 / 98, down at 1600 87.5 / 63.2, at 6000 190 / 163.
+  const int heavy_t = heavy_m * ntn, light_t = light_m * ntn;
+  const int cut = CUT ? cut_tiles(heavy_t, light_t) : 0;
+  int b = blockIdx.x, part = -1, bid, mtn = heavy_m;
+  if (b < heavy_t - cut) {
+    bid = xcd_remap(b, heavy_t - cut);
+  } else if (b < heavy_t + cut) {
+    b = xcd_remap(b - (heavy_t - cut), 2 * cut);
+    bid = heavy_t - cut + (b >> 1);
+    part = b & 1;
+  } else {
+    if (b >= heavy_t + cut + light_t) return;
+    bid = xcd_remap(b - heavy_t - cut, light_t);
+    light = true;
+    mtn = light_m;
+    if constexpr (MOE && SHAPE == WIDE)
+#pragma unroll
+      for (int i = 0; i < WORDS; ++i)
+        pick[i] = __builtin_amdgcn_ballot_w64(64 * i + lane < mtn1) & ~pick[i];
+  }
   const int64_t w_rows = gated(EPI) ? 2 * p.N : p.N;
   const int gm = w_rows * p.K > (1 << 26) ? 8 : 4;  // 128 MB of W
   const int per_group = gm * ntn;
@@ -775,6 +806,11 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
       return;
     }
   }
+  if constexpr (CUT)
+    if (part >= 0) {
+      tile<EPI, NARROW>(p, lds, mt, 2 * nt + part, ks);
+      return;
+    }
   tile<EPI, SHAPE>(p, lds, mt, nt, ks);
 }
 
@@ -853,7 +889,7 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
   PArgs a{out, (const bf16_t*)X, (const bf16_t*)W, M, N, K, ldo, ss_in, ss_in_n, inv_d, eps,
           ss_out, positions, cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache, slots, hq, hkv,
           block_size, 1, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, bias};
-  const dim3 grid((unsigned)blocks);
+  const dim3 grid((unsigned)(blocks + (narrow || !cuts(epi) ? 0 : cut_tiles((int)blocks, 0))));
 #define OMNIA_PGEMM(EPI)                                       \
   do {                                                         \
     if (narrow)                                                \
@@ -931,7 +967,7 @@ int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int
   PArgs a{out, (const bf16_t*)A, (const bf16_t*)W, max_blocks * 256, N, K, N, nullptr, 0, 0.f,
           0.f, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 1, sorted,
           blk_expert, n_blocks, route_w, topk, n_assign, e_lo, nullptr, alpha, limit};
-  const dim3 grid((unsigned)blocks);
+  const dim3 grid((unsigned)(blocks + (narrow ? 0 : 128)));  // (128: the most that are cut)
 #define OMNIA_PGEMM(EPI)                            \
   do {                                              \
     if (narrow)                                     \

@@ -346,6 +346,26 @@ def test_narrow_tile(gen, M, N, K):
             assert torch.equal(parts.half(), half)
 
 
+@pytest.mark.parametrize("M,tiles", [(255, 1), (512, 128), (257, 130), (700, 255), (250, 257),
+                                     (1000, 384), (900, 388), (2049, 513)])
+def test_tiles_cut_in_two(gen, M, tiles):
+    """Wide tiles of a last round of 128 or fewer are cut: the bits of the narrow tile, every element
+    once, for sizes of less than a round, of one and more, on both sides of half a round."""
+    K, mt = 256, -(-M // 256)
+    n = -(-tiles // mt)
+    x = _rand(M, K, gen=gen)
+    w = _rand(512 * n, K, std=0.05, gen=gen)
+    ss = torch.rand(M, 3, device=DEV, generator=gen) * K
+    for kw in (dict(epi=0, w=w[:256 * n]), dict(epi=0, w=w[:256 * n], ss_in=ss, inv_d=1.0 / K, eps=1e-5),
+               dict(epi=1, w=w[:256 * n]), dict(epi=1, w=w[:256 * n], gelu=True),
+               dict(epi=1, w=w[:256 * n], bias=torch.randn(256 * n, device=DEV, generator=gen))):
+        cols = kw["w"].shape[0] // (1 + kw["epi"])
+        out = torch.full((2, M + 1, cols), 7.0, dtype=torch.bfloat16, device=DEV)
+        for o, c in zip(out, (128, 256)):
+            ops.pgemm(x=x, out=o[:M], cols=c, **kw)
+        assert torch.equal(out[0], out[1]) and (out[:, M] == 7.0).all()
+
+
 def test_narrow_tile_refuses(gen):
     x, w = _rand(4, 128, gen=gen), _rand(192, 128, gen=gen)
     for call in (lambda: ops.pgemm(0, x, w, cols=128), lambda: ops.pgemm(0, x, w[:128], cols=64),
