@@ -19,16 +19,19 @@
 //     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
 //     depend on how many rows the step has;
 //   * rows of a weight are a power of two of bytes apart, or nearly, and blocks walk them in step, so
-//     at any time all would ask a few memory channels for their 128 bytes of every row.  Blocks of
-//     row-major weights of 64 MB and more therefore take the chunks of a power of two each in another
-//     order: by the number of its eight weight units, whatever the waves and rows, so that bits do not
-//     depend on them, and its bits reversed, so that blocks that run together are far apart.  us, in
-//     order / apart: gated 28672 x 4096 at 32 / 77 / 128 rows 45.2 / 36.8, 49.3 / 42.0, 54.4 / 49.4;
-//     gated 22016 x 4096 38.0 / 32.1, 42.7 / 39.6, 49.3 / 47.0; 4096 x 14336 25.8 / 20.6, 28.6 / 24.6,
-//     31.9 / 28.6; gated 16384 x 2048 15.8 / 12.6, 18.6 / 16.5, 22.9 / 21.7; 32768 x 2048 32.0 / 22.9,
-//     32.8 / 24.3, 34.6 / 28.6.  Smaller ones have little to gain and may lose (8192 x 2048 gated at 32
-//     9.6 / 9.2, 4096 x 4096 7.9 / 8.8), packed ones, 2 KB a chunk and unit, as well (28672 x 4096 40.3
-//     / 47.1);
+//     at any time all would ask a few memory channels for their 128 bytes of every row.  Where it is
+//     faster, blocks therefore take the chunks of a power of two each in another order: by the number
+//     of its eight weight units, whatever the waves and rows, so that bits do not depend on them, and
+//     its bits reversed, so that blocks that run together are far apart.  It is with row-major weights
+//     of 64 MB and more in walks of 32 chunks (rows, or their slices, of 4 KB), gated also of 64.  us, in
+//     order / apart, at 32 / 77 / 128 rows: gated 28672 x 4096 42.8 / 39.0, 47.4 / 44.9, 55.1 / 53.4; gated
+//     16384 x 4096 28.9 / 24.6, 33.9 / 31.0, 42.4 / 41.5; gated 16384 x 2048 17.3 / 14.5, 20.5 / 18.6,
+//     24.1 / 23.1; 32768 x 2048 30.8 / 23.0, 32.6 / 24.8, 34.9 / 29.0; 131072 x 2048 103 / 88, 117 / 103,
+//     144 / 125; 4096 x 14336 in 7 slices 25.9 / 20.9, 28.8 / 25.2, 32.8 / 29.7; 8192 x 8192 in 4 33.0 / 25.0,
+//     35.3 / 27.1, 38.1 / 35.4.  Others lose or gain nothing (at 32 rows, plain 12288 x 4096 22.7 / 35.4,
+//     28672 x 4096 43.0 / 62.4, 128256 x 4096 181 / 199, gated 8192 x 8192 30.9 / 43.3, 8192 x 4096 in 4
+//     slices 13.9 / 15.7, 5120 x 13824 in 6 25.7 / 25.5), smaller ones may (8192 x 2048 gated 9.6 / 9.2,
+//     4096 x 4096 7.9 / 8.8), and packed ones, 2 KB a chunk and unit (28672 x 4096 40.3 / 47.1);
 //   * a ring of NS stages, of which NS - 1 stay in flight across the one raw barrier of a stage.
 //     Past the end the loads go to one line, so that every wait counts the same number of loads.
 //     The DMA is written as asm: hipcc, not knowing which stage a fragment read belongs to,
@@ -136,7 +139,8 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(const bf16_t* x, cons
   const int c0 = split * nch / p.S, n = (split + 1) * nch / p.S - c0;  // 64-k chunks: stages
   // stage s of this block is chunk s ^ turn of its slice, by its weights' place alone
   int turn = 0;
-  if (!PK && !grouped(EPI) && (int64_t)p.N * K >= (paired(EPI) ? 1 << 24 : 1 << 25))
+  if (!PK && !grouped(EPI) && (n == 32 || (paired(EPI) && n == 64)) &&
+      (int64_t)p.N * K >= (paired(EPI) ? 1 << 24 : 1 << 25))
     turn = (int)(__builtin_bitreverse32(tile * WN >> 3) >> 26) & ((n & -n) - 1);
 
   // this wave's weights: row-major, rows 8h.. of the unit and 16-byte chunk lane & 7 of each;
