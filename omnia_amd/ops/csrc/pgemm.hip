@@ -10,7 +10,13 @@
 //     128 x 64 read 224; the products go in a snake, each keeps an operand of the one before;
 //   * a K-tile is four 16 KB half-tiles (A0 A1: rows 0-127, 128-255 of X, B0 B1: of W), filled
 //     by LDS-DMA (16 bytes a lane; chunk c of row r at c ^ (r & 7), so that fragment reads have
-//     no bank conflicts), in a ring of ten: two K-tiles and A of a third.  Two barriers a K-tile:
+//     no bank conflicts), in a ring of ten: two K-tiles and B of a third, as W often comes from HBM
+//     and x from the L2 of the XCD (us with A / B of the third: gated 28672 x 4096 at 512 rows 98 /
+//     95.6, at 2001 329 / 324, at 2560 in a model 444 / 425, 16384 x 2048 at 16384 744 / 740, plain
+//     4096 x 14336 in 8 slices at 512 49.3 / 47.7, experts' down of 8 x 2048 x 4096 at 2001 tokens
+//     83 / 79, up at 16384 882 / 876).  EPI 2 and 3, of the dense models' large prompts, A of a third
+//     (in a model, us a product, A / B: EPI 2 at 2560 rows 180 / 182, 8192 408 / 415, 16384 811 / 824,
+//     EPI 3 103 / 104, 307 / 309, 608 / 611).  Two barriers a K-tile:
 //     one once every wave has read it (its slots are asked for again), one once the next has
 //     landed, 40 products later; up to 96 KB are in flight, waits are counted;
 //   * fragments of 32 k are read half a K-tile ahead, one read every other product, and the 16
@@ -304,13 +310,16 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     }
   }
 
-  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10 (narrow, flat: (3t + h) mod 9)
+  // ---- the ring: half h of K-tile t lies in slot (4t + h) mod 10 (narrow, flat: (3t + h) mod 9),
+  // the halves first of which a third is held
+  constexpr bool W_AHEAD = SHAPE == WIDE && EPI != 2 && EPI != 3;
+  constexpr int SLOT_A = W_AHEAD ? NB * HALF : 0, SLOT_B = W_AHEAD ? 0 : NA * HALF;
   const uint32_t dst0 =
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)lds + 32 * w * 128;
   auto next = [&](int s) __attribute__((always_inline)) {  // a K-tile on
     return s + KT * HALF >= RING ? s + KT * HALF - RING : s + KT * HALF;
   };
-  int da = 0, db = NA * HALF, ka = 0, kb = 0;  // slots and K-tiles to ask for next
+  int da = SLOT_A, db = SLOT_B, ka = 0, kb = 0;  // slots and K-tiles to ask for next
   uint32_t qa = 0, qb = 0;                    // of the DMAs under way: LDS address, sources
   const char *pa[2], *pb[2];
   int64_t koff = 0;
@@ -338,13 +347,15 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   auto dma_b = [&](int d) __attribute__((always_inline)) {
     dma16(vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb, (d >> 2) * HALF * 2 + (d & 3) * 1024);
   };
-  // K-tiles 0 and 1, and A of 2 (narrow, flat: all of it)
+  // K-tiles 0 and 1, and A or B of 2 (narrow, flat: all of it)
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
-    set_a();
+    if (t < 2 || !W_AHEAD) {
+      set_a();
 #pragma unroll
-    for (int d = 0; d < 4 * NA; ++d) dma_a(d);
-    if (t < 2 || SHAPE != WIDE) {
+      for (int d = 0; d < 4 * NA; ++d) dma_a(d);
+    }
+    if (t < 2 || W_AHEAD || SHAPE != WIDE) {
       set_b();
 #pragma unroll
       for (int d = 0; d < 4 * NB; ++d) dma_b(d);
@@ -354,7 +365,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   // ---- fragments: A rows wr*128 + 16m + fr; B's columns wc*WCOL + 16n + fr, gated those of the
   // gate's part for n < NG and of the up's, GU columns on, for the rest; k chunk 4s + fq of step s
   const bf16_t *fa[2], *fb[2];
-  int ra = wr * HALF, rb = NA * HALF;
+  int ra = SLOT_A + wr * HALF, rb = SLOT_B;
   auto set_r = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -398,7 +409,8 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     const int m = j / NF, n = (m & 1) ? NF - 1 - j % NF : j % NF;
     if (first) {
       mfma16_first(acc[m][n], fw[set][n], fx[set][m]);
-      if (d >= 0) dma_b(d);
+      if (d >= 8) dma_a(d - 8);
+      else if (d >= 0) dma_b(d);
     } else if (d < 0) {
       mfma16(acc[m][n], fw[set][n], fx[set][m]);
     } else if (d < 8) {
@@ -413,18 +425,19 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     }
   };
   // Step s of K-tile t: 8 NF products of 32 k.  FREE: every wave has read the K-tile (its last
-  // fragments are asked for by product 30 of step 0, NF 4: 22); its slots take B of t + 2, then,
-  // behind LAND, A of t + 3 (NF 4: B and A of t + 3).  LAND: the loads younger than K-tile t + 1
-  // may be under way (NF 8: A and B of t + 2; NF 4: all of t + 2, 5 of t + 3), K-tile t + 1 is
+  // fragments are asked for by product 30 of step 0, NF 4: 22); its slots take A of t + 2, then,
+  // behind LAND, B of t + 3 (not W_AHEAD: B and A; NF 4: B and A of t + 3).  LAND: the loads younger than K-tile t + 1
+  // may be under way (NF 8: B and A of t + 2; NF 4: all of t + 2, 5 of t + 3), K-tile t + 1 is
   // there, and its first fragments are read.
   constexpr int P = 8 * NF, FREE = NF == 8 ? 36 : 26, LAND = NF == 8 ? 12 : 6;
   constexpr int YOUNGER = NF == 8 ? 16 : 17;
   // the DMA behind product j: B's are 0 to 4 NB - 1, A's from 8 on; -1: none
   auto dma_at = [](int s, int j) constexpr {
     if (NF == 8) {
-      if (s == 0 && j >= FREE && (j - FREE) % 3 == 0 && (j - FREE) / 3 < 8) return (j - FREE) / 3;
+      if (s == 0 && j >= FREE && (j - FREE) % 3 == 0 && (j - FREE) / 3 < 8)
+        return (W_AHEAD ? 8 : 0) + (j - FREE) / 3;
       if (s == 1 && j > LAND && (j - LAND) % 6 == 3 && (j - LAND) / 6 < 8)
-        return 8 + (j - LAND) / 6;
+        return (W_AHEAD ? 0 : 8) + (j - LAND) / 6;
     } else {
       int q = -1;
       if (s == 0 && j >= FREE && (j - FREE) % 2 == 0) q = (j - FREE) / 2;  // 0 to 2
@@ -461,9 +474,9 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
       if (s == 0 && !(j & 1) && j < 2 * (8 + NF)) read(1, 1, j >> 1);
       if (s == 1 && !(j & 1) && j >= LAND && j < LAND + 2 * (8 + NF)) read(0, 0, (j - LAND) >> 1);
       // addresses of what comes next, between products that hide them
-      if (s == 0 && j == FREE - 3) set_b();
+      if (s == 0 && j == FREE - 3) W_AHEAD ? set_a() : set_b();
       if (s == 0 && j == (NF == 8 ? 48 : 29)) set_r();
-      if (s == 1 && j == 2) set_a();
+      if (s == 1 && j == 2) W_AHEAD ? set_b() : set_a();
       __builtin_amdgcn_sched_barrier(0);
     }
   };
