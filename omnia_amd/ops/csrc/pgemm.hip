@@ -236,10 +236,10 @@ __device__ __forceinline__ float row_scale(const PArgs& p, int m0, int Mt, int i
   return __builtin_amdgcn_rsqf(t * p.inv_d + p.eps);
 }
 
-// Tile (mt, nt) of K-slice ks
+// Tile (mt, nt) of K-slice ks; step t is K-tile t ^ turn
 template <int EPI, int SHAPE>
 __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, int mt, int nt,
-                                     int ks) {
+                                     int ks, int turn) {
   constexpr int NF = SHAPE == WIDE ? 8 : 4;  // 16-column fragments of a wave
   constexpr int KT = SHAPE == WIDE ? 4 : 3;  // half-tiles of a K-tile: NA of x, then NB of W
   constexpr int NA = SHAPE == FLAT ? 1 : 2, NB = KT - NA, RING = ring(SHAPE);
@@ -326,7 +326,7 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   // past the end the last K-tile is loaded again, into slots that nothing reads
   auto set_a = [&]() __attribute__((always_inline)) {
     qa = dst0 + da * 2;
-    koff = (int64_t)ka * (BK * 2);
+    koff = (int64_t)(gathered(EPI) ? ka ^ turn : ka) * (BK * 2);
     pa[0] = base[0] + koff;
     if constexpr (NA == 2) pa[1] = base[1] + koff;
     ka = ka + 1 < nk ? ka + 1 : nk - 1;
@@ -334,8 +334,9 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   };
   auto set_b = [&]() __attribute__((always_inline)) {
     qb = dst0 + db * 2;
-    pb[0] = base[2] + (int64_t)kb * (BK * 2);
-    if constexpr (NB == 2) pb[1] = base[3] + (int64_t)kb * (BK * 2);
+    const int64_t off = (int64_t)(gathered(EPI) ? kb ^ turn : kb) * (BK * 2);
+    pb[0] = base[2] + off;
+    if constexpr (NB == 2) pb[1] = base[3] + off;
     kb = kb + 1 < nk ? kb + 1 : nk - 1;
     db = next(db);
   };
@@ -814,17 +815,33 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
       }
       mt = seg;
     }
+  }
+  // Experts' rows of 4 KB of W, of which all blocks would ask for the same 128 bytes at a time, and so
+  // for a few memory channels: eight column tiles, whose blocks share x in an XCD, walk K in an order of
+  // their own, with the bits of their number reversed, so that neighbours are far apart.  While the
+  // tiles are some rounds only; then blocks are apart by themselves.  us, up products in order / apart: 8
+  // experts of 2048 x 4096 at 600 / 1000 / 2001 / 4000 / 16384 tokens of two 83 / 68, 107 / 92, 168 / 143,
+  // 248 / 249, 907 / 917; 16 of 2048 x 2048 at 2400 140 / 121; 64 of 2048 x 1024 at 3000 of six 229 / 230.
+  // Rows of other lengths lose or gain nothing (8 of 4096 x 14336 at 1001 508 / 532, down of
+  // 2048 x 4096 at 2001 79 / 78).
+  int turn = 0;
+  if constexpr (gathered(EPI)) {
+    constexpr int PART = SHAPE == NARROW ? 2 : 1;  // of a wide column tile
+    const int octets = (ntn / PART + 7) >> 3;
+    if (p.K == 32 * BK && mtn1 * ntn <= 3 * 256 * PART)
+      turn = (int)(__builtin_bitreverse32(nt / PART / 8 + octets * (p.blk_expert[mt] - p.e_lo)) >> 27);
+  }
+  if constexpr (MOE && SHAPE == WIDE)
     if (light) {
-      tile<EPI, FLAT>(p, lds, mt, nt, 0);
+      tile<EPI, FLAT>(p, lds, mt, nt, 0, turn);
       return;
     }
-  }
   if constexpr (CUT)
     if (part >= 0) {
-      tile<EPI, NARROW>(p, lds, mt, 2 * nt + part, ks);
+      tile<EPI, NARROW>(p, lds, mt, 2 * nt + part, ks, turn);
       return;
     }
-  tile<EPI, SHAPE>(p, lds, mt, nt, ks);
+  tile<EPI, SHAPE>(p, lds, mt, nt, ks, turn);
 }
 
 template <int EPI, int SHAPE>

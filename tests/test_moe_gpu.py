@@ -311,6 +311,39 @@ def test_segments_of_few_rows(E, rows):
             torch.testing.assert_close(y[0][of].float(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("rows", [[300, 5, 700], [0, 1, 256], [5376] * 4, [5632] * 4])
+def test_column_tiles_that_walk_k_in_orders_of_their_own(rows):
+    """Experts of 4 KB rows, 9 wide column tiles (two octets): tiles wide, narrow, cut in two and of
+    half height take the K-tiles in the same order, each once; 756 tiles are the last to, 792 do not."""
+    kk, dev, E, d, I = ops.kernels(), "cuda", len(rows), 2048, 1152
+    n = sum(rows)
+    ids = torch.arange(E).repeat_interleave(torch.tensor(rows)).int().view(n, 1).to(dev)
+    x = torch.randn(n, d, device=dev).to(torch.bfloat16)
+    up = (torch.randn(E, 2 * I, d, device=dev) * 0.02).to(torch.bfloat16)
+    wts = torch.rand(n, device=dev)
+    mb = kk.moe_max_blocks(n, E, 256)
+    order = torch.empty(mb * 256, dtype=torch.int32, device=dev)
+    blk = torch.empty(mb, dtype=torch.int32, device=dev)
+    nb = torch.empty(1, dtype=torch.int32, device=dev)
+    kk.moe_align(order, blk, nb, ids, E, 0, E)
+    live = (order < n) & (torch.arange(mb * 256, device=dev) < nb * 256)
+    for mode, w, rw in ((0, up, None), (2, up, wts), (3, up[:, :I - 128].contiguous(), None)):
+        out = w.shape[1] // (1 if mode == 3 else 2)
+        acts = [torch.zeros(mb * 256, out, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+        for act, cols in zip(acts, (256, 128)):
+            kk.pgemm_moe(mode, act, x, w, order, blk, nb, rw, 1, n, 0, 1.702, 7.0, cols)
+        assert torch.equal(*(a[live] for a in acts))
+        if mode:
+            continue
+        for e in (e for e in range(E) if rows[e]):
+            of = ids.view(-1) == e
+            a, b = (x[of][:64].float() @ up[e].float().t()).split(I, 1)
+            got = torch.empty(n, I, device=dev)
+            got[order[live].long()] = acts[0][live].float()
+            torch.testing.assert_close(got[of][:64], torch.nn.functional.silu(a) * b,
+                                       atol=2e-2, rtol=2e-2)
+
+
 def test_segments_of_few_rows_take_no_longer_than_full_ones():
     """Apart from their expert's others, light segments read its weights once more, so many of them
     stay where they are: 8 light segments of 24 against 24 full ones (1.26 times as long apart)."""
