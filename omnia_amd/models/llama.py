@@ -216,7 +216,9 @@ class LlamaModel(Projections):
     # ones ~6.0 TB/s; inside the full kernel, next to the x re-reads and the
     # MFMAs, the gain is 0-3 % per projection (profiles/r5/decode_gemm/); end to
     # end the closed-loop bench gains +0.8 % tok/s and -2 % TPOT, 3 of 3
-    # interleaved pairs (profiles/r6/bench/tgemm_pack/).  Only batches past the
+    # interleaved pairs (profiles/r6/bench/tgemm_pack/, of all projections; gate_up
+    # and down have since gone on to the prefill tile, which reads row-major weights:
+    # 256 rows of an 8B model, 577 keys each, 8824 / 8683 us).  Only batches past the
     # few-row kernels (193 to 256 rows) run it.  The copy is built before the KV
     # pool is sized, by default whenever it and the few-row copies fit
     # pack_budget_frac of HBM (70B TP=1 and MoE models: never);
@@ -286,7 +288,7 @@ class LlamaModel(Projections):
             if a is None:
                 a = ops.linear_silu(h, layer["gate_up"])  # SwiGLU fused into decode GEMMs
         elif cfg[1] == ops.PGEMM_SPLIT and cfg[2] == 1:
-            a = ops.pgemm(1, h, layer["gate_up"])  # mid-size step: the unsplit fused tile
+            a = ops.pgemm(1, h, layer["gate_up"])  # the unsplit fused tile
         else:
             nw, nwaves, S = cfg
             if S == 1 and nwaves != ops.PGEMM_SPLIT:

@@ -228,7 +228,7 @@ WGEMM_MAX_M = 256
 _wgemm_table: dict | None = None
 _wgemm_on = os.environ.get("OMNIA_WGEMM", "1") != "0"
 WGEMM_BUCKETS = (16, 32, 64, 128, 192, 256)
-PGEMM_SPLIT = -64  # table nwaves code: pgemm 256x256 split-K tile, fp16 slabs (or ``out``'s fp32)
+PGEMM_SPLIT = -64  # table nwaves code: pgemm's tile, in slices fp16 slabs (or ``out``'s fp32)
 
 
 def wgemm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | None:
@@ -236,7 +236,9 @@ def wgemm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | No
     (nwaves == 0 selects the wide-batch 32x32x16 kernel, wgemm_wide.hip, with nw
     32-column tiles per wave; nwaves < 0 the full-batch tile kernel, tgemm.hip,
     with nw weight rows per block and non-temporal weight loads when -2;
-    nwaves == PGEMM_SPLIT the 256x256 split-K tile, pgemm.hip EPI 4, 11),
+    nwaves == PGEMM_SPLIT the prefill tile with nw columns, pgemm.hip, in slices (EPI 4, 11) or, one
+    of a gate_up, whole (EPI 1): us at 256 rows, weights from HBM, tgemm on packed copies / so: gated 28672 x 4096
+    71.7 / 67.1, 4096 x 14336 39.8 / 35.8, 8192 x 28672 126 / 118),
     or None to keep the library / gemm.hip path.  ``mode`` 0 = plain projection
     (its split-K slabs are reduced by the consumer kernel), 1 = gate_up + SwiGLU.
     Measured dispatch: ``ops/tuned/wgemm_mi355x.json`` (scripts/wgemm_sweep.py +
@@ -297,7 +299,7 @@ def wgemm(mode: int, x: torch.Tensor, w: torch.Tensor, splits: int = 1, nw: int 
     mode 0: bf16 ``x @ w.T``; mode 1: bf16 ``silu(x Wg^T) * (x Wu^T)`` with
     ``w = [Wg; Wu]``; mode 2: fp32 split-K partial slabs ``[splits, M, N]`` whose
     sum is ``x @ w.T`` (reduced by the consumer kernel)."""
-    if nwaves == PGEMM_SPLIT:  # table code for the 256x256 split-K tile
+    if nwaves == PGEMM_SPLIT:  # table code for the prefill tile in slices
         if mode not in (2, 3):
             raise ValueError("the pgemm split-K table entry produces slabs (mode 2/3)")
         return pgemm_splitk(x, w, splits, out, cols=nw)

@@ -144,17 +144,25 @@ __device__ __forceinline__ void mfma16(float4v& acc, short8 a, short8 b) {
 __device__ __forceinline__ void mfma16_first(float4v& acc, short8 a, short8 b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
 }
-// ... and behind it a DMA of 16 bytes a lane to LDS address ``at`` + OFF (lane-linear)
+// ... and behind it a DMA of 16 bytes a lane to LDS address ``at`` + OFF (lane-linear); ONCE: of what
+// no later block reads
+#define OMNIA_PRODUCT_DMA(HINT)                                         \
+  asm volatile(                                                         \
+      "s_add_u32 m0, %5, %6\n\t"                                        \
+      "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\t"                     \
+      "global_load_lds_dwordx4 %3, %4" HINT                             \
+      : "+a"(acc)                                                       \
+      : "v"(a), "v"(b), "v"(voff), "s"(base), "s"(at), "i"(off)         \
+      : "memory", "scc")
+template <bool ONCE = false>
 __device__ __forceinline__ void mfma16_dma(float4v& acc, short8 a, short8 b, uint32_t voff,
                                            const void* base, uint32_t at, int off) {
-  asm volatile(
-      "s_add_u32 m0, %5, %6\n\t"
-      "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\t"
-      "global_load_lds_dwordx4 %3, %4"
-      : "+a"(acc)
-      : "v"(a), "v"(b), "v"(voff), "s"(base), "s"(at), "i"(off)
-      : "memory", "scc");
+  if constexpr (ONCE)
+    OMNIA_PRODUCT_DMA(" nt");
+  else
+    OMNIA_PRODUCT_DMA("");
 }
+#undef OMNIA_PRODUCT_DMA
 __device__ __forceinline__ void mfma16_dma(float4v& acc, short8 a, short8 b, const void* src,
                                            uint32_t at, int off) {
   asm volatile(
@@ -236,8 +244,8 @@ __device__ __forceinline__ float row_scale(const PArgs& p, int m0, int Mt, int i
   return __builtin_amdgcn_rsqf(t * p.inv_d + p.eps);
 }
 
-// Tile (mt, nt) of K-slice ks; step t is K-tile t ^ turn
-template <int EPI, int SHAPE>
+// Tile (mt, nt) of K-slice ks; step t is K-tile t ^ turn; ONCE: W is not read by later tiles
+template <int EPI, int SHAPE, bool ONCE = false>
 __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, int mt, int nt,
                                      int ks, int turn) {
   constexpr int NF = SHAPE == WIDE ? 8 : 4;  // 16-column fragments of a wave
@@ -415,8 +423,8 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
     } else if (d < 0) {
       mfma16(acc[m][n], fw[set][n], fx[set][m]);
     } else if (d < 8) {
-      mfma16_dma(acc[m][n], fw[set][n], fx[set][m], vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb,
-                 (d >> 2) * HALF * 2 + (d & 3) * 1024);
+      mfma16_dma<ONCE>(acc[m][n], fw[set][n], fx[set][m], vo[2 + (d >> 2)][d & 3], pb[d >> 2], qb,
+                       (d >> 2) * HALF * 2 + (d & 3) * 1024);
     } else {
       const int h = (d >> 2) - 2, i = d & 3, off = h * HALF * 2 + i * 1024;
       if constexpr (GATHER)
@@ -699,8 +707,8 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
 }
 
 // What the first loads need comes as arguments of their own: 14 words that are in registers when a
-// wave starts (a struct is loaded from memory).
-template <int EPI, int SHAPE>
+// wave starts (a struct is loaded from memory).  ONCE: W does not push x out of L2.
+template <int EPI, int SHAPE, bool ONCE>
 __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf16_t* W, int M,
                                                        int N, int K, int splits,
                                                        const int* n_blocks, const int* blk_expert,
@@ -841,13 +849,25 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
       tile<EPI, NARROW>(p, lds, mt, 2 * nt + part, ks, turn);
       return;
     }
-  tile<EPI, SHAPE>(p, lds, mt, nt, ks, turn);
+  tile<EPI, SHAPE, ONCE>(p, lds, mt, nt, ks, turn);
 }
 
-template <int EPI, int SHAPE>
+template <int EPI, int SHAPE, bool ONCE = false>
 void launch(const PArgs& a, dim3 grid, hipStream_t s) {
-  pgemm_kernel<EPI, SHAPE><<<grid, 256, 0, s>>>(a.X, a.W, a.M, a.N, a.K, a.splits, a.n_blocks,
-                                                a.blk_expert, a.sorted, a);
+  pgemm_kernel<EPI, SHAPE, ONCE><<<grid, 256, 0, s>>>(a.X, a.W, a.M, a.N, a.K, a.splits, a.n_blocks,
+                                                      a.blk_expert, a.sorted, a);
+}
+// Narrow tiles of up to two m-tiles, which read W together, ask for it past the caches' order of use:
+// us before / now, gated 28672 x 4096 at 224 / 256 rows 71.5 / 67.1, 70.7 / 67.1, 16384 x 2048 at 300 31.6 /
+// 30.6, 4096 x 14336 in 8 slices at 256 37.3 / 35.8, 2048 x 8192 at 400 23.4 / 22.1.  More rows read it at
+// different times (plain 4096 x 2048 at 1999 31.7 / 33.6), and so do more rounds (the wide tile, gated
+// 28672 x 4096 at 8192 1248 / 1288).
+template <int EPI>
+void launch_narrow(const PArgs& a, dim3 grid, hipStream_t s) {
+  if (a.M <= 512)
+    launch<EPI, NARROW, true>(a, grid, s);
+  else
+    launch<EPI, NARROW>(a, grid, s);
 }
 
 // one workgroup (256 threads) per row: ss[r] = sum(x[r]^2) (layer-0 input of the
@@ -923,7 +943,7 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
 #define OMNIA_PGEMM(EPI)                                       \
   do {                                                         \
     if (narrow)                                                \
-      launch<EPI, NARROW>(a, grid, s);            \
+      launch_narrow<EPI>(a, grid, s);             \
     else                                                       \
       launch<EPI, WIDE>(a, grid, s);            \
     return (int)hipGetLastError();                             \
@@ -959,11 +979,11 @@ int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, 
           nullptr, 0, 0, 0};
   const dim3 grid((unsigned)blocks);
   if (f32 && tn == 128)
-    launch<11, NARROW>(a, grid, s);
+    launch_narrow<11>(a, grid, s);
   else if (f32)
     launch<11, WIDE>(a, grid, s);
   else if (tn == 128)
-    launch<4, NARROW>(a, grid, s);
+    launch_narrow<4>(a, grid, s);
   else
     launch<4, WIDE>(a, grid, s);
   return (int)hipGetLastError();
