@@ -16,6 +16,7 @@ import torch.nn.functional as F
 from .. import ops
 from ..ops import mixers as mops
 from .layers import GQA_WIDTHS
+from .projection import Projections
 
 
 def _pad2(w: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
@@ -145,11 +146,20 @@ class LatentAttention(Mixer):
             o = mops.latent_attend(qa, pages, fb.block_tables, fb.q_start_loc, positions, s)
             return mops.latent_expand(o, w["uv"], s, gate, out)
         mops.latent_rotate(q, s, positions, self.table)
+        # Many keys: their rows, zeros behind them, are whole column tiles of the prefill GEMM, also where
+        # they are the weight (us, library / tile, of 2048 x 512: keys at 2112 / 6016 / 16384 / 16640 rows
+        # 17.0 / 12.1, 33.5 / 19.6, 41.9 / 41.5, 75.9 / 46.5, values 16.7 / 12.3, 34.0 / 19.6, 43.5 / 42.5,
+        # 75.2 / 47.2; at 4416 17.5 / 19.7 and 24.7 / 18.9)
+        uk, uv, rows = w["uk"], w["uv"].view(s.heads * s.v_pad, s.latent_pad), fb.kv_rows
+        m = self.model
+        tiles = isinstance(m, Projections) and m._pgemm_ok(rows, s.latent_pad, uk.shape[0], False)
+        if tiles:
+            rows = -(-rows // 256) * 256
         c, kr = mops.latent_gather(pages, fb.block_tables, fb.kv_start, fb.kv_first, fb.seq_lens,
-                                   fb.kv_rows, s)
-        kx = ops.linear(c, w["uk"])
+                                   rows, s)
+        kx = ops.pgemm(0, c, uk) if tiles else ops.linear(c, uk)
         # values transposed ([head dims, keys]): the product with swapped operands
-        vt = ops.linear(w["uv"].view(s.heads * s.v_pad, s.latent_pad), c)
+        vt = ops.pgemm(0, uv, c) if tiles else ops.linear(uv, c)
         return mops.latent_prefill(q, kx, kr, vt, fb, s, gate, out)
 
     def mix(self, w: dict, x: torch.Tensor, fb, cache) -> torch.Tensor:

@@ -341,6 +341,38 @@ def test_latent_attention(size, how, run):
         assert rel(project_out(y, w), want(h)) < LIMIT[run[1]]
 
 
+@GPU
+@pytest.mark.parametrize("size", [LATENTS[3], LATENTS[4], dict(LATENTS[3], window=0)],
+                         ids=lambda s: f"c{s['kv_rank']}w{s['window']}")
+@pytest.mark.parametrize("lens", [[256, 200], [64], [150, 36, 67, 1], [513]])
+def test_latent_attention_on_whole_tiles_of_keys(size, lens, monkeypatch):
+    """Keys and values expanded on the prefill tile, their rows made whole column tiles with zeros:
+    row counts that are and are not, first portions and ones behind a past."""
+    from omnia_amd.models.projection import Projections
+
+    class Served(Projections, Stub):
+        tp, _min_rows = 1, 1
+
+    seen, pgemm = [], ops.pgemm
+    monkeypatch.setattr(ops, "pgemm", lambda epi, x, w: seen.append((len(x), len(w))) or
+                        pgemm(epi, x, w))
+    run = "cuda", torch.bfloat16
+    spec = sc.latent(**size)["mixer"]
+    mixer, w, W, want = mixer_case("latent_attention", spec, 40, run, 13)
+    mixer.model = Served("cuda", torch.bfloat16, 1e-5)
+    mixer.model.project = lambda x, w, is_decode: torch.nn.functional.linear(x, w)
+    g = gen(14)
+    hs = [rnd(n, 40, g=g) for n in lens]
+    steps = [[(s, n) for s, n in enumerate(lens)]] if lens[0] > 256 else \
+        [[(s, n // 2) for s, n in enumerate(lens) if n > 1],
+         [(s, n - n // 2 if n > 1 else 1) for s, n in enumerate(lens)]]
+    for h, y in zip(hs, run_mixer(mixer, w, hs, steps, 32, 17)):
+        assert rel(project_out(y, w), want(h)) < LIMIT[torch.bfloat16]
+    assert len(seen) == 2 * len(steps)
+    assert all(a % 256 == 0 == c % 256 and (b, c) == (len(w["uk"]), a)
+               for (a, b), (_, c) in zip(seen[::2], seen[1::2]))
+
+
 # ------------------------------------------------- one key that stands out
 def attended(q, c, kr, W_uk, W_uv, spec, gate, visible):
     """Plain attention of one query over the keys `visible`."""
