@@ -152,14 +152,15 @@ class LatentAttention(Mixer):
         # 75.2 / 47.2; at 4416 17.5 / 19.7 and 24.7 / 18.9)
         uk, uv, rows = w["uk"], w["uv"].view(s.heads * s.v_pad, s.latent_pad), fb.kv_rows
         m = self.model
-        tiles = isinstance(m, Projections) and m._pgemm_ok(rows, s.latent_pad, uk.shape[0], False)
-        if tiles:
-            rows = -(-rows // 256) * 256
+        own = isinstance(m, Projections) and m._pgemm_covers(s.latent_pad, uk.shape[0], False)
+        tiles = own and m._pgemm_ok(rows, s.latent_pad, uk.shape[0], False)
+        if own:  # fewer, those of tiles of 128 x 128
+            rows = -(-rows // 256) * 256 if tiles else -(-rows // 128) * 128
         c, kr = mops.latent_gather(pages, fb.block_tables, fb.kv_start, fb.kv_first, fb.seq_lens,
                                    rows, s)
-        kx = ops.pgemm(0, c, uk) if tiles else ops.linear(c, uk)
+        kx = ops.pgemm(0, c, uk) if tiles else ops.linear(c, uk, tiles=own)
         # values transposed ([head dims, keys]): the product with swapped operands
-        vt = ops.pgemm(0, uv, c) if tiles else ops.linear(uv, c)
+        vt = ops.pgemm(0, uv, c) if tiles else ops.linear(uv, c, tiles=own)
         return mops.latent_prefill(q, kx, kr, vt, fb, s, gate, out)
 
     def mix(self, w: dict, x: torch.Tensor, fb, cache) -> torch.Tensor:

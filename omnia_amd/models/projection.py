@@ -245,8 +245,8 @@ class Projections:
 
     def _mid(self, x: torch.Tensor, w: torch.Tensor, is_decode: bool, slabs: bool):
         """More rows than the few-row kernels take and fewer than ``_pgemm_ok`` asks for: the
-        prefill tile where it fills the chip, whole or in slices of K (fp32 :class:`Parts`), else
-        the library."""
+        prefill tile where it fills the chip, whole or in slices of K (fp32 :class:`Parts`), tiles of
+        128 x 128 where those do, else the library."""
         M, K = x.shape
         if M > ops.PANEL_MAX_M and self.tp == 1 and ops._on_grid(x, w) and \
                 self._pgemm_covers(K, w.shape[0], is_decode):
@@ -258,6 +258,7 @@ class Projections:
             if S:
                 out = torch.empty(S, M, w.shape[0], dtype=torch.float32, device=x.device)
                 return Parts(ops.pgemm_splitk(x, w, S, out, cols=128))
+            return ops.linear(x, w, tiles=True)
         return ops.linear(x, w)
 
     _min_rows = int(os.environ.get("OMNIA_PGEMM_MIN_ROWS", "2049"))  # this forward's threshold (mixed steps: the higher one)

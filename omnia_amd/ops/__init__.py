@@ -522,6 +522,31 @@ def plain_tile_fills(M: int, w: torch.Tensor) -> bool:
         tile_cols(M, R) == 128 and _tile_rounds(M, R, 128) == 1 and w.is_contiguous() and _on_grid(w)
 
 
+def small_tile_pays(M: int, w: torch.Tensor) -> bool:
+    """Whether :func:`pgemm_small` covers ``w`` and beats the library for more rows than the panel kernel
+    takes: one round of its tiles over 256 CUs, .55 of their work useful, or three quarters where K is
+    long (useful part, us here / library: 2048 x 2048 at 999 rows .49 17.1 / 16.1, 4096 x 2048 at 512 .50
+    21.0 / 17.0; 2048 x 2048 at 1300 .63 17.7 / 21.7,
+    2001 .98 19.0 / 21.7; 4608 x 2048 at 508 .56 18.4 / 21.2; 3072 x 1024 at 999 .73 11.6 / 14.3; 2048 x
+    512 at 2048 1.0 8.9 / 11.1; 4096 x 4096 at 700 .68 34.3 / 32.6, 999 .98 38.7 / 40.9; 2560 x 4096 at
+    1316 .80 34.4 / 42.0; 5888 x 6144 at 512 .72 62.3 / 55.0, 3712 x 6144 at 897 .79 50.0 / 58.5).  Over 60
+    such sizes the library takes 1.03 to 1.45 as long."""
+    if M <= PANEL_MAX_M or w.dim() != 2:
+        return False
+    R, K = w.shape
+    return R % 128 == 0 and K % 64 == 0 and K <= 6144 and -(-M // 128) * (R // 128) <= 256 and \
+        M * R > (0.55 if K <= 2048 else 0.75) * 256 * 128 * 128 and w.is_contiguous() and _on_grid(w)
+
+
+def pgemm_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x @ w.T`` on MFMA tiles of 128 x 128 (``csrc/pgemm.hip``): whole ones of ``w``, K of whole 64."""
+    if not x.is_cuda:
+        return (x.float() @ w.float().t()).to(x.dtype)
+    out = x.new_empty(x.shape[0], w.shape[0])
+    kernels().pgemm_small(out, x.contiguous(), w)
+    return out
+
+
 @functools.lru_cache(maxsize=8192)
 def tile_slices(M: int, R: int, K: int) -> int:
     """K slices in which :func:`pgemm_splitk`'s narrow tile runs ``M`` rows of a weight [R, K] into
@@ -826,12 +851,19 @@ def splitk_reduce(parts: torch.Tensor) -> torch.Tensor:
     return parts.sum(0).to(torch.bfloat16)
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
+           tiles: bool = False) -> torch.Tensor:
     """``x @ w.T`` (w in [out, in] layout).  Decode-sized GPU batches (M <= 256)
-    run the hand MFMA kernel (gemm.hip); larger batches (prefill) hipBLASLt."""
+    run the hand MFMA kernel (gemm.hip); larger batches (prefill) hipBLASLt or, with
+    ``tiles`` (no other rank's blocks spin on this device), :func:`pgemm_small` where
+    that pays."""
     r = _dgemm(0, x, w, out)
     if r is not None:
         return r
+    if tiles and out is None and x.is_cuda and x.dim() == 2 and \
+            x.dtype == w.dtype == torch.bfloat16 and _on_grid(x) and \
+            small_tile_pays(x.shape[0], w):
+        return pgemm_small(x, w)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     return F.linear(x, w)

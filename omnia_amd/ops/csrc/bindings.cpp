@@ -24,6 +24,7 @@ int omnia_ar_alltoall(void* out, const void* in, void* const* regions, int* epoc
 int omnia_ar_sendrecv(void* out, const void* in, void* const* regions, int* epochs, int* err,
                       int64_t nbytes, int64_t slot_bytes, int rank, int world, int src_rank,
                       hipStream_t s);
+int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K, hipStream_t s);
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
                        int cols, int f32, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
@@ -1182,6 +1183,18 @@ void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t cols) {
            "pgemm_splitk");
 }
 
+void pgemm_small(at::Tensor out, at::Tensor x, at::Tensor W) {
+  CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W); CHECK_BF16(out);
+  TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1), "x [M, K], W [N, K]");
+  TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "contiguous x / W");
+  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == x.size(0) &&
+              out.size(1) == W.size(0), "out [M, N] contiguous");
+  TORCH_CHECK(x.device() == W.device() && x.device() == out.device(), "same device");
+  if (x.size(0) == 0) return;
+  CHECK_RC(omnia_pgemm_small(out.data_ptr(), x.data_ptr(), W.data_ptr(), x.size(0), W.size(0),
+                             x.size(1), cur_stream()), "pgemm_small");
+}
+
 void row_sumsq(at::Tensor ss, at::Tensor x) {
   CHECK_GPU(x); CHECK_BF16(x);
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "x [M, d] rows contiguous");
@@ -2306,6 +2319,7 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("pgemm", &pgemm);
   m.def("row_sumsq", &row_sumsq);
   m.def("pgemm_splitk", &pgemm_splitk);
+  m.def("pgemm_small", &pgemm_small);
   m.def("ar_twoshot", &ar_twoshot);
   m.def("ar_region_bytes", &omnia_ar_region_bytes);
   m.def("splitk_add_rmsnorm", &splitk_add_rmsnorm);

@@ -95,6 +95,18 @@ def test_plain_projections_on_both_sides_of_the_rule(M, R, K, fills):
     assert ops.plain_tile_fills(M, w) == fills
 
 
+@pytest.mark.parametrize("M,R,K,pays", [
+    (256, 16384, 512, False), (257, 16384, 512, False), (257, 10240, 512, True),  # 384, 240 tiles
+    (1126, 2048, 2048, False), (1127, 2048, 2048, True), (2048, 2048, 2048, True),  # .55 of a round
+    (2049, 2048, 2048, False), (1536, 2048, 2112, False), (1537, 2048, 2112, True),  # K past 2048: .75
+    (2048, 2048, 6144, True), (2048, 2048, 6208, False), (2000, 2000, 2048, False),
+    (2000, 2048, 2048 + 32, False)])
+def test_tiles_of_128_on_both_sides_of_the_rule(M, R, K, pays):
+    w = torch.empty(R, K, dtype=torch.bfloat16, device="meta")
+    assert ops.small_tile_pays(M, w) == pays
+    assert not ops.small_tile_pays(M, w[:, ::2])
+
+
 def test_down_tile_cols():
     """Narrow while the segments to be expected are one round of narrow tiles, half of each expert's
     last one empty; of a shard's experts, their part of the assignments."""

@@ -345,17 +345,19 @@ def test_latent_attention(size, how, run):
 @pytest.mark.parametrize("size", [LATENTS[3], LATENTS[4], dict(LATENTS[3], window=0)],
                          ids=lambda s: f"c{s['kv_rank']}w{s['window']}")
 @pytest.mark.parametrize("lens", [[256, 200], [64], [150, 36, 67, 1], [513]])
-def test_latent_attention_on_whole_tiles_of_keys(size, lens, monkeypatch):
-    """Keys and values expanded on the prefill tile, their rows made whole column tiles with zeros:
-    row counts that are and are not, first portions and ones behind a past."""
+@pytest.mark.parametrize("whole,kernel", [(256, "pgemm"), (128, "pgemm_small")])
+def test_latent_attention_on_whole_tiles_of_keys(size, lens, whole, kernel, monkeypatch):
+    """Keys and values expanded on the prefill tile, or the one of 128 x 128, their rows made whole column
+    tiles with zeros: row counts that are and are not, first portions and ones behind a past."""
     from omnia_amd.models.projection import Projections
 
     class Served(Projections, Stub):
-        tp, _min_rows = 1, 1
+        tp, _min_rows = 1, 1 if whole == 256 else 1 << 20
 
-    seen, pgemm = [], ops.pgemm
-    monkeypatch.setattr(ops, "pgemm", lambda epi, x, w: seen.append((len(x), len(w))) or
-                        pgemm(epi, x, w))
+    seen, run_it = [], getattr(ops, kernel)
+    monkeypatch.setattr(ops, kernel, lambda *a: seen.append((len(a[-2]), len(a[-1]))) or run_it(*a))
+    monkeypatch.setattr(ops, "small_tile_pays", lambda M, w: True)
+    monkeypatch.setattr(ops, "_dgemm", lambda *a: None)
     run = "cuda", torch.bfloat16
     spec = sc.latent(**size)["mixer"]
     mixer, w, W, want = mixer_case("latent_attention", spec, 40, run, 13)
@@ -369,7 +371,7 @@ def test_latent_attention_on_whole_tiles_of_keys(size, lens, monkeypatch):
     for h, y in zip(hs, run_mixer(mixer, w, hs, steps, 32, 17)):
         assert rel(project_out(y, w), want(h)) < LIMIT[torch.bfloat16]
     assert len(seen) == 2 * len(steps)
-    assert all(a % 256 == 0 == c % 256 and (b, c) == (len(w["uk"]), a)
+    assert all(a % whole == 0 and (b, c) == (len(w["uk"]), a)
                for (a, b), (_, c) in zip(seen[::2], seen[1::2]))
 
 
