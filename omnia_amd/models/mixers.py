@@ -154,7 +154,7 @@ class LatentAttention(Mixer):
         m = self.model
         own = isinstance(m, Projections) and m._pgemm_covers(s.latent_pad, uk.shape[0], False)
         tiles = own and m._pgemm_ok(rows, s.latent_pad, uk.shape[0], False)
-        if own:  # fewer, those of tiles of 128 x 128
+        if own:  # fewer, those of smaller tiles
             rows = -(-rows // 256) * 256 if tiles else -(-rows // 128) * 128
         c, kr = mops.latent_gather(pages, fb.block_tables, fb.kv_start, fb.kv_first, fb.seq_lens,
                                    rows, s)

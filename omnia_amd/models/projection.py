@@ -245,8 +245,8 @@ class Projections:
 
     def _mid(self, x: torch.Tensor, w: torch.Tensor, is_decode: bool, slabs: bool):
         """More rows than the few-row kernels take and fewer than ``_pgemm_ok`` asks for: the
-        prefill tile where it fills the chip, whole or in slices of K (fp32 :class:`Parts`), tiles of
-        128 x 128 where those do, else the library."""
+        prefill tile where it fills the chip, whole or in slices of K (fp32 :class:`Parts`), smaller
+        tiles where those do (:func:`ops.small_tile_cols`), else the library."""
         M, K = x.shape
         if M > ops.PANEL_MAX_M and self.tp == 1 and ops._on_grid(x, w) and \
                 self._pgemm_covers(K, w.shape[0], is_decode):

@@ -522,28 +522,35 @@ def plain_tile_fills(M: int, w: torch.Tensor) -> bool:
         tile_cols(M, R) == 128 and _tile_rounds(M, R, 128) == 1 and w.is_contiguous() and _on_grid(w)
 
 
-def small_tile_pays(M: int, w: torch.Tensor) -> bool:
-    """Whether :func:`pgemm_small` covers ``w`` and beats the library for more rows than the panel kernel
-    takes: one round of its tiles over 256 CUs, .55 of their work useful, or three quarters where K is
-    long (useful part, us here / library: 2048 x 2048 at 999 rows .49 17.1 / 16.1, 4096 x 2048 at 512 .50
-    21.0 / 17.0; 2048 x 2048 at 1300 .63 17.7 / 21.7,
-    2001 .98 19.0 / 21.7; 4608 x 2048 at 508 .56 18.4 / 21.2; 3072 x 1024 at 999 .73 11.6 / 14.3; 2048 x
-    512 at 2048 1.0 8.9 / 11.1; 4096 x 4096 at 700 .68 34.3 / 32.6, 999 .98 38.7 / 40.9; 2560 x 4096 at
-    1316 .80 34.4 / 42.0; 5888 x 6144 at 512 .72 62.3 / 55.0, 3712 x 6144 at 897 .79 50.0 / 58.5).  Over 60
-    such sizes the library takes 1.03 to 1.45 as long."""
-    if M <= PANEL_MAX_M or w.dim() != 2:
-        return False
+def small_tile_cols(M: int, w: torch.Tensor) -> int:
+    """Columns (128, 64) of the tile on which :func:`pgemm_small` beats the library for more rows than the
+    panel kernel takes, 0: none.  One round of its tiles over 256 CUs, .55 of their work useful, where K is
+    long three quarters, of the smaller .65 (useful part, us here / library: 128 columns: 4096 x 2048 at 512
+    rows .50 21.0 / 17.0; 2048 x 2048 at 1300 .63 17.7 / 21.7, 2001 .98 19.0 / 21.7; 4608 x 2048 at 508 .56
+    18.4 / 21.2; 3072 x 1024 at 999 .73 11.6 / 14.3; 2048 x 512 at 2048 1.0 8.9 / 11.1; 4096 x 4096 at 700
+    .68 34.3 / 32.6, 999 .98 38.7 / 40.9; 5888 x 6144 at 512 .72 62.3 / 55.0, 3712 x 6144 at 897 .79 50.0 /
+    58.5.  64: 2048 x 2048 at 512 .50 13.1 / 12.5, 700 .68 13.8 / 14.7, 999 .98 14.6 / 17.3; 4096 x 2048 at
+    512 1.0 14.7 / 17.1; 1472 x 512 at 1075 .75 6.9 / 10.3; 1600 x 2560 at 726 .55 16.9 / 17.3, 2688 x 2560
+    at 550 .70 17.6 / 17.4; 3584 x 4096 at 393 .67 24.5 / 29.2; 2048 x 6144 at 860 .84 39.0 / 42.0).  Over
+    160 such sizes the library takes .99 to 1.5 as long."""
+    if M <= PANEL_MAX_M or w.dim() != 2 or not (w.is_contiguous() and _on_grid(w)):
+        return 0
     R, K = w.shape
-    return R % 128 == 0 and K % 64 == 0 and K <= 6144 and -(-M // 128) * (R // 128) <= 256 and \
-        M * R > (0.55 if K <= 2048 else 0.75) * 256 * 128 * 128 and w.is_contiguous() and _on_grid(w)
+    if K % 64 or K > 6144:
+        return 0
+    for cols, useful in ((128, 0.55 if K <= 2048 else 0.75), (64, 0.55 if K <= 2048 else 0.65)):
+        if R % cols == 0 and -(-M // 128) * (R // cols) <= 256 and M * R > useful * 256 * 128 * cols:
+            return cols
+    return 0
 
 
-def pgemm_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w.T`` on MFMA tiles of 128 x 128 (``csrc/pgemm.hip``): whole ones of ``w``, K of whole 64."""
+def pgemm_small(x: torch.Tensor, w: torch.Tensor, cols: int = 128) -> torch.Tensor:
+    """``x @ w.T`` on MFMA tiles of 128 x ``cols`` (``csrc/pgemm.hip``): whole ones of ``w``, K of whole 64;
+    the bits of :func:`pgemm`."""
     if not x.is_cuda:
         return (x.float() @ w.float().t()).to(x.dtype)
     out = x.new_empty(x.shape[0], w.shape[0])
-    kernels().pgemm_small(out, x.contiguous(), w)
+    kernels().pgemm_small(out, x.contiguous(), w, cols)
     return out
 
 
@@ -861,9 +868,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
     if r is not None:
         return r
     if tiles and out is None and x.is_cuda and x.dim() == 2 and \
-            x.dtype == w.dtype == torch.bfloat16 and _on_grid(x) and \
-            small_tile_pays(x.shape[0], w):
-        return pgemm_small(x, w)
+            x.dtype == w.dtype == torch.bfloat16 and _on_grid(x):
+        cols = small_tile_cols(x.shape[0], w)
+        if cols:
+            return pgemm_small(x, w, cols)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     return F.linear(x, w)

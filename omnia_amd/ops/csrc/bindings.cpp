@@ -24,7 +24,8 @@ int omnia_ar_alltoall(void* out, const void* in, void* const* regions, int* epoc
 int omnia_ar_sendrecv(void* out, const void* in, void* const* regions, int* epochs, int* err,
                       int64_t nbytes, int64_t slot_bytes, int rank, int world, int src_rank,
                       hipStream_t s);
-int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K, hipStream_t s);
+int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K, int cols,
+                      hipStream_t s);
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
                        int cols, int f32, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
@@ -1183,7 +1184,7 @@ void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t cols) {
            "pgemm_splitk");
 }
 
-void pgemm_small(at::Tensor out, at::Tensor x, at::Tensor W) {
+void pgemm_small(at::Tensor out, at::Tensor x, at::Tensor W, int64_t cols) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W); CHECK_BF16(out);
   TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1), "x [M, K], W [N, K]");
   TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "contiguous x / W");
@@ -1192,7 +1193,7 @@ void pgemm_small(at::Tensor out, at::Tensor x, at::Tensor W) {
   TORCH_CHECK(x.device() == W.device() && x.device() == out.device(), "same device");
   if (x.size(0) == 0) return;
   CHECK_RC(omnia_pgemm_small(out.data_ptr(), x.data_ptr(), W.data_ptr(), x.size(0), W.size(0),
-                             x.size(1), cur_stream()), "pgemm_small");
+                             x.size(1), (int)cols, cur_stream()), "pgemm_small");
 }
 
 void row_sumsq(at::Tensor ss, at::Tensor x) {

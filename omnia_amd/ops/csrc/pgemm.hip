@@ -872,15 +872,20 @@ void launch_narrow(const PArgs& a, dim3 grid, hipStream_t s) {
 
 // out = X . W^T on tiles of 128 x 128, a wave 64 x 64 of them, for steps whose larger tiles are half a
 // round or less: us, library / here and narrow tile, 2048 x 2048 at 2001 rows 21.7 / 19.0 and 24.2, 4096
-// x 2048 at 999 24.6 / 21.2 and 28.7, 3072 x 1024 at 999 14.3 / 11.6 and 15.2 (ops.small_tile_pays).  A K-tile is a half-tile of each operand in a ring of five, 128 KB in flight; its 32
-// products a wave take half of the 0.42 us of its intake (78 GB/s a CU), so one barrier a K-tile does: every wave has read K-tile
-// t, and t + 1 has landed.
+// x 2048 at 999 24.6 / 21.2 and 28.7, 3072 x 1024 at 999 14.3 / 11.6 and 15.2 (ops.small_tile_pays).  A K-tile
+// is a half-tile of each operand in a ring of five, 128 KB in flight; its 32 products a wave take half of
+// the 0.42 us of its intake (78 GB/s a CU), so one barrier a K-tile does: every wave has read K-tile t,
+// and t + 1 has landed.
+// NF 2: 128 x 64, a wave 64 x 32, in a ring of six (2048 x 2048 at 999 rows 14.6, NF 4 18.5, library 17.3; 2048
+// x 4096 24.6, 31.5, 27.7; 2048 x 1024 9.5, 11.5, 11.8).
+template <int NF>
 __global__ __launch_bounds__(256, 1) void pgemm_small_kernel(bf16_t* out, const bf16_t* X,
                                                              const bf16_t* W, int M, int N, int K,
                                                              int64_t ldo) {
-  constexpr int F = 4, RING = 10 * HALF;  // fragments of a wave, either way
+  constexpr int MF = 4, TN = 32 * NF, L = 4 + NF;  // fragments of a wave; DMAs of one a K-tile
+  constexpr int DEPTH = NF == 4 ? 5 : 6, STAGE = HALF + TN * BK, RING = DEPTH * STAGE;
   __shared__ __attribute__((aligned(1024))) bf16_t lds[RING];
-  const int ntn = N >> 7, mtn = (M + 127) >> 7, nk = K / BK;
+  const int ntn = N / TN, mtn = (M + 127) >> 7, nk = K / BK;
   const int bid = xcd_remap(blockIdx.x, mtn * ntn), per_group = 4 * ntn;
   const int grp = bid / per_group, gsz = mtn - 4 * grp < 4 ? mtn - 4 * grp : 4;
   const int idx = bid - grp * per_group, mt = 4 * grp + idx % gsz, nt = idx / gsz;
@@ -888,39 +893,43 @@ __global__ __launch_bounds__(256, 1) void pgemm_small_kernel(bf16_t* out, const 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = w >> 1, wc = w & 1, fr = lane & 15, fq = lane >> 4;
 
-  // ---- DMAs, as in tile()
+  // ---- DMAs, as in tile(): a wave's of x 32 rows, of W 8 NF
   const char* xb = (const char*)(X + (int64_t)m0 * K);
-  const char* wb = (const char*)(W + (int64_t)nt * 128 * K);
-  uint32_t vx[4], vw[4];
+  const char* wb = (const char*)(W + (int64_t)nt * TN * K);
+  uint32_t vx[4], vw[NF];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 32 * w + 8 * i + (lane >> 3);
-    const uint32_t ch = ((lane & 7) ^ (r & 7)) << 4;
-    vx[i] = (uint32_t)(r < Mt ? r : Mt - 1) * (uint32_t)K * 2u + ch;
-    vw[i] = (uint32_t)r * (uint32_t)K * 2u + ch;
+    vx[i] = (uint32_t)(r < Mt ? r : Mt - 1) * (uint32_t)K * 2u + (((lane & 7) ^ (r & 7)) << 4);
   }
-  const uint32_t dst0 =
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)lds + 32 * w * 128;
-  auto next = [](int s) { return s + 2 * HALF == RING ? 0 : s + 2 * HALF; };
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int r = 8 * (NF * w + i) + (lane >> 3);
+    vw[i] = (uint32_t)r * (uint32_t)K * 2u + (((lane & 7) ^ (r & 7)) << 4);
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const bf16_t*)lds;
+  const uint32_t dx = lds0 + 32 * w * 128, dw = lds0 + HALF * 2 + 8 * NF * w * 128;
+  auto next = [](int s) { return s + STAGE == RING ? 0 : s + STAGE; };
   int ds = 0, kt = 0;
-  uint32_t at = 0;
+  uint32_t ax = 0, aw = 0;
   const char *px = xb, *pw = wb;
   auto set = [&]() __attribute__((always_inline)) {  // past the end the last K-tile again
-    at = dst0 + ds * 2;
+    ax = dx + ds * 2;
+    aw = dw + ds * 2;
     px = xb + (int64_t)kt * (BK * 2);
     pw = wb + (int64_t)kt * (BK * 2);
     kt = kt + 1 < nk ? kt + 1 : nk - 1;
     ds = next(ds);
   };
   auto dma = [&](int d) __attribute__((always_inline)) {
-    if (d < 4) dma16(vx[d], px, at, d * 1024);
-    else dma16(vw[d - 4], pw, at, HALF * 2 + (d - 4) * 1024);
+    if (d < 4) dma16(vx[d], px, ax, d * 1024);
+    else dma16(vw[d - 4], pw, aw, (d - 4) * 1024);
   };
 #pragma unroll
-  for (int t = 0; t < 5; ++t) {
+  for (int t = 0; t < DEPTH; ++t) {
     set();
 #pragma unroll
-    for (int d = 0; d < 8; ++d) dma(d);
+    for (int d = 0; d < L; ++d) dma(d);
   }
 
   int rs = 0;
@@ -930,67 +939,72 @@ __global__ __launch_bounds__(256, 1) void pgemm_small_kernel(bf16_t* out, const 
     for (int s = 0; s < 2; ++s) {
       const int o = rs + fr * BK + (((4 * s + fq) ^ (fr & 7)) << 3);
       fa[s] = lds + o + wr * 64 * BK;
-      fb[s] = lds + o + HALF + wc * 64 * BK;
+      fb[s] = lds + o + HALF + wc * 16 * NF * BK;
     }
     rs = next(rs);
   };
-  short8 fx[2][F], fw[2][F];
+  short8 fx[2][MF], fw[2][NF];
   auto read = [&](int s, int j) __attribute__((always_inline)) {
-    if (j < F) fx[s][j] = *reinterpret_cast<const short8*>(fa[s] + j * 16 * BK);
-    else fw[s][j - F] = *reinterpret_cast<const short8*>(fb[s] + (j - F) * 16 * BK);
+    if (j < MF) fx[s][j] = *reinterpret_cast<const short8*>(fa[s] + j * 16 * BK);
+    else fw[s][j - MF] = *reinterpret_cast<const short8*>(fb[s] + (j - MF) * 16 * BK);
   };
   auto wait_lds = [] __attribute__((always_inline)) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     asm volatile("" ::: "memory");
   };
-  float4v acc[F][F];  // [m][n]: rows 16m + fr, columns 16n + 4fq + j
+  float4v acc[MF][NF];  // [m][n]: rows 16m + fr, columns 16n + 4fq + j
   auto k_tile = [&](auto FIRST) __attribute__((always_inline)) {
     wait_lds();
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       if (s) {
         wait_lds();
-        wait_vm<24>();
+        wait_vm<(DEPTH - 2) * L>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         set();
         set_r();
       }
 #pragma unroll
-      for (int j = 0; j < F * F; ++j) {
-        const int m = j / F, n = (m & 1) ? F - 1 - j % F : j % F;
+      for (int j = 0; j < MF * NF; ++j) {
+        const int m = j / NF, n = (m & 1) ? NF - 1 - j % NF : j % NF;
         if (decltype(FIRST)::value && !s) mfma16_first(acc[m][n], fw[s][n], fx[s][m]);
         else mfma16(acc[m][n], fw[s][n], fx[s][m]);
-        if (!(j & 1)) read(1 - s, j >> 1);
-        else if (s) dma(j >> 1);
+        // L reads, and L DMAs behind them
+        const int rd = NF == 4 ? (j & 1 ? -1 : j >> 1) : j < L ? j : -1;
+        const int dm = NF == 4 ? (j & 1 ? j >> 1 : -1) : j - (MF * NF - L);
+        if (rd >= 0) read(1 - s, rd);
+        if (s && dm >= 0) dma(dm);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  wait_vm<32>();
+  wait_vm<(DEPTH - 1) * L>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   set_r();
 #pragma unroll
-  for (int j = 0; j < 2 * F; ++j) read(0, j);
+  for (int j = 0; j < L; ++j) read(0, j);
   k_tile(std::true_type{});
   for (int t = 1; t < nk; ++t) k_tile(std::false_type{});
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < F * F; ++i) asm volatile("" : "+a"(acc[i / F][i % F]));
+  for (int i = 0; i < MF * NF; ++i) asm volatile("" : "+a"(acc[i / NF][i % NF]));
   asm volatile("s_nop 15" ::: "memory");
   wait_vm<0>();  // the reloads past the end land before LDS is left
 
   const int ccol = 16 * (fq & 1) + 8 * (fq >> 1);
 #pragma unroll
-  for (int m = 0; m < F; ++m) {
+  for (int m = 0; m < MF; ++m) {
     const int r = wr * 64 + 16 * m + fr;
-    const uint4v a = chunk<0>(acc[m][0], acc[m][1]), b = chunk<0>(acc[m][2], acc[m][3]);
+    uint4v v[NF / 2];
+#pragma unroll
+    for (int n = 0; n < NF; n += 2) v[n / 2] = chunk<0>(acc[m][n], acc[m][n + 1]);
     if (r < Mt) {
-      bf16_t* o = out + (int64_t)(m0 + r) * ldo + nt * 128 + wc * 64 + ccol;
-      *reinterpret_cast<uint4v*>(o) = a;
-      *reinterpret_cast<uint4v*>(o + 32) = b;
+      bf16_t* o = out + (int64_t)(m0 + r) * ldo + nt * TN + wc * 16 * NF + ccol;
+#pragma unroll
+      for (int n = 0; n < NF; n += 2) *reinterpret_cast<uint4v*>(o + 16 * n) = v[n / 2];
     }
   }
 }
@@ -1158,19 +1172,21 @@ int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int
 #undef OMNIA_PGEMM
 }
 
-// out[M, N] = X . W^T on tiles of 128 x 128
-int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K,
+// out[M, N] = X . W^T on tiles of 128 x cols (128 or 64)
+int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K, int cols,
                       hipStream_t s) {
+  if (cols != 64 && cols != 128) return -16;
   if (M < 1) return -2;
   if (K <= 0 || K % BK || K > (1 << 23)) return -3;
-  if (N <= 0 || N % 128) return -4;
+  if (N <= 0 || N % cols) return -4;
   if ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
        reinterpret_cast<uintptr_t>(out)) & 15)
     return -5;
-  const int64_t blocks = (int64_t)((M + 127) / 128) * (N / 128);
+  const int64_t blocks = (int64_t)((M + 127) / 128) * (N / cols);
   if (blocks > (1 << 30)) return -13;
-  pgemm_small_kernel<<<(unsigned)blocks, 256, 0, s>>>((bf16_t*)out, (const bf16_t*)X,
-                                                      (const bf16_t*)W, M, N, K, N);
+  const auto kernel = cols == 128 ? pgemm_small_kernel<4> : pgemm_small_kernel<2>;
+  kernel<<<(unsigned)blocks, 256, 0, s>>>((bf16_t*)out, (const bf16_t*)X, (const bf16_t*)W, M, N, K,
+                                          N);
   return (int)hipGetLastError();
 }
 

@@ -95,16 +95,18 @@ def test_plain_projections_on_both_sides_of_the_rule(M, R, K, fills):
     assert ops.plain_tile_fills(M, w) == fills
 
 
-@pytest.mark.parametrize("M,R,K,pays", [
-    (256, 16384, 512, False), (257, 16384, 512, False), (257, 10240, 512, True),  # 384, 240 tiles
-    (1126, 2048, 2048, False), (1127, 2048, 2048, True), (2048, 2048, 2048, True),  # .55 of a round
-    (2049, 2048, 2048, False), (1536, 2048, 2112, False), (1537, 2048, 2112, True),  # K past 2048: .75
-    (2048, 2048, 6144, True), (2048, 2048, 6208, False), (2000, 2000, 2048, False),
-    (2000, 2048, 2048 + 32, False)])
-def test_tiles_of_128_on_both_sides_of_the_rule(M, R, K, pays):
+@pytest.mark.parametrize("M,R,K,cols", [
+    (256, 10240, 512, 0), (257, 10240, 512, 128), (257, 16384, 512, 0),      # 240 and 384 tiles
+    (1126, 2048, 2048, 0), (1127, 2048, 2048, 128), (2048, 2048, 2048, 128),  # .55 of a round
+    (563, 2048, 2048, 0), (564, 2048, 2048, 64), (1024, 2048, 2048, 64), (1025, 2048, 2048, 0),
+    (1536, 2048, 2112, 0), (1537, 2048, 2112, 128),                          # K past 2048: .75
+    (665, 2048, 2112, 0), (666, 2048, 2112, 64),                             # and .65
+    (2048, 2048, 6144, 128), (2048, 2048, 6208, 0), (2049, 2048, 2048, 0),
+    (999, 1664 + 64, 2048, 64), (999, 1664 + 32, 2048, 0), (2000, 2048, 2048 + 32, 0)])
+def test_smaller_tiles_on_both_sides_of_the_rule(M, R, K, cols):
     w = torch.empty(R, K, dtype=torch.bfloat16, device="meta")
-    assert ops.small_tile_pays(M, w) == pays
-    assert not ops.small_tile_pays(M, w[:, ::2])
+    assert ops.small_tile_cols(M, w) == cols
+    assert not ops.small_tile_cols(M, w[:, ::2])
 
 
 def test_down_tile_cols():

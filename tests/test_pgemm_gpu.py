@@ -348,13 +348,14 @@ def test_narrow_tile(gen, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(1, 128, 64), (127, 384, 128), (129, 128, 320), (300, 256, 384),
                                    (641, 640, 1152), (2048, 2048, 2048)])
-def test_small_tile(gen, M, N, K):
-    """Tiles of 128 x 128, fewer K-tiles than their ring has and more, groups of four m-tiles and a rest:
+@pytest.mark.parametrize("cols", [64, 128])
+def test_small_tile(gen, M, N, K, cols):
+    """Tiles of 128 x 128 and 128 x 64, fewer K-tiles than their ring has and more, groups of four m-tiles and a rest:
     the bits of the wide tile where that has whole columns, nothing outside."""
     x = _rand(M, K, gen=gen)
     w = _rand(N, K, std=0.05, gen=gen)
     whole = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
-    ops.kernels().pgemm_small(whole[:M], x, w)
+    ops.kernels().pgemm_small(whole[:M], x, w, cols)
     want = x.float() @ w.float().t()
     assert ((whole[:M].float() - want).abs() <= 2 ** -8 * (want.abs() + K ** 0.5 * 0.05)).all()
     assert (whole[M] == 7.0).all()
@@ -362,7 +363,7 @@ def test_small_tile(gen, M, N, K):
         assert torch.equal(whole[:M], ops.pgemm(0, x, w))
     for bad in (w[:, :K // 2], w[1:], torch.empty(N * K + 4, dtype=w.dtype, device=DEV)[4:].view(N, K)):
         with pytest.raises(RuntimeError):
-            ops.kernels().pgemm_small(whole[:M], x[:, :bad.shape[1]].contiguous(), bad)
+            ops.kernels().pgemm_small(whole[:M], x[:, :bad.shape[1]].contiguous(), bad, cols)
 
 
 @pytest.mark.parametrize("M,tiles", [(255, 1), (512, 128), (257, 130), (700, 255), (250, 257),

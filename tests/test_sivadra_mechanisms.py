@@ -347,7 +347,7 @@ def test_latent_attention(size, how, run):
 @pytest.mark.parametrize("lens", [[256, 200], [64], [150, 36, 67, 1], [513]])
 @pytest.mark.parametrize("whole,kernel", [(256, "pgemm"), (128, "pgemm_small")])
 def test_latent_attention_on_whole_tiles_of_keys(size, lens, whole, kernel, monkeypatch):
-    """Keys and values expanded on the prefill tile, or the one of 128 x 128, their rows made whole column
+    """Keys and values expanded on the prefill tile, or a smaller one, their rows made whole column
     tiles with zeros: row counts that are and are not, first portions and ones behind a past."""
     from omnia_amd.models.projection import Projections
 
@@ -355,8 +355,9 @@ def test_latent_attention_on_whole_tiles_of_keys(size, lens, whole, kernel, monk
         tp, _min_rows = 1, 1 if whole == 256 else 1 << 20
 
     seen, run_it = [], getattr(ops, kernel)
-    monkeypatch.setattr(ops, kernel, lambda *a: seen.append((len(a[-2]), len(a[-1]))) or run_it(*a))
-    monkeypatch.setattr(ops, "small_tile_pays", lambda M, w: True)
+    monkeypatch.setattr(ops, kernel, lambda *a: seen.append(tuple(len(t) for t in a if not isinstance(t, int)))
+                        or run_it(*a))
+    monkeypatch.setattr(ops, "small_tile_cols", lambda M, w: 128 if len(w) % 128 == 0 else 64)
     monkeypatch.setattr(ops, "_dgemm", lambda *a: None)
     run = "cuda", torch.bfloat16
     spec = sc.latent(**size)["mixer"]
