@@ -174,7 +174,9 @@ class Projections:
             # mid-size steps below the prefill tile's row threshold: split-K on
             # the 256x256 tile where the table lists a win (ops.midm_config)
             if self.tp == 1 and self.use_pgemm and M < self._min_rows:
-                return ops.midm_config(M, N, K, mode)
+                cfg = ops.midm_config(M, N, K, mode)
+                return cfg if cfg is None or mode else \
+                    (*cfg[:2], ops.midm_slices(M, N, K, cfg[2]))
             return None  # up to 256 rows among them
         # up to 192 rows the few-row kernels come before the tables.  With the consumer's reads of
         # the slabs, us at 64 / 128 / 192 rows, packed panel (fp32 slabs) and table (fp16 from 65
@@ -201,7 +203,7 @@ class Projections:
         """ops.wgemm, on the tile-packed copy of ``w`` when one exists for this
         tgemm config; split-K slabs in fp16 on the tile GEMM (``out``'s dtype)."""
         if nwaves == ops.PGEMM_SPLIT:
-            return ops.pgemm_splitk(x, w, S, out, cols=nw)
+            return ops.pgemm_splitk(x, w, S, out, cols=nw, uneven=True)
         if nwaves < 0 and mode == 2 and out is not None and out.dtype == torch.float16:
             mode = 3
         packed = getattr(self, "_packed", None)

@@ -292,6 +292,25 @@ def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | Non
     return (256, PGEMM_SPLIT, S) if S else None
 
 
+@functools.lru_cache(maxsize=8192)
+def midm_slices(M: int, N: int, K: int, S: int) -> int:
+    """Slices of K, uneven ones among them, for ``M`` rows of a weight [N, K] on the wide tile where
+    :func:`midm_config` says ``S``: more where rows of its bucket leave CUs without a tile, by what a
+    K-tile of 64 and a slab's write and read take (us with the residual step, the table's / more: 4096 x
+    14336 at 600 rows 94 / 83, 1100 142 / 120; 4096 x 4096 39.8 / 37.1, 55.3 / 48.3; products alone 6144 x
+    4096 at 512 30.5 / 28.3, at 600 44.7 / 36.6).  Never fewer, as each fp16 slab saturates."""
+    tiles, nk = -(-M // 256) * (N // 256), K // 64
+
+    def us(s):
+        return -(-nk // s) * 1.35 + s * M * N * 2 * (1 / 3.6e6 + 1 / 7e6)
+
+    best = S
+    for s in range(S + 1, 17):
+        if tiles * s <= 256 and us(s) < 0.98 * us(best):
+            best = s
+    return best
+
+
 def wgemm(mode: int, x: torch.Tensor, w: torch.Tensor, splits: int = 1, nw: int = 2,
           nwaves: int = 4, out: torch.Tensor | None = None) -> torch.Tensor:
     """Decode GEMM with W streamed HBM -> MFMA registers (``csrc/wgemm.hip``).
@@ -579,21 +598,23 @@ def tile_slices(M: int, R: int, K: int) -> int:
 
 
 def pgemm_splitk(x: torch.Tensor, w: torch.Tensor, splits: int, out: torch.Tensor | None = None,
-                 cols: int = 0) -> torch.Tensor:
+                 cols: int = 0, uneven: bool = False) -> torch.Tensor:
     """Split-K slabs ``[splits, M, N]`` of ``x @ w.T`` on the MFMA tile of 256 rows and ``cols``
     (128, else 256) columns (``csrc/pgemm.hip`` EPI 4, 11).  Each
     slab is one K-slice's fp32 sum, saturated to fp16 unless ``out`` is fp32; the splitk consumers
-    reduce them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip)."""
+    reduce them.  Decode projections at M <= 256 (one m-tile; the K split fills the chip).
+    ``uneven``: slices of any whole 64 of K, else all alike and of whole 128."""
     M, K = x.shape
     N = w.shape[0]
     if out is None:
         out = torch.empty(splits, M, N, dtype=torch.float16, device=x.device)
     if x.is_cuda:
-        kernels().pgemm_splitk(out, x.contiguous(), w, 128 if cols == 128 else 256)
+        kernels().pgemm_splitk(out, x.contiguous(), w, 128 if cols == 128 else 256, uneven)
         return out
-    ks = K // splits
-    for s in range(splits):
-        r = x[:, s * ks:(s + 1) * ks].float() @ w[:, s * ks:(s + 1) * ks].float().t()
+    at = [s * (K // 64) // splits * 64 for s in range(splits)] + [K] if uneven else \
+        range(0, K + 1, K // splits)
+    for s, (a, b) in zip(range(splits), zip(at, at[1:])):
+        r = x[:, a:b].float() @ w[:, a:b].float().t()
         out[s].copy_(r if out.dtype == torch.float32 else r.clamp(-65504.0, 65504.0))
     return out
 

@@ -27,7 +27,7 @@ int omnia_ar_sendrecv(void* out, const void* in, void* const* regions, int* epoc
 int omnia_pgemm_small(void* out, const void* X, const void* W, int M, int N, int K, int cols,
                       hipStream_t s);
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int cols, int f32, hipStream_t s);
+                       int cols, int f32, int uneven, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
@@ -1169,7 +1169,7 @@ void panel_gemm(int64_t epi, at::Tensor out, at::Tensor x, at::Tensor W, int64_t
 
 // split-K MFMA GEMM (pgemm.hip EPI 4, 11): parts fp16 or fp32 [S, M, N] whose sum
 // over S is x @ W^T; cols of a tile: 128, 256 (0)
-void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t cols) {
+void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t cols, bool uneven) {
   CHECK_GPU(x); CHECK_BF16(x); CHECK_BF16(W);
   TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && W.size(1) == x.size(1), "x [M, K], W [N, K]");
   TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "contiguous x / W");
@@ -1180,7 +1180,7 @@ void pgemm_splitk(at::Tensor parts, at::Tensor x, at::Tensor W, int64_t cols) {
   TORCH_CHECK(x.device() == W.device() && x.device() == parts.device(), "same device");
   if (x.size(0) == 0) return;
   CHECK_RC(omnia_pgemm_splitk(parts.data_ptr(), x.data_ptr(), W.data_ptr(), x.size(0), W.size(0),
-                              x.size(1), parts.size(0), (int)cols, f32, cur_stream()),
+                              x.size(1), parts.size(0), (int)cols, f32, uneven, cur_stream()),
            "pgemm_splitk");
 }
 
@@ -2319,7 +2319,8 @@ PYBIND11_MODULE(_omnia_kernels, m) {
   m.def("tgemm", &tgemm);
   m.def("pgemm", &pgemm);
   m.def("row_sumsq", &row_sumsq);
-  m.def("pgemm_splitk", &pgemm_splitk);
+  m.def("pgemm_splitk", &pgemm_splitk, py::arg("parts"), py::arg("x"), py::arg("W"),
+        py::arg("cols"), py::arg("uneven") = false);
   m.def("pgemm_small", &pgemm_small);
   m.def("ar_twoshot", &ar_twoshot);
   m.def("ar_region_bytes", &omnia_ar_region_bytes);

@@ -256,8 +256,8 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   const int S = sliced(EPI) ? p.splits : 1, ntn = p.N / TN;
   // (flat: grouped only, the first rows of a segment of 256)
   const int m0 = mt << 8, Mt = p.M - m0 < 256 ? p.M - m0 : 256;
-  const int K = p.K, nk = K / S / BK;
-  const int64_t kbase = (int64_t)ks * (K / S);
+  const int K = p.K, kt0 = ks * (K / BK) / S, nk = (ks + 1) * (K / BK) / S - kt0;
+  const int64_t kbase = (int64_t)kt0 * BK;
   const bf16_t* Wb = p.W + kbase;
   if constexpr (grouped(EPI))
     Wb += (int64_t)(p.blk_expert[mt] - p.e_lo) * (gated(EPI) ? 2 * p.N : p.N) * K;
@@ -1036,7 +1036,7 @@ extern "C" {
 // Returns 0 on success, < 0 for a shape / argument the kernel does not cover
 // (checked BEFORE any launch).
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int cols, int f32, hipStream_t s);
+                       int cols, int f32, int uneven, hipStream_t s);
 int omnia_pgemm_moe(int mode, void* out, const void* A, const void* W, const int* sorted,
                     const int* blk_expert, const int* n_blocks, const float* route_w, int K,
                     int N, int topk, int n_assign, int e_lo, int max_blocks, float alpha,
@@ -1054,7 +1054,7 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
   if (bias && (epi != 1 || ss_in)) return -14;
   if (gelu && (epi != 1 || ss_in || bias)) return -15;
   if (M < 1) return -2;
-  if (K <= 0 || K % (2 * BK)) return -3;  // (the loop takes any K-tiles; odd numbers go untested)
+  if (K <= 0 || K % (2 * BK)) return -3;
   const int tn = (epi == 1 ? 128 : 256) >> (narrow ? 1 : 0);
   if (N <= 0 || N % tn) return -4;
   if ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
@@ -1100,13 +1100,15 @@ int omnia_pgemm(int epi, void* out, const void* X, const void* W, int M, int N, 
 }
 
 // split-K GEMM: parts[S][M][N] fp16 or fp32, sum over s of parts[s] = X . W^T (EPI 4, 11).
-// cols: of a tile, 128 or 256 (0).
+// cols: of a tile, 128 or 256 (0).  uneven: slices of any whole K-tiles, as alike as they can be
+// (ops.midm_slices); else all of the same number, an even one.
 int omnia_pgemm_splitk(void* parts, const void* X, const void* W, int M, int N, int K, int S,
-                       int cols, int f32, hipStream_t s) {
+                       int cols, int f32, int uneven, hipStream_t s) {
   if (cols && cols != 128 && cols != 256) return -16;
   const int tn = cols == 128 ? 128 : 256;
   if (M < 1 || S < 1 || S > 16) return -1;
-  if (K <= 0 || K % S || (K / S) % (2 * BK)) return -3;
+  if (K <= 0) return -3;
+  if (uneven ? K % BK || K / BK < S : K % S || (K / S) % (2 * BK)) return -3;
   if (N <= 0 || N % tn) return -4;
   if ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) |
        reinterpret_cast<uintptr_t>(parts)) & 15)

@@ -36,6 +36,20 @@ def test_slices_are_the_tables():
         assert ops.midm_config(b, N, K, mode) == (256, ops.PGEMM_SPLIT, S)
 
 
+def test_more_slices_where_tiles_leave_cus_idle():
+    """3 and 5 tiles of 256 rows: slices of uneven length; never fewer than the table's, one round."""
+    more = ops.midm_slices
+    assert more(600, 4096, 14336, 4) == 5 and more(1100, 4096, 14336, 2) == 3
+    assert more(512, 4096, 14336, 8) == 8 and more(1024, 4096, 4096, 4) == 4
+    assert more(512, 6144, 4096, 4) == 5 and more(1400, 4096, 4096, 2) == 2
+    for M in range(257, 2049, 37):
+        for N in (1024, 4096, 6144, 10240):
+            for K in (2048, 4096, 14336):
+                for S in (2, 4):
+                    s = more(M, N, K, S)
+                    assert s == S or (S < s <= 16 and -(-M // 256) * (N // 256) * s <= 256)
+
+
 def test_kill_switch(monkeypatch):
     monkeypatch.setattr(ops, "_midm_on", False)
     assert ops.midm_config(600, 4096, 14336, 0) is None

@@ -268,6 +268,25 @@ def test_splitk_rejects_bad_split(gen):
         ops.pgemm_splitk(x, w, 16)
 
 
+@pytest.mark.parametrize("M,N,K,S", [(300, 256, 320, 5), (129, 512, 448, 4), (257, 256, 1152, 5),
+                                     (513, 256, 64, 1), (700, 512, 4096, 3)])
+@pytest.mark.parametrize("cols", [128, 256])
+def test_uneven_slices(gen, M, N, K, S, cols):
+    """One K-tile a slice, odd numbers of them and slices of two lengths: each slab is its slice's sum, to
+    K roundings of at most 2^-24 of the sum of magnitudes."""
+    x, w = _rand(M, K, gen=gen), _rand(N, K, std=0.05, gen=gen)
+    parts = torch.empty(S, M, N, device=DEV)
+    ops.pgemm_splitk(x, w, S, parts, cols=cols, uneven=True)
+    at = [s * (K // 64) // S * 64 for s in range(S + 1)]
+    for s, (a, b) in enumerate(zip(at, at[1:])):
+        xs, ws = x[:, a:b].double(), w[:, a:b].double().t()
+        assert ((parts[s].double() - xs @ ws).abs() <= K * 2.0 ** -24 * (xs.abs() @ ws.abs())).all()
+    assert torch.equal(ops.pgemm_splitk(x, w, S, cols=cols, uneven=True), parts.half())
+    with pytest.raises(RuntimeError):  # a slice without a K-tile
+        ops.pgemm_splitk(x, w, K // 64 + 1, cols=cols, uneven=True) if K < 1024 else \
+            ops.pgemm_splitk(x, w, S, cols=cols)
+
+
 @pytest.mark.parametrize("hq,hkv", [(8, 1), (4, 1), (6, 1)])
 def test_qkv_epilogue_tp_shard_heads(gen, hq, hkv):
     """TP shards' QKV: one KV head per rank (Llama-3-70B at TP=8: hq 8, hkv 1 ->
