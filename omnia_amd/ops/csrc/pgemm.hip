@@ -435,9 +435,9 @@ __device__ __forceinline__ void tile(const PArgs& p, bf16_t* __restrict__ lds, i
   };
   // Step s of K-tile t: 8 NF products of 32 k.  FREE: every wave has read the K-tile (its last
   // fragments are asked for by product 30 of step 0, NF 4: 22); its slots take A of t + 2, then,
-  // behind LAND, B of t + 3 (not W_AHEAD: B and A; NF 4: B and A of t + 3).  LAND: the loads younger than K-tile t + 1
-  // may be under way (NF 8: B and A of t + 2; NF 4: all of t + 2, 5 of t + 3), K-tile t + 1 is
-  // there, and its first fragments are read.
+  // behind LAND, B of t + 3 (not W_AHEAD: B and A; NF 4: B and A of t + 3).  LAND: the loads younger
+  // than K-tile t + 1 may be under way (NF 8: B and A of t + 2; NF 4: all of t + 2, 5 of t + 3),
+  // K-tile t + 1 is there, and its first fragments are read.
   constexpr int P = 8 * NF, FREE = NF == 8 ? 36 : 26, LAND = NF == 8 ? 12 : 6;
   constexpr int YOUNGER = NF == 8 ? 16 : 17;
   // the DMA behind product j: B's are 0 to 4 NB - 1, A's from 8 on; -1: none
@@ -750,9 +750,10 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
   // 383; 8 x 2048 x 6144 at 1300, 8 of 16, 165 / 189; 64 x 2048 x 1024 at 3000 of six, 59 of 123, 226 /
   // 281; 2 of 10 113 / 106, 200 / 198 and, of 4096 x 14336, 545 / 520), but where all tiles are one
   // round and, cut, are not (down of 16 x 2048 x 2048 at 2400, 16 of 32, 58.5 / 51; of 8 x 2048 x 4096
-  // at 1000, 4 of 12, all of them cut 60, light ones half as high 63).  Nor where they are few, rounds are few and a tile is soon done (up at 2001, one of
-  // 17, 155 / 158; but K = 4096, up of 8 x 4096 x 4096 at 1600, one of 16, 250 / 219, down at 4096,
-  // three of 35, 268 / 254).  Over 160 such products the rule takes 0.7 % longer than the better of both.
+  // at 1000, 4 of 12, all of them cut 60, light ones half as high 63).  Nor where they are few, rounds
+  // are few and a tile is soon done (up at 2001, one of 17, 155 / 158; but K = 4096, up of 8 x 4096 x 4096
+  // at 1600, one of 16, 250 / 219, down at 4096, three of 35, 268 / 254).  Over 160 such products the rule
+  // takes 0.7 % longer than the better of both.
   uint64_t pick[WORDS];
   if constexpr (MOE && SHAPE == WIDE) {
     if (ordered) {
