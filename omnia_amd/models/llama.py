@@ -249,7 +249,7 @@ class LlamaModel(Projections):
                     known[kind] = {self._wcfg(M, N, w.shape[1], mode, True, w)
                                    for M in range(1, top + 1)}
                 for cfg in known[kind]:
-                    if cfg is None or cfg[1] >= 0 or (-1 - cfg[1]) & 2:
+                    if cfg is None or cfg[1] >= 0 or cfg[1] == ops.PGEMM_SPLIT or (-1 - cfg[1]) & 2:
                         continue  # not tgemm, or its 32-k stage form
                     pmode = 1 if mode == 1 and cfg[2] == 1 else 0
                     want[(w.data_ptr(), cfg[0], pmode)] = w

@@ -187,6 +187,12 @@ class Projections:
         if M <= 192 and w is not None and self.tp == 1 and \
                 few_weight(self, M, w, mode == 1, slabs):
             return None
+        # the prefill tile asks of decode steps what it asks of others (False); else the table's tgemm
+        if self._pgemm_covers(K, N << mode, False) and \
+                (w is None or (w.is_contiguous() and ops._on_grid(w))):
+            cfg = ops.decode_tile_config(M, N, K, mode)
+            if cfg is not None:
+                return cfg
         return ops.wgemm_config(M, N, K, mode)
 
     # split-K slabs of the tile GEMMs in fp16 (tgemm mode 3, pgemm): half the slab bytes

@@ -236,9 +236,7 @@ def wgemm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | No
     (nwaves == 0 selects the wide-batch 32x32x16 kernel, wgemm_wide.hip, with nw
     32-column tiles per wave; nwaves < 0 the full-batch tile kernel, tgemm.hip,
     with nw weight rows per block and non-temporal weight loads when -2;
-    nwaves == PGEMM_SPLIT the prefill tile with nw columns, pgemm.hip, in slices (EPI 4, 11) or, one
-    of a gate_up, whole (EPI 1): us at 256 rows, weights from HBM, tgemm on packed copies / so: gated 28672 x 4096
-    71.7 / 67.1, 4096 x 14336 39.8 / 35.8, 8192 x 28672 126 / 118),
+    nwaves == PGEMM_SPLIT the 256x256 split-K tile, pgemm.hip EPI 4, 11),
     or None to keep the library / gemm.hip path.  ``mode`` 0 = plain projection
     (its split-K slabs are reduced by the consumer kernel), 1 = gate_up + SwiGLU.
     Measured dispatch: ``ops/tuned/wgemm_mi355x.json`` (scripts/wgemm_sweep.py +
@@ -259,6 +257,29 @@ def wgemm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | No
     if cfg is None and b == 192:  # the 192 bucket only lists its own wins
         cfg = _wgemm_table.get(f"{mode}:256:{N}:{K}")
     return cfg
+
+
+_decode_tiles: dict | None = None
+
+
+def decode_tile_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | None:
+    """(columns, PGEMM_SPLIT, splits) of the prefill tile (``csrc/pgemm.hip``, in slices EPI 4, 11, one of
+    a gate_up whole, EPI 1) for decode projections of 193 to 256 rows that it runs in the place of
+    :func:`wgemm_config`'s entry, where a model may use it (``ops/tuned/decode_tile_mi355x.json``), or
+    None.  us at 256 rows, weights from HBM, tgemm on packed copies / so: gated 28672 x 4096 71.7 / 67.1,
+    4096 x 14336 39.8 / 35.8, 8192 x 28672 126 / 118."""
+    global _decode_tiles
+    if not _wgemm_on or not 192 < M <= WGEMM_MAX_M:
+        return None
+    if _decode_tiles is None:
+        import json
+
+        p = os.path.join(os.path.dirname(__file__), "tuned", "decode_tile_mi355x.json")
+        _decode_tiles = {}
+        if os.path.exists(p):
+            with open(p) as f:
+                _decode_tiles = {k: (v[0], PGEMM_SPLIT, v[1]) for k, v in json.load(f).items()}
+    return _decode_tiles.get(f"{mode}:{N}:{K}")
 
 
 MIDM_BUCKETS = (512, 768, 1024, 1536, 2048, 3072, 4096)

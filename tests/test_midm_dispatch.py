@@ -4,7 +4,11 @@ entries, and the OMNIA_MIDM kill switch -- pure table logic, CPU."""
 import json
 import os
 
+import pytest
+import torch
+
 from omnia_amd import ops
+from omnia_amd.models import projection
 
 
 def test_table_file_is_well_formed():
@@ -48,6 +52,27 @@ def test_more_slices_where_tiles_leave_cus_idle():
                 for S in (2, 4):
                     s = more(M, N, K, S)
                     assert s == S or (S < s <= 16 and -(-M // 256) * (N // 256) * s <= 256)
+
+
+@pytest.mark.parametrize("how", ["own device", "switch", "shared device", "off grid", "192 rows"])
+def test_decode_rows_on_the_prefill_tile_only_where_it_may_run(how, monkeypatch):
+    """193 to 256 decode rows: the tile's entry, but the table's tgemm entry with OMNIA_PGEMM=0, beside ranks
+    on one device (whose all-reduce blocks spin), for weights off the 16-byte grid and for fewer rows."""
+    class Model(projection.Projections):
+        device, dtype, tp, use_pgemm = torch.device("cuda"), torch.bfloat16, 2, how != "switch"
+
+    monkeypatch.setattr(projection.pstate, "ranks_per_device", lambda: 2 if how == "shared device" else 1)
+    p = os.path.join(os.path.dirname(ops.__file__), "tuned", "decode_tile_mi355x.json")
+    tiles = json.load(open(p))
+    assert tiles
+    M = 192 if how == "192 rows" else 256
+    for key, (cols, S) in tiles.items():
+        mode, N, K = (int(x) for x in key.split(":"))
+        w = torch.empty(N << mode, K, dtype=torch.bfloat16, device="meta") if how != "off grid" else \
+            torch.empty(K * (N << mode) + 1, dtype=torch.bfloat16)[1:].view(-1, K)
+        cfg, table = Model()._wcfg(M, N, K, mode, True, w), ops.wgemm_config(M, N, K, mode)
+        assert table is not None and ops.PGEMM_SPLIT < table[1] < 0
+        assert cfg == ((cols, ops.PGEMM_SPLIT, S) if how == "own device" else table)
 
 
 def test_kill_switch(monkeypatch):

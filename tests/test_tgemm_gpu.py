@@ -258,3 +258,58 @@ def test_every_tgemm_table_entry_matches_fp32():
         checked += 1
         del x, w
     assert checked >= 10
+
+
+@pytest.mark.parametrize("M", [193, 256])
+def test_every_decode_tile_entry_matches_fp64(M):
+    """Entries of 193 to 256 rows that run on the prefill tile, as the engine runs them: fp16 slabs, each
+    rounded by at most 2^-11 of itself behind K roundings of at most 2^-24 of the sum of magnitudes, or a
+    gated product, rounded to bf16 once, with both halves' roundings."""
+    import json
+    import os
+
+    path = os.path.join(os.path.dirname(ops.__file__), "tuned", "decode_tile_mi355x.json")
+    for key, (cols, S) in json.load(open(path)).items():
+        mode, N, K = (int(v) for v in key.split(":"))
+        assert ops.decode_tile_config(M, N, K, mode) == (cols, ops.PGEMM_SPLIT, S)
+        x, w = _mk(M, N << mode, K, seed=M + N + K)
+        if mode:
+            assert S == 1 and ops.tile_cols(M, 2 * N) == cols
+            got, want, sums = ops.pgemm(1, x, w), [], []
+            for h in w.chunk(2):
+                want.append(x.double() @ h.double().t())
+                sums.append(K * 2.0 ** -24 * (x.double().abs() @ h.double().abs().t()))
+            (g, u), (dg, du) = want, sums
+            want = torch.nn.functional.silu(g) * u
+            # the slope of silu stays below 1.1
+            bound = 2.0 ** -8 * want.abs() + 1.1 * (dg * (u.abs() + du) + g.abs() * du)
+        else:
+            got = ops.pgemm_splitk(x, w, S, cols=cols, uneven=True).double()
+            want, bound = torch.zeros_like(got[0]), torch.zeros_like(got[0])
+            for s in range(S):
+                xs, ws = (t[:, s * K // S:(s + 1) * K // S].double() for t in (x, w))
+                slab, mags = xs @ ws.t(), xs.abs() @ ws.abs().t()
+                want += slab
+                bound += 2.0 ** -11 * slab.abs() + 1.001 * K * 2.0 ** -24 * mags + 2.0 ** -25
+            got = got.sum(0)
+        assert ((got.double() - want).abs() <= bound).all()
+        del x, w, got, want, bound
+
+
+def test_without_the_prefill_tile_gate_up_and_down_run_packed(monkeypatch):
+    """OMNIA_PGEMM=0: 256 decode rows run tgemm on packed copies of all four projections."""
+    from omnia_amd.models import build_model
+    from omnia_amd.models.config import resolve
+
+    mc = resolve("llama-3-8b").replace(name="llama-3-8b-1l", num_layers=1, vocab_size=512)
+    m = build_model(mc, device=torch.device("cuda"), dtype=torch.bfloat16, seed=3)
+    layer = m.w["layers"][0]
+    h = (torch.randn(256, mc.hidden_size, device="cuda") * 0.5).to(torch.bfloat16)
+    want = m.mlp(layer, h, is_decode=True).t.float().sum(0)
+    monkeypatch.setattr(m, "use_pgemm", False, raising=False)
+    for name in ("pgemm", "pgemm_splitk"):
+        monkeypatch.setattr(ops, name, lambda *a, **kw: pytest.fail("the prefill tile"))
+    assert m.prepack_decode(256) and {k[0] for k in m._packed} == \
+        {layer[k].data_ptr() for k in ("qkv", "o", "gate_up", "down")}
+    got = m.mlp(layer, h, is_decode=True).t.float().sum(0)
+    torch.testing.assert_close(got, want, rtol=1e-2, atol=2e-2)
