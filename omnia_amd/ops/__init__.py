@@ -266,8 +266,10 @@ def decode_tile_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int
     """(columns, PGEMM_SPLIT, splits) of the prefill tile (``csrc/pgemm.hip``, in slices EPI 4, 11, one of
     a gate_up whole, EPI 1) for decode projections of 193 to 256 rows that it runs in the place of
     :func:`wgemm_config`'s entry, where a model may use it (``ops/tuned/decode_tile_mi355x.json``), or
-    None.  us at 256 rows, weights from HBM, tgemm on packed copies / so: gated 28672 x 4096 71.7 / 67.1,
-    4096 x 14336 39.8 / 35.8, 8192 x 28672 126 / 118."""
+    None.  us, weights from HBM, tgemm on packed copies / so, at 193, 224 and 256 rows: gated 28672 x 4096
+    68.6 / 65.2, 69.8 / 63.8, 71.1 / 64.4, in a model of them at 256 69.9 / 63.6; 4096 x 14336 38.6 / 36.8,
+    38.2 / 37.5, 39.0 / 37.6, in the model 39.9 / 38.9.  Not 8192 x 28672, with its consumer (row-major) 126 /
+    126, 129 / 125, 129 / 129."""
     global _decode_tiles
     if not _wgemm_on or not 192 < M <= WGEMM_MAX_M:
         return None
