@@ -827,18 +827,21 @@ __global__ __launch_bounds__(256, 1) void pgemm_kernel(const bf16_t* X, const bf
   }
   // Experts' rows of 4 KB of W, of which all blocks would ask for the same 128 bytes at a time, and so
   // for a few memory channels: eight column tiles, whose blocks share x in an XCD, walk K in an order of
-  // their own, with the bits of their number reversed, so that neighbours are far apart.  While the
-  // tiles are some rounds only; then blocks are apart by themselves.  us, up products in order / apart: 8
-  // experts of 2048 x 4096 at 600 / 1000 / 2001 / 4000 / 16384 tokens of two 83 / 68, 107 / 92, 168 / 143,
-  // 248 / 249, 907 / 917; 16 of 2048 x 2048 at 2400 140 / 121; 64 of 2048 x 1024 at 3000 of six 229 / 230.
-  // Rows of other lengths lose or gain nothing (8 of 4096 x 14336 at 1001 508 / 532, down of
-  // 2048 x 4096 at 2001 79 / 78).
+  // their own, with the bits of their number reversed, so that neighbours are far apart.  The order follows
+  // the weights' place alone, the expert's own number and the column tile's, so that a row's bits depend
+  // neither on the rows beside it nor on the experts that a rank has.  us, up products in order / apart: 8
+  // experts of 2048 x 4096 at 600 / 1000 / 2001 tokens of two 83 / 68, 107 / 92, 168 / 143; 16 of 2048 x 2048
+  // at 2400 140 / 121; 64 of 2048 x 1024 at 3000 of six 229 / 230; of more than three rounds of tiles, which
+  // are apart by themselves, 8 of 2048 x 4096 at 4000 / 8000 / 16384 250 / 252, 460 / 452, 909 / 912.
+  // Rows of 2 and 8 KB gain nothing (8 experts of 1024 x 2048 at 2001 48.5 / 49.5, of 1024 x 4096 83.4 / 85.1,
+  // of 4096 x 1024 81.1 / 80.4, of 4096 x 2048 145 / 146, 32 of 1024 x 1024 at 2001 of four 57.8 / 63.2; 8 of
+  // 4096 x 14336 at 1001 506 / 514), nor do those of the down product (2048 x 4096 at 2001 79 / 78).
   int turn = 0;
   if constexpr (gathered(EPI)) {
     constexpr int PART = SHAPE == NARROW ? 2 : 1;  // of a wide column tile
     const int octets = (ntn / PART + 7) >> 3;
-    if (p.K == 32 * BK && mtn1 * ntn <= 3 * 256 * PART)
-      turn = (int)(__builtin_bitreverse32(nt / PART / 8 + octets * (p.blk_expert[mt] - p.e_lo)) >> 27);
+    if (p.K == 32 * BK)
+      turn = (int)(__builtin_bitreverse32(nt / PART / 8 + octets * p.blk_expert[mt]) >> 27);
   }
   if constexpr (MOE && SHAPE == WIDE)
     if (light) {

@@ -314,7 +314,7 @@ def test_segments_of_few_rows(E, rows):
 @pytest.mark.parametrize("rows", [[300, 5, 700], [0, 1, 256], [5376] * 4, [5632] * 4])
 def test_column_tiles_that_walk_k_in_orders_of_their_own(rows):
     """Experts of 4 KB rows, 9 wide column tiles (two octets): tiles wide, narrow, cut in two and of
-    half height take the K-tiles in the same order, each once; 756 tiles are the last to, 792 do not."""
+    half height take the K-tiles in the same order, each once, of less than a round, three and more."""
     kk, dev, E, d, I = ops.kernels(), "cuda", len(rows), 2048, 1152
     n = sum(rows)
     ids = torch.arange(E).repeat_interleave(torch.tensor(rows)).int().view(n, 1).to(dev)
@@ -342,6 +342,43 @@ def test_column_tiles_that_walk_k_in_orders_of_their_own(rows):
             got[order[live].long()] = acts[0][live].float()
             torch.testing.assert_close(got[of][:64], torch.nn.functional.silu(a) * b,
                                        atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("cols", [256, 128])
+def test_an_experts_rows_bits_are_their_own(cols):
+    """Experts of 4 KB rows: a row's bits follow neither the rows beside it, in steps of 9 tiles to more
+    than three rounds, nor the experts that are there."""
+    kk, dev, E, d, I, most = ops.kernels(), "cuda", 4, 2048, 1152, 5632
+    x = torch.randn(E, most, d, device=dev).to(torch.bfloat16)
+    up = (torch.randn(E, 2 * I, d, device=dev) * 0.02).to(torch.bfloat16)
+    wts = torch.rand(E, most, device=dev)
+
+    def run(mode, rows, lo=0, hi=E):
+        """{expert: its rows' activations} of the first rows[e] tokens of each expert."""
+        n = sum(rows)
+        ids = torch.arange(E).repeat_interleave(torch.tensor(rows)).int().view(n, 1).to(dev)
+        rw = torch.cat([w[:r] for w, r in zip(wts, rows)]) if mode == 2 else None
+        mb = kk.moe_max_blocks(n, E, 256)
+        order = torch.empty(mb * 256, dtype=torch.int32, device=dev)
+        blk = torch.empty(mb, dtype=torch.int32, device=dev)
+        nb = torch.empty(1, dtype=torch.int32, device=dev)
+        kk.moe_align(order, blk, nb, ids, E, lo, hi)
+        w = up[lo:hi] if mode != 3 else up[lo:hi, :I - 128].contiguous()
+        act = torch.zeros(mb * 256, w.shape[1] // (1 if mode == 3 else 2), device=dev,
+                          dtype=torch.bfloat16)
+        kk.pgemm_moe(mode, act, torch.cat([t[:r] for t, r in zip(x, rows)]), w, order, blk, nb, rw, 1,
+                     n, lo, 1.702, 7.0, cols)
+        live = (order < n) & (torch.arange(mb * 256, device=dev) < nb * 256)
+        got = torch.zeros(n, act.shape[1], device=dev, dtype=act.dtype)
+        got[order[live].long()] = act[live]
+        return {e: t for e, t in enumerate(got.split(rows)) if lo <= e < hi}
+
+    for mode in (0, 2, 3):
+        whole = run(mode, [most] * E)  # 88 segments of 9 (of mode 3: 4) wide column tiles
+        for rows, lo, hi in (([300, 5, 700, 1], 0, E), ([0, 0, 1, 0], 0, E), ([3000] * E, 0, E),
+                             ([300, 5, 700, 1], 2, 4), ([most] * E, 1, 3)):
+            for e, got in run(mode, rows, lo, hi).items():
+                assert torch.equal(got, whole[e][:rows[e]]), (mode, rows, lo, e)
 
 
 def test_segments_of_few_rows_take_no_longer_than_full_ones():
