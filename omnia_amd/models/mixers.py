@@ -149,13 +149,19 @@ class LatentAttention(Mixer):
         # Many keys: their rows, zeros behind them, are whole column tiles of the prefill GEMM, also where
         # they are the weight (us, library / tile, of 2048 x 512: keys at 2112 / 6016 / 16384 / 16640 rows
         # 17.0 / 12.1, 33.5 / 19.6, 41.9 / 41.5, 75.9 / 46.5, values 16.7 / 12.3, 34.0 / 19.6, 43.5 / 42.5,
-        # 75.2 / 47.2; at 4416 17.5 / 19.7 and 24.7 / 18.9)
+        # 75.2 / 47.2; at 4416 17.5 / 19.7 and 24.7 / 18.9); fewer, of smaller ones where a product takes them
+        # (576 / 960 / 1344 / 1984 9.3 / 6.0, 8.8 / 6.1, 10.0 / 7.9, 10.9 / 8.4, values alike), since zeros
+        # cost time elsewhere (64 rows as they are / as 128 5.6 / 6.9, values 5.5 / 6.3)
         uk, uv, rows = w["uk"], w["uv"].view(s.heads * s.v_pad, s.latent_pad), fb.kv_rows
         m = self.model
         own = isinstance(m, Projections) and m._pgemm_covers(s.latent_pad, uk.shape[0], False)
         tiles = own and m._pgemm_ok(rows, s.latent_pad, uk.shape[0], False)
-        if own:  # fewer, those of smaller tiles
-            rows = -(-rows // 256) * 256 if tiles else -(-rows // 128) * 128
+        if tiles:
+            rows = -(-rows // 256) * 256
+        elif own:
+            whole = -(-rows // 128) * 128
+            if ops.small_tile_cols(whole, uk) or ops.small_cols(len(uv), whole, s.latent_pad):
+                rows = whole
         c, kr = mops.latent_gather(pages, fb.block_tables, fb.kv_start, fb.kv_first, fb.seq_lens,
                                    rows, s)
         kx = ops.pgemm(0, c, uk) if tiles else ops.linear(c, uk, tiles=own)

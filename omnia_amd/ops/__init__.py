@@ -575,10 +575,12 @@ def small_tile_cols(M: int, w: torch.Tensor) -> int:
     512 1.0 14.7 / 17.1; 1472 x 512 at 1075 .75 6.9 / 10.3; 1600 x 2560 at 726 .55 16.9 / 17.3, 2688 x 2560
     at 550 .70 17.6 / 17.4; 3584 x 4096 at 393 .67 24.5 / 29.2; 2048 x 6144 at 860 .84 39.0 / 42.0).  Over
     160 such sizes the library takes .99 to 1.5 as long."""
-    if M <= PANEL_MAX_M or w.dim() != 2 or not (w.is_contiguous() and _on_grid(w)):
-        return 0
-    R, K = w.shape
-    if K % 64 or K > 6144:
+    return small_cols(M, *w.shape) if w.dim() == 2 and w.is_contiguous() and _on_grid(w) else 0
+
+
+def small_cols(M: int, R: int, K: int) -> int:
+    """:func:`small_tile_cols` of a contiguous weight [R, K] on the 16-byte grid."""
+    if M <= PANEL_MAX_M or K % 64 or K > 6144:
         return 0
     for cols, useful in ((128, 0.55 if K <= 2048 else 0.75), (64, 0.55 if K <= 2048 else 0.65)):
         if R % cols == 0 and -(-M // 128) * (R // cols) <= 256 and M * R > useful * 256 * 128 * cols:

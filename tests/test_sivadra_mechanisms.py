@@ -376,6 +376,29 @@ def test_latent_attention_on_whole_tiles_of_keys(size, lens, whole, kernel, monk
                for (a, b), (_, c) in zip(seen[::2], seen[1::2]))
 
 
+@GPU
+@pytest.mark.parametrize("lens", [[40], [64], [3, 70], [100, 60]])
+def test_few_latent_keys_are_not_padded(lens, monkeypatch):
+    """Prompts whose products take no tile of 128 rows: the rows of their keys and no more."""
+    from omnia_amd.models import mixers
+    from omnia_amd.models.projection import Projections
+
+    class Served(Projections, Stub):
+        tp = 1
+
+    rows, gather = [], mixers.mops.latent_gather
+    monkeypatch.setattr(mixers.mops, "latent_gather", lambda *a: rows.append(a[5]) or gather(*a))
+    mixer, w, W, want = mixer_case("latent_attention", sc.latent(**LATENTS[3])["mixer"], 40,
+                                   ("cuda", torch.bfloat16), 15)
+    mixer.model = Served("cuda", torch.bfloat16, 1e-5)
+    mixer.model.project = lambda x, w, is_decode: torch.nn.functional.linear(x, w)
+    g = gen(16)
+    hs = [rnd(n, 40, g=g) for n in lens]
+    for h, y in zip(hs, run_mixer(mixer, w, hs, [list(enumerate(lens))], 32, 17)):
+        assert rel(project_out(y, w), want(h)) < LIMIT[torch.bfloat16]
+    assert rows == [sum(-(-n // 64) * 64 for n in lens)]
+
+
 # ------------------------------------------------- one key that stands out
 def attended(q, c, kr, W_uk, W_uv, spec, gate, visible):
     """Plain attention of one query over the keys `visible`."""
