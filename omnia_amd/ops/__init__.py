@@ -319,9 +319,13 @@ def midm_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int] | Non
 def midm_slices(M: int, N: int, K: int, S: int) -> int:
     """Slices of K, uneven ones among them, for ``M`` rows of a weight [N, K] on the wide tile where
     :func:`midm_config` says ``S``: more where rows of its bucket leave CUs without a tile, by what a
-    K-tile of 64 and a slab's write and read take (us with the residual step, the table's / more: 4096 x
-    14336 at 600 rows 94 / 83, 1100 142 / 120; 4096 x 4096 39.8 / 37.1, 55.3 / 48.3; products alone 6144 x
-    4096 at 512 30.5 / 28.3, at 600 44.7 / 36.6).  Never fewer, as each fp16 slab saturates."""
+    K-tile of 64 and an fp16 slab's write and read take.  us with the consumer, the table's / more: 4096 x 14336
+    at 600 rows 87.8 / 78.4, 1100 142 / 119; 4096 x 4096 36.6 / 35.1, 54.8 / 48.8; 6144 x 4096 at 257 / 300 /
+    400 / 512 35.4 / 36.0, 35.3 / 33.8, 36.3 / 34.9, 37.2 / 36.9, at 600 / 768 52.1 / 45.0, 50.8 / 45.8; 10240
+    x 8192 at 257 / 400 / 512 96 / 78, 90 / 79, 91 / 80.  The same numbers do for fp32 slabs (OMNIA_SPLITK_FP32;
+    6144 x 4096 at 400 / 512 / 768 42.6 / 42.0, 44.6 / 44.7, 56.9 / 54.5; 4096 x 4096 at 600 / 1100 42.6 /
+    41.6, 58.5 / 54.4; 4096 x 14336 92.7 / 85.4, 148 / 127), where by twice the bytes the first, second and
+    fourth of these would not be cut.  Never fewer, as each fp16 slab saturates."""
     tiles, nk = -(-M // 256) * (N // 256), K // 64
 
     def us(s):
