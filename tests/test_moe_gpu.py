@@ -344,6 +344,57 @@ def test_column_tiles_that_walk_k_in_orders_of_their_own(rows):
                                        atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("rows", [[1100] * 4, [2300, 0, 2700, 300]])
+@pytest.mark.parametrize("K,N", [(384, 2048), (1152, 1792), (4224, 2048)])
+def test_experts_wide_tiles_left_whole(rows, K, N):
+    """More than 128 wide tiles are not all cut, over rings that turn often: the bits of the narrow tile, and against 64 bits the roundings of K sums, of at most 2^-24 of the sum of
+    magnitudes, and of the result to bf16."""
+    kk, dev, E, n = ops.kernels(), "cuda", len(rows), sum(rows)
+    ids = torch.arange(E).repeat_interleave(torch.tensor(rows)).int().view(n, 1).to(dev)
+    x = torch.randn(n, K, device=dev).to(torch.bfloat16)
+    up = (torch.randn(E, 2 * N, K, device=dev) * 0.05).to(torch.bfloat16)
+    wts = torch.rand(n, device=dev)
+    mb = kk.moe_max_blocks(n, E, 256)
+    order = torch.empty(mb * 256, dtype=torch.int32, device=dev)
+    blk = torch.empty(mb, dtype=torch.int32, device=dev)
+    nb = torch.empty(1, dtype=torch.int32, device=dev)
+    kk.moe_align(order, blk, nb, ids, E, 0, E)
+    live = (order < n) & (torch.arange(mb * 256, device=dev) < nb * 256)
+    at = order[live].long()
+    rowed = torch.zeros(mb * 256, K, device=dev, dtype=torch.bfloat16)  # down: rows in sorted order
+    rowed[live] = x[at]
+    for mode in (0, 1, 2, 3):
+        w = up if mode in (0, 2) else up[:, :N].contiguous()
+        tiles = nb.item() * (N // (128 if mode in (0, 2) else 256))
+        assert tiles > 128
+        res = []
+        for cols in (256, 128):
+            act = torch.zeros(n if mode == 1 else mb * 256, N, device=dev, dtype=torch.bfloat16)
+            kk.pgemm_moe(mode, act, rowed if mode == 1 else x, w, order, blk, nb,
+                         wts if mode in (1, 2) else None, 1, n, 0, 1.702, 7.0, cols)
+            if mode != 1:
+                got = torch.zeros(n, N, device=dev, dtype=torch.bfloat16)
+                got[at] = act[live]
+                act = got
+            res.append(act)
+        assert torch.equal(*res)
+        if mode > 1:
+            continue
+        for e in (e for e in range(E) if rows[e]):
+            of = (ids.view(-1) == e).nonzero().view(-1)[::7]
+            parts = [(x[of].double() @ h.double().t(),
+                      K * 2.0 ** -24 * (x[of].double().abs() @ h.double().abs().t()))
+                     for h in w[e].chunk(1 if mode else 2)]
+            if mode:
+                want, bound = (t * wts[of, None].double() for t in parts[0])
+            else:
+                (g, dg), (u, du) = parts
+                want = torch.nn.functional.silu(g) * u
+                bound = 1.2 * (dg * (u.abs() + du) + g.abs() * du) + 1e-5 * g.abs() * u.abs()
+            err = (res[0][of].double() - want).abs()
+            assert (err <= bound + 2.0 ** -8 * want.abs()).all()
+
+
 @pytest.mark.parametrize("cols", [256, 128])
 def test_an_experts_rows_bits_are_their_own(cols):
     """Experts of 4 KB rows: a row's bits follow neither the rows beside it, in steps of 9 tiles to more

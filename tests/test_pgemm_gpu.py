@@ -405,6 +405,44 @@ def test_tiles_cut_in_two(gen, M, tiles):
         assert torch.equal(out[0], out[1]) and (out[:, M] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(2049, 3840, 384), (100, 33024, 1152), (1030, 6656, 4224),
+                                   (4000, 6400, 640)])
+@pytest.mark.parametrize("how", ["plain", "scaled", "silu", "silu scaled", "silu bias", "gelu"])
+def test_wide_tiles_left_whole(gen, M, N, K, how):
+    """More than 128 wide tiles in the last round are not cut: 135, 129, 130 and 400, over rings that turn
+    often.  The bits of the narrow tile, of tiles of 128 rows and of fewer rows, which are cut; against 64
+    bits the roundings of K sums, of at most 2^-24 of the sum of magnitudes, and of the result to bf16."""
+    tiles = -(-M // 256) * (N // 256)
+    assert tiles % 256 > 128  # a whole round, or tiles % 256 of one, stays
+    x, w = _rand(M, K, gen=gen), _rand(N, K, std=0.05, gen=gen)
+    kw, one = {}, torch.ones(M, 1, device=DEV, dtype=torch.float64)
+    if "scaled" in how:
+        ss = torch.rand(M, 3, device=DEV, generator=gen) * K
+        kw, one = dict(ss_in=ss, inv_d=1.0 / K, eps=1e-5), \
+            torch.rsqrt(ss.double().sum(1) / K + 1e-5)[:, None]
+    if "bias" in how:
+        kw["bias"] = torch.randn(N, device=DEV, generator=gen)
+    epi = int(how.startswith(("silu", "gelu")))
+    got = ops.pgemm(epi, x, w, cols=256, gelu=how == "gelu", **kw)
+    assert torch.equal(got, ops.pgemm(epi, x, w, cols=128, gelu=how == "gelu", **kw))
+    few = dict(kw, ss_in=kw["ss_in"][:60]) if "scaled" in how else kw
+    assert torch.equal(got[:60], ops.pgemm(epi, x[:60], w, cols=256, gelu=how == "gelu", **few))
+    if how == "plain":
+        for cols in (64, 128):
+            assert torch.equal(got, ops.pgemm_small(x, w, cols))
+    parts = []
+    for h, b in zip(w.chunk(1 + epi), kw["bias"].chunk(2) if "bias" in how else (0.0, 0.0)):
+        mags = x.double().abs() @ h.double().abs().t()
+        parts.append(((x.double() @ h.double().t()) * one + b, K * 2.0 ** -24 * mags * one))
+    want, bound = parts[0]
+    if epi:  # the activations' slopes stay below 1.2
+        (g, dg), (u, du) = parts
+        f = torch.nn.functional
+        want = (f.gelu(g, approximate="tanh") if how == "gelu" else f.silu(g)) * u
+        bound = 1.2 * (dg * (u.abs() + du) + g.abs() * du) + 1e-5 * g.abs() * u.abs()
+    assert ((got.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()
+
+
 def test_narrow_tile_refuses(gen):
     x, w = _rand(4, 128, gen=gen), _rand(192, 128, gen=gen)
     for call in (lambda: ops.pgemm(0, x, w, cols=128), lambda: ops.pgemm(0, x, w[:128], cols=64),
