@@ -15,15 +15,21 @@
 //     x half as often and were no faster (28672 x 4096 at 77 51.6, at 256 92): half as many waves
 //     issue the DMA;
 //   * WN is 8, or 4 where few columns would leave CUs without a block, unsliced 2 while its blocks
-//     are one a CU; S blocks share a column tile's K and write fp32 slabs, which the next kernel sums.  A wave walks its slice's K in
-//     order, and S depends on the weight alone (ops.panel_slices): a row's result does not
-//     depend on how many rows the step has;
+//     are one a CU; S blocks share a column tile's K and write fp32 slabs, which the next kernel sums.  S depends on
+//     the weight alone (ops.panel_slices), and so does the order in which a wave walks its slice's K: a
+//     row's result does not depend on how many rows the step has;
 //   * rows of a weight are a power of two of bytes apart, or nearly, and blocks walk them in step, so
 //     at any time all would ask a few memory channels for their 128 bytes of every row.  Where it is
-//     faster, blocks therefore take the chunks of a power of two each in another order: by the number
-//     of its eight weight units, whatever the waves and rows, so that bits do not depend on them, and
-//     its bits reversed, so that blocks that run together are far apart.  It is with row-major weights
-//     of 64 MB and more in walks of 32 chunks (rows, or their slices, of 4 KB), gated also of 64.  us, in
+//     faster, blocks therefore take the chunks of a power of two in other orders: by the number of
+//     their eight weight units, whatever the waves and rows, so that bits do not depend on them, and
+//     with its bits reversed, so that blocks that run together are far apart.  Of 64 chunks each such
+//     block has an order of its own, of 32 two next to each other share one, which is the better of both
+//     (us at 8 / 32 / 77 / 128 rows, shared / each its own: gated 16384 x 2048 12.2 / 13.8, 13.2 / 14.8, 17.4
+//     / 18.3, 22.7 / 23.2; 8192 x 8192 in 4 slices 23.6 / 29.1, 23.1 / 29.9, 25.5 / 32.1, 30.1 / 34.3; 4096 x
+//     14336 in 7 alike; but 32768 x 2048 at 8 26.4 / 22.4, above alike).  It is faster with row-major weights
+//     of 64 MB and more in walks of 32 chunks (rows, or their slices, of 4 KB), gated also of 64: where the
+//     line lies is measured, not derived, since plain walks of 64 lose.  A packed copy of such a weight is
+//     walked in order, so its products have other roundings than the weight's own.  us, in
 //     order / apart, at 32 / 77 / 128 rows: gated 28672 x 4096 42.8 / 39.0, 47.4 / 44.9, 55.1 / 53.4; gated
 //     16384 x 4096 28.9 / 24.6, 33.9 / 31.0, 42.4 / 41.5; gated 16384 x 2048 17.3 / 14.5, 20.5 / 18.6,
 //     24.1 / 23.1; 32768 x 2048 30.8 / 23.0, 32.6 / 24.8, 34.9 / 29.0; 131072 x 2048 103 / 88, 117 / 103,
@@ -137,7 +143,8 @@ __global__ __launch_bounds__(64 * WN, 1) void panel_kernel(const bf16_t* x, cons
   const bool full = XW == 0 || wv < WN - XW;
   const int K = p.K, nch = K >> 6;
   const int c0 = split * nch / p.S, n = (split + 1) * nch / p.S - c0;  // 64-k chunks: stages
-  // stage s of this block is chunk s ^ turn of its slice, by its weights' place alone
+  // stage s of this block is chunk s ^ turn of its slice, by its weights' place alone (of 32 chunks the
+  // lowest bit of the number falls off: two neighbours share an order)
   int turn = 0;
   if (!PK && !grouped(EPI) && (n == 32 || (paired(EPI) && n == 64)) &&
       (int64_t)p.N * K >= (paired(EPI) ? 1 << 24 : 1 << 25))

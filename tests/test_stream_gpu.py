@@ -461,9 +461,9 @@ def test_panel_gated_in_blocks_of_two_waves(M, R, K, packed, monkeypatch):
 @pytest.mark.parametrize("gated,R,K", [(False, 32784, 1024), (False, 32768, 1088), (False, 2048, 16448),
                                        (True, 16416, 2112), (True, 16384, 2048)])
 def test_panel_of_weights_whose_chunks_are_taken_apart(gated, R, K):
-    """Row-major weights of 64 MB and more: of every chunk once, also where their number is odd, has
-    a small power of two or more than 64, in slices too; a row's bits are the same whatever the rows
-    beside it and in blocks of other waves."""
+    """Row-major weights of 64 MB and more: of every chunk once, in order where a walk has not 32 of them (gated:
+    nor 64), also where their number is odd, has a small power of two or more than 64, in slices too; a row's
+    bits are the same whatever the rows beside it and in blocks of other waves."""
     x, w = _mk(200, R, K, R + K)
     whole = ops.panel(int(gated), x, w, slabs=not gated)
     y = whole.sum(0) if whole.dim() == 3 else whole
@@ -479,6 +479,35 @@ def test_panel_of_weights_whose_chunks_are_taken_apart(gated, R, K):
         for o, wn in zip(out, (2, 4, 8)):
             ops.kernels().panel_gemm(int(gated), o, x, w, wn, False, None, False)
             assert torch.equal(o, whole)
+
+
+@pytest.mark.parametrize("gated,R,K,S,apart", [
+    (False, 32768, 2048, 1, True), (False, 4096, 14336, 7, True), (False, 8192, 8192, 4, True),
+    (True, 16384, 2048, 1, True), (True, 16384, 4096, 1, True),
+    (False, 16368, 2048, 1, False), (True, 16352, 2048, 1, False),  # below 64 MB
+    (False, 16384, 4096, 1, False), (True, 16384, 2112, 1, False)])
+def test_panel_walks_of_32_chunks_are_apart(gated, R, K, S, apart):
+    """Large row-major weights in walks of 32 chunks, gated also of 64: every chunk once, in an order that is
+    not the packed copy's; others have its bits.  A row's bits are the same whatever the rows beside it and in
+    blocks of other waves."""
+    x, w = _mk(200, R, K, R + K)
+    slabs = S > 1
+    whole, packed = (ops.panel(int(gated), x, v, packed=p, slabs=slabs)
+                     for v, p in ((w, False), (ops.stream_pack(w), True)))
+    assert (whole.shape[0] == S and whole.dim() == 3) == slabs
+    want = x.double() @ w.double().T
+    if gated:
+        g, u = want.chunk(2, 1)
+        want = F.silu(g) * u
+    for got in (whole, packed):
+        _close(got.sum(0) if slabs else got, want, 4 * K, 1.1)
+    assert torch.equal(whole, packed) != apart
+    for M in (1, 33, 100):
+        assert torch.equal(ops.panel(int(gated), x[:M], w, slabs=slabs), whole[..., :M, :])
+    for wn in (4, 8) if slabs else (2, 4, 8):
+        out = torch.empty_like(whole)
+        ops.kernels().panel_gemm(2 if slabs else int(gated), out, x, w, wn, False, None, False)
+        assert torch.equal(out, whole)
 
 
 def test_panel_plans_fit_the_kernel():
