@@ -861,17 +861,25 @@ void launch(const PArgs& a, dim3 grid, hipStream_t s) {
   pgemm_kernel<EPI, SHAPE, ONCE><<<grid, 256, 0, s>>>(a.X, a.W, a.M, a.N, a.K, a.splits, a.n_blocks,
                                                       a.blk_expert, a.sorted, a);
 }
-// Narrow tiles of up to two m-tiles, which read W together, ask for it past the caches' order of use:
-// us before / now, gated 28672 x 4096 at 224 / 256 rows 71.5 / 67.1, 70.7 / 67.1, 16384 x 2048 at 300 31.6 /
-// 30.6, 4096 x 14336 in 8 slices at 256 37.3 / 35.8, 2048 x 8192 at 400 23.4 / 22.1.  More rows read it at
-// different times (plain 4096 x 2048 at 1999 31.7 / 33.6), and so do more rounds (the wide tile, gated
-// 28672 x 4096 at 8192 1248 / 1288).
+// Narrow tiles of one m-tile, and of two whose second is more than half full, so that both read W
+// together, ask for it past the caches' order of use: us in order / past it, gated 28672 x 4096 at 224 / 256
+// rows 67.4 / 61.3, 64.6 / 61.8, 22016 x 4096 at 256 58.7 / 56.5, 16384 x 4096 at 256 / 512 55.4 / 53.8, 61.0
+// / 60.4, 16384 x 2048 at 256 / 512 29.8 / 30.0, 32.7 / 32.2, 14336 x 2048 28.9 / 29.4, 30.5 / 30.8, 16384 x
+// 1024 at 512 19.6 / 19.1; over 17 sizes at 400 and 512 rows 0.98 to 1.04, 1.2 % faster.  A second m-tile of few
+// rows is ahead, and W is read twice (at 257 15360 x 2560 36.5 / 44.4, 16384 x 5120 73.4 / 86.0, 4096 x 14336
+// 135 / 179); so do more rows (plain 4096 x 2048 at 1999 31.7 / 33.6) and more rounds (the wide tile, gated
+// 28672 x 4096 at 8192 1248 / 1288).  Not beside fp32 slabs (2560 x 10240 in 5 at 257 / 512 30.6 / 35.3, 36.1 /
+// 39.1, 4096 x 14336 in 4 53.8 / 59.9, 60.3 / 61.3, 4096 x 8192 34.3 / 33.5, 37.0 / 37.9; 2048 x 8192 in 8
+// would gain, 24.3 / 22.0, 23.3 / 23.1); fp16 ones are of one m-tile (4096 x 14336 in 8 at 224 / 256 36.4 /
+// 37.5, 37.9 / 36.7).
 template <int EPI>
 void launch_narrow(const PArgs& a, dim3 grid, hipStream_t s) {
-  if (a.M <= 512)
-    launch<EPI, NARROW, true>(a, grid, s);
-  else
-    launch<EPI, NARROW>(a, grid, s);
+  if constexpr (EPI != 11)
+    if (a.M <= 256 || (a.M > 384 && a.M <= 512)) {
+      launch<EPI, NARROW, true>(a, grid, s);
+      return;
+    }
+  launch<EPI, NARROW>(a, grid, s);
 }
 
 // out = X . W^T on tiles of 128 x 128, a wave 64 x 64 of them, for steps whose larger tiles are half a
