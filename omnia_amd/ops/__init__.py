@@ -267,9 +267,10 @@ def decode_tile_config(M: int, N: int, K: int, mode: int) -> tuple[int, int, int
     a gate_up whole, EPI 1) for decode projections of 193 to 256 rows that it runs in the place of
     :func:`wgemm_config`'s entry, where a model may use it (``ops/tuned/decode_tile_mi355x.json``), or
     None.  us, weights from HBM, tgemm on packed copies / so, at 193, 224 and 256 rows: gated 28672 x 4096
-    68.6 / 65.2, 69.8 / 63.8, 71.1 / 64.4, in a model of them at 256 69.9 / 63.6; 4096 x 14336 38.6 / 36.8,
-    38.2 / 37.5, 39.0 / 37.6, in the model 39.9 / 38.9.  Not 8192 x 28672, with its consumer (row-major) 126 /
-    126, 129 / 125, 129 / 129."""
+    68.6 / 65.2, 69.8 / 63.8, 71.1 / 64.4; 4096 x 14336 38.6 / 36.8, 38.2 / 37.5, 39.0 / 37.6.  In a model's
+    step under the trace, by the run, 66.9 to 69.9 / 63.6 to 68.7 and 37.8 to 39.9 / 38.3 to 38.9; the step is
+    1.01 to 1.04 times as fast.  Not 8192 x 28672, with its consumer (row-major) 126 / 126, 129 / 125, 129 /
+    129."""
     global _decode_tiles
     if not _wgemm_on or not 192 < M <= WGEMM_MAX_M:
         return None
@@ -578,7 +579,8 @@ def small_tile_cols(M: int, w: torch.Tensor) -> int:
     58.5.  64: 2048 x 2048 at 512 .50 13.1 / 12.5, 700 .68 13.8 / 14.7, 999 .98 14.6 / 17.3; 4096 x 2048 at
     512 1.0 14.7 / 17.1; 1472 x 512 at 1075 .75 6.9 / 10.3; 1600 x 2560 at 726 .55 16.9 / 17.3, 2688 x 2560
     at 550 .70 17.6 / 17.4; 3584 x 4096 at 393 .67 24.5 / 29.2; 2048 x 6144 at 860 .84 39.0 / 42.0).  Over
-    160 such sizes the library takes .99 to 1.5 as long."""
+    160 such sizes the library takes .99 to 1.5 as long.  Models ask for whole 128 of rows and K
+    (``Projections._pgemm_covers``), :func:`linear` for any of these."""
     return small_cols(M, *w.shape) if w.dim() == 2 and w.is_contiguous() and _on_grid(w) else 0
 
 

@@ -13,9 +13,9 @@
 //     no bank conflicts), in a ring of ten: two K-tiles and B of a third, as W often comes from HBM
 //     and x from the L2 of the XCD (us with A / B of the third: gated 28672 x 4096 at 512 rows 98 /
 //     95.6, at 2001 329 / 324, at 2560 in a model 444 / 425, 16384 x 2048 at 16384 744 / 740, plain
-//     4096 x 14336 in 8 slices at 512 49.3 / 47.7, experts' down of 8 x 2048 x 4096 at 2001 tokens
-//     83 / 79, up at 16384 882 / 876).  EPI 2 and 3, of the dense models' large prompts, A of a third
-//     (in a model, us a product, A / B: EPI 2 at 2560 rows 180 / 182, 8192 408 / 415, 16384 811 / 824,
+//     4096 x 14336 in 8 slices at 512 49.3 / 47.7, experts' up of 8 x 2048 x 4096 at 16384 tokens
+//     882 / 876, down at 2001 / 2400 / 8000 / 16384 85.5 / 84, 86.5 / 84.5, 208 / 211, 424 / 427).  EPI 2
+//     and 3, of the dense models' large prompts, A of a third (in a model, us a product, A / B: EPI 2 at 2560 rows 180 / 182, 8192 408 / 415, 16384 811 / 824,
 //     EPI 3 103 / 104, 307 / 309, 608 / 611).  Two barriers a K-tile:
 //     one once every wave has read it (its slots are asked for again), one once the next has
 //     landed, 40 products later; up to 96 KB are in flight, waits are counted;
@@ -884,7 +884,7 @@ void launch_narrow(const PArgs& a, dim3 grid, hipStream_t s) {
 
 // out = X . W^T on tiles of 128 x 128, a wave 64 x 64 of them, for steps whose larger tiles are half a
 // round or less: us, library / here and narrow tile, 2048 x 2048 at 2001 rows 21.7 / 19.0 and 24.2, 4096
-// x 2048 at 999 24.6 / 21.2 and 28.7, 3072 x 1024 at 999 14.3 / 11.6 and 15.2 (ops.small_tile_pays).  A K-tile
+// x 2048 at 999 24.6 / 21.2 and 28.7, 3072 x 1024 at 999 14.3 / 11.6 and 15.2 (ops.small_tile_cols).  A K-tile
 // is a half-tile of each operand in a ring of five, 128 KB in flight; its 32 products a wave take half of
 // the 0.42 us of its intake (78 GB/s a CU), so one barrier a K-tile does: every wave has read K-tile t,
 // and t + 1 has landed.
