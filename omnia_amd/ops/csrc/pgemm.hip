@@ -15,8 +15,9 @@
 //     95.6, at 2001 329 / 324, at 2560 in a model 444 / 425, 16384 x 2048 at 16384 744 / 740, plain
 //     4096 x 14336 in 8 slices at 512 49.3 / 47.7, experts' up of 8 x 2048 x 4096 at 16384 tokens
 //     882 / 876, down at 2001 / 2400 / 8000 / 16384 85.5 / 84, 86.5 / 84.5, 208 / 211, 424 / 427).  EPI 2
-//     and 3, of the dense models' large prompts, A of a third (in a model, us a product, A / B: EPI 2 at 2560 rows 180 / 182, 8192 408 / 415, 16384 811 / 824,
-//     EPI 3 103 / 104, 307 / 309, 608 / 611).  Two barriers a K-tile:
+//     and 3, of the dense models' large prompts, A of a third (in a model, us a product, A / B: EPI 2
+//     at 2560 rows 180 / 182, 8192 408 / 415, 16384 811 / 824, EPI 3 103 / 104, 307 / 309, 608 / 611).
+//     Two barriers a K-tile:
 //     one once every wave has read it (its slots are asked for again), one once the next has
 //     landed, 40 products later; up to 96 KB are in flight, waits are counted;
 //   * fragments of 32 k are read half a K-tile ahead, one read every other product, and the 16
